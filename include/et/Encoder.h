@@ -267,6 +267,38 @@ template <typename attn_t, typename linear1_t, typename linear2_t, typename ACT_
             return false;
         }
     }
+    // This layer's weights of a token-local launch (et_encoder_layer_f32), the QKV projection left to the caller, and
+    // that projection as the layer before needs it.  false when the layer's types have no such form.
+    bool local_weights(et_layer_weights &w) {
+        if constexpr (attn_has_split<attn_t>::value && std::is_same_v<linear1_t, Linear<tile_mat>> &&
+                      std::is_same_v<linear2_t, Linear<tile_mat>>) {
+            set_weight(w, 0, attn->o_linear());
+            set_weight(w, 1, *linear1);
+            set_weight(w, 2, *linear2);
+            w.gamma[0] = f16(LN1->gamma());
+            w.beta[0] = f16(LN1->beta());
+            w.gamma[1] = f16(LN2->gamma());
+            w.beta[1] = f16(LN2->beta());
+            return true;
+        } else {
+            (void)w;
+            return false;
+        }
+    }
+    bool local_qkv(et_layer_weights &w) {
+        if constexpr (attn_has_split<attn_t>::value) set_weight(w, 3, attn->qkv_linear());
+        else (void)w;
+        return attn_has_split<attn_t>::value;
+    }
+    half *qkv_buffer() {
+        if constexpr (attn_has_split<attn_t>::value) return attn->qkv_buffer();
+        else return nullptr;
+    }
+    half *z_buffer() {
+        if constexpr (attn_has_split<attn_t>::value) return attn->z_buffer();
+        else return nullptr;
+    }
+    float epsilon(int k) const { return k ? LN2->epsilon() : LN1->epsilon(); }
     // the first layer's QKV projection of the binary16 input, and the attention kernel alone
     void chain_qkv_first(half *x16, stream_t stream = nullptr) {
         if constexpr (attn_has_split<attn_t>::value) attn->qkv_linear().forward(attn->qkv_buffer(), x16, stream);
@@ -313,6 +345,13 @@ template <typename attn_t, typename linear1_t, typename linear2_t, typename ACT_
     }
 
   private:
+    static void set_weight(et_layer_weights &w, int i, Linear<tile_mat> &l) {
+        w.row_ptr[i] = l.weight.row_ptr.get();
+        w.col_idx[i] = l.weight.row_offset.get();
+        w.tiles[i] = f16(l.weight.data.get());
+        w.bias[i] = f16(l.bias.get());
+    }
+    template <typename other> static void set_weight(et_layer_weights &, int, other &) {}
     bool wide = false, wide_split = false;
     std::unique_ptr<DeviceBuffer<float>> src32;
     std::unique_ptr<DeviceBuffer<float>> stats1, stats2, fin_in, fin1;

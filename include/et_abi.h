@@ -270,6 +270,37 @@ int et_encoder_chain_supported(const et_chain_desc *desc);
 int et_encoder_chain_f32(const et_chain_desc *desc, int *stat_groups2, et_stream stream);
 int et_encoder_chain_status(const uint32_t *sync, int *gave_up, int *misplaced);
 
+/* Everything of a tile-sparse encoder layer that is local to a token, in one launch (two with
+ * parts > 1): from the attention output Z and the layer input x,
+ *   y = LN1(Z Wo^T + bo + x);  x' = LN2(act(y W1^T + b1) W2^T + b2 + y);  QKV = x' Wq^T + bq
+ * (Encoder/Encoder.h:81-96 and the next layer's projection, Attention/Attention.h:246-265), sums and
+ * normalisations in binary32, matrix-core operands in binary16.
+ * et_encoder_layer_pack_create copies the weights into the order the launch streams them in; all
+ * pointers of et_layer_weights are device pointers: [0] Wo, [1] W1, [2] W2, [3] Wq (16x16 BSR and
+ * bias; [3] unread with qkv_out = 0), gamma / beta of LN1 and LN2.  mt: token rows of a workgroup
+ * over 16 (1 or 2); parts: workgroups that share them (1, or with mt = 1 up to 32, for few token rows).
+ * et_encoder_layer_supported: 1 where a pack can be built: T and all widths multiples of 16, emdim <=
+ * 1024, dimFF <= 4096, qkv_out <= 3072 (0: no projection follows).
+ * et_encoder_layer_f32: Z [T x emdim]; the residual x in binary32 (x32, in tile order) or, with x32
+ * NULL, binary16 (x16 [T x emdim]); x' goes to x32_out in tile order and to out16 [T x emdim] (either
+ * may be NULL); QKV [T x qkv_out]; partial: parts * T * emdim floats of workspace (unread with parts =
+ * 1).  x32_out may not be x32.  Tile order, of T * emdim floats: for 16 tokens after 16 tokens, and 16
+ * features after 16 features in them, 256 values: token r, features 4g .. 4g + 3 at 4 (16 g + r). */
+struct et_layer_pack_s;
+typedef struct et_layer_weights {
+    const int32_t *row_ptr[4], *col_idx[4];
+    const et_f16 *tiles[4], *bias[4];
+    const et_f16 *gamma[2], *beta[2];
+} et_layer_weights;
+int et_encoder_layer_supported(int T, int emdim, int dimFF, int qkv_out);
+int et_encoder_layer_pack_create(const et_layer_weights *w, int T, int emdim, int dimFF, int qkv_out, int mt, int parts,
+                                 struct et_layer_pack_s **pack);
+int et_encoder_layer_pack_destroy(struct et_layer_pack_s *pack);
+int et_encoder_layer_f32(const struct et_layer_pack_s *pack, const et_f16 *Z, const float *x32, const et_f16 *x16,
+                         float *x32_out, et_f16 *out16, et_f16 *QKV, float *partial, int act, float eps1, float eps2,
+                         et_stream stream);
+
+
 /* SkipLayerNorm fused into the tile-sparse Linear that consumes it:
  *   ln_out = LayerNorm(src + skip) * gamma + beta      (written, [T x in])
  *   Y      = act(ln_out * W^T + bias)
@@ -811,7 +842,10 @@ typedef struct et_model_desc {
                     *    4: as 1, with the QKV projection of every layer after the first inside
                     *    its attention kernel (et_norm_qkv_mha_f32in: four launches per layer)
                     *    where the shapes allow, else as 1; 5: as 1, always with five launches.
-                    * 0: every activation is stored as binary16 (the reference's storage) */
+                    * 0: every activation is stored as binary16 (the reference's storage).
+                    * 0 and 1 run everything between two attention kernels in one or two
+                    * token-local launches (et_encoder_layer_f32; the residual is binary32 then,
+                    * under 0 too) where the layers are tile-sparse and it measured faster */
 } et_model_desc;
 
 /* which matrix of a layer */
@@ -853,10 +887,11 @@ int et_model_forward(et_model m, et_f16 *out, const et_f16 *in, et_stream stream
 int et_model_forward_layer(et_model m, int layer, et_f16 *out, const et_f16 *in,
                            et_stream stream);
 int et_model_sync(et_model m);
-/* kernel launches per encoder layer of a finalized model in the mode it actually runs
- * (2: chain launches, 5: SkipLayerNorm folded into the projections, 7: SkipLayerNorm on its own;
- * 0 before et_model_finalize).  A model asked for mixed = 3 reports 5 once it has gone back to
- * separate launches. */
+/* kernel launches an encoder layer of a finalized model is divided into, projection by projection
+ * (2: chain launches, 4: the QKV projection inside the attention kernel, 5: SkipLayerNorm folded into
+ * the projections, 7: SkipLayerNorm on its own; 0 before et_model_finalize).  et_model_forward may
+ * issue several of them as one token-local launch (et_encoder_layer_f32).  A model asked for mixed = 3
+ * reports 5 once it has gone back to separate launches. */
 int et_model_launches_per_layer(et_model m, int *launches);
 int et_model_destroy(et_model m);
 

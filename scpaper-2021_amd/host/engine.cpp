@@ -31,6 +31,11 @@ struct ILayer {
     virtual void chain_qkv_first(half *x16, stream_t stream) = 0;
     virtual void chain_attention(stream_t stream) = 0;
     virtual et::AttnState &attn() = 0;
+    virtual bool local_weights(et_layer_weights &w) = 0;
+    virtual bool local_qkv(et_layer_weights &w) = 0;
+    virtual half *qkv_buffer() = 0;
+    virtual half *z_buffer() = 0;
+    virtual float epsilon(int k) const = 0;
 };
 
 template <typename EncoderT> struct LayerOf final : ILayer {
@@ -56,6 +61,14 @@ template <typename EncoderT> struct LayerOf final : ILayer {
     void chain_qkv_first(half *x16, stream_t stream) override { enc->chain_qkv_first(x16, stream); }
     void chain_attention(stream_t stream) override { enc->chain_attention(stream); }
     et::AttnState &attn() override { return enc->attention(); }
+    bool local_weights(et_layer_weights &w) override { return enc->local_weights(w); }
+    bool local_qkv(et_layer_weights &w) override { return enc->local_qkv(w); }
+    half *qkv_buffer() override { return enc->qkv_buffer(); }
+    half *z_buffer() override { return enc->z_buffer(); }
+    float epsilon(int k) const override { return enc->epsilon(k); }
+};
+struct LayerPackDeleter {
+    void operator()(et_layer_pack_s *p) const { (void)et_encoder_layer_pack_destroy(p); }
 };
 
 // One weight matrix as handed over by the caller (host memory).
@@ -100,6 +113,10 @@ struct et_model_s {
     bool chain = false;
     std::vector<et_chain_desc> chain_desc;
     std::unique_ptr<et::DeviceBuffer<int>> chain_sync;
+    // everything between two attention kernels in one token-local launch (et_encoder_layer_f32), or in two with
+    // several workgroups to a token strip: one pack per layer, the residual between layers, the shares of a strip
+    std::vector<std::unique_ptr<et_layer_pack_s, LayerPackDeleter>> local;
+    std::unique_ptr<et::DeviceBuffer<float>> local_x[2], local_partial;
 
     stream_t own_stream = nullptr;
     et_graph graph = nullptr;
@@ -288,6 +305,89 @@ bool chain_ran_clean(et_model_s &m, std::string &why) {
     return true;
 }
 
+// How a stack divides a token strip: token rows of a workgroup over 16, and workgroups that share a strip; mt == 0: the
+// separate launches are faster.
+struct LocalPlan {
+    int mt = 0, parts = 1;
+};
+// Every workgroup streams the kept tiles of the output projection and its share of the others at about 112 KiB/us, and
+// sharing a strip costs a second launch and the exchange of the shares, about 5 us and half a microsecond per share
+// (fitted at 768 wide, 60 to 95 % sparsity, 256 to 2048 rows): the number of parts that makes the sum least, while there
+// is a compute unit for every workgroup of an XCD.  Above 256 strips of 16 rows a workgroup takes 32.
+// Against the separate launches (two- to four-layer stacks, 384 to 1024 wide, 40 to 95 % sparsity) it is 1.04 - 2.3 times
+// as fast above 512 rows (1.5 - 2.3 at 8192; 0.93 for 1024 wide at 40 % in binary16, which runs dense GEMMs) and at any row
+// count up to 512 wide, and 1.19 - 1.27 between 256 and 512 rows that are not a whole number of 32-row strips per XCD.  Of
+// the rest the estimate decides: at 512 rows 1.00 - 1.10 up to 14.5 us, 0.92 - 0.97 above; at 128 rows 1.00 - 1.08 up to
+// 10.5 us, 0.89 - 0.92 above.
+LocalPlan plan_local(const et_model_s &m) {
+    LocalPlan p;
+    const et_model_desc &d = m.desc;
+    double kib[4] = {0, 0, 0, 0};  // of a layer, on average
+    for (const HostLayer &h : m.host)
+        for (int w = 0; w < 4; w++) {
+            if (h.w[(size_t)w].kind != HostMatrix::Bsr16) return p;
+            kib[w] += 0.5 * (double)h.w[(size_t)w].column.size() / (double)m.host.size();
+        }
+    const int rows = m.rows(), strips = (rows + 15) / 16;
+    if (strips > 256) {
+        p.mt = 2;
+        return p;
+    }
+    // (all binary16: small stacks keep the launches whose results et_model_forward_layer repeats bit for bit)
+    if (d.mixed == 0 && rows < 256) return p;
+    const double shared = kib[ET_W_QKV] + kib[ET_W_FF1] + kib[ET_W_FF2];
+    double best = 0;
+    for (int parts = 1; parts <= 12 && parts * ((strips + 7) / 8) <= 32; parts++) {
+        const double us = (kib[ET_W_O] + shared / parts) / 112.0 + (parts > 1 ? 5.0 + 0.5 * parts : 0.0);
+        if (parts == 1 || us < best) {
+            best = us;
+            p.parts = parts;
+        }
+    }
+    const bool uneven = rows > 256 && (rows + 31) / 32 % 8 != 0;
+    const double most = rows >= 512 || (rows >= 256 && d.emdim <= 768) ? 14.5 : 10.5;
+    if (rows > 512 || uneven || d.emdim <= 512 || best <= most) p.mt = 1;
+    const double dense = (4.0 * d.emdim + 2.0 * d.dimFF) * d.emdim / 512.0;  // KiB of all tiles
+    if (d.mixed == 0 && d.emdim > 768 && rows <= 4096 && kib[ET_W_O] + shared > 0.5 * dense) p.mt = 0;
+    return p;
+}
+
+// The packs of the token-local launches; leaves m.local empty where a layer has no such form.
+void build_local(et_model_s &m) {
+    const LocalPlan plan = plan_local(m);
+    const et_model_desc &d = m.desc;
+    const int n = (int)m.layers.size(), ldq = 2 * d.kdim + d.vdim;
+    if (plan.mt == 0 || d.kdim != d.emdim || d.vdim != d.emdim || et_encoder_layer_supported(m.rows(), d.emdim, d.dimFF, ldq) != 1) return;
+    std::vector<std::unique_ptr<et_layer_pack_s, LayerPackDeleter>> packs;
+    for (int i = 0; i < n; i++) {
+        et_layer_weights w{};
+        if (!m.layers[(size_t)i]->local_weights(w) || (i + 1 < n && !m.layers[(size_t)i + 1]->local_qkv(w))) return;
+        et_layer_pack_s *p = nullptr;
+        const int s = et_encoder_layer_pack_create(&w, m.rows(), d.emdim, d.dimFF, i + 1 < n ? ldq : 0, plan.mt, plan.parts, &p);
+        if (s == ET_ERR_UNSUPPORTED) return;
+        etChk(s);
+        packs.emplace_back(p);
+    }
+    const size_t elems = (size_t)m.rows() * d.emdim;
+    for (auto &b : m.local_x) b = std::make_unique<et::DeviceBuffer<float>>(elems);
+    if (plan.parts > 1) m.local_partial = std::make_unique<et::DeviceBuffer<float>>(elems * plan.parts);
+    m.local = std::move(packs);
+}
+
+void run_layers_local(et_model_s &m, half *out, half *in, stream_t stream) {
+    const int n = (int)m.layers.size();
+    m.layers[0]->chain_qkv_first(in, stream);
+    for (int i = 0; i < n; i++) {
+        ILayer &l = *m.layers[(size_t)i];
+        const bool last = i == n - 1;
+        l.chain_attention(stream);
+        etChk(et_encoder_layer_f32(m.local[(size_t)i].get(), et::f16(l.z_buffer()), i ? m.local_x[(i - 1) & 1]->get() : nullptr,
+                                   et::f16(in), last ? nullptr : m.local_x[i & 1]->get(), last ? et::f16(out) : nullptr,
+                                   last ? nullptr : et::f16(m.layers[(size_t)i + 1]->qkv_buffer()),
+                                   m.local_partial ? m.local_partial->get() : nullptr, m.desc.act, l.epsilon(0), l.epsilon(1), stream));
+    }
+}
+
 void run_layers_split(et_model_s &m, half *out, half *in, stream_t stream) {
     if (m.chain) return run_layers_chain(m, out, in, stream);
     const int n = (int)m.layers.size();
@@ -317,6 +417,7 @@ void run_layers_mixed(et_model_s &m, half *out, half *in, stream_t stream) {
 }
 
 void run_layers(et_model_s &m, half *out, half *in, stream_t stream) {
+    if (!m.local.empty()) return run_layers_local(m, out, in, stream);
     if (m.desc.mixed) return run_layers_mixed(m, out, in, stream);
     const int n = (int)m.layers.size();
     half *src = in;
@@ -489,23 +590,28 @@ int et_model_finalize(et_model m) {
         const size_t act_elems = (size_t)m->rows() * m->desc.emdim;
         for (auto &b : m->pp) b = std::make_unique<et::DeviceBuffer<half>>(act_elems);
         m->warm = std::make_unique<et::DeviceBuffer<half>>(act_elems);
+        // The QKV projection inside the attention kernel: asked for (mixed == 4), or where it measured faster than
+        // the two launches it replaces — one workgroup per (sequence, head) that reads and normalises its whole
+        // sequence: 12-layer 768-wide stacks at 80 / 90 / 95 % sparsity ran 0.89 - 0.99 of the five-launch time
+        // with 96 to 384 such workgroups (sequences of 32 to 128 tokens) — 96 of them on sequences of 96 or 128
+        // tokens 0.99 - 1.01 —, 1.04 - 1.05 at 72 and below, 1.09 - 1.11 at 768.
+        const et_model_desc &d = m->desc;
+        const long heads = (long)d.batch * d.nhead;
+        const bool want_fused = (d.mixed == 4 || (d.mixed == 1 && heads >= 96 && heads <= 400)) && m->layers.size() > 1;
+        const bool fused_ok = want_fused && et_norm_qkv_mha_f32in_supported(d.batch, d.seq_len, d.emdim, d.nhead, d.kdim / d.nhead) == 1;
+        if (d.mixed == 0 || d.mixed == 1 || (d.mixed == 4 && !fused_ok)) build_local(*m);
         if (m->desc.mixed) {
             for (auto &b : m->pp32) b = std::make_unique<et::DeviceBuffer<float>>(act_elems);
             for (auto &l : m->layers) l->enable_mixed();
             // mixed == 1: the engine folds SkipLayerNorm into the projections where every layer can
             m->split = (m->desc.mixed == 1 || m->desc.mixed == 3 || m->desc.mixed == 4 || m->desc.mixed == 5) && !m->layers.empty();
             for (auto &l : m->layers) m->split = m->split && l->split_ok();
-            if (m->split) {
+            if (m->split && !m->local.empty()) {
+                m->fused_qkv = fused_ok;  // (the form the layers have without the token-local launches)
+            } else if (m->split) {
                 for (auto &l : m->layers) l->enable_split();
                 m->chain = m->desc.mixed == 3 && build_chain(*m);
-                // The QKV projection inside the attention kernel: asked for (mixed == 4), or where it measured faster than
-                // the two launches it replaces — one workgroup per (sequence, head) that reads and normalises its whole
-                // sequence: 12-layer 768-wide stacks at 80 / 90 / 95 % sparsity ran 0.89 - 0.99 of the five-launch time
-                // with 96 to 384 such workgroups (sequences of 32 to 128 tokens) — 96 of them on sequences of 96 or 128
-                // tokens 0.99 - 1.01 —, 1.04 - 1.05 at 72 and below, 1.09 - 1.11 at 768.
-                const long heads = (long)m->desc.batch * m->desc.nhead;
-                const bool pays = heads >= 96 && heads <= 400;
-                if ((m->desc.mixed == 4 || (m->desc.mixed == 1 && pays)) && m->layers.size() > 1) {
+                if (want_fused) {
                     m->fused_qkv = true;
                     // (the affine part of the normalisation a layer is handed — the second one of the layer before —
                     // goes into its projection's pack)

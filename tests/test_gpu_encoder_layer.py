@@ -1,0 +1,139 @@
+"""The token-local launches of an encoder layer (et_encoder_layer_f32: output projection, LayerNorm, FFN, LayerNorm and
+the next QKV projection of a strip of token rows in one workgroup, or in several that share the strip) against the
+binary32 mathematics of the same steps."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import layers as L
+from tests import harness as Hn
+from tests.harness import up
+
+pytestmark = pytest.mark.gpu
+
+
+class Weights(C.Structure):
+    """et_layer_weights of include/et_abi.h"""
+    _fields_ = [(n, C.c_void_p * 4) for n in ("row_ptr", "col_idx", "tiles", "bias")] + [(n, C.c_void_p * 2) for n in ("gamma", "beta")]
+
+
+def tile_order(x):
+    """[T x H] -> tile order: 16 tokens x 16 features together, token r, features 4g .. 4g + 3 at 4 (16 g + r)."""
+    T, H = x.shape
+    return np.ascontiguousarray(x.reshape(T // 16, 16, H // 16, 4, 4).transpose(0, 2, 3, 1, 4))
+
+
+def row_order(t, T, H):
+    return np.ascontiguousarray(t.reshape(T // 16, H // 16, 4, 16, 4).transpose(0, 3, 1, 2, 4)).reshape(T, H)
+
+
+# widths at the edges: one block-row per wave and fewer (16, 48, 240, 256), two to four with waves that hold one less
+# (272, 384, 800), the widest; hidden widths of one block-row, of one chunk, of several; 16 to 80 rows so that a 32-row
+# strip ends in half a strip; shares that divide the block-rows and that do not; empty and nearly full weights
+CASES = [(16, 16, 16, 1, 1, 0.0), (48, 48, 32, 2, 1, 0.5), (240, 256, 80, 1, 3, 0.7), (256, 1024, 16, 1, 7, 0.95),
+         (272, 208, 48, 2, 1, 0.8), (384, 1536, 64, 1, 4, 0.6), (768, 3072, 48, 1, 1, 0.8), (768, 3072, 80, 2, 1, 0.8),
+         (768, 3072, 32, 1, 5, 0.9), (800, 208, 48, 1, 2, 0.3), (800, 208, 48, 2, 1, 0.6), (1024, 4096, 48, 2, 1, 0.9),
+         (1024, 4096, 32, 1, 12, 0.95), (1024, 4096, 16, 1, 1, 0.1)]
+
+
+@pytest.mark.parametrize("H,FF,T,mt,parts,sparsity", CASES)
+@pytest.mark.parametrize("project,act", [(True, 2), (False, 1)])
+def test_token_local_layer(et, H, FF, T, mt, parts, sparsity, project, act):
+    lib = et.lib()
+    Q = 3 * H if project else 0
+    mats = [Hn.BsrWeight(o, i, sparsity, seed=31 + k, std=0.05, bias_std=0.1)
+            for k, (o, i) in enumerate(((H, H), (FF, H), (H, FF), (3 * H, H)))]
+    norms = [Hn.randn((H,), 60 + k, 0.1) for k in range(4)]
+    norms[0], norms[2] = norms[0] + np.float16(1), norms[2] + np.float16(1)
+    Z, x16 = Hn.randn((T, H), 70), Hn.randn((T, H), 71)
+    x32 = Hn.randn((T, H), 72, dtype=np.float32)
+    w, keep = Weights(), []
+    for k, m in enumerate(mats):
+        for name, arr in (("row_ptr", m.row_ptr), ("col_idx", m.col_idx if len(m.col_idx) else np.zeros(1, np.int32)),
+                          ("tiles", m.tiles if len(m.tiles) else np.zeros((1, 256), np.float16)), ("bias", m.bias)):
+            keep.append(up(et, arr))
+            getattr(w, name)[k] = keep[-1].ptr
+    for k in range(2):
+        for name, arr in (("gamma", norms[2 * k]), ("beta", norms[2 * k + 1])):
+            keep.append(up(et, arr))
+            getattr(w, name)[k] = keep[-1].ptr
+    assert lib.et_encoder_layer_supported(T, H, FF, Q) == 1
+    pack = C.c_void_p()
+    et.check(lib.et_encoder_layer_pack_create(C.byref(w), T, H, FF, Q, mt, parts, C.byref(pack)))
+    dZ, d16 = up(et, Z), up(et, x16)
+    f = Hn.f32
+
+    def half(t):  # what a matrix-core operand is rounded to
+        return t.to(torch.float16).float()
+
+    for wide in (True, False):
+        d32 = up(et, tile_order(x32))
+        o32 = et.DeviceBuffer.empty((T, H), np.float32)
+        o16 = et.DeviceBuffer.empty((T, H), np.float16)
+        qkv = et.DeviceBuffer.empty((T, 3 * H), np.float16)
+        partial = et.DeviceBuffer.empty((parts, T, H), np.float32)
+        for _ in range(2):  # the second run on what the first left in the workspace
+            et.check(lib.et_encoder_layer_f32(pack, dZ.ptr, d32.ptr if wide else None, None if wide else d16.ptr, o32.ptr, o16.ptr,
+                                              qkv.ptr if Q else None, partial.ptr, act, 1e-5, 1e-5, None))
+        x = torch.from_numpy(x32) if wide else f(x16)
+
+        def norm(v, k):
+            return torch.nn.functional.layer_norm(v, (H,), f(norms[2 * k]), f(norms[2 * k + 1]), 1e-5)
+
+        def lin(v, m):
+            return v @ f(m.dense).T + f(m.bias)
+
+        y = norm(lin(f(Z), mats[0]) + x, 0)
+        h = lin(half(y), mats[1])
+        h = torch.relu(h) if act == 1 else torch.nn.functional.gelu(h, approximate="tanh")
+        want = norm(lin(half(h), mats[2]) + y, 1)
+        got = torch.from_numpy(row_order(o32.numpy(), T, H).copy())
+        # the hidden operand's rounding (2^-11 of its values) may fall the other way where the sums differ in their last
+        # bits: relative error of the layer's result well below one binary16 unit
+        assert torch.norm(got - want) / torch.norm(want) <= 2e-4
+        assert Hn.max_abs(o16.numpy(), got.numpy()) <= 4e-3
+        if Q:
+            want_q = lin(half(got), mats[3])
+            assert torch.norm(f(qkv.numpy()) - want_q) / torch.norm(want_q) <= 5e-4
+    et.check(lib.et_encoder_layer_pack_destroy(pack))
+
+
+@pytest.mark.parametrize("H,nh,FF,S,B,sparsity,mixed", [(256, 4, 512, 32, 3, 0.7, 1), (768, 12, 512, 112, 7, 0.8, 0),
+                                                        (384, 6, 1536, 16, 1, 0.9, 1), (128, 2, 256, 16, 270, 0.6, 1)])
+def test_stacks_on_token_local_launches(et, H, nh, FF, S, B, sparsity, mixed):
+    """Stacks the engine runs this way by itself (48 to 4320 rows: shared strips, one workgroup a strip, 32-row strips):
+    graph and eager the same bits, in place, and near the oracle."""
+    layers = [Hn.LayerWeights(H, nh, FF, sparsity, seed=800 + i) for i in range(3)]
+    lens = np.random.default_rng(S).integers(S // 2, S + 1, B).astype(np.int32)
+    x = Hn.randn((B * S, H), 811)
+    outs = []
+    for use_graph in (True, False):
+        m = Hn.build_model(et, layers, S, B, lens=lens, mixed=mixed, use_graph=use_graph)
+        d = et.DeviceBuffer.from_numpy(x)
+        o = et.DeviceBuffer.empty(x.shape, np.float16)
+        m.forward(o, d)
+        m.sync()
+        outs.append(o.numpy())
+        m.forward(d, d)
+        m.sync()
+        outs.append(d.numpy())
+    for o in outs[1:]:
+        assert np.array_equal(outs[0], o)
+    want = Hn.oracle_stack(x, layers, B, lens, store=torch.float16, resid=torch.float32)
+    a, b = outs[0].astype(np.float32), want.astype(np.float32)
+    for i in range(B):
+        a[i * S + lens[i]:(i + 1) * S] = 0
+        b[i * S + lens[i]:(i + 1) * S] = 0
+    assert Hn.max_abs(a, b) <= 4e-3  # one binary16 unit at |x| <= 4 and noise, as for the other forms of the residual
+
+
+def test_token_local_refusals(et):
+    lib, w, pack = et.lib(), Weights(), C.c_void_p()
+    assert lib.et_encoder_layer_supported(32, 1040, 256, 0) == 0 and lib.et_encoder_layer_supported(24, 256, 256, 0) == 0
+    assert lib.et_encoder_layer_supported(32, 256, 4112, 0) == 0 and lib.et_encoder_layer_supported(32, 256, 256, 3088) == 0
+    assert lib.et_encoder_layer_pack_create(C.byref(w), 32, 256, 256, 0, 1, 1, C.byref(pack)) == et.ET_ERR_INVALID_ARG
+    assert lib.et_encoder_layer_pack_create(C.byref(w), 32, 256, 256, 0, 2, 2, C.byref(pack)) == et.ET_ERR_INVALID_ARG
+    assert lib.et_encoder_layer_pack_create(None, 32, 256, 256, 0, 1, 1, C.byref(pack)) == et.ET_ERR_INVALID_ARG
+    assert lib.et_encoder_layer_f32(None, None, None, None, None, None, None, None, 0, 1e-5, 1e-5, None) == et.ET_ERR_INVALID_ARG
