@@ -137,12 +137,18 @@ __global__ __launch_bounds__(256) void linear_dense_f32_kernel(const LinearF32Ar
 }
 
 // ---- fused attention ------------------------------------------------------------
-// One workgroup = 16 queries of one head of one sequence.  The 16 x S strip of scores
-// lives in LDS as fp32; K and V pass through LDS in blocks of 64 keys.  Thread
-// (q = tid/16, c = tid%16) owns scores of keys c, c+16, .. of query q and output
-// features c, c+16, .. of query q.
+// One workgroup of 4 waves = 16 queries of one head of one sequence.  The 16 x S strip of scores lives in LDS; Q, K and V
+// go from memory straight into the operands of v_mfma_f32_16x16x4_f32, with a lane's four k-values a 16-wide cell's
+// 4q .. 4q+3 (a sum over k does not care which k a lane brings as long as both operands bring the same one).
+//   scores: waves take 16 keys in turn; A = K (row = key), B = Q, so lane (r, q) ends with keys 4q .. 4q+3 of query r
+//   softmax: 16 threads a query
+//   Z: waves take 16 features in turn; A = V transposed (row = feature), B = P: features 4q .. 4q+3 of query r
+// A few hundred workgroups is all a verification batch has, so the length of one workgroup's chain is its time: HD / 4
+// products a key block and S / 4 a feature block, 32 cycles each.  2 x 128 tokens, 12 heads of 64: 20.3 -> 7.1 us, 1 x 512 tokens 85 -> 26 (the
+// former kernel staged K and V element by element and multiplied on the vector unit).
 constexpr int kAttQ = 16;
-constexpr int kAttKeys = 64;
+constexpr int kAttKeys = 64;  // (of the LDS limit of et_mha_fused_f32)
+constexpr int kAttPad = 4;    // floats between the rows of the strip: 16 rows' cells in different banks, 16-byte aligned
 
 struct MhaF32Args {
     const float *Q, *K, *V;
@@ -155,93 +161,103 @@ struct MhaF32Args {
     int causal;
 };
 
-template <int HD>
+template <bool VEC> __device__ __forceinline__ f4 load_quad_f32(const float *p) {
+    if constexpr (VEC) return *reinterpret_cast<const f4 *>(p);
+    else return f4{p[0], p[1], p[2], p[3]};
+}
+
+// VEC: rows of Q and K start at multiples of 16 bytes.  MAXC: cells of 16 features of a head, at most.
+template <int MAXC, bool VEC>
 __global__ __launch_bounds__(256) void mha_fused_f32_kernel(const MhaF32Args a) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    float *qs = reinterpret_cast<float *>(smem_raw);  // [16][HD]
-    float *kv = qs + kAttQ * HD;                       // [64][HD + 1]
-    float *sc = kv + kAttKeys * (HD + 1);              // [16][S]
+    float *sc = reinterpret_cast<float *>(smem_raw);  // [16][S + kAttPad]
+    __shared__ float inv_sum[kAttQ];
     const int q0 = blockIdx.x * kAttQ, h = blockIdx.y, b = blockIdx.z;
-    const int q = threadIdx.x >> 4, c = threadIdx.x & 15;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, g = lane >> 4;
     const int len = a.lens ? min(max(a.lens[b], 0), a.S) : a.S;
     const size_t row0 = (size_t)b * a.S;
-    constexpr int kF = HD / 16;  // output features per thread
-
-    // head sizes between the template sizes: columns [hd, HD) are staged as zero, not written
-    const int hd = a.hd;
-    float *zrow = a.Z + (row0 + q0 + q) * a.ldz + h * hd;
+    const int hd = a.hd, ncell = hd >> 4, ld = a.S + kAttPad;
+    float *zrow = a.Z + (row0 + q0 + r16) * a.ldz + h * hd + 4 * g;
     if (len == 0) {  // a sequence without keys: zeros
+        for (int c = wave; c < ncell; c += 4)
 #pragma unroll
-        for (int i = 0; i < kF; i++)
-            if (c + 16 * i < hd) zrow[c + 16 * i] = 0.0f;
+            for (int e = 0; e < 4; e++) zrow[c * 16 + e] = 0.0f;
         return;
-    }
-    for (int i = threadIdx.x; i < kAttQ * HD; i += 256) {
-        const int r = i / HD, d = i - r * HD;
-        qs[i] = d < hd ? a.Q[(row0 + q0 + r) * a.ldq + h * hd + d] * a.scale : 0.0f;
     }
     // keys this block of queries can see
     int kend = len;
     if (a.causal) kend = min(kend, q0 + kAttQ);
+    const int nkb = (kend + 15) >> 4;
     const float ninf = -__builtin_inff();
 
-    // ---- scores
-    for (int kb = 0; kb < kend; kb += kAttKeys) {
-        __syncthreads();
-        for (int i = threadIdx.x; i < kAttKeys * HD; i += 256) {
-            const int r = i / HD, d = i - r * HD;
-            kv[r * (HD + 1) + d] = (kb + r < kend && d < hd) ? a.K[(row0 + kb + r) * a.ldk + h * hd + d] : 0.0f;
-        }
-        __syncthreads();
+    f4 qv[MAXC];
+    const float *qp = a.Q + (row0 + q0 + r16) * a.ldq + h * hd + 4 * g;
 #pragma unroll
-        for (int i = 0; i < kAttKeys / 16; i++) {
-            const int kl = c + 16 * i, key = kb + kl;
-            if (key >= kend) continue;
-            float s = 0.0f;
-#pragma unroll 8
-            for (int d = 0; d < HD; d++) s += qs[q * HD + d] * kv[kl * (HD + 1) + d];
-            if (a.mask) s += a.mask[(size_t)(q0 + q) * a.S + key];
-            if (a.causal && key > q0 + q) s = ninf;
-            sc[q * a.S + key] = s;
+    for (int c = 0; c < MAXC; c++)
+        if (c < ncell) qv[c] = load_quad_f32<VEC>(qp + 16 * c) * a.scale;
+
+    // ---- scores (a block's keys past kend: the last one again, not used below)
+    for (int kb = wave; kb < nkb; kb += 4) {
+        const float *kp = a.K + (row0 + min(kb * 16 + r16, kend - 1)) * a.ldk + h * hd + 4 * g;
+        f4 kv[MAXC];
+#pragma unroll
+        for (int c = 0; c < MAXC; c++)
+            if (c < ncell) kv[c] = load_quad_f32<VEC>(kp + 16 * c);
+        f4 s = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < MAXC; c++)
+            if (c < ncell)
+#pragma unroll
+                for (int j = 0; j < 4; j++) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[c][j], qv[c][j], s, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int key = kb * 16 + 4 * g + e;
+            if (a.mask && key < kend) s[e] += a.mask[(size_t)(q0 + r16) * a.S + key];
+            if (key >= kend || (a.causal && key > q0 + r16)) s[e] = ninf;
         }
+        *reinterpret_cast<f4 *>(sc + r16 * ld + kb * 16 + 4 * g) = s;
     }
     __syncthreads();
-    // ---- softmax over keys [0, kend) of row q: 16 threads per row
-    float m = ninf;
-    for (int k = c; k < kend; k += 16) m = fmaxf(m, sc[q * a.S + k]);
+    // ---- softmax over the keys of row q: 16 threads per row (keys past kend become zeros)
+    {
+        const int q = threadIdx.x >> 4, c = threadIdx.x & 15;
+        float m = ninf;
+        for (int k = c; k < nkb * 16; k += 16) m = fmaxf(m, sc[q * ld + k]);
 #pragma unroll
-    for (int off = 8; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 16));
-    float l = 0.0f;
-    for (int k = c; k < kend; k += 16) {
-        const float p = m == ninf ? 0.0f : __expf(sc[q * a.S + k] - m);
-        sc[q * a.S + k] = p;
-        l += p;
-    }
-#pragma unroll
-    for (int off = 8; off >= 1; off >>= 1) l += __shfl_xor(l, off, 16);
-
-    // ---- Z = P V
-    float acc[kF];
-#pragma unroll
-    for (int i = 0; i < kF; i++) acc[i] = 0.0f;
-    for (int kb = 0; kb < kend; kb += kAttKeys) {
-        __syncthreads();
-        for (int i = threadIdx.x; i < kAttKeys * HD; i += 256) {
-            const int r = i / HD, d = i - r * HD;
-            kv[r * (HD + 1) + d] = (kb + r < kend && d < hd) ? a.V[(row0 + kb + r) * a.ldv + h * hd + d] : 0.0f;
+        for (int off = 8; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 16));
+        float l = 0.0f;
+        for (int k = c; k < nkb * 16; k += 16) {
+            const float p = m == ninf || k >= kend ? 0.0f : __expf(sc[q * ld + k] - m);
+            sc[q * ld + k] = p;
+            l += p;
         }
-        __syncthreads();
-        const int nk = min(kAttKeys, kend - kb);
-        for (int k = 0; k < nk; k++) {
-            const float p = sc[q * a.S + kb + k];
 #pragma unroll
-            for (int i = 0; i < kF; i++) acc[i] += p * kv[k * (HD + 1) + c + 16 * i];
-        }
+        for (int off = 8; off >= 1; off >>= 1) l += __shfl_xor(l, off, 16);
+        if (c == 0) inv_sum[q] = l > 0.0f ? 1.0f / l : 0.0f;
     }
-    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    __syncthreads();
+    // ---- Z = P V (rows of V past kend are not multiplied, whatever they hold)
+    const float inv = inv_sum[r16];
+    for (int c = wave; c < ncell; c += 4) {
+        const float *vp = a.V + row0 * a.ldv + h * hd + c * 16 + r16;
+        f4 acc = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+        for (int kb = 0; kb < nkb; kb++) {
+            f4 v;
 #pragma unroll
-    for (int i = 0; i < kF; i++)
-        if (c + 16 * i < hd) zrow[c + 16 * i] = acc[i] * inv;
+            for (int j = 0; j < 4; j++) {
+                const int key = kb * 16 + 4 * g + j;
+                const float x = vp[(size_t)min(key, kend - 1) * a.ldv];
+                v[j] = key < kend ? x : 0.0f;
+            }
+            const f4 p = *reinterpret_cast<const f4 *>(sc + r16 * ld + kb * 16 + 4 * g);
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(v[j], p[j], acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) zrow[c * 16 + e] = acc[e] * inv;
+    }
 }
 
 template <int OP>
@@ -375,22 +391,30 @@ int et_mha_fused_f32(const float *Q, const float *K, const float *V, int ldq, in
     const int width = nh * hd;
     ET_REQUIRE(ldq >= width && ldk >= width && ldv >= width && ldz >= width, ET_ERR_INVALID_ARG,
                "et_mha_fused_f32: row strides must cover nh*hd=%d", width);
-    const int hdt = hd <= 32 ? 32 : hd <= 64 ? 64 : 128;  // kernel template size
+    // (as large as with K and V staged in blocks of 64 rows, the form of the kernel that set the limit)
+    const int hdt = hd <= 32 ? 32 : hd <= 64 ? 64 : 128;
     const size_t lds = sizeof(float) * ((size_t)kAttQ * hdt + (size_t)kAttKeys * (hdt + 1) + (size_t)kAttQ * S);
     ET_REQUIRE(lds <= 160 * 1024, ET_ERR_UNSUPPORTED, "et_mha_fused_f32: S=%d does not fit the on-chip score strip", S);
     if (B == 0) return ET_OK;
     MhaF32Args a{Q, K, V, Z, mask, lens, ldq, ldk, ldv, ldz, B, S, nh, hd, scale, (flags & ET_MHA_CAUSAL) ? 1 : 0};
     const dim3 grid(S / kAttQ, nh, B);
+    const size_t strip = sizeof(float) * kAttQ * (size_t)(S + kAttPad);  // (less than the limit above is for)
     hipStream_t st = as_stream(stream);
-#define ET_MHA32(HD)                                                                                         \
+#define ET_MHA32(MAXC, VEC)                                                                                  \
     {                                                                                                        \
-        auto kern = mha_fused_f32_kernel<HD>;                                                                \
-        if (lds > 64 * 1024)                                                                                 \
+        auto kern = mha_fused_f32_kernel<MAXC, VEC>;                                                         \
+        if (strip > 64 * 1024)                                                                               \
             ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),                                 \
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));               \
-        kern<<<grid, 256, lds, st>>>(a);                                                                     \
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)strip));             \
+        kern<<<grid, 256, strip, st>>>(a);                                                                   \
     }
-    if (hdt == 32) ET_MHA32(32) else if (hdt == 64) ET_MHA32(64) else ET_MHA32(128)
+    // 16-byte loads of Q and K where every row starts at a multiple of 16 bytes
+    const bool vec = aligned16(Q) && aligned16(K) && ldq % 4 == 0 && ldk % 4 == 0;
+    if (hd <= 64) {
+        if (vec) ET_MHA32(4, true) else ET_MHA32(4, false)
+    } else {
+        if (vec) ET_MHA32(8, true) else ET_MHA32(8, false)
+    }
 #undef ET_MHA32
     return check_launch("mha_fused_f32_kernel");
 }

@@ -9,6 +9,8 @@
 // B[k_q][r].  A sum over k does not care which k a lane brings as long as A and B bring the
 // same one, so lane q holds k = 4q .. 4q+3 of a 16-wide cell (one 16-byte load per operand)
 // and the cell takes four instructions, the j-th contracting k = {j, 4+j, 8+j, 12+j}.
+#include <algorithm>
+
 #include "common.hip.h"
 
 namespace et {
@@ -40,39 +42,104 @@ __device__ __forceinline__ void store_cell_f32(float *Y, const float *bias, f4 a
 }
 
 // ---- 16x16 tiles ----------------------------------------------------------------
-// A wave owns one block-row (16 output features) and MT blocks of 16 tokens; the four
-// waves of a workgroup take four neighbouring block-rows over the same tokens, so the rows
-// of X they read are shared through the cache.  Tile t of the block-row: A = its 16 x 16
-// weights (row = feature), B = X[tokens][16 col_idx[t] ..].
-template <int MT>
-__global__ __launch_bounds__(256) void bsr16_linear_f32_kernel(const Bsr32Args a) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// Tile t of a block-row: A = its 16 x 16 weights (row = feature), B = X[16 tokens][16 col_idx[t] ..], four products of 32
+// cycles.  A verification batch has few (block-row, 16 tokens) pairs with a chain of loads and products each, so what
+// bounds it is the length of that chain; with many pairs it is the reads of X (below).  Two forms: one, for many pairs, with
+// the tokens' rows in LDS; one that reads them from memory.  Against the former kernel (a wave per block-row and 32 or
+// 64 tokens, nothing requested ahead), us, at 80 %: 256 tokens 768 -> 2304 10.7 -> 8.3, 768 -> 3072 11.6 -> 8.7, 3072 -> 768
+// 21.5 -> 8.3; 16 tokens 6.2 -> 4.0 and 14.7 -> 4.8; 4096 tokens 95 -> 69 and 129 -> 105.
+//
+// The waves of a workgroup share one (block-row, 16 tokens), each every WAVES-th tile; the sums meet in LDS and are added
+// in the order of the waves.  A lane reads the column index of one of its wave's tiles, 64 at a time, so no operand waits
+// for an index from memory, and kAhead tiles are requested ahead of the products.
+constexpr int kAhead = 4;
+template <int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void bsr16_linear_split_f32_kernel(const Bsr32Args a) {
+    __shared__ f4 part[WAVES][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, q = lane >> 4;
-    const int br = blockIdx.x * 4 + wave;
-    if (br >= (a.out >> 4)) return;  // no workgroup barrier below
-    const int tok0 = blockIdx.y * (MT * 16);
-    const float *xrow[MT];
+    const int strip = blockIdx.y + blockIdx.z * gridDim.y;
+    if (strip * 16 >= a.T) return;  // padding of the grid (whole workgroup)
+    const int br = blockIdx.x, tok = strip * 16 + r16;
+    const float *xp = a.X + (size_t)min(tok, a.T - 1) * a.in + 4 * q;  // rows past the end: the last one, not stored
+    const float *wp = a.tiles + r16 * 16 + 4 * q;
+    f4 acc = f4{0.f, 0.f, 0.f, 0.f};
+    const int ts = a.row_ptr[br] + wave, te = a.row_ptr[br + 1];
+    const int n = ts < te ? (te - ts + WAVES - 1) / WAVES : 0;  // tiles of this wave
+    for (int base = 0; base < n; base += 64) {
+        const int here = min(n - base, 64), t0 = ts + base * WAVES;
+        const int cols = a.col_idx[t0 + min(lane, here - 1) * WAVES];
+        float4 w[kAhead], x[kAhead];
+        auto ask = [&](int slot, int i) {  // (past the last: the last again, not multiplied)
+            i = min(i, here - 1);
+            w[slot] = *reinterpret_cast<const float4 *>(wp + (size_t)(t0 + i * WAVES) * 256);
+            x[slot] = *reinterpret_cast<const float4 *>(xp + __builtin_amdgcn_readlane(cols, i) * 16);
+        };
 #pragma unroll
-    for (int m = 0; m < MT; m++) {
-        const int tok = tok0 + m * 16 + r16;
-        xrow[m] = a.X + (size_t)(tok < a.T ? tok : a.T - 1) * a.in + 4 * q;  // rows past the end: clamped, not stored
+        for (int s = 0; s < kAhead; s++) ask(s, s);
+        for (int i = 0; i < here; i += kAhead) {
+#pragma unroll
+            for (int s = 0; s < kAhead; s++) {
+                if (i + s < here) acc = mfma_cell_f32(w[s], x[s], acc);  // uniform
+                ask(s, i + s + kAhead);
+            }
+        }
     }
-    f4 acc[MT];
+    if constexpr (WAVES > 1) {
+        part[wave][lane] = acc;
+        __syncthreads();
+        if (wave) return;
 #pragma unroll
-    for (int m = 0; m < MT; m++) acc[m] = f4{0.f, 0.f, 0.f, 0.f};
-    const int ts = a.row_ptr[br], te = a.row_ptr[br + 1];
-    const float *wp = a.tiles + (size_t)ts * 256 + r16 * 16 + 4 * q;
-#pragma unroll 2
-    for (int t = ts; t < te; t++, wp += 256) {
-        const int c = a.col_idx[t];
-        const float4 w = *reinterpret_cast<const float4 *>(wp);
-#pragma unroll
-        for (int m = 0; m < MT; m++)
-            acc[m] = mfma_cell_f32(w, *reinterpret_cast<const float4 *>(xrow[m] + c * 16), acc[m]);
+        for (int v = 1; v < WAVES; v++) acc += part[v][lane];
     }
+    store_cell_f32(a.Y, a.bias, acc, tok, a.T, a.out, br * 16 + 4 * q, a.act);
+}
+
+// Eight waves, eight neighbouring block-rows, 16 tokens, whose rows of X lie in LDS (kStripPad floats between two rows:
+// the 16 cells of a fragment read lie in different banks).  Read from memory, the fragment of a tile is 16 rows x 64 bytes,
+// and 16 neighbouring lanes touch 16 lines: with many tiles that is what the kernel above waits for.  The first
+// weights travel while the strip is staged.
+constexpr int kStripPad = 4, kStripWaves = 8;
+__global__ __launch_bounds__(kStripWaves * 64) void bsr16_linear_strip_f32_kernel(const Bsr32Args a) {
+    extern __shared__ __align__(16) unsigned char strip_smem[];
+    float *xs = reinterpret_cast<float *>(strip_smem);  // [16][in + kStripPad]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, q = lane >> 4;
+    const int strip = blockIdx.y + blockIdx.z * gridDim.y;
+    if (strip * 16 >= a.T) return;  // padding of the grid (whole workgroup)
+    const int ld = a.in + kStripPad, tok0 = strip * 16, quads = a.in >> 2;
+    for (int row = wave; row < 16; row += kStripWaves) {  // past the end: the last row, not stored
+        const float *src = a.X + (size_t)min(tok0 + row, a.T - 1) * a.in;
+        for (int i = lane; i < quads; i += 64)
+            *reinterpret_cast<float4 *>(xs + row * ld + i * 4) = *reinterpret_cast<const float4 *>(src + i * 4);
+    }
+    const int br = blockIdx.x * kStripWaves + wave;
+    const bool mine = br < (a.out >> 4);  // uniform
+    const int ts = mine ? a.row_ptr[br] : 0, n = mine ? a.row_ptr[br + 1] - ts : 0;
+    const float *xp = xs + r16 * ld + 4 * q;
+    const float *wp = a.tiles + r16 * 16 + 4 * q;
+    f4 acc = f4{0.f, 0.f, 0.f, 0.f};
+    if (n == 0) __syncthreads();
+    for (int base = 0; base < n; base += 64) {
+        const int here = min(n - base, 64), t0 = ts + base;
+        const int cols = a.col_idx[t0 + min(lane, here - 1)];
+        float4 w[kAhead];
+        auto ask = [&](int slot, int i) {  // (past the last: the last again, not multiplied)
+            w[slot] = *reinterpret_cast<const float4 *>(wp + (size_t)(t0 + min(i, here - 1)) * 256);
+        };
 #pragma unroll
-    for (int m = 0; m < MT; m++)
-        store_cell_f32(a.Y, a.bias, acc[m], tok0 + m * 16 + r16, a.T, a.out, br * 16 + 4 * q, a.act);
+        for (int s = 0; s < kAhead; s++) ask(s, s);
+        if (base == 0) __syncthreads();  // the strip is complete (every wave passes one barrier, here or above)
+        for (int i = 0; i < here; i += kAhead) {
+#pragma unroll
+            for (int s = 0; s < kAhead; s++) {
+                if (i + s < here)  // uniform
+                    acc = mfma_cell_f32(w[s], *reinterpret_cast<const float4 *>(xp + __builtin_amdgcn_readlane(cols, i + s) * 16), acc);
+                ask(s, i + s + kAhead);
+            }
+        }
+    }
+    if (mine) store_cell_f32(a.Y, a.bias, acc, tok0 + r16, a.T, a.out, br * 16 + 4 * q, a.act);
 }
 
 // ---- 1x16 vectors ---------------------------------------------------------------
@@ -200,13 +267,27 @@ int et_linear_bsr16_f32(const int32_t *row_ptr, const int32_t *col_idx, const fl
                "et_linear_bsr16_f32: tiles, X and Y must be 16-byte aligned");
     if (T == 0) return ET_OK;
     const Bsr32Args a{row_ptr, col_idx, tiles, bias, X, Y, T, in, out, act};
-    const int mt = token_blocks(T);
-    const dim3 grid((out / 16 + 3) / 4, (T + 16 * mt - 1) / (16 * mt));
     hipStream_t st = as_stream(stream);
-    if (mt == 4) bsr16_linear_f32_kernel<4><<<grid, 256, 0, st>>>(a);
-    else if (mt == 2) bsr16_linear_f32_kernel<2><<<grid, 256, 0, st>>>(a);
-    else bsr16_linear_f32_kernel<1><<<grid, 256, 0, st>>>(a);
-    return check_launch("bsr16_linear_f32_kernel");
+    const int strips = (T + 15) / 16;
+    const int gy = std::min(strips, 32768);
+    const long long pairs = (long long)(out / 16) * strips;
+    const size_t lds = (size_t)16 * (in + kStripPad) * sizeof(float);
+    // The strip form where two workgroups fit a compute unit and there are six pairs or more for each: 80 %, us, strip
+    // against not: 2304 pairs of 768 values 8.2 / 8.8, 3072 8.7 / 11.5, 1536 6.2 / 6.6, 768 6.1 / 4.6.
+    if (pairs >= 1536 && lds <= 80 * 1024) {
+        if (lds > 64 * 1024)
+            ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(bsr16_linear_strip_f32_kernel),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        const dim3 grid((out / 16 + kStripWaves - 1) / kStripWaves, gy, (strips + gy - 1) / gy);
+        bsr16_linear_strip_f32_kernel<<<grid, kStripWaves * 64, lds, st>>>(a);
+        return check_launch("bsr16_linear_strip_f32_kernel");
+    }
+    // Two waves a pair below two pairs a compute unit: 192 pairs of 38 tiles 5.2 us against 7.3, 576 pairs of 10 tiles 4.9
+    // against 4.7; four waves are no faster.
+    const dim3 grid(out / 16, gy, (strips + gy - 1) / gy);
+    if (pairs < 512) bsr16_linear_split_f32_kernel<2><<<grid, 128, 0, st>>>(a);
+    else bsr16_linear_split_f32_kernel<1><<<grid, 64, 0, st>>>(a);
+    return check_launch("bsr16_linear_split_f32_kernel");
 }
 
 int et_linear_vec1x16_f32(const int32_t *tile_idx, const int32_t *row_idx, const float *data, const float *bias,

@@ -68,6 +68,29 @@ def test_mha_fused_f32(et, B, S, nh, hd, causal, lens, mask):
     assert Hn.max_abs(d_z.numpy(), want.numpy()) <= 1e-5
 
 
+@pytest.mark.parametrize("B,S,nh,hd,shift,causal,lens", [
+    (2, 64, 2, 64, 1, False, [64, 17]), (2, 32, 3, 80, 0, True, [32, 1]), (1, 80, 2, 112, 3, False, [79]), (2, 16, 5, 16, 2, False, [16, 0])])
+def test_mha_fused_f32_strides_and_rows_past_the_length(et, B, S, nh, hd, shift, causal, lens):
+    """Operands `shift` floats past a 16-byte boundary in rows of 3 H + shift floats; K and V past a sequence's length hold
+    NaN, which no result may show.  Sums of hd and S products of values near 1: 1e-5, as above."""
+    H = nh * hd
+    ld = 3 * H + shift
+    rows = randf((B * S, 3 * H), 16)
+    given = rows.copy()
+    for b in range(B):
+        given[b * S + lens[b]:(b + 1) * S, H:] = np.nan
+    flat = np.zeros(shift + B * S * ld, np.float32)
+    flat[shift:].reshape(B * S, ld)[:, :3 * H] = given
+    d = up(et, flat)
+    d_z = et.DeviceBuffer.empty((B * S, H), np.float32)
+    d_l = up(et, np.asarray(lens, np.int32))
+    et.check(et.lib().et_mha_fused_f32(d.offset(4 * shift), d.offset(4 * (shift + H)), d.offset(4 * (shift + 2 * H)), ld, ld, ld,
+                                       d_z.ptr, H, None, d_l.ptr, B, S, nh, hd, hd ** -0.5, et.MHA_CAUSAL if causal else 0, None))
+    t = torch.from_numpy(rows)
+    want = L.mha(t[:, :H], t[:, H:2 * H], t[:, 2 * H:], nh, B, lens=lens, causal=causal)
+    assert Hn.max_abs(d_z.numpy(), want.numpy()) <= 1e-5
+
+
 @pytest.mark.parametrize("rows,H", [(128, 768), (33, 1024), (5, 4100), (7, 64)])
 def test_layernorm_f32(et, rows, H):
     src, skip = randf((rows, H), 8, 2.0), randf((rows, H), 9)
@@ -182,6 +205,16 @@ def test_linear_bsr16_f32(et, T, inp, out, sp, act):
     et.check(et.lib().et_linear_bsr16_f32(up(et, row_ptr).ptr, up(et, ci).ptr, up(et, tiles).ptr, up(et, b).ptr,
                                           up(et, x).ptr, d_y.ptr, T, inp, out, act, None))
     assert Hn.max_abs(d_y.numpy(), _want64(x, Wd, b, act)) <= 5e-5
+
+
+# Both sides of the rule that divides the work: block-rows x 16-token strips below 512, from there to 1536, and above
+# (rows of X in LDS), widths at and past what LDS holds there, rows of more than 64 tiles a wave, block-rows that do not
+# fill the last workgroup, tokens that do not fill the last strip.
+@pytest.mark.parametrize("T,inp,out,sp,act", [(16, 3072, 768, 0.0, 0), (17, 64, 16 * 255, 0.7, 1), (256, 16, 512, 0.0, 2),
+                                              (500, 3072, 96, 0.2, 0), (2001, 1264, 208, 0.8, 2), (2000, 1280, 208, 0.8, 0),
+                                              (1536, 1040, 272, 0.0, 1), (33, 128, 16 * 800, 0.99, 0)])
+def test_linear_bsr16_f32_division_of_the_work(et, T, inp, out, sp, act):
+    test_linear_bsr16_f32(et, T, inp, out, sp, act)
 
 
 def test_linear_bsr16_f32_closed_form_and_bad_args(et):
