@@ -155,6 +155,259 @@ static int launch_mha_nw(const MhaArgs &args, hipStream_t stream) {
     return check_launch("mha_fused_kernel");
 }
 
+// ---- two groups of waves in turn ------------------------------------------------------------------------
+// Eight waves of two query tiles take all registers of a compute unit, so no second workgroup is there to fill the matrix
+// cores while this one forms its exponentials, and with the waves of a workgroup at the same place of a block the two
+// kinds of work never meet.  Here waves 4-7 (the second wave of every SIMD) run one phase behind waves 0-3.
+// A block of 128 keys is two phases, each ended by a workgroup barrier:
+//   products: O^T += V^T P^T of the block before, then this block's scores (64 MFMAs, 1024 cycles)
+//   softmax:  scores -> probabilities, and the wave's share of the staging
+// so at any time one wave of a SIMD issues matrix and the other vector instructions.  K and V^T have two buffers each; with
+// half-steps counted from the first group's first products, the first group has products of block j in 2j and softmax in
+// 2j + 1, the second one half-step later:
+//   K of block j is read in 2j and 2j + 1, V^T of block j (by the products of j + 1) in 2j + 2 and 2j + 3;
+//   the second group writes K of block j + 2 in 2j + 2: behind the last reads of block j, before 2j + 4;
+//   the first group writes V^T of block j in 2j + 1: behind the last reads of block j - 2, in 2j - 1, before 2j + 2.
+// Both groups pass the same number of barriers: the second one more in front, the first one more at the end.
+// 16 x 16 heads of 64, 2048 keys: 440 -> 393 us against the form whose waves run together on the same card, causal
+// 344 -> 276.  A block takes 6200 cycles; the vector unit is busy for 3700 of them and the matrix cores for 2050.  With one
+// barrier a block and no phases 414, with the groups' waves on the same SIMD 459; row sums by an MFMA against ones, or a
+// priority for either phase: 1-3 % slower.
+// For S a multiple of 256, no additive mask and a positive scale; padded keys and the causal mask are applied to the
+// blocks they cut, and a wave skips the blocks past its last query.
+constexpr int kPpQ = 256;  // queries of a workgroup
+__global__ __launch_bounds__(512) void mha_pingpong_kernel(const MhaArgs a) {
+    constexpr int HD = 64, KS = 2, DB = 4, QT = 2;
+    using L = MhaLds<HD>;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    _Float16 *const Kb = reinterpret_cast<_Float16 *>(smem_raw);  // [2][128][ldk]
+    _Float16 *const Vb = Kb + 2 * L::k_halfs;                     // [2][64][ldvt]
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool second = wave >= 4;
+    const int r16 = lane & 15, g = lane >> 4;
+    const int S = a.S, hd = a.hd;
+    // as in the kernel above: the query strips of a (sequence, head) on one XCD
+    const int qstrips = S / kPpQ;
+    const int xcd = blockIdx.x % kXcds, k_in_xcd = blockIdx.x / kXcds;
+    const int bh = xcd + kXcds * (k_in_xcd / qstrips);
+    if (bh >= a.nbh) return;  // padding of the last round (whole workgroup)
+    const int qstrip = k_in_xcd % qstrips;
+    const int b = bh / a.nh, h = bh - b * a.nh;
+    const size_t row0 = (size_t)b * S;
+    const int wave_q = qstrip * kPpQ + wave * QT * 16;  // first query of the wave
+    int klimit = S;
+    if (a.lens) klimit = min(S, max(a.lens[b], 0));
+    if (a.causal) klimit = min(klimit, (qstrip + 1) * kPpQ);
+    const int nblocks = (klimit + kKeyBlock - 1) / kKeyBlock;  // (of 128 whole rows each: S is a multiple of 256)
+
+    h8 qf[QT][KS];
+#pragma unroll
+    for (int t = 0; t < QT; t++)
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            const bool in = 32 * ks + 8 * g < hd;  // columns past the head size: zero
+            qf[t][ks] = *reinterpret_cast<const h8 *>(a.Q + (row0 + wave_q + t * 16 + r16) * a.ldq + h * hd + (in ? 32 * ks + 8 * g : 0));
+            if (!in) qf[t][ks] = h8{0, 0, 0, 0, 0, 0, 0, 0};
+        }
+    f4 o[QT][DB];
+    float m_run[QT], l_part[QT];
+#pragma unroll
+    for (int t = 0; t < QT; t++) {
+#pragma unroll
+        for (int d = 0; d < DB; d++) o[t][d] = f4{0.f, 0.f, 0.f, 0.f};
+        m_run[t] = -INFINITY;
+        l_part[t] = 0.0f;
+    }
+
+    // staging: a thread of the first group holds 4 keys x 8 dimensions of V, one of the second 8 dimensions of 4 keys of K
+    const int u = threadIdx.x & 255, dg = u & 7;
+    const int key_v = vt_unit_keys<HD>(u >> 3) * 4, key_k = u >> 3;
+    const int ld = second ? a.ldk : a.ldv;
+    const bool col_in = dg * 8 < hd;
+    const _Float16 *const src = (second ? a.K : a.V) + (row0 + (second ? key_k : key_v)) * ld + h * hd + (col_in ? dg * 8 : 0);
+    const size_t step = (size_t)ld * (second ? 32 : 1);
+    h8 st[4];
+    auto load = [&](int blk) {  // (past the last block: the last again, not read)
+        const _Float16 *p = src + (size_t)(min(blk, nblocks - 1) * kKeyBlock) * ld;
+#pragma unroll
+        for (int i = 0; i < 4; i++) st[i] = *reinterpret_cast<const h8 *>(p + i * step);
+    };
+    const int v_pos = [&] {
+        const int kg = key_v >> 2;
+        return (32 * (kg >> 3) + 8 * (kg & 3) + 4 * ((kg >> 2) & 1)) ^ vt_swizzle<HD>(dg >> 1);
+    }();
+    auto store = [&](int buf) {
+        const h8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+        if (!col_in)
+#pragma unroll
+            for (int i = 0; i < 4; i++) st[i] = zero8;
+        if (second) {
+            _Float16 *kp = Kb + buf * L::k_halfs + key_k * L::ldk + dg * 8;
+#pragma unroll
+            for (int i = 0; i < 4; i++) *reinterpret_cast<h8 *>(kp + i * 32 * L::ldk) = st[i];
+        } else {
+            _Float16 *vp = Vb + buf * L::vt_halfs + dg * 8 * L::ldvt + v_pos;
+#pragma unroll
+            for (int d = 0; d < 8; d++) *reinterpret_cast<h4 *>(vp + d * L::ldvt) = h4{st[0][d], st[1][d], st[2][d], st[3][d]};
+        }
+    };
+    // the end of a phase: LDS accesses are complete, requests to memory stay in flight
+    auto phase_end = [] {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    f4 sc[QT][kNKB];
+    h8 pf[QT][kNKB / 2];
+    // The products of a phase: O^T += V^T P^T of the block in V^T buffer vbuf (WEIGHTED), the scores against K buffer kbuf
+    // (SCORES).  An operand fragment read from LDS feeds two MFMAs (32 cycles), and is read kRing fragments ahead of them, in
+    // an order that is fixed here: left to the compiler, which needs few registers that way, every pair of fragments is
+    // waited for as it is read.
+    constexpr int kRing = 6, kFragV = kNKB / 2 * DB, kFragK = kNKB * KS;
+    auto products = [&](auto weighted_tag, auto scores_tag, int vbuf, int kbuf) {
+        constexpr bool WEIGHTED = decltype(weighted_tag)::value, SCORES = decltype(scores_tag)::value;
+        constexpr int first = WEIGHTED ? 0 : kFragV, last = SCORES ? kFragV + kFragK : kFragV;
+        const _Float16 *vt = Vb + vbuf * L::vt_halfs + r16 * L::ldvt;
+        const _Float16 *vt8 = vt + 8 * g, *vt8x = vt + ((8 * g) ^ 16);
+        const _Float16 *kp = Kb + kbuf * L::k_halfs + r16 * L::ldk + 8 * g;
+        h8 ring[kRing];
+        // fragments of K in the order (kb, 0), (kb + 1, 0), (kb, 1), (kb + 1, 1): four MFMAs between two of one sum
+        auto key_block = [](int k) { return k / 4 * 2 + (k & 1); };
+        auto read = [&](int i) {
+            if (i < kFragV) {
+                const int s2 = i / DB, d = i % DB, swz = vt_swizzle<HD>(d);
+                ring[i % kRing] = *reinterpret_cast<const h8 *>(((swz & 16) ? vt8x : vt8) + d * 16 * L::ldvt + ((s2 * 32) ^ (swz & 32)));
+            } else {
+                const int k = i - kFragV;
+                ring[i % kRing] = *reinterpret_cast<const h8 *>(kp + key_block(k) * 16 * L::ldk + 32 * (k >> 1 & 1));
+            }
+        };
+#pragma unroll
+        for (int i = first; i < first + kRing; i++) read(i);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = first; i < last; i++) {
+#pragma unroll
+            for (int t = 0; t < QT; t++) {
+                if (i < kFragV) {
+                    o[t][i % DB] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ring[i % kRing], pf[t][i / DB], o[t][i % DB], 0, 0, 0);
+                } else {
+                    const int k = i - kFragV, kb = key_block(k), ks = k >> 1 & 1;
+                    const f4 zero = {0.f, 0.f, 0.f, 0.f};
+                    sc[t][kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ring[i % kRing], qf[t][ks], ks ? sc[t][kb] : zero, 0, 0, 0);
+                }
+            }
+            if (i + kRing < last) read(i + kRing);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto softmax = [&](int k0) {
+        // keys past the limit or past the query: 16 kb + j >= lim (the left side a constant once unrolled)
+        if (k0 + kKeyBlock > klimit || (a.causal && k0 + kKeyBlock > wave_q + 1)) {  // wave-uniform
+#pragma unroll
+            for (int t = 0; t < QT; t++) {
+                int lim = klimit - k0;
+                if (a.causal) lim = min(lim, wave_q + t * 16 + r16 + 1 - k0);
+                lim -= 4 * g;
+#pragma unroll
+                for (int kb = 0; kb < kNKB; kb++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) sc[t][kb][j] = (kb * 16 + j >= lim) ? -INFINITY : sc[t][kb][j];
+            }
+        }
+        const h2 ones = {(_Float16)1.0f, (_Float16)1.0f};
+#pragma unroll
+        for (int t = 0; t < QT; t++) {
+            float m_blk = -INFINITY;
+#pragma unroll
+            for (int kb = 0; kb < kNKB; kb++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) m_blk = fmaxf(m_blk, sc[t][kb][j]);
+            m_blk = rows_max(m_blk * a.scale_log2e);
+            const float m_new = fmaxf(m_run[t], m_blk);
+            const float m_use = (m_new == -INFINITY) ? 0.0f : m_new;  // all keys so far masked
+            const float alpha = __builtin_amdgcn_exp2f(m_run[t] - m_use);
+            m_run[t] = m_new;
+            if (!__all(alpha == 1.0f)) {
+                l_part[t] *= alpha;
+#pragma unroll
+                for (int d = 0; d < DB; d++) o[t][d] *= alpha;
+            }
+#pragma unroll
+            for (int s2 = 0; s2 < kNKB / 2; s2++)
+#pragma unroll
+                for (int pr = 0; pr < 4; pr++) {
+                    const int kb = 2 * s2 + (pr >> 1), j = 2 * (pr & 1);
+                    const float e0 = sc[t][kb][j] * a.scale_log2e - m_use, e1 = sc[t][kb][j + 1] * a.scale_log2e - m_use;
+                    const h2 hp = {(_Float16)__builtin_amdgcn_exp2f(e0), (_Float16)__builtin_amdgcn_exp2f(e1)};
+                    l_part[t] = __builtin_amdgcn_fdot2(hp, ones, l_part[t], false);
+                    pf[t][s2][2 * pr] = hp[0];
+                    pf[t][s2][2 * pr + 1] = hp[1];
+                }
+        }
+    };
+    // (a block whose keys all lie past the wave's last query has no part in its result)
+    auto live = [&](int blk) { return !a.causal || blk * kKeyBlock < wave_q + QT * 16; };
+
+    if (nblocks > 0) {  // uniform over the workgroup
+        load(0);
+        if (second) {
+            store(0);
+            load(1);
+        }
+        phase_end();
+        if (second) {
+            store(1);
+            load(2);
+            phase_end();
+        }
+        for (int j = 0; j < nblocks; j++) {
+            // (a block past the wave's last query has none before it that is not: the wave's blocks end together)
+            if (live(j)) {
+                if (j > 0) products(std::true_type{}, std::true_type{}, (j - 1) & 1, j & 1);
+                else products(std::false_type{}, std::true_type{}, 0, 0);
+            } else if (live(j - 1)) {
+                products(std::true_type{}, std::false_type{}, (j - 1) & 1, 0);
+            }
+            phase_end();
+            store(j & 1);  // V of block j, or K of block j + 2
+            load(second ? j + 3 : j + 1);
+            if (live(j)) softmax(j * kKeyBlock);
+            phase_end();
+        }
+        if (live(nblocks - 1)) products(std::true_type{}, std::false_type{}, (nblocks - 1) & 1, 0);
+        if (!second) phase_end();
+    }
+
+#pragma unroll
+    for (int t = 0; t < QT; t++) {
+        const float l = rows_sum(l_part[t]);
+        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        _Float16 *zp = a.Z + (row0 + wave_q + t * 16 + r16) * a.ldz + h * hd + 4 * g;
+#pragma unroll
+        for (int d = 0; d < DB; d++) {
+            h4 out;
+#pragma unroll
+            for (int j = 0; j < 4; j++) out[j] = (_Float16)(o[t][d][j] * inv);
+            if (16 * d + 4 * g < hd) *reinterpret_cast<h4 *>(zp + 16 * d) = out;  // (a head size of 8 k may end inside a block)
+        }
+    }
+}
+
+static int launch_mha_pingpong(const MhaArgs &args, hipStream_t stream) {
+    constexpr size_t lds = 2 * MhaLds<64>::bytes;
+    static bool raised = false;
+    if (!raised) {
+        ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(mha_pingpong_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        raised = true;
+    }
+    const int qstrips = args.S / kPpQ, rounds = (args.nbh + kXcds - 1) / kXcds;
+    mha_pingpong_kernel<<<dim3((unsigned)(rounds * kXcds * qstrips)), 512, lds, stream>>>(args);
+    return check_launch("mha_pingpong_kernel");
+}
+
 // 4 waves per workgroup and one 16-query tile per wave; 2 or 1 waves when 4 would leave a
 // half-empty strip (S = 32, 96, 16, ...).  Larger workgroups stage each key block for more
 // queries and pay once the grid still fills the chip: 8 waves (128 queries) from 256 such
@@ -169,6 +422,12 @@ static int launch_mha(const MhaArgs &args, int B, hipStream_t stream) {
     (void)B;
     const int qblocks = args.S / 16;
     if constexpr (!COMPACT) {
+        // The two groups of waves in turn: 256-query strips like the next form, but from 192 of them on (2 x 16 heads, 2048
+        // keys, 256 strips: 58.7 -> 45.2 us; 4 x 12 heads, 1024 keys, 192: 30.3 -> 24.0; with 128 strips 35 -> 41) and from
+        // 512 keys on (512 strips of 512 keys 32.4 either way, of 256 keys 32.3 -> 34): a sequence of one or two blocks
+        // has nothing to take turns with.
+        if (HD == 64 && qblocks % 16 == 0 && args.S >= 512 && (long)args.nbh * (qblocks / 16) >= 192 && !args.mask && args.scale_log2e > 0.0f)
+            return launch_mha_pingpong(args, stream);
         if (HD == 64 && qblocks % 16 == 0 && (long)args.nbh * (qblocks / 16) >= 512)
             return launch_mha_nw<(HD == 64 ? HD : 64), COMPACT, 8, 2>(args, stream);
         if (HD == 128 && qblocks % 16 == 0 && (long)args.nbh * (qblocks / 16) >= 512)

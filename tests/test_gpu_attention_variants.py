@@ -259,3 +259,30 @@ def test_compact_v_attention_random_shapes(et, B, S, nh, hd, keep, causal, seed)
     assert Hn.max_abs(got, want) <= 2e-3
     dead = np.setdiff1d(np.arange(H), col_id)
     assert np.all(got[:, dead] == 0)
+
+
+# The form of the fused attention whose two groups of waves take turns (256-query strips of 64-wide heads, 192 of them
+# or more and 512 keys or more, no additive mask; the first two cases are below): two to sixteen key blocks, lengths that end on a block, inside one and at nothing, causal
+# strips whose first waves skip the last blocks, head sizes that fill 64 columns and that do not, Q, K and V as one matrix
+# and as three.  Probabilities and Z are binary16: 4e-3, as for the other forms.
+@pytest.mark.parametrize("B,S,nh,hd,causal,lens,scale", [
+    (8, 256, 64, 64, False, None, 1), (1, 512, 95, 64, True, [511], 1),
+    (8, 512, 24, 64, True, [512, 1, 128, 129, 0, 255, 127, 17], 1), (2, 512, 48, 64, True, None, 3), (1, 512, 96, 56, False, [385], 1), (3, 768, 57, 40, False, [768, 129, 640], 1), (3, 768, 57, 48, True, [300, 768, 0], 1),
+    (1, 2048, 64, 64, False, [1999], 30)])
+def test_mha_fused_waves_in_turn(et, B, S, nh, hd, causal, lens, scale):
+    H, T = nh * hd, B * S
+    one = hd == 64
+    qkv = Hn.randn((T, 3 * H), 91)
+    d_l = up(et, np.array(lens, np.int32)) if lens is not None else None
+    d_z = et.DeviceBuffer.empty((T, H), np.float16)
+    if one:
+        d = up(et, qkv)
+        ptrs, ld = (d.ptr, d.offset(2 * H), d.offset(4 * H)), 3 * H
+    else:
+        keep = [up(et, np.ascontiguousarray(qkv[:, i * H:(i + 1) * H])) for i in range(3)]
+        ptrs, ld = tuple(k.ptr for k in keep), H
+    et.mha_fused(*ptrs, ld, ld, ld, d_z.ptr, H, None, None if d_l is None else d_l.ptr, B, S, nh, hd, scale * hd ** -0.5,
+                 et.MHA_CAUSAL if causal else 0, None)
+    x = Hn.f32(qkv)
+    want = L.mha(x[:, :H] * scale, x[:, H:2 * H], x[:, 2 * H:], nh, B, lens=lens, causal=causal)
+    assert Hn.max_abs(d_z.numpy(), want.numpy()) <= 4e-3
