@@ -9,12 +9,12 @@ token embeddings that already sit in HBM (one HIP-graph replay through the C ABI
 in the engine's mixed-precision mode: fp16 matrix-core operands, fp32 accumulation,
 fp32 softmax, LayerNorm and residual stream.
 Prints ONE JSON line: sequences/s (value), ms per step, per-layer latency, the
-roofline of the dominant kernel — the launch with the largest share of the step's GPU time
-in the committed rocprofv3 kernel trace: the tile-sparse FFN up-projection, 3072 x 768 at
-80 %, which normalises the output projection's binary32 sum while it stages its token strip
-and applies GELU in its epilogue (timed with HIP events on its own stream over a HIP graph
-of such launches, each on another layer's weights and another set of buffers, so nothing
-is warm in a cache) — and the CPU oracle timed on the host cores.
+roofline of the dominant kernel — the one with the largest share of the step's GPU time
+in the committed rocprofv3 kernel trace: the token-local kernel, which takes a strip of token
+rows through the output projection, both LayerNorms, the FFN and the next QKV projection in
+two launches (timed with HIP events on its own stream over a HIP graph of such pairs, each on
+another layer's weights and another set of buffers, so nothing is warm in a cache) — and the
+CPU oracle timed on the host cores.
 """
 from __future__ import annotations
 
@@ -240,6 +240,74 @@ def time_dominant_kernel(et, layers, T, folded, rounds_per_graph=6, replays=8):
     return t.ms * 1e-3 / (rounds_per_graph * n * replays), name, what
 
 
+def time_token_local(et, layers, T, rounds_per_graph=6, replays=8):
+    """(seconds per layer, kernel names, description, flops, algorithmic bytes) of what the default stack runs between
+    two attention kernels at this workload's shape: et_encoder_layer_f32, divided as the engine divides 1024 token rows
+    (strips of 16 rows, four workgroups to a strip, hence two launches), timed as time_dominant_kernel does."""
+    import ctypes as C
+    lib = et.lib()
+
+    class Weights(C.Structure):
+        """et_layer_weights of include/et_abi.h"""
+        _fields_ = [(k, C.c_void_p * 4) for k in ("row_ptr", "col_idx", "tiles", "bias")] + [(k, C.c_void_p * 2) for k in ("gamma", "beta")]
+
+    PARTS = 4
+    stream = C.c_void_p()
+    et.check(lib.et_stream_create(C.byref(stream)))
+    rng = np.random.default_rng(0)
+    D = et.DeviceBuffer
+    n = len(layers)
+    packs, norms = [], []
+    for l in layers:
+        for w in (l.qkv, l.o, l.l1, l.l2):
+            w.upload(et)
+        norms.append([D.from_numpy(v) for v in (l.g1, l.be1, l.g2, l.be2)])
+    for i, l in enumerate(layers):
+        w = Weights()
+        for k, m in enumerate((l.o, l.l1, l.l2, layers[(i + 1) % n].qkv)):
+            w.row_ptr[k], w.col_idx[k], w.tiles[k], w.bias[k] = m.d_row_ptr.ptr, m.d_col_idx.ptr, m.d_tiles.ptr, m.d_bias.ptr
+        for k in range(2):
+            w.gamma[k], w.beta[k] = norms[i][2 * k].ptr, norms[i][2 * k + 1].ptr
+        h = C.c_void_p()
+        et.check(lib.et_encoder_layer_pack_create(C.byref(w), T, H, FF, 3 * H, 1, PARTS, C.byref(h)))
+        packs.append(h)
+    zs = [D.from_numpy(rng.standard_normal((T, H), dtype=np.float32).astype(np.float16)) for _ in layers]
+    xs = [D.from_numpy(rng.standard_normal((T, H), dtype=np.float32)) for _ in layers]
+    qkvs = [D.empty((T, 3 * H), np.float16) for _ in layers]
+    outs = [D.empty((T, H), np.float32) for _ in layers]
+    partial = D.empty((PARTS, T, H), np.float32)
+
+    def local(i):
+        et.check(lib.et_encoder_layer_f32(packs[i], zs[i].ptr, xs[i].ptr, None, outs[i].ptr, None, qkvs[i].ptr, partial.ptr,
+                                          et.ACT_GELU, 1e-5, 1e-5, stream))
+
+    for i in range(n):  # eager once: one-time kernel setup
+        local(i)
+    et.check(lib.et_stream_sync(stream))
+    et.check(lib.et_graph_begin_capture(stream))
+    for _ in range(rounds_per_graph):
+        for i in range(n):
+            local(i)
+    graph = C.c_void_p()
+    et.check(lib.et_graph_end_capture(stream, C.byref(graph)))
+    et.check(lib.et_graph_launch(graph, stream))  # warm
+    et.check(lib.et_stream_sync(stream))
+    with et.Timer(stream) as t:
+        for _ in range(replays):
+            et.check(lib.et_graph_launch(graph, stream))
+    et.check(lib.et_graph_destroy(graph))
+    et.check(lib.et_stream_sync(stream))
+    for h in packs:
+        et.check(lib.et_encoder_layer_pack_destroy(h))
+    et.check(lib.et_stream_destroy(stream))
+    tiles = sum(len(w.col_idx) for l in layers for w in (l.qkv, l.o, l.l1, l.l2)) / n
+    # Z and QKV' binary16, the residual stream binary32 in and out, tiles with their indices, biases and norms
+    nbytes = 2.0 * T * H + 8.0 * T * H + 6.0 * T * H + 516.0 * tiles + 2.0 * (9 * H + FF)
+    name = "void et::encoder_layer_kernel<1, 3, 1>(et::LayerArgs) + void et::encoder_layer_kernel<1, 3, 2>(et::LayerArgs)"
+    what = f"output projection, LayerNorms, FFN + GELU and next QKV projection of a layer @80%, T={T}, two launches"
+    return t.ms * 1e-3 / (rounds_per_graph * n * replays), name, what, 2.0 * 256 * tiles * T, nbytes
+
+
 def oracle_params(layers):
     import torch
     from oracle import formats as F
@@ -341,13 +409,21 @@ def main():
 
     sec = time_stack(et, model, d_out, d_in, args.steps, args.warmup)
 
-    # dominant kernel (largest share of the step in the committed kernel trace): the FFN up-projection,
-    # 3072x768 BSR at 80 %, T = 1024, + GELU; in the default stack it also normalises its input strip
+    # dominant kernel (largest share of the step in the committed kernel trace): the token-local kernel; in the other launch
+    # forms the FFN up-projection, 3072x768 BSR at 80 %, T = 1024, + GELU
     T = B * S
-    folded = not args.separate_ln
-    ntile = len(layers[0].l1.col_idx)  # the same count in every layer: int(9216 * (1 - 0.8))
-    flops = 2.0 * 256 * ntile * T  # algorithmic: 2 * 16*16 * surviving tiles * token rows
-    ksec, kname, kwhat = time_dominant_kernel(et, layers, T, folded)
+    if not (args.separate_ln or args.chain or args.five_launches):
+        ksec, kname, kwhat, flops, alg_bytes = time_token_local(et, layers, T)
+    else:
+        folded = not args.separate_ln
+        ntile = len(layers[0].l1.col_idx)  # the same count in every layer: int(9216 * (1 - 0.8))
+        flops = 2.0 * 256 * ntile * T  # algorithmic: 2 * 16*16 * surviving tiles * token rows
+        ksec, kname, kwhat = time_dominant_kernel(et, layers, T, folded)
+        # 2 T out (binary16 result) + 516 ntile + 4 (out/16 + 1) + 2 out + the input strip: 2 T in as binary16, or folded
+        # 4 T in (the binary32 sum) + 8 T groups (its row sums, 8 block-row groups) + 4 in (gamma, beta) + 8 T (row
+        # statistics written)
+        alg_bytes = 2.0 * T * FF + 516.0 * ntile + 4.0 * (FF // 16 + 1) + 2.0 * FF
+        alg_bytes += (4.0 * T * H + 8.0 * T * 8 + 4.0 * H + 8.0 * T) if folded else 2.0 * T * H
     achieved = flops / ksec / 1e12
     traffic, traffic_note = traffic_from_profile(kname)
     prof, prof_note = profile_line(STATS_PROFILE, kname)
@@ -361,12 +437,7 @@ def main():
                 "profile_source": prof_note,
                 "flop_per_launch": flops, "traffic": None if traffic is None else round(traffic),
                 "traffic_source": traffic_note}
-    # The same launch against the other roof: algorithmic bytes 2 T out (binary16 result) + 516 ntile +
-    # 4 (out/16 + 1) + 2 out + the input strip: 2 T in as binary16, or folded 4 T in (the binary32 sum) +
-    # 8 T groups (its row sums, 8 block-row groups) + 4 in (gamma, beta) + 8 T (row statistics written).
-    # At about 100 flop per byte the shape sits below the ridge of the machine (312 flop/B), i.e. on the HBM roof.
-    alg_bytes = 2.0 * T * FF + 516.0 * ntile + 4.0 * (FF // 16 + 1) + 2.0 * FF
-    alg_bytes += (4.0 * T * H + 8.0 * T * 8 + 4.0 * H + 8.0 * T) if folded else 2.0 * T * H
+    # the same against the other roof
     roofline["hbm_view"] = {"bound": "hbm", "achieved": round(alg_bytes / ksec / 1e9, 1), "peak": 8000.0, "unit": "GB/s",
                             "frac": round(alg_bytes / ksec / 8e12, 5), "bytes_per_launch": alg_bytes}
 
