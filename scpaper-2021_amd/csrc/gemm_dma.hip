@@ -533,7 +533,7 @@ static bool pick_dma_tile(const GemmArgs &g, int batch, bool trans_b, DmaTile *o
         // reads costs more than it saves elsewhere (Linear_VO 28 -> 78 us), those stay on the
         // register-staged kernel.
         if ((batch != 1 || !trans_b) && (w > 256 || g.K / kDmaK < 16)) return false;
-        *out = {1, 1, (w <= 512 && g.K / kDmaK >= 24) ? 3 : 2, true};  // third buffer: as below
+        *out = {1, 1, g.K / kDmaK < 24 || w > 512 ? 2 : w > 256 || !trans_b ? 3 : 4, true};  // third and fourth buffer: as below
         return true;
     }
     auto wgs = [&](int tmw, int tnw) -> long long {
@@ -548,7 +548,9 @@ static bool pick_dma_tile(const GemmArgs &g, int batch, bool trans_b, DmaTile *o
     // few workgroups with a long K loop are bound by the latency of a stage: a third buffer keeps
     // two stages in flight (2048 x 3072 -> 768: 29.5 -> 24.7 us; from 12 stages on it still gives
     // 3-5 %: 2048 x 768 -> 768 9.6 -> 9.1 us); elsewhere it only costs occupancy
-    *out = {1, 1, (w11 <= 512 && g.K / kDmaK >= 12) ? 3 : 2, false};
+    // With at most one workgroup a compute unit and 24 stages a fourth: 1024 x 3072 -> 768 16.3 -> 14.5, 512 x 4096 -> 1024 19.1
+    // -> 17.1, 208 x 3600 -> 3264 19.5 -> 18.4 (384 workgroups: 21.6 -> 22.0).
+    *out = {1, 1, (w11 <= 256 && g.K / kDmaK >= 24) ? 4 : (w11 <= 512 && g.K / kDmaK >= 12) ? 3 : 2, false};
     return true;
 }
 
@@ -611,8 +613,9 @@ int launch_gemm_dma(const GemmArgs &g, int batch, bool trans_b, hipStream_t stre
         if (t.tmw == 4) return launch_dma_tile<4, 4, 2, true>(g, batch, stream);
         if (t.tmw == 2) return t.tnw == 2 ? launch_dma_tile<2, 2, 2, true>(g, batch, stream)
                                           : launch_dma_tile<2, 1, 2, true>(g, batch, stream);
-        return t.nbuf == 3 ? launch_dma_tile<1, 1, 3, true>(g, batch, stream)
-                           : launch_dma_tile<1, 1, 2, true>(g, batch, stream);
+        return t.nbuf == 4   ? launch_dma_tile<1, 1, 4, true>(g, batch, stream)
+               : t.nbuf == 3 ? launch_dma_tile<1, 1, 3, true>(g, batch, stream)
+                             : launch_dma_tile<1, 1, 2, true>(g, batch, stream);
     }
     switch (t.tmw * 100 + t.tnw * 10 + t.nbuf) {
         // 256 x 256: eight waves of 128 x 64, half stages through four buffers (four waves of 128 x 128 in the same
@@ -622,6 +625,7 @@ int launch_gemm_dma(const GemmArgs &g, int batch, bool trans_b, hipStream_t stre
         case 212: return launch_dma_tile<2, 1, 2>(g, 1, stream);
         case 112: return launch_dma_tile<1, 1, 2>(g, 1, stream);
         case 113: return launch_dma_tile<1, 1, 3>(g, 1, stream);
+        case 114: return launch_dma_tile<1, 1, 4>(g, 1, stream);
         default: return ET_ERR_UNSUPPORTED;
     }
 }

@@ -289,3 +289,28 @@ def test_linear_csr_reference_fixture(et):
                                         up(et, b).ptr, up(et, x).ptr, d_y.ptr, 5, ncol, nrow, 0, None))
     want = (x.astype(np.float32).sum(1, keepdims=True) + b.astype(np.float32)).astype(np.float16)
     assert Hn.max_abs(d_y.numpy(), want) <= 2e-3
+
+
+# Few token rows and a long K: tiles of 16 x 16 up to 1024 of them, then tiles of 64 x 64 with a fourth LDS buffer (at most 256
+# of them, 24 stages and more; whole and ragged, K ending inside a stage) and both sides of the lines; a kept-row weight
+# stores the same products through scattered columns.  The operands are exact in binary16, so what differs is the rounding
+# of the result and of its sum: 2^-11 of the largest value, and K additions of 2^-24 of it.
+@pytest.mark.parametrize("T,K,N", [(16, 1536, 16), (64, 1536, 4096), (64, 1536, 4112), (64, 1520, 4112), (128, 1536, 2112), (176, 1552, 2224),
+                                   (112, 3600, 3744), (1024, 1536, 1024), (1024, 1600, 1088), (1008, 1552, 1040), (528, 2064, 1456)])
+def test_linear_dense_few_rows_long_k(et, T, K, N):
+    x, w, b = Hn.randn((T, K), 401), Hn.randn((N, K), 402, 0.02), Hn.randn((N,), 403, 0.1)
+    d_x, d_w, d_b = up(et, x), up(et, w), up(et, b)
+    d_y = et.DeviceBuffer.from_numpy(np.full((T, N), np.nan, np.float16))
+    want = Hn.f32(x).double() @ Hn.f32(w).double().T
+    et.linear_dense(d_w, d_b, d_x, d_y, T, K, N)
+    full = (want + Hn.f32(b).double()).numpy()
+    bound = float(np.abs(full).max()) * (2.0 ** -11 + K * 2.0 ** -24)
+    assert Hn.max_abs(d_y.numpy(), full) <= bound
+    # every second row of a weight twice as high
+    ids = np.arange(1, 2 * N, 2, dtype=np.int32)
+    d_z = et.DeviceBuffer.from_numpy(np.full((T, 2 * N), np.nan, np.float16))
+    b2 = np.zeros(2 * N, np.float16)
+    b2[ids] = b
+    et.check(et.lib().et_linear_rowpruned_f16(d_w.ptr, up(et, ids).ptr, N, up(et, b2).ptr, d_x.ptr, d_z.ptr, T, K, 2 * N, 0, None))
+    got = d_z.numpy()
+    assert Hn.max_abs(got[:, 1::2], full) <= bound and np.all(got[:, ::2] == 0)
