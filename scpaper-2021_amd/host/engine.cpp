@@ -317,8 +317,8 @@ struct LocalPlan {
 // Against the separate launches (two- to four-layer stacks, 384 to 1024 wide, 40 to 95 % sparsity) it is 1.04 - 2.3 times
 // as fast above 512 rows (1.5 - 2.3 at 8192; 0.93 for 1024 wide at 40 % in binary16, which runs dense GEMMs) and at any row
 // count up to 512 wide, and 1.19 - 1.27 between 256 and 512 rows that are not a whole number of 32-row strips per XCD.  Of
-// the rest the estimate decides: at 512 rows 1.00 - 1.10 up to 14.5 us, 0.92 - 0.97 above; at 128 rows 1.00 - 1.08 up to
-// 10.5 us, 0.89 - 0.92 above.
+// the rest the estimate decides: at 512 rows 1.00 - 1.10 up to 14.5 us, 0.92 - 0.97 above; below 256 rows 1.02 - 1.25 up to
+// 10.5 us.
 LocalPlan plan_local(const et_model_s &m) {
     LocalPlan p;
     const et_model_desc &d = m.desc;
@@ -344,8 +344,13 @@ LocalPlan plan_local(const et_model_s &m) {
             p.parts = parts;
         }
     }
+    // With an FFN of some size, four parts are the least where there is room for four (five layers, us, four parts / what the
+    // estimate takes: 384 wide at 70 % 123 / 135 at 128 rows and 130 / 136 at 1024, 768 wide at 95 % 134 / 148 at 128 and
+    // 136 / 149 at 256); without one the single launch is the fastest form (800 wide, 208 hidden features: 171 / 162).
+    if (kib[ET_W_FF1] + kib[ET_W_FF2] >= 256.0 && 4 * ((strips + 7) / 8) <= 32) p.parts = std::max(p.parts, 4);
     const bool uneven = rows > 256 && (rows + 31) / 32 % 8 != 0;
-    const double most = rows >= 512 || (rows >= 256 && d.emdim <= 768) ? 14.5 : 10.5;
+    // (128 rows: the separate launches' strips come out even there, and they are ahead by 2 to 7 % from 6 us on)
+    const double most = rows >= 512 || (rows >= 256 && d.emdim <= 768) ? 14.5 : rows == 128 ? 5.0 : 10.5;
     if (rows > 512 || uneven || d.emdim <= 512 || best <= most) p.mt = 1;
     const double dense = (4.0 * d.emdim + 2.0 * d.dimFF) * d.emdim / 512.0;  // KiB of all tiles
     if (d.mixed == 0 && d.emdim > 768 && rows <= 4096 && kib[ET_W_O] + shared > 0.5 * dense) p.mt = 0;
