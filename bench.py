@@ -154,7 +154,7 @@ def time_dominant_kernel(et, layers, T, folded, rounds_per_graph=6, replays=8):
     kernel at the workload's shape: the FFN up-projection through the tile-sparse W1 (3072 x 768 at
     80 %) + GELU, T token rows, launched exactly as the stack launches it.
 
-    `folded` (the default stack, four launches per layer): the launch normalises the output
+    `folded` (--chain, --five-launches): the launch normalises the output
     projection's binary32 sum V1 with that projection's row sums while it stages its token strip
     (et_norm_linear_bsr16_packed_f32in on a 12-wave pack, as the layer builds it); V1 and the sums are
     made here by the producer itself from random operands.  Otherwise (seven launches): the plain
@@ -383,13 +383,12 @@ def main():
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline leg")
     ap.add_argument("--eager", action="store_true", help="launch kernel by kernel instead of replaying a graph")
     ap.add_argument("--separate-ln", action="store_true",
-                    help="SkipLayerNorm as launches of its own (seven launches per layer) instead of folded into the "
-                         "neighbouring projections (five)")
+                    help="every projection and every SkipLayerNorm as a launch of its own (seven launches per layer)")
     ap.add_argument("--chain", action="store_true",
                     help="everything between two attention kernels in one launch (two launches per layer)")
     ap.add_argument("--five-launches", action="store_true",
-                    help="the QKV projection as a launch of its own in every layer (five launches per layer) instead of "
-                         "inside the attention kernel (four), which the engine picks for this batch by itself")
+                    help="every projection as a launch of its own (five launches per layer) instead of attention and "
+                         "the token-local launch in two parts (three), which the engine picks for this batch by itself")
     ap.add_argument("--calibrate", action="store_true",
                     help="also launch a plain streaming kernel of known size (ReLU over 64 MiB in, 64 MiB out) "
                          "three times, as the reference point for rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE")

@@ -887,11 +887,12 @@ int et_model_forward(et_model m, et_f16 *out, const et_f16 *in, et_stream stream
 int et_model_forward_layer(et_model m, int layer, et_f16 *out, const et_f16 *in,
                            et_stream stream);
 int et_model_sync(et_model m);
-/* kernel launches an encoder layer of a finalized model is divided into, projection by projection
- * (2: chain launches, 4: the QKV projection inside the attention kernel, 5: SkipLayerNorm folded into
- * the projections, 7: SkipLayerNorm on its own; 0 before et_model_finalize).  et_model_forward may
- * issue several of them as one token-local launch (et_encoder_layer_f32).  A model asked for mixed = 3
- * reports 5 once it has gone back to separate launches. */
+/* kernel launches per encoder layer of a finalized model in the form et_model_forward runs
+ * (2: attention and one token-local launch, et_encoder_layer_f32, or, under mixed = 3, one chain
+ * launch; 3: attention and a token-local launch in two parts; 4: the QKV projection inside the
+ * attention kernel; 5: SkipLayerNorm folded into the projections; 7: SkipLayerNorm on its own; 0 before
+ * et_model_finalize).  A model asked for mixed = 3 reports 5 once it has gone back to separate
+ * launches. */
 int et_model_launches_per_layer(et_model m, int *launches);
 int et_model_destroy(et_model m);
 

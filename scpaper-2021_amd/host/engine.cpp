@@ -611,9 +611,7 @@ int et_model_finalize(et_model m) {
             // mixed == 1: the engine folds SkipLayerNorm into the projections where every layer can
             m->split = (m->desc.mixed == 1 || m->desc.mixed == 3 || m->desc.mixed == 4 || m->desc.mixed == 5) && !m->layers.empty();
             for (auto &l : m->layers) m->split = m->split && l->split_ok();
-            if (m->split && !m->local.empty()) {
-                m->fused_qkv = fused_ok;  // (the form the layers have without the token-local launches)
-            } else if (m->split) {
+            if (m->split && m->local.empty()) {
                 for (auto &l : m->layers) l->enable_split();
                 m->chain = m->desc.mixed == 3 && build_chain(*m);
                 if (want_fused) {
@@ -710,7 +708,9 @@ int et_model_sync(et_model m) {
 int et_model_launches_per_layer(et_model m, int *launches) {
     return guarded([&]() -> int {
         et::require(m != nullptr && launches != nullptr, "et_model_launches_per_layer: NULL argument");
-        *launches = !m->finalized ? 0 : m->chain ? 2 : m->fused_qkv ? 4 : m->split ? 5 : 7;
+        if (!m->finalized) *launches = 0;
+        else if (!m->local.empty()) *launches = m->local_partial ? 3 : 2;
+        else *launches = m->chain ? 2 : m->fused_qkv ? 4 : m->split ? 5 : 7;
         return ET_OK;
     });
 }
