@@ -842,10 +842,13 @@ typedef struct et_model_desc {
                     *    4: as 1, with the QKV projection of every layer after the first inside
                     *    its attention kernel (et_norm_qkv_mha_f32in: four launches per layer)
                     *    where the shapes allow, else as 1; 5: as 1, always with five launches.
-                    * 0: every activation is stored as binary16 (the reference's storage).
-                    * 0 and 1 run everything between two attention kernels in one or two
-                    * token-local launches (et_encoder_layer_f32; the residual is binary32 then,
-                    * under 0 too) where the layers are tile-sparse and it measured faster */
+                    * 0: every activation is stored as binary16 (the reference's storage), and
+                    * et_model_forward gives the same bits as a chain of et_model_forward_layer.
+                    * Where the layers are tile-sparse and it measured faster, 1 runs everything
+                    * between two attention kernels in one or two token-local launches
+                    * (et_encoder_layer_f32), and 0 everything from an attention kernel to the end of
+                    * its layer; sums and normalisations inside a launch are binary32, what goes
+                    * from layer to layer is not changed by it */
 } et_model_desc;
 
 /* which matrix of a layer */
@@ -883,15 +886,18 @@ int et_model_load(const char *weights_txt, const char *dir,
 /* out, in: device [batch*seq_len x emdim].  Asynchronous; stream NULL = the
  * model's own stream (wait with et_model_sync).  in and out may not alias. */
 int et_model_forward(et_model m, et_f16 *out, const et_f16 *in, et_stream stream);
-/* one layer, launched kernel by kernel (Encoder<cfg>::forward) */
+/* one layer between binary16 buffers, launched kernel by kernel (Encoder<cfg>::forward): under mixed =
+ * 0 the launches et_model_forward runs; else with SkipLayerNorm as launches of its own, the residual
+ * starting from the binary16 input, so that a chain of these calls rounds at every layer and
+ * et_model_forward does not */
 int et_model_forward_layer(et_model m, int layer, et_f16 *out, const et_f16 *in,
                            et_stream stream);
 int et_model_sync(et_model m);
 /* kernel launches per encoder layer of a finalized model in the form et_model_forward runs
  * (2: attention and one token-local launch, et_encoder_layer_f32, or, under mixed = 3, one chain
- * launch; 3: attention and a token-local launch in two parts; 4: the QKV projection inside the
- * attention kernel; 5: SkipLayerNorm folded into the projections; 7: SkipLayerNorm on its own; 0 before
- * et_model_finalize).  A model asked for mixed = 3 reports 5 once it has gone back to separate
+ * launch; 3: attention and a token-local launch in two parts; one more than these under mixed = 0,
+ * where QKV is a launch of its own; 4 otherwise: the QKV projection inside the attention kernel; 5:
+ * SkipLayerNorm folded into the projections; 7: SkipLayerNorm on its own; 0 before et_model_finalize).  A model asked for mixed = 3 reports 5 once it has gone back to separate
  * launches. */
 int et_model_launches_per_layer(et_model m, int *launches);
 int et_model_destroy(et_model m);

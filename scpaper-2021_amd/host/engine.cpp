@@ -3,6 +3,7 @@
 // weights the way the reference's example does (example/main.cu:24-182), chains
 // the layers (example/main.cu:175-177) and replays the whole stack as one HIP
 // graph.
+#include <algorithm>
 #include <array>
 #include <memory>
 #include <string>
@@ -315,7 +316,7 @@ struct LocalPlan {
 // (fitted at 768 wide, 60 to 95 % sparsity, 256 to 2048 rows): the number of parts that makes the sum least, while there
 // is a compute unit for every workgroup of an XCD.  Above 256 strips of 16 rows a workgroup takes 32.
 // Against the separate launches (two- to four-layer stacks, 384 to 1024 wide, 40 to 95 % sparsity) it is 1.04 - 2.3 times
-// as fast above 512 rows (1.5 - 2.3 at 8192; 0.93 for 1024 wide at 40 % in binary16, which runs dense GEMMs) and at any row
+// as fast above 512 rows (1.5 - 2.3 at 8192) and at any row
 // count up to 512 wide, and 1.19 - 1.27 between 256 and 512 rows that are not a whole number of 32-row strips per XCD.  Of
 // the rest the estimate decides: at 512 rows 1.00 - 1.10 up to 14.5 us, 0.92 - 0.97 above; below 256 rows 1.02 - 1.25 up to
 // 10.5 us.
@@ -329,15 +330,24 @@ LocalPlan plan_local(const et_model_s &m) {
             kib[w] += 0.5 * (double)h.w[(size_t)w].column.size() / (double)m.host.size();
         }
     const int rows = m.rows(), strips = (rows + 15) / 16;
+    const double shared = kib[ET_W_QKV] + kib[ET_W_FF1] + kib[ET_W_FF2], kept = kib[ET_W_O] + shared;
+    const double all = (4.0 * d.emdim + 2.0 * d.dimFF) * d.emdim / 512.0;  // KiB of all tiles
+    if (d.mixed == 0) {
+        // Three layers, 384 to 1024 wide, time of the separate launches over that of these.  Above 512 rows 1.01 - 1.84 where at
+        // most half of the tiles are kept (an FFN narrower than the model, up to 2048 rows: 0.85 - 1.03 at 40 and 50 % kept,
+        // 0.88 - 1.30 at 20 and 10 %); denser layers, which run dense GEMMs, 0.69 - 1.07, but from 4096 rows on 1.04 - 1.34 up
+        // to 11 KiB a feature.  257 to 512 rows: 1.01 - 1.22 up to 512 wide, 0.86 - 1.08 wider.  Fewer: 0.81 - 1.02.
+        const double most_kept = (d.dimFF >= d.emdim || rows > 2048 ? 0.5 : 0.25) * all;
+        const bool on = rows > 512 ? kept <= most_kept || (rows > 2048 && kept <= 11.0 * d.emdim)
+                                   : rows > 256 && d.emdim <= 512 && kept <= 0.5 * all;
+        if (!on) return p;
+    }
     if (strips > 256) {
         p.mt = 2;
         return p;
     }
-    // (all binary16: small stacks keep the launches whose results et_model_forward_layer repeats bit for bit)
-    if (d.mixed == 0 && rows < 256) return p;
-    const double shared = kib[ET_W_QKV] + kib[ET_W_FF1] + kib[ET_W_FF2];
     double best = 0;
-    for (int parts = 1; parts <= 12 && parts * ((strips + 7) / 8) <= 32; parts++) {
+    for (int parts = 1; parts <= std::min(12, d.dimFF / 16) && parts * ((strips + 7) / 8) <= 32; parts++) {
         const double us = (kib[ET_W_O] + shared / parts) / 112.0 + (parts > 1 ? 5.0 + 0.5 * parts : 0.0);
         if (parts == 1 || us < best) {
             best = us;
@@ -351,9 +361,7 @@ LocalPlan plan_local(const et_model_s &m) {
     const bool uneven = rows > 256 && (rows + 31) / 32 % 8 != 0;
     // (128 rows: the separate launches' strips come out even there, and they are ahead by 2 to 7 % from 6 us on)
     const double most = rows >= 512 || (rows >= 256 && d.emdim <= 768) ? 14.5 : rows == 128 ? 5.0 : 10.5;
-    if (rows > 512 || uneven || d.emdim <= 512 || best <= most) p.mt = 1;
-    const double dense = (4.0 * d.emdim + 2.0 * d.dimFF) * d.emdim / 512.0;  // KiB of all tiles
-    if (d.mixed == 0 && d.emdim > 768 && rows <= 4096 && kib[ET_W_O] + shared > 0.5 * dense) p.mt = 0;
+    if (d.mixed == 0 || rows > 512 || uneven || d.emdim <= 512 || best <= most) p.mt = 1;
     return p;
 }
 
@@ -366,17 +374,31 @@ void build_local(et_model_s &m) {
     std::vector<std::unique_ptr<et_layer_pack_s, LayerPackDeleter>> packs;
     for (int i = 0; i < n; i++) {
         et_layer_weights w{};
-        if (!m.layers[(size_t)i]->local_weights(w) || (i + 1 < n && !m.layers[(size_t)i + 1]->local_qkv(w))) return;
+        const bool project = d.mixed && i + 1 < n;
+        if (!m.layers[(size_t)i]->local_weights(w) || (project && !m.layers[(size_t)i + 1]->local_qkv(w))) return;
         et_layer_pack_s *p = nullptr;
-        const int s = et_encoder_layer_pack_create(&w, m.rows(), d.emdim, d.dimFF, i + 1 < n ? ldq : 0, plan.mt, plan.parts, &p);
+        const int s = et_encoder_layer_pack_create(&w, m.rows(), d.emdim, d.dimFF, project ? ldq : 0, plan.mt, plan.parts, &p);
         if (s == ET_ERR_UNSUPPORTED) return;
         etChk(s);
         packs.emplace_back(p);
     }
     const size_t elems = (size_t)m.rows() * d.emdim;
-    for (auto &b : m.local_x) b = std::make_unique<et::DeviceBuffer<float>>(elems);
+    if (d.mixed)
+        for (auto &b : m.local_x) b = std::make_unique<et::DeviceBuffer<float>>(elems);
     if (plan.parts > 1) m.local_partial = std::make_unique<et::DeviceBuffer<float>>(elems * plan.parts);
     m.local = std::move(packs);
+}
+
+// One layer from binary16 to binary16, as et_model_forward under mixed = 0 chains it and et_model_forward_layer issues it.
+// Token-local launches take the layer's input and leave its result in binary16, and the QKV projection stays a launch of
+// its own, so that a layer does the same whether the one before it ran in the same call or not.
+void run_layer_f16(et_model_s &m, int i, half *out, half *in, stream_t stream) {
+    ILayer &l = *m.layers[(size_t)i];
+    if (m.local.empty()) return l.forward(out, in, stream);
+    l.chain_qkv_first(in, stream);
+    l.chain_attention(stream);
+    etChk(et_encoder_layer_f32(m.local[(size_t)i].get(), et::f16(l.z_buffer()), nullptr, et::f16(in), nullptr, et::f16(out), nullptr,
+                               m.local_partial ? m.local_partial->get() : nullptr, m.desc.act, l.epsilon(0), l.epsilon(1), stream));
 }
 
 void run_layers_local(et_model_s &m, half *out, half *in, stream_t stream) {
@@ -422,13 +444,12 @@ void run_layers_mixed(et_model_s &m, half *out, half *in, stream_t stream) {
 }
 
 void run_layers(et_model_s &m, half *out, half *in, stream_t stream) {
-    if (!m.local.empty()) return run_layers_local(m, out, in, stream);
-    if (m.desc.mixed) return run_layers_mixed(m, out, in, stream);
+    if (m.desc.mixed) return m.local.empty() ? run_layers_mixed(m, out, in, stream) : run_layers_local(m, out, in, stream);
     const int n = (int)m.layers.size();
     half *src = in;
     for (int i = 0; i < n; i++) {
         half *dst = (i == n - 1) ? out : m.pp[i % et_model_s::kRing]->get();
-        m.layers[(size_t)i]->forward(dst, src, stream);
+        run_layer_f16(m, i, dst, src, stream);
         src = dst;
     }
 }
@@ -644,7 +665,7 @@ int et_model_forward_layer(et_model m, int layer, et_f16 *out, const et_f16 *in,
             etChk(et_f16_to_f32(m->pp32[0]->get(), in, (std::size_t)m->rows() * m->desc.emdim, stream));
             m->layers[(size_t)layer]->forward_mixed(nullptr, o, m->pp32[0]->get(), i, stream);
         } else {
-            m->layers[(size_t)layer]->forward(o, i, stream);
+            run_layer_f16(*m, layer, o, i, stream);
         }
         return ET_OK;
     });
@@ -709,7 +730,7 @@ int et_model_launches_per_layer(et_model m, int *launches) {
     return guarded([&]() -> int {
         et::require(m != nullptr && launches != nullptr, "et_model_launches_per_layer: NULL argument");
         if (!m->finalized) *launches = 0;
-        else if (!m->local.empty()) *launches = m->local_partial ? 3 : 2;
+        else if (!m->local.empty()) *launches = (m->local_partial ? 3 : 2) + (m->desc.mixed == 0);
         else *launches = m->chain ? 2 : m->fused_qkv ? 4 : m->split ? 5 : 7;
         return ET_OK;
     });

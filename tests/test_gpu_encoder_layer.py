@@ -111,7 +111,8 @@ def test_stacks_on_token_local_launches(et, H, nh, FF, S, B, sparsity, mixed):
     outs = []
     for use_graph in (True, False):
         m = Hn.build_model(et, layers, S, B, lens=lens, mixed=mixed, use_graph=use_graph)
-        assert m.launches_per_layer() in (2, 3)  # attention, and the token-local part in one launch or two
+        # attention, and the token-local part in one launch or two; all binary16: the QKV projection besides
+        assert m.launches_per_layer() in ((2, 3) if mixed else (3, 4))
         d = et.DeviceBuffer.from_numpy(x)
         o = et.DeviceBuffer.empty(x.shape, np.float16)
         m.forward(o, d)
@@ -122,12 +123,14 @@ def test_stacks_on_token_local_launches(et, H, nh, FF, S, B, sparsity, mixed):
         outs.append(d.numpy())
     for o in outs[1:]:
         assert np.array_equal(outs[0], o)
-    want = Hn.oracle_stack(x, layers, B, lens, store=torch.float16, resid=torch.float32)
+    want = Hn.oracle_stack(x, layers, B, lens, store=torch.float16, resid=torch.float32 if mixed else "same")
     a, b = outs[0].astype(np.float32), want.astype(np.float32)
     for i in range(B):
         a[i * S + lens[i]:(i + 1) * S] = 0
         b[i * S + lens[i]:(i + 1) * S] = 0
-    assert Hn.max_abs(a, b) <= 4e-3  # one binary16 unit at |x| <= 4 and noise, as for the other forms of the residual
+    # binary32 residual: one binary16 unit at |x| <= 4 and noise, as for the other forms of it; a binary16 one is rounded
+    # in every layer, and the oracle rounds the two projections ahead of it besides
+    assert Hn.max_abs(a, b) <= (4e-3 if mixed else 2e-2)
 
 
 def test_token_local_refusals(et):

@@ -70,6 +70,25 @@ def test_layer_by_layer_equals_stack(et):
     assert Hn.max_abs(full, Hn.oracle_stack(x, layers, B, act="relu")) <= TOL_F16
 
 
+@pytest.mark.parametrize("H,nh,FF,S,B,launches", [(384, 6, 1536, 176, 3, 4), (256, 4, 512, 64, 5, 3), (256, 4, 512, 128, 33, 3),
+                                                  (768, 12, 512, 112, 2, 7)])
+def test_layer_by_layer_equals_stack_in_every_form(et, H, nh, FF, S, B, launches):
+    """All activations binary16 (mixed = 0): the stack and a chain of et_model_forward_layer agree bit for bit on the
+    token-local launches too, shared strips (528 rows), one workgroup a strip (320) and 32-row strips (4224), as on the
+    separate ones (224), and stay near the storage the mode promises."""
+    layers = [Hn.LayerWeights(H, nh, FF, 0.7, seed=45 + i) for i in range(3)]
+    m = Hn.build_model(et, layers, S, B, act=1)
+    assert m.launches_per_layer() == launches
+    x = Hn.randn((B * S, H), 3)
+    full = run_model(et, m, x)[0]
+    bufs = [et.DeviceBuffer.from_numpy(x), et.DeviceBuffer.empty((B * S, H), np.float16)]
+    for i in range(3):
+        m.forward_layer(i, bufs[(i + 1) % 2], bufs[i % 2])
+    et.sync()
+    assert np.array_equal(full, bufs[1].numpy(np.float16, (B * S, H)))
+    assert Hn.max_abs(full, Hn.oracle_stack(x, layers, B, act="relu")) <= TOL_F16
+
+
 def headline_layers(seed0):
     H, nh, FF = 768, 12, 3072
     return [Hn.LayerWeights(H, nh, FF, 0.8, seed=seed0 + i, attention_aware=0.25) for i in range(12)]
