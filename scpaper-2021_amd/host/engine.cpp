@@ -315,12 +315,19 @@ struct LocalPlan {
 // sharing a strip costs a second launch and the exchange of the shares, about 5 us and half a microsecond per share
 // (fitted at 768 wide, 60 to 95 % sparsity, 256 to 2048 rows): the number of parts that makes the sum least, while there
 // is a compute unit for every workgroup of an XCD.  Above 256 strips of 16 rows a workgroup takes 32.
-// Against the separate launches (two- to four-layer stacks, 384 to 1024 wide, 40 to 95 % sparsity) it is 1.04 - 2.3 times
-// as fast above 512 rows (1.5 - 2.3 at 8192) and at any row
-// count up to 512 wide, and 1.19 - 1.27 between 256 and 512 rows that are not a whole number of 32-row strips per XCD.  Of
-// the rest the estimate decides: at 512 rows 1.00 - 1.10 up to 14.5 us, 0.92 - 0.97 above; below 256 rows 1.02 - 1.25 up to
-// 10.5 us.
-LocalPlan plan_local(const et_model_s &m) {
+// Which stacks run it: time of the separate launches over that of these, two- to four-layer stacks, 384, 768 and 1024 wide
+// (and 512 up to 512 rows), 0 to 95 % sparsity.  `fused`: the separate launches would hold QKV in the attention kernel.
+//   above 4096 rows                                       1.04 - 2.0
+//   kept tiles above 16.5 KiB a feature (768 wide below 10 % sparsity, 1024 below 30 %: dense GEMMs beside) 0.76 - 1.06
+//   up to 512 wide                                        0.96 - 1.98 (0.96 - 0.98: 64 and 128 rows)
+//   above 512 rows                                        0.95 - 1.98 (0.95 - 0.97: FFN of a quarter of the width, 1024 rows)
+//   257 to 480 rows (a 32-row strip more for some XCDs)   0.95 - 1.43 (below 1: unpruned)
+//   481 to 512 rows: denser than half 1.18 - 1.25 (unpruned 0.99), else up to 14.5 us of the estimate 0.98 - 1.13, above 0.93 - 0.98
+//   256 rows and fewer, denser than half                  0.75 - 1.04
+//     112 and 128 rows (the separate launches have a strip for each XCD)      0.85 - 1.00, at 95 % sparsity 0.94 - 1.05
+//     up to 48 rows, 144 to 192 (one XCD more than another has two strips)    1.00 - 1.95, measured up to 19 us
+//     others: up to 14.5 us 1.00 - 1.16 (with `fused` above 192 rows 0.94 - 1.02), above 0.91 - 1.04
+LocalPlan plan_local(const et_model_s &m, bool fused) {
     LocalPlan p;
     const et_model_desc &d = m.desc;
     double kib[4] = {0, 0, 0, 0};  // of a layer, on average
@@ -358,16 +365,22 @@ LocalPlan plan_local(const et_model_s &m) {
     // estimate takes: 384 wide at 70 % 123 / 135 at 128 rows and 130 / 136 at 1024, 768 wide at 95 % 134 / 148 at 128 and
     // 136 / 149 at 256); without one the single launch is the fastest form (800 wide, 208 hidden features: 171 / 162).
     if (kib[ET_W_FF1] + kib[ET_W_FF2] >= 256.0 && 4 * ((strips + 7) / 8) <= 32) p.parts = std::max(p.parts, 4);
-    const bool uneven = rows > 256 && (rows + 31) / 32 % 8 != 0;
-    // (128 rows: the separate launches' strips come out even there, and they are ahead by 2 to 7 % from 6 us on)
-    const double most = rows >= 512 || (rows >= 256 && d.emdim <= 768) ? 14.5 : rows == 128 ? 5.0 : 10.5;
-    if (d.mixed == 0 || rows > 512 || uneven || d.emdim <= 512 || best <= most) p.mt = 1;
+    bool on;
+    if (d.mixed == 0) on = true;
+    else if (kept > 16.5 * d.emdim) on = false;
+    else if (d.emdim <= 512 || rows > 512) on = true;
+    else if (rows > 256) on = rows <= 480 || kept > 0.5 * all || best <= 14.5;
+    else if (kept > 0.5 * all) on = false;
+    else if (strips == 7 || strips == 8) on = best <= 5.0;
+    else if (strips <= 3 || (strips >= 9 && strips <= 12)) on = best <= 19.0;
+    else on = best <= 14.5 && !(fused && strips > 12);
+    p.mt = on ? 1 : 0;
     return p;
 }
 
-// The packs of the token-local launches; leaves m.local empty where a layer has no such form.
-void build_local(et_model_s &m) {
-    const LocalPlan plan = plan_local(m);
+// The packs of the token-local launches (`fused` as plan_local takes it); leaves m.local empty where a layer has no such form.
+void build_local(et_model_s &m, bool fused) {
+    const LocalPlan plan = plan_local(m, fused);
     const et_model_desc &d = m.desc;
     const int n = (int)m.layers.size(), ldq = 2 * d.kdim + d.vdim;
     if (plan.mt == 0 || d.kdim != d.emdim || d.vdim != d.emdim || et_encoder_layer_supported(m.rows(), d.emdim, d.dimFF, ldq) != 1) return;
@@ -625,7 +638,7 @@ int et_model_finalize(et_model m) {
         const long heads = (long)d.batch * d.nhead;
         const bool want_fused = (d.mixed == 4 || (d.mixed == 1 && heads >= 96 && heads <= 400)) && m->layers.size() > 1;
         const bool fused_ok = want_fused && et_norm_qkv_mha_f32in_supported(d.batch, d.seq_len, d.emdim, d.nhead, d.kdim / d.nhead) == 1;
-        if (d.mixed == 0 || d.mixed == 1 || (d.mixed == 4 && !fused_ok)) build_local(*m);
+        if (d.mixed == 0 || d.mixed == 1 || (d.mixed == 4 && !fused_ok)) build_local(*m, fused_ok);
         if (m->desc.mixed) {
             for (auto &b : m->pp32) b = std::make_unique<et::DeviceBuffer<float>>(act_elems);
             for (auto &l : m->layers) l->enable_mixed();

@@ -170,6 +170,21 @@ def test_qkv_inside_attention_chosen_by_batch(et):
         assert Hn.max_abs(got, want) <= 4e-3
 
 
+@pytest.mark.parametrize("H,sparsity,B,S,launches", [
+    (768, 0.6, 3, 16, 3), (768, 0.8, 1, 64, 3), (768, 0.6, 1, 64, 5), (768, 0.8, 1, 112, 5), (768, 0.8, 1, 128, 5), (768, 0.6, 1, 144, 3),
+    (768, 0.8, 2, 128, 3), (768, 0.8, 8, 32, 4), (768, 0.6, 1, 240, 5), (768, 0.6, 1, 272, 3), (768, 0.6, 4, 128, 5), (768, 0.4, 4, 128, 3),
+    (768, 0.4, 2, 128, 7), (1024, 0.8, 4, 128, 5), (1024, 0.9, 4, 128, 3), (768, 0.0, 4, 144, 7), (1024, 0.2, 4, 144, 7), (512, 0.0, 2, 64, 3)])
+def test_token_local_form_chosen_by_rows_and_tiles(et, H, sparsity, B, S, launches):
+    """Both sides of every line mixed = 1 draws between the token-local launches and the separate ones (rows, strips for
+    each XCD, tiles kept), by the launches a layer has; the result is the oracle's in either form."""
+    layers = [Hn.LayerWeights(H, H // 64, 4 * H, sparsity, seed=960 + i) for i in range(2)]
+    m = Hn.build_model(et, layers, S, B, mixed=1)
+    assert m.launches_per_layer() == launches
+    x = Hn.randn((B * S, H), 969)
+    want = Hn.oracle_stack(x, layers, B, store=torch.float16, resid=torch.float32)
+    assert Hn.max_abs(run_model(et, m, x)[0], want) <= 4e-3
+
+
 def test_qkv_inside_attention_falls_back(et):
     """Shapes the fused kernel does not take (here a 256-wide model) run mixed = 4 exactly as mixed = 1."""
     H, nh, FF, S, B = 256, 4, 512, 64, 2
