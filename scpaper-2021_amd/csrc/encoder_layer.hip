@@ -52,7 +52,7 @@ constexpr size_t kElLds = 160 * 1024;
 // of its block-rows, in the same way: one request each at the start, read with v_readlane
 constexpr int kElTabSeg = 0, kElTabCount = kElTabSeg + kElMaxSeg, kElTab = 64, kElRowRegs = 2;
 // descriptor: slots (bits 0-7), kind (8-9), operand in the hidden chunk (10), target (11-20), bias over 16 (21-31)
-constexpr int kElKindSum = 0, kElKindHidden = 1, kElKindQkv = 2;
+constexpr int kElKindSum = 0, kElKindHidden = 1, kElKindQkv = 2, kElMaxSlots = 255;
 
 struct LayerArgs {
     const char *slots;
@@ -711,6 +711,7 @@ int et_encoder_layer_pack_create(const et_layer_weights *w, int T, int emdim, in
         std::vector<std::pair<int, int>> offs;
     };
     std::vector<Stream> streams;
+    int most_slots = 0;  // of a block-row in a segment (a column may occur in it more than once)
     auto tiles_of = [](const HostBsr &m, int mat, int r) {
         std::vector<std::pair<int32_t, int32_t>> v;
         for (int t = m.rp[(size_t)r]; t < m.rp[(size_t)r + 1]; t++) v.push_back({t | mat << 28, m.ci[(size_t)t] * 32});
@@ -738,6 +739,7 @@ int et_encoder_layer_pack_create(const et_layer_weights *w, int T, int emdim, in
             for (size_t sg = 0; sg < segs.size(); sg++) {
                 st.tab[kElTabSeg + sg] = (int32_t)segs[sg][(size_t)v].size();
                 for (const ElRow &r : segs[sg][(size_t)v]) {
+                    most_slots = std::max(most_slots, r.slots());
                     st.rows.push_back((uint32_t)r.slots() | (uint32_t)r.kind << 8 | (uint32_t)r.hidden << 10 | (uint32_t)r.target << 11 |
                                       (uint32_t)(r.bias / 16) << 21);
                     for (size_t t = 0; t < r.tiles.size(); t += 2) {
@@ -810,6 +812,8 @@ int et_encoder_layer_pack_create(const et_layer_weights *w, int T, int emdim, in
         most_rows = std::max(most_rows, st.rows.size());
     }
     cap = (cap + kElRing - 1) / kElRing * kElRing + kElRing;
+    ET_REQUIRE(most_slots <= kElMaxSlots, ET_ERR_UNSUPPORTED, "et_encoder_layer_pack_create: %d slots in one block-row, at most %d fit its descriptor",
+               most_slots, kElMaxSlots);
     ET_REQUIRE(most_rows <= 64 * kElRowRegs, ET_ERR_UNSUPPORTED, "et_encoder_layer_pack_create: %zu block-rows in one wave", most_rows);
     std::vector<int32_t> tab, order(streams.size() * cap * 2, -1);
     std::vector<uint32_t> rows(streams.size() * 64 * kElRowRegs, 0);

@@ -141,3 +141,55 @@ def test_token_local_refusals(et):
     assert lib.et_encoder_layer_pack_create(C.byref(w), 32, 256, 256, 0, 2, 2, C.byref(pack)) == et.ET_ERR_INVALID_ARG
     assert lib.et_encoder_layer_pack_create(None, 32, 256, 256, 0, 1, 1, C.byref(pack)) == et.ET_ERR_INVALID_ARG
     assert lib.et_encoder_layer_f32(None, None, None, None, None, None, None, None, 0, 1e-5, 1e-5, None) == et.ET_ERR_INVALID_ARG
+
+
+def layer_pack(et, T, H, FF, parts, tiles_of_first_row=None):
+    """(status, pack, what has to stay alive) of a layer without projection; the first block-row of Wo may be given as that
+    many tiles on column 0."""
+    w, keep, pack = Weights(), [], C.c_void_p()
+    for k, (o, i) in enumerate(((H, H), (FF, H), (H, FF))):
+        m = Hn.BsrWeight(o, i, 0.5, seed=91 + k, std=0.01, bias_std=0.1)
+        row_ptr, col_idx, tiles = m.row_ptr, m.col_idx, m.tiles
+        if k == 0 and tiles_of_first_row is not None:
+            first = int(row_ptr[1])
+            row_ptr = np.concatenate([row_ptr[:1], row_ptr[1:] - first + tiles_of_first_row]).astype(np.int32)
+            col_idx = np.concatenate([np.zeros(tiles_of_first_row, np.int32), col_idx[first:]])
+            tiles = np.concatenate([Hn.randn((tiles_of_first_row, 256), 97, 0.01), tiles[first:]])
+        for name, arr in (("row_ptr", row_ptr), ("col_idx", col_idx), ("tiles", tiles), ("bias", m.bias)):
+            keep.append(up(et, arr))
+            getattr(w, name)[k] = keep[-1].ptr
+        keep.append((row_ptr, col_idx, tiles, m.bias))
+    for k in range(2):
+        for name, arr in (("gamma", np.ones(H, np.float16)), ("beta", np.zeros(H, np.float16))):
+            keep.append(up(et, arr))
+            getattr(w, name)[k] = keep[-1].ptr
+    return et.lib().et_encoder_layer_pack_create(C.byref(w), T, H, FF, 0, 1, parts, C.byref(pack)), pack, keep, w
+
+
+def test_token_local_longest_block_row(et):
+    """A descriptor counts up to 255 slots of two tiles: 510 tiles in a block-row (columns may occur more than once) are
+    multiplied, 511 have no pack."""
+    T, H, FF = 32, 48, 32
+    st, pack, _, _ = layer_pack(et, T, H, FF, 1, 511)
+    assert st == et.ET_ERR_UNSUPPORTED and not pack.value
+    st, pack, keep, _ = layer_pack(et, T, H, FF, 1, 510)
+    et.check(st)
+    mats = [k for k in keep if isinstance(k, tuple)]
+
+    def dense(m, n_in):  # tiles of one position add up
+        d = torch.zeros(16 * (len(m[0]) - 1), n_in)
+        for r in range(len(m[0]) - 1):
+            for t in range(m[0][r], m[0][r + 1]):
+                d[16 * r:16 * r + 16, 16 * m[1][t]:16 * m[1][t] + 16] += torch.from_numpy(m[2][t].astype(np.float32)).view(16, 16)
+        return d
+
+    Z, x = Hn.randn((T, H), 98), Hn.randn((T, H), 99)
+    out = et.DeviceBuffer.empty((T, H), np.float16)
+    dZ, dx = up(et, Z), up(et, x)
+    et.check(et.lib().et_encoder_layer_f32(pack, dZ.ptr, None, dx.ptr, None, out.ptr, None, None, 0, 1e-5, 1e-5, None))
+    f, norm = Hn.f32, lambda v: torch.nn.functional.layer_norm(v, (H,), eps=1e-5)
+    y = norm(f(Z) @ dense(mats[0], H).T + f(mats[0][3]) + f(x))
+    h = (y.half().float() @ dense(mats[1], H).T + f(mats[1][3])).half().float()
+    want = norm(h @ dense(mats[2], FF).T + f(mats[2][3]) + y)
+    assert Hn.max_abs(out.numpy(), want.numpy()) <= 4e-3
+    et.check(et.lib().et_encoder_layer_pack_destroy(pack))
