@@ -284,8 +284,9 @@ int et_encoder_chain_status(const uint32_t *sync, int *gave_up, int *misplaced);
  * et_encoder_layer_f32: Z [T x emdim]; the residual x in binary32 (x32, in tile order) or, with x32
  * NULL, binary16 (x16 [T x emdim]); x' goes to x32_out in tile order and to out16 [T x emdim] (either
  * may be NULL); QKV [T x qkv_out]; partial: parts * T * emdim floats of workspace (unread with parts =
- * 1).  x32_out may not be x32.  A block-row of more than 510 tiles (columns that occur more than once)
- * has no pack.  Tile order, of T * emdim floats: for 16 tokens after 16 tokens, and 16
+ * 1).  x32_out may not overlap x32.  x16 and out16 8-byte aligned, everything else, and the tiles of
+ * et_layer_weights, 16-byte aligned; a block-row of more than 510 tiles (columns that occur more than
+ * once) has no pack.  Tile order, of T * emdim floats: for 16 tokens after 16 tokens, and 16
  * features after 16 features in them, 256 values: token r, features 4g .. 4g + 3 at 4 (16 g + r). */
 struct et_layer_pack_s;
 typedef struct et_layer_weights {

@@ -659,9 +659,12 @@ int et_encoder_layer_pack_create(const et_layer_weights *w, int T, int emdim, in
     ET_REQUIRE((mt == 1 || mt == 2) && parts >= 1 && parts <= 32 && (parts == 1 || mt == 1), ET_ERR_INVALID_ARG,
                "et_encoder_layer_pack_create: mt=%d parts=%d", mt, parts);
     const int nmat = qkv_out ? 4 : 3;
-    for (int i = 0; i < nmat; i++)
+    for (int i = 0; i < nmat; i++) {
         ET_REQUIRE(w->row_ptr[i] && w->col_idx[i] && w->tiles[i] && w->bias[i], ET_ERR_INVALID_ARG,
                    "et_encoder_layer_pack_create: NULL weight %d", i);
+        ET_REQUIRE((reinterpret_cast<uintptr_t>(w->tiles[i]) & 15) == 0, ET_ERR_UNSUPPORTED,
+                   "et_encoder_layer_pack_create: the tiles of weight %d must be 16-byte aligned", i);
+    }
     for (int i = 0; i < 2; i++)
         ET_REQUIRE(w->gamma[i] && w->beta[i], ET_ERR_INVALID_ARG, "et_encoder_layer_pack_create: NULL norm %d", i);
     const int H = emdim, FF = dimFF, Q = qkv_out, nbH = H / 16, nbF = FF / 16, nbQ = Q / 16;
@@ -908,6 +911,13 @@ extern "C" int et_encoder_layer_f32(const struct et_layer_pack_s *p, const et_f1
     ET_REQUIRE(p && Z && (x32 || x16) && (p->Q == 0 || QKV) && (p->parts == 1 || partial), ET_ERR_INVALID_ARG,
                "et_encoder_layer_f32: NULL pointer");
     ET_REQUIRE(act >= ET_ACT_NONE && act <= ET_ACT_GELU, ET_ERR_INVALID_ARG, "et_encoder_layer_f32: act=%d", act);
+    const auto at = [](const void *q) { return reinterpret_cast<uintptr_t>(q); };
+    ET_REQUIRE(((at(Z) | at(x32) | at(x32_out) | at(QKV) | at(partial)) & 15) == 0, ET_ERR_UNSUPPORTED,
+               "et_encoder_layer_f32: Z, x32, x32_out, QKV and partial must be 16-byte aligned");
+    ET_REQUIRE(((at(x16) | at(out16)) & 7) == 0, ET_ERR_UNSUPPORTED, "et_encoder_layer_f32: x16 and out16 must be 8-byte aligned");
+    const size_t x32_bytes = (size_t)p->T * p->H * 4;
+    ET_REQUIRE(!x32 || !x32_out || at(x32_out) >= at(x32) + x32_bytes || at(x32) >= at(x32_out) + x32_bytes, ET_ERR_INVALID_ARG,
+               "et_encoder_layer_f32: x32_out overlaps x32");
     LayerArgs a{};
     a.slots = static_cast<const char *>(p->slots);
     a.offs = static_cast<const char *>(p->offs);

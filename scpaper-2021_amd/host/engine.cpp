@@ -402,6 +402,21 @@ void build_local(et_model_s &m, bool fused) {
     m.local = std::move(packs);
 }
 
+// The token-local launches read the model's input and write its result eight bytes at a time; at another address (which
+// the separate launches take) they pass through buffers of the model: `warm` is free but for the pass that precedes a
+// capture, whose result it is, and layer kRing - 1 comes to its ring slot after the first layer has read the input.
+bool local_aligned(const half *p) { return (reinterpret_cast<std::uintptr_t>(p) & 7) == 0; }
+half *local_input(et_model_s &m, half *in, stream_t stream) {
+    if (local_aligned(in)) return in;
+    half *staged = m.pp[et_model_s::kRing - 1]->get();
+    etChk(et_memcpy_d2d(staged, in, (std::size_t)m.rows() * m.desc.emdim * sizeof(half), stream));
+    return staged;
+}
+half *local_result(et_model_s &m, half *out) { return local_aligned(out) ? out : m.warm->get(); }
+void local_deliver(et_model_s &m, half *out, const half *from, stream_t stream) {
+    if (from != out) etChk(et_memcpy_d2d(out, from, (std::size_t)m.rows() * m.desc.emdim * sizeof(half), stream));
+}
+
 // One layer from binary16 to binary16, as et_model_forward under mixed = 0 chains it and et_model_forward_layer issues it.
 // Token-local launches take the layer's input and leave its result in binary16, and the QKV projection stays a launch of
 // its own, so that a layer does the same whether the one before it ran in the same call or not.
@@ -410,22 +425,26 @@ void run_layer_f16(et_model_s &m, int i, half *out, half *in, stream_t stream) {
     if (m.local.empty()) return l.forward(out, in, stream);
     l.chain_qkv_first(in, stream);
     l.chain_attention(stream);
-    etChk(et_encoder_layer_f32(m.local[(size_t)i].get(), et::f16(l.z_buffer()), nullptr, et::f16(in), nullptr, et::f16(out), nullptr,
+    half *x = local_input(m, in, stream), *to = local_result(m, out);
+    etChk(et_encoder_layer_f32(m.local[(size_t)i].get(), et::f16(l.z_buffer()), nullptr, et::f16(x), nullptr, et::f16(to), nullptr,
                                m.local_partial ? m.local_partial->get() : nullptr, m.desc.act, l.epsilon(0), l.epsilon(1), stream));
+    local_deliver(m, out, to, stream);
 }
 
 void run_layers_local(et_model_s &m, half *out, half *in, stream_t stream) {
     const int n = (int)m.layers.size();
     m.layers[0]->chain_qkv_first(in, stream);
+    half *x = local_input(m, in, stream), *to = local_result(m, out);
     for (int i = 0; i < n; i++) {
         ILayer &l = *m.layers[(size_t)i];
         const bool last = i == n - 1;
         l.chain_attention(stream);
         etChk(et_encoder_layer_f32(m.local[(size_t)i].get(), et::f16(l.z_buffer()), i ? m.local_x[(i - 1) & 1]->get() : nullptr,
-                                   et::f16(in), last ? nullptr : m.local_x[i & 1]->get(), last ? et::f16(out) : nullptr,
+                                   i ? nullptr : et::f16(x), last ? nullptr : m.local_x[i & 1]->get(), last ? et::f16(to) : nullptr,
                                    last ? nullptr : et::f16(m.layers[(size_t)i + 1]->qkv_buffer()),
                                    m.local_partial ? m.local_partial->get() : nullptr, m.desc.act, l.epsilon(0), l.epsilon(1), stream));
     }
+    local_deliver(m, out, to, stream);
 }
 
 void run_layers_split(et_model_s &m, half *out, half *in, stream_t stream) {

@@ -193,3 +193,52 @@ def test_token_local_longest_block_row(et):
     want = norm(h @ dense(mats[2], FF).T + f(mats[2][3]) + y)
     assert Hn.max_abs(out.numpy(), want.numpy()) <= 4e-3
     et.check(et.lib().et_encoder_layer_pack_destroy(pack))
+
+
+def test_token_local_refuses_addresses_and_overlap(et):
+    """Before any launch: buffers off the addresses the kernel's loads and stores need, and a result over the residual."""
+    lib, T, H, FF, parts = et.lib(), 32, 48, 32, 2
+    st, pack, keep, w = layer_pack(et, T, H, FF, parts)
+    et.check(st)
+    half, wide = T * H * 2, T * H * 4
+    buf = et.DeviceBuffer.empty((4 * half + 8 * wide,), np.uint8)
+    Z, x16, out16 = buf.ptr, buf.ptr + half + 64, buf.ptr + 2 * half + 128
+    x32 = buf.ptr + 4 * half
+    o32, partial = x32 + wide, x32 + 2 * wide
+
+    def call(Z=Z, x32=x32, x16=None, o32=o32, out16=out16, partial=partial):
+        return lib.et_encoder_layer_f32(pack, Z, x32, x16, o32, out16, None, partial, 0, 1e-5, 1e-5, None)
+
+    for bad in (dict(Z=Z + 8), dict(x32=x32 + 4), dict(o32=o32 + 8), dict(partial=partial + 4), dict(out16=out16 + 4),
+                dict(x32=None, x16=x16 + 4)):
+        assert call(**bad) == et.ET_ERR_UNSUPPORTED, bad
+    for bad in (dict(o32=x32), dict(o32=x32 + 16), dict(o32=x32 + wide - 16, partial=partial + wide), dict(o32=x32 - wide + 16)):
+        assert call(**bad) == et.ET_ERR_INVALID_ARG, bad
+    w.tiles[1] = w.tiles[1] + 8
+    other = C.c_void_p()
+    assert lib.et_encoder_layer_pack_create(C.byref(w), T, H, FF, 0, 1, parts, C.byref(other)) == et.ET_ERR_UNSUPPORTED
+    et.check(lib.et_encoder_layer_pack_destroy(pack))
+
+
+@pytest.mark.parametrize("mixed", [0, 1])
+@pytest.mark.parametrize("use_graph", [True, False])
+def test_token_local_stack_at_any_address(et, mixed, use_graph):
+    """A model takes its input and result where the separate launches took them: the input four bytes, the result two off
+    the alignment of the token-local launches, the same bits as at aligned addresses, on every replay."""
+    H, nh, FF, S, B = 256, 4, 512, 64, 5
+    layers = [Hn.LayerWeights(H, nh, FF, 0.7, seed=830 + i) for i in range(5)]
+    m = Hn.build_model(et, layers, S, B, mixed=mixed, use_graph=use_graph)
+    assert m.launches_per_layer() == (2 if mixed else 3)
+    x = Hn.randn((B * S, H), 831)
+    want = et.DeviceBuffer.empty(x.shape, np.float16)
+    d = et.DeviceBuffer.from_numpy(x)
+    m.forward(want, d)
+    m.sync()
+    shifted_in = et.DeviceBuffer.from_numpy(np.concatenate([np.zeros(2, np.float16), x.reshape(-1)]))
+    shifted_out = et.DeviceBuffer.from_numpy(np.zeros(x.size + 1, np.float16))
+    for _ in range(3):
+        m.forward(shifted_out.ptr + 2, shifted_in.ptr + 4)
+        m.sync()
+        assert np.array_equal(shifted_out.numpy(np.float16, (x.size + 1,))[1:].reshape(x.shape), want.numpy())
+        et.check(et.lib().et_fill_f16(shifted_out.ptr, x.size + 1, 0x7E00, None))
+        et.sync()
