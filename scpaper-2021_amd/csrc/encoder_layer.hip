@@ -85,7 +85,8 @@ struct LayerArgs {
 // request can stay in flight across anything the compiler puts between two block-rows (left to the compiler, the
 // ring was copied between registers at every block-row, in flight or not).  vmcnt counts in order: behind the request of
 // a slot lie seven of later slots and one of offsets (the slot at position 7: seven), so a slot has arrived at vmcnt(8) (7); whatever else the compiler issues
-// in between only makes the wait longer.
+// in between only makes the wait longer.  The compiler warns that it does not expect assembly to touch registers it was
+// told to leave; what it makes of this file is held to these rules, instruction by instruction, by a test.
 #define ET_EL_CLOBBERS                                                                                                   \
     "v88", "v89", "v90", "v91", "v92", "v93", "v94", "v95", "v96", "v97", "v98", "v99", "v100", "v101", "v102", "v103", \
         "v104", "v105", "v106", "v107", "v108", "v109", "v110", "v111", "v112", "v113", "v114", "v115", "v116", "v117",  \

@@ -37,3 +37,16 @@ def test_the_analysis_sees_a_wait_that_ends_too_soon(assembly):
     for wait, short in (("vmcnt(9)", "vmcnt(10)"), ("vmcnt(8) lgkmcnt(1)", "vmcnt(9) lgkmcnt(1)"), ("vmcnt(7)\n\tv_mov_b32 v88", "vmcnt(9)\n\tv_mov_b32 v88")):
         early = {n: isa_waits.early_uses(*k) for n, k in token_local(assembly.replace(wait, short)).items()}
         assert any(early.values()), wait
+
+
+def test_the_compiler_stays_out_of_the_ring(assembly):
+    """The kernel is compiled for 88 registers and the ring lies in those above, reserved by an attribute the compiler
+    warns about: nothing it wrote itself may name one of them (nor an accumulation register, which would be its way to
+    spill), and the kernel has to be started with all 128."""
+    for name, (code, _) in token_local(assembly).items():
+        taken = [(i.line, i.text) for i in code if not i.in_asm and any(kind == "a" or n >= 88 for kind, n in i.regs)]
+        assert taken == [], name
+        assert any(i.in_asm and ("v", 127) in i.regs for i in code), name
+        block = assembly[assembly.index(f".amdhsa_kernel {name}\n"):]
+        block = block[:block.index(".end_amdhsa_kernel")]
+        assert ".amdhsa_next_free_vgpr 128\n" in block and ".amdhsa_private_segment_fixed_size 0\n" in block, name
