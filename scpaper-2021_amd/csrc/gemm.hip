@@ -277,7 +277,11 @@ __global__ __launch_bounds__(256) void gemm_skinny_kernel(const GemmArgs g) {
 // 2048 tiles of 16 x 16 it beats the 64 x 64 tiles (512 x 768 -> 768: 6.1 against 7.3 us; 128 x 768
 // -> 2304: 5.4 against 7.0), from about 2300 on it loses (256 x 768 -> 2304: 8.0 against 7.4).  With a long K the 64 x 64
 // tiles have a fourth LDS buffer and the line lies lower, at 1024 (us, this kernel / 64 x 64 tiles: 768 tiles of 3072 10.7 /
-// 13.7, 1024 of 4096 16.1 / 17.0, 1152 of 3072 15.2 / 14.2, 1536 of 3072 17.3 / 14.2, 1638 of 3600 39.5 / 17.9).
+// 13.7, 1024 of 4096 16.1 / 17.0, 1152 of 3072 15.2 / 14.2, 1536 of 3072 17.3 / 14.2, 1638 of 3600 39.5 / 17.9; at 24 stages,
+// K = 1536, 1056 to 1792 tiles 0.89 to 1.21 of them).  Operands the 64 x 64 tiles do not take (a result off their alignment, as
+// a row-pruned Linear may be given) would fall to the register-staged kernel, so there the line stays: 512 x 3072 -> 528 scattered
+// 20.0 / 37.4, 1024 x 1536 -> 448 14.3 / 23.1, 1024 x 4096 -> 448 29.2 / 46.7.  (Batched problems do not come near it:
+// with more than 1024 tiles each, two of them have more than 128 of 64 x 64.)
 static bool gemm_skinny_applies(const GemmArgs &g, int batch, bool trans_b) {
     const auto misaligned = [](const void *p, int a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) != 0; };
     if (!trans_b || g.a_gather || batch < 1 || batch > 65535) return false;
@@ -287,7 +291,7 @@ static bool gemm_skinny_applies(const GemmArgs &g, int batch, bool trans_b) {
     if (batch > 1 && (((g.sAo | g.sAi | g.sBo | g.sBi) & 7) || ((g.sCo | g.sCi) & 3))) return false;
     const long long tiles64 = (long long)((g.M + 63) / 64) * ((g.N + 63) / 64) * batch;
     const long long tiles16 = (long long)(g.M / 16) * (g.N / 16);
-    return tiles64 < 128 && tiles16 <= (g.K / 64 >= 24 ? 1024 : 2048);
+    return tiles64 < 128 && tiles16 <= (g.K / 64 >= 24 && gemm_dma_applies(g, batch, trans_b) ? 1024 : 2048);
 }
 
 // C[r][c] = act(bias[c]) for the columns a row-pruned weight does not produce.

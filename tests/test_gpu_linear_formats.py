@@ -314,3 +314,21 @@ def test_linear_dense_few_rows_long_k(et, T, K, N):
     et.check(et.lib().et_linear_rowpruned_f16(d_w.ptr, up(et, ids).ptr, N, up(et, b2).ptr, d_x.ptr, d_z.ptr, T, K, 2 * N, 0, None))
     got = d_z.numpy()
     assert Hn.max_abs(got[:, 1::2], full) <= bound and np.all(got[:, ::2] == 0)
+
+
+@pytest.mark.parametrize("T,K,N", [(512, 3072, 528), (1024, 1536, 272), (2048, 2304, 256), (1024, 1552, 528)])
+def test_few_rows_long_k_off_alignment(et, T, K, N):
+    """A row-pruned Linear whose result lies two bytes off every alignment: more than 1024 tiles of 16 x 16 (up to 2048, and
+    above) with a long K, where whole and ragged 64 x 64 tiles are not taken.  Bound as above."""
+    x, w, b = Hn.randn((T, K), 411), Hn.randn((N, K), 412, 0.02), Hn.randn((2 * N,), 413, 0.1)
+    ids = np.arange(1, 2 * N, 2, dtype=np.int32)
+    b[::2] = 0
+    d_y = et.DeviceBuffer.from_numpy(np.full(T * 2 * N + 2, np.nan, np.float16))
+    d = [up(et, a) for a in (w, ids, b, x)]
+    et.check(et.lib().et_linear_rowpruned_f16(d[0].ptr, d[1].ptr, N, d[2].ptr, d[3].ptr, d_y.ptr + 2, T, K, 2 * N, 0, None))
+    got = d_y.numpy(np.float16, (T * 2 * N + 2,))
+    full = (Hn.f32(x).double() @ Hn.f32(w).double().T + Hn.f32(b[ids]).double()).numpy()
+    bound = float(np.abs(full).max()) * (2.0 ** -11 + K * 2.0 ** -24)
+    y = got[1:-1].reshape(T, 2 * N)
+    assert Hn.max_abs(y[:, 1::2], full) <= bound and np.all(y[:, ::2] == 0)
+    assert np.isnan(got[0]) and np.isnan(got[-1])
