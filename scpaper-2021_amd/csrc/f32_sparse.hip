@@ -44,10 +44,39 @@ __device__ __forceinline__ void store_cell_f32(float *Y, const float *bias, f4 a
 // ---- 16x16 tiles ----------------------------------------------------------------
 // Tile t of a block-row: A = its 16 x 16 weights (row = feature), B = X[16 tokens][16 col_idx[t] ..], four products of 32
 // cycles.  A verification batch has few (block-row, 16 tokens) pairs with a chain of loads and products each, so what
-// bounds it is the length of that chain; with many pairs it is the reads of X (below).  Two forms: one, for many pairs, with
-// the tokens' rows in LDS; one that reads them from memory.  Against the former kernel (a wave per block-row and 32 or
-// 64 tokens, nothing requested ahead), us, at 80 %: 256 tokens 768 -> 2304 10.7 -> 8.3, 768 -> 3072 11.6 -> 8.7, 3072 -> 768
-// 21.5 -> 8.3; 16 tokens 6.2 -> 4.0 and 14.7 -> 4.8; 4096 tokens 95 -> 69 and 129 -> 105.
+// bounds it is the length of that chain; with many pairs it is the reads of X and of the weights.  Three forms: one that
+// keeps pairs short, one for many pairs with the tokens' rows in LDS, and one for many pairs of an input too wide for
+// that, in which a wave multiplies a tile with several blocks of 16 tokens.
+//
+// The wide form: a wave has one block-row and MT blocks of 16 tokens; the four waves of a workgroup take neighbouring
+// block-rows over the same tokens and meet in the cache.
+template <int MT> __global__ __launch_bounds__(256) void bsr16_linear_wide_f32_kernel(const Bsr32Args a) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, q = lane >> 4;
+    const int br = blockIdx.x * 4 + wave, tok0 = (blockIdx.y + blockIdx.z * gridDim.y) * (MT * 16);
+    if (br >= (a.out >> 4) || tok0 >= a.T) return;  // no barrier below
+    const float *xrow[MT];
+    f4 acc[MT];
+#pragma unroll
+    for (int m = 0; m < MT; m++) {  // rows past the end: the last one, not stored
+        xrow[m] = a.X + (size_t)min(tok0 + m * 16 + r16, a.T - 1) * a.in + 4 * q;
+        acc[m] = f4{0.f, 0.f, 0.f, 0.f};
+    }
+    const int ts = a.row_ptr[br], te = a.row_ptr[br + 1];
+    const float *wp = a.tiles + (size_t)ts * 256 + r16 * 16 + 4 * q;
+#pragma unroll 2
+    for (int t = ts; t < te; t++, wp += 256) {
+        const int c = a.col_idx[t];
+        const float4 w = *reinterpret_cast<const float4 *>(wp);
+#pragma unroll
+        for (int m = 0; m < MT; m++) acc[m] = mfma_cell_f32(w, *reinterpret_cast<const float4 *>(xrow[m] + c * 16), acc[m]);
+    }
+#pragma unroll
+    for (int m = 0; m < MT; m++) store_cell_f32(a.Y, a.bias, acc[m], tok0 + m * 16 + r16, a.T, a.out, br * 16 + 4 * q, a.act);
+}
+
+// The short form, for few pairs.  Against the wide one, us, at 80 %: 256 tokens 768 -> 2304 8.0 / 10.4, 768 -> 3072 8.4 / 11.0,
+// 3072 -> 768 8.9 / 21.5; 16 tokens 4.0 / 6.2 and 4.8 / 14.7.
 //
 // The waves of a workgroup share one (block-row, 16 tokens), each every WAVES-th tile; the sums meet in LDS and are added
 // in the order of the waves.  A lane reads the column index of one of its wave's tiles, 64 at a time, so no operand waits
@@ -97,8 +126,9 @@ __global__ __launch_bounds__(WAVES * 64) void bsr16_linear_split_f32_kernel(cons
 
 // Eight waves, eight neighbouring block-rows, 16 tokens, whose rows of X lie in LDS (kStripPad floats between two rows:
 // the 16 cells of a fragment read lie in different banks).  Read from memory, the fragment of a tile is 16 rows x 64 bytes,
-// and 16 neighbouring lanes touch 16 lines: with many tiles that is what the kernel above waits for.  The first
-// weights travel while the strip is staged.
+// and 16 neighbouring lanes touch 16 lines: with many tiles that is what the kernels above wait for.  The first
+// weights travel while the strip is staged.  Against the wide form: 4096 tokens 768 -> 3072 at 50 / 80 / 90 / 95 % 116 / 188, 70 / 96,
+// 56 / 56, 51 / 37 (staging a strip for a few tiles; the number of tiles is not known on the host).
 constexpr int kStripPad = 4, kStripWaves = 8;
 __global__ __launch_bounds__(kStripWaves * 64) void bsr16_linear_strip_f32_kernel(const Bsr32Args a) {
     extern __shared__ __align__(16) unsigned char strip_smem[];
@@ -281,6 +311,17 @@ int et_linear_bsr16_f32(const int32_t *row_ptr, const int32_t *col_idx, const fl
         const dim3 grid((out / 16 + kStripWaves - 1) / kStripWaves, gy, (strips + gy - 1) / gy);
         bsr16_linear_strip_f32_kernel<<<grid, kStripWaves * 64, lds, st>>>(a);
         return check_launch("bsr16_linear_strip_f32_kernel");
+    }
+    // Wider than that, the wide form from two of its workgroups a compute unit on: 80 %, us, wide against short: 512 workgroups
+    // 1024 x 4096 -> 1024 40 / 51, 512 x 2048 -> 2048 22 / 31; 768 1024 x 1536 -> 1536 23 / 31, 4096 x 3072 -> 768 99 / 106; 384 2048 x 3072 ->
+    // 768 69 / 54, 512 x 1536 -> 1536 17.1 / 17.2.  (90 % and many rows of a narrow result 1.04 the other way.)
+    const int mt = token_blocks(T), wide_strips = (T + 16 * mt - 1) / (16 * mt), wide_x = (out / 16 + 3) / 4;
+    if (mt > 1 && lds > 80 * 1024 && (long long)wide_x * wide_strips >= 512) {
+        const int wide_y = std::min(wide_strips, 32768);
+        const dim3 grid(wide_x, wide_y, (wide_strips + wide_y - 1) / wide_y);
+        if (mt == 4) bsr16_linear_wide_f32_kernel<4><<<grid, 256, 0, st>>>(a);
+        else bsr16_linear_wide_f32_kernel<2><<<grid, 256, 0, st>>>(a);
+        return check_launch("bsr16_linear_wide_f32_kernel");
     }
     // Two waves a pair below two pairs a compute unit: 192 pairs of 38 tiles 5.2 us against 7.3, 576 pairs of 10 tiles 4.9
     // against 4.7; four waves are no faster.

@@ -208,11 +208,12 @@ def test_linear_bsr16_f32(et, T, inp, out, sp, act):
 
 
 # Both sides of the rule that divides the work: block-rows x 16-token strips below 512, from there to 1536, and above
-# (rows of X in LDS), widths at and past what LDS holds there, rows of more than 64 tiles a wave, block-rows that do not
+# (rows of X in LDS), widths at and past what LDS holds there, past it with several token blocks a wave (two and four), rows of more than 64 tiles a wave, block-rows that do not
 # fill the last workgroup, tokens that do not fill the last strip.
 @pytest.mark.parametrize("T,inp,out,sp,act", [(16, 3072, 768, 0.0, 0), (17, 64, 16 * 255, 0.7, 1), (256, 16, 512, 0.0, 2),
                                               (500, 3072, 96, 0.2, 0), (2001, 1264, 208, 0.8, 2), (2000, 1280, 208, 0.8, 0),
-                                              (1536, 1040, 272, 0.0, 1), (33, 128, 16 * 800, 0.99, 0)])
+                                              (1536, 1040, 272, 0.0, 1), (33, 128, 16 * 800, 0.99, 0),
+                                              (1030, 1296, 1040, 0.95, 0), (2001, 1280, 1040, 0.9, 2)])
 def test_linear_bsr16_f32_division_of_the_work(et, T, inp, out, sp, act):
     test_linear_bsr16_f32(et, T, inp, out, sp, act)
 
