@@ -287,7 +287,10 @@ int et_encoder_chain_status(const uint32_t *sync, int *gave_up, int *misplaced);
  * 1).  x32_out may not overlap x32.  x16 and out16 8-byte aligned, everything else, and the tiles of
  * et_layer_weights, 16-byte aligned; a block-row of more than 510 tiles (columns that occur more than
  * once) has no pack.  Tile order, of T * emdim floats: for 16 tokens after 16 tokens, and 16
- * features after 16 features in them, 256 values: token r, features 4g .. 4g + 3 at 4 (16 g + r). */
+ * features after 16 features in them, 256 values: token r, features 4g .. 4g + 3 at 4 (16 g + r).
+ * et_encoder_layer_project_f16: QKV of x' [T x emdim] as et_encoder_layer_f32 left it in out16, the same
+ * bits as that call left in QKV, for a caller that runs its layers one at a time (packs with parts > 1
+ * and a projection; x16 and QKV 16-byte aligned). */
 struct et_layer_pack_s;
 typedef struct et_layer_weights {
     const int32_t *row_ptr[4], *col_idx[4];
@@ -301,6 +304,7 @@ int et_encoder_layer_pack_destroy(struct et_layer_pack_s *pack);
 int et_encoder_layer_f32(const struct et_layer_pack_s *pack, const et_f16 *Z, const float *x32, const et_f16 *x16,
                          float *x32_out, et_f16 *out16, et_f16 *QKV, float *partial, int act, float eps1, float eps2,
                          et_stream stream);
+int et_encoder_layer_project_f16(const struct et_layer_pack_s *pack, const et_f16 *x16, et_f16 *QKV, et_stream stream);
 
 
 /* SkipLayerNorm fused into the tile-sparse Linear that consumes it:
@@ -848,9 +852,9 @@ typedef struct et_model_desc {
                     * et_model_forward gives the same bits as a chain of et_model_forward_layer.
                     * Where the layers are tile-sparse and it measured faster, 1 runs everything
                     * between two attention kernels in one or two token-local launches
-                    * (et_encoder_layer_f32), and 0 everything from an attention kernel to the end of
-                    * its layer; sums and normalisations inside a launch are binary32, what goes
-                    * from layer to layer is not changed by it */
+                    * (et_encoder_layer_f32), and so does 0, with the QKV projection as a launch of its
+                    * own where they are one; sums and normalisations inside a launch are binary32, what
+                    * goes from layer to layer is not changed by it */
 } et_model_desc;
 
 /* which matrix of a layer */
@@ -897,9 +901,9 @@ int et_model_forward_layer(et_model m, int layer, et_f16 *out, const et_f16 *in,
 int et_model_sync(et_model m);
 /* kernel launches per encoder layer of a finalized model in the form et_model_forward runs
  * (2: attention and one token-local launch, et_encoder_layer_f32, or, under mixed = 3, one chain
- * launch; 3: attention and a token-local launch in two parts; one more than these under mixed = 0,
- * where QKV is a launch of its own; 4 otherwise: the QKV projection inside the attention kernel; 5:
- * SkipLayerNorm folded into the projections; 7: SkipLayerNorm on its own; 0 before et_model_finalize).  A model asked for mixed = 3 reports 5 once it has gone back to separate
+ * launch; 3: attention and a token-local launch in two parts, or, under mixed = 0, QKV, attention and a
+ * token-local launch; 4: the QKV projection inside the attention kernel; 5: SkipLayerNorm folded into
+ * the projections; 7: SkipLayerNorm on its own; 0 before et_model_finalize).  A model asked for mixed = 3 reports 5 once it has gone back to separate
  * launches. */
 int et_model_launches_per_layer(et_model m, int *launches);
 int et_model_destroy(et_model m);

@@ -221,7 +221,8 @@ __device__ __forceinline__ int el_here(int v) {
     return v;
 }
 
-// MODE 0: all steps.  1: up to the second product, binary32 share to `partial`.  2: from the sum of the shares on.
+// MODE 0: all steps.  1: up to the second product, binary32 share to `partial`.  2: from the sum of the shares on.  3: the
+// projection alone, of x' as 2 rounds it, given in `Z`: the same products in the same order.
 // NR: block-rows of the model width a wave holds the sums of.
 template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) __attribute__((amdgpu_num_vgpr(kElOwnVgprs))) void encoder_layer_kernel(const LayerArgs a) {
     extern __shared__ __align__(256) unsigned char el_smem[];
@@ -320,7 +321,9 @@ template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) 
                 }
             }
     };
-    if constexpr (MODE == 2) {
+    if constexpr (MODE == 3) {
+        ask_vectors();
+    } else if constexpr (MODE == 2) {
         ask_vectors();
         constexpr int kTogether = NR > 3 ? 2 : 4;  // shares requested together
 #pragma unroll
@@ -358,7 +361,7 @@ template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) 
     el_ring_start(lane_off, offs_off, slots, offs);
     asm volatile("s_waitcnt vmcnt(%0)" ::"i"(kElRingAsks) : "memory");  // everything but the ring
     keep_vectors();
-    if constexpr (MODE != 2) keep_residual(V);
+    if constexpr (MODE < 2) keep_residual(V);
     el_tie(tab);
 #pragma unroll
     for (int i = 0; i < kElRowRegs; i++) el_tie(desc[i]);
@@ -466,7 +469,7 @@ template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) 
             }
     };
 
-    const int first_seg = MODE == 2 ? a.nseg_ff : 0, last_seg = a.nseg_ff + (MODE == 1 ? 0 : a.nseg_q);
+    const int first_seg = MODE == 3 ? a.nseg_ff + 1 : MODE == 2 ? a.nseg_ff : 0, last_seg = a.nseg_ff + (MODE == 1 ? 0 : a.nseg_q);
     const int q_first = MODE == 1 ? 0 : (a.Q >> 4) * part / a.parts, q_rows = MODE == 1 ? 0 : (a.Q >> 4) * (part + 1) / a.parts - q_first;
     const int act = a.act;
     int pos = 0;
@@ -482,11 +485,13 @@ template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) 
             const bool hid = (d >> 10) & 1;
             const unsigned ld = hid ? a.hs : a.xs;
             const unsigned base = (hid ? MT * 16 * a.xs + hb_dn : 0u) + (unsigned)el_here(lane & 15) * ld, step = 16 * ld;
-            if (kind == kElKindSum) {
+            if constexpr (MODE != 3) {
+                if (kind == kElKindSum) {
 #pragma unroll
-                for (int j = 0; j < NR; j++)
-                    if (target == j) el_row<MT>(V[j], n, pos, base, step, kx, lane_off, offs_off, slots, offs);
-                continue;
+                    for (int j = 0; j < NR; j++)
+                        if (target == j) el_row<MT>(V[j], n, pos, base, step, kx, lane_off, offs_off, slots, offs);
+                    continue;
+                }
             }
             const h4 bv = *reinterpret_cast<const h4 *>(vec + bias_at + el_here(lane >> 4) * 4);
             f4 acc[MT];
@@ -513,8 +518,8 @@ template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) 
                 *reinterpret_cast<h4 *>(Hb + hb_up + (m * 16 + r16) * a.hs + ((u ^ r16) << 4) + gbit * 8) =
                     h4{(_Float16)acc[m][0], (_Float16)acc[m][1], (_Float16)acc[m][2], (_Float16)acc[m][3]};
         }
-        const bool first = MODE != 2 && seg == 0;
-        if (first || (MODE != 1 && seg == a.nseg_ff)) {
+        const bool first = MODE < 2 && seg == 0;
+        if (first || ((MODE == 0 || MODE == 2) && seg == a.nseg_ff)) {
             norm(first ? bo : nullptr, first ? g1 : g2, first ? be1 : be2, first ? a.eps1 : a.eps2);
             if (first) {
                 if (MODE == 1 && part != 0) {
@@ -907,6 +912,41 @@ template <int MT, int MODE> static int el_dispatch(const LayerArgs &a, const et_
 }
 }  // namespace et
 
+// the arguments a pack gives, and those of the second launch of a pack of several parts
+static LayerArgs el_args(const et_layer_pack_s &p) {
+    LayerArgs a{};
+    a.slots = static_cast<const char *>(p.slots);
+    a.offs = static_cast<const char *>(p.offs);
+    a.rows = static_cast<const uint32_t *>(p.rows);
+    a.tab = static_cast<const int32_t *>(p.tab);
+    a.vec = static_cast<const _Float16 *>(p.vec);
+    a.cap = p.cap;
+    std::copy(p.sums, p.sums + kElWaves, a.sums);
+    a.T = p.T, a.H = p.H, a.FF = p.FF, a.Q = p.Q;
+    a.xs = p.xs, a.hs = p.hs, a.nseg_ff = p.nseg_ff, a.nseg_q = p.nseg_q, a.hbuf = p.hbuf, a.parts = a.nshare = p.parts;
+    return a;
+}
+static void el_second(LayerArgs &a, const et_layer_pack_s &p) {
+    a.tab += (size_t)p.second * kElTab;
+    a.rows += (size_t)p.second * 64 * kElRowRegs;
+    a.slots += (size_t)p.second * p.cap * 1024;
+    a.offs += (size_t)p.second * p.cap * 4;
+    a.parts = p.Q ? p.parts : 1;  // without a projection only the normalisation is left
+}
+
+extern "C" int et_encoder_layer_project_f16(const struct et_layer_pack_s *p, const et_f16 *x16, et_f16 *QKV, et_stream stream) {
+    ET_REQUIRE(p && x16 && QKV, ET_ERR_INVALID_ARG, "et_encoder_layer_project_f16: NULL pointer");
+    ET_REQUIRE(p->parts > 1 && p->Q > 0, ET_ERR_UNSUPPORTED, "et_encoder_layer_project_f16: the pack has parts=%d qkv_out=%d", p->parts, p->Q);
+    ET_REQUIRE(((reinterpret_cast<uintptr_t>(x16) | reinterpret_cast<uintptr_t>(QKV)) & 15) == 0, ET_ERR_UNSUPPORTED,
+               "et_encoder_layer_project_f16: x16 and QKV must be 16-byte aligned");
+    LayerArgs a = el_args(*p);
+    a.Z = reinterpret_cast<const _Float16 *>(x16);
+    a.qkv = reinterpret_cast<_Float16 *>(QKV);
+    el_second(a, *p);
+    const int strips = p->T / 16;
+    return el_launch<1, 2, 3>(a, p->lds, (strips + 7) / 8 * 8 * a.parts, as_stream(stream));
+}
+
 extern "C" int et_encoder_layer_f32(const struct et_layer_pack_s *p, const et_f16 *Z, const float *x32, const et_f16 *x16, float *x32_out,
                                     et_f16 *out16, et_f16 *QKV, float *partial, int act, float eps1, float eps2, et_stream stream) {
     ET_REQUIRE(p && Z && (x32 || x16) && (p->Q == 0 || QKV) && (p->parts == 1 || partial), ET_ERR_INVALID_ARG,
@@ -919,12 +959,7 @@ extern "C" int et_encoder_layer_f32(const struct et_layer_pack_s *p, const et_f1
     const size_t x32_bytes = (size_t)p->T * p->H * 4;
     ET_REQUIRE(!x32 || !x32_out || at(x32_out) >= at(x32) + x32_bytes || at(x32) >= at(x32_out) + x32_bytes, ET_ERR_INVALID_ARG,
                "et_encoder_layer_f32: x32_out overlaps x32");
-    LayerArgs a{};
-    a.slots = static_cast<const char *>(p->slots);
-    a.offs = static_cast<const char *>(p->offs);
-    a.rows = static_cast<const uint32_t *>(p->rows);
-    a.tab = static_cast<const int32_t *>(p->tab);
-    a.vec = static_cast<const _Float16 *>(p->vec);
+    LayerArgs a = el_args(*p);
     a.Z = reinterpret_cast<const _Float16 *>(Z);
     a.x32 = x32;
     a.x16 = x32 ? nullptr : reinterpret_cast<const _Float16 *>(x16);
@@ -932,20 +967,13 @@ extern "C" int et_encoder_layer_f32(const struct et_layer_pack_s *p, const et_f1
     a.out16 = reinterpret_cast<_Float16 *>(out16);
     a.qkv = reinterpret_cast<_Float16 *>(QKV);
     a.partial = partial;
-    a.cap = p->cap;
-    std::copy(p->sums, p->sums + kElWaves, a.sums);
-    a.T = p->T, a.H = p->H, a.FF = p->FF, a.Q = p->Q;
-    a.xs = p->xs, a.hs = p->hs, a.nseg_ff = p->nseg_ff, a.nseg_q = p->nseg_q, a.hbuf = p->hbuf, a.parts = a.nshare = p->parts, a.act = act;
+    a.act = act;
     a.eps1 = eps1, a.eps2 = eps2;
     const int strips = (p->T + p->mt * 16 - 1) / (p->mt * 16);
     hipStream_t st = as_stream(stream);
     if (p->parts == 1) return p->mt == 2 ? el_dispatch<2, 0>(a, *p, strips, st) : el_dispatch<1, 0>(a, *p, strips, st);
     const int s = el_dispatch<1, 1>(a, *p, (strips + 7) / 8 * 8 * p->parts, st);
     if (s != ET_OK) return s;
-    a.tab += (size_t)p->second * kElTab;
-    a.rows += (size_t)p->second * 64 * kElRowRegs;
-    a.slots += (size_t)p->second * p->cap * 1024;
-    a.offs += (size_t)p->second * p->cap * 4;
-    a.parts = p->Q ? p->parts : 1;  // without a projection only the normalisation is left
+    el_second(a, *p);
     return el_dispatch<1, 2>(a, *p, (strips + 7) / 8 * 8 * a.parts, st);
 }

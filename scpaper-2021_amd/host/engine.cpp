@@ -340,13 +340,19 @@ LocalPlan plan_local(const et_model_s &m, bool fused) {
     const double shared = kib[ET_W_QKV] + kib[ET_W_FF1] + kib[ET_W_FF2], kept = kib[ET_W_O] + shared;
     const double all = (4.0 * d.emdim + 2.0 * d.dimFF) * d.emdim / 512.0;  // KiB of all tiles
     if (d.mixed == 0) {
-        // Three layers, 384 to 1024 wide, time of the separate launches over that of these.  Above 512 rows 1.01 - 1.84 where at
-        // most half of the tiles are kept (an FFN narrower than the model, up to 2048 rows: 0.85 - 1.03 at 40 and 50 % kept,
-        // 0.88 - 1.30 at 20 and 10 %); denser layers, which run dense GEMMs, 0.69 - 1.07, but from 4096 rows on 1.04 - 1.34 up
-        // to 11 KiB a feature.  257 to 512 rows: 1.01 - 1.22 up to 512 wide, 0.86 - 1.08 wider.  Fewer: 0.81 - 1.02.
-        const double most_kept = (d.dimFF >= d.emdim || rows > 2048 ? 0.5 : 0.25) * all;
-        const bool on = rows > 512 ? kept <= most_kept || (rows > 2048 && kept <= 11.0 * d.emdim)
-                                   : rows > 256 && d.emdim <= 512 && kept <= 0.5 * all;
+        // As above under mixed = 0, three layers.  "Light" is up to 11 KiB of tiles a feature, "half" at most half of the tiles
+        // kept (denser layers run dense GEMMs beside).
+        //   above 4096 rows: up to 18 KiB a feature 1.08 - 1.84, 1024 wide unpruned (24) 0.82
+        //   513 to 4096: half 1.08 - 1.64 (an FFN narrower than the model 0.92 - 1.42), denser and light 1.06 - 1.20, else 0.65 - 1.04
+        //   481 to 512: denser and light 1.07, half up to 512 wide 1.09 - 1.13, half and wider 0.77 - 0.99 (narrow FFN to 1.17)
+        //   257 to 480: up to 45 % kept 1.01 - 1.24 (800 wide, 208 hidden 0.94 once), narrow FFN at 50 % 0.92 - 0.99, denser and light
+        //   1.01 - 1.10, else 0.70 - 0.99
+        //   256 and fewer: 0.59 - 1.20, left to the separate launches
+        const bool light = kept <= 11.0 * d.emdim, half = kept <= 0.5 * all;
+        const bool on = rows > 4096  ? kept <= 18.0 * d.emdim
+                        : rows > 512 ? half || light
+                        : rows > 256 ? (light && (!half || d.emdim <= 512)) || (rows <= 480 && kept <= 0.45 * all)
+                                     : false;
         if (!on) return p;
     }
     if (strips > 256) {
@@ -387,7 +393,7 @@ void build_local(et_model_s &m, bool fused) {
     std::vector<std::unique_ptr<et_layer_pack_s, LayerPackDeleter>> packs;
     for (int i = 0; i < n; i++) {
         et_layer_weights w{};
-        const bool project = d.mixed && i + 1 < n;
+        const bool project = (d.mixed || plan.parts > 1) && i + 1 < n;
         if (!m.layers[(size_t)i]->local_weights(w) || (project && !m.layers[(size_t)i + 1]->local_qkv(w))) return;
         et_layer_pack_s *p = nullptr;
         const int s = et_encoder_layer_pack_create(&w, m.rows(), d.emdim, d.dimFF, project ? ldq : 0, plan.mt, plan.parts, &p);
@@ -402,10 +408,10 @@ void build_local(et_model_s &m, bool fused) {
     m.local = std::move(packs);
 }
 
-// The token-local launches read the model's input and write its result eight bytes at a time; at another address (which
+// The token-local launches read and write up to 16 bytes at a time; input and result at another address (which
 // the separate launches take) they pass through buffers of the model: `warm` is free but for the pass that precedes a
 // capture, whose result it is, and layer kRing - 1 comes to its ring slot after the first layer has read the input.
-bool local_aligned(const half *p) { return (reinterpret_cast<std::uintptr_t>(p) & 7) == 0; }
+bool local_aligned(const half *p) { return (reinterpret_cast<std::uintptr_t>(p) & 15) == 0; }
 half *local_input(et_model_s &m, half *in, stream_t stream) {
     if (local_aligned(in)) return in;
     half *staged = m.pp[et_model_s::kRing - 1]->get();
@@ -417,16 +423,22 @@ void local_deliver(et_model_s &m, half *out, const half *from, stream_t stream) 
     if (from != out) etChk(et_memcpy_d2d(out, from, (std::size_t)m.rows() * m.desc.emdim * sizeof(half), stream));
 }
 
-// One layer from binary16 to binary16, as et_model_forward under mixed = 0 chains it and et_model_forward_layer issues it.
-// Token-local launches take the layer's input and leave its result in binary16, and the QKV projection stays a launch of
-// its own, so that a layer does the same whether the one before it ran in the same call or not.
-void run_layer_f16(et_model_s &m, int i, half *out, half *in, stream_t stream) {
+// One layer from binary16 to binary16, as et_model_forward under mixed = 0 chains it (`chained`: behind the layer before it)
+// and et_model_forward_layer issues it.  The token-local launches take the layer's input and leave its result in binary16,
+// and a layer does the same whether the one before it ran in the same call or not: in two parts the launches also leave the
+// next layer's QKV, made from the result as they round it, and a layer that runs alone makes its own with the products of
+// the second of them; in one part QKV is a launch of its own.
+void run_layer_f16(et_model_s &m, int i, half *out, half *in, bool chained, stream_t stream) {
     ILayer &l = *m.layers[(size_t)i];
     if (m.local.empty()) return l.forward(out, in, stream);
-    l.chain_qkv_first(in, stream);
-    l.chain_attention(stream);
+    const bool last = i + 1 == (int)m.layers.size();
+    if (i == 0 || !m.local_partial) l.chain_qkv_first(in, stream);
     half *x = local_input(m, in, stream), *to = local_result(m, out);
-    etChk(et_encoder_layer_f32(m.local[(size_t)i].get(), et::f16(l.z_buffer()), nullptr, et::f16(x), nullptr, et::f16(to), nullptr,
+    if (i > 0 && m.local_partial && !chained)
+        etChk(et_encoder_layer_project_f16(m.local[(size_t)i - 1].get(), et::f16(x), et::f16(l.qkv_buffer()), stream));
+    l.chain_attention(stream);
+    etChk(et_encoder_layer_f32(m.local[(size_t)i].get(), et::f16(l.z_buffer()), nullptr, et::f16(x), nullptr, et::f16(to),
+                               last || !m.local_partial ? nullptr : et::f16(m.layers[(size_t)i + 1]->qkv_buffer()),
                                m.local_partial ? m.local_partial->get() : nullptr, m.desc.act, l.epsilon(0), l.epsilon(1), stream));
     local_deliver(m, out, to, stream);
 }
@@ -481,7 +493,7 @@ void run_layers(et_model_s &m, half *out, half *in, stream_t stream) {
     half *src = in;
     for (int i = 0; i < n; i++) {
         half *dst = (i == n - 1) ? out : m.pp[i % et_model_s::kRing]->get();
-        run_layer_f16(m, i, dst, src, stream);
+        run_layer_f16(m, i, dst, src, true, stream);
         src = dst;
     }
 }
@@ -697,7 +709,7 @@ int et_model_forward_layer(et_model m, int layer, et_f16 *out, const et_f16 *in,
             etChk(et_f16_to_f32(m->pp32[0]->get(), in, (std::size_t)m->rows() * m->desc.emdim, stream));
             m->layers[(size_t)layer]->forward_mixed(nullptr, o, m->pp32[0]->get(), i, stream);
         } else {
-            run_layer_f16(*m, layer, o, i, stream);
+            run_layer_f16(*m, layer, o, i, false, stream);
         }
         return ET_OK;
     });
@@ -762,7 +774,7 @@ int et_model_launches_per_layer(et_model m, int *launches) {
     return guarded([&]() -> int {
         et::require(m != nullptr && launches != nullptr, "et_model_launches_per_layer: NULL argument");
         if (!m->finalized) *launches = 0;
-        else if (!m->local.empty()) *launches = (m->local_partial ? 3 : 2) + (m->desc.mixed == 0);
+        else if (!m->local.empty()) *launches = m->local_partial || m->desc.mixed == 0 ? 3 : 2;
         else *launches = m->chain ? 2 : m->fused_qkv ? 4 : m->split ? 5 : 7;
         return ET_OK;
     });

@@ -111,8 +111,8 @@ def test_stacks_on_token_local_launches(et, H, nh, FF, S, B, sparsity, mixed):
     outs = []
     for use_graph in (True, False):
         m = Hn.build_model(et, layers, S, B, lens=lens, mixed=mixed, use_graph=use_graph)
-        # attention, and the token-local part in one launch or two; all binary16: the QKV projection besides
-        assert m.launches_per_layer() in ((2, 3) if mixed else (3, 4))
+        # attention, and the token-local part in one launch or two; all binary16: in two, or in one with QKV besides
+        assert m.launches_per_layer() in ((2, 3) if mixed else (3,))
         d = et.DeviceBuffer.from_numpy(x)
         o = et.DeviceBuffer.empty(x.shape, np.float16)
         m.forward(o, d)
@@ -217,6 +217,38 @@ def test_token_local_refuses_addresses_and_overlap(et):
     w.tiles[1] = w.tiles[1] + 8
     other = C.c_void_p()
     assert lib.et_encoder_layer_pack_create(C.byref(w), T, H, FF, 0, 1, parts, C.byref(other)) == et.ET_ERR_UNSUPPORTED
+    assert lib.et_encoder_layer_project_f16(pack, x16, Z, None) == et.ET_ERR_UNSUPPORTED  # no projection in the pack
+    assert lib.et_encoder_layer_project_f16(pack, None, Z, None) == et.ET_ERR_INVALID_ARG
+    et.check(lib.et_encoder_layer_pack_destroy(pack))
+
+
+@pytest.mark.parametrize("H,FF,T,parts,sparsity", [(16, 32, 16, 2, 0.0), (48, 80, 48, 3, 0.5), (272, 208, 144, 4, 0.8), (768, 3072, 80, 7, 0.9),
+                                                   (1024, 4096, 32, 12, 0.6)])
+def test_projection_alone_repeats_the_launches(et, H, FF, T, parts, sparsity):
+    """QKV made from the rounded result on its own: the bits the launches of the layer left, and the Linear of that result
+    (as test_token_local_layer bounds it).  One part, and a pack without projection, have no such launch."""
+    lib, w, keep, pack = et.lib(), Weights(), [], C.c_void_p()
+    mats = [Hn.BsrWeight(o, i, sparsity, seed=31 + k, std=0.05, bias_std=0.1) for k, (o, i) in enumerate(((H, H), (FF, H), (H, FF), (3 * H, H)))]
+    for k, m in enumerate(mats):
+        for name, arr in (("row_ptr", m.row_ptr), ("col_idx", m.col_idx), ("tiles", m.tiles), ("bias", m.bias)):
+            keep.append(up(et, arr))
+            getattr(w, name)[k] = keep[-1].ptr
+    for k in range(2):
+        for name, arr in (("gamma", np.ones(H, np.float16)), ("beta", np.zeros(H, np.float16))):
+            keep.append(up(et, arr))
+            getattr(w, name)[k] = keep[-1].ptr
+    et.check(lib.et_encoder_layer_pack_create(C.byref(w), T, H, FF, 3 * H, 1, parts, C.byref(pack)))
+    Z, x = up(et, Hn.randn((T, H), 70)), up(et, Hn.randn((T, H), 71))
+    out, partial = et.DeviceBuffer.empty((T, H), np.float16), et.DeviceBuffer.empty((parts, T, H), np.float32)
+    qkv = [et.DeviceBuffer.from_numpy(np.full((T, 3 * H), np.nan, np.float16)) for _ in range(2)]
+    et.check(lib.et_encoder_layer_f32(pack, Z.ptr, None, x.ptr, None, out.ptr, qkv[0].ptr, partial.ptr, 2, 1e-5, 1e-5, None))
+    et.check(lib.et_encoder_layer_project_f16(pack, out.ptr, qkv[1].ptr, None))
+    assert np.array_equal(qkv[0].numpy(), qkv[1].numpy())
+    want = Hn.f32(out.numpy()) @ Hn.f32(mats[3].dense).T + Hn.f32(mats[3].bias)
+    assert torch.norm(Hn.f32(qkv[1].numpy()) - want) / torch.norm(want) <= 5e-4
+    et.check(lib.et_encoder_layer_pack_destroy(pack))
+    et.check(lib.et_encoder_layer_pack_create(C.byref(w), T, H, FF, 3 * H, 1, 1, C.byref(pack)))
+    assert lib.et_encoder_layer_project_f16(pack, out.ptr, qkv[1].ptr, None) == et.ET_ERR_UNSUPPORTED
     et.check(lib.et_encoder_layer_pack_destroy(pack))
 
 
