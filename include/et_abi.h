@@ -289,8 +289,9 @@ int et_encoder_chain_status(const uint32_t *sync, int *gave_up, int *misplaced);
  * once) has no pack.  Tile order, of T * emdim floats: for 16 tokens after 16 tokens, and 16
  * features after 16 features in them, 256 values: token r, features 4g .. 4g + 3 at 4 (16 g + r).
  * et_encoder_layer_project_f16: QKV of x' [T x emdim] as et_encoder_layer_f32 left it in out16, the same
- * bits as that call left in QKV, for a caller that runs its layers one at a time (packs with parts > 1
- * and a projection; x16 and QKV 16-byte aligned). */
+ * bits as that call left in QKV, for a caller that runs its layers one at a time (packs with a projection
+ * and either parts > 1 or made by et_encoder_layer_pack_create_projecting, which holds it once more
+ * with parts = 1; x16 and QKV 16-byte aligned). */
 struct et_layer_pack_s;
 typedef struct et_layer_weights {
     const int32_t *row_ptr[4], *col_idx[4];
@@ -300,6 +301,8 @@ typedef struct et_layer_weights {
 int et_encoder_layer_supported(int T, int emdim, int dimFF, int qkv_out);
 int et_encoder_layer_pack_create(const et_layer_weights *w, int T, int emdim, int dimFF, int qkv_out, int mt, int parts,
                                  struct et_layer_pack_s **pack);
+int et_encoder_layer_pack_create_projecting(const et_layer_weights *w, int T, int emdim, int dimFF, int qkv_out, int mt,
+                                            int parts, struct et_layer_pack_s **pack);
 int et_encoder_layer_pack_destroy(struct et_layer_pack_s *pack);
 int et_encoder_layer_f32(const struct et_layer_pack_s *pack, const et_f16 *Z, const float *x32, const et_f16 *x16,
                          float *x32_out, et_f16 *out16, et_f16 *QKV, float *partial, int act, float eps1, float eps2,
@@ -852,9 +855,8 @@ typedef struct et_model_desc {
                     * et_model_forward gives the same bits as a chain of et_model_forward_layer.
                     * Where the layers are tile-sparse and it measured faster, 1 runs everything
                     * between two attention kernels in one or two token-local launches
-                    * (et_encoder_layer_f32), and so does 0, with the QKV projection as a launch of its
-                    * own where they are one; sums and normalisations inside a launch are binary32, what
-                    * goes from layer to layer is not changed by it */
+                    * (et_encoder_layer_f32), and so does 0; sums and normalisations inside a launch are
+                    * binary32, what goes from layer to layer is not changed by it */
 } et_model_desc;
 
 /* which matrix of a layer */
@@ -901,9 +903,9 @@ int et_model_forward_layer(et_model m, int layer, et_f16 *out, const et_f16 *in,
 int et_model_sync(et_model m);
 /* kernel launches per encoder layer of a finalized model in the form et_model_forward runs
  * (2: attention and one token-local launch, et_encoder_layer_f32, or, under mixed = 3, one chain
- * launch; 3: attention and a token-local launch in two parts, or, under mixed = 0, QKV, attention and a
- * token-local launch; 4: the QKV projection inside the attention kernel; 5: SkipLayerNorm folded into
- * the projections; 7: SkipLayerNorm on its own; 0 before et_model_finalize).  A model asked for mixed = 3 reports 5 once it has gone back to separate
+ * launch; 3: attention and a token-local launch in two parts; 4: the QKV projection inside the
+ * attention kernel; 5: SkipLayerNorm folded into the projections; 7: SkipLayerNorm on its own; 0 before
+ * et_model_finalize).  A model asked for mixed = 3 reports 5 once it has gone back to separate
  * launches. */
 int et_model_launches_per_layer(et_model m, int *launches);
 int et_model_destroy(et_model m);

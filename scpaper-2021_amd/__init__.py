@@ -83,6 +83,7 @@ _SIGNATURES = {
     "et_encoder_chain_status": (_vp, C.POINTER(_i), C.POINTER(_i)),
     "et_encoder_layer_supported": (_i, _i, _i, _i),
     "et_encoder_layer_pack_create": (_vp, _i, _i, _i, _i, _i, _i, C.POINTER(_vp)),
+    "et_encoder_layer_pack_create_projecting": (_vp, _i, _i, _i, _i, _i, _i, C.POINTER(_vp)),
     "et_encoder_layer_pack_destroy": (_vp,),
     "et_encoder_layer_f32": (_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _f, _f, _vp),
     "et_encoder_layer_project_f16": (_vp, _vp, _vp, _vp),

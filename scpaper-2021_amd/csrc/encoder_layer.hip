@@ -609,7 +609,8 @@ struct et_layer_pack_s {
     int mt = 1, nr = 1, parts = 1, nseg_ff = 0, nseg_q = 0, hbuf = 0, xs = 0, hs = 0;
     size_t lds = 0;
     uint32_t sums[et::kElWaves] = {};
-    int second = 0, cap = 0;  // first stream of the second launch (parts > 1), slots from one stream to the next
+    int second = 0, nstream = 0;  // first stream of the second launch (or of the projection alone), all streams
+    int cap = 0, cap2 = 0;        // slots from one stream to the next, before and from there on
     void *slots = nullptr, *offs = nullptr, *rows = nullptr, *tab = nullptr, *vec = nullptr;
     ~et_layer_pack_s() {
         for (void *p : {slots, offs, rows, tab, vec}) (void)et_free(p);
@@ -656,8 +657,8 @@ int et_encoder_layer_supported(int T, int emdim, int dimFF, int qkv_out) {
            qkv_out >= 0 && qkv_out % 16 == 0 && qkv_out <= 3072;
 }
 
-int et_encoder_layer_pack_create(const et_layer_weights *w, int T, int emdim, int dimFF, int qkv_out, int mt, int parts,
-                                 struct et_layer_pack_s **pack) {
+static int el_pack_create(const et_layer_weights *w, int T, int emdim, int dimFF, int qkv_out, int mt, int parts, bool projecting,
+                          struct et_layer_pack_s **pack) {
     ET_REQUIRE(pack != nullptr && w != nullptr, ET_ERR_INVALID_ARG, "et_encoder_layer_pack_create: NULL pointer");
     *pack = nullptr;
     ET_REQUIRE(et_encoder_layer_supported(T, emdim, dimFF, qkv_out) == 1, ET_ERR_UNSUPPORTED,
@@ -807,33 +808,36 @@ int et_encoder_layer_pack_create(const et_layer_weights *w, int T, int emdim, in
         emit(segs);
     }
     const int second = (int)streams.size();
-    if (parts > 1)
+    if (parts > 1 || (projecting && Q))
         for (int p = 0; p < (Q ? parts : 1); p++) {
             std::vector<std::vector<std::vector<ElRow>>> segs((size_t)nseg, empty());
             if (Q) qkv_segments(segs, p, parts);
             emit(segs);
         }
-    // the streams at one distance from each other, so that a wave finds its own without reading anything; a wave
-    // requests a ring of slots, and two of offsets, past its own
-    size_t cap = 0, most_rows = 0;
-    for (const Stream &st : streams) {
-        cap = std::max(cap, st.order.size() / 2);
-        most_rows = std::max(most_rows, st.rows.size());
+    // the streams of a launch at one distance from each other, so that a wave finds its own without reading anything; a
+    // wave requests a ring of slots, and two of offsets, past its own
+    size_t cap_of[2] = {0, 0}, most_rows = 0;
+    for (size_t i = 0; i < streams.size(); i++) {
+        size_t &cap = cap_of[(int)i >= second];
+        cap = std::max(cap, streams[i].order.size() / 2);
+        most_rows = std::max(most_rows, streams[i].rows.size());
     }
-    cap = (cap + kElRing - 1) / kElRing * kElRing + kElRing;
+    for (size_t &cap : cap_of) cap = (cap + kElRing - 1) / kElRing * kElRing + kElRing;
+    const auto first_slot = [&](size_t i) { return std::min(i, (size_t)second) * cap_of[0] + (i > (size_t)second ? i - (size_t)second : 0) * cap_of[1]; };
+    const size_t all_slots = first_slot(streams.size());
     ET_REQUIRE(most_slots <= kElMaxSlots, ET_ERR_UNSUPPORTED, "et_encoder_layer_pack_create: %d slots in one block-row, at most %d fit its descriptor",
                most_slots, kElMaxSlots);
     ET_REQUIRE(most_rows <= 64 * kElRowRegs, ET_ERR_UNSUPPORTED, "et_encoder_layer_pack_create: %zu block-rows in one wave", most_rows);
-    std::vector<int32_t> tab, order(streams.size() * cap * 2, -1);
+    std::vector<int32_t> tab, order(all_slots * 2, -1);
     std::vector<uint32_t> rows(streams.size() * 64 * kElRowRegs, 0);
-    std::vector<uint16_t> offs((streams.size() * cap + 2 * kElRing) * 2, 0);
+    std::vector<uint16_t> offs((all_slots + 2 * kElRing) * 2, 0);
     for (size_t i = 0; i < streams.size(); i++) {
         const Stream &st = streams[i];
         tab.insert(tab.end(), st.tab.begin(), st.tab.end());
         std::copy(st.rows.begin(), st.rows.end(), rows.begin() + (long)(i * 64 * kElRowRegs));
-        std::copy(st.order.begin(), st.order.end(), order.begin() + (long)(i * cap * 2));
+        std::copy(st.order.begin(), st.order.end(), order.begin() + (long)(first_slot(i) * 2));
         for (size_t k = 0; k < st.offs.size(); k++) {
-            const size_t at = (i * cap + k / kElRing * kElRing) * 2 + k % kElRing;
+            const size_t at = (first_slot(i) + k / kElRing * kElRing) * 2 + k % kElRing;
             offs[at] = (uint16_t)st.offs[k].first;
             offs[at + kElRing] = (uint16_t)st.offs[k].second;
         }
@@ -847,7 +851,8 @@ int et_encoder_layer_pack_create(const et_layer_weights *w, int T, int emdim, in
         for (size_t j = 0; j < sums[(size_t)v].size(); j++)
             p->sums[v] = (p->sums[v] & ~(255u << (8 * j))) | (uint32_t)sums[(size_t)v][j] << (8 * j);
     }
-    p->nseg_ff = nseg_ff, p->nseg_q = nchunk_q, p->hbuf = nbuf == 2 ? mt * 16 * hs : 0, p->xs = xs, p->hs = hs, p->second = second, p->cap = (int)cap;
+    p->nseg_ff = nseg_ff, p->nseg_q = nchunk_q, p->hbuf = nbuf == 2 ? mt * 16 * hs : 0, p->xs = xs, p->hs = hs, p->second = second, p->nstream = (int)streams.size();
+    p->cap = (int)cap_of[0], p->cap2 = (int)cap_of[1];
     p->lds = el_lds(mt, xs, hs, nbuf, H, FF, Q);
     auto upload = [](void **dst, const void *src, size_t bytes) -> int {
         const int st = et_malloc(dst, bytes);
@@ -884,6 +889,16 @@ int et_encoder_layer_pack_create(const et_layer_weights *w, int T, int emdim, in
     return ET_OK;
 }
 
+int et_encoder_layer_pack_create(const et_layer_weights *w, int T, int emdim, int dimFF, int qkv_out, int mt, int parts,
+                                 struct et_layer_pack_s **pack) {
+    return el_pack_create(w, T, emdim, dimFF, qkv_out, mt, parts, false, pack);
+}
+
+int et_encoder_layer_pack_create_projecting(const et_layer_weights *w, int T, int emdim, int dimFF, int qkv_out, int mt, int parts,
+                                            struct et_layer_pack_s **pack) {
+    return el_pack_create(w, T, emdim, dimFF, qkv_out, mt, parts, true, pack);
+}
+
 int et_encoder_layer_pack_destroy(struct et_layer_pack_s *pack) {
     delete pack;
     return ET_OK;
@@ -912,7 +927,7 @@ template <int MT, int MODE> static int el_dispatch(const LayerArgs &a, const et_
 }
 }  // namespace et
 
-// the arguments a pack gives, and those of the second launch of a pack of several parts
+// the arguments a pack gives, and those of its second launch (or of the projection alone)
 static LayerArgs el_args(const et_layer_pack_s &p) {
     LayerArgs a{};
     a.slots = static_cast<const char *>(p.slots);
@@ -931,19 +946,21 @@ static void el_second(LayerArgs &a, const et_layer_pack_s &p) {
     a.rows += (size_t)p.second * 64 * kElRowRegs;
     a.slots += (size_t)p.second * p.cap * 1024;
     a.offs += (size_t)p.second * p.cap * 4;
+    a.cap = p.cap2;
     a.parts = p.Q ? p.parts : 1;  // without a projection only the normalisation is left
 }
 
 extern "C" int et_encoder_layer_project_f16(const struct et_layer_pack_s *p, const et_f16 *x16, et_f16 *QKV, et_stream stream) {
     ET_REQUIRE(p && x16 && QKV, ET_ERR_INVALID_ARG, "et_encoder_layer_project_f16: NULL pointer");
-    ET_REQUIRE(p->parts > 1 && p->Q > 0, ET_ERR_UNSUPPORTED, "et_encoder_layer_project_f16: the pack has parts=%d qkv_out=%d", p->parts, p->Q);
+    ET_REQUIRE(p->Q > 0 && p->nstream > p->second, ET_ERR_UNSUPPORTED,
+               "et_encoder_layer_project_f16: the pack has no projection of its own (parts=%d qkv_out=%d)", p->parts, p->Q);
     ET_REQUIRE(((reinterpret_cast<uintptr_t>(x16) | reinterpret_cast<uintptr_t>(QKV)) & 15) == 0, ET_ERR_UNSUPPORTED,
                "et_encoder_layer_project_f16: x16 and QKV must be 16-byte aligned");
     LayerArgs a = el_args(*p);
     a.Z = reinterpret_cast<const _Float16 *>(x16);
     a.qkv = reinterpret_cast<_Float16 *>(QKV);
     el_second(a, *p);
-    const int strips = p->T / 16;
+    const int strips = p->T / 16;  // one token tile a workgroup, whatever the pack's strips are: the sums are the same
     return el_launch<1, 2, 3>(a, p->lds, (strips + 7) / 8 * 8 * a.parts, as_stream(stream));
 }
 

@@ -326,7 +326,16 @@ struct LocalPlan {
 //   256 rows and fewer, denser than half                  0.75 - 1.04
 //     112 and 128 rows (the separate launches have a strip for each XCD)      0.85 - 1.00, at 95 % sparsity 0.94 - 1.05
 //     up to 48 rows, 144 to 192 (one XCD more than another has two strips)    1.00 - 1.95, measured up to 19 us
-//     others: up to 14.5 us 1.00 - 1.16 (with `fused` above 192 rows 0.94 - 1.02), above 0.91 - 1.04
+//     others: up to 14.5 us 1.00 - 1.16 (with `fused` above 192 rows 0.94 - 1.02; 800 wide, 208 hidden, 256 rows 0.92 at 13.8), above
+//     0.91 - 1.04
+// And under mixed = 0, three layers; "light" is up to 11 KiB of tiles a feature, "half" at most half of the tiles kept (denser
+// layers run dense GEMMs beside):
+//   above 4096 rows: up to 18 KiB a feature 1.07 - 1.98, 1024 wide unpruned (24) 0.78
+//   513 to 4096: half 1.01 - 1.77 (an FFN narrower than the model 0.94 - 1.53), denser and light 1.03 - 1.43 (512 wide unpruned
+//     0.90 at 2048 and 4096), else 0.67 - 1.03
+//   481 to 512: denser and light 1.04 - 1.24, half up to 512 wide 1.05 - 1.20, wider up to 11 us 1.00 - 1.20, above 0.87 - 1.06
+//   257 to 480: up to 45 % kept 1.01 - 1.31 (800 wide, 208 hidden, 40 % kept 0.96 once), denser and light 0.97 - 1.21, else 0.70 - 0.99
+//   256: up to 6 us 1.00 - 1.09, else 0.69 - 1.02; fewer: left to the separate launches
 LocalPlan plan_local(const et_model_s &m, bool fused) {
     LocalPlan p;
     const et_model_desc &d = m.desc;
@@ -339,24 +348,8 @@ LocalPlan plan_local(const et_model_s &m, bool fused) {
     const int rows = m.rows(), strips = (rows + 15) / 16;
     const double shared = kib[ET_W_QKV] + kib[ET_W_FF1] + kib[ET_W_FF2], kept = kib[ET_W_O] + shared;
     const double all = (4.0 * d.emdim + 2.0 * d.dimFF) * d.emdim / 512.0;  // KiB of all tiles
-    if (d.mixed == 0) {
-        // As above under mixed = 0, three layers.  "Light" is up to 11 KiB of tiles a feature, "half" at most half of the tiles
-        // kept (denser layers run dense GEMMs beside).
-        //   above 4096 rows: up to 18 KiB a feature 1.08 - 1.84, 1024 wide unpruned (24) 0.82
-        //   513 to 4096: half 1.08 - 1.64 (an FFN narrower than the model 0.92 - 1.42), denser and light 1.06 - 1.20, else 0.65 - 1.04
-        //   481 to 512: denser and light 1.07, half up to 512 wide 1.09 - 1.13, half and wider 0.77 - 0.99 (narrow FFN to 1.17)
-        //   257 to 480: up to 45 % kept 1.01 - 1.24 (800 wide, 208 hidden 0.94 once), narrow FFN at 50 % 0.92 - 0.99, denser and light
-        //   1.01 - 1.10, else 0.70 - 0.99
-        //   256 and fewer: 0.59 - 1.20, left to the separate launches
-        const bool light = kept <= 11.0 * d.emdim, half = kept <= 0.5 * all;
-        const bool on = rows > 4096  ? kept <= 18.0 * d.emdim
-                        : rows > 512 ? half || light
-                        : rows > 256 ? (light && (!half || d.emdim <= 512)) || (rows <= 480 && kept <= 0.45 * all)
-                                     : false;
-        if (!on) return p;
-    }
     if (strips > 256) {
-        p.mt = 2;
+        if (d.mixed || kept <= 18.0 * d.emdim) p.mt = 2;
         return p;
     }
     double best = 0;
@@ -372,8 +365,13 @@ LocalPlan plan_local(const et_model_s &m, bool fused) {
     // 136 / 149 at 256); without one the single launch is the fastest form (800 wide, 208 hidden features: 171 / 162).
     if (kib[ET_W_FF1] + kib[ET_W_FF2] >= 256.0 && 4 * ((strips + 7) / 8) <= 32) p.parts = std::max(p.parts, 4);
     bool on;
-    if (d.mixed == 0) on = true;
-    else if (kept > 16.5 * d.emdim) on = false;
+    if (d.mixed == 0) {
+        const bool light = kept <= 11.0 * d.emdim, half = kept <= 0.5 * all;
+        if (rows > 512) on = half || light;
+        else if (rows > 480) on = half ? d.emdim <= 512 || best <= 11.0 : light;
+        else if (rows > 256) on = kept <= 0.45 * all || (light && (!half || d.emdim <= 512));
+        else on = rows == 256 && best <= 6.0;
+    } else if (kept > 16.5 * d.emdim) on = false;
     else if (d.emdim <= 512 || rows > 512) on = true;
     else if (rows > 256) on = rows <= 480 || kept > 0.5 * all || best <= 14.5;
     else if (kept > 0.5 * all) on = false;
@@ -393,10 +391,10 @@ void build_local(et_model_s &m, bool fused) {
     std::vector<std::unique_ptr<et_layer_pack_s, LayerPackDeleter>> packs;
     for (int i = 0; i < n; i++) {
         et_layer_weights w{};
-        const bool project = (d.mixed || plan.parts > 1) && i + 1 < n;
-        if (!m.layers[(size_t)i]->local_weights(w) || (project && !m.layers[(size_t)i + 1]->local_qkv(w))) return;
+        if (!m.layers[(size_t)i]->local_weights(w) || (i + 1 < n && !m.layers[(size_t)i + 1]->local_qkv(w))) return;
         et_layer_pack_s *p = nullptr;
-        const int s = et_encoder_layer_pack_create(&w, m.rows(), d.emdim, d.dimFF, project ? ldq : 0, plan.mt, plan.parts, &p);
+        const auto create = d.mixed ? et_encoder_layer_pack_create : et_encoder_layer_pack_create_projecting;
+        const int s = create(&w, m.rows(), d.emdim, d.dimFF, i + 1 < n ? ldq : 0, plan.mt, plan.parts, &p);
         if (s == ET_ERR_UNSUPPORTED) return;
         etChk(s);
         packs.emplace_back(p);
@@ -425,20 +423,18 @@ void local_deliver(et_model_s &m, half *out, const half *from, stream_t stream) 
 
 // One layer from binary16 to binary16, as et_model_forward under mixed = 0 chains it (`chained`: behind the layer before it)
 // and et_model_forward_layer issues it.  The token-local launches take the layer's input and leave its result in binary16,
-// and a layer does the same whether the one before it ran in the same call or not: in two parts the launches also leave the
-// next layer's QKV, made from the result as they round it, and a layer that runs alone makes its own with the products of
-// the second of them; in one part QKV is a launch of its own.
+// and the next layer's QKV made from the result as they round it; a layer that runs alone makes its QKV from its input with
+// the same products, so that it does the same whether the one before it ran in the same call or not.
 void run_layer_f16(et_model_s &m, int i, half *out, half *in, bool chained, stream_t stream) {
     ILayer &l = *m.layers[(size_t)i];
     if (m.local.empty()) return l.forward(out, in, stream);
-    const bool last = i + 1 == (int)m.layers.size();
-    if (i == 0 || !m.local_partial) l.chain_qkv_first(in, stream);
+    if (i == 0) l.chain_qkv_first(in, stream);
     half *x = local_input(m, in, stream), *to = local_result(m, out);
-    if (i > 0 && m.local_partial && !chained)
-        etChk(et_encoder_layer_project_f16(m.local[(size_t)i - 1].get(), et::f16(x), et::f16(l.qkv_buffer()), stream));
+    if (i > 0 && !chained) etChk(et_encoder_layer_project_f16(m.local[(size_t)i - 1].get(), et::f16(x), et::f16(l.qkv_buffer()), stream));
     l.chain_attention(stream);
+    const bool last = i + 1 == (int)m.layers.size();
     etChk(et_encoder_layer_f32(m.local[(size_t)i].get(), et::f16(l.z_buffer()), nullptr, et::f16(x), nullptr, et::f16(to),
-                               last || !m.local_partial ? nullptr : et::f16(m.layers[(size_t)i + 1]->qkv_buffer()),
+                               last ? nullptr : et::f16(m.layers[(size_t)i + 1]->qkv_buffer()),
                                m.local_partial ? m.local_partial->get() : nullptr, m.desc.act, l.epsilon(0), l.epsilon(1), stream));
     local_deliver(m, out, to, stream);
 }
@@ -774,7 +770,7 @@ int et_model_launches_per_layer(et_model m, int *launches) {
     return guarded([&]() -> int {
         et::require(m != nullptr && launches != nullptr, "et_model_launches_per_layer: NULL argument");
         if (!m->finalized) *launches = 0;
-        else if (!m->local.empty()) *launches = m->local_partial || m->desc.mixed == 0 ? 3 : 2;
+        else if (!m->local.empty()) *launches = m->local_partial ? 3 : 2;
         else *launches = m->chain ? 2 : m->fused_qkv ? 4 : m->split ? 5 : 7;
         return ET_OK;
     });

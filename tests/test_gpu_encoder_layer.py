@@ -111,8 +111,7 @@ def test_stacks_on_token_local_launches(et, H, nh, FF, S, B, sparsity, mixed):
     outs = []
     for use_graph in (True, False):
         m = Hn.build_model(et, layers, S, B, lens=lens, mixed=mixed, use_graph=use_graph)
-        # attention, and the token-local part in one launch or two; all binary16: in two, or in one with QKV besides
-        assert m.launches_per_layer() in ((2, 3) if mixed else (3,))
+        assert m.launches_per_layer() in (2, 3)  # attention, and the token-local part in one launch or two
         d = et.DeviceBuffer.from_numpy(x)
         o = et.DeviceBuffer.empty(x.shape, np.float16)
         m.forward(o, d)
@@ -222,11 +221,12 @@ def test_token_local_refuses_addresses_and_overlap(et):
     et.check(lib.et_encoder_layer_pack_destroy(pack))
 
 
-@pytest.mark.parametrize("H,FF,T,parts,sparsity", [(16, 32, 16, 2, 0.0), (48, 80, 48, 3, 0.5), (272, 208, 144, 4, 0.8), (768, 3072, 80, 7, 0.9),
-                                                   (1024, 4096, 32, 12, 0.6)])
-def test_projection_alone_repeats_the_launches(et, H, FF, T, parts, sparsity):
+@pytest.mark.parametrize("H,FF,T,mt,parts,sparsity", [
+    (16, 32, 16, 1, 2, 0.0), (48, 80, 48, 1, 3, 0.5), (272, 208, 144, 1, 4, 0.8), (768, 3072, 80, 1, 7, 0.9), (1024, 4096, 32, 1, 12, 0.6),
+    (48, 32, 48, 2, 1, 0.5), (384, 1536, 64, 1, 1, 0.6), (768, 3072, 80, 2, 1, 0.8), (1024, 4096, 48, 2, 1, 0.9)])
+def test_projection_alone_repeats_the_launches(et, H, FF, T, mt, parts, sparsity):
     """QKV made from the rounded result on its own: the bits the launches of the layer left, and the Linear of that result
-    (as test_token_local_layer bounds it).  One part, and a pack without projection, have no such launch."""
+    (as test_token_local_layer bounds it).  Packs of one part have such a launch only when asked for it."""
     lib, w, keep, pack = et.lib(), Weights(), [], C.c_void_p()
     mats = [Hn.BsrWeight(o, i, sparsity, seed=31 + k, std=0.05, bias_std=0.1) for k, (o, i) in enumerate(((H, H), (FF, H), (H, FF), (3 * H, H)))]
     for k, m in enumerate(mats):
@@ -237,7 +237,7 @@ def test_projection_alone_repeats_the_launches(et, H, FF, T, parts, sparsity):
         for name, arr in (("gamma", np.ones(H, np.float16)), ("beta", np.zeros(H, np.float16))):
             keep.append(up(et, arr))
             getattr(w, name)[k] = keep[-1].ptr
-    et.check(lib.et_encoder_layer_pack_create(C.byref(w), T, H, FF, 3 * H, 1, parts, C.byref(pack)))
+    et.check(lib.et_encoder_layer_pack_create_projecting(C.byref(w), T, H, FF, 3 * H, mt, parts, C.byref(pack)))
     Z, x = up(et, Hn.randn((T, H), 70)), up(et, Hn.randn((T, H), 71))
     out, partial = et.DeviceBuffer.empty((T, H), np.float16), et.DeviceBuffer.empty((parts, T, H), np.float32)
     qkv = [et.DeviceBuffer.from_numpy(np.full((T, 3 * H), np.nan, np.float16)) for _ in range(2)]
@@ -260,7 +260,7 @@ def test_token_local_stack_at_any_address(et, mixed, use_graph):
     H, nh, FF, S, B = 256, 4, 512, 64, 5
     layers = [Hn.LayerWeights(H, nh, FF, 0.7, seed=830 + i) for i in range(5)]
     m = Hn.build_model(et, layers, S, B, mixed=mixed, use_graph=use_graph)
-    assert m.launches_per_layer() == (2 if mixed else 3)
+    assert m.launches_per_layer() == 2
     x = Hn.randn((B * S, H), 831)
     want = et.DeviceBuffer.empty(x.shape, np.float16)
     d = et.DeviceBuffer.from_numpy(x)

@@ -70,7 +70,7 @@ def test_layer_by_layer_equals_stack(et):
     assert Hn.max_abs(full, Hn.oracle_stack(x, layers, B, act="relu")) <= TOL_F16
 
 
-@pytest.mark.parametrize("H,nh,FF,S,B,launches", [(384, 6, 1536, 176, 3, 3), (256, 4, 512, 64, 5, 3), (256, 4, 512, 128, 33, 3),
+@pytest.mark.parametrize("H,nh,FF,S,B,launches", [(384, 6, 1536, 176, 3, 3), (256, 4, 512, 64, 5, 2), (256, 4, 512, 128, 33, 2),
                                                   (768, 12, 512, 112, 2, 7)])
 def test_layer_by_layer_equals_stack_in_every_form(et, H, nh, FF, S, B, launches):
     """All activations binary16 (mixed = 0): the stack and a chain of et_model_forward_layer agree bit for bit on the
@@ -186,7 +186,8 @@ def test_token_local_form_chosen_by_rows_and_tiles(et, H, sparsity, B, S, launch
 
 
 @pytest.mark.parametrize("H,sparsity,B,S,launches", [
-    (768, 0.8, 2, 128, 7), (768, 0.8, 1, 272, 3), (768, 0.8, 1, 496, 7), (768, 0.4, 1, 496, 3), (512, 0.6, 1, 496, 3), (768, 0.4, 3, 176, 3),
+    (768, 0.8, 2, 128, 7), (256, 0.8, 2, 128, 2), (256, 0.8, 1, 240, 7), (768, 0.8, 1, 272, 3), (768, 0.8, 1, 496, 7), (768, 0.95, 1, 496, 3),
+    (768, 0.4, 1, 496, 3), (512, 0.6, 1, 496, 3), (768, 0.4, 3, 176, 3),
     (768, 0.2, 3, 176, 7), (768, 0.6, 3, 176, 3)])
 def test_token_local_form_chosen_under_all_binary16(et, H, sparsity, B, S, launches):
     """The same for mixed = 0, whose lines lie elsewhere."""
