@@ -185,6 +185,50 @@ class Bench:
             et.check(destroy(handle))
         self.record(f"linear_bsr16 ({entry})", f"T{T} in{n_in} out{n_out} sparsity {sparsity}", us, 2 * 256 * ntile * T, "mfma")
 
+    def token_local(self, T, mt, parts, H, FF, launches, nset=12):
+        """What lies between two attention kernels of a tile-sparse layer (et_encoder_layer_f32): at 80 % sparsity, and with
+        no tile in any weight, which is what the launches cost beside them; every launch of a graph on another of `nset`
+        layers with buffers of their own."""
+        et, lib = self.et, self.lib
+
+        class Weights(C.Structure):
+            _fields_ = [(k, C.c_void_p * 4) for k in ("row_ptr", "col_idx", "tiles", "bias")] + [(k, C.c_void_p * 2) for k in ("gamma", "beta")]
+
+        for sparsity in (0.8, 1.0):
+            layers, ntile, i = [], 0, {"i": 0}
+            partial = et.DeviceBuffer.empty((parts, T, H), np.float32)
+            for n in range(nset):
+                w, keep, pack, ntile = Weights(), [], C.c_void_p(), 0
+                for k, (n_out, n_in) in enumerate(((H, H), (FF, H), (H, FF), (3 * H, H))):
+                    if sparsity == 1.0:
+                        row_ptr, col, count = np.zeros(n_out // 16 + 1, np.int32), np.zeros(1, np.int32), 0
+                    else:
+                        row_ptr, col, count = self.tile_pattern(n_out, n_in, sparsity, 80 + 4 * n + k)
+                    ntile += count
+                    arrays = (row_ptr, col, self.rnd((max(count, 1), 256), 0.02), np.zeros(n_out, np.float16))
+                    keep += [self.dev(a) for a in arrays]
+                    for name, a in zip(("row_ptr", "col_idx", "tiles", "bias"), keep[-4:]):
+                        getattr(w, name)[k] = a.ptr
+                for k in range(2):
+                    keep += [self.dev(np.ones(H, np.float16)), self.dev(np.zeros(H, np.float16))]
+                    w.gamma[k], w.beta[k] = keep[-2].ptr, keep[-1].ptr
+                et.check(lib.et_encoder_layer_pack_create(C.byref(w), T, H, FF, 3 * H, mt, parts, C.byref(pack)))
+                x = self.dev(self.rnd((T, H)).astype(np.float32))
+                layers.append((pack, self.dev(self.rnd((T, H))), x, et.DeviceBuffer.empty((T, H), np.float32), self.empty((T, 3 * H))))
+
+            def layer():
+                pack, z, x, out, qkv = layers[i["i"] % nset]
+                i["i"] += 1
+                et.check(lib.et_encoder_layer_f32(pack, z.ptr, x.ptr, None, out.ptr, None, qkv.ptr, partial.ptr, et.ACT_GELU, 1e-5, 1e-5,
+                                                  self.stream))
+
+            us = self.time_us(layer, launches)
+            self.record("encoder_layer" + (" (no tiles)" if sparsity == 1.0 else ""), f"T{T} {H} wide FFN {FF} {16 * mt}-row strips, {parts} parts", us,
+                        2 * 256 * ntile * T, "mfma")
+            et.check(lib.et_stream_sync(self.stream))
+            for l in layers:
+                et.check(lib.et_encoder_layer_pack_destroy(l[0]))
+
     def fuseo(self, B, S, sparsity, launches, nh=12, hd=64, nset=12):
         """Fused attention followed by the tile-sparse output projection: the one launch (et_mha_fuseo_f16, with the
         number of waves picked and forced) against the two launches it replaces (the projection through the plain
@@ -546,7 +590,7 @@ def run_scale(b: Bench):
 
 def main():
     ap = argparse.ArgumentParser()
-    ap.add_argument("--set", choices=("configs", "scale", "vo", "mha", "qkv", "fuseo", "plan", "machine", "all"), default="all")
+    ap.add_argument("--set", choices=("configs", "scale", "vo", "mha", "qkv", "fuseo", "local", "plan", "machine", "all"), default="all")
     ap.add_argument("--json", default=None, help="also write the rows as JSON to this file")
     args = ap.parse_args()
     b = Bench()
@@ -570,6 +614,11 @@ def main():
         for B, S, sp in ((4, 128, 0.8), (8, 128, 0.8), (8, 128, 0.9), (12, 128, 0.8), (16, 128, 0.8), (16, 128, 0.9), (24, 128, 0.8),
                          (32, 128, 0.8), (16, 64, 0.8), (32, 64, 0.8), (64, 32, 0.8)):
             b.qkv_mha(B, S, sp, 48)
+    if args.set == "local":
+        print("# everything between two attention kernels of a layer (binary32 residual), and the same launches without any tile")
+        for T, mt, parts, H, FF in ((128, 1, 4, 768, 3072), (528, 1, 4, 768, 3072), (1024, 1, 4, 768, 3072), (2048, 1, 2, 1024, 4096),
+                                    (4096, 1, 1, 768, 3072), (8192, 2, 1, 768, 3072)):
+            b.token_local(T, mt, parts, H, FF, 48)
     if args.set == "fuseo":
         print("# attention + tile-sparse output projection: one launch against the two it replaces (768-wide, 12 heads of 64)")
         for B, S, sp in ((1, 128, 0.8), (1, 384, 0.8), (2, 128, 0.8), (4, 128, 0.8), (8, 128, 0.8), (8, 128, 0.9), (16, 128, 0.8),
