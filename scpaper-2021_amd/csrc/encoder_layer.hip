@@ -18,18 +18,19 @@
 // Against separate launches per matrix (five to seven a layer) this removes the intermediate activations (at 8192 rows
 // and BERT-base sizes about 300 MB of reads and writes per layer) and the launch boundaries (1.6 us each), and the weight
 // requests never drain: the ring of a wave is filled across barriers, since no weight depends on an activation.
-// 12 layers of BERT-base at 80 %: 64 x 128 tokens 2101 -> 1043 us, 8 x 128 540 -> 474; BERT-large 4 x 512 at 90 % 1842 ->
-// 1401.  On the way: the residual and the shares in tile order instead of rows (lines written in halves by two waves),
+// 12 layers of BERT-base at 80 %: 64 x 128 tokens 2101 -> 1041 us, 8 x 128 540 -> 476; BERT-large 4 x 512 at 90 % 1842 ->
+// 1412.  On the way: the residual and the shares in tile order instead of rows (lines written in halves by two waves),
 // QKV' through LDS as whole rows instead of 32 bytes a token, and the parts of a strip on one XCD: 1150 -> 1060 at 64 x
 // 128, 562 -> 480 at 8 x 128; accumulating in place of a zeroed sum and a later addition: 2 %.
 //
 // Few rows leave most compute units without a strip.  Then PARTS workgroups share a strip in two launches: the first
 // repeats the output projection and LN1, and each part runs its share of the hidden features, leaving its share of
 // the second product in binary32; the second adds the shares in a fixed order, applies LN2 and runs its share of
-// the QKV block-rows.
+// the QKV block-rows.  That projection can be had alone, of x' as it was rounded for it (et_encoder_layer_project_f16), so
+// that a stack whose layers hand binary16 to each other gives the same bits layer by layer.
 //
-// Streams (built on the host, et_encoder_layer_pack_create): per (part, wave) the slots in the order they are
-// multiplied, the byte offsets of their two column tiles in the strip, and a descriptor
+// Streams (built on the host, et_encoder_layer_pack_create; those of the second launch, or of the projection alone, behind
+// those of the first): per (part, wave) the slots in the order they are multiplied, the byte offsets of their two column tiles in the strip, and a descriptor
 // per block-row: slots, kind, where the result goes, where its bias lies.  A segment is what lies between two
 // workgroup barriers: Wo; the first chunk of hidden features; (chunk c + 1 of W1, the columns of chunk c of W2)...; the
 // last columns of W2; Wq.  Hidden chunks alternate between two LDS buffers, so one barrier per chunk is enough.
@@ -84,8 +85,8 @@ struct LayerArgs {
 // the eight after them.  The kernel is compiled for 88 registers, and only the assembly below touches the others, so a
 // request can stay in flight across anything the compiler puts between two block-rows (left to the compiler, the
 // ring was copied between registers at every block-row, in flight or not).  vmcnt counts in order: behind the request of
-// a slot lie seven of later slots and one of offsets (the slot at position 7: seven), so a slot has arrived at vmcnt(8) (7); whatever else the compiler issues
-// in between only makes the wait longer.  The compiler warns that it does not expect assembly to touch registers it was
+// a slot lie seven of later slots and one of offsets (the slot at position 7: seven), so a slot has arrived at vmcnt(8)
+// (7); whatever else the compiler issues in between only makes the wait longer.  The compiler warns that it does not expect assembly to touch registers it was
 // told to leave; what it makes of this file is held to these rules, instruction by instruction, by a test.
 #define ET_EL_CLOBBERS                                                                                                   \
     "v88", "v89", "v90", "v91", "v92", "v93", "v94", "v95", "v96", "v97", "v98", "v99", "v100", "v101", "v102", "v103", \
