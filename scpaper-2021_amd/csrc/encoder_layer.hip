@@ -30,8 +30,8 @@
 // that a stack whose layers hand binary16 to each other gives the same bits layer by layer.
 //
 // Streams (built on the host, et_encoder_layer_pack_create; those of the second launch, or of the projection alone, behind
-// those of the first): per (part, wave) the slots in the order they are multiplied, the byte offsets of their two column tiles in the strip, and a descriptor
-// per block-row: slots, kind, where the result goes, where its bias lies.  A segment is what lies between two
+// those of the first): per (part, wave) the slots in the order they are multiplied, the byte offsets of their two column
+// tiles in the strip, and a descriptor per block-row: slots, kind, where the result goes, where its bias lies.  A segment is what lies between two
 // workgroup barriers: Wo; the first chunk of hidden features; (chunk c + 1 of W1, the columns of chunk c of W2)...; the
 // last columns of W2; Wq.  Hidden chunks alternate between two LDS buffers, so one barrier per chunk is enough.
 // Block-rows are dealt to the waves longest first, within a segment.
@@ -86,8 +86,9 @@ struct LayerArgs {
 // request can stay in flight across anything the compiler puts between two block-rows (left to the compiler, the
 // ring was copied between registers at every block-row, in flight or not).  vmcnt counts in order: behind the request of
 // a slot lie seven of later slots and one of offsets (the slot at position 7: seven), so a slot has arrived at vmcnt(8)
-// (7); whatever else the compiler issues in between only makes the wait longer.  The compiler warns that it does not expect assembly to touch registers it was
-// told to leave; what it makes of this file is held to these rules, instruction by instruction, by a test.
+// (7); whatever else the compiler issues in between only makes the wait longer.  The compiler warns that it does not
+// expect assembly to touch registers it was told to leave; what it makes of this file is held to these rules, instruction
+// by instruction, by a test.
 #define ET_EL_CLOBBERS                                                                                                   \
     "v88", "v89", "v90", "v91", "v92", "v93", "v94", "v95", "v96", "v97", "v98", "v99", "v100", "v101", "v102", "v103", \
         "v104", "v105", "v106", "v107", "v108", "v109", "v110", "v111", "v112", "v113", "v114", "v115", "v116", "v117",  \
@@ -824,10 +825,13 @@ static int el_pack_create(const et_layer_weights *w, int T, int emdim, int dimFF
         most_rows = std::max(most_rows, streams[i].rows.size());
     }
     for (size_t &cap : cap_of) cap = (cap + kElRing - 1) / kElRing * kElRing + kElRing;
-    const auto first_slot = [&](size_t i) { return std::min(i, (size_t)second) * cap_of[0] + (i > (size_t)second ? i - (size_t)second : 0) * cap_of[1]; };
+    const auto first_slot = [&](size_t i) {
+        const size_t ahead = std::min(i, (size_t)second);
+        return ahead * cap_of[0] + (i - ahead) * cap_of[1];
+    };
     const size_t all_slots = first_slot(streams.size());
-    ET_REQUIRE(most_slots <= kElMaxSlots, ET_ERR_UNSUPPORTED, "et_encoder_layer_pack_create: %d slots in one block-row, at most %d fit its descriptor",
-               most_slots, kElMaxSlots);
+    ET_REQUIRE(most_slots <= kElMaxSlots, ET_ERR_UNSUPPORTED,
+               "et_encoder_layer_pack_create: %d slots in one block-row, at most %d fit its descriptor", most_slots, kElMaxSlots);
     ET_REQUIRE(most_rows <= 64 * kElRowRegs, ET_ERR_UNSUPPORTED, "et_encoder_layer_pack_create: %zu block-rows in one wave", most_rows);
     std::vector<int32_t> tab, order(all_slots * 2, -1);
     std::vector<uint32_t> rows(streams.size() * 64 * kElRowRegs, 0);
@@ -852,7 +856,8 @@ static int el_pack_create(const et_layer_weights *w, int T, int emdim, int dimFF
         for (size_t j = 0; j < sums[(size_t)v].size(); j++)
             p->sums[v] = (p->sums[v] & ~(255u << (8 * j))) | (uint32_t)sums[(size_t)v][j] << (8 * j);
     }
-    p->nseg_ff = nseg_ff, p->nseg_q = nchunk_q, p->hbuf = nbuf == 2 ? mt * 16 * hs : 0, p->xs = xs, p->hs = hs, p->second = second, p->nstream = (int)streams.size();
+    p->nseg_ff = nseg_ff, p->nseg_q = nchunk_q, p->hbuf = nbuf == 2 ? mt * 16 * hs : 0, p->xs = xs, p->hs = hs;
+    p->second = second, p->nstream = (int)streams.size();
     p->cap = (int)cap_of[0], p->cap2 = (int)cap_of[1];
     p->lds = el_lds(mt, xs, hs, nbuf, H, FF, Q);
     auto upload = [](void **dst, const void *src, size_t bytes) -> int {

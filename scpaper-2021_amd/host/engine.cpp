@@ -36,6 +36,8 @@ struct ILayer {
     virtual bool local_qkv(et_layer_weights &w) = 0;
     virtual half *qkv_buffer() = 0;
     virtual half *z_buffer() = 0;
+    virtual half *spare_in() = 0;   // [rows x emdim] each, buffers of the separate launches
+    virtual half *spare_out() = 0;
     virtual float epsilon(int k) const = 0;
 };
 
@@ -66,6 +68,8 @@ template <typename EncoderT> struct LayerOf final : ILayer {
     bool local_qkv(et_layer_weights &w) override { return enc->local_qkv(w); }
     half *qkv_buffer() override { return enc->qkv_buffer(); }
     half *z_buffer() override { return enc->z_buffer(); }
+    half *spare_in() override { return enc->temp_attn.get(); }
+    half *spare_out() override { return enc->temp_ffn.get(); }
     float epsilon(int k) const override { return enc->epsilon(k); }
 };
 struct LayerPackDeleter {
@@ -115,9 +119,13 @@ struct et_model_s {
     std::vector<et_chain_desc> chain_desc;
     std::unique_ptr<et::DeviceBuffer<int>> chain_sync;
     // everything between two attention kernels in one token-local launch (et_encoder_layer_f32), or in two with
-    // several workgroups to a token strip: one pack per layer, the residual between layers, the shares of a strip
+    // several workgroups to a token strip: one pack per layer, the residual between layers, the shares of a strip.  mixed =
+    // 0: shares for every layer, which may run on streams of their own (et_model_forward_layer); a whole forward keeps to
+    // the first, which stays in the caches (six layers of 768, 528 rows: 309 us, 318 with a buffer a layer)
     std::vector<std::unique_ptr<et_layer_pack_s, LayerPackDeleter>> local;
-    std::unique_ptr<et::DeviceBuffer<float>> local_x[2], local_partial;
+    std::unique_ptr<et::DeviceBuffer<float>> local_x[2];
+    std::vector<std::unique_ptr<et::DeviceBuffer<float>>> local_shares;
+    float *shares(int layer) const { return local_shares.empty() ? nullptr : local_shares[(size_t)layer]->get(); }
 
     stream_t own_stream = nullptr;
     et_graph graph = nullptr;
@@ -402,47 +410,47 @@ void build_local(et_model_s &m, bool fused) {
     const size_t elems = (size_t)m.rows() * d.emdim;
     if (d.mixed)
         for (auto &b : m.local_x) b = std::make_unique<et::DeviceBuffer<float>>(elems);
-    if (plan.parts > 1) m.local_partial = std::make_unique<et::DeviceBuffer<float>>(elems * plan.parts);
+    if (plan.parts > 1)
+        for (int i = 0; i < (d.mixed ? 1 : n); i++) m.local_shares.push_back(std::make_unique<et::DeviceBuffer<float>>(elems * plan.parts));
     m.local = std::move(packs);
 }
 
-// The token-local launches read and write up to 16 bytes at a time; input and result at another address (which
-// the separate launches take) they pass through buffers of the model: `warm` is free but for the pass that precedes a
-// capture, whose result it is, and layer kRing - 1 comes to its ring slot after the first layer has read the input.
+// The token-local launches read and write up to 16 bytes at a time; input and result at another address (which the
+// separate launches take) pass through buffers of the layer that these launches leave alone.
 bool local_aligned(const half *p) { return (reinterpret_cast<std::uintptr_t>(p) & 15) == 0; }
-half *local_input(et_model_s &m, half *in, stream_t stream) {
+void copy_rows(et_model_s &m, half *to, const half *from, stream_t stream) {
+    etChk(et_memcpy_d2d(to, from, (std::size_t)m.rows() * m.desc.emdim * sizeof(half), stream));
+}
+half *local_input(et_model_s &m, ILayer &l, half *in, stream_t stream) {
     if (local_aligned(in)) return in;
-    half *staged = m.pp[et_model_s::kRing - 1]->get();
-    etChk(et_memcpy_d2d(staged, in, (std::size_t)m.rows() * m.desc.emdim * sizeof(half), stream));
-    return staged;
+    copy_rows(m, l.spare_in(), in, stream);
+    return l.spare_in();
 }
-half *local_result(et_model_s &m, half *out) { return local_aligned(out) ? out : m.warm->get(); }
-void local_deliver(et_model_s &m, half *out, const half *from, stream_t stream) {
-    if (from != out) etChk(et_memcpy_d2d(out, from, (std::size_t)m.rows() * m.desc.emdim * sizeof(half), stream));
-}
+half *local_result(ILayer &l, half *out) { return local_aligned(out) ? out : l.spare_out(); }
 
 // One layer from binary16 to binary16, as et_model_forward under mixed = 0 chains it (`chained`: behind the layer before it)
 // and et_model_forward_layer issues it.  The token-local launches take the layer's input and leave its result in binary16,
 // and the next layer's QKV made from the result as they round it; a layer that runs alone makes its QKV from its input with
-// the same products, so that it does the same whether the one before it ran in the same call or not.
+// the same products, so that it does the same whether the one before it ran in the same call or not, and leaves the next
+// one's where its own was read: it touches no buffer of another layer.
 void run_layer_f16(et_model_s &m, int i, half *out, half *in, bool chained, stream_t stream) {
     ILayer &l = *m.layers[(size_t)i];
     if (m.local.empty()) return l.forward(out, in, stream);
     if (i == 0) l.chain_qkv_first(in, stream);
-    half *x = local_input(m, in, stream), *to = local_result(m, out);
+    half *x = local_input(m, l, in, stream), *to = local_result(l, out);
     if (i > 0 && !chained) etChk(et_encoder_layer_project_f16(m.local[(size_t)i - 1].get(), et::f16(x), et::f16(l.qkv_buffer()), stream));
     l.chain_attention(stream);
     const bool last = i + 1 == (int)m.layers.size();
-    etChk(et_encoder_layer_f32(m.local[(size_t)i].get(), et::f16(l.z_buffer()), nullptr, et::f16(x), nullptr, et::f16(to),
-                               last ? nullptr : et::f16(m.layers[(size_t)i + 1]->qkv_buffer()),
-                               m.local_partial ? m.local_partial->get() : nullptr, m.desc.act, l.epsilon(0), l.epsilon(1), stream));
-    local_deliver(m, out, to, stream);
+    half *qkv = last ? nullptr : chained ? m.layers[(size_t)i + 1]->qkv_buffer() : l.qkv_buffer();
+    etChk(et_encoder_layer_f32(m.local[(size_t)i].get(), et::f16(l.z_buffer()), nullptr, et::f16(x), nullptr, et::f16(to), et::f16(qkv),
+                               m.shares(chained ? 0 : i), m.desc.act, l.epsilon(0), l.epsilon(1), stream));
+    if (to != out) copy_rows(m, out, to, stream);
 }
 
 void run_layers_local(et_model_s &m, half *out, half *in, stream_t stream) {
     const int n = (int)m.layers.size();
     m.layers[0]->chain_qkv_first(in, stream);
-    half *x = local_input(m, in, stream), *to = local_result(m, out);
+    half *x = local_input(m, *m.layers[0], in, stream), *to = local_result(*m.layers[(size_t)n - 1], out);
     for (int i = 0; i < n; i++) {
         ILayer &l = *m.layers[(size_t)i];
         const bool last = i == n - 1;
@@ -450,9 +458,9 @@ void run_layers_local(et_model_s &m, half *out, half *in, stream_t stream) {
         etChk(et_encoder_layer_f32(m.local[(size_t)i].get(), et::f16(l.z_buffer()), i ? m.local_x[(i - 1) & 1]->get() : nullptr,
                                    i ? nullptr : et::f16(x), last ? nullptr : m.local_x[i & 1]->get(), last ? et::f16(to) : nullptr,
                                    last ? nullptr : et::f16(m.layers[(size_t)i + 1]->qkv_buffer()),
-                                   m.local_partial ? m.local_partial->get() : nullptr, m.desc.act, l.epsilon(0), l.epsilon(1), stream));
+                                   m.shares(0), m.desc.act, l.epsilon(0), l.epsilon(1), stream));
     }
-    local_deliver(m, out, to, stream);
+    if (to != out) copy_rows(m, out, to, stream);
 }
 
 void run_layers_split(et_model_s &m, half *out, half *in, stream_t stream) {
@@ -770,7 +778,7 @@ int et_model_launches_per_layer(et_model m, int *launches) {
     return guarded([&]() -> int {
         et::require(m != nullptr && launches != nullptr, "et_model_launches_per_layer: NULL argument");
         if (!m->finalized) *launches = 0;
-        else if (!m->local.empty()) *launches = m->local_partial ? 3 : 2;
+        else if (!m->local.empty()) *launches = m->local_shares.empty() ? 2 : 3;
         else *launches = m->chain ? 2 : m->fused_qkv ? 4 : m->split ? 5 : 7;
         return ET_OK;
     });

@@ -1,5 +1,7 @@
 """GPU parity of the encoder-stack handle (et_model_*), i.e. of the C++ class layer
 (Linear / Attention / SkipLayerNorm / Encoder) it is built from, against the CPU oracle."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -87,6 +89,40 @@ def test_layer_by_layer_equals_stack_in_every_form(et, H, nh, FF, S, B, launches
     et.sync()
     assert np.array_equal(full, bufs[1].numpy(np.float16, (B * S, H)))
     assert Hn.max_abs(full, Hn.oracle_stack(x, layers, B, act="relu")) <= TOL_F16
+
+
+@pytest.mark.parametrize("H,nh,FF,S,B,launches", [(384, 6, 1536, 176, 3, 3), (256, 4, 512, 64, 5, 2), (256, 4, 512, 32, 2, 7)])
+def test_layers_of_one_model_on_streams_of_their_own(et, H, nh, FF, S, B, launches):
+    """mixed = 0: a layer touches no buffer of another one, so two batches can go through a model one layer apart, each on
+    its stream; addresses off the launches' alignment included."""
+    lib, n = et.lib(), 4
+    layers = [Hn.LayerWeights(H, nh, FF, 0.7, seed=55 + i) for i in range(n)]
+    m = Hn.build_model(et, layers, S, B)
+    assert m.launches_per_layer() == launches
+    inputs = [[et.DeviceBuffer.from_numpy(Hn.randn((B * S, H), 60 + i)) for i in range(n)], []]
+    inputs[1] = [et.DeviceBuffer.from_numpy(np.concatenate([np.zeros(4, np.float16), b.numpy().reshape(-1)])) for b in inputs[0]]
+    want = []
+    for i in range(n):
+        out = et.DeviceBuffer.empty((B * S, H), np.float16)
+        m.forward_layer(i, out, inputs[0][i])
+        et.sync()
+        want.append(out.numpy())
+    streams = [C.c_void_p() for _ in range(n)]
+    for st in streams:
+        et.check(lib.et_stream_create(C.byref(st)))
+    for shift in (0, 8):
+        outs = [et.DeviceBuffer.empty((B * S * H + 8,), np.float16) for _ in range(n)]
+        et.sync()
+        for _ in range(8):
+            for i in range(n):
+                m.forward_layer(i, outs[i].ptr + shift, inputs[shift // 8][i].ptr + shift, streams[i])
+        for st in streams:
+            et.check(lib.et_stream_sync(st))
+        for i in range(n):
+            got = outs[i].numpy()[shift // 2:shift // 2 + B * S * H].reshape(B * S, H)
+            assert np.array_equal(got, want[i]), (shift, i)
+    for st in streams:
+        et.check(lib.et_stream_destroy(st))
 
 
 def headline_layers(seed0):
