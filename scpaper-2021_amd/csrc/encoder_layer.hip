@@ -18,8 +18,8 @@
 // Against separate launches per matrix (five to seven a layer) this removes the intermediate activations (at 8192 rows
 // and BERT-base sizes about 300 MB of reads and writes per layer) and the launch boundaries (1.6 us each), and the weight
 // requests never drain: the ring of a wave is filled across barriers, since no weight depends on an activation.
-// 12 layers of BERT-base at 80 %: 64 x 128 tokens 2101 -> 1041 us, 8 x 128 540 -> 476; BERT-large 4 x 512 at 90 % 1842 ->
-// 1412.  On the way: the residual and the shares in tile order instead of rows (lines written in halves by two waves),
+// 12 layers of BERT-base at 80 %: 64 x 128 tokens 2101 -> 1003 us, 8 x 128 540 -> 457; BERT-large 4 x 512 at 90 % 1842 ->
+// 1355.  On the way: the residual and the shares in tile order instead of rows (lines written in halves by two waves),
 // QKV' through LDS as whole rows instead of 32 bytes a token, and the parts of a strip on one XCD: 1150 -> 1060 at 64 x
 // 128, 562 -> 480 at 8 x 128; accumulating in place of a zeroed sum and a later addition: 2 %.
 //
@@ -51,9 +51,12 @@ constexpr int kElMaxSeg = 24;  // segments of a launch
 constexpr size_t kElLds = 160 * 1024;
 // table of a (part, wave), 64 words, a lane holds one: block-rows of every segment, sums of every wave; and the descriptors
 // of its block-rows, in the same way: one request each at the start, read with v_readlane
-constexpr int kElTabSeg = 0, kElTabCount = kElTabSeg + kElMaxSeg, kElTab = 64, kElRowRegs = 2;
+constexpr int kElTabSeg = 0, kElTabCount = kElTabSeg + kElMaxSeg, kElTabSlots = kElTabCount + kElWaves, kElTab = 64, kElRowRegs = 2;
 // descriptor: slots (bits 0-7), kind (8-9), operand in the hidden chunk (10), target (11-20), bias over 16 (21-31)
+constexpr int kElBufferWord = 0x00020000;  // of a raw buffer resource
 constexpr int kElKindSum = 0, kElKindHidden = 1, kElKindQkv = 2, kElMaxSlots = 255;
+
+typedef int i4 __attribute__((ext_vector_type(4)));
 
 struct LayerArgs {
     const char *slots;
@@ -105,18 +108,18 @@ __device__ __forceinline__ void el_ask_offsets(unsigned offs_off, const char *of
 // fills the ring behind it: `slots` + lane_off and `offs` + offs_off point at the wave's first slot and offsets; both are
 // left behind what was requested
 constexpr int kElRingAsks = kElRing + 1;  // requests of a ring filled
-__device__ __forceinline__ void el_ring_start(unsigned &lane_off, unsigned &offs_off, const char *slots, const char *offs) {
+__device__ __forceinline__ void el_ring_start(unsigned &lane_off, unsigned &offs_off, i4 slots, const char *offs) {
     asm volatile(
-        "global_load_dwordx4 v[96:99], %0, %2\n\t"
-        "global_load_dwordx4 v[100:103], %0, %2 offset:1024\n\t"
-        "global_load_dwordx4 v[104:107], %0, %2 offset:2048\n\t"
-        "global_load_dwordx4 v[108:111], %0, %2 offset:3072\n\t"
+        "buffer_load_dwordx4 v[96:99], %0, %2, 0 offen\n\t"
+        "buffer_load_dwordx4 v[100:103], %0, %2, 0 offen offset:1024\n\t"
+        "buffer_load_dwordx4 v[104:107], %0, %2, 0 offen offset:2048\n\t"
+        "buffer_load_dwordx4 v[108:111], %0, %2, 0 offen offset:3072\n\t"
         "v_add_u32 %0, 0x1000, %0\n\t"
-        "global_load_dwordx4 v[112:115], %0, %2\n\t"
-        "global_load_dwordx4 v[116:119], %0, %2 offset:1024\n\t"
-        "global_load_dwordx4 v[120:123], %0, %2 offset:2048\n\t"
+        "buffer_load_dwordx4 v[112:115], %0, %2, 0 offen\n\t"
+        "buffer_load_dwordx4 v[116:119], %0, %2, 0 offen offset:1024\n\t"
+        "buffer_load_dwordx4 v[120:123], %0, %2, 0 offen offset:2048\n\t"
         "global_load_dwordx4 v[92:95], %1, %3 offset:32\n\t"
-        "global_load_dwordx4 v[124:127], %0, %2 offset:3072\n\t"
+        "buffer_load_dwordx4 v[124:127], %0, %2, 0 offen offset:3072\n\t"
         "v_add_u32 %0, 0x1000, %0\n\t"
         "v_add_u32 %1, 64, %1"
         : "+v"(lane_off), "+v"(offs_off)
@@ -132,7 +135,7 @@ __device__ __forceinline__ void el_ring_start(unsigned &lane_off, unsigned &offs
 #define ET_EL_FRAG2(U, SH, X) ET_EL_FRAG1(U, SH, X) "v_add_u32 %[t], %[t], %[step]\n\tds_read_b128 %[" X "1], %[t]\n\t"
 #define ET_EL_MUL1(W, X, VM, LG) "s_waitcnt vmcnt(" VM ") lgkmcnt(" LG ")\n\tv_mfma_f32_16x16x32_f16 %[a0], v[" W "], %[" X "0], %[a0]\n\t"
 #define ET_EL_MUL2(W, X, VM, LG) ET_EL_MUL1(W, X, VM, LG) "v_mfma_f32_16x16x32_f16 %[a1], v[" W "], %[" X "1], %[a1]\n\t"
-#define ET_EL_REQ(W, OFF, ADV) "global_load_dwordx4 v[" W "], %[lo], %[slots]" OFF "\n\t" ADV
+#define ET_EL_REQ(W, OFF, ADV) "buffer_load_dwordx4 v[" W "], %[lo], %[slots], 0 offen" OFF "\n\t" ADV
 #define ET_EL_ADV "v_add_u32 %[lo], 0x1000, %[lo]\n\t"
 #define ET_EL_NEXT                                                                                       \
     "s_waitcnt vmcnt(7)\n\t"                                                                             \
@@ -178,7 +181,7 @@ __device__ __forceinline__ void el_ring_start(unsigned &lane_off, unsigned &offs
     "el_done%=:\n\ts_nop 15\n\ts_nop 7"  /* the products have left the matrix pipe */
 template <int MT>
 __device__ __forceinline__ void el_row(f4 (&acc)[MT], int n, int &pos, unsigned base, unsigned step, unsigned kx, unsigned &lane_off,
-                                       unsigned &offs_off, const char *slots, const char *offs) {
+                                       unsigned &offs_off, i4 slots, const char *offs) {
     pos = __builtin_amdgcn_readfirstlane(pos);
     unsigned t;
     h8 x0, x1, y0, y1;
@@ -245,7 +248,11 @@ template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) 
 
     // ---- requests: the strip, the vectors, the residual or the shares, all at addresses the arguments give
     const int stream = part * kElWaves + wave;
-    const char *slots = a.slots + (size_t)stream * a.cap * 1024, *offs = a.offs + (size_t)stream * a.cap * 4;  // uniform
+    // A buffer that ends with the wave's last slot: the ring's requests past it go nowhere.  Answered, they were 128 KiB of the
+    // 0.9 MiB a workgroup of the first launch took in at 8 x 128 tokens, and of the 0.6 of the second.
+    const uint64_t slots_at = (uint64_t)(a.slots + (size_t)stream * a.cap * 1024);
+    i4 slots = {(int)(unsigned)slots_at, (int)(unsigned)(slots_at >> 32), a.cap * 1024, kElBufferWord};
+    const char *offs = a.offs + (size_t)stream * a.cap * 4;  // uniform
     unsigned lane_off = lane * 16, offs_off = (g >> 1) * 16;
     el_ask_offsets(offs_off, offs);
     if constexpr (MODE != 2) {
@@ -274,19 +281,11 @@ template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) 
     const int tiles_here = min(MT, (a.T - tok0) >> 4);
     auto tile_at = [&](int m, int j) { return (unsigned)(min(m, tiles_here - 1) * H + max(rb[j], 0) * 16) * 64; };
 
-    constexpr int kVecLoads = 2;  // 8 values a thread and load: up to 16384 in all
-    h8 vl[kVecLoads];
-    const int nvec = (6 * H + a.FF + (MODE == 1 ? 0 : a.Q)) >> 3;
-    auto ask_vectors = [&] {
-#pragma unroll
-        for (int i = 0; i < kVecLoads; i++) el_ask(vl[i], (unsigned)min((int)threadIdx.x + i * kElWaves * 64, nvec - 1) * 16, a.vec);
-    };
-    auto keep_vectors = [&] {
-#pragma unroll
-        for (int i = 0; i < kVecLoads; i++) {
-            el_tie(vl[i]);
-            if ((int)threadIdx.x + i * kElWaves * 64 < nvec) reinterpret_cast<h8 *>(vec)[threadIdx.x + i * kElWaves * 64] = vl[i];
-        }
+    auto ask_vectors = [&] {  // straight into LDS, 512 values an instruction
+        const int nvec = (6 * H + a.FF + (MODE == 1 ? 0 : a.Q)) >> 3;
+        const unsigned lds0 = (unsigned)(size_t)((__attribute__((address_space(3))) void *)vec);
+        for (int i = wave * 64; i < nvec; i += kElWaves * 64)
+            if (i + lane < nvec) el_load_to_lds(a.vec, (unsigned)(i + lane) * 16u, lds0 + (unsigned)i * 16u);
     };
     const bool half_in = MODE != 2 && a.x16 != nullptr;  // uniform
     f4 V[NR][MT];
@@ -323,8 +322,17 @@ template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) 
                 }
             }
     };
+    // The ring goes out behind what every wave needs to begin with: 128 KiB of it ahead of a later wave's strip, vectors and
+    // residual would hold up all, since a compute unit takes in 64 bytes a cycle (8 x 128 tokens, 12 layers, weights in the
+    // memory-side cache: 390 -> 382 us).  Ends with everything but the ring there.
+    auto ring_start = [&] {
+        asm volatile("s_barrier" ::: "memory");
+        el_ring_start(lane_off, offs_off, slots, offs);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"i"(kElRingAsks) : "memory");
+    };
     if constexpr (MODE == 3) {
         ask_vectors();
+        ring_start();
     } else if constexpr (MODE == 2) {
         ask_vectors();
         constexpr int kTogether = NR > 3 ? 2 : 4;  // shares requested together
@@ -332,17 +340,24 @@ template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) 
         for (int j = 0; j < NR; j++)
 #pragma unroll
             for (int m = 0; m < MT; m++) V[j][m] = f4{0.f, 0.f, 0.f, 0.f};
-        for (int p = 0; p < a.nshare; p += kTogether) {
-            f4 u[kTogether][NR][MT];
+        f4 u[kTogether][NR][MT];
+        auto ask_shares = [&](int p) {
 #pragma unroll
             for (int q = 0; q < kTogether; q++) {
                 const char *src = reinterpret_cast<const char *>(a.partial + ((size_t)min(p + q, a.nshare - 1) * a.T + tok0) * H);
 #pragma unroll
                 for (int j = 0; j < NR; j++)
 #pragma unroll
-                    for (int m = 0; m < MT; m++)
-                        u[q][j][m] = *reinterpret_cast<const f4 *>(src + (tile_at(m, j) + lane * 16));
+                    for (int m = 0; m < MT; m++) el_ask(u[q][j][m], tile_at(m, j) + lane * 16, src);
             }
+        };
+        auto add_shares = [&](int p) {
+#pragma unroll
+            for (int q = 0; q < kTogether; q++)
+#pragma unroll
+                for (int j = 0; j < NR; j++)
+#pragma unroll
+                    for (int m = 0; m < MT; m++) el_tie(u[q][j][m]);
 #pragma unroll
             for (int q = 0; q < kTogether; q++)
                 if (p + q < a.nshare) {  // uniform
@@ -351,22 +366,26 @@ template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) 
 #pragma unroll
                         for (int m = 0; m < MT; m++) V[j][m] += u[q][j][m];
                 }
+        };
+        int p = 0;
+        for (; p + kTogether < a.nshare; p += kTogether) {
+            ask_shares(p);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            add_shares(p);
         }
-#pragma unroll
-        for (int j = 0; j < NR; j++)
-#pragma unroll
-            for (int m = 0; m < MT; m++) el_tie(V[j][m]);  // the shares are added up by now
+        ask_shares(p);
+        ring_start();
+        add_shares(p);
     } else {
         ask_vectors();
         ask_residual(V);
+        ring_start();
     }
-    el_ring_start(lane_off, offs_off, slots, offs);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(kElRingAsks) : "memory");  // everything but the ring
-    keep_vectors();
     if constexpr (MODE < 2) keep_residual(V);
     el_tie(tab);
 #pragma unroll
     for (int i = 0; i < kElRowRegs; i++) el_tie(desc[i]);
+    slots[2] = __builtin_amdgcn_readlane(tab, kElTabSlots) * 1024;
     el_barrier();
 
     const unsigned kx = (unsigned)((gbit ^ r16) & 15) << 4;
@@ -483,6 +502,11 @@ template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) 
         for (int r = 0; r < nrows; r++) {
             const uint32_t d = (uint32_t)__builtin_amdgcn_readlane(row_no < 64 ? desc[0] : desc[1], row_no & 63);
             row_no++;
+            // A SIMD's oldest wave is served first by the memory pipe, which bounds a segment, and the youngest ones end it
+            // a third later: more rows left go first (390 -> 382 us at 8 x 128, 1026 -> 1003 at 64 x 128).
+            if (nrows - r >= 3) __builtin_amdgcn_s_setprio(3);
+            else if (nrows - r == 2) __builtin_amdgcn_s_setprio(2);
+            else __builtin_amdgcn_s_setprio(1);
             const int n = d & 255, kind = (d >> 8) & 3, target = (d >> 11) & 1023, bias_at = (d >> 21) * 16;
             const bool hid = (d >> 10) & 1;
             const unsigned ld = hid ? a.hs : a.xs;
@@ -762,6 +786,7 @@ static int el_pack_create(const et_layer_weights *w, int T, int emdim, int dimFF
                     }
                 }
             }
+            st.tab[kElTabSlots] = (int32_t)(st.order.size() / 2);
             streams.push_back(std::move(st));
         }
     };
