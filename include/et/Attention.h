@@ -306,15 +306,21 @@ class Attention<_config, std::enable_if_t<_config::isSingleKernel>> : public et:
         mat_z = std::make_unique<ptr_t>(T * model->vdim);
     }
 
+    // Where a call keeps Q/K/V and the attention's result: this object's own buffers, or those of another layer of the same
+    // sizes that does not run at the same time (a stack that hands one layer's result to the next).
+    struct Buffers {
+        half *qkv = nullptr, *z = nullptr;
+    };
+    Buffers buffers() { return {mat_qkv->get(), mat_z->get()}; }
+
     void forward(half *out, half *query, half *key, half *value, et::stream_t stream = nullptr) {
+        forward_in(buffers(), out, query, key, value, stream);
+    }
+    void forward_in(const Buffers &b, half *out, half *query, half *key, half *value, et::stream_t stream = nullptr) {
         et::require(query == key && key == value, "single-projection attention is self-attention");
-        linearQKV->forward(mat_qkv->get(), query, stream);
-        const int ldm = model->kdim * 2 + model->vdim;
-        half *Q = mat_qkv->get();
-        half *K = Q + model->kdim;
-        half *V = K + model->kdim;
-        et::fused_mha(Q, K, V, ldm, ldm, ldm, mat_z->get(), model->vdim, *model, run(stream));
-        linearO->forward(out, mat_z->get(), stream);
+        linearQKV->forward(b.qkv, query, stream);
+        core(b, stream);
+        linearO->forward(out, b.z, stream);
     }
 
     // Split normalisation (mixed-precision layer, tile-sparse projections): the QKV projection
@@ -358,42 +364,43 @@ class Attention<_config, std::enable_if_t<_config::isSingleKernel>> : public et:
     linearO_t &o_linear() { return *linearO; }
     half *qkv_buffer() { return mat_qkv->get(); }
     half *z_buffer() { return mat_z->get(); }
-    void core(et::stream_t stream = nullptr) {
+    void core(et::stream_t stream = nullptr) { core(buffers(), stream); }
+    void core(const Buffers &b, et::stream_t stream = nullptr) {
         const int ldm = model->kdim * 2 + model->vdim;
-        half *Q = mat_qkv->get();
+        half *Q = b.qkv;
         half *K = Q + model->kdim;
         half *V = K + model->kdim;
-        et::fused_mha(Q, K, V, ldm, ldm, ldm, mat_z->get(), model->vdim, *model, run(stream));
+        et::fused_mha(Q, K, V, ldm, ldm, ldm, b.z, model->vdim, *model, run(stream));
     }
     void forward_split(float *v1, float *stats1, int *groups1, float *fin_in, const et::SplitSum *in, const float *x32,
                        half *x16, et::stream_t stream = nullptr) {
+        forward_split_in(buffers(), v1, stats1, groups1, fin_in, in, x32, x16, stream);
+    }
+    void forward_split_in(const Buffers &b, float *v1, float *stats1, int *groups1, float *fin_in, const et::SplitSum *in,
+                          const float *x32, half *x16, et::stream_t stream = nullptr) {
         if constexpr (std::is_same<linearQKV_t, Linear<tile_mat>>::value && std::is_same<linearO_t, Linear<tile_mat>>::value) {
             if (in && fused_qkv_) {
                 const et::AttnRun r = run(stream);
                 const float scale = r.scale != 0.0f ? r.scale : 1.0f / std::sqrt((float)(model->kdim / model->nhead));
-                linearQKV->forward_norm_qkv_mha(mat_z->get(), model->vdim, in->v, in->stats, in->groups, in->gamma, in->beta,
+                linearQKV->forward_norm_qkv_mha(b.z, model->vdim, in->v, in->stats, in->groups, in->gamma, in->beta,
                                                 in->eps, fin_in, r.mask, r.lens, r.batch, model->seq_len, scale,
                                                 r.causal ? ET_MHA_CAUSAL : 0, stream);
             } else {
                 if (in)
-                    linearQKV->forward_norm_f32in(mat_qkv->get(), in->v, in->stats, in->groups, in->gamma, in->beta,
+                    linearQKV->forward_norm_f32in(b.qkv, in->v, in->stats, in->groups, in->gamma, in->beta,
                                                   in->eps, fin_in, nullptr, nullptr, ET_ACT_NONE, stream);
                 else
-                    linearQKV->forward(mat_qkv->get(), x16, stream);
-                const int ldm = model->kdim * 2 + model->vdim;
-                half *Q = mat_qkv->get();
-                half *K = Q + model->kdim;
-                half *V = K + model->kdim;
-                et::fused_mha(Q, K, V, ldm, ldm, ldm, mat_z->get(), model->vdim, *model, run(stream));
+                    linearQKV->forward(b.qkv, x16, stream);
+                core(b, stream);
             }
             if (!in && !x32)  // first layer, residual = the binary16 input itself
-                linearO->forward_resid16_stats_f32(v1, stats1, groups1, mat_z->get(), x16, stream);
+                linearO->forward_resid16_stats_f32(v1, stats1, groups1, b.z, x16, stream);
             else
-                linearO->forward_resid_stats_f32(v1, stats1, groups1, mat_z->get(), in ? in->v : x32,
+                linearO->forward_resid_stats_f32(v1, stats1, groups1, b.z, in ? in->v : x32,
                                                  in ? fin_in : nullptr, in ? in->gamma : nullptr, in ? in->beta : nullptr,
                                                  stream);
         } else {
-            (void)v1; (void)stats1; (void)groups1; (void)fin_in; (void)in; (void)x32; (void)x16; (void)stream;
+            (void)b; (void)v1; (void)stats1; (void)groups1; (void)fin_in; (void)in; (void)x32; (void)x16; (void)stream;
             et::require(false, "Attention: the split normalisation needs tile-sparse projections");
         }
     }
@@ -401,13 +408,13 @@ class Attention<_config, std::enable_if_t<_config::isSingleKernel>> : public et:
     // the same with the output projection stored as binary32 (mixed-precision layer)
     void forward_f32(float *out, half *query, half *key, half *value, half *scratch16,
                      et::stream_t stream = nullptr) {
+        forward_f32_in(buffers(), out, query, key, value, scratch16, stream);
+    }
+    void forward_f32_in(const Buffers &b, float *out, half *query, half *key, half *value, half *scratch16,
+                        et::stream_t stream = nullptr) {
         et::require(query == key && key == value, "single-projection attention is self-attention");
-        linearQKV->forward(mat_qkv->get(), query, stream);
-        const int ldm = model->kdim * 2 + model->vdim;
-        half *Q = mat_qkv->get();
-        half *K = Q + model->kdim;
-        half *V = K + model->kdim;
-        et::fused_mha(Q, K, V, ldm, ldm, ldm, mat_z->get(), model->vdim, *model, run(stream));
-        et::linear_forward_f32(*linearO, out, mat_z->get(), scratch16, stream);
+        linearQKV->forward(b.qkv, query, stream);
+        core(b, stream);
+        et::linear_forward_f32(*linearO, out, b.z, scratch16, stream);
     }
 };

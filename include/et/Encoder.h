@@ -77,6 +77,13 @@ struct ChainParts {
     int act = ET_ACT_NONE;
 };
 
+// Where a forward keeps what it computes on the way.  Null: the layer does not have it (yet).
+struct LayerBuffers {
+    half *qkv = nullptr, *z = nullptr;  // single-projection attention
+    half *attn = nullptr, *LN = nullptr, *linear = nullptr, *ffn = nullptr;
+    float *attn32 = nullptr, *LN32 = nullptr, *ffn32 = nullptr, *stats1 = nullptr, *stats2 = nullptr, *fin_in = nullptr, *fin1 = nullptr;
+};
+
 // The layer body shared by Encoder and Encoder_fuse.
 template <typename attn_t, typename linear1_t, typename linear2_t, typename ACT_OP_t> class EncoderLayer {
   protected:
@@ -141,8 +148,11 @@ template <typename attn_t, typename linear1_t, typename linear2_t, typename ACT_
     bool wide_residual() const { return wide; }
 
     // Every activation stored as binary16, the reference's own arithmetic.
-    void forward_f16(half *out, half *src, stream_t stream = nullptr) {
-        attn->forward(temp_attn.get(), src, src, src, stream);
+    void forward_f16(half *out, half *src, stream_t stream = nullptr) { forward_f16_in(buffers(), out, src, stream); }
+    // (..._in: in the buffers of another layer of the same sizes that does not run at the same time)
+    void forward_f16_in(const LayerBuffers &b, half *out, half *src, stream_t stream = nullptr) {
+        if constexpr (attn_has_split<attn_t>::value) attn->forward_in({b.qkv, b.z}, b.attn, src, src, src, stream);
+        else attn->forward(b.attn, src, src, src, stream);
         bool fused_ln1 = false;
         if constexpr (std::is_same_v<linear1_t, Linear<tile_mat>>) {
             // Up to kFusedLnMaxRows token rows SkipLayerNorm rides in the prologue of the tile-sparse
@@ -150,17 +160,17 @@ template <typename attn_t, typename linear1_t, typename linear2_t, typename ACT_
             // every workgroup of a strip repeating the normalisation costs more than the launch
             // (batch 8: 544 against 534 us, batch 32: 1240 against 1184 us).
             if (rows <= kFusedLnMaxRows) {
-                linear1->forward_skipln_act(temp_linear.get(), temp_LN.get(), temp_attn.get(), src, *LN1,
+                linear1->forward_skipln_act(b.linear, b.LN, b.attn, src, *LN1,
                                             act_code<ACT_OP_t>(), stream);
                 fused_ln1 = true;
             }
         }
         if (!fused_ln1) {
-            LN1->forward(temp_LN.get(), temp_attn.get(), src, rows, stream);
-            linear1->forward_act(temp_linear.get(), temp_LN.get(), act_code<ACT_OP_t>(), stream);
+            LN1->forward(b.LN, b.attn, src, rows, stream);
+            linear1->forward_act(b.linear, b.LN, act_code<ACT_OP_t>(), stream);
         }
-        linear2->forward(temp_ffn.get(), temp_linear.get(), stream);
-        LN2->forward(out, temp_ffn.get(), temp_LN.get(), rows, stream);
+        linear2->forward(b.ffn, b.linear, stream);
+        LN2->forward(out, b.ffn, b.LN, rows, stream);
     }
 
     // Mixed precision.  The residual stream — the layer input, both projections that feed a
@@ -177,12 +187,15 @@ template <typename attn_t, typename linear1_t, typename linear2_t, typename ACT_
         if (!temp_ffn32) temp_ffn32 = std::make_unique<DeviceBuffer<float>>((std::size_t)rows * model->emdim);
     }
     void forward_mixed(float *out32, half *out16, const float *src32, half *src16, stream_t stream = nullptr) {
-        require(temp_attn32 && temp_LN32, "Encoder: call enable_mixed() before forward_mixed()");
-        attn_forward_f32(temp_attn32->get(), src16, stream);
-        LN1->forward_mixed(temp_LN32->get(), temp_LN.get(), temp_attn32->get(), src32, rows, stream);
-        linear1->forward_act(temp_linear.get(), temp_LN.get(), act_code<ACT_OP_t>(), stream);
-        linear_forward_f32(*linear2, temp_ffn32->get(), temp_linear.get(), temp_ffn.get(), stream);
-        LN2->forward_mixed(out32, out16, temp_ffn32->get(), temp_LN32->get(), rows, stream);
+        forward_mixed_in(buffers(), out32, out16, src32, src16, stream);
+    }
+    void forward_mixed_in(const LayerBuffers &b, float *out32, half *out16, const float *src32, half *src16, stream_t stream = nullptr) {
+        require(b.attn32 && b.LN32, "Encoder: call enable_mixed() before forward_mixed()");
+        attn_forward_f32(b, b.attn32, src16, stream);
+        LN1->forward_mixed(b.LN32, b.LN, b.attn32, src32, rows, stream);
+        linear1->forward_act(b.linear, b.LN, act_code<ACT_OP_t>(), stream);
+        linear_forward_f32(*linear2, b.ffn32, b.linear, b.ffn, stream);
+        LN2->forward_mixed(out32, out16, b.ffn32, b.LN32, rows, stream);
     }
 
     // Split normalisation: five launches per layer, no SkipLayerNorm launch and no normalised
@@ -239,11 +252,11 @@ template <typename attn_t, typename linear1_t, typename linear2_t, typename ACT_
                 return false;
             p.qkv = lq.pack_consumer.get();
             p.bias_qkv = lq.bias.get();
-            p.QKV = attn->qkv_buffer();
+            p.QKV = attn->buffers().qkv;
             p.fin_in = fin_in->get();
             p.o = lo.pack_producer.get();
             p.bias_o = lo.bias.get();
-            p.Z = attn->z_buffer();
+            p.Z = attn->buffers().z;
             p.V1 = temp_attn32->get();
             p.stats1 = stats1->get();
             p.up = linear1->pack_consumer.get();
@@ -290,44 +303,56 @@ template <typename attn_t, typename linear1_t, typename linear2_t, typename ACT_
         else (void)w;
         return attn_has_split<attn_t>::value;
     }
-    half *qkv_buffer() {
-        if constexpr (attn_has_split<attn_t>::value) return attn->qkv_buffer();
-        else return nullptr;
+    LayerBuffers buffers() {
+        const auto at = [](auto &p) { return p ? p->get() : nullptr; };
+        LayerBuffers b;
+        if constexpr (attn_has_split<attn_t>::value) {
+            b.qkv = attn->buffers().qkv;
+            b.z = attn->buffers().z;
+        }
+        b.attn = temp_attn.get(), b.LN = temp_LN.get(), b.linear = temp_linear.get(), b.ffn = temp_ffn.get();
+        b.attn32 = at(temp_attn32), b.LN32 = at(temp_LN32), b.ffn32 = at(temp_ffn32);
+        b.stats1 = at(stats1), b.stats2 = at(stats2), b.fin_in = at(fin_in), b.fin1 = at(fin1);
+        return b;
     }
-    half *z_buffer() {
-        if constexpr (attn_has_split<attn_t>::value) return attn->z_buffer();
-        else return nullptr;
-    }
+    half *qkv_buffer() { return buffers().qkv; }
+    half *z_buffer() { return buffers().z; }
     float epsilon(int k) const { return k ? LN2->epsilon() : LN1->epsilon(); }
     // the first layer's QKV projection of the binary16 input, and the attention kernel alone
-    void chain_qkv_first(half *x16, stream_t stream = nullptr) {
-        if constexpr (attn_has_split<attn_t>::value) attn->qkv_linear().forward(attn->qkv_buffer(), x16, stream);
-        else (void)x16, (void)stream;
+    void chain_qkv_first(half *x16, stream_t stream = nullptr) { chain_qkv_first_in(buffers(), x16, stream); }
+    void chain_qkv_first_in(const LayerBuffers &b, half *x16, stream_t stream = nullptr) {
+        if constexpr (attn_has_split<attn_t>::value) attn->qkv_linear().forward(b.qkv, x16, stream);
+        else (void)b, (void)x16, (void)stream;
     }
-    void chain_attention(stream_t stream = nullptr) {
-        if constexpr (attn_has_split<attn_t>::value) attn->core(stream);
-        else (void)stream;
+    void chain_attention(stream_t stream = nullptr) { chain_attention_in(buffers(), stream); }
+    void chain_attention_in(const LayerBuffers &b, stream_t stream = nullptr) {
+        if constexpr (attn_has_split<attn_t>::value) attn->core({b.qkv, b.z}, stream);
+        else (void)b, (void)stream;
     }
+    // (`in` may lie in other buffers than this call's)
     SplitSum forward_split(const SplitSum *in, const float *x32, half *x16, stream_t stream = nullptr) {
+        return forward_split_in(buffers(), in, x32, x16, stream);
+    }
+    SplitSum forward_split_in(const LayerBuffers &b, const SplitSum *in, const float *x32, half *x16, stream_t stream = nullptr) {
         SplitSum out;
         if constexpr (attn_has_split<attn_t>::value && std::is_same_v<linear1_t, Linear<tile_mat>> &&
                       std::is_same_v<linear2_t, Linear<tile_mat>>) {
-            require(stats1 && stats2 && fin_in && fin1, "Encoder: call enable_split() before forward_split()");
+            require(b.stats1 && b.stats2 && b.fin_in && b.fin1, "Encoder: call enable_split() before forward_split()");
             int g1 = 0, g2 = 0;
-            attn->forward_split(temp_attn32->get(), stats1->get(), &g1, fin_in->get(), in, x32, x16, stream);
-            linear1->forward_norm_f32in(temp_linear.get(), temp_attn32->get(), stats1->get(), g1,
-                                        LN1->gamma(), LN1->beta(), LN1->epsilon(), fin1->get(), nullptr, nullptr,
+            attn->forward_split_in({b.qkv, b.z}, b.attn32, b.stats1, &g1, b.fin_in, in, x32, x16, stream);
+            linear1->forward_norm_f32in(b.linear, b.attn32, b.stats1, g1,
+                                        LN1->gamma(), LN1->beta(), LN1->epsilon(), b.fin1, nullptr, nullptr,
                                         act_code<ACT_OP_t>(), stream);
-            linear2->forward_resid_stats_f32(temp_ffn32->get(), stats2->get(), &g2, temp_linear.get(),
-                                             temp_attn32->get(), fin1->get(), LN1->gamma(), LN1->beta(), stream);
-            out.v = temp_ffn32->get();
-            out.stats = stats2->get();
+            linear2->forward_resid_stats_f32(b.ffn32, b.stats2, &g2, b.linear,
+                                             b.attn32, b.fin1, LN1->gamma(), LN1->beta(), stream);
+            out.v = b.ffn32;
+            out.stats = b.stats2;
             out.groups = g2;
             out.gamma = LN2->gamma();
             out.beta = LN2->beta();
             out.eps = LN2->epsilon();
         } else {
-            (void)in; (void)x32; (void)x16; (void)stream;
+            (void)b; (void)in; (void)x32; (void)x16; (void)stream;
             require(false, "Encoder: the split normalisation needs tile-sparse projections");
         }
         return out;
@@ -371,12 +396,14 @@ template <typename attn_t, typename linear1_t, typename linear2_t, typename ACT_
                                static_cast<float *>(nullptr), static_cast<half *>(nullptr),
                                static_cast<half *>(nullptr), static_cast<half *>(nullptr),
                                static_cast<half *>(nullptr), static_cast<stream_t>(nullptr)))>> : std::true_type {};
-    void attn_forward_f32(float *out32, half *src16, stream_t stream) {
-        if constexpr (attn_has_f32<attn_t>::value) {
-            attn->forward_f32(out32, src16, src16, src16, temp_attn.get(), stream);
+    void attn_forward_f32(const LayerBuffers &b, float *out32, half *src16, stream_t stream) {
+        if constexpr (attn_has_split<attn_t>::value) {
+            attn->forward_f32_in({b.qkv, b.z}, out32, src16, src16, src16, b.attn, stream);
+        } else if constexpr (attn_has_f32<attn_t>::value) {
+            attn->forward_f32(out32, src16, src16, src16, b.attn, stream);
         } else {  // attention forms without a binary32 output projection: widen their result
-            attn->forward(temp_attn.get(), src16, src16, src16, stream);
-            etChk(et_f16_to_f32(out32, f16(temp_attn.get()), (std::size_t)rows * model->emdim, stream));
+            attn->forward(b.attn, src16, src16, src16, stream);
+            etChk(et_f16_to_f32(out32, f16(b.attn), (std::size_t)rows * model->emdim, stream));
         }
     }
 };

@@ -18,58 +18,52 @@ using et::stream_t;
 
 struct ILayer {
     virtual ~ILayer() = default;
-    virtual void forward(half *out, half *src, stream_t stream) = 0;
+    virtual et::LayerBuffers buffers() = 0;  // its own; the forwards below are given those they shall use
+    virtual void forward(const et::LayerBuffers &b, half *out, half *src, stream_t stream) = 0;
     virtual void enable_mixed() = 0;
-    virtual void forward_mixed(float *out32, half *out16, const float *src32, half *src16, stream_t stream) = 0;
+    virtual void forward_mixed(const et::LayerBuffers &b, float *out32, half *out16, const float *src32, half *src16, stream_t stream) = 0;
     virtual bool split_ok() const = 0;
     virtual void enable_split() = 0;
     virtual bool enable_fused_qkv(const half *gamma, const half *beta) = 0;
     virtual const half *norm2_gamma() const = 0;
     virtual const half *norm2_beta() const = 0;
-    virtual et::SplitSum forward_split(const et::SplitSum *in, const float *x32, half *x16, stream_t stream) = 0;
+    virtual et::SplitSum forward_split(const et::LayerBuffers &b, const et::SplitSum *in, const float *x32, half *x16, stream_t stream) = 0;
     virtual void finish_split(float *out32, half *out16, const et::SplitSum &s, stream_t stream) = 0;
     virtual bool chain_parts(et::ChainParts &p) = 0;
-    virtual void chain_qkv_first(half *x16, stream_t stream) = 0;
-    virtual void chain_attention(stream_t stream) = 0;
+    virtual void chain_qkv_first(const et::LayerBuffers &b, half *x16, stream_t stream) = 0;
+    virtual void chain_attention(const et::LayerBuffers &b, stream_t stream) = 0;
     virtual et::AttnState &attn() = 0;
     virtual bool local_weights(et_layer_weights &w) = 0;
     virtual bool local_qkv(et_layer_weights &w) = 0;
-    virtual half *qkv_buffer() = 0;
-    virtual half *z_buffer() = 0;
-    virtual half *spare_in() = 0;   // [rows x emdim] each, buffers of the separate launches
-    virtual half *spare_out() = 0;
     virtual float epsilon(int k) const = 0;
 };
 
 template <typename EncoderT> struct LayerOf final : ILayer {
     std::unique_ptr<EncoderT> enc;
     explicit LayerOf(std::unique_ptr<EncoderT> e) : enc(std::move(e)) {}
-    void forward(half *out, half *src, stream_t stream) override { enc->forward_f16(out, src, stream); }
+    et::LayerBuffers buffers() override { return enc->buffers(); }
+    void forward(const et::LayerBuffers &b, half *out, half *src, stream_t stream) override { enc->forward_f16_in(b, out, src, stream); }
     void enable_mixed() override { enc->enable_mixed(); }
-    void forward_mixed(float *out32, half *out16, const float *src32, half *src16, stream_t stream) override {
-        enc->forward_mixed(out32, out16, src32, src16, stream);
+    void forward_mixed(const et::LayerBuffers &b, float *out32, half *out16, const float *src32, half *src16, stream_t stream) override {
+        enc->forward_mixed_in(b, out32, out16, src32, src16, stream);
     }
     bool split_ok() const override { return enc->split_ok(); }
     void enable_split() override { enc->enable_split(); }
     bool enable_fused_qkv(const half *gamma, const half *beta) override { return enc->enable_fused_qkv(gamma, beta); }
     const half *norm2_gamma() const override { return enc->norm2_gamma(); }
     const half *norm2_beta() const override { return enc->norm2_beta(); }
-    et::SplitSum forward_split(const et::SplitSum *in, const float *x32, half *x16, stream_t stream) override {
-        return enc->forward_split(in, x32, x16, stream);
+    et::SplitSum forward_split(const et::LayerBuffers &b, const et::SplitSum *in, const float *x32, half *x16, stream_t stream) override {
+        return enc->forward_split_in(b, in, x32, x16, stream);
     }
     void finish_split(float *out32, half *out16, const et::SplitSum &s, stream_t stream) override {
         enc->finish_split(out32, out16, s, stream);
     }
     bool chain_parts(et::ChainParts &p) override { return enc->chain_parts(p); }
-    void chain_qkv_first(half *x16, stream_t stream) override { enc->chain_qkv_first(x16, stream); }
-    void chain_attention(stream_t stream) override { enc->chain_attention(stream); }
+    void chain_qkv_first(const et::LayerBuffers &b, half *x16, stream_t stream) override { enc->chain_qkv_first_in(b, x16, stream); }
+    void chain_attention(const et::LayerBuffers &b, stream_t stream) override { enc->chain_attention_in(b, stream); }
     et::AttnState &attn() override { return enc->attention(); }
     bool local_weights(et_layer_weights &w) override { return enc->local_weights(w); }
     bool local_qkv(et_layer_weights &w) override { return enc->local_qkv(w); }
-    half *qkv_buffer() override { return enc->qkv_buffer(); }
-    half *z_buffer() override { return enc->z_buffer(); }
-    half *spare_in() override { return enc->temp_attn.get(); }
-    half *spare_out() override { return enc->temp_ffn.get(); }
     float epsilon(int k) const override { return enc->epsilon(k); }
 };
 struct LayerPackDeleter {
@@ -141,6 +135,12 @@ struct et_model_s {
             default: return {desc.emdim, desc.dimFF};
         }
     }
+    // The buffers layer i runs in as part of et_model_forward.  A whole forward keeps to those of one layer, with separate
+    // launches of two: what it touches decides how much of the weights stays in the memory-side cache (256 MB) from one
+    // forward to the next.  12 layers of BERT-base at 80 %, 64 x 128 tokens 1007 -> 860 us (a set a layer is 0.75 GB),
+    // BERT-large 4 x 512 1352 -> 1165, 16 x 128 dense 1022 -> 992; 8 x 128 with two more models run in between 457 -> 396.
+    // (Separate launches in one set: 16 x 128 dense 980, but 2 x 128 under mixed = 0 370 where two sets take 361.)
+    et::LayerBuffers stack_buffers(int i) const { return layers[(size_t)(local.empty() ? i % 2 : 0) % layers.size()]->buffers(); }
     void drop_graph() {
         if (graph) (void)et_graph_destroy(graph);
         graph = nullptr;
@@ -278,10 +278,10 @@ bool build_chain(et_model_s &m) {
 void run_layers_chain(et_model_s &m, half *out, half *in, stream_t stream) {
     const int n = (int)m.layers.size();
     etChk(et_fill_i32(m.chain_sync->get(), m.chain_sync->size, 0, stream));
-    m.layers[0]->chain_qkv_first(in, stream);
+    m.layers[0]->chain_qkv_first(m.layers[0]->buffers(), in, stream);
     et::SplitSum carry;
     for (int i = 0; i < n; i++) {
-        m.layers[(size_t)i]->chain_attention(stream);
+        m.layers[(size_t)i]->chain_attention(m.layers[(size_t)i]->buffers(), stream);
         et_chain_desc d = m.chain_desc[(size_t)i];
         if (i == 0) d.resid16 = et::f16(in);
         int groups2 = 0;
@@ -421,12 +421,12 @@ bool local_aligned(const half *p) { return (reinterpret_cast<std::uintptr_t>(p) 
 void copy_rows(et_model_s &m, half *to, const half *from, stream_t stream) {
     etChk(et_memcpy_d2d(to, from, (std::size_t)m.rows() * m.desc.emdim * sizeof(half), stream));
 }
-half *local_input(et_model_s &m, ILayer &l, half *in, stream_t stream) {
+half *local_input(et_model_s &m, const et::LayerBuffers &b, half *in, stream_t stream) {
     if (local_aligned(in)) return in;
-    copy_rows(m, l.spare_in(), in, stream);
-    return l.spare_in();
+    copy_rows(m, b.attn, in, stream);
+    return b.attn;
 }
-half *local_result(ILayer &l, half *out) { return local_aligned(out) ? out : l.spare_out(); }
+half *local_result(const et::LayerBuffers &b, half *out) { return local_aligned(out) ? out : b.ffn; }
 
 // One layer from binary16 to binary16, as et_model_forward under mixed = 0 chains it (`chained`: behind the layer before it)
 // and et_model_forward_layer issues it.  The token-local launches take the layer's input and leave its result in binary16,
@@ -435,29 +435,32 @@ half *local_result(ILayer &l, half *out) { return local_aligned(out) ? out : l.s
 // one's where its own was read: it touches no buffer of another layer.
 void run_layer_f16(et_model_s &m, int i, half *out, half *in, bool chained, stream_t stream) {
     ILayer &l = *m.layers[(size_t)i];
-    if (m.local.empty()) return l.forward(out, in, stream);
-    if (i == 0) l.chain_qkv_first(in, stream);
-    half *x = local_input(m, l, in, stream), *to = local_result(l, out);
-    if (i > 0 && !chained) etChk(et_encoder_layer_project_f16(m.local[(size_t)i - 1].get(), et::f16(x), et::f16(l.qkv_buffer()), stream));
-    l.chain_attention(stream);
+    const et::LayerBuffers b = chained ? m.stack_buffers(i) : l.buffers();
+    if (m.local.empty()) return l.forward(b, out, in, stream);
+    if (i == 0) l.chain_qkv_first(b, in, stream);
+    half *x = local_input(m, b, in, stream), *to = local_result(b, out);
+    if (i > 0 && !chained) etChk(et_encoder_layer_project_f16(m.local[(size_t)i - 1].get(), et::f16(x), et::f16(b.qkv), stream));
+    l.chain_attention(b, stream);
     const bool last = i + 1 == (int)m.layers.size();
-    half *qkv = last ? nullptr : chained ? m.layers[(size_t)i + 1]->qkv_buffer() : l.qkv_buffer();
-    etChk(et_encoder_layer_f32(m.local[(size_t)i].get(), et::f16(l.z_buffer()), nullptr, et::f16(x), nullptr, et::f16(to), et::f16(qkv),
+    half *qkv = last ? nullptr : chained ? m.stack_buffers(i + 1).qkv : b.qkv;
+    etChk(et_encoder_layer_f32(m.local[(size_t)i].get(), et::f16(b.z), nullptr, et::f16(x), nullptr, et::f16(to), et::f16(qkv),
                                m.shares(chained ? 0 : i), m.desc.act, l.epsilon(0), l.epsilon(1), stream));
     if (to != out) copy_rows(m, out, to, stream);
 }
 
 void run_layers_local(et_model_s &m, half *out, half *in, stream_t stream) {
     const int n = (int)m.layers.size();
-    m.layers[0]->chain_qkv_first(in, stream);
-    half *x = local_input(m, *m.layers[0], in, stream), *to = local_result(*m.layers[(size_t)n - 1], out);
+    const et::LayerBuffers first = m.stack_buffers(0), end = m.stack_buffers(n - 1);
+    m.layers[0]->chain_qkv_first(first, in, stream);
+    half *x = local_input(m, first, in, stream), *to = local_result(end, out);
     for (int i = 0; i < n; i++) {
         ILayer &l = *m.layers[(size_t)i];
+        const et::LayerBuffers b = m.stack_buffers(i);
         const bool last = i == n - 1;
-        l.chain_attention(stream);
-        etChk(et_encoder_layer_f32(m.local[(size_t)i].get(), et::f16(l.z_buffer()), i ? m.local_x[(i - 1) & 1]->get() : nullptr,
+        l.chain_attention(b, stream);
+        etChk(et_encoder_layer_f32(m.local[(size_t)i].get(), et::f16(b.z), i ? m.local_x[(i - 1) & 1]->get() : nullptr,
                                    i ? nullptr : et::f16(x), last ? nullptr : m.local_x[i & 1]->get(), last ? et::f16(to) : nullptr,
-                                   last ? nullptr : et::f16(m.layers[(size_t)i + 1]->qkv_buffer()),
+                                   last ? nullptr : et::f16(m.stack_buffers(i + 1).qkv),
                                    m.shares(0), m.desc.act, l.epsilon(0), l.epsilon(1), stream));
     }
     if (to != out) copy_rows(m, out, to, stream);
@@ -469,7 +472,7 @@ void run_layers_split(et_model_s &m, half *out, half *in, stream_t stream) {
     // the first layer adds the binary16 input as its residual: no widened copy
     et::SplitSum carry;
     for (int i = 0; i < n; i++)
-        carry = m.layers[(size_t)i]->forward_split(i ? &carry : nullptr, nullptr, in, stream);
+        carry = m.layers[(size_t)i]->forward_split(m.stack_buffers(i), i ? &carry : nullptr, nullptr, in, stream);
     m.layers[(size_t)n - 1]->finish_split(nullptr, out, carry, stream);
 }
 
@@ -485,7 +488,7 @@ void run_layers_mixed(et_model_s &m, half *out, half *in, stream_t stream) {
         const bool last = i == n - 1;
         float *dst32 = last ? nullptr : m.pp32[i % R]->get();
         half *dst16 = last ? out : m.pp[i % R]->get();
-        m.layers[(size_t)i]->forward_mixed(dst32, dst16, src32, src16, stream);
+        m.layers[(size_t)i]->forward_mixed(m.stack_buffers(i), dst32, dst16, src32, src16, stream);
         src32 = dst32;
         src16 = dst16;
     }
@@ -711,7 +714,7 @@ int et_model_forward_layer(et_model m, int layer, et_f16 *out, const et_f16 *in,
         half *i = reinterpret_cast<half *>(const_cast<et_f16 *>(in));
         if (m->desc.mixed) {  // one layer between binary16 buffers: the residual starts from the binary16 input
             etChk(et_f16_to_f32(m->pp32[0]->get(), in, (std::size_t)m->rows() * m->desc.emdim, stream));
-            m->layers[(size_t)layer]->forward_mixed(nullptr, o, m->pp32[0]->get(), i, stream);
+            m->layers[(size_t)layer]->forward_mixed(m->layers[(size_t)layer]->buffers(), nullptr, o, m->pp32[0]->get(), i, stream);
         } else {
             run_layer_f16(*m, layer, o, i, false, stream);
         }
