@@ -62,6 +62,9 @@ struct AttnRun {
     // Multihead_atttion_fuseO only: attention and output projection as ONE launch (et_mha_fuseo_f16), as the
     // reference runs them, instead of the two stream-ordered launches, which are several times faster here
     bool one_launch = false;
+    // fused attention: weights that later launches read, asked for meanwhile (et_mha_fused_ahead_f16)
+    const et_span *ahead = nullptr;
+    int nahead = 0;
 };
 
 inline void fused_mha(const half *q, const half *k, const half *v, int ldq, int ldk, int ldv, half *z,
@@ -69,9 +72,9 @@ inline void fused_mha(const half *q, const half *k, const half *v, int ldq, int 
     const int hd = m.kdim / m.nhead;
     require(m.vdim == m.kdim, "fused attention: vdim must equal kdim");
     const float scale = run.scale != 0.0f ? run.scale : 1.0f / std::sqrt((float)hd);
-    etChk(et_mha_fused_f16(f16(q), f16(k), f16(v), ldq, ldk, ldv, f16(z), ldz, f16(run.mask), run.lens,
-                           run.batch, m.seq_len, m.nhead, hd, scale, run.causal ? ET_MHA_CAUSAL : 0,
-                           run.stream));
+    etChk(et_mha_fused_ahead_f16(f16(q), f16(k), f16(v), ldq, ldk, ldv, f16(z), ldz, f16(run.mask), run.lens,
+                                 run.batch, m.seq_len, m.nhead, hd, scale, run.causal ? ET_MHA_CAUSAL : 0, run.ahead,
+                                 run.nahead, run.stream));
 }
 
 }  // namespace et
@@ -310,8 +313,10 @@ class Attention<_config, std::enable_if_t<_config::isSingleKernel>> : public et:
     // sizes that does not run at the same time (a stack that hands one layer's result to the next).
     struct Buffers {
         half *qkv = nullptr, *z = nullptr;
+        const et_span *ahead = nullptr;  // as AttnRun's
+        int nahead = 0;
     };
-    Buffers buffers() { return {mat_qkv->get(), mat_z->get()}; }
+    Buffers buffers() { return {mat_qkv->get(), mat_z->get(), nullptr, 0}; }
 
     void forward(half *out, half *query, half *key, half *value, et::stream_t stream = nullptr) {
         forward_in(buffers(), out, query, key, value, stream);
@@ -370,7 +375,10 @@ class Attention<_config, std::enable_if_t<_config::isSingleKernel>> : public et:
         half *Q = b.qkv;
         half *K = Q + model->kdim;
         half *V = K + model->kdim;
-        et::fused_mha(Q, K, V, ldm, ldm, ldm, b.z, model->vdim, *model, run(stream));
+        et::AttnRun r = run(stream);
+        r.ahead = b.ahead;
+        r.nahead = b.nahead;
+        et::fused_mha(Q, K, V, ldm, ldm, ldm, b.z, model->vdim, *model, r);
     }
     void forward_split(float *v1, float *stats1, int *groups1, float *fin_in, const et::SplitSum *in, const float *x32,
                        half *x16, et::stream_t stream = nullptr) {

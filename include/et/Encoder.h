@@ -79,7 +79,9 @@ struct ChainParts {
 
 // Where a forward keeps what it computes on the way.  Null: the layer does not have it (yet).
 struct LayerBuffers {
-    half *qkv = nullptr, *z = nullptr;  // single-projection attention
+    half *qkv = nullptr, *z = nullptr;  // single-projection attention, which also asks for these while it runs:
+    const et_span *ahead = nullptr;     // weights that the launches behind it read
+    int nahead = 0;
     half *attn = nullptr, *LN = nullptr, *linear = nullptr, *ffn = nullptr;
     float *attn32 = nullptr, *LN32 = nullptr, *ffn32 = nullptr, *stats1 = nullptr, *stats2 = nullptr, *fin_in = nullptr, *fin1 = nullptr;
 };
@@ -151,7 +153,7 @@ template <typename attn_t, typename linear1_t, typename linear2_t, typename ACT_
     void forward_f16(half *out, half *src, stream_t stream = nullptr) { forward_f16_in(buffers(), out, src, stream); }
     // (..._in: in the buffers of another layer of the same sizes that does not run at the same time)
     void forward_f16_in(const LayerBuffers &b, half *out, half *src, stream_t stream = nullptr) {
-        if constexpr (attn_has_split<attn_t>::value) attn->forward_in({b.qkv, b.z}, b.attn, src, src, src, stream);
+        if constexpr (attn_has_split<attn_t>::value) attn->forward_in({b.qkv, b.z, b.ahead, b.nahead}, b.attn, src, src, src, stream);
         else attn->forward(b.attn, src, src, src, stream);
         bool fused_ln1 = false;
         if constexpr (std::is_same_v<linear1_t, Linear<tile_mat>>) {
@@ -315,6 +317,17 @@ template <typename attn_t, typename linear1_t, typename linear2_t, typename ACT_
         b.stats1 = at(stats1), b.stats2 = at(stats2), b.fin_in = at(fin_in), b.fin1 = at(fin1);
         return b;
     }
+    // the values of the layer's dense weights in the order QKV, O, linear1, linear2; false where one is not dense
+    bool dense_weights(et_span (&w)[4]) {
+        if constexpr (attn_has_split<attn_t>::value && std::is_same_v<linear1_t, Linear<base_mat>> && std::is_same_v<linear2_t, Linear<base_mat>>) {
+            const auto span = [](auto &l) { return et_span{l.weight.get(), l.weight.size * sizeof(half)}; };
+            w[0] = span(attn->qkv_linear()), w[1] = span(attn->o_linear()), w[2] = span(*linear1), w[3] = span(*linear2);
+            return true;
+        } else {
+            (void)w;
+            return false;
+        }
+    }
     half *qkv_buffer() { return buffers().qkv; }
     half *z_buffer() { return buffers().z; }
     float epsilon(int k) const { return k ? LN2->epsilon() : LN1->epsilon(); }
@@ -326,7 +339,7 @@ template <typename attn_t, typename linear1_t, typename linear2_t, typename ACT_
     }
     void chain_attention(stream_t stream = nullptr) { chain_attention_in(buffers(), stream); }
     void chain_attention_in(const LayerBuffers &b, stream_t stream = nullptr) {
-        if constexpr (attn_has_split<attn_t>::value) attn->core({b.qkv, b.z}, stream);
+        if constexpr (attn_has_split<attn_t>::value) attn->core({b.qkv, b.z, b.ahead, b.nahead}, stream);
         else (void)b, (void)stream;
     }
     // (`in` may lie in other buffers than this call's)
@@ -339,7 +352,7 @@ template <typename attn_t, typename linear1_t, typename linear2_t, typename ACT_
                       std::is_same_v<linear2_t, Linear<tile_mat>>) {
             require(b.stats1 && b.stats2 && b.fin_in && b.fin1, "Encoder: call enable_split() before forward_split()");
             int g1 = 0, g2 = 0;
-            attn->forward_split_in({b.qkv, b.z}, b.attn32, b.stats1, &g1, b.fin_in, in, x32, x16, stream);
+            attn->forward_split_in({b.qkv, b.z, b.ahead, b.nahead}, b.attn32, b.stats1, &g1, b.fin_in, in, x32, x16, stream);
             linear1->forward_norm_f32in(b.linear, b.attn32, b.stats1, g1,
                                         LN1->gamma(), LN1->beta(), LN1->epsilon(), b.fin1, nullptr, nullptr,
                                         act_code<ACT_OP_t>(), stream);
@@ -398,7 +411,7 @@ template <typename attn_t, typename linear1_t, typename linear2_t, typename ACT_
                                static_cast<half *>(nullptr), static_cast<stream_t>(nullptr)))>> : std::true_type {};
     void attn_forward_f32(const LayerBuffers &b, float *out32, half *src16, stream_t stream) {
         if constexpr (attn_has_split<attn_t>::value) {
-            attn->forward_f32_in({b.qkv, b.z}, out32, src16, src16, src16, b.attn, stream);
+            attn->forward_f32_in({b.qkv, b.z, b.ahead, b.nahead}, out32, src16, src16, src16, b.attn, stream);
         } else if constexpr (attn_has_f32<attn_t>::value) {
             attn->forward_f32(out32, src16, src16, src16, b.attn, stream);
         } else {  // attention forms without a binary32 output projection: widen their result

@@ -26,6 +26,12 @@ extern "C" {
 #endif
 
 typedef uint16_t et_f16;  /* IEEE binary16 bit pattern */
+
+/* a piece of device memory */
+typedef struct et_span {
+    const void *data;
+    size_t bytes;
+} et_span;
 typedef void *et_stream;  /* hipStream_t; NULL = the null stream */
 typedef void *et_event;   /* hipEvent_t */
 typedef void *et_graph;   /* a captured HIP graph with its executable instance (opaque) */
@@ -303,6 +309,8 @@ int et_encoder_layer_pack_create(const et_layer_weights *w, int T, int emdim, in
                                  struct et_layer_pack_s **pack);
 int et_encoder_layer_pack_create_projecting(const et_layer_weights *w, int T, int emdim, int dimFF, int qkv_out, int mt,
                                             int parts, struct et_layer_pack_s **pack);
+/* where the streams of a pack lie, for et_mha_fused_ahead_f16 */
+int et_encoder_layer_pack_streams(const struct et_layer_pack_s *pack, et_span *streams);
 int et_encoder_layer_pack_destroy(struct et_layer_pack_s *pack);
 int et_encoder_layer_f32(const struct et_layer_pack_s *pack, const et_f16 *Z, const float *x32, const et_f16 *x16,
                          float *x32_out, et_f16 *out16, et_f16 *QKV, float *partial, int act, float eps1, float eps2,
@@ -563,6 +571,16 @@ int et_mha_fused_f16(const et_f16 *Q, const et_f16 *K, const et_f16 *V,
                      int ldq, int ldk, int ldv, et_f16 *Z, int ldz,
                      const et_f16 *mask, const int32_t *lens, int B, int S,
                      int nh, int hd, float scale, int flags, et_stream stream);
+/* The same; while it runs, a few of its workgroups ask for the bytes of up to four spans of device memory that later
+ * launches read (weights), so that these find them in the memory-side cache (heads up to 64 wide, sequences of multiples of 64;
+ * others ignore the spans).  Nothing else depends on the spans; they must be
+ * readable until the launch has ended, 4-byte aligned and under 2 GiB each. */
+#define ET_MHA_AHEAD 4
+int et_mha_fused_ahead_f16(const et_f16 *Q, const et_f16 *K, const et_f16 *V,
+                           int ldq, int ldk, int ldv, et_f16 *Z, int ldz,
+                           const et_f16 *mask, const int32_t *lens, int B, int S,
+                           int nh, int hd, float scale, int flags,
+                           const et_span *ahead, int nahead, et_stream stream);
 
 /* Fused attention and the tile-sparse output projection in ONE launch:
  *   Z = attention as et_mha_fused_f16 (Z is written, [B*S x ldz]),

@@ -85,6 +85,7 @@ _SIGNATURES = {
     "et_encoder_layer_pack_create": (_vp, _i, _i, _i, _i, _i, _i, C.POINTER(_vp)),
     "et_encoder_layer_pack_create_projecting": (_vp, _i, _i, _i, _i, _i, _i, C.POINTER(_vp)),
     "et_encoder_layer_pack_destroy": (_vp,),
+    "et_encoder_layer_pack_streams": (_vp, _vp),
     "et_encoder_layer_f32": (_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _f, _f, _vp),
     "et_encoder_layer_project_f16": (_vp, _vp, _vp, _vp),
     "et_probe_empty": (_i, _i, _vp),
@@ -116,6 +117,7 @@ _SIGNATURES = {
     "et_linear_rowpruned_compact_f16": (_vp, _vp, _i, _vp, _vp, _vp, _i, _i, _vp),
     "et_linear_colpruned_f16": (_vp, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _i, _vp),
     "et_mha_fused_f16": (_vp, _vp, _vp, _i, _i, _i, _vp, _i, _vp, _vp, _i, _i, _i, _i, _f, _i, _vp),
+    "et_mha_fused_ahead_f16": (_vp, _vp, _vp, _i, _i, _i, _vp, _i, _vp, _vp, _i, _i, _i, _i, _f, _i, _vp, _i, _vp),
     "et_mha_fuseo_f16": (_vp, _vp, _vp, _i, _i, _i, _vp, _i, _vp, _vp, _i, _i, _i, _i, _f, _i,
                          _vp, _vp, _vp, _vp, _vp, _i, _vp),
     "et_mha_fuseo_f16_geom": (_vp, _vp, _vp, _i, _i, _i, _vp, _i, _vp, _vp, _i, _i, _i, _i, _f, _i,

@@ -54,6 +54,10 @@ struct MhaArgs {
     const int32_t *v_col_id;
     const int32_t *v_head_ptr;
     int v_nnz = 0;  // entries of v_col_id (> 0 in the compact-V form)
+    // weights that later launches read (ahead_of below): lines of 128 bytes of each span, and the workgroups that ask for them
+    const char *ahead[ET_MHA_AHEAD] = {};
+    unsigned ahead_lines[ET_MHA_AHEAD] = {};
+    unsigned ahead_blocks = 0;
 };
 
 constexpr int kXcds = 8;                // accelerator dies, each with a private L2
@@ -98,6 +102,29 @@ template <int HD> __device__ __forceinline__ constexpr int vt_unit_keys(int kg) 
     return kg;
 }
 
+// The first `ahead_blocks` workgroups of a launch (a multiple of 8: the others keep their XCD) attend to nothing: each thread
+// asks for one line of a weight that the launches behind this one read.  Where weights do not stay in the memory-side
+// cache from one forward to the next, those launches would wait for HBM with every compute unit; here the requests cost
+// a few workgroups' slots, and nobody waits for them but the end of the launch.
+__device__ __forceinline__ void ahead_of(const MhaArgs &a) {
+    unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
+#pragma unroll
+    for (int s = 0; s < ET_MHA_AHEAD; s++) {
+        if (i < a.ahead_lines[s]) {
+            int line;
+            asm volatile("global_load_dword %0, %1, off" : "=v"(line) : "v"(a.ahead[s] + (size_t)i * 128) : "memory");
+            break;
+        }
+        i -= a.ahead_lines[s];
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+static unsigned ahead_blocks(const MhaArgs &a, int threads) {
+    unsigned lines = 0;
+    for (unsigned n : a.ahead_lines) lines += n;
+    return ((lines + threads - 1) / threads + kXcds - 1) / kXcds * kXcds;
+}
+
 // QT = 16-query tiles per wave: with QT = 2 every K and V^T fragment read from LDS feeds
 // two MFMAs and a workgroup covers 32*NW queries per staged key block.
 //
@@ -134,14 +161,34 @@ __global__ __launch_bounds__(64 * NW)
     __attribute__((amdgpu_waves_per_eu(mha_three_waves<HD, NW, COMPACT, QT>() ? 3 : 1, mha_three_waves<HD, NW, COMPACT, QT>() ? 3 : 8))) void
     mha_fused_kernel(const MhaArgs a) {
     constexpr bool kCoherentZ = false;
+    const unsigned block = blockIdx.x;
 #include "attention_body.inc"
 }
 
+// the same behind workgroups that ask for later launches' weights (heads up to 64, four or eight waves; a kernel of its own,
+// since the argument to tell them apart by is a wait of its own at the start: 12 layers of one sequence 335 -> 342 us)
+template <int HD, int NW, int QT>
+__global__ __launch_bounds__(64 * NW)
+    __attribute__((amdgpu_waves_per_eu(mha_three_waves<HD, NW, false, QT>() ? 3 : 1, mha_three_waves<HD, NW, false, QT>() ? 3 : 8))) void
+    mha_fused_ahead_kernel(const MhaArgs a) {
+    constexpr bool kCoherentZ = false, COMPACT = false;
+    if (blockIdx.x < a.ahead_blocks) return ahead_of(a);
+    const unsigned block = blockIdx.x - a.ahead_blocks;
+#include "attention_body.inc"
+}
+template <int HD, bool COMPACT, int NW> constexpr bool mha_takes_ahead() { return HD <= 64 && !COMPACT && NW >= 4; }
+
 template <int HD, bool COMPACT, int NW, int QT>
 static int launch_mha_nw(const MhaArgs &args, hipStream_t stream) {
-    auto kernel = mha_fused_kernel<HD, COMPACT, NW, QT>;
+    void (*kernel)(MhaArgs) = mha_fused_kernel<HD, COMPACT, NW, QT>;
+    MhaArgs a = args;
+    if constexpr (mha_takes_ahead<HD, COMPACT, NW>()) {
+        a.ahead_blocks = ahead_blocks(a, 64 * NW);
+        if (a.ahead_blocks) kernel = mha_fused_ahead_kernel<HD, NW, QT>;
+    }
     constexpr size_t lds = MhaLds<HD>::bytes;
     if (lds > 64 * 1024) {
+        static_assert(!mha_takes_ahead<HD, COMPACT, NW>() || lds <= 64 * 1024, "the attribute is set for one kernel");
         static bool raised = false;
         if (!raised) {
             ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
@@ -151,7 +198,7 @@ static int launch_mha_nw(const MhaArgs &args, hipStream_t stream) {
     }
     const int qstrips = (args.S + 16 * NW * QT - 1) / (16 * NW * QT);
     const int rounds = (args.nbh + kXcds - 1) / kXcds;
-    kernel<<<dim3((unsigned)(rounds * kXcds * qstrips)), 64 * NW, lds, stream>>>(args);
+    kernel<<<dim3(a.ahead_blocks + (unsigned)(rounds * kXcds * qstrips)), 64 * NW, lds, stream>>>(a);
     return check_launch("mha_fused_kernel");
 }
 
@@ -176,7 +223,7 @@ static int launch_mha_nw(const MhaArgs &args, hipStream_t stream) {
 // For S a multiple of 256, no additive mask and a positive scale; padded keys and the causal mask are applied to the
 // blocks they cut, and a wave skips the blocks past its last query.
 constexpr int kPpQ = 256;  // queries of a workgroup
-__global__ __launch_bounds__(512) void mha_pingpong_kernel(const MhaArgs a) {
+__device__ __forceinline__ void mha_pingpong(const MhaArgs &a, unsigned block) {
     constexpr int HD = 64, KS = 2, DB = 4, QT = 2;
     using L = MhaLds<HD>;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -189,7 +236,7 @@ __global__ __launch_bounds__(512) void mha_pingpong_kernel(const MhaArgs a) {
     const int S = a.S, hd = a.hd;
     // as in the kernel above: the query strips of a (sequence, head) on one XCD
     const int qstrips = S / kPpQ;
-    const int xcd = blockIdx.x % kXcds, k_in_xcd = blockIdx.x / kXcds;
+    const int xcd = block % kXcds, k_in_xcd = block / kXcds;
     const int bh = xcd + kXcds * (k_in_xcd / qstrips);
     if (bh >= a.nbh) return;  // padding of the last round (whole workgroup)
     const int qstrip = k_in_xcd % qstrips;
@@ -396,15 +443,24 @@ __global__ __launch_bounds__(512) void mha_pingpong_kernel(const MhaArgs a) {
     }
 }
 
+__global__ __launch_bounds__(512) void mha_pingpong_kernel(const MhaArgs a) { mha_pingpong(a, blockIdx.x); }
+__global__ __launch_bounds__(512) void mha_pingpong_ahead_kernel(const MhaArgs a) {
+    if (blockIdx.x < a.ahead_blocks) return ahead_of(a);
+    mha_pingpong(a, blockIdx.x - a.ahead_blocks);
+}
+
 static int launch_mha_pingpong(const MhaArgs &args, hipStream_t stream) {
     constexpr size_t lds = 2 * MhaLds<64>::bytes;
     static bool raised = false;
     if (!raised) {
-        ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(mha_pingpong_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        for (auto k : {mha_pingpong_kernel, mha_pingpong_ahead_kernel})
+            ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         raised = true;
     }
     const int qstrips = args.S / kPpQ, rounds = (args.nbh + kXcds - 1) / kXcds;
-    mha_pingpong_kernel<<<dim3((unsigned)(rounds * kXcds * qstrips)), 512, lds, stream>>>(args);
+    MhaArgs a = args;
+    a.ahead_blocks = ahead_blocks(a, 512);
+    (a.ahead_blocks ? mha_pingpong_ahead_kernel : mha_pingpong_kernel)<<<dim3(a.ahead_blocks + (unsigned)(rounds * kXcds * qstrips)), 512, lds, stream>>>(a);
     return check_launch("mha_pingpong_kernel");
 }
 
@@ -477,6 +533,7 @@ template <int HD, int NW, int QT>
 __global__ __launch_bounds__(64 * NW) void mha_fuseo_kernel(const MhaArgs a, const FuseOArgs f) {
     constexpr bool COMPACT = false;
     constexpr bool kCoherentZ = true;
+    const unsigned block = blockIdx.x;
 #include "attention_body.inc"
     // ---- arrival.  Z was stored at device scope, and such a store counts as complete only once it has
     // reached the memory side: when every wave's stores are complete the count moves.  A device-wide fence
@@ -1127,6 +1184,12 @@ extern "C" {
 int et_mha_fused_f16(const et_f16 *Q, const et_f16 *K, const et_f16 *V, int ldq, int ldk, int ldv,
                      et_f16 *Z, int ldz, const et_f16 *mask, const int32_t *lens, int B, int S,
                      int nh, int hd, float scale, int flags, et_stream stream) {
+    return et_mha_fused_ahead_f16(Q, K, V, ldq, ldk, ldv, Z, ldz, mask, lens, B, S, nh, hd, scale, flags, nullptr, 0, stream);
+}
+
+int et_mha_fused_ahead_f16(const et_f16 *Q, const et_f16 *K, const et_f16 *V, int ldq, int ldk, int ldv,
+                           et_f16 *Z, int ldz, const et_f16 *mask, const int32_t *lens, int B, int S,
+                           int nh, int hd, float scale, int flags, const et_span *ahead, int nahead, et_stream stream) {
     ET_REQUIRE(Q && K && V && Z, ET_ERR_INVALID_ARG, "et_mha_fused_f16: NULL pointer");
     ET_REQUIRE(B >= 0 && S > 0 && nh > 0 && hd > 0, ET_ERR_INVALID_ARG,
                "et_mha_fused_f16: B=%d S=%d nh=%d hd=%d", B, S, nh, hd);
@@ -1148,8 +1211,15 @@ int et_mha_fused_f16(const et_f16 *Q, const et_f16 *K, const et_f16 *V, int ldq,
                    (reinterpret_cast<uintptr_t>(Z) & 7) == 0,
                ET_ERR_UNSUPPORTED, "et_mha_fused_f16: operands must be 16-byte aligned");
     ET_REQUIRE((long long)B * nh * (S / 16) < (1LL << 30), ET_ERR_UNSUPPORTED, "et_mha_fused_f16: grid too large");
+    ET_REQUIRE(nahead >= 0 && nahead <= ET_MHA_AHEAD && (nahead == 0 || ahead), ET_ERR_INVALID_ARG, "et_mha_fused_ahead_f16: %d spans", nahead);
     if (B == 0) return ET_OK;
     MhaArgs args;
+    for (int i = 0; i < nahead; i++) {
+        ET_REQUIRE(ahead[i].bytes == 0 || (ahead[i].data && (reinterpret_cast<uintptr_t>(ahead[i].data) & 3) == 0 && ahead[i].bytes < (1ull << 31)),
+                   ET_ERR_INVALID_ARG, "et_mha_fused_ahead_f16: span %d", i);
+        args.ahead[i] = static_cast<const char *>(ahead[i].data);
+        args.ahead_lines[i] = (unsigned)(ahead[i].bytes / 128);  // (a piece of a line at the end is not worth a request)
+    }
     args.Q = reinterpret_cast<const _Float16 *>(Q);
     args.K = reinterpret_cast<const _Float16 *>(K);
     args.V = reinterpret_cast<const _Float16 *>(V);

@@ -981,6 +981,12 @@ static void el_second(LayerArgs &a, const et_layer_pack_s &p) {
     a.parts = p.Q ? p.parts : 1;  // without a projection only the normalisation is left
 }
 
+extern "C" int et_encoder_layer_pack_streams(const struct et_layer_pack_s *p, et_span *streams) {
+    ET_REQUIRE(p && streams, ET_ERR_INVALID_ARG, "et_encoder_layer_pack_streams: NULL pointer");
+    *streams = {p->slots, ((size_t)p->second * p->cap + (size_t)(p->nstream - p->second) * p->cap2) * 1024};
+    return ET_OK;
+}
+
 extern "C" int et_encoder_layer_project_f16(const struct et_layer_pack_s *p, const et_f16 *x16, et_f16 *QKV, et_stream stream) {
     ET_REQUIRE(p && x16 && QKV, ET_ERR_INVALID_ARG, "et_encoder_layer_project_f16: NULL pointer");
     ET_REQUIRE(p->Q > 0 && p->nstream > p->second, ET_ERR_UNSUPPORTED,

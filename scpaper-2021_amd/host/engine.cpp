@@ -35,6 +35,7 @@ struct ILayer {
     virtual et::AttnState &attn() = 0;
     virtual bool local_weights(et_layer_weights &w) = 0;
     virtual bool local_qkv(et_layer_weights &w) = 0;
+    virtual bool dense_weights(et_span (&w)[4]) = 0;
     virtual float epsilon(int k) const = 0;
 };
 
@@ -64,6 +65,7 @@ template <typename EncoderT> struct LayerOf final : ILayer {
     et::AttnState &attn() override { return enc->attention(); }
     bool local_weights(et_layer_weights &w) override { return enc->local_weights(w); }
     bool local_qkv(et_layer_weights &w) override { return enc->local_qkv(w); }
+    bool dense_weights(et_span (&w)[4]) override { return enc->dense_weights(w); }
     float epsilon(int k) const override { return enc->epsilon(k); }
 };
 struct LayerPackDeleter {
@@ -140,7 +142,12 @@ struct et_model_s {
     // forward to the next.  12 layers of BERT-base at 80 %, 64 x 128 tokens 1007 -> 860 us (a set a layer is 0.75 GB),
     // BERT-large 4 x 512 1352 -> 1165, 16 x 128 dense 1022 -> 992; 8 x 128 with two more models run in between 457 -> 396.
     // (Separate launches in one set: 16 x 128 dense 980, but 2 x 128 under mixed = 0 370 where two sets take 361.)
-    et::LayerBuffers stack_buffers(int i) const { return layers[(size_t)(local.empty() ? i % 2 : 0) % layers.size()]->buffers(); }
+    et::LayerBuffers stack_buffers(int i) const {
+        et::LayerBuffers b = layers[(size_t)(local.empty() ? i % 2 : 0) % layers.size()]->buffers();
+        if (!ahead.empty()) b.ahead = ahead[(size_t)i].data(), b.nahead = (int)ahead[(size_t)i].size();
+        return b;
+    }
+    std::vector<std::vector<et_span>> ahead;  // of every layer (plan_ahead), or none
     void drop_graph() {
         if (graph) (void)et_graph_destroy(graph);
         graph = nullptr;
@@ -413,6 +420,37 @@ void build_local(et_model_s &m, bool fused) {
     if (plan.parts > 1)
         for (int i = 0; i < (d.mixed ? 1 : n); i++) m.local_shares.push_back(std::make_unique<et::DeviceBuffer<float>>(elems * plan.parts));
     m.local = std::move(packs);
+}
+
+// Weights that a layer's launches read, asked for by its attention kernel (et_mha_fused_ahead_f16): the streams of the
+// token-local launches, or O, FFN and the next QKV of a dense layer.  For a model whose weights and activations do not stay
+// in the memory-side cache from one forward to the next, and enough token rows that the attention takes about as long as the
+// requests.  us, off / on: 12 layers of BERT-base at 80 %, 64 x 128 tokens, three models in turn 990 / 890, one model again and
+// again 855 / 856; BERT-large at 90 %, 4 x 512 1349 / 1238, 1172 / 1171; 16 x 128 dense 1017 / 997, 996 / 992; 32 x 128 dense one
+// model 1685 / 1612.  On the other side of the lines: 8 x 128 at 80 % (70 MB in all) 394 / 401, 384 / 392; 4 x 128 dense 604 / 619.
+void plan_ahead(et_model_s &m) {
+    const size_t n = m.layers.size();
+    const et_model_desc &d = m.desc;
+    const int ldq = 2 * d.kdim + d.vdim;
+    std::vector<std::vector<et_span>> ahead(n);
+    double bytes = 0;
+    for (size_t i = 0; i < n; i++) {
+        et_span w[4], next[4];
+        if (!m.local.empty()) {
+            ahead[i].resize(1);
+            etChk(et_encoder_layer_pack_streams(m.local[i].get(), ahead[i].data()));
+        } else if (m.layers[i]->dense_weights(w)) {
+            ahead[i] = {w[1], w[2], w[3]};
+            if (i + 1 < n && m.layers[i + 1]->dense_weights(next)) ahead[i].push_back(next[0]);
+        } else {
+            return;
+        }
+        for (const et_span &s : ahead[i]) bytes += (double)s.bytes;
+    }
+    // a row of what the forward writes: binary16 projections and results, the binary32 residual and shares
+    const int parts = m.local_shares.empty() ? 0 : (int)(m.local_shares[0]->size / ((size_t)m.rows() * d.emdim));
+    const double row = m.local.empty() ? 4.0 * (ldq + d.vdim + 3 * d.emdim + d.dimFF) : 2.0 * (ldq + d.vdim) + (8.0 + 4.0 * parts) * d.emdim;
+    if (m.rows() >= 2048 && bytes + row * m.rows() >= 96.0 * (1 << 20)) m.ahead = std::move(ahead);
 }
 
 // The token-local launches read and write up to 16 bytes at a time; input and result at another address (which the
@@ -696,6 +734,7 @@ int et_model_finalize(et_model m) {
                 }
             }
         }
+        plan_ahead(*m);
         etChk(et_stream_create(&m->own_stream));
         apply_attention_state(*m);
         m->host.clear();
