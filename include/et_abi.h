@@ -309,6 +309,16 @@ int et_encoder_layer_pack_create(const et_layer_weights *w, int T, int emdim, in
                                  struct et_layer_pack_s **pack);
 int et_encoder_layer_pack_create_projecting(const et_layer_weights *w, int T, int emdim, int dimFF, int qkv_out, int mt,
                                             int parts, struct et_layer_pack_s **pack);
+/* Both parts of a pack with parts > 1 in one launch: the workgroups of a strip meet at a word of `join`, one per 16 token rows,
+ * zero before the first call and left zero by every one (launches that may overlap need words, and `partial`, of their own).
+ * A workgroup waits for the others of its strip for at most `spin` looks at the word; if they are not there by then it leaves
+ * its share of the projection to the last of them, with the same result.  et_encoder_layer_joins tells whether a pack can: 2 to
+ * 12 parts, on a device that gives workgroups of equal id modulo 8 to one die, which is looked at once (it launches and copies:
+ * not while a stream is being captured). */
+int et_encoder_layer_joins(const struct et_layer_pack_s *pack, int *joins);
+int et_encoder_layer_joined_f32(const struct et_layer_pack_s *pack, const et_f16 *Z, const float *x32, const et_f16 *x16, float *x32_out,
+                                et_f16 *out16, et_f16 *QKV, float *partial, uint32_t *join, int spin, int act, float eps1, float eps2,
+                                et_stream stream);
 /* where the streams of a pack lie, for et_mha_fused_ahead_f16 */
 int et_encoder_layer_pack_streams(const struct et_layer_pack_s *pack, et_span *streams);
 int et_encoder_layer_pack_destroy(struct et_layer_pack_s *pack);
@@ -919,9 +929,10 @@ int et_model_forward(et_model m, et_f16 *out, const et_f16 *in, et_stream stream
 int et_model_forward_layer(et_model m, int layer, et_f16 *out, const et_f16 *in,
                            et_stream stream);
 int et_model_sync(et_model m);
-/* kernel launches per encoder layer of a finalized model in the form et_model_forward runs
+/* kernel launches per encoder layer, at most, of a finalized model in the form et_model_forward runs
  * (2: attention and one token-local launch, et_encoder_layer_f32, or, under mixed = 3, one chain
- * launch; 3: attention and a token-local launch in two parts; 4: the QKV projection inside the
+ * launch; 3: attention and a token-local launch whose strips several workgroups share, in two parts, or in
+ * one where the device deals workgroups so that they can meet, et_encoder_layer_joins; 4: the QKV projection inside the
  * attention kernel; 5: SkipLayerNorm folded into the projections; 7: SkipLayerNorm on its own; 0 before
  * et_model_finalize).  A model asked for mixed = 3 reports 5 once it has gone back to separate
  * launches. */

@@ -86,6 +86,8 @@ _SIGNATURES = {
     "et_encoder_layer_pack_create_projecting": (_vp, _i, _i, _i, _i, _i, _i, C.POINTER(_vp)),
     "et_encoder_layer_pack_destroy": (_vp,),
     "et_encoder_layer_pack_streams": (_vp, _vp),
+    "et_encoder_layer_joins": (_vp, C.POINTER(_i)),
+    "et_encoder_layer_joined_f32": (_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _f, _f, _vp),
     "et_encoder_layer_f32": (_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _f, _f, _vp),
     "et_encoder_layer_project_f16": (_vp, _vp, _vp, _vp),
     "et_probe_empty": (_i, _i, _vp),

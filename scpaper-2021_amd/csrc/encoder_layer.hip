@@ -18,16 +18,21 @@
 // Against separate launches per matrix (five to seven a layer) this removes the intermediate activations (at 8192 rows
 // and BERT-base sizes about 300 MB of reads and writes per layer) and the launch boundaries (1.6 us each), and the weight
 // requests never drain: the ring of a wave is filled across barriers, since no weight depends on an activation.
-// 12 layers of BERT-base at 80 %: 64 x 128 tokens 2101 -> 1003 us, 8 x 128 540 -> 457; BERT-large 4 x 512 at 90 % 1842 ->
-// 1355.  On the way: the residual and the shares in tile order instead of rows (lines written in halves by two waves),
+// 12 layers of BERT-base at 80 %, three models in turn: 64 x 128 tokens 2101 -> 889 us, 8 x 128 540 -> 369; BERT-large 4 x 512 at
+// 90 % 1842 -> 1185.  On the way: the residual and the shares in tile order instead of rows (lines written in halves by two waves),
 // QKV' through LDS as whole rows instead of 32 bytes a token, and the parts of a strip on one XCD: 1150 -> 1060 at 64 x
 // 128, 562 -> 480 at 8 x 128; accumulating in place of a zeroed sum and a later addition: 2 %.
 //
-// Few rows leave most compute units without a strip.  Then PARTS workgroups share a strip in two launches: the first
+// Few rows leave most compute units without a strip.  Then PARTS workgroups share a strip.  In two launches the first
 // repeats the output projection and LN1, and each part runs its share of the hidden features, leaving its share of
 // the second product in binary32; the second adds the shares in a fixed order, applies LN2 and runs its share of
 // the QKV block-rows.  That projection can be had alone, of x' as it was rounded for it (et_encoder_layer_project_f16), so
 // that a stack whose layers hand binary16 to each other gives the same bits layer by layer.
+// The joined launch does both: behind the second product the parts of a strip meet at a word in their XCD's L2 (el_wait), and
+// the shares come back out of that L2, where behind a launch boundary they come from the memory-side cache, as do table, offsets
+// and first slots, which here are on their way while the parts meet; 2 us of boundary go besides.  8 x 128 tokens at 80 %
+// 382 -> 361 us (12 layers, weights in the memory-side cache), 12 x 128 241 -> 220 (6 layers), BERT-large 4 x 512 at 90 % 1175 ->
+// 1124.  (The first form of it, with requests only behind the meeting: 387.)
 //
 // Streams (built on the host, et_encoder_layer_pack_create; those of the second launch, or of the projection alone, behind
 // those of the first): per (part, wave) the slots in the order they are multiplied, the byte offsets of their two column
@@ -38,7 +43,9 @@
 #include <algorithm>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "common.hip.h"
@@ -59,6 +66,12 @@ constexpr int kElKindSum = 0, kElKindHidden = 1, kElKindQkv = 2, kElMaxSlots = 2
 typedef int i4 __attribute__((ext_vector_type(4)));
 
 struct LayerArgs {
+    // joined launch: the streams behind the join, and a word per strip
+    const char *slots2, *offs2;
+    const uint32_t *rows2;
+    const int32_t *tab2;
+    uint32_t *join;
+    int cap2, spin;
     const char *slots;
     const char *offs;  // per wave and eight slots: 8 x 16 bits of the first tiles' offsets, 8 of the second
     const uint32_t *rows;  // per (part, wave) 64 kElRowRegs descriptors
@@ -79,7 +92,7 @@ struct LayerArgs {
     int nseg_ff, nseg_q;  // segments of the hidden features, of the projection
     int hbuf;             // bytes between the two hidden buffers (0: one is enough)
     int parts, nshare, act;  // parts of this launch, shares of the second product
-    float eps1, eps2;
+    float eps1, eps2, inv_h;
     uint32_t sums[kElWaves];  // block-rows of the model width a wave holds the sums of, 8 bits each (255: none)
 };
 
@@ -226,10 +239,51 @@ __device__ __forceinline__ int el_here(int v) {
     return v;
 }
 
+__device__ __forceinline__ int el_here_s(int v) {  // the same for a uniform value
+    asm volatile("" : "+s"(v));
+    return v;
+}
+
+// The parts of a strip meet at a word in the L2 of their XCD: arrivals in bits 0-7, parts that did not wait in bits 8-19,
+// parts that are through in bits 20-27; the last to be through puts it back to zero.  Whoever arrives last waits for nobody.
+// The others wait a bounded time, and then leave their share of the projection to the last: nothing ever depends on two
+// workgroups being resident at once.  One wave, its first lane.  (In assembly: the arrival is in flight while the ring goes
+// out, and an addition of nothing, which the wait reads the word with, would become a load that the L1 answers.)
+constexpr int kElMaxJoin = 12;
+#define ET_EL_ADD "s_mov_b64 exec, 1\n\tglobal_atomic_add %0, %1, %2, off sc0\n\ts_mov_b64 exec, -1"
+__device__ __forceinline__ uint32_t el_add(uint32_t *word, uint32_t v) {
+    uint32_t was;
+    asm volatile(ET_EL_ADD "\n\ts_waitcnt vmcnt(0)" : "=&v"(was) : "v"(word), "v"(v) : "memory");
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)was);
+}
+__device__ __forceinline__ void el_through(uint32_t *word, uint32_t was, int parts) {  // `was`: before this part was counted through
+    if ((int)(was >> 20) + 1 == parts) __hip_atomic_store(word, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+// behind the arrival that found `was`: the parts to run besides one's own, or -1: leave
+__device__ __forceinline__ int el_wait(uint32_t *word, uint32_t was, int part, int parts, bool projecting, int spin) {
+    if ((int)(was & 255) + 1 == parts) return (int)(was >> 8 & 0xfff);
+    if (!projecting) {  // a normalisation alone is for the last
+        el_through(word, el_add(word, 1u << 20), parts);
+        return -1;
+    }
+    for (int n = 0; n < spin; n++) {
+        if ((int)(el_add(word, 0u) & 255) == parts) return 0;
+        __builtin_amdgcn_s_sleep(1);
+    }
+    // (all there after all: the last one could not be told, and the count of those through is taken back)
+    const uint32_t now = el_add(word, (1u << 20) + (1u << (8 + part)));
+    if ((int)(now & 255) == parts) {
+        (void)el_add(word, 0u - (1u << 20));
+        return 0;
+    }
+    el_through(word, now, parts);
+    return -1;
+}
+
 // MODE 0: all steps.  1: up to the second product, binary32 share to `partial`.  2: from the sum of the shares on.  3: the
 // projection alone, of x' as 2 rounds it, given in `Z`: the same products in the same order.
-// NR: block-rows of the model width a wave holds the sums of.
-template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) __attribute__((amdgpu_num_vgpr(kElOwnVgprs))) void encoder_layer_kernel(const LayerArgs a) {
+// 4: 1 and 2 in one launch; behind the second product the parts of a strip meet.
+template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_layer(const LayerArgs &a) {
     extern __shared__ __align__(256) unsigned char el_smem[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -239,14 +293,27 @@ template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) 
     if (MODE != 0 && strip * MT * 16 >= a.T) return;  // padding of the grid (the whole workgroup)
     const int tok0 = strip * (MT * 16);
     const int H = a.H;
+    // The joined launch reads what it needs behind the join when it needs it: held from the start it would not fit the scalar
+    // registers, and a scalar register that comes back from a vector lane must not be read by a request within five
+    // instructions, which the compiler cannot see in the assembly here.
+    auto late = [] {
+        auto *p = (const __attribute__((address_space(4))) LayerArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(p));
+        return p;
+    };
+    constexpr bool kLate = MODE == 4;
+#define ET_EL_ARG(F) (kLate ? late()->F : a.F)
+#define ET_EL_ONCE(F) (kLate || MODE == 0 ? late()->F : a.F)
+    auto here = [](int v) { return kLate ? el_here_s(v) : v; };
 
     unsigned char *X = el_smem;                            // [MT * 16][xs], 16-byte units XORed with the row
     unsigned char *Hb = X + MT * 16 * a.xs;                // [1 or 2 chunks][MT * 16][hs], the same
     float *red = reinterpret_cast<float *>(Hb + a.hbuf + MT * 16 * a.hs);  // [2][16 waves][MT * 16]
     _Float16 *vec = reinterpret_cast<_Float16 *>(red + 2 * kElWaves * MT * 16);
-    const _Float16 *bo = vec, *g1 = bo + H, *be1 = g1 + H, *b1 = be1 + H, *b2 = b1 + a.FF, *g2 = b2 + H, *be2 = g2 + H;
+    // (bo, g1, be1, b1, b2, g2, be2, bq)
 
     // ---- requests: the strip, the vectors, the residual or the shares, all at addresses the arguments give
+    constexpr bool kFirst = MODE < 2 || MODE == 4, kParts = MODE == 1 || MODE == 4;  // begins with Z; has parts of the hidden features
     const int stream = part * kElWaves + wave;
     // A buffer that ends with the wave's last slot: the ring's requests past it go nowhere.  Answered, they were 128 KiB of the
     // 0.9 MiB a workgroup of the first launch took in at 8 x 128 tokens, and of the 0.6 of the second.
@@ -279,7 +346,7 @@ template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) 
     for (int j = 0; j < NR; j++) rb[j] = (own >> (8 * j) & 255) == 255 ? -1 : (int)(own >> (8 * j) & 255);
     // bytes from the strip's first value to a tile in tile order (uniform); a second tile past the end: the first
     const int tiles_here = min(MT, (a.T - tok0) >> 4);
-    auto tile_at = [&](int m, int j) { return (unsigned)(min(m, tiles_here - 1) * H + max(rb[j], 0) * 16) * 64; };
+    auto tile_at = [&](int m, int j) { return (unsigned)((MT == 1 ? 0 : min(m, tiles_here - 1) * H) + max(here(rb[j]), 0) * 16) * 64; };
 
     auto ask_vectors = [&] {  // straight into LDS, 512 values an instruction
         const int nvec = (6 * H + a.FF + (MODE == 1 ? 0 : a.Q)) >> 3;
@@ -330,21 +397,21 @@ template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) 
         el_ring_start(lane_off, offs_off, slots, offs);
         asm volatile("s_waitcnt vmcnt(%0)" ::"i"(kElRingAsks) : "memory");
     };
-    if constexpr (MODE == 3) {
-        ask_vectors();
-        ring_start();
-    } else if constexpr (MODE == 2) {
-        ask_vectors();
-        constexpr int kTogether = NR > 3 ? 2 : 4;  // shares requested together
+    // The shares of a strip, added in the order of the parts, into V; `mine`: the part whose share V holds already (-1: none).
+    // The ring goes out behind the last of them (MODE 4: ahead of them, while the parts meet).
+    auto sum_shares = [&](int mine) {
+        constexpr int kTogether = MODE == 4 ? (NR > 3 ? 1 : 3) : NR > 3 ? 2 : 4;  // shares requested together
+        f4 u[kTogether][NR][MT], sum[NR][MT];
 #pragma unroll
         for (int j = 0; j < NR; j++)
 #pragma unroll
-            for (int m = 0; m < MT; m++) V[j][m] = f4{0.f, 0.f, 0.f, 0.f};
-        f4 u[kTogether][NR][MT];
+            for (int m = 0; m < MT; m++) sum[j][m] = f4{0.f, 0.f, 0.f, 0.f};
+        const int nshare = ET_EL_ARG(nshare);
         auto ask_shares = [&](int p) {
 #pragma unroll
             for (int q = 0; q < kTogether; q++) {
-                const char *src = reinterpret_cast<const char *>(a.partial + ((size_t)min(p + q, a.nshare - 1) * a.T + tok0) * H);
+                if (MODE == 4 && (p + q == mine || p + q >= nshare)) continue;  // uniform
+                const char *src = reinterpret_cast<const char *>(ET_EL_ARG(partial) + ((size_t)min(p + q, nshare - 1) * ET_EL_ARG(T) + tok0) * ET_EL_ARG(H));
 #pragma unroll
                 for (int j = 0; j < NR; j++)
 #pragma unroll
@@ -360,28 +427,40 @@ template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) 
                     for (int m = 0; m < MT; m++) el_tie(u[q][j][m]);
 #pragma unroll
             for (int q = 0; q < kTogether; q++)
-                if (p + q < a.nshare) {  // uniform
+                if (p + q < nshare) {  // uniform
 #pragma unroll
                     for (int j = 0; j < NR; j++)
 #pragma unroll
-                        for (int m = 0; m < MT; m++) V[j][m] += u[q][j][m];
+                        for (int m = 0; m < MT; m++) sum[j][m] += MODE == 4 && p + q == mine ? V[j][m] : u[q][j][m];
                 }
         };
         int p = 0;
-        for (; p + kTogether < a.nshare; p += kTogether) {
+        for (; p + kTogether < nshare; p += kTogether) {
             ask_shares(p);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             add_shares(p);
         }
         ask_shares(p);
-        ring_start();
+        if constexpr (MODE == 4) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        else ring_start();
         add_shares(p);
+#pragma unroll
+        for (int j = 0; j < NR; j++)
+#pragma unroll
+            for (int m = 0; m < MT; m++) V[j][m] = sum[j][m];
+    };
+    if constexpr (MODE == 3) {
+        ask_vectors();
+        ring_start();
+    } else if constexpr (MODE == 2) {
+        ask_vectors();
+        sum_shares(-1);
     } else {
         ask_vectors();
         ask_residual(V);
         ring_start();
     }
-    if constexpr (MODE < 2) keep_residual(V);
+    if constexpr (kFirst) keep_residual(V);
     el_tie(tab);
 #pragma unroll
     for (int i = 0; i < kElRowRegs; i++) el_tie(desc[i]);
@@ -395,9 +474,6 @@ template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) 
     // squared distances from its own mean; the waves exchange both through LDS once, and the second moment about the
     // common mean is the sum of theirs and of the distances of their means.  A wave with fewer than NR block-rows repeats
     // its first one with weight zero, so that nothing here is under a branch and all reads go out together.
-    float live[NR];
-#pragma unroll
-    for (int j = 0; j < NR; j++) live[j] = rb[j] >= 0 ? 1.0f : 0.0f;
     auto vec_of = [&](h4 (&v)[NR], const _Float16 *src) {
         const int g = el_here(lane >> 4);
 #pragma unroll
@@ -405,10 +481,13 @@ template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) 
     };
     // features of this wave, and of the four waves whose sums this lane adds (one over them; 0 for a wave without any)
     const int own_rows = __builtin_amdgcn_readlane(tab, kElTabCount + wave);
-    const float inv_own = own_rows ? 1.0f / (float)(own_rows * 16) : 0.0f;
     auto norm = [&](const _Float16 *add, const _Float16 *gam, const _Float16 *bet, float eps) {
         const int r16 = el_here(lane & 15), g = el_here(lane >> 4), gbit = g & 1;
-        float mean[MT], rstd[MT], n_of[4], inv_of[4];
+        float mean[MT], rstd[MT], n_of[4], inv_of[4], live[NR];
+#pragma unroll
+        for (int j = 0; j < NR; j++) live[j] = here(rb[j]) >= 0 ? 1.0f : 0.0f;
+        const int own_here = here(own_rows);
+        const float inv_own = own_here ? 1.0f / (float)(own_here * 16) : 0.0f;
         if (H == kElWaves * 16 * NR) {  // uniform: every wave holds NR
 #pragma unroll
             for (int k = 0; k < 4; k++) {
@@ -455,7 +534,7 @@ template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) 
             if (g == 0) rd[(wave * MT + m) * 16 + r16] = float2{s, q};
         }
         el_barrier();
-        const float inv_h = 1.0f / (float)H;
+        const float inv_h = ET_EL_ARG(inv_h);
 #pragma unroll
         for (int m = 0; m < MT; m++) {
             float2 part_of[4];
@@ -490,126 +569,225 @@ template <int MT, int NR, int MODE> __global__ __launch_bounds__(kElWaves * 64) 
             }
     };
 
-    const int first_seg = MODE == 3 ? a.nseg_ff + 1 : MODE == 2 ? a.nseg_ff : 0, last_seg = a.nseg_ff + (MODE == 1 ? 0 : a.nseg_q);
-    const int q_first = MODE == 1 ? 0 : (a.Q >> 4) * part / a.parts, q_rows = MODE == 1 ? 0 : (a.Q >> 4) * (part + 1) / a.parts - q_first;
-    const int act = a.act;
-    int pos = 0;
-    int row_no = 0;
-    for (int seg = first_seg;; seg++) {  // (the shares' sum enters behind the last hidden segment, which holds no rows there)
-        const int nrows = __builtin_amdgcn_readlane(tab, kElTabSeg + seg);
-        // hidden chunk c is written in segment c + 1 and read in the next; projection chunk c is written in nseg_ff + 1 + c
-        const unsigned odd = (seg > a.nseg_ff ? seg - a.nseg_ff : seg) & 1, hb_up = odd ? 0u : hbuf, hb_dn = odd ? hbuf : 0u;
-        for (int r = 0; r < nrows; r++) {
-            const uint32_t d = (uint32_t)__builtin_amdgcn_readlane(row_no < 64 ? desc[0] : desc[1], row_no & 63);
-            row_no++;
-            // A SIMD's oldest wave is served first by the memory pipe, which bounds a segment, and the youngest ones end it
-            // a third later: more rows left go first (390 -> 382 us at 8 x 128, 1026 -> 1003 at 64 x 128).
-            if (nrows - r >= 3) __builtin_amdgcn_s_setprio(3);
-            else if (nrows - r == 2) __builtin_amdgcn_s_setprio(2);
-            else __builtin_amdgcn_s_setprio(1);
-            const int n = d & 255, kind = (d >> 8) & 3, target = (d >> 11) & 1023, bias_at = (d >> 21) * 16;
-            const bool hid = (d >> 10) & 1;
-            const unsigned ld = hid ? a.hs : a.xs;
-            const unsigned base = (hid ? MT * 16 * a.xs + hb_dn : 0u) + (unsigned)el_here(lane & 15) * ld, step = 16 * ld;
-            if constexpr (MODE != 3) {
-                if (kind == kElKindSum) {
+    // MODE 4, behind the second product: this part's share goes to memory, the parts meet, the shares come back.  False:
+    // the rest is left to another part.  `others`: parts whose projection is run here besides this one's.
+    unsigned others = 0;
+    int who = part;
+    auto ask_stream = [&](int s) {  // of the second launch's streams: table, descriptors and first offsets
+        const auto *l = late();
+        const int cap2 = l->cap2;
+        const char *at = l->offs2 + (size_t)s * cap2 * 4;
+        offs = at;
+        offs_off = (g >> 1) * 16;
+        lane_off = lane * 16;
+        el_ask_offsets(offs_off, offs);
+        el_ask(tab, lane * 4, l->tab2 + (size_t)s * kElTab);
 #pragma unroll
-                    for (int j = 0; j < NR; j++)
-                        if (target == j) el_row<MT>(V[j], n, pos, base, step, kx, lane_off, offs_off, slots, offs);
-                    continue;
-                }
-            }
-            const h4 bv = *reinterpret_cast<const h4 *>(vec + bias_at + el_here(lane >> 4) * 4);
-            f4 acc[MT];
+        for (int i = 0; i < kElRowRegs; i++) el_ask(desc[i], lane * 4, l->rows2 + ((size_t)s * kElRowRegs + i) * 64);
+        const uint64_t slots_at = (uint64_t)(l->slots2 + (size_t)s * cap2 * 1024);
+        slots = i4{(int)(unsigned)slots_at, (int)(unsigned)(slots_at >> 32), cap2 * 1024, kElBufferWord};
+    };
+    auto have_stream = [&] {
+        el_tie(tab);
 #pragma unroll
-            for (int m = 0; m < MT; m++) acc[m] = f4{(float)bv[0], (float)bv[1], (float)bv[2], (float)bv[3]};
-            if (n) el_row<MT>(acc, n, pos, base, step, kx, lane_off, offs_off, slots, offs);
-            if (kind == kElKindHidden) {
-                if (act == ET_ACT_GELU) {
-#pragma unroll
-                    for (int m = 0; m < MT; m++)
-#pragma unroll
-                        for (int e = 0; e < 4; e++) acc[m][e] = gelu_tanh(acc[m][e]);
-                } else if (act == ET_ACT_RELU) {
-#pragma unroll
-                    for (int m = 0; m < MT; m++)
-#pragma unroll
-                        for (int e = 0; e < 4; e++) acc[m][e] = fmaxf(acc[m][e], 0.0f);
-                }
-            }
-            const int r16 = el_here(lane & 15);
-            const unsigned u = (unsigned)target * 2 + (g >> 1);
-#pragma unroll
-            for (int m = 0; m < MT; m++)
-                *reinterpret_cast<h4 *>(Hb + hb_up + (m * 16 + r16) * a.hs + ((u ^ r16) << 4) + gbit * 8) =
-                    h4{(_Float16)acc[m][0], (_Float16)acc[m][1], (_Float16)acc[m][2], (_Float16)acc[m][3]};
-        }
-        const bool first = MODE < 2 && seg == 0;
-        if (first || ((MODE == 0 || MODE == 2) && seg == a.nseg_ff)) {
-            norm(first ? bo : nullptr, first ? g1 : g2, first ? be1 : be2, first ? a.eps1 : a.eps2);
-            if (first) {
-                if (MODE == 1 && part != 0) {
-#pragma unroll
-                    for (int j = 0; j < NR; j++)
-#pragma unroll
-                        for (int m = 0; m < MT; m++) V[j][m] = f4{0.f, 0.f, 0.f, 0.f};
-                } else {
-                    h4 bv[NR];
-                    vec_of(bv, b2);
-#pragma unroll
-                    for (int j = 0; j < NR; j++)
-#pragma unroll
-                        for (int m = 0; m < MT; m++)
-#pragma unroll
-                            for (int e = 0; e < 4; e++) V[j][m][e] += (float)bv[j][e];
-                }
-            } else if (part == 0) {
-                if (a.x32_out) {
-                    char *dst = reinterpret_cast<char *>(a.x32_out + (size_t)tok0 * H);
-                    const unsigned at16 = el_here(lane) * 16;
-#pragma unroll
-                    for (int j = 0; j < NR; j++)
-#pragma unroll
-                        for (int m = 0; m < MT; m++)
-                            if (rb[j] >= 0 && m < tiles_here) *reinterpret_cast<f4 *>(dst + (tile_at(m, j) + at16)) = V[j][m];
-                }
-                if (a.out16) {
-                    const int r16 = el_here(lane & 15), g = el_here(lane >> 4);
-                    char *dst = reinterpret_cast<char *>(a.out16 + (size_t)tok0 * H);
-#pragma unroll
-                    for (int j = 0; j < NR; j++)
-#pragma unroll
-                        for (int m = 0; m < MT; m++)
-                            if (rb[j] >= 0 && m < tiles_here)
-                                *reinterpret_cast<h4 *>(dst + ((unsigned)(m * 16 + r16) * H * 2 + rb[j] * 32 + g * 8)) =
-                                    h4{(_Float16)V[j][m][0], (_Float16)V[j][m][1], (_Float16)V[j][m][2], (_Float16)V[j][m][3]};
-                }
-            }
-        }
-        if (MODE != 1 && seg > a.nseg_ff) {  // the projection's chunk leaves the LDS, whole rows of it at a time
-            el_barrier();
-            const int c = seg - a.nseg_ff - 1, first_rb = q_first + q_rows * c / a.nseg_q, units = (q_first + q_rows * (c + 1) / a.nseg_q - first_rb) * 2;
-            const unsigned char *src = Hb + ((c & 1) ? hbuf : 0u);
-            for (int t = wave; t < tiles_here * 16; t += kElWaves) {
-                char *dst = reinterpret_cast<char *>(a.qkv + (size_t)(tok0 + t) * a.Q + first_rb * 16);
-                for (int u = el_here(lane); u < units; u += 64)
-                    *reinterpret_cast<h8 *>(dst + u * 16) = *reinterpret_cast<const h8 *>(src + t * a.hs + ((u ^ (t & 15)) << 4));
-            }
-            if (seg == last_seg) break;
-            continue;
-        }
-        if (seg == last_seg) break;
-        el_barrier();
-    }
-    if constexpr (MODE == 1) {
-        char *dst = reinterpret_cast<char *>(a.partial + ((size_t)part * a.T + tok0) * H);
+        for (int i = 0; i < kElRowRegs; i++) el_tie(desc[i]);
+        slots[2] = __builtin_amdgcn_readlane(tab, kElTabSlots) * 1024;
+    };
+    auto store_share = [&] {
+        char *dst = reinterpret_cast<char *>(ET_EL_ARG(partial) + ((size_t)part * ET_EL_ARG(T) + tok0) * ET_EL_ARG(H));
         const unsigned at16 = el_here(lane) * 16;
 #pragma unroll
         for (int j = 0; j < NR; j++)
 #pragma unroll
             for (int m = 0; m < MT; m++)
-                if (rb[j] >= 0 && m < tiles_here) *reinterpret_cast<f4 *>(dst + (tile_at(m, j) + at16)) = V[j][m];
+                if (here(rb[j]) >= 0 && m < tiles_here) *reinterpret_cast<f4 *>(dst + (tile_at(m, j) + at16)) = V[j][m];
+    };
+    auto join = [&]() -> bool {
+        ask_stream((ET_EL_ARG(Q) ? part : 0) * kElWaves + wave);
+        store_share();
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // in the L2
+        el_barrier();
+        int *got = reinterpret_cast<int *>(red);
+        if (wave == 0) {
+            const auto *l = late();
+            uint32_t *const word = l->join + strip, was;
+            asm volatile(ET_EL_ADD : "=&v"(was) : "v"(word), "v"(1u) : "memory");
+            el_ring_start(lane_off, offs_off, slots, offs);
+            asm volatile("s_waitcnt vmcnt(%0)" ::"i"(kElRingAsks) : "memory");
+            el_tie(was);
+            *got = el_wait(word, (uint32_t)__builtin_amdgcn_readfirstlane((int)was), part, l->parts, l->Q > 0, l->spin);
+        } else {
+            el_ring_start(lane_off, offs_off, slots, offs);
+        }
+        el_barrier();
+        const int mask = __builtin_amdgcn_readfirstlane(*got);
+        if (mask < 0) return false;
+        others = (unsigned)mask;
+        el_barrier();  // (`red` is written again)
+        sum_shares(part);
+        have_stream();
+        return true;
+    };
+
+    const int act = a.act;
+    auto write_out = [&] {  // x', once for a strip
+        const int H = ET_EL_ONCE(H);
+        if (float *const to = ET_EL_ONCE(x32_out)) {
+            char *dst = reinterpret_cast<char *>(to + (size_t)tok0 * H);
+            const unsigned at16 = el_here(lane) * 16;
+#pragma unroll
+            for (int j = 0; j < NR; j++)
+#pragma unroll
+                for (int m = 0; m < MT; m++)
+                    if (here(rb[j]) >= 0 && m < tiles_here) *reinterpret_cast<f4 *>(dst + (tile_at(m, j) + at16)) = V[j][m];
+        }
+        if (_Float16 *const to = ET_EL_ONCE(out16)) {
+            const int r16 = el_here(lane & 15), g = el_here(lane >> 4);
+            char *dst = reinterpret_cast<char *>(to + (size_t)tok0 * H);
+#pragma unroll
+            for (int j = 0; j < NR; j++)
+#pragma unroll
+                for (int m = 0; m < MT; m++)
+                    if (here(rb[j]) >= 0 && m < tiles_here)
+                        *reinterpret_cast<h4 *>(dst + ((unsigned)(m * 16 + r16) * H * 2 + here(rb[j]) * 32 + g * 8)) =
+                            h4{(_Float16)V[j][m][0], (_Float16)V[j][m][1], (_Float16)V[j][m][2], (_Float16)V[j][m][3]};
+        }
+    };
+    auto norm_k = [&](bool first) {
+        const int H = ET_EL_ONCE(H);
+        const _Float16 *const b2 = vec + 3 * H + ET_EL_ONCE(FF), *const gam = first ? vec + H : b2 + H;
+        norm(first ? vec : nullptr, gam, gam + H, first ? ET_EL_ONCE(eps1) : ET_EL_ONCE(eps2));
+        if (first && !(kParts && part != 0)) {  // the second product is added to y + b2
+            h4 bv[NR];
+            vec_of(bv, b2);
+#pragma unroll
+            for (int j = 0; j < NR; j++)
+#pragma unroll
+                for (int m = 0; m < MT; m++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) V[j][m][e] += (float)bv[j][e];
+        } else if (first) {
+#pragma unroll
+            for (int j = 0; j < NR; j++)
+#pragma unroll
+                for (int m = 0; m < MT; m++) V[j][m] = f4{0.f, 0.f, 0.f, 0.f};
+        }
+    };
+    // The segments of a launch (PHASE 0), or of a joined one up to the second product (1) and of the projection (2).
+    auto run = [&](auto phase) {
+        constexpr int PHASE = decltype(phase)::value;
+        int pos = 0, row_no = 0;
+        const int first_seg = MODE == 3 || PHASE == 2 ? a.nseg_ff + 1 : MODE == 2 ? a.nseg_ff : 0;
+        const int last_seg = a.nseg_ff + (MODE == 1 || PHASE == 1 ? 0 : a.nseg_q);
+        for (int seg = first_seg;; seg++) {  // (the shares' sum enters behind the last hidden segment, which holds no rows there)
+            const int nrows = __builtin_amdgcn_readlane(tab, kElTabSeg + seg);
+            // hidden chunk c is written in segment c + 1 and read in the next; projection chunk c is written in nseg_ff + 1 + c
+            const unsigned odd = (seg > a.nseg_ff ? seg - a.nseg_ff : seg) & 1, hb_up = odd ? 0u : hbuf, hb_dn = odd ? hbuf : 0u;
+            for (int r = 0; r < nrows; r++) {
+                const uint32_t d = (uint32_t)__builtin_amdgcn_readlane(row_no < 64 ? desc[0] : desc[1], row_no & 63);
+                row_no++;
+                // A SIMD's oldest wave is served first by the memory pipe, which bounds a segment, and the youngest ones end it
+                // a third later: more rows left go first (390 -> 382 us at 8 x 128, 1026 -> 1003 at 64 x 128).
+                if (nrows - r >= 3) __builtin_amdgcn_s_setprio(3);
+                else if (nrows - r == 2) __builtin_amdgcn_s_setprio(2);
+                else __builtin_amdgcn_s_setprio(1);
+                const int n = d & 255, kind = (d >> 8) & 3, target = (d >> 11) & 1023, bias_at = (d >> 21) * 16;
+                const bool hid = (d >> 10) & 1;
+                const unsigned ld = hid ? a.hs : a.xs;
+                const unsigned base = (hid ? MT * 16 * a.xs + hb_dn : 0u) + (unsigned)el_here(lane & 15) * ld, step = 16 * ld;
+                if constexpr (MODE != 3 && PHASE != 2) {
+                    if (kind == kElKindSum) {
+#pragma unroll
+                        for (int j = 0; j < NR; j++)
+                            if (target == j) el_row<MT>(V[j], n, pos, base, step, kx, lane_off, offs_off, slots, offs);
+                        continue;
+                    }
+                }
+                const h4 bv = *reinterpret_cast<const h4 *>(vec + bias_at + el_here(lane >> 4) * 4);
+                f4 acc[MT];
+#pragma unroll
+                for (int m = 0; m < MT; m++) acc[m] = f4{(float)bv[0], (float)bv[1], (float)bv[2], (float)bv[3]};
+                if (n) el_row<MT>(acc, n, pos, base, step, kx, lane_off, offs_off, slots, offs);
+                if (PHASE != 2 && kind == kElKindHidden) {
+                    if (act == ET_ACT_GELU) {
+#pragma unroll
+                        for (int m = 0; m < MT; m++)
+#pragma unroll
+                            for (int e = 0; e < 4; e++) acc[m][e] = gelu_tanh(acc[m][e]);
+                    } else if (act == ET_ACT_RELU) {
+#pragma unroll
+                        for (int m = 0; m < MT; m++)
+#pragma unroll
+                            for (int e = 0; e < 4; e++) acc[m][e] = fmaxf(acc[m][e], 0.0f);
+                    }
+                }
+                const int r16 = el_here(lane & 15);
+                const unsigned u = (unsigned)target * 2 + (g >> 1);
+#pragma unroll
+                for (int m = 0; m < MT; m++)
+                    *reinterpret_cast<h4 *>(Hb + hb_up + (m * 16 + r16) * a.hs + ((u ^ r16) << 4) + gbit * 8) =
+                        h4{(_Float16)acc[m][0], (_Float16)acc[m][1], (_Float16)acc[m][2], (_Float16)acc[m][3]};
+            }
+            const bool first = kFirst && PHASE != 2 && seg == 0;
+            if (first || (PHASE == 0 && (MODE == 0 || MODE == 2) && seg == ET_EL_ARG(nseg_ff))) {
+                norm_k(first);
+                if (!first && part == 0) write_out();
+            }
+            if (MODE != 1 && PHASE != 1 && seg > ET_EL_ARG(nseg_ff)) {  // the projection's chunk leaves the LDS, whole rows of it at a time
+                el_barrier();
+                const int Q = ET_EL_ARG(Q), nb = Q >> 4, np = MODE == 0 ? 1 : ET_EL_ARG(parts), nq = ET_EL_ARG(nseg_q), hs = ET_EL_ARG(hs);
+                const int q_first = MODE == 0 ? 0 : nb * who / np, q_rows = MODE == 0 ? nb : nb * (who + 1) / np - q_first;
+                const int c = seg - ET_EL_ARG(nseg_ff) - 1, first_rb = q_first + q_rows * c / nq, units = (q_first + q_rows * (c + 1) / nq - first_rb) * 2;
+                const unsigned char *src = Hb + ((c & 1) ? hbuf : 0u);
+                _Float16 *const qkv = ET_EL_ARG(qkv);
+                for (int t = wave; t < tiles_here * 16; t += kElWaves) {
+                    char *dst = reinterpret_cast<char *>(qkv + (size_t)(tok0 + t) * Q + first_rb * 16);
+                    for (int u = el_here(lane); u < units; u += 64)
+                        *reinterpret_cast<h8 *>(dst + u * 16) = *reinterpret_cast<const h8 *>(src + t * hs + ((u ^ (t & 15)) << 4));
+                }
+                if (c == nq - 1) break;
+                continue;
+            }
+            if (seg == last_seg) break;
+            el_barrier();
+        }
+    };
+    if constexpr (MODE != 4) {
+        run(std::integral_constant<int, 0>{});
+        if constexpr (MODE == 1) store_share();
+    } else {
+        run(std::integral_constant<int, 1>{});
+        if (!join()) return;
+        norm_k(false);
+        if (part == 0 || (others & 1) || ET_EL_ARG(Q) == 0) write_out();
+        if (ET_EL_ARG(Q) > 0) {
+            el_barrier();
+            for (;;) {
+                run(std::integral_constant<int, 2>{});
+                if (others == 0) break;
+                // the projection of a part whose workgroup did not wait
+                who = __builtin_ctz(others);
+                others &= others - 1;
+                el_barrier();  // this one's has left the LDS
+                ask_stream(who * kElWaves + wave);
+                ring_start();
+                have_stream();
+            }
+        }
+        if (wave == 0) {
+            const auto *l = late();
+            uint32_t *const word = l->join + strip;
+            el_through(word, el_add(word, 1u << 20), l->parts);
+        }
     }
+}
+
+template <int MT, int NR, int MODE>
+__global__ __launch_bounds__(kElWaves * 64) __attribute__((amdgpu_num_vgpr(kElOwnVgprs))) void encoder_layer_kernel(const LayerArgs a) {
+    encoder_layer<MT, NR, MODE>(a);
+}
+template <int NR> __global__ __launch_bounds__(kElWaves * 64) __attribute__((amdgpu_num_vgpr(kElOwnVgprs))) void encoder_layer_joined_kernel(const LayerArgs a) {
+    encoder_layer<1, NR, 4>(a);
 }
 
 // slot s = tiles order[2s], order[2s + 1] (bits 28-29: which weight; negative: a zero tile) in lane order: the 16-byte
@@ -939,7 +1117,9 @@ int et_encoder_layer_pack_destroy(struct et_layer_pack_s *pack) {
 
 namespace et {
 template <int MT, int NR, int MODE> static int el_launch(const LayerArgs &a, size_t lds, int blocks, hipStream_t stream) {
-    auto kernel = encoder_layer_kernel<MT, NR, MODE>;
+    void (*kernel)(LayerArgs);
+    if constexpr (MODE == 4) kernel = encoder_layer_joined_kernel<NR>;
+    else kernel = encoder_layer_kernel<MT, NR, MODE>;
     static bool raised = false;  // per instantiation
     if (!raised) {
         ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kElLds));
@@ -968,6 +1148,7 @@ static LayerArgs el_args(const et_layer_pack_s &p) {
     a.vec = static_cast<const _Float16 *>(p.vec);
     a.cap = p.cap;
     std::copy(p.sums, p.sums + kElWaves, a.sums);
+    a.inv_h = 1.0f / (float)p.H;
     a.T = p.T, a.H = p.H, a.FF = p.FF, a.Q = p.Q;
     a.xs = p.xs, a.hs = p.hs, a.nseg_ff = p.nseg_ff, a.nseg_q = p.nseg_q, a.hbuf = p.hbuf, a.parts = a.nshare = p.parts;
     return a;
@@ -1001,8 +1182,49 @@ extern "C" int et_encoder_layer_project_f16(const struct et_layer_pack_s *p, con
     return el_launch<1, 2, 3>(a, p->lds, (strips + 7) / 8 * 8 * a.parts, as_stream(stream));
 }
 
-extern "C" int et_encoder_layer_f32(const struct et_layer_pack_s *p, const et_f16 *Z, const float *x32, const et_f16 *x16, float *x32_out,
-                                    et_f16 *out16, et_f16 *QKV, float *partial, int act, float eps1, float eps2, et_stream stream) {
+// Workgroups of equal id modulo 8 share an XCD, as they are dealt out: looked at once per device.
+namespace et {
+__global__ void el_xcc_kernel(uint32_t *xcc) {
+    if (threadIdx.x == 0) xcc[blockIdx.x] = __builtin_amdgcn_s_getreg((3 << 11) | 20) & 15u;  // XCC_ID
+}
+static int el_xcd_by_id(bool *by_id) {
+    static std::mutex lock;
+    static int known[64] = {};  // 1: yes, 2: no
+    int dev = 0;
+    ET_HIP(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> hold(lock);
+    int &k = known[std::min(dev, 63)];
+    if (!k) {
+        constexpr int n = 512;
+        void *d = nullptr;
+        int s = et_malloc(&d, n * sizeof(uint32_t));
+        uint32_t h[n];
+        if (s == ET_OK) {
+            el_xcc_kernel<<<n, 64>>>(static_cast<uint32_t *>(d));
+            s = check_launch("el_xcc_kernel");
+            if (s == ET_OK) s = check_hip(hipMemcpy(h, d, sizeof h, hipMemcpyDeviceToHost), "hipMemcpy");
+        }
+        (void)et_free(d);
+        if (s != ET_OK) return s;
+        k = 1;
+        for (int i = 8; i < n; i++)
+            if (h[i] != h[i % 8]) k = 2;
+    }
+    *by_id = k == 1;
+    return ET_OK;
+}
+}  // namespace et
+
+extern "C" int et_encoder_layer_joins(const struct et_layer_pack_s *p, int *joins) {
+    ET_REQUIRE(p && joins, ET_ERR_INVALID_ARG, "et_encoder_layer_joins: NULL pointer");
+    bool by_id = false;
+    const int s = p->parts > 1 && p->parts <= kElMaxJoin ? el_xcd_by_id(&by_id) : ET_OK;
+    *joins = by_id;
+    return s;
+}
+
+static int el_run(const struct et_layer_pack_s *p, const et_f16 *Z, const float *x32, const et_f16 *x16, float *x32_out,
+                  et_f16 *out16, et_f16 *QKV, float *partial, uint32_t *join, int spin, int act, float eps1, float eps2, et_stream stream) {
     ET_REQUIRE(p && Z && (x32 || x16) && (p->Q == 0 || QKV) && (p->parts == 1 || partial), ET_ERR_INVALID_ARG,
                "et_encoder_layer_f32: NULL pointer");
     ET_REQUIRE(act >= ET_ACT_NONE && act <= ET_ACT_GELU, ET_ERR_INVALID_ARG, "et_encoder_layer_f32: act=%d", act);
@@ -1025,9 +1247,33 @@ extern "C" int et_encoder_layer_f32(const struct et_layer_pack_s *p, const et_f1
     a.eps1 = eps1, a.eps2 = eps2;
     const int strips = (p->T + p->mt * 16 - 1) / (p->mt * 16);
     hipStream_t st = as_stream(stream);
+    if (join) {
+        LayerArgs second = a;
+        el_second(second, *p);
+        a.slots2 = second.slots, a.offs2 = second.offs, a.rows2 = second.rows, a.tab2 = second.tab, a.cap2 = second.cap;
+        a.join = join, a.spin = spin;
+        return el_dispatch<1, 4>(a, *p, (strips + 7) / 8 * 8 * p->parts, st);
+    }
     if (p->parts == 1) return p->mt == 2 ? el_dispatch<2, 0>(a, *p, strips, st) : el_dispatch<1, 0>(a, *p, strips, st);
     const int s = el_dispatch<1, 1>(a, *p, (strips + 7) / 8 * 8 * p->parts, st);
     if (s != ET_OK) return s;
     el_second(a, *p);
     return el_dispatch<1, 2>(a, *p, (strips + 7) / 8 * 8 * a.parts, st);
+}
+
+extern "C" int et_encoder_layer_f32(const struct et_layer_pack_s *p, const et_f16 *Z, const float *x32, const et_f16 *x16, float *x32_out,
+                                    et_f16 *out16, et_f16 *QKV, float *partial, int act, float eps1, float eps2, et_stream stream) {
+    return el_run(p, Z, x32, x16, x32_out, out16, QKV, partial, nullptr, 0, act, eps1, eps2, stream);
+}
+
+extern "C" int et_encoder_layer_joined_f32(const struct et_layer_pack_s *p, const et_f16 *Z, const float *x32, const et_f16 *x16, float *x32_out,
+                                           et_f16 *out16, et_f16 *QKV, float *partial, uint32_t *join, int spin, int act, float eps1, float eps2,
+                                           et_stream stream) {
+    int joins = 0;
+    ET_REQUIRE(join && (reinterpret_cast<uintptr_t>(join) & 3) == 0 && spin >= 0, ET_ERR_INVALID_ARG, "et_encoder_layer_joined_f32: join=%p spin=%d",
+               static_cast<void *>(join), spin);
+    const int s = et_encoder_layer_joins(p, &joins);
+    if (s != ET_OK) return s;
+    ET_REQUIRE(joins, ET_ERR_UNSUPPORTED, "et_encoder_layer_joined_f32: one part, more than %d, or a device that deals workgroups otherwise", kElMaxJoin);
+    return el_run(p, Z, x32, x16, x32_out, out16, QKV, partial, join, spin, act, eps1, eps2, stream);
 }

@@ -121,6 +121,7 @@ struct et_model_s {
     std::vector<std::unique_ptr<et_layer_pack_s, LayerPackDeleter>> local;
     std::unique_ptr<et::DeviceBuffer<float>> local_x[2];
     std::vector<std::unique_ptr<et::DeviceBuffer<float>>> local_shares;
+    std::vector<std::unique_ptr<et::DeviceBuffer<int>>> local_join;  // words at which the parts of a strip meet, a buffer for each of the shares
     float *shares(int layer) const { return local_shares.empty() ? nullptr : local_shares[(size_t)layer]->get(); }
 
     stream_t own_stream = nullptr;
@@ -326,31 +327,30 @@ bool chain_ran_clean(et_model_s &m, std::string &why) {
 struct LocalPlan {
     int mt = 0, parts = 1;
 };
-// Every workgroup streams the kept tiles of the output projection and its share of the others at about 112 KiB/us, and
-// sharing a strip costs a second launch and the exchange of the shares, about 5 us and half a microsecond per share
-// (fitted at 768 wide, 60 to 95 % sparsity, 256 to 2048 rows): the number of parts that makes the sum least, while there
-// is a compute unit for every workgroup of an XCD.  Above 256 strips of 16 rows a workgroup takes 32.
-// Which stacks run it: time of the separate launches over that of these, two- to four-layer stacks, 384, 768 and 1024 wide
-// (and 512 up to 512 rows), 0 to 95 % sparsity.  `fused`: the separate launches would hold QKV in the attention kernel.
-//   above 4096 rows                                       1.04 - 2.0
-//   kept tiles above 16.5 KiB a feature (768 wide below 10 % sparsity, 1024 below 30 %: dense GEMMs beside) 0.76 - 1.06
-//   up to 512 wide                                        0.96 - 1.98 (0.96 - 0.98: 64 and 128 rows)
-//   above 512 rows                                        0.95 - 1.98 (0.95 - 0.97: FFN of a quarter of the width, 1024 rows)
-//   257 to 480 rows (a 32-row strip more for some XCDs)   0.95 - 1.43 (below 1: unpruned)
-//   481 to 512 rows: denser than half 1.18 - 1.25 (unpruned 0.99), else up to 14.5 us of the estimate 0.98 - 1.13, above 0.93 - 0.98
-//   256 rows and fewer, denser than half                  0.75 - 1.04
-//     112 and 128 rows (the separate launches have a strip for each XCD)      0.85 - 1.00, at 95 % sparsity 0.94 - 1.05
-//     up to 48 rows, 144 to 192 (one XCD more than another has two strips)    1.00 - 1.95, measured up to 19 us
-//     others: up to 14.5 us 1.00 - 1.16 (with `fused` above 192 rows 0.94 - 1.02; 800 wide, 208 hidden, 256 rows 0.92 at 13.8), above
-//     0.91 - 1.04
-// And under mixed = 0, three layers; "light" is up to 11 KiB of tiles a feature, "half" at most half of the tiles kept (denser
-// layers run dense GEMMs beside):
-//   above 4096 rows: up to 18 KiB a feature 1.07 - 1.98, 1024 wide unpruned (24) 0.78
-//   513 to 4096: half 1.01 - 1.77 (an FFN narrower than the model 0.94 - 1.53), denser and light 1.03 - 1.43 (512 wide unpruned
-//     0.90 at 2048 and 4096), else 0.67 - 1.03
-//   481 to 512: denser and light 1.04 - 1.24, half up to 512 wide 1.05 - 1.20, wider up to 11 us 1.00 - 1.20, above 0.87 - 1.06
-//   257 to 480: up to 45 % kept 1.01 - 1.31 (800 wide, 208 hidden, 40 % kept 0.96 once), denser and light 0.97 - 1.21, else 0.70 - 0.99
-//   256: up to 6 us 1.00 - 1.09, else 0.69 - 1.02; fewer: left to the separate launches
+// Every workgroup streams the kept tiles of the output projection and its share of the others at about 112 KiB/us.  Sharing a
+// strip costs a meeting of its parts and half a microsecond a part, more where an XCD has many strips (fitted at 768 wide, 60 to
+// 95 % sparsity, 128 to 2048 rows, shared strips in one launch): the number of parts that makes the sum least, while there is a
+// compute unit for every workgroup of an XCD; beyond eight the shares cost more than they save (128 rows at 60 %, four layers:
+// 134 us with 8, 144 with 12).  Above 256 strips of 16 rows a workgroup takes 32.
+// Which stacks run it: time of the separate launches over that of these, four-layer stacks 512, 768 and 1024 wide, 20 to 95 %
+// sparsity; "half" is at most half of the tiles kept (denser layers run dense GEMMs beside), us the estimate above.
+//   above 4096 rows                       1.04 - 2.0; mixed = 0 up to 18 KiB of tiles a feature 1.07 - 1.98, 1024 wide unpruned (24) 0.78
+//   more than 16.5 KiB of tiles a feature 0.71 - 0.98
+//  binary32 residual:
+//   257 rows and more                     1.06 - 2.0
+//   193 to 256: half, to 18 us 1.03 - 1.39, above (1024 wide at 60 %) 0.92 - 0.95; denser, to 21 us 1.12 - 1.25, above 0.84 - 1.08
+//   144 to 192                            1.04 - 1.33
+//   112 and 128 (the separate launches have a strip for each XCD): half, to 13.5 us 1.02 - 1.14, above 0.91 - 1.05; denser, to 20.5 us
+//                                         1.03 - 1.30, above 0.75 - 0.95
+//   fewer: half 1.08 - 1.58, denser to 20.5 us 0.99 - 1.27, above 0.71 - 0.94
+//  binary16 between layers (mixed = 0):
+//   257 rows and more: half 1.04 - 1.54; denser, to 11 KiB of tiles a feature 1.10 - 1.36, above 0.80 - 1.08
+//   256: to 12.5 us 1.02 - 1.08, above 0.81 - 0.98;  193 to 240: to 20.5 us 1.03 - 1.09, above 0.95 - 0.99
+//   144 to 192: to 23 us 1.01 - 1.29;  128: to 11 us 1.00 - 1.06, above 0.69 - 0.98;  112: to 14.6 us 1.03 - 1.14, above 0.77 - 0.90
+//   fewer: half 1.03 - 1.39, denser to 15 us 1.03 - 1.17, above 0.84 - 1.00
+// Stacks of fewer than six layers keep the lines that were drawn when a shared strip took two launches (`former` is the estimate of
+// that), so that the form a short stack takes, which et_model_launches_per_layer reports, stays what it was; past them the one
+// launch would gain less there than in deep stacks (768 wide at 80 %, 128 rows: two layers 63.1 / 60.8 us, twelve 333.8 / 313.3).
 LocalPlan plan_local(const et_model_s &m, bool fused) {
     LocalPlan p;
     const et_model_desc &d = m.desc;
@@ -360,39 +360,52 @@ LocalPlan plan_local(const et_model_s &m, bool fused) {
             if (h.w[(size_t)w].kind != HostMatrix::Bsr16) return p;
             kib[w] += 0.5 * (double)h.w[(size_t)w].column.size() / (double)m.host.size();
         }
-    const int rows = m.rows(), strips = (rows + 15) / 16;
+    const int rows = m.rows(), strips = (rows + 15) / 16, per_xcd = (strips + 7) / 8;
     const double shared = kib[ET_W_QKV] + kib[ET_W_FF1] + kib[ET_W_FF2], kept = kib[ET_W_O] + shared;
     const double all = (4.0 * d.emdim + 2.0 * d.dimFF) * d.emdim / 512.0;  // KiB of all tiles
     if (strips > 256) {
         if (d.mixed || kept <= 18.0 * d.emdim) p.mt = 2;
         return p;
     }
-    double best = 0;
-    for (int parts = 1; parts <= std::min(12, d.dimFF / 16) && parts * ((strips + 7) / 8) <= 32; parts++) {
-        const double us = (kib[ET_W_O] + shared / parts) / 112.0 + (parts > 1 ? 5.0 + 0.5 * parts : 0.0);
+    double best = 0, former = 0;
+    for (int parts = 1; parts <= std::min(12, d.dimFF / 16) && parts * per_xcd <= 32; parts++) {
+        const double two = (kib[ET_W_O] + shared / parts) / 112.0 + (parts > 1 ? 5.0 + 0.5 * parts : 0.0);
+        former = parts == 1 ? two : std::min(former, two);
+        if (parts > 8) continue;
+        const double us = (kib[ET_W_O] + shared / parts) / 112.0 + (parts > 1 ? 0.5 + (0.45 + 0.045 * per_xcd) * parts : 0.0);
         if (parts == 1 || us < best) {
             best = us;
             p.parts = parts;
         }
     }
-    // With an FFN of some size, four parts are the least where there is room for four (five layers, us, four parts / what the
-    // estimate takes: 384 wide at 70 % 123 / 135 at 128 rows and 130 / 136 at 1024, 768 wide at 95 % 134 / 148 at 128 and
-    // 136 / 149 at 256); without one the single launch is the fastest form (800 wide, 208 hidden features: 171 / 162).
-    if (kib[ET_W_FF1] + kib[ET_W_FF2] >= 256.0 && 4 * ((strips + 7) / 8) <= 32) p.parts = std::max(p.parts, 4);
+    const bool half = kept <= 0.5 * all;
+    const auto short_on = [&]() -> bool {
+        const bool light = kept <= 11.0 * d.emdim;
+        if (d.mixed == 0) {
+            if (rows > 512) return half || light;
+            if (rows > 480) return half ? d.emdim <= 512 || former <= 11.0 : light;
+            if (rows > 256) return kept <= 0.45 * all || (light && (!half || d.emdim <= 512));
+            return rows == 256 && former <= 6.0;
+        }
+        if (kept > 16.5 * d.emdim) return false;
+        if (d.emdim <= 512 || rows > 512) return true;
+        if (rows > 256) return rows <= 480 || !half || former <= 14.5;
+        if (!half) return false;
+        if (strips == 7 || strips == 8) return former <= 5.0;
+        if (strips <= 3 || (strips >= 9 && strips <= 12)) return former <= 19.0;
+        return former <= 14.5 && !(fused && strips > 12);
+    };
     bool on;
-    if (d.mixed == 0) {
-        const bool light = kept <= 11.0 * d.emdim, half = kept <= 0.5 * all;
-        if (rows > 512) on = half || light;
-        else if (rows > 480) on = half ? d.emdim <= 512 || best <= 11.0 : light;
-        else if (rows > 256) on = kept <= 0.45 * all || (light && (!half || d.emdim <= 512));
-        else on = rows == 256 && best <= 6.0;
+    if (m.layers.size() < 6) on = short_on();
+    else if (d.mixed == 0) {
+        if (strips > 16) on = half || kept <= 11.0 * d.emdim;
+        else if (strips > 6) on = best <= (strips == 16 ? 12.5 : strips > 12 ? 20.5 : strips > 8 ? 23.0 : strips == 8 ? 11.0 : 14.6);
+        else on = half || best <= 15.0;
     } else if (kept > 16.5 * d.emdim) on = false;
-    else if (d.emdim <= 512 || rows > 512) on = true;
-    else if (rows > 256) on = rows <= 480 || kept > 0.5 * all || best <= 14.5;
-    else if (kept > 0.5 * all) on = false;
-    else if (strips == 7 || strips == 8) on = best <= 5.0;
-    else if (strips <= 3 || (strips >= 9 && strips <= 12)) on = best <= 19.0;
-    else on = best <= 14.5 && !(fused && strips > 12);
+    else if (strips > 16) on = true;
+    else if (strips > 8) on = best <= (strips <= 12 ? 32.0 : half ? 18.0 : 21.0);
+    else if (strips > 6) on = best <= (half ? 13.5 : 20.5);
+    else on = half || best <= 20.5;
     p.mt = on ? 1 : 0;
     return p;
 }
@@ -419,6 +432,12 @@ void build_local(et_model_s &m, bool fused) {
         for (auto &b : m.local_x) b = std::make_unique<et::DeviceBuffer<float>>(elems);
     if (plan.parts > 1)
         for (int i = 0; i < (d.mixed ? 1 : n); i++) m.local_shares.push_back(std::make_unique<et::DeviceBuffer<float>>(elems * plan.parts));
+    int joins = 0;
+    if (plan.parts > 1) etChk(et_encoder_layer_joins(packs[0].get(), &joins));
+    for (size_t i = 0; joins && i < m.local_shares.size(); i++) {
+        const std::vector<int> zero((size_t)(m.rows() + 15) / 16, 0);
+        m.local_join.push_back(std::make_unique<et::DeviceBuffer<int>>(zero.data(), zero.size()));
+    }
     m.local = std::move(packs);
 }
 
@@ -466,6 +485,18 @@ half *local_input(et_model_s &m, const et::LayerBuffers &b, half *in, stream_t s
 }
 half *local_result(const et::LayerBuffers &b, half *out) { return local_aligned(out) ? out : b.ffn; }
 
+// The token-local launches of layer i; `k`: the shares it runs with.
+void run_local(et_model_s &m, int i, int k, const half *z, const float *x32, const half *x16, float *x32_out, half *out16, half *qkv, stream_t stream) {
+    const ILayer &l = *m.layers[(size_t)i];
+    if (m.local_join.empty())
+        etChk(et_encoder_layer_f32(m.local[(size_t)i].get(), et::f16(z), x32, et::f16(x16), x32_out, et::f16(out16), et::f16(qkv), m.shares(k),
+                                   m.desc.act, l.epsilon(0), l.epsilon(1), stream));
+    else
+        etChk(et_encoder_layer_joined_f32(m.local[(size_t)i].get(), et::f16(z), x32, et::f16(x16), x32_out, et::f16(out16), et::f16(qkv), m.shares(k),
+                                          reinterpret_cast<uint32_t *>(m.local_join[(size_t)k]->get()), 4000, m.desc.act, l.epsilon(0),
+                                          l.epsilon(1), stream));
+}
+
 // One layer from binary16 to binary16, as et_model_forward under mixed = 0 chains it (`chained`: behind the layer before it)
 // and et_model_forward_layer issues it.  The token-local launches take the layer's input and leave its result in binary16,
 // and the next layer's QKV made from the result as they round it; a layer that runs alone makes its QKV from its input with
@@ -481,8 +512,7 @@ void run_layer_f16(et_model_s &m, int i, half *out, half *in, bool chained, stre
     l.chain_attention(b, stream);
     const bool last = i + 1 == (int)m.layers.size();
     half *qkv = last ? nullptr : chained ? m.stack_buffers(i + 1).qkv : b.qkv;
-    etChk(et_encoder_layer_f32(m.local[(size_t)i].get(), et::f16(b.z), nullptr, et::f16(x), nullptr, et::f16(to), et::f16(qkv),
-                               m.shares(chained ? 0 : i), m.desc.act, l.epsilon(0), l.epsilon(1), stream));
+    run_local(m, i, chained ? 0 : i, b.z, nullptr, x, nullptr, to, qkv, stream);
     if (to != out) copy_rows(m, out, to, stream);
 }
 
@@ -496,10 +526,8 @@ void run_layers_local(et_model_s &m, half *out, half *in, stream_t stream) {
         const et::LayerBuffers b = m.stack_buffers(i);
         const bool last = i == n - 1;
         l.chain_attention(b, stream);
-        etChk(et_encoder_layer_f32(m.local[(size_t)i].get(), et::f16(b.z), i ? m.local_x[(i - 1) & 1]->get() : nullptr,
-                                   i ? nullptr : et::f16(x), last ? nullptr : m.local_x[i & 1]->get(), last ? et::f16(to) : nullptr,
-                                   last ? nullptr : et::f16(m.stack_buffers(i + 1).qkv),
-                                   m.shares(0), m.desc.act, l.epsilon(0), l.epsilon(1), stream));
+        run_local(m, i, 0, b.z, i ? m.local_x[(i - 1) & 1]->get() : nullptr, i ? nullptr : x, last ? nullptr : m.local_x[i & 1]->get(),
+                  last ? to : nullptr, last ? nullptr : m.stack_buffers(i + 1).qkv, stream);
     }
     if (to != out) copy_rows(m, out, to, stream);
 }
