@@ -242,8 +242,9 @@ def time_dominant_kernel(et, layers, T, folded, rounds_per_graph=6, replays=8):
 
 def time_token_local(et, layers, T, rounds_per_graph=6, replays=8):
     """(seconds per layer, kernel names, description, flops, algorithmic bytes) of what the default stack runs between
-    two attention kernels at this workload's shape: et_encoder_layer_f32, divided as the engine divides 1024 token rows
-    (strips of 16 rows, four workgroups to a strip, hence two launches), timed as time_dominant_kernel does."""
+    two attention kernels at this workload's shape: a token-local launch divided as the engine divides 1024 token rows (strips of
+    16 rows, four workgroups to a strip, which meet inside one launch where the device lets them, else two launches), timed
+    as time_dominant_kernel does."""
     import ctypes as C
     lib = et.lib()
 
@@ -276,10 +277,16 @@ def time_token_local(et, layers, T, rounds_per_graph=6, replays=8):
     qkvs = [D.empty((T, 3 * H), np.float16) for _ in layers]
     outs = [D.empty((T, H), np.float32) for _ in layers]
     partial = D.empty((PARTS, T, H), np.float32)
+    words = D.from_numpy(np.zeros(T // 16, np.int32))
+    joins = C.c_int()
+    et.check(lib.et_encoder_layer_joins(packs[0], C.byref(joins)))
 
     def local(i):
-        et.check(lib.et_encoder_layer_f32(packs[i], zs[i].ptr, xs[i].ptr, None, outs[i].ptr, None, qkvs[i].ptr, partial.ptr,
-                                          et.ACT_GELU, 1e-5, 1e-5, stream))
+        buffers = (packs[i], zs[i].ptr, xs[i].ptr, None, outs[i].ptr, None, qkvs[i].ptr, partial.ptr)
+        if joins.value:
+            et.check(lib.et_encoder_layer_joined_f32(*buffers, words.ptr, 4000, et.ACT_GELU, 1e-5, 1e-5, stream))
+        else:
+            et.check(lib.et_encoder_layer_f32(*buffers, et.ACT_GELU, 1e-5, 1e-5, stream))
 
     for i in range(n):  # eager once: one-time kernel setup
         local(i)
@@ -303,8 +310,10 @@ def time_token_local(et, layers, T, rounds_per_graph=6, replays=8):
     tiles = sum(len(w.col_idx) for l in layers for w in (l.qkv, l.o, l.l1, l.l2)) / n
     # Z and QKV' binary16, the residual stream binary32 in and out, tiles with their indices, biases and norms
     nbytes = 2.0 * T * H + 8.0 * T * H + 6.0 * T * H + 516.0 * tiles + 2.0 * (9 * H + FF)
-    name = "void et::encoder_layer_kernel<1, 3, 1>(et::LayerArgs) + void et::encoder_layer_kernel<1, 3, 2>(et::LayerArgs)"
-    what = f"output projection, LayerNorms, FFN + GELU and next QKV projection of a layer @80%, T={T}, two launches"
+    name = "void et::encoder_layer_joined_kernel<3>(et::LayerArgs)" if joins.value else \
+        "void et::encoder_layer_kernel<1, 3, 1>(et::LayerArgs) + void et::encoder_layer_kernel<1, 3, 2>(et::LayerArgs)"
+    what = f"output projection, LayerNorms, FFN + GELU and next QKV projection of a layer @80%, T={T}, " + \
+        ("one launch" if joins.value else "two launches")
     return t.ms * 1e-3 / (rounds_per_graph * n * replays), name, what, 2.0 * 256 * tiles * T, nbytes
 
 

@@ -13,6 +13,9 @@
 
 #include "common.hip.h"
 
+#define ET_GLOBAL_PTR(p) ((const __attribute__((address_space(1))) void *)(p))
+#define ET_LDS_PTR(p) ((__attribute__((address_space(3))) void *)(p))
+
 namespace et {
 
 struct Bsr32Args {
@@ -20,6 +23,7 @@ struct Bsr32Args {
     const float *tiles, *bias, *X;
     float *Y;
     int T, in, out, act;
+    int strip_dies;  // 1, 2, 4 or 8: see strip_of
 };
 
 __device__ __forceinline__ f4 mfma_cell_f32(const float4 w, const float4 x, f4 acc) {
@@ -30,14 +34,17 @@ __device__ __forceinline__ f4 mfma_cell_f32(const float4 w, const float4 x, f4 a
     return acc;
 }
 
+__device__ __forceinline__ f4 bias_cell_f32(const float *bias, int f0) {
+    return bias ? f4{bias[f0], bias[f0 + 1], bias[f0 + 2], bias[f0 + 3]} : f4{0.f, 0.f, 0.f, 0.f};
+}
+
 // lane (r, q) holds features f0 + 4q .. 4q+3 of token `tok`: bias, activation, one 16-byte store
-__device__ __forceinline__ void store_cell_f32(float *Y, const float *bias, f4 acc, int tok, int T, int out,
-                                               int f0, int act) {
+__device__ __forceinline__ void store_cell_f32(float *Y, f4 bias, f4 acc, int tok, int T, int out, int f0, int act) {
     if (tok >= T) return;
     float4 o;
     float *po = reinterpret_cast<float *>(&o);
 #pragma unroll
-    for (int e = 0; e < 4; e++) po[e] = apply_act(acc[e] + (bias ? bias[f0 + e] : 0.0f), act);
+    for (int e = 0; e < 4; e++) po[e] = apply_act(acc[e] + bias[e], act);
     *reinterpret_cast<float4 *>(Y + (size_t)tok * out + f0) = o;
 }
 
@@ -72,7 +79,7 @@ template <int MT> __global__ __launch_bounds__(256) void bsr16_linear_wide_f32_k
         for (int m = 0; m < MT; m++) acc[m] = mfma_cell_f32(w, *reinterpret_cast<const float4 *>(xrow[m] + c * 16), acc[m]);
     }
 #pragma unroll
-    for (int m = 0; m < MT; m++) store_cell_f32(a.Y, a.bias, acc[m], tok0 + m * 16 + r16, a.T, a.out, br * 16 + 4 * q, a.act);
+    for (int m = 0; m < MT; m++) store_cell_f32(a.Y, bias_cell_f32(a.bias, br * 16 + 4 * q), acc[m], tok0 + m * 16 + r16, a.T, a.out, br * 16 + 4 * q, a.act);
 }
 
 // The short form, for few pairs.  Against the wide one, us, at 80 %: 256 tokens 768 -> 2304 8.0 / 10.4, 768 -> 3072 8.4 / 11.0,
@@ -80,29 +87,46 @@ template <int MT> __global__ __launch_bounds__(256) void bsr16_linear_wide_f32_k
 //
 // The waves of a workgroup share one (block-row, 16 tokens), each every WAVES-th tile; the sums meet in LDS and are added
 // in the order of the waves.  A lane reads the column index of one of its wave's tiles, 64 at a time, so no operand waits
-// for an index from memory, and kAhead tiles are requested ahead of the products.
+// for an index from memory, and kAhead tiles are requested ahead of the products.  The requests are straight-line and go
+// through buffer resources that end with the tiles: one past the last moves nothing (asking for the last tile again, as
+// before, cost 16 tokens of a 6-layer stack of 768 at 80 % 13 us of 175).  8 ahead are slower, 300 us against 292 for 256
+// tokens of that stack: it is no longer the latency of a load that bounds a pair.
+//
+// The workgroups of one die (blockIdx.x % 8) keep to a part of the strips and a part of the columns of the grid, so that what an L2
+// has to fetch is a part of X and a part of the weights: strip_dies parts of the strips, 8 / strip_dies of the columns.
+__device__ __forceinline__ int strip_of(int strip_dies) {
+    return (int)(blockIdx.x & (strip_dies - 1)) + strip_dies * (int)(blockIdx.y + blockIdx.z * gridDim.y);
+}
+__device__ __forceinline__ int column_of(int strip_dies) { return (int)((blockIdx.x & 7) / strip_dies) + 8 / strip_dies * (int)(blockIdx.x >> 3); }
+
 constexpr int kAhead = 4;
+constexpr int kRawBuffer = 0x00020000;   // word 3 of a resource: raw, 32-bit data
+constexpr int kPastEnd = 0x7fffff00;     // an offset past the end of any resource here
+constexpr int kSplitMaxIn = 1 << 24;     // 16 rows of X lie within the offsets of a resource, and below kPastEnd
 template <int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void bsr16_linear_split_f32_kernel(const Bsr32Args a) {
     __shared__ f4 part[WAVES][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, q = lane >> 4;
-    const int strip = blockIdx.y + blockIdx.z * gridDim.y;
-    if (strip * 16 >= a.T) return;  // padding of the grid (whole workgroup)
-    const int br = blockIdx.x, tok = strip * 16 + r16;
-    const float *xp = a.X + (size_t)min(tok, a.T - 1) * a.in + 4 * q;  // rows past the end: the last one, not stored
-    const float *wp = a.tiles + r16 * 16 + 4 * q;
+    const int strip = strip_of(a.strip_dies), br = column_of(a.strip_dies);
+    if (strip * 16 >= a.T || br >= (a.out >> 4)) return;  // padding of the grid (whole workgroup)
+    const int tok = strip * 16 + r16;
+    const f4 bias = bias_cell_f32(a.bias, br * 16 + 4 * q);
+    const auto xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.X) + (size_t)strip * 16 * a.in, 0, 16 * a.in * 4, kRawBuffer);
+    const int xo = (min(r16, a.T - 1 - strip * 16) * a.in + 4 * q) * 4;  // rows past the end: the last one, not stored
+    const int wo = (r16 * 16 + 4 * q) * 4;
     f4 acc = f4{0.f, 0.f, 0.f, 0.f};
     const int ts = a.row_ptr[br] + wave, te = a.row_ptr[br + 1];
     const int n = ts < te ? (te - ts + WAVES - 1) / WAVES : 0;  // tiles of this wave
     for (int base = 0; base < n; base += 64) {
         const int here = min(n - base, 64), t0 = ts + base * WAVES;
         const int cols = a.col_idx[t0 + min(lane, here - 1) * WAVES];
+        const auto wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.tiles) + (size_t)t0 * 256, 0, ((here - 1) * WAVES + 1) * 1024, kRawBuffer);
         float4 w[kAhead], x[kAhead];
-        auto ask = [&](int slot, int i) {  // (past the last: the last again, not multiplied)
-            i = min(i, here - 1);
-            w[slot] = *reinterpret_cast<const float4 *>(wp + (size_t)(t0 + i * WAVES) * 256);
-            x[slot] = *reinterpret_cast<const float4 *>(xp + __builtin_amdgcn_readlane(cols, i) * 16);
+        auto ask = [&](int slot, int i) {
+            const int xat = i < here ? __builtin_amdgcn_readlane(cols, i & 63) * 64 : kPastEnd;
+            w[slot] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(wr, wo, i * WAVES * 1024, 0));
+            x[slot] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xr, xo, xat, 0));
         };
 #pragma unroll
         for (int s = 0; s < kAhead; s++) ask(s, s);
@@ -121,13 +145,14 @@ __global__ __launch_bounds__(WAVES * 64) void bsr16_linear_split_f32_kernel(cons
 #pragma unroll
         for (int v = 1; v < WAVES; v++) acc += part[v][lane];
     }
-    store_cell_f32(a.Y, a.bias, acc, tok, a.T, a.out, br * 16 + 4 * q, a.act);
+    store_cell_f32(a.Y, bias, acc, tok, a.T, a.out, br * 16 + 4 * q, a.act);
 }
 
 // Eight waves, eight neighbouring block-rows, 16 tokens, whose rows of X lie in LDS (kStripPad floats between two rows:
 // the 16 cells of a fragment read lie in different banks).  Read from memory, the fragment of a tile is 16 rows x 64 bytes,
-// and 16 neighbouring lanes touch 16 lines: with many tiles that is what the kernels above wait for.  The first
-// weights travel while the strip is staged.  Against the wide form: 4096 tokens 768 -> 3072 at 50 / 80 / 90 / 95 % 116 / 188, 70 / 96,
+// and 16 neighbouring lanes touch 16 lines: with many tiles that is what the kernels above wait for.  The rows go straight
+// to LDS, all of them requested before anything is waited for, with the first weights behind them.  Against the wide
+// form: 4096 tokens 768 -> 3072 at 50 / 80 / 90 / 95 % 116 / 188, 70 / 96,
 // 56 / 56, 51 / 37 (staging a strip for a few tiles; the number of tiles is not known on the host).
 constexpr int kStripPad = 4, kStripWaves = 8;
 __global__ __launch_bounds__(kStripWaves * 64) void bsr16_linear_strip_f32_kernel(const Bsr32Args a) {
@@ -135,31 +160,37 @@ __global__ __launch_bounds__(kStripWaves * 64) void bsr16_linear_strip_f32_kerne
     float *xs = reinterpret_cast<float *>(strip_smem);  // [16][in + kStripPad]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, q = lane >> 4;
-    const int strip = blockIdx.y + blockIdx.z * gridDim.y;
-    if (strip * 16 >= a.T) return;  // padding of the grid (whole workgroup)
+    const int strip = strip_of(a.strip_dies), br = column_of(a.strip_dies) * kStripWaves + wave;
+    if (strip * 16 >= a.T || br - wave >= (a.out >> 4)) return;  // padding of the grid (whole workgroup)
     const int ld = a.in + kStripPad, tok0 = strip * 16, quads = a.in >> 2;
-    for (int row = wave; row < 16; row += kStripWaves) {  // past the end: the last row, not stored
-        const float *src = a.X + (size_t)min(tok0 + row, a.T - 1) * a.in;
-        for (int i = lane; i < quads; i += 64)
-            *reinterpret_cast<float4 *>(xs + row * ld + i * 4) = *reinterpret_cast<const float4 *>(src + i * 4);
-    }
-    const int br = blockIdx.x * kStripWaves + wave;
     const bool mine = br < (a.out >> 4);  // uniform
     const int ts = mine ? a.row_ptr[br] : 0, n = mine ? a.row_ptr[br + 1] - ts : 0;
+    for (int row = wave; row < 16; row += kStripWaves) {  // past the end: the last row, not stored
+        const float *src = a.X + (size_t)min(tok0 + row, a.T - 1) * a.in;
+        for (int i = 0; i < quads; i += 64)
+            if (i + lane < quads)
+                __builtin_amdgcn_global_load_lds(ET_GLOBAL_PTR(src + (i + lane) * 4), ET_LDS_PTR(xs + row * ld + i * 4), 16, 0, 0);
+    }
+    const f4 bias = bias_cell_f32(mine ? a.bias : nullptr, br * 16 + 4 * q);
     const float *xp = xs + r16 * ld + 4 * q;
-    const float *wp = a.tiles + r16 * 16 + 4 * q;
+    const int wo = (r16 * 16 + 4 * q) * 4;
     f4 acc = f4{0.f, 0.f, 0.f, 0.f};
-    if (n == 0) __syncthreads();
+    auto staged = [] {                        // the strip is complete (every wave passes here once)
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's rows have landed
+        __syncthreads();
+    };
+    if (n == 0) staged();
     for (int base = 0; base < n; base += 64) {
         const int here = min(n - base, 64), t0 = ts + base;
         const int cols = a.col_idx[t0 + min(lane, here - 1)];
+        const auto wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.tiles) + (size_t)t0 * 256, 0, here * 1024, kRawBuffer);
         float4 w[kAhead];
-        auto ask = [&](int slot, int i) {  // (past the last: the last again, not multiplied)
-            w[slot] = *reinterpret_cast<const float4 *>(wp + (size_t)(t0 + min(i, here - 1)) * 256);
+        auto ask = [&](int slot, int i) {
+            w[slot] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(wr, wo, i * 1024, 0));
         };
 #pragma unroll
         for (int s = 0; s < kAhead; s++) ask(s, s);
-        if (base == 0) __syncthreads();  // the strip is complete (every wave passes one barrier, here or above)
+        if (base == 0) staged();
         for (int i = 0; i < here; i += kAhead) {
 #pragma unroll
             for (int s = 0; s < kAhead; s++) {
@@ -169,7 +200,7 @@ __global__ __launch_bounds__(kStripWaves * 64) void bsr16_linear_strip_f32_kerne
             }
         }
     }
-    if (mine) store_cell_f32(a.Y, a.bias, acc, tok0 + r16, a.T, a.out, br * 16 + 4 * q, a.act);
+    if (mine) store_cell_f32(a.Y, bias, acc, tok0 + r16, a.T, a.out, br * 16 + 4 * q, a.act);
 }
 
 // ---- 1x16 vectors ---------------------------------------------------------------
@@ -225,7 +256,7 @@ __global__ __launch_bounds__(256) void vec1x16_linear_f32_kernel(const V16F32Arg
     }
 #pragma unroll
     for (int m = 0; m < MT; m++)
-        store_cell_f32(a.Y, a.bias, acc[m], tok0 + m * 16 + r16, a.T, a.out, rset * 16 + 4 * q, a.act);
+        store_cell_f32(a.Y, bias_cell_f32(a.bias, rset * 16 + 4 * q), acc[m], tok0 + m * 16 + r16, a.T, a.out, rset * 16 + 4 * q, a.act);
 }
 
 // ---- CSR ------------------------------------------------------------------------
@@ -296,10 +327,18 @@ int et_linear_bsr16_f32(const int32_t *row_ptr, const int32_t *col_idx, const fl
     ET_REQUIRE(aligned16(tiles) && aligned16(X) && aligned16(Y), ET_ERR_UNSUPPORTED,
                "et_linear_bsr16_f32: tiles, X and Y must be 16-byte aligned");
     if (T == 0) return ET_OK;
-    const Bsr32Args a{row_ptr, col_idx, tiles, bias, X, Y, T, in, out, act};
+    Bsr32Args a{row_ptr, col_idx, tiles, bias, X, Y, T, in, out, act, 1};
     hipStream_t st = as_stream(stream);
     const int strips = (T + 15) / 16;
-    const int gy = std::min(strips, 32768);
+    // The parts of the strips and of the columns the dies keep to: the split that leaves one die the fewest bytes, taking
+    // a fifth of the tiles as kept (their number is not known here).
+    auto place = [&](int columns) {
+        auto bytes = [&](int d) { return (double)T / d + 0.2 * out * d / 8; };  // in units of a row of X
+        for (int d = 2; d <= 8 && d <= strips; d *= 2)
+            if (bytes(d) < bytes(a.strip_dies)) a.strip_dies = d;
+        const int column_dies = 8 / a.strip_dies, rows = (strips + a.strip_dies - 1) / a.strip_dies, gy = std::min(rows, 32768);
+        return dim3(8 * ((columns + column_dies - 1) / column_dies), gy, (rows + gy - 1) / gy);
+    };
     const long long pairs = (long long)(out / 16) * strips;
     const size_t lds = (size_t)16 * (in + kStripPad) * sizeof(float);
     // The strip form where two workgroups fit a compute unit and there are six pairs or more for each: 80 %, us, strip
@@ -308,7 +347,7 @@ int et_linear_bsr16_f32(const int32_t *row_ptr, const int32_t *col_idx, const fl
         if (lds > 64 * 1024)
             ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(bsr16_linear_strip_f32_kernel),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        const dim3 grid((out / 16 + kStripWaves - 1) / kStripWaves, gy, (strips + gy - 1) / gy);
+        const dim3 grid = place((out / 16 + kStripWaves - 1) / kStripWaves);
         bsr16_linear_strip_f32_kernel<<<grid, kStripWaves * 64, lds, st>>>(a);
         return check_launch("bsr16_linear_strip_f32_kernel");
     }
@@ -316,7 +355,7 @@ int et_linear_bsr16_f32(const int32_t *row_ptr, const int32_t *col_idx, const fl
     // 1024 x 4096 -> 1024 40 / 51, 512 x 2048 -> 2048 22 / 31; 768 1024 x 1536 -> 1536 23 / 31, 4096 x 3072 -> 768 99 / 106; 384 2048 x 3072 ->
     // 768 69 / 54, 512 x 1536 -> 1536 17.1 / 17.2.  (90 % and many rows of a narrow result 1.04 the other way.)
     const int mt = token_blocks(T), wide_strips = (T + 16 * mt - 1) / (16 * mt), wide_x = (out / 16 + 3) / 4;
-    if (mt > 1 && lds > 80 * 1024 && (long long)wide_x * wide_strips >= 512) {
+    if (in > kSplitMaxIn || (mt > 1 && lds > 80 * 1024 && (long long)wide_x * wide_strips >= 512)) {
         const int wide_y = std::min(wide_strips, 32768);
         const dim3 grid(wide_x, wide_y, (wide_strips + wide_y - 1) / wide_y);
         if (mt == 4) bsr16_linear_wide_f32_kernel<4><<<grid, 256, 0, st>>>(a);
@@ -325,7 +364,7 @@ int et_linear_bsr16_f32(const int32_t *row_ptr, const int32_t *col_idx, const fl
     }
     // Two waves a pair below two pairs a compute unit: 192 pairs of 38 tiles 5.2 us against 7.3, 576 pairs of 10 tiles 4.9
     // against 4.7; four waves are no faster.
-    const dim3 grid(out / 16, gy, (strips + gy - 1) / gy);
+    const dim3 grid = place(out / 16);
     if (pairs < 512) bsr16_linear_split_f32_kernel<2><<<grid, 128, 0, st>>>(a);
     else bsr16_linear_split_f32_kernel<1><<<grid, 64, 0, st>>>(a);
     return check_launch("bsr16_linear_split_f32_kernel");

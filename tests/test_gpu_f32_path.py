@@ -218,6 +218,30 @@ def test_linear_bsr16_f32_division_of_the_work(et, T, inp, out, sp, act):
     test_linear_bsr16_f32(et, T, inp, out, sp, act)
 
 
+# Tile counts of the block-rows around the tiles asked for ahead (4) and the indices read at once (64) in the three forms that ask
+# ahead: two waves a pair, one, rows of X in LDS.  What lies behind the tiles and behind the rows of X is not a number, and the
+# strips and columns are dealt to 1, 2, 4 and 8 groups of dies with a remainder.  Bound: a value of k products of
+# size 1 and 0.05, k at most 16 x 130, rounds to 0.05 sqrt(k) 2^-24 sqrt(k) at worst a step, 6e-6 over all of them.
+@pytest.mark.parametrize("T,inp", [(15, 2080), (33, 2080), (250, 2080), (200, 1264), (530, 1264)])
+def test_linear_bsr16_f32_ends_of_block_rows(et, T, inp):
+    from oracle import formats as F
+    counts = [0, 1, 2, 3, 4, 5, 7, 8, 9, 12, 16, 17, 63, 64, 65, 66, 68, 69, 72, 73, 79, 0, 78, 70] * (1 if T < 256 else 2) + [1, 79, 4]
+    if inp > 1264: counts[5:9] = [127, 128, 129, 130]
+    out, nc = 16 * len(counts), inp // 16
+    rng = np.random.default_rng(7)
+    row_ptr = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    col_idx = np.concatenate([rng.permutation(nc)[:n] for n in counts]).astype(np.int32)  # any order inside a block-row
+    tiles, x = randf((len(col_idx) + 8, 256), 41, 0.05), randf((T + 16, inp), 42)
+    tiles[len(col_idx):], x[T:] = np.nan, np.nan
+    Wd, b = F.bsr16_to_dense(row_ptr, col_idx, tiles[:len(col_idx)], inp), randf((out,), 43, 0.1)
+    d_y = up(et, np.full((T + 16, out), 7, np.float32))
+    et.check(et.lib().et_linear_bsr16_f32(up(et, row_ptr).ptr, up(et, col_idx).ptr, up(et, tiles).ptr, up(et, b).ptr, up(et, x).ptr, d_y.ptr,
+                                          T, inp, out, 0, None))
+    y = d_y.numpy()
+    assert Hn.max_abs(y[:T], _want64(x[:T], Wd, b, 0)) <= 5e-5
+    assert (y[T:] == 7).all()
+
+
 def test_linear_bsr16_f32_closed_form_and_bad_args(et):
     """All-ones tiles and inputs: every output is 16 x (tiles of its block-row) + bias, exactly."""
     from oracle import formats as F
