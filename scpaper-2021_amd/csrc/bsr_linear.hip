@@ -28,8 +28,12 @@
 //
 // Tile order inside a block-row is free (the sum commutes), as in the
 // reference kernel (Linear/SPMM_tile.cu:277-283).
+#include <algorithm>
+
 #include "common.hip.h"
 #include "../../include/et_tuning.h"
+
+#define ET_LDS_PTR(p) ((__attribute__((address_space(3))) void *)(p))
 
 namespace et {
 
@@ -110,6 +114,9 @@ template <int ACT> __device__ __forceinline__ float act_fixed(float x) {
 __device__ __forceinline__ int lane_read(int v, int lane) {
     return __builtin_amdgcn_readlane(v, lane);
 }
+
+// column tiles of the first of the two halves a wide strip is staged in
+__host__ __device__ __forceinline__ int half_tiles(int in) { return (in / 16 + 1) / 2; }
 
 // ACT is a template parameter: the epilogue carries no run-time branch and each
 // fused activation is a separately named kernel in a profile.
@@ -692,6 +699,233 @@ __global__ __launch_bounds__(((MT == 1 && (FX & kFxRes32) && !(FX & kFxRes16)) |
     }
 }
 
+// ---- strips of 32 rows whose inputs do not fit the LDS at once
+// The plain kernel on strips of 16 rows (inputs too wide for 32) spends its time between the operands and the products: a wave
+// finds the columns of a slot by lane reads, waits for two LDS reads and multiplies, 313 cycles a slot at three
+// waves a SIMD (4096 x 3072 -> 768, 80 %), and every strip fetches all of its group's tiles, 1.04 MB a workgroup.  Here a strip has
+// 32 rows, staged one half of its columns after the other, so that a tile is fetched for twice the rows (0.67 MB), and a
+// wave keeps the sums of its block-rows (at most RW) through both halves.  A block-row's tiles may come in any order:
+// its wave lists them by halves in LDS, as a lane uses them, four slots to an item, so an item is one read of its list
+// and then straight-line requests, 8 LDS reads and 8 products.  (A row with more tiles in a half than columns, some column
+// twice, is not listed: it takes its operands from memory at the end.)
+// 16-row strips against this, us: 4096 x 3072 -> 768 at 80 % 21.1 / 14.9, 70 % of 3072 rows 24.8 / 16.6, 16384 82 / 55,
+// 16384 x 4096 -> 1024 148 / 88, 16384 x 2048 -> 2048 152 / 97; two items asked for ahead 14.9, three 15.5, four 17; 16 waves 15.6; the
+// second half asked for into registers during the first 15.3; lists without the straight-line items 23.3.
+constexpr int kHalfWaves = 12;
+constexpr int kHalfAhead = 2;           // items asked for ahead
+constexpr int kRawBuffer = 0x00020000;  // word 3 of a resource: raw, 32-bit data
+constexpr int kNoTile = 0xffff;         // past the tiles of any listed row
+template <int ACT, int RW>
+__global__ __launch_bounds__(kHalfWaves * 64) void bsr16_linear_halves_kernel(const BsrArgs a) {
+    constexpr int MT = 2, kNB = kHalfAhead;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    _Float16 *xs = reinterpret_cast<_Float16 *>(smem_raw);  // [32][half * 16 + kLdsPad]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, g = lane >> 4;
+    const int sel = g >> 1, koff = (g & 1) << 3;  // as in the kernel above
+    const int nbr = a.out >> 4;
+    const int ngroups = (nbr + a.rows_per_wg - 1) / a.rows_per_wg;
+    const int xcd = blockIdx.x % kXcds, k_in_xcd = blockIdx.x / kXcds;
+    const int strip = xcd + kXcds * (k_in_xcd / ngroups), group = k_in_xcd % ngroups;
+    const int tok0 = strip * (MT * 16);
+    if (tok0 >= a.T) return;  // padding of the last round of strips (whole workgroup)
+    const int rb_begin = group * a.rows_per_wg, rb_end = min(rb_begin + a.rows_per_wg, nbr);
+    const int nrw = max(0, (rb_end - rb_begin - wave + kHalfWaves - 1) / kHalfWaves);  // at most RW
+    const int half = half_tiles(a.in), lds_ld = half * 16 + kLdsPad;
+    const h8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+
+    int rp_lo = 0, rp_hi = 0;  // lane i: row i of this wave
+    if (lane < nrw) {
+        const int rb = rb_begin + wave + kHalfWaves * lane;
+        rp_lo = a.row_ptr[rb];
+        rp_hi = a.row_ptr[rb + 1];
+    }
+    auto stage = [&](int h) {  // rows past the end: the last one, not stored
+        const int c0 = h * half * 16, nvec = ((h ? a.in - c0 : half * 16)) >> 3;
+        for (int row = wave; row < MT * 16; row += kHalfWaves) {
+            const _Float16 *src = a.X + (size_t)min(tok0 + row, a.T - 1) * a.in + c0;
+            for (int i = 0; i < nvec; i += 64)
+                if (i + lane < nvec) {
+                    // 16 bytes a lane, behind the compiler's back: it would wait for them before any other access to
+                    // the LDS.  (The s_nop also covers a base that a vector instruction has just written.)
+                    const unsigned to = (unsigned)(uintptr_t)ET_LDS_PTR(xs + row * lds_ld + i * 8);
+                    asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane * 16), "s"(src + i * 8), "s"(to)
+                                 : "memory", "m0");
+                }
+        }
+    };
+    stage(0);
+    h4 bias[RW];
+#pragma unroll
+    for (int r = 0; r < RW; r++) {
+        bias[r] = h4{0, 0, 0, 0};
+        if (a.bias && r < nrw) bias[r] = *reinterpret_cast<const h4 *>(a.bias + (rb_begin + wave + kHalfWaves * r) * 16 + g * 4);
+    }
+
+    // ---- the lists: items of four slots, a slot's first tiles and second tiles apart, so that a lane reads the four tiles it
+    // multiplies at once; an entry is the tile of the row << 16 | its column in the half.  ends[h][r]: items up to
+    // row r's last in half h.
+    const int most = a.in >> 4, per_row = (half + 7) >> 3;  // tiles of a row, items of a row and half, at most
+    int *list = reinterpret_cast<int *>(xs + MT * 16 * lds_ld) + wave * (2 * RW * per_row * 8);
+    auto entry = [&](int h, int item, int k) -> int & { return list[(h * RW * per_row + item) * 8 + (k & 7 & 1) * 4 + ((k & 7) >> 1)]; };
+    int ends[2][RW];
+    unsigned unlisted = 0;
+    {
+        int first[RW];  // the first 64 columns of every row, in flight together
+#pragma unroll
+        for (int r = 0; r < RW; r++) {
+            const int i = lane_read(rp_lo, r) + lane;
+            first[r] = r < nrw && i < lane_read(rp_hi, r) ? a.col_idx[i] : 0;
+        }
+        int at[2] = {0, 0};
+#pragma unroll
+        for (int r = 0; r < RW; r++) {
+            const int t0 = lane_read(rp_lo, r), n = r < nrw ? lane_read(rp_hi, r) - t0 : 0;
+            int have[2] = {0, 0}, some[2] = {0, 0};
+            if (n > most) unlisted |= 1u << r;
+            else
+                for (int base = 0; base < n; base += 64) {
+                    const bool real = base + lane < n;
+                    const int c = base == 0 ? first[r] : real ? a.col_idx[t0 + base + lane] : 0;
+                    const unsigned long long in_half[2] = {__ballot(real && c < half), __ballot(real && c >= half)};
+                    const int h = c >= half;
+                    const unsigned long long mine = h ? in_half[1] : in_half[0];
+                    const int k = (h ? have[1] : have[0]) + __builtin_amdgcn_mbcnt_hi((unsigned)(mine >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mine, 0));
+                    if (real && k < half) entry(h, (h ? at[1] : at[0]) + (k >> 3), k) = (base + lane) << 16 | (c - h * half);
+#pragma unroll
+                    for (int k2 = 0; k2 < 2; k2++) {
+                        have[k2] += __popcll(in_half[k2]);
+                        if (in_half[k2]) some[k2] = lane_read(c, __builtin_ctzll(in_half[k2])) - k2 * half;
+                    }
+                }
+            if (have[0] > half || have[1] > half) {
+                unlisted |= 1u << r;
+                have[0] = have[1] = 0;
+            }
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int items = (have[h] + 7) >> 3;
+                if (have[h] & 7) {  // the last item is filled up with a tile past the row (zero) and a column the row has
+                    const int fill = kNoTile << 16 | some[h];
+                    if (lane < 8 && lane >= (have[h] & 7)) entry(h, at[h] + items - 1, lane) = fill;
+                }
+                at[h] += items;
+                ends[h][r] = __builtin_amdgcn_readfirstlane(at[h]);
+            }
+        }
+    }
+
+    f4 sum[RW][MT];
+#pragma unroll
+    for (int r = 0; r < RW; r++)
+#pragma unroll
+        for (int m = 0; m < MT; m++) sum[r][m] = f4{0.f, 0.f, 0.f, 0.f};
+    const _Float16 *xrow[MT];
+#pragma unroll
+    for (int m = 0; m < MT; m++) xrow[m] = xs + (m * 16 + r16) * lds_ld + koff;
+    const int wo = (r16 * 16 + koff) * 2;
+
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        if (h) {
+            __syncthreads();  // every wave has read the first half
+            stage(1);
+        }
+        const int total = ends[h][RW - 1];
+        h8 w[kNB][4];
+        int4 e[kNB];
+        auto row_of = [&](int item) {
+            int r = 0;
+#pragma unroll
+            for (int k = 0; k < RW - 1; k++) r += item >= ends[h][k];
+            return r;
+        };
+        // straight-line, so that the wait for an item counts the requests behind it; past the last item they move nothing
+        auto ask = [&](int buf, int item) __attribute__((always_inline)) {
+            const bool real = item < total;
+            const int row = row_of(min(item, total - 1));
+            const int t0 = lane_read(rp_lo, row), n = lane_read(rp_hi, row) - t0;
+            const auto wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16 *>(a.tiles) + (size_t)t0 * 256, 0, real ? n * 512 : 0, kRawBuffer);
+            e[buf] = *reinterpret_cast<const int4 *>(&list[(h * RW * per_row + (real ? item : 0)) * 8 + sel * 4]);
+            const int *ei = reinterpret_cast<const int *>(&e[buf]);
+#pragma unroll
+            for (int p = 0; p < 4; p++)
+                w[buf][p] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(wr, (int)((unsigned)ei[p] >> 16) * 512 + wo, 0, 0));
+        };
+#pragma unroll
+        for (int buf = 0; buf < kNB; buf++) ask(buf, buf);
+        // all but the requests above, so this wave's part of the strip has landed; they cannot move past the wait
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * kNB) : "memory");
+        __syncthreads();
+
+        f4 acc[MT];
+#pragma unroll
+        for (int m = 0; m < MT; m++) acc[m] = f4{0.f, 0.f, 0.f, 0.f};
+        auto multiply = [&](int buf, int item) __attribute__((always_inline)) {
+            const int *ei = reinterpret_cast<const int *>(&e[buf]);
+            h8 x[4][MT];
+#pragma unroll
+            for (int p = 0; p < 4; p++)
+#pragma unroll
+                for (int m = 0; m < MT; m++) x[p][m] = *reinterpret_cast<const h8 *>(xrow[m] + (ei[p] & 0xffff) * 16);
+#pragma unroll
+            for (int p = 0; p < 4; p++)
+#pragma unroll
+                for (int m = 0; m < MT; m++) acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[buf][p], x[p][m], acc[m], 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < RW; r++)
+                if (item + 1 == ends[h][r]) {  // the row's last item in this half (rows behind it without any: nothing is added)
+#pragma unroll
+                    for (int m = 0; m < MT; m++) {
+                        sum[r][m] += acc[m];
+                        acc[m] = f4{0.f, 0.f, 0.f, 0.f};
+                    }
+                }
+        };
+        int i0 = 0;
+        for (; i0 + kNB < total; i0 += kNB) {
+#pragma unroll
+            for (int buf = 0; buf < kNB; buf++) {
+                multiply(buf, i0 + buf);
+                ask(buf, i0 + buf + kNB);
+            }
+        }
+#pragma unroll
+        for (int buf = 0; buf < kNB; buf++)
+            if (i0 + buf < total) multiply(buf, i0 + buf);  // uniform
+    }
+    // rows that are not listed: both operands from memory, a slot at a time
+#pragma unroll
+    for (int r = 0; r < RW; r++) {
+        if (!((unlisted >> r) & 1)) continue;
+        const int t0 = lane_read(rp_lo, r), t1 = lane_read(rp_hi, r);
+        for (int t = t0; t < t1; t += 2) {
+            const int mine = min(t + sel, t1 - 1);
+            const h8 wv = t + sel < t1 ? *reinterpret_cast<const h8 *>(a.tiles + (size_t)mine * 256 + r16 * 16 + koff) : zero8;
+            const size_t at = (size_t)a.col_idx[mine] * 16 + koff;
+#pragma unroll
+            for (int m = 0; m < MT; m++)
+                sum[r][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                    wv, *reinterpret_cast<const h8 *>(a.X + (size_t)min(tok0 + m * 16 + r16, a.T - 1) * a.in + at), sum[r][m], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < RW; r++) {
+        if (r >= nrw) continue;
+        const int f0 = (rb_begin + wave + kHalfWaves * r) * 16 + g * 4;
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+            const int tok = tok0 + m * 16 + r16;
+            if (tok >= a.T) continue;
+            f4 v;
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = act_fixed<ACT>(sum[r][m][j] + (float)bias[r][j]);
+            if (a.Y32) *reinterpret_cast<f4 *>(a.Y32 + (size_t)tok * a.out + f0) = v;
+            else *reinterpret_cast<h4 *>(a.Y + (size_t)tok * a.out + f0) = h4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+        }
+    }
+}
+
 struct BsrPlan {
     int mt;        // 16-token blocks per workgroup strip
     bool stage;    // X strip staged in LDS
@@ -943,6 +1177,43 @@ static int dispatch_bsr_res(const BsrArgs &args, const BsrPlan &p, hipStream_t s
                      : launch_bsr_act<1, true, ET_ACT_NONE, 0, kFxRes>(args, p, stream);
 }
 
+// LDS of a workgroup of the halves form: half a strip of 32 rows, and a list of the tiles of each block-row of a wave.
+static size_t halves_lds_bytes(int in, int rows_per_wg) {
+    const int rw = rows_per_wg <= 2 * kHalfWaves ? 2 : 4;
+    return (size_t)32 * (half_tiles(in) * 16 + kLdsPad) * sizeof(_Float16) + (size_t)kHalfWaves * 2 * rw * ((half_tiles(in) + 7) / 8) * 8 * sizeof(int);
+}
+
+template <int ACT>
+static int launch_bsr_halves(const BsrArgs &args, int rows_per_wg, hipStream_t stream) {
+    auto kernel = rows_per_wg <= 2 * kHalfWaves ? bsr16_linear_halves_kernel<ACT, 2> : bsr16_linear_halves_kernel<ACT, 4>;
+    const size_t lds = halves_lds_bytes(args.in, rows_per_wg);
+    if (lds > 64 * 1024)
+        ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    const int nbr = args.out / 16, ngroups = (nbr + rows_per_wg - 1) / rows_per_wg;
+    const int strips = (args.T + 31) / 32;
+    kernel<<<(unsigned)((strips + kXcds - 1) / kXcds * kXcds * ngroups), kHalfWaves * 64, lds, stream>>>(args);
+    return check_launch("bsr16_linear_halves_kernel");
+}
+
+// Block-rows of a workgroup of the halves form, 0 where another form is the faster one.
+static int plan_halves(int T, int in, int out) {
+    // A list costs a wave a round trip to the columns before the first weights, and the second half another: the fewer
+    // tiles a workgroup has, the less there is to win them back.  16-row strips against halves, us: 2048 x 3072 -> 768 at 80 % 11.3 / 9.8,
+    // 2560 at 90 % 12.2 / 9.5, 2048 x 4096 -> 1024 at 50 % 39 / 25, 4096 x 4096 -> 1024 at 90 % 25.3 / 24.2, 8192 x 3072 -> 768 at
+    // 95 % 21.1 / 20.4, but 4096 at 95 % 9.9 / 11.1, 2048 at 95 % 6.9 / 8.4 (the number of tiles is not known on the host); fewer
+    // than a block-row a wave 2048 x 4096 -> 256 9.5 / 9.8, 4096 x 3072 -> 96 7.3 / 8.4.
+    const size_t lds_cap = 160 * 1024;
+    if ((size_t)32 * (in + kLdsPad) * sizeof(_Float16) <= lds_cap / 2) return 0;  // 32 rows in one piece
+    const int nbr = out / 16, strips = (T + 31) / 32;
+    if (strips < 64) return 0;
+    const int most = halves_lds_bytes(in, 4 * kHalfWaves) <= lds_cap ? 4 * kHalfWaves : halves_lds_bytes(in, 2 * kHalfWaves) <= lds_cap ? 2 * kHalfWaves : 0;
+    if (!most) return 0;
+    int groups = strips >= 256 ? 1 : 256 / strips;
+    groups = std::max(groups, (nbr + most - 1) / most);
+    const int rows = (nbr + groups - 1) / groups;
+    return rows >= kHalfWaves ? rows : 0;
+}
+
 static int dispatch_bsr(const BsrArgs &args, const BsrPlan &p, hipStream_t stream) {
     ET_REQUIRE(p.rows_per_wg >= 1 && p.rows_per_wg <= kMaxWaveRows * (p.threads / 64), ET_ERR_UNSUPPORTED,
                "tile-sparse Linear: %d block-rows per workgroup of %d waves exceed %d per wave", p.rows_per_wg,
@@ -959,6 +1230,21 @@ static int dispatch_bsr(const BsrArgs &args, const BsrPlan &p, hipStream_t strea
         case 2: return launch_bsr<2, false>(args, p, stream);
         default: return launch_bsr<1, false>(args, p, stream);
     }
+}
+
+static int launch_bsr_plain(BsrArgs args, hipStream_t stream) {
+    const int rows = plan_halves(args.T, args.in, args.out);
+    if (rows && ((reinterpret_cast<uintptr_t>(args.X) | reinterpret_cast<uintptr_t>(args.tiles)) & 15) == 0) {  // pieces of 16 bytes
+        args.rows_per_wg = rows;
+        switch (args.act) {
+            case ET_ACT_RELU: return launch_bsr_halves<ET_ACT_RELU>(args, rows, stream);
+            case ET_ACT_GELU: return launch_bsr_halves<ET_ACT_GELU>(args, rows, stream);
+            default: return launch_bsr_halves<ET_ACT_NONE>(args, rows, stream);
+        }
+    }
+    const BsrPlan p = plan_bsr(args.T, args.in, args.out);
+    args.rows_per_wg = p.rows_per_wg;
+    return dispatch_bsr(args, p, stream);
 }
 
 }  // namespace et
@@ -998,9 +1284,7 @@ int et_linear_bsr16_f16(const int32_t *row_ptr, const int32_t *col_idx, const et
                  0,
                  act,
                  nullptr, nullptr, nullptr, nullptr, nullptr, 0.0f, nullptr, 0, nullptr, nullptr};
-    BsrPlan p = plan_bsr(T, in, out);
-    args.rows_per_wg = p.rows_per_wg;
-    return dispatch_bsr(args, p, as_stream(stream));
+    return launch_bsr_plain(args, as_stream(stream));
 }
 
 int et_linear_bsr16_f16_f32out(const int32_t *row_ptr, const int32_t *col_idx, const et_f16 *tiles,
@@ -1022,9 +1306,7 @@ int et_linear_bsr16_f16_f32out(const int32_t *row_ptr, const int32_t *col_idx, c
     args.out = out;
     args.act = act;
     args.Y32 = Y;
-    BsrPlan p = plan_bsr(T, in, out);
-    args.rows_per_wg = p.rows_per_wg;
-    return dispatch_bsr(args, p, as_stream(stream));
+    return launch_bsr_plain(args, as_stream(stream));
 }
 
 int et_skipln_linear_bsr16_f16(const et_f16 *src, const et_f16 *skip, const et_f16 *gamma,

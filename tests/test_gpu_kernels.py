@@ -278,6 +278,43 @@ def test_linear_bsr16_f32_output(et, T, inp, out, sp, act):
         assert np.mean(a != b) < 1e-3
 
 
+# Strips of 32 rows staged a half of the columns at a time: the smallest and the largest width, an odd number of column tiles, a last
+# strip of 16 rows, one block-row a wave to four and waves with fewer, block-rows without tiles, with tiles in one
+# half only, with all of them, and (ids drawn twice) with more tiles than columns; columns in any order.
+@pytest.mark.parametrize("T,inp,out,act", [(2048, 1280, 768, 0), (2064, 3072, 816, 2), (2064, 2000, 800, 1), (8208, 3056, 208, 0),
+                                           (8192, 4096, 400, 0), (16400, 1296, 800, 2)])
+@pytest.mark.parametrize("order", ["rising", "falling", "drawn", "twice"])
+def test_linear_bsr16_strip_halves(et, T, inp, out, act, order):
+    rng = np.random.default_rng(inp + out)
+    nc, rows = inp // 16, []
+    for b in range(out // 16):
+        lo, hi = ((0, nc), (0, nc), (0, (nc + 1) // 2), ((nc + 1) // 2, nc), (0, nc))[b % 5]
+        n = (0, 1, 2, 15, 16, 17, 33, 64, 65, 1000)[int(rng.integers(0, 10))]
+        ids = rng.permutation(np.arange(lo, hi))[:n]
+        if order == "twice" and b % 3 == 0:
+            ids = rng.integers(0, nc, nc + 1 + int(rng.integers(0, 70)))
+        rows.append({"rising": np.sort(ids), "falling": -np.sort(-ids)}.get(order, ids))
+    row_ptr = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    col_idx = np.concatenate(rows).astype(np.int32)
+    tiles, bias, x = Hn.randn((len(col_idx), 256), 1, 0.02), Hn.randn((out,), 2, 0.1), Hn.randn((T, inp), 3)
+    dense = np.zeros((out, inp), np.float32)
+    for b in range(out // 16):
+        for t in range(row_ptr[b], row_ptr[b + 1]):
+            dense[16 * b:16 * b + 16, 16 * col_idx[t]:16 * col_idx[t] + 16] += tiles[t].reshape(16, 16).astype(np.float32)
+    d = [up(et, v) for v in (row_ptr, col_idx, tiles, bias, x)]
+    d_y, d_y32 = up(et, np.full((T + 16, out), 7, np.float16)), up(et, np.full((T + 16, out), 7, np.float32))
+    et.check(et.lib().et_linear_bsr16_f16(*[v.ptr for v in d], d_y.ptr, T, inp, out, act, None))
+    et.check(et.lib().et_linear_bsr16_f16_f32out(*[v.ptr for v in d], d_y32.ptr, T, inp, out, act, None))
+    want = L.linear(Hn.f32(x), Hn.f32(dense), Hn.f32(bias), {0: None, 1: "relu", 2: "gelu"}[act], None).numpy()
+    scale = max(1.0, float(np.abs(want).max()))
+    y, y32 = d_y.numpy(), d_y32.numpy()
+    # binary32 sums of at most 2 x 4096 exact products (a column drawn twice is one sum in the reference): order of
+    # accumulation only; a binary16 rounding of the result on top
+    assert Hn.max_abs(y32[:T], want) <= 5e-5 * scale
+    assert Hn.max_abs(y[:T], want) <= 1e-3 * scale
+    assert (y[T:] == 7).all() and (y32[T:] == 7).all()
+
+
 PLANNED_CASES = [
     # T, in, out, sparsity, act, (mt, kc, rows_per_wg) or None for the automatic geometry
     (1024, 768, 2304, 0.8, 0, None),
