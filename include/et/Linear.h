@@ -178,13 +178,15 @@ template <> class Linear<tile_mat> {
     tile_mat weight;
     et::DeviceBuffer<half> bias;
     // Re-ordered copy of the weight for the streaming kernel (et_bsr16_plan_create), held where
-    // that kernel is the faster one: inputs too wide for an LDS-resident token strip, and wide
-    // inputs at many token rows (measured: 1.6-2x at in > 5112, 1.1-1.4x at in >= 3072 from 4096 rows).
+    // that kernel is the faster one: inputs too wide for an LDS-resident token strip (1.6-2x at in > 5112), and at many
+    // token rows those too wide for half a strip of 32 (8192 x 5008 -> 1024 at 80 % 96 against 81 us, 16384 188 / 114).  Up to 4224 the
+    // plain call takes strips in halves and is the faster one: 4096 x 3072 -> 768 at 55 / 80 / 95 % 24 / 16 / 12 against 45 / 27 / 21 us,
+    // 16384 88 / 56 / 42 against 114 / 65 / 50, 16384 x 4096 -> 1024 161 / 98 / 67 against 166 / 96 / 70.
     struct PlanDeleter {
         void operator()(et_bsr_plan_s *p) const { (void)et_bsr16_plan_destroy(p); }
     };
     std::unique_ptr<et_bsr_plan_s, PlanDeleter> plan;
-    static bool wants_plan(int in, int rows) { return in >= 128 && (in > 5112 || (in >= 3072 && rows >= 4096)); }
+    static bool wants_plan(int in, int rows) { return in >= 128 && (in > 5112 || (in > 4224 && rows >= 4096)); }
     // Copies of the weight in the order one launch of the packed kernel reads it (et_bsr16_pack_create),
     // held where that kernel applies — up to kPackMaxRows token rows, inputs that are multiples of 128
     // up to 4096: a launch whose loads are all issued at its start, with no row-pointer round trip.
