@@ -710,7 +710,8 @@ __global__ __launch_bounds__(((MT == 1 && (FX & kFxRes32) && !(FX & kFxRes16)) |
 // twice, is not listed: it takes its operands from memory at the end.)
 // 16-row strips against this, us: 4096 x 3072 -> 768 at 80 % 21.1 / 14.9, 70 % of 3072 rows 24.8 / 16.6, 16384 82 / 55,
 // 16384 x 4096 -> 1024 148 / 88, 16384 x 2048 -> 2048 152 / 97; two items asked for ahead 14.9, three 15.5, four 17; 16 waves 15.6; the
-// second half asked for into registers during the first 15.3; lists without the straight-line items 23.3.
+// second half asked for into registers during the first 15.3, behind it 15.8; a kernel of its own for one block-row a wave 9.1 against
+// 9.8 at 2048 x 3072 -> 768; lists without the straight-line items 23.3.
 // Error of the sums against binary64: 0.7 times that of the other form (two shorter sums to a value).
 constexpr int kHalfWaves = 12;
 constexpr int kHalfAhead = 2;           // items asked for ahead
@@ -768,7 +769,7 @@ __global__ __launch_bounds__(kHalfWaves * 64) void bsr16_linear_halves_kernel(co
     // row r's last in half h.
     const int most = a.in >> 4, per_row = (half + 7) >> 3;  // tiles of a row, items of a row and half, at most
     int *list = reinterpret_cast<int *>(xs + MT * 16 * lds_ld) + wave * (2 * RW * per_row * 8);
-    auto entry = [&](int h, int item, int k) -> int & { return list[(h * RW * per_row + item) * 8 + (k & 7 & 1) * 4 + ((k & 7) >> 1)]; };
+    auto place = [](int k) { return (k & ~7) | (k & 1) << 2 | (k >> 1 & 3); };  // of the k-th tile behind the start of its row's first item
     int ends[2][RW];
     unsigned unlisted = 0;
     {
@@ -785,19 +786,18 @@ __global__ __launch_bounds__(kHalfWaves * 64) void bsr16_linear_halves_kernel(co
             int have[2] = {0, 0}, some[2] = {0, 0};
             if (n > most) unlisted |= 1u << r;
             else
-                for (int base = 0; base < n; base += 64) {
+                for (int base = 0; base < n; base += 64) {  // the lanes with a tile are the first ones
                     const bool real = base + lane < n;
                     const int c = base == 0 ? first[r] : real ? a.col_idx[t0 + base + lane] : 0;
-                    const unsigned long long in_half[2] = {__ballot(real && c < half), __ballot(real && c >= half)};
-                    const int h = c >= half;
-                    const unsigned long long mine = h ? in_half[1] : in_half[0];
-                    const int k = (h ? have[1] : have[0]) + __builtin_amdgcn_mbcnt_hi((unsigned)(mine >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mine, 0));
-                    if (real && k < half) entry(h, (h ? at[1] : at[0]) + (k >> 3), k) = (base + lane) << 16 | (c - h * half);
-#pragma unroll
-                    for (int k2 = 0; k2 < 2; k2++) {
-                        have[k2] += __popcll(in_half[k2]);
-                        if (in_half[k2]) some[k2] = lane_read(c, __builtin_ctzll(in_half[k2])) - k2 * half;
-                    }
+                    const unsigned long long low = __ballot(real && c < half), high = __ballot(real && c >= half);
+                    const int before = __builtin_amdgcn_mbcnt_hi((unsigned)(low >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)low, 0));
+                    const int k = c < half ? have[0] + before : have[1] + lane - before;
+                    const int start = (c < half ? at[0] : RW * per_row + at[1]) * 8;
+                    if (real && k < half) list[start + place(k)] = (base + lane) << 16 | (c < half ? c : c - half);
+                    have[0] += __popcll(low);
+                    have[1] += __popcll(high);
+                    if (low) some[0] = lane_read(c, __builtin_ctzll(low));
+                    if (high) some[1] = lane_read(c, __builtin_ctzll(high)) - half;
                 }
             if (have[0] > half || have[1] > half) {
                 unlisted |= 1u << r;
@@ -808,7 +808,7 @@ __global__ __launch_bounds__(kHalfWaves * 64) void bsr16_linear_halves_kernel(co
                 const int items = (have[h] + 7) >> 3;
                 if (have[h] & 7) {  // the last item is filled up with a tile past the row (zero) and a column the row has
                     const int fill = kNoTile << 16 | some[h];
-                    if (lane < 8 && lane >= (have[h] & 7)) entry(h, at[h] + items - 1, lane) = fill;
+                    if (lane < 8 && lane >= (have[h] & 7)) list[(h * RW * per_row + at[h] + items - 1) * 8 + place(lane)] = fill;
                 }
                 at[h] += items;
                 ends[h][r] = __builtin_amdgcn_readfirstlane(at[h]);
@@ -1180,13 +1180,13 @@ static int dispatch_bsr_res(const BsrArgs &args, const BsrPlan &p, hipStream_t s
 
 // LDS of a workgroup of the halves form: half a strip of 32 rows, and a list of the tiles of each block-row of a wave.
 static size_t halves_lds_bytes(int in, int rows_per_wg) {
-    const int rw = rows_per_wg <= 2 * kHalfWaves ? 2 : 4;
+    const int rw = rows_per_wg <= kHalfWaves ? 1 : rows_per_wg <= 2 * kHalfWaves ? 2 : 4;
     return (size_t)32 * (half_tiles(in) * 16 + kLdsPad) * sizeof(_Float16) + (size_t)kHalfWaves * 2 * rw * ((half_tiles(in) + 7) / 8) * 8 * sizeof(int);
 }
 
 template <int ACT>
 static int launch_bsr_halves(const BsrArgs &args, int rows_per_wg, hipStream_t stream) {
-    auto kernel = rows_per_wg <= 2 * kHalfWaves ? bsr16_linear_halves_kernel<ACT, 2> : bsr16_linear_halves_kernel<ACT, 4>;
+    auto kernel = rows_per_wg <= kHalfWaves ? bsr16_linear_halves_kernel<ACT, 1> : rows_per_wg <= 2 * kHalfWaves ? bsr16_linear_halves_kernel<ACT, 2> : bsr16_linear_halves_kernel<ACT, 4>;
     const size_t lds = halves_lds_bytes(args.in, rows_per_wg);
     if (lds > 64 * 1024)
         ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -1199,9 +1199,9 @@ static int launch_bsr_halves(const BsrArgs &args, int rows_per_wg, hipStream_t s
 // Block-rows of a workgroup of the halves form, 0 where another form is the faster one.
 static int plan_halves(int T, int in, int out) {
     // A list costs a wave a round trip to the columns before the first weights, and the second half another: the fewer
-    // tiles a workgroup has, the less there is to win them back.  16-row strips against halves, us: 2048 x 3072 -> 768 at 80 % 11.3 / 9.8,
-    // 2560 at 90 % 12.2 / 9.5, 2048 x 4096 -> 1024 at 50 % 39 / 25, 4096 x 4096 -> 1024 at 90 % 25.3 / 24.2, 8192 x 3072 -> 768 at
-    // 95 % 21.1 / 20.4, but 4096 at 95 % 9.9 / 11.1, 2048 at 95 % 6.9 / 8.4 (the number of tiles is not known on the host); fewer
+    // tiles a workgroup has, the less there is to win them back.  16-row strips against halves, us: 2048 x 3072 -> 768 at 80 % 11.5 / 9.1,
+    // 2560 at 90 % 12.2 / 9.3, 2048 x 4096 -> 1024 at 50 % 39 / 24, 4096 x 4096 -> 1024 at 90 % 25.3 / 24.2, 8192 x 3072 -> 768 at
+    // 95 % 21.1 / 20.4, but 4096 at 95 % 9.9 / 11.1, 2048 at 95 % 6.6 / 7.5 (the number of tiles is not known on the host); fewer
     // than a block-row a wave 2048 x 4096 -> 256 9.5 / 9.8, 4096 x 3072 -> 96 7.3 / 8.4.
     const size_t lds_cap = 160 * 1024;
     if ((size_t)32 * (in + kLdsPad) * sizeof(_Float16) <= lds_cap / 2) return 0;  // 32 rows in one piece
