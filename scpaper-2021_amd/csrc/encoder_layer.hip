@@ -28,7 +28,7 @@
 // the second product in binary32; the second adds the shares in a fixed order, applies LN2 and runs its share of
 // the QKV block-rows.  That projection can be had alone, of x' as it was rounded for it (et_encoder_layer_project_f16), so
 // that a stack whose layers hand binary16 to each other gives the same bits layer by layer.
-// The joined launch does both: behind the second product the parts of a strip meet at a word in their XCD's L2 (el_wait), and
+// The joined launch does both: behind the second product the parts of a strip meet at a word in their XCD's L2 (meet_wait), and
 // the shares come back out of that L2, where behind a launch boundary they come from the memory-side cache, as do table, offsets
 // and first slots, which here are on their way while the parts meet; 2 us of boundary go besides.  8 x 128 tokens at 80 %
 // 382 -> 361 us (12 layers, weights in the memory-side cache), 12 x 128 241 -> 220 (6 layers), BERT-large 4 x 512 at 90 % 1175 ->
@@ -49,6 +49,7 @@
 #include <vector>
 
 #include "common.hip.h"
+#include "strip_meeting.h"
 
 namespace et {
 
@@ -244,41 +245,20 @@ __device__ __forceinline__ int el_here_s(int v) {  // the same for a uniform val
     return v;
 }
 
-// The parts of a strip meet at a word in the L2 of their XCD: arrivals in bits 0-7, parts that did not wait in bits 8-19,
-// parts that are through in bits 20-27; the last to be through puts it back to zero.  Whoever arrives last waits for nobody.
-// The others wait a bounded time, and then leave their share of the projection to the last: nothing ever depends on two
-// workgroups being resident at once.  One wave, its first lane.  (In assembly: the arrival is in flight while the ring goes
-// out, and an addition of nothing, which the wait reads the word with, would become a load that the L1 answers.)
-constexpr int kElMaxJoin = 12;
+// The word in the L2 of their XCD at which the parts of a strip meet (strip_meeting.h).  One wave, its first lane.  (In assembly:
+// the arrival is in flight while the ring goes out, and an addition of nothing, which a part that waits reads the word with, would
+// become a load that the L1 answers.)
 #define ET_EL_ADD "s_mov_b64 exec, 1\n\tglobal_atomic_add %0, %1, %2, off sc0\n\ts_mov_b64 exec, -1"
-__device__ __forceinline__ uint32_t el_add(uint32_t *word, uint32_t v) {
-    uint32_t was;
-    asm volatile(ET_EL_ADD "\n\ts_waitcnt vmcnt(0)" : "=&v"(was) : "v"(word), "v"(v) : "memory");
-    return (uint32_t)__builtin_amdgcn_readfirstlane((int)was);
-}
-__device__ __forceinline__ void el_through(uint32_t *word, uint32_t was, int parts) {  // `was`: before this part was counted through
-    if ((int)(was >> 20) + 1 == parts) __hip_atomic_store(word, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-// behind the arrival that found `was`: the parts to run besides one's own, or -1: leave
-__device__ __forceinline__ int el_wait(uint32_t *word, uint32_t was, int part, int parts, bool projecting, int spin) {
-    if ((int)(was & 255) + 1 == parts) return (int)(was >> 8 & 0xfff);
-    if (!projecting) {  // a normalisation alone is for the last
-        el_through(word, el_add(word, 1u << 20), parts);
-        return -1;
+struct ElWord {
+    uint32_t *at;
+    __device__ __forceinline__ uint32_t add(uint32_t v) {
+        uint32_t was;
+        asm volatile(ET_EL_ADD "\n\ts_waitcnt vmcnt(0)" : "=&v"(was) : "v"(at), "v"(v) : "memory");
+        return (uint32_t)__builtin_amdgcn_readfirstlane((int)was);
     }
-    for (int n = 0; n < spin; n++) {
-        if ((int)(el_add(word, 0u) & 255) == parts) return 0;
-        __builtin_amdgcn_s_sleep(1);
-    }
-    // (all there after all: the last one could not be told, and the count of those through is taken back)
-    const uint32_t now = el_add(word, (1u << 20) + (1u << (8 + part)));
-    if ((int)(now & 255) == parts) {
-        (void)el_add(word, 0u - (1u << 20));
-        return 0;
-    }
-    el_through(word, now, parts);
-    return -1;
-}
+    __device__ __forceinline__ void clear() { __hip_atomic_store(at, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+    __device__ __forceinline__ void pause() { __builtin_amdgcn_s_sleep(1); }
+};
 
 // MODE 0: all steps.  1: up to the second product, binary32 share to `partial`.  2: from the sum of the shares on.  3: the
 // projection alone, of x' as 2 rounds it, given in `Z`: the same products in the same order.
@@ -611,11 +591,11 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
         if (wave == 0) {
             const auto *l = late();
             uint32_t *const word = l->join + strip, was;
-            asm volatile(ET_EL_ADD : "=&v"(was) : "v"(word), "v"(1u) : "memory");
+            asm volatile(ET_EL_ADD : "=&v"(was) : "v"(word), "v"(kMeetArrived) : "memory");
             el_ring_start(lane_off, offs_off, slots, offs);
             asm volatile("s_waitcnt vmcnt(%0)" ::"i"(kElRingAsks) : "memory");
             el_tie(was);
-            *got = el_wait(word, (uint32_t)__builtin_amdgcn_readfirstlane((int)was), part, l->parts, l->Q > 0, l->spin);
+            *got = meet_wait(ElWord{word}, (uint32_t)__builtin_amdgcn_readfirstlane((int)was), part, l->parts, l->Q > 0, l->spin);
         } else {
             el_ring_start(lane_off, offs_off, slots, offs);
         }
@@ -776,8 +756,7 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
         }
         if (wave == 0) {
             const auto *l = late();
-            uint32_t *const word = l->join + strip;
-            el_through(word, el_add(word, 1u << 20), l->parts);
+            meet_through(ElWord{l->join + strip}, l->parts);
         }
     }
 }
@@ -1218,7 +1197,7 @@ static int el_xcd_by_id(bool *by_id) {
 extern "C" int et_encoder_layer_joins(const struct et_layer_pack_s *p, int *joins) {
     ET_REQUIRE(p && joins, ET_ERR_INVALID_ARG, "et_encoder_layer_joins: NULL pointer");
     bool by_id = false;
-    const int s = p->parts > 1 && p->parts <= kElMaxJoin ? el_xcd_by_id(&by_id) : ET_OK;
+    const int s = p->parts > 1 && p->parts <= kMeetMaxParts ? el_xcd_by_id(&by_id) : ET_OK;
     *joins = by_id;
     return s;
 }
@@ -1274,6 +1253,6 @@ extern "C" int et_encoder_layer_joined_f32(const struct et_layer_pack_s *p, cons
                static_cast<void *>(join), spin);
     const int s = et_encoder_layer_joins(p, &joins);
     if (s != ET_OK) return s;
-    ET_REQUIRE(joins, ET_ERR_UNSUPPORTED, "et_encoder_layer_joined_f32: one part, more than %d, or a device that deals workgroups otherwise", kElMaxJoin);
+    ET_REQUIRE(joins, ET_ERR_UNSUPPORTED, "et_encoder_layer_joined_f32: one part, more than %d, or a device that deals workgroups otherwise", kMeetMaxParts);
     return el_run(p, Z, x32, x16, x32_out, out16, QKV, partial, join, spin, act, eps1, eps2, stream);
 }
