@@ -88,8 +88,8 @@ template <int MT> __global__ __launch_bounds__(256) void bsr16_linear_wide_f32_k
 // The waves of a workgroup share one (block-row, 16 tokens), each every WAVES-th tile; the sums meet in LDS and are added
 // in the order of the waves.  A lane reads the column index of one of its wave's tiles, 64 at a time, so no operand waits
 // for an index from memory, and kAhead tiles are requested ahead of the products.  The requests are straight-line and go
-// through buffer resources that end with the tiles: one past the last moves nothing (asking for the last tile again, as
-// before, cost 16 tokens of a 6-layer stack of 768 at 80 % 13 us of 175).  8 ahead are slower, 300 us against 292 for 256
+// through buffer resources that end with the tiles: one past the last moves nothing.  (Its whole offset is in the vector
+// operand, which the bounds check is documented to look at.  Asking for the last tile again, as before, cost 16 tokens of a 6-layer stack of 768 at 80 % 13 us of 175).  8 ahead are slower, 300 us against 292 for 256
 // tokens of that stack: it is no longer the latency of a load that bounds a pair.
 //
 // The workgroups of one die (blockIdx.x % 8) keep to a part of the strips and a part of the columns of the grid, so that what an L2
@@ -125,8 +125,8 @@ __global__ __launch_bounds__(WAVES * 64) void bsr16_linear_split_f32_kernel(cons
         float4 w[kAhead], x[kAhead];
         auto ask = [&](int slot, int i) {
             const int xat = i < here ? __builtin_amdgcn_readlane(cols, i & 63) * 64 : kPastEnd;
-            w[slot] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(wr, wo, i * WAVES * 1024, 0));
-            x[slot] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xr, xo, xat, 0));
+            w[slot] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(wr, wo + i * WAVES * 1024, 0, 0));
+            x[slot] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xr, xo + xat, 0, 0));
         };
 #pragma unroll
         for (int s = 0; s < kAhead; s++) ask(s, s);
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(kStripWaves * 64) void bsr16_linear_strip_f32_kerne
         const auto wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.tiles) + (size_t)t0 * 256, 0, here * 1024, kRawBuffer);
         float4 w[kAhead];
         auto ask = [&](int slot, int i) {
-            w[slot] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(wr, wo, i * 1024, 0));
+            w[slot] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(wr, wo + i * 1024, 0, 0));
         };
 #pragma unroll
         for (int s = 0; s < kAhead; s++) ask(s, s);
