@@ -23,7 +23,7 @@ struct Bsr32Args {
     const float *tiles, *bias, *X;
     float *Y;
     int T, in, out, act;
-    int strip_dies;  // 1, 2, 4 or 8: see strip_of
+    int die_bits;  // 0 to 3: see strip_of
 };
 
 __device__ __forceinline__ f4 mfma_cell_f32(const float4 w, const float4 x, f4 acc) {
@@ -93,11 +93,12 @@ template <int MT> __global__ __launch_bounds__(256) void bsr16_linear_wide_f32_k
 // tokens of that stack: it is no longer the latency of a load that bounds a pair.
 //
 // The workgroups of one die (blockIdx.x % 8) keep to a part of the strips and a part of the columns of the grid, so that what an L2
-// has to fetch is a part of X and a part of the weights: strip_dies parts of the strips, 8 / strip_dies of the columns.
-__device__ __forceinline__ int strip_of(int strip_dies) {
-    return (int)(blockIdx.x & (strip_dies - 1)) + strip_dies * (int)(blockIdx.y + blockIdx.z * gridDim.y);
+// has to fetch is a part of X and a part of the weights: 2^die_bits parts of the strips, 8 / 2^die_bits of the columns.  (By shifts:
+// two divisions by the number of parts cost every wave 0.3 us.)
+__device__ __forceinline__ int strip_of(int die_bits) {
+    return (int)(blockIdx.x & ((1u << die_bits) - 1)) + ((int)(blockIdx.y + blockIdx.z * gridDim.y) << die_bits);
 }
-__device__ __forceinline__ int column_of(int strip_dies) { return (int)((blockIdx.x & 7) / strip_dies) + 8 / strip_dies * (int)(blockIdx.x >> 3); }
+__device__ __forceinline__ int column_of(int die_bits) { return (int)((blockIdx.x & 7) >> die_bits) + ((int)(blockIdx.x >> 3) << (3 - die_bits)); }
 
 constexpr int kAhead = 4;
 constexpr int kRawBuffer = 0x00020000;   // word 3 of a resource: raw, 32-bit data
@@ -108,7 +109,7 @@ __global__ __launch_bounds__(WAVES * 64) void bsr16_linear_split_f32_kernel(cons
     __shared__ f4 part[WAVES][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, q = lane >> 4;
-    const int strip = strip_of(a.strip_dies), br = column_of(a.strip_dies);
+    const int strip = strip_of(a.die_bits), br = column_of(a.die_bits);
     if (strip * 16 >= a.T || br >= (a.out >> 4)) return;  // padding of the grid (whole workgroup)
     const int tok = strip * 16 + r16;
     const f4 bias = bias_cell_f32(a.bias, br * 16 + 4 * q);
@@ -160,7 +161,7 @@ __global__ __launch_bounds__(kStripWaves * 64) void bsr16_linear_strip_f32_kerne
     float *xs = reinterpret_cast<float *>(strip_smem);  // [16][in + kStripPad]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, q = lane >> 4;
-    const int strip = strip_of(a.strip_dies), br = column_of(a.strip_dies) * kStripWaves + wave;
+    const int strip = strip_of(a.die_bits), br = column_of(a.die_bits) * kStripWaves + wave;
     if (strip * 16 >= a.T || br - wave >= (a.out >> 4)) return;  // padding of the grid (whole workgroup)
     const int ld = a.in + kStripPad, tok0 = strip * 16, quads = a.in >> 2;
     const bool mine = br < (a.out >> 4);  // uniform
@@ -327,17 +328,26 @@ int et_linear_bsr16_f32(const int32_t *row_ptr, const int32_t *col_idx, const fl
     ET_REQUIRE(aligned16(tiles) && aligned16(X) && aligned16(Y), ET_ERR_UNSUPPORTED,
                "et_linear_bsr16_f32: tiles, X and Y must be 16-byte aligned");
     if (T == 0) return ET_OK;
-    Bsr32Args a{row_ptr, col_idx, tiles, bias, X, Y, T, in, out, act, 1};
+    Bsr32Args a{row_ptr, col_idx, tiles, bias, X, Y, T, in, out, act, 0};
     hipStream_t st = as_stream(stream);
     const int strips = (T + 15) / 16;
-    // The parts of the strips and of the columns the dies keep to: the split that leaves one die the fewest bytes, taking
-    // a fifth of the tiles as kept (their number is not known here).
+    // The parts of the strips and of the columns the dies keep to: of the splits that leave the busiest die the fewest
+    // (strip, column) pairs, or up to 3 % more, the one that leaves a die the fewest bytes, taking a fifth of the tiles as kept
+    // (their number is not known here).  Against the best of the four splits, 23 shapes of 16 to 4096 rows: 1.00 - 1.03 of its
+    // time at 50 % sparsity, 1.00 - 1.04 at 80 %, 1.00 - 1.05 at 95 %.  (By bytes alone the dies were loaded unevenly: 160 rows
+    // 3072 -> 768 at 50 % 15.2 us, now 10.7.)
     auto place = [&](int columns) {
-        auto bytes = [&](int d) { return (double)T / d + 0.2 * out * d / 8; };  // in units of a row of X
-        for (int d = 2; d <= 8 && d <= strips; d *= 2)
-            if (bytes(d) < bytes(a.strip_dies)) a.strip_dies = d;
-        const int column_dies = 8 / a.strip_dies, rows = (strips + a.strip_dies - 1) / a.strip_dies, gy = std::min(rows, 32768);
-        return dim3(8 * ((columns + column_dies - 1) / column_dies), gy, (rows + gy - 1) / gy);
+        auto parts = [](int n, int d) { return (n + d - 1) / d; };
+        auto load = [&](int k) { return (double)parts(strips, 1 << k) * parts(columns, 8 >> k); };
+        auto bytes = [&](int k) { return (double)T / (1 << k) + 0.2 * out * (1 << k) / 8; };  // in units of a row of X
+        double least = load(0);
+        for (int k = 1; k <= 3; k++) least = std::min(least, load(k));
+        int best = -1;
+        for (int k = 0; k <= 3; k++)
+            if (load(k) <= 1.03 * least && (best < 0 || bytes(k) < bytes(best))) best = k;
+        a.die_bits = best;
+        const int rows = parts(strips, 1 << best), gy = std::min(rows, 32768);
+        return dim3(8 * parts(columns, 8 >> best), gy, parts(rows, gy));
     };
     const long long pairs = (long long)(out / 16) * strips;
     const size_t lds = (size_t)16 * (in + kStripPad) * sizeof(float);
