@@ -13,7 +13,6 @@
 
 #include "common.hip.h"
 
-#define ET_GLOBAL_PTR(p) ((const __attribute__((address_space(1))) void *)(p))
 #define ET_LDS_PTR(p) ((__attribute__((address_space(3))) void *)(p))
 
 namespace et {
@@ -152,9 +151,9 @@ __global__ __launch_bounds__(WAVES * 64) void bsr16_linear_split_f32_kernel(cons
 // Eight waves, eight neighbouring block-rows, 16 tokens, whose rows of X lie in LDS (kStripPad floats between two rows:
 // the 16 cells of a fragment read lie in different banks).  Read from memory, the fragment of a tile is 16 rows x 64 bytes,
 // and 16 neighbouring lanes touch 16 lines: with many tiles that is what the kernels above wait for.  The rows go straight
-// to LDS, all of them requested before anything is waited for, with the first weights behind them.  Against the wide
-// form: 4096 tokens 768 -> 3072 at 50 / 80 / 90 / 95 % 116 / 188, 70 / 96,
-// 56 / 56, 51 / 37 (staging a strip for a few tiles; the number of tiles is not known on the host).
+// to LDS, all of them requested before anything is waited for, with the first weights behind them, which stay in flight
+// across the barrier (waited for with the rows, 256 tokens 768 -> 2304 at 80 % 8.05 us, now 6.7; 2048 768 -> 3072 35.8 / 29.1).
+// Against the wide form: 4096 tokens 768 -> 3072 at 50 / 80 / 90 / 95 % 109 / 163, 52 / 78, 39 / 48, 33 / 34.
 constexpr int kStripPad = 4, kStripWaves = 8;
 __global__ __launch_bounds__(kStripWaves * 64) void bsr16_linear_strip_f32_kernel(const Bsr32Args a) {
     extern __shared__ __align__(16) unsigned char strip_smem[];
@@ -165,22 +164,27 @@ __global__ __launch_bounds__(kStripWaves * 64) void bsr16_linear_strip_f32_kerne
     if (strip * 16 >= a.T || br - wave >= (a.out >> 4)) return;  // padding of the grid (whole workgroup)
     const int ld = a.in + kStripPad, tok0 = strip * 16, quads = a.in >> 2;
     const bool mine = br < (a.out >> 4);  // uniform
-    const int ts = mine ? a.row_ptr[br] : 0, n = mine ? a.row_ptr[br + 1] - ts : 0;
+    const int at = mine ? br : 0, ts = a.row_ptr[at], te = a.row_ptr[at + 1];  // (used behind the rows' requests)
     for (int row = wave; row < 16; row += kStripWaves) {  // past the end: the last row, not stored
         const float *src = a.X + (size_t)min(tok0 + row, a.T - 1) * a.in;
         for (int i = 0; i < quads; i += 64)
-            if (i + lane < quads)
-                __builtin_amdgcn_global_load_lds(ET_GLOBAL_PTR(src + (i + lane) * 4), ET_LDS_PTR(xs + row * ld + i * 4), 16, 0, 0);
+            if (i + lane < quads) {
+                // (behind the compiler's back: it would wait for every request, the weights among them, before the LDS is read)
+                const unsigned to = (unsigned)(uintptr_t)ET_LDS_PTR(xs + row * ld + i * 4);
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane * 16), "s"(src + i * 4), "s"(to) : "memory", "m0");
+            }
     }
+    const int n = mine ? te - ts : 0;
     const f4 bias = bias_cell_f32(mine ? a.bias : nullptr, br * 16 + 4 * q);
     const float *xp = xs + r16 * ld + 4 * q;
     const int wo = (r16 * 16 + 4 * q) * 4;
     f4 acc = f4{0.f, 0.f, 0.f, 0.f};
-    auto staged = [] {                        // the strip is complete (every wave passes here once)
-        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's rows have landed
+    // the strip is complete (every wave passes one of the two once): behind the requests for weights, at most 4 of which
+    // may be outstanding, or behind the rows alone
+    if (n == 0) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-    };
-    if (n == 0) staged();
+    }
     for (int base = 0; base < n; base += 64) {
         const int here = min(n - base, 64), t0 = ts + base;
         const int cols = a.col_idx[t0 + min(lane, here - 1)];
@@ -191,7 +195,10 @@ __global__ __launch_bounds__(kStripWaves * 64) void bsr16_linear_strip_f32_kerne
         };
 #pragma unroll
         for (int s = 0; s < kAhead; s++) ask(s, s);
-        if (base == 0) staged();
+        if (base == 0) {
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kAhead) : "memory");
+            __syncthreads();
+        }
         for (int i = 0; i < here; i += kAhead) {
 #pragma unroll
             for (int s = 0; s < kAhead; s++) {
@@ -352,7 +359,7 @@ int et_linear_bsr16_f32(const int32_t *row_ptr, const int32_t *col_idx, const fl
     const long long pairs = (long long)(out / 16) * strips;
     const size_t lds = (size_t)16 * (in + kStripPad) * sizeof(float);
     // The strip form where two workgroups fit a compute unit and there are six pairs or more for each: 80 %, us, strip
-    // against not: 2304 pairs of 768 values 8.2 / 8.8, 3072 8.7 / 11.5, 1536 6.2 / 6.6, 768 6.1 / 4.6.
+    // against not: 2304 pairs of 768 values 6.7 / 7.2, 3072 7.0 / 9.7, 1536 5.2 / 5.8, 768 5.1 / 4.0 (95 %: 2304 4.8 / 4.3, 3072 5.0 / 5.9).
     if (pairs >= 1536 && lds <= 80 * 1024) {
         if (lds > 64 * 1024)
             ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(bsr16_linear_strip_f32_kernel),
@@ -362,8 +369,8 @@ int et_linear_bsr16_f32(const int32_t *row_ptr, const int32_t *col_idx, const fl
         return check_launch("bsr16_linear_strip_f32_kernel");
     }
     // Wider than that, the wide form from two of its workgroups a compute unit on: 80 %, us, wide against short: 512 workgroups
-    // 1024 x 4096 -> 1024 40 / 51, 512 x 2048 -> 2048 22 / 31; 768 1024 x 1536 -> 1536 23 / 31, 4096 x 3072 -> 768 99 / 106; 384 2048 x 3072 ->
-    // 768 69 / 54, 512 x 1536 -> 1536 17.1 / 17.2.  (90 % and many rows of a narrow result 1.04 the other way.)
+    // 1024 x 4096 -> 1024 38 / 43, 512 x 2048 -> 2048 21 / 25; 768 1024 x 1536 -> 1536 22 / 27; 384 2048 x 3072 -> 768 52 / 46,
+    // 512 x 1536 -> 1536 15.4 / 14.3.  (Many rows of a narrow result 1.04 the other way: 768 4096 x 3072 -> 768 93 / 89.)
     const int mt = token_blocks(T), wide_strips = (T + 16 * mt - 1) / (16 * mt), wide_x = (out / 16 + 3) / 4;
     if (in > kSplitMaxIn || (mt > 1 && lds > 80 * 1024 && (long long)wide_x * wide_strips >= 512)) {
         const int wide_y = std::min(wide_strips, 32768);
