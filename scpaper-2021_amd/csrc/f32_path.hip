@@ -146,11 +146,13 @@ __global__ __launch_bounds__(256) void linear_dense_f32_kernel(const LinearF32Ar
 // A few hundred workgroups is all a verification batch has, so the length of one workgroup's chain is its time: HD / 4
 // products a key block and S / 4 a feature block, 32 cycles each.  2 x 128 tokens, 12 heads of 64: 20.3 -> 7.1 us, 1 x 512 tokens 85 -> 26 (the
 // former kernel staged K and V element by element and multiplied on the vector unit).
-// So the first keys and the first values are requested together at the start, and the next ones always ahead of the products:
-// the attention launch of a stack 1.2 us shorter at 2 x 128 tokens (9.9 before), 2.5 at 1 x 256, 0.3 longer at 16 tokens.
+// So the query and the first keys are requested together at the start, the next keys ahead of the products, and the first
+// values before the softmax: 12 heads of 64, 16 tokens 3.9 us, 1 x 64 4.9, 2 x 128 6.6, 1 x 256 9.8.  With neither ahead 3.9, 5.1,
+// 7.2 and 11.0; with the first values at the start, a branch around each cell and four blocks of values at once 4.2, 5.4, 7.6
+// and 11.5 (6 layers of 256 tokens 286 us, now 276).
 constexpr int kAttQ = 16;
 constexpr int kAttKeys = 64;  // (of the LDS limit of et_mha_fused_f32)
-constexpr int kAttAhead = 4;  // blocks of 16 keys whose values are asked for at once
+constexpr int kAttAhead = 2;  // blocks of 16 keys whose values are asked for at once
 constexpr int kAttPad = 4;    // floats between the rows of the strip: 16 rows' cells in different banks, 16-byte aligned
 
 struct MhaF32Args {
@@ -194,19 +196,15 @@ __global__ __launch_bounds__(256) void mha_fused_f32_kernel(const MhaF32Args a) 
     const int nkb = (kend + 15) >> 4;
     const float ninf = -__builtin_inff();
 
-    f4 qv[MAXC];
-    const float *qp = a.Q + (row0 + q0 + r16) * a.ldq + h * hd + 4 * g;
+    // (Cells past the head: its last one again, not multiplied.  With a branch around each, a wave waited for every cell of its
+    // query.)
+    f4 qv[MAXC], kv[MAXC], v[kAttAhead];
+    auto ask_row = [&](f4 (&to)[MAXC], const float *row) {
 #pragma unroll
-    for (int c = 0; c < MAXC; c++)
-        if (c < ncell) qv[c] = load_quad_f32<VEC>(qp + 16 * c) * a.scale;
-
-    // the first keys, and behind them the first values of the product at the end, travel together
-    f4 kv[MAXC], v[kAttAhead];
+        for (int c = 0; c < MAXC; c++) to[c] = load_quad_f32<VEC>(row + 16 * min(c, ncell - 1));
+    };
     auto ask_keys = [&](f4 (&k)[MAXC], int kb) {  // (keys past kend: the last one again, not used below)
-        const float *kp = a.K + (row0 + min(kb * 16 + r16, kend - 1)) * a.ldk + h * hd + 4 * g;
-#pragma unroll
-        for (int c = 0; c < MAXC; c++)
-            if (c < ncell) k[c] = load_quad_f32<VEC>(kp + 16 * c);
+        ask_row(k, a.K + (row0 + min(kb * 16 + r16, kend - 1)) * a.ldk + h * hd + 4 * g);
     };
     auto ask_values = [&](int c, int kb) {  // of kAttAhead blocks of keys
         const float *vp = a.V + row0 * a.ldv + h * hd + c * 16 + r16;
@@ -216,13 +214,15 @@ __global__ __launch_bounds__(256) void mha_fused_f32_kernel(const MhaF32Args a) 
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[s][j] = vp[(size_t)min((kb + s) * 16 + 4 * g + j, kend - 1) * a.ldv];
     };
-    if (wave < nkb) ask_keys(kv, wave);
-    if (wave < ncell) ask_values(wave, 0);
+    ask_row(qv, a.Q + (row0 + q0 + r16) * a.ldq + h * hd + 4 * g);
+    ask_keys(kv, wave);
+#pragma unroll
+    for (int c = 0; c < MAXC; c++) qv[c] *= a.scale;
 
     // ---- scores
     for (int kb = wave; kb < nkb; kb += 4) {
         f4 next[MAXC];
-        if (kb + 4 < nkb) ask_keys(next, kb + 4);
+        ask_keys(next, kb + 4);
         f4 s = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int c = 0; c < MAXC; c++)
@@ -239,6 +239,7 @@ __global__ __launch_bounds__(256) void mha_fused_f32_kernel(const MhaF32Args a) 
 #pragma unroll
         for (int c = 0; c < MAXC; c++) kv[c] = next[c];
     }
+    if (wave < ncell) ask_values(wave, 0);
     __syncthreads();
     // ---- softmax over the keys of row q: 16 threads per row (keys past kend become zeros)
     {
@@ -266,9 +267,12 @@ __global__ __launch_bounds__(256) void mha_fused_f32_kernel(const MhaF32Args a) 
         for (int kb = 0; kb < nkb; kb += kAttAhead) {
             f4 now[kAttAhead];
 #pragma unroll
-            for (int s = 0; s < kAttAhead; s++)
+            for (int s = 0; s < kAttAhead; s++) {
+                now[s] = v[s];
+                if ((kb + s + 1) * 16 > kend)  // uniform
 #pragma unroll
-                for (int j = 0; j < 4; j++) now[s][j] = (kb + s) * 16 + 4 * g + j < kend ? v[s][j] : 0.0f;
+                    for (int j = 0; j < 4; j++) now[s][j] = (kb + s) * 16 + 4 * g + j < kend ? v[s][j] : 0.0f;
+            }
             if (kb + kAttAhead < nkb) ask_values(c, kb + kAttAhead);
 #pragma unroll
             for (int s = 0; s < kAttAhead; s++) {
