@@ -111,13 +111,13 @@ __device__ __forceinline__ void ahead_of(const MhaArgs &a) {
 #pragma unroll
     for (int s = 0; s < ET_MHA_AHEAD; s++) {
         if (i < a.ahead_lines[s]) {
+            // (with its wait: nothing else knows that the register is written later)
             int line;
-            asm volatile("global_load_dword %0, %1, off" : "=v"(line) : "v"(a.ahead[s] + (size_t)i * 128) : "memory");
-            break;
+            asm volatile("global_load_dword %0, %1, off\n\ts_waitcnt vmcnt(0)" : "=v"(line) : "v"(a.ahead[s] + (size_t)i * 128) : "memory");
+            return;
         }
         i -= a.ahead_lines[s];
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 static unsigned ahead_blocks(const MhaArgs &a, int threads) {
     unsigned lines = 0;

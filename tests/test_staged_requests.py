@@ -72,3 +72,12 @@ def test_waits_for_staged_rows_count_what_is_behind_them(assemblies, source, ker
     later = re.sub(r"(ASMSTART\s+s_waitcnt vmcnt\()([1-9]\d*)", lambda m: m[1] + str(int(m[2]) + 40), assemblies[source])
     for name, (code, labels) in isa_waits.kernels(later).items():
         assert kernel not in name or short_waits(code, labels)[1], name
+
+
+def test_a_load_whose_value_nobody_wants_ends_with_its_wait():
+    """attention.hip asks for lines in assembly and drops their values: a register the compiler takes as free would be written
+    when the line arrives, unless the same block waits for it."""
+    source = (entry.PKG_DIR / "csrc" / "attention.hip").read_text()
+    blocks = re.findall(r"asm volatile\(((?:\s*\"(?:[^\"\\]|\\.)*\")+)\s*:\s*\"=&?v\"", source)
+    loads = [b for b in blocks if "_load_" in b]
+    assert loads and all("s_waitcnt vmcnt(0)" in b.split("_load_")[-1] for b in loads), loads
