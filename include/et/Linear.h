@@ -315,11 +315,14 @@ template <> class Linear<tile_mat> {
     // The split normalisation of the mixed-precision layer (et_linear_bsr16_resid_stats_f32 /
     // et_norm_linear_bsr16_f32in): this Linear as the producer of a binary32 sum with its row
     // sums, or as the consumer that normalises such a sum while it stages its token strip.
+    // Not for wide inputs at many rows: two 768-wide layers with 3072 hidden features, five launches / SkipLayerNorm on its own
+    // at 60 / 80 / 90 % sparsity, 4096 rows 302 / 198, 209 / 167, 154 / 151 us, 8192 rows 484 / 365, 349 / 305, 295 / 273.
+    static bool split_pays(int in, int rows) { return in < 3072 || rows < 4096; }
     bool split_producer_ok() const {
-        return !dense && !plan && size > 0 && et_linear_bsr16_resid_stats_f32_supported(size, (int)in_size, (int)out_size) == 1;
+        return !dense && !plan && size > 0 && split_pays((int)in_size, size) && et_linear_bsr16_resid_stats_f32_supported(size, (int)in_size, (int)out_size) == 1;
     }
     bool split_consumer_ok() const {
-        return !dense && !plan && size > 0 && et_norm_linear_bsr16_f32in_supported(size, (int)in_size, (int)out_size) == 1;
+        return !dense && !plan && size > 0 && split_pays((int)in_size, size) && et_norm_linear_bsr16_f32in_supported(size, (int)in_size, (int)out_size) == 1;
     }
     // Packs for the two roles (called once, outside any stream capture; a shape the packed kernel does
     // not take keeps the unpacked one)

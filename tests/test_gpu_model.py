@@ -392,17 +392,29 @@ def test_random_stacks(et, H, nh, FF, S, B, nlayer, sp, mode, padded, causal, se
 
 
 @pytest.mark.parametrize("mixed", [False, True])
-def test_layer_at_4096_rows_uses_the_streaming_linear(et, mixed):
-    """32 sequences of 128 tokens: the FFN down-projection (3072 inputs, 4096 token rows) runs on the
-    planned streaming kernel inside the class layer; binary16 and binary32 results of it."""
-    H, nh, FF, S, B = 768, 12, 3072, 128, 32
+@pytest.mark.parametrize("FF", [3072, 4240])
+def test_layer_at_4096_rows_uses_the_streaming_linear(et, mixed, FF):
+    """32 sequences of 128 tokens: the FFN down-projection runs on the planned streaming kernel (4240 inputs) or on strips in
+    halves (3072; with binary16 residuals that stack is token-local) inside the class layer; binary16 and binary32 results."""
+    H, nh, S, B = 768, 12, 128, 32
     layers = [Hn.LayerWeights(H, nh, FF, 0.8, seed=400)]
-    m = Hn.build_model(et, layers, S, B, mixed=mixed)
+    m = Hn.build_model(et, layers, S, B, mixed=2 if mixed else 0)
     x = Hn.randn((B * S, H), 401)
     got = run_model(et, m, x, reps=2)
     want = Hn.oracle_stack(x, layers, B, store=torch.float16, resid=torch.float32 if mixed else "same")
     assert Hn.max_abs(got[0], want) <= 4e-3
     assert np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("rows,FF,launches", [(4080, 3072, 5), (4096, 3072, 7), (4096, 3056, 5)])
+def test_wide_inputs_at_many_rows_keep_their_normalisation_apart(et, rows, FF, launches):
+    """SkipLayerNorm folded into the projections (mixed = 5), and not where it measured slower."""
+    layers = [Hn.LayerWeights(768, 12, FF, 0.9, seed=405)]
+    m = Hn.build_model(et, layers, 16, rows // 16, mixed=5)
+    assert m.launches_per_layer() == launches
+    x = Hn.randn((rows, 768), 406)
+    want = Hn.oracle_stack(x, layers, rows // 16, store=torch.float16, resid=torch.float32)
+    assert Hn.max_abs(run_model(et, m, x)[0], want) <= 4e-3
 
 
 @pytest.mark.parametrize("mode", [0, 1, 2])
