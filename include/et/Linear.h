@@ -186,7 +186,12 @@ template <> class Linear<tile_mat> {
         void operator()(et_bsr_plan_s *p) const { (void)et_bsr16_plan_destroy(p); }
     };
     std::unique_ptr<et_bsr_plan_s, PlanDeleter> plan;
-    static bool wants_plan(int in, int rows) { return in >= 128 && (in > 5112 || (in > 4224 && rows >= 4096)); }
+    // Outputs under 12 block-rows are not staged in halves: plain call over plan at 50 / 80 % sparsity, 3072 -> 128 0.99 / 0.82 at 16384
+    // rows, 1.45 / 1.11 at 32768, 4096 -> 64 1.02 / 0.75 and 1.53 / 1.12, 4096 -> 176 1.49 / 1.01 and 2.1 / 1.36 (12288 rows 1.20 / 0.80).
+    static bool wants_plan(int in, int out, int rows, int ntile) {
+        return in >= 128 && (in > 5112 || (in > 4224 && rows >= 4096) ||
+                             (in >= 3072 && out < 192 && (rows >= 24576 || (out > 128 && rows >= 12288 && ntile * 256.0 >= 0.4 * in * out))));
+    }
     // Copies of the weight in the order one launch of the packed kernel reads it (et_bsr16_pack_create),
     // held where that kernel applies — up to kPackMaxRows token rows, inputs that are multiples of 128
     // up to 4096: a launch whose loads are all issued at its start, with no row-pointer round trip.
@@ -463,7 +468,7 @@ template <> class Linear<tile_mat> {
             etChk(et_device_sync());
             return;
         }
-        if (size > 0 && size % 16 == 0 && wants_plan((int)in_size, size)) {
+        if (size > 0 && size % 16 == 0 && wants_plan((int)in_size, (int)out_size, size, weight.num_blk)) {
             et_bsr_plan p = nullptr;
             etChk(et_bsr16_plan_create(weight.row_ptr.get(), weight.row_offset.get(), et::f16(weight.data.get()), size,
                                        (int)in_size, (int)out_size, 0, 0, 0, &p));

@@ -144,7 +144,8 @@ class Bench:
             kept = ntile * 256.0 / (n_in * n_out)
             if kept > 0.5:
                 entry = "dense image"
-            elif n_in >= 128 and (n_in > 5112 or (n_in > 4224 and T >= 4096)):
+            elif n_in >= 128 and (n_in > 5112 or (n_in > 4224 and T >= 4096) or
+                                  (n_in >= 3072 and n_out < 192 and (T >= 24576 or (n_out > 128 and T >= 12288 and kept >= 0.4)))):
                 entry = "plan"
             elif T >= 2048 and n_in % 128 == 0 and n_in <= 1536:
                 entry = "row loop"  # falls back below when its launch would not fill the chip
