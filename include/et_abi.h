@@ -929,10 +929,10 @@ int et_model_forward(et_model m, et_f16 *out, const et_f16 *in, et_stream stream
 int et_model_forward_layer(et_model m, int layer, et_f16 *out, const et_f16 *in,
                            et_stream stream);
 int et_model_sync(et_model m);
-/* kernel launches per encoder layer, at most, of a finalized model in the form et_model_forward runs
- * (2: attention and one token-local launch, et_encoder_layer_f32, or, under mixed = 3, one chain
- * launch; 3: attention and a token-local launch whose strips several workgroups share, in two parts, or in
- * one where the device deals workgroups so that they can meet, et_encoder_layer_joins; 4: the QKV projection inside the
+/* kernel launches per encoder layer of a finalized model in the form et_model_forward runs
+ * (2: attention and one token-local launch, et_encoder_layer_f32 or, where several workgroups share a strip and the device
+ * deals them so that they can meet, et_encoder_layer_joined_f32, or, under mixed = 3, one chain
+ * launch; 3: attention and a token-local launch in two parts, where they cannot meet; 4: the QKV projection inside the
  * attention kernel; 5: SkipLayerNorm folded into the projections; 7: SkipLayerNorm on its own; 0 before
  * et_model_finalize).  A model asked for mixed = 3 reports 5 once it has gone back to separate
  * launches. */

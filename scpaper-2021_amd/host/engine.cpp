@@ -349,7 +349,7 @@ struct LocalPlan {
 //   144 to 192: to 23 us 1.01 - 1.29;  128: to 11 us 1.00 - 1.06, above 0.69 - 0.98;  112: to 14.6 us 1.03 - 1.14, above 0.77 - 0.90
 //   fewer: half 1.03 - 1.39, denser to 15 us 1.03 - 1.17, above 0.84 - 1.00
 // Stacks of fewer than six layers keep the lines that were drawn when a shared strip took two launches (`former` is the estimate of
-// that), so that the form a short stack takes, which et_model_launches_per_layer reports, stays what it was; past them the one
+// that), so that the form a short stack takes stays what it was; past them the one
 // launch would gain less there than in deep stacks (768 wide at 80 %, 128 rows: two layers 63.1 / 60.8 us, twelve 333.8 / 313.3).
 LocalPlan plan_local(const et_model_s &m, bool fused) {
     LocalPlan p;
@@ -848,7 +848,7 @@ int et_model_launches_per_layer(et_model m, int *launches) {
     return guarded([&]() -> int {
         et::require(m != nullptr && launches != nullptr, "et_model_launches_per_layer: NULL argument");
         if (!m->finalized) *launches = 0;
-        else if (!m->local.empty()) *launches = m->local_shares.empty() ? 2 : 3;
+        else if (!m->local.empty()) *launches = m->local_shares.empty() || !m->local_join.empty() ? 2 : 3;
         else *launches = m->chain ? 2 : m->fused_qkv ? 4 : m->split ? 5 : 7;
         return ET_OK;
     });

@@ -111,7 +111,7 @@ def test_stacks_on_token_local_launches(et, H, nh, FF, S, B, sparsity, mixed):
     outs = []
     for use_graph in (True, False):
         m = Hn.build_model(et, layers, S, B, lens=lens, mixed=mixed, use_graph=use_graph)
-        assert m.launches_per_layer() in (2, 3)  # attention, and the token-local part in one launch or two
+        assert m.launches_per_layer() == 2  # attention, and the token-local part in one launch, whether or not strips are shared
         d = et.DeviceBuffer.from_numpy(x)
         o = et.DeviceBuffer.empty(x.shape, np.float16)
         m.forward(o, d)
