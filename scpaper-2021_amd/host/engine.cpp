@@ -332,26 +332,39 @@ struct LocalPlan {
 // 95 % sparsity, 128 to 2048 rows, shared strips in one launch): the number of parts that makes the sum least, while there is a
 // compute unit for every workgroup of an XCD; beyond eight the shares cost more than they save (128 rows at 60 %, four layers:
 // 134 us with 8, 144 with 12).  Above 256 strips of 16 rows a workgroup takes 32.
-// Which stacks run it: time of the separate launches over that of these, four-layer stacks 512, 768 and 1024 wide, 20 to 95 %
-// sparsity; "half" is at most half of the tiles kept (denser layers run dense GEMMs beside), us the estimate above.
-//   above 4096 rows                       1.04 - 2.0; mixed = 0 up to 18 KiB of tiles a feature 1.07 - 1.98, 1024 wide unpruned (24) 0.78
-//   more than 16.5 KiB of tiles a feature 0.71 - 0.98
+// Which stacks run it: time of the separate launches over that of these, stacks of two and of six layers (whose ratios differ
+// by 0.05 in the mean: what the first layer's projection takes), 384 to 1024 wide with an FFN of four times the width, 512 to 800
+// with 208 to 768 hidden features, 20 to 95 % sparsity, 16 to 1024 rows, and 768 wide with the QKV projection inside the attention
+// kernel (four launches, 128 to 1024 rows: 0.93 - 1.33).  "half" is at most half of the tiles kept (denser layers run dense
+// GEMMs beside), us the estimate above; of 3036 stacks the lines take the better form or one within 3 % for all but 98, 0.3 % from
+// it on average.  On the side that takes the token-local launches, and on the other:
 //  binary32 residual:
-//   257 rows and more                     1.06 - 2.0
-//   193 to 256: half, to 18 us 1.03 - 1.39, above (1024 wide at 60 %) 0.92 - 0.95; denser, to 21 us 1.12 - 1.25, above 0.84 - 1.08
-//   144 to 192                            1.04 - 1.33
-//   112 and 128 (the separate launches have a strip for each XCD): half, to 13.5 us 1.02 - 1.14, above 0.91 - 1.05; denser, to 20.5 us
-//                                         1.03 - 1.30, above 0.75 - 0.95
-//   fewer: half 1.08 - 1.58, denser to 20.5 us 0.99 - 1.27, above 0.71 - 0.94
+//   more than 16.5 KiB of tiles a feature                                0.66 - 1.13
+//   257 rows and more                      1.01 - 1.68
+//   193 to 256: half, to 18 us             0.97 - 1.31   above           0.95 - 1.03;  denser 1.03 - 1.51
+//   144 to 192: to 32 us                   0.96 - 1.49
+//   112 and 128 (the separate launches have a strip for each XCD):
+//     half, to 13.5 us                     0.97 - 1.27   above           0.93 - 1.06
+//       FFN narrower than the model, to 6.5  1.03 - 1.26 above           0.94 - 1.14
+//     denser, to 20.5 us                   1.04 - 1.40   above           0.89 - 0.96
+//   fewer: half                            0.98 - 2.23
+//     denser, to 18.5 us                   0.95 - 1.36   above           0.77 - 1.05
 //  binary16 between layers (mixed = 0):
-//   257 rows and more: half 1.04 - 1.54; denser, to 11 KiB of tiles a feature 1.10 - 1.36, above 0.80 - 1.08
-//   256: to 12.5 us 1.02 - 1.08, above 0.81 - 0.98;  193 to 240: to 20.5 us 1.03 - 1.09, above 0.95 - 0.99
-//   144 to 192: to 23 us 1.01 - 1.29;  128: to 11 us 1.00 - 1.06, above 0.69 - 0.98;  112: to 14.6 us 1.03 - 1.14, above 0.77 - 0.90
-//   fewer: half 1.03 - 1.39, denser to 15 us 1.03 - 1.17, above 0.84 - 1.00
-// Stacks of fewer than six layers keep the lines that were drawn when a shared strip took two launches (`former` is the estimate of
-// that), so that the form a short stack takes stays what it was; past them the one
-// launch would gain less there than in deep stacks (768 wide at 80 %, 128 rows: two layers 63.1 / 60.8 us, twelve 333.8 / 313.3).
-LocalPlan plan_local(const et_model_s &m, bool fused) {
+//   above 4096 rows up to 18 KiB of tiles a feature 1.07 - 1.98, 1024 wide unpruned (24) 0.78
+//   257 rows and more: half                0.98 - 1.57
+//     denser, to 11 KiB of tiles a feature 0.95 - 1.43   above           0.74 - 1.15
+//   FFN narrower than the model: 144 to 240 rows, to 15 us 0.90 - 1.31, up to 64, to 12 us 0.93 - 1.41, others, to 6.5 us
+//                                          0.99 - 1.22;  above 0.91 - 0.97, 0.78 - 0.96, 0.81 - 1.07
+//   256: to 12.5 us                        0.93 - 1.17   above           0.84 - 1.03
+//   193 to 240: to 20.5 us                 0.93 - 1.34   above           0.89 - 1.15
+//   144 to 192: to 23 us                   0.90 - 1.39   above           0.91 - 1.06
+//   128: up to 512 wide, to 11 us          0.97 - 1.14   above           0.92 - 0.94
+//     wider, to 6.5 us                     0.93 - 1.06   above           0.69 - 1.01
+//   112: to 14.6 us                        0.85 - 1.23   above           0.70 - 0.97
+//   fewer: half                            0.94 - 2.25
+//     denser, to 13 us                     0.96 - 1.19   above           0.69 - 1.25
+//  A single layer has no projection behind it to run in the launch: at 112 and 128 rows, to 5 us 0.97 - 1.07, above 0.84 - 0.96.
+LocalPlan plan_local(const et_model_s &m) {
     LocalPlan p;
     const et_model_desc &d = m.desc;
     double kib[4] = {0, 0, 0, 0};  // of a layer, on average
@@ -367,52 +380,35 @@ LocalPlan plan_local(const et_model_s &m, bool fused) {
         if (d.mixed || kept <= 18.0 * d.emdim) p.mt = 2;
         return p;
     }
-    double best = 0, former = 0;
-    for (int parts = 1; parts <= std::min(12, d.dimFF / 16) && parts * per_xcd <= 32; parts++) {
-        const double two = (kib[ET_W_O] + shared / parts) / 112.0 + (parts > 1 ? 5.0 + 0.5 * parts : 0.0);
-        former = parts == 1 ? two : std::min(former, two);
-        if (parts > 8) continue;
+    double best = 0;
+    for (int parts = 1; parts <= std::min(8, d.dimFF / 16) && parts * per_xcd <= 32; parts++) {
         const double us = (kib[ET_W_O] + shared / parts) / 112.0 + (parts > 1 ? 0.5 + (0.45 + 0.045 * per_xcd) * parts : 0.0);
         if (parts == 1 || us < best) {
             best = us;
             p.parts = parts;
         }
     }
-    const bool half = kept <= 0.5 * all;
-    const auto short_on = [&]() -> bool {
-        const bool light = kept <= 11.0 * d.emdim;
-        if (d.mixed == 0) {
-            if (rows > 512) return half || light;
-            if (rows > 480) return half ? d.emdim <= 512 || former <= 11.0 : light;
-            if (rows > 256) return kept <= 0.45 * all || (light && (!half || d.emdim <= 512));
-            return rows == 256 && former <= 6.0;
-        }
-        if (kept > 16.5 * d.emdim) return false;
-        if (d.emdim <= 512 || rows > 512) return true;
-        if (rows > 256) return rows <= 480 || !half || former <= 14.5;
-        if (!half) return false;
-        if (strips == 7 || strips == 8) return former <= 5.0;
-        if (strips <= 3 || (strips >= 9 && strips <= 12)) return former <= 19.0;
-        return former <= 14.5 && !(fused && strips > 12);
-    };
+    const bool half = kept <= 0.5 * all, narrow = d.dimFF < d.emdim;
     bool on;
-    if (m.layers.size() < 6) on = short_on();
-    else if (d.mixed == 0) {
+    if (d.mixed == 0) {
         if (strips > 16) on = half || kept <= 11.0 * d.emdim;
-        else if (strips > 6) on = best <= (strips == 16 ? 12.5 : strips > 12 ? 20.5 : strips > 8 ? 23.0 : strips == 8 ? 11.0 : 14.6);
-        else on = half || best <= 15.0;
+        else if (narrow) on = best <= (strips > 8 && strips < 16 ? 15.0 : strips <= 4 ? 12.0 : 6.5);
+        else if (strips > 8) on = best <= (strips == 16 ? 12.5 : strips > 12 ? 20.5 : 23.0);
+        else if (strips > 6) on = best <= (strips == 7 ? 14.6 : d.emdim <= 512 ? 11.0 : 6.5);
+        else on = half || best <= 13.0;
     } else if (kept > 16.5 * d.emdim) on = false;
     else if (strips > 16) on = true;
-    else if (strips > 8) on = best <= (strips <= 12 ? 32.0 : half ? 18.0 : 21.0);
-    else if (strips > 6) on = best <= (half ? 13.5 : 20.5);
-    else on = half || best <= 20.5;
+    else if (strips > 8) on = best <= (strips > 12 && half ? 18.0 : 32.0);
+    else if (strips > 6) on = best <= (!half ? 20.5 : narrow ? 6.5 : 13.5);
+    else on = half || best <= 18.5;
+    if (m.host.size() == 1 && (strips == 7 || strips == 8)) on = on && best <= 5.0;
     p.mt = on ? 1 : 0;
     return p;
 }
 
-// The packs of the token-local launches (`fused` as plan_local takes it); leaves m.local empty where a layer has no such form.
-void build_local(et_model_s &m, bool fused) {
-    const LocalPlan plan = plan_local(m, fused);
+// The packs of the token-local launches; leaves m.local empty where a layer has no such form.
+void build_local(et_model_s &m) {
+    const LocalPlan plan = plan_local(m);
     const et_model_desc &d = m.desc;
     const int n = (int)m.layers.size(), ldq = 2 * d.kdim + d.vdim;
     if (plan.mt == 0 || d.kdim != d.emdim || d.vdim != d.emdim || et_encoder_layer_supported(m.rows(), d.emdim, d.dimFF, ldq) != 1) return;
@@ -742,7 +738,7 @@ int et_model_finalize(et_model m) {
         const long heads = (long)d.batch * d.nhead;
         const bool want_fused = (d.mixed == 4 || (d.mixed == 1 && heads >= 96 && heads <= 400)) && m->layers.size() > 1;
         const bool fused_ok = want_fused && et_norm_qkv_mha_f32in_supported(d.batch, d.seq_len, d.emdim, d.nhead, d.kdim / d.nhead) == 1;
-        if (d.mixed == 0 || d.mixed == 1 || (d.mixed == 4 && !fused_ok)) build_local(*m, fused_ok);
+        if (d.mixed == 0 || d.mixed == 1 || (d.mixed == 4 && !fused_ok)) build_local(*m);
         if (m->desc.mixed) {
             for (auto &b : m->pp32) b = std::make_unique<et::DeviceBuffer<float>>(act_elems);
             for (auto &l : m->layers) l->enable_mixed();

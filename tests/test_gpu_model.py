@@ -73,11 +73,11 @@ def test_layer_by_layer_equals_stack(et):
 
 
 @pytest.mark.parametrize("H,nh,FF,S,B,launches", [(384, 6, 1536, 176, 3, 2), (256, 4, 512, 64, 5, 2), (256, 4, 512, 128, 33, 2),
-                                                  (768, 12, 512, 112, 2, 7)])
+                                                  (768, 12, 512, 128, 1, 7)])
 def test_layer_by_layer_equals_stack_in_every_form(et, H, nh, FF, S, B, launches):
     """All activations binary16 (mixed = 0): the stack and a chain of et_model_forward_layer agree bit for bit on the
     token-local launches too, shared strips (528 rows), one workgroup a strip (320) and 32-row strips (4224), as on the
-    separate ones (224), and stay near the storage the mode promises."""
+    separate ones (128), and stay near the storage the mode promises."""
     layers = [Hn.LayerWeights(H, nh, FF, 0.7, seed=45 + i) for i in range(3)]
     m = Hn.build_model(et, layers, S, B, act=1)
     assert m.launches_per_layer() == launches
@@ -91,7 +91,7 @@ def test_layer_by_layer_equals_stack_in_every_form(et, H, nh, FF, S, B, launches
     assert Hn.max_abs(full, Hn.oracle_stack(x, layers, B, act="relu")) <= TOL_F16
 
 
-@pytest.mark.parametrize("H,nh,FF,S,B,launches", [(384, 6, 1536, 176, 3, 2), (256, 4, 512, 64, 5, 2), (256, 4, 512, 32, 2, 7)])
+@pytest.mark.parametrize("H,nh,FF,S,B,launches", [(384, 6, 1536, 176, 3, 2), (256, 4, 512, 64, 5, 2), (768, 12, 512, 32, 4, 7)])
 def test_layers_of_one_model_on_streams_of_their_own(et, H, nh, FF, S, B, launches):
     """mixed = 0: a layer touches no buffer of another one, so two batches can go through a model one layer apart, each on
     its stream; addresses off the launches' alignment included."""
@@ -206,32 +206,78 @@ def test_qkv_inside_attention_chosen_by_batch(et):
         assert Hn.max_abs(got, want) <= 4e-3
 
 
-@pytest.mark.parametrize("H,sparsity,B,S,launches", [
-    (768, 0.6, 3, 16, 2), (768, 0.8, 1, 64, 2), (768, 0.6, 1, 64, 5), (768, 0.8, 1, 112, 5), (768, 0.8, 1, 128, 5), (768, 0.6, 1, 144, 2),
-    (768, 0.8, 2, 128, 2), (768, 0.8, 8, 32, 4), (768, 0.6, 1, 240, 5), (768, 0.6, 1, 272, 2), (768, 0.6, 4, 128, 5), (768, 0.4, 4, 128, 2),
-    (768, 0.4, 2, 128, 7), (1024, 0.8, 4, 128, 5), (1024, 0.9, 4, 128, 2), (768, 0.0, 4, 144, 7), (1024, 0.2, 4, 144, 7), (512, 0.0, 2, 64, 2)])
-def test_token_local_form_chosen_by_rows_and_tiles(et, H, sparsity, B, S, launches):
-    """Both sides of every line mixed = 1 draws between the token-local launches and the separate ones (rows, strips for
-    each XCD, tiles kept), by the launches a layer has; the result is the oracle's in either form."""
-    layers = [Hn.LayerWeights(H, H // 64, 4 * H, sparsity, seed=960 + i) for i in range(2)]
-    m = Hn.build_model(et, layers, S, B, mixed=1)
+# (H, sparsity, B, S, launches of the separate form) on both sides of every line the engine draws between the token-local launches
+# (2 a layer: strips one workgroup has to itself, and shared ones, whose workgroups meet) and the separate ones: rows, strips
+# for each XCD, tiles kept.
+FORMS_MIXED = [
+    (768, 0.4, 1, 48, 7), (768, 0.5, 1, 48, 2), (768, 0.8, 1, 64, 2), (512, 0.0, 2, 64, 2),                            # fewer than 112 rows
+    (768, 0.6, 1, 112, 5), (768, 0.8, 1, 112, 2), (768, 0.3, 1, 128, 7), (768, 0.4, 1, 128, 2), (768, 0.8, 1, 128, 2),  # 112 and 128
+    (1024, 0.7, 1, 128, 5), (1024, 0.8, 1, 128, 2),
+    (768, 0.0, 1, 144, 7), (768, 0.6, 1, 144, 2), (1024, 0.3, 1, 144, 7), (1024, 0.4, 1, 144, 2),                      # 144 to 192
+    (768, 0.8, 2, 128, 2), (768, 0.8, 8, 32, 2), (1024, 0.6, 1, 240, 5), (1024, 0.7, 1, 240, 2), (768, 0.4, 2, 128, 2),  # 193 to 256
+    (768, 0.6, 1, 272, 2), (768, 0.6, 4, 128, 2), (1024, 0.9, 4, 128, 2), (768, 0.0, 4, 144, 7), (1024, 0.2, 4, 144, 7)]
+FORMS_BINARY16 = [
+    (512, 0.2, 1, 48, 7), (512, 0.4, 1, 48, 2), (768, 0.4, 1, 64, 7), (768, 0.8, 1, 64, 2),
+    (768, 0.5, 1, 112, 7), (768, 0.6, 1, 112, 2), (768, 0.8, 1, 128, 7), (768, 0.9, 1, 128, 2), (512, 0.4, 1, 128, 2),
+    (768, 0.2, 1, 144, 7), (768, 0.4, 1, 192, 2), (768, 0.2, 1, 240, 7), (768, 0.4, 1, 240, 2),
+    (768, 0.6, 2, 128, 7), (768, 0.8, 2, 128, 2), (256, 0.8, 2, 128, 2),
+    (768, 0.8, 1, 272, 2), (768, 0.4, 1, 496, 2), (768, 0.4, 3, 176, 2), (768, 0.2, 3, 176, 7), (768, 0.6, 3, 176, 2)]
+
+
+def check_form(et, H, sparsity, B, S, launches, nlayer, mixed, FF=0):
+    layers = [Hn.LayerWeights(H, H // 64 if FF == 0 else 4, FF or 4 * H, sparsity, seed=960 + i) for i in range(nlayer)]
+    m = Hn.build_model(et, layers, S, B, mixed=mixed)
     assert m.launches_per_layer() == launches
     x = Hn.randn((B * S, H), 969)
+    got = run_model(et, m, x, reps=2)
+    assert np.array_equal(got[0], got[1])
+    return got[0], x, layers
+
+
+@pytest.mark.parametrize("H,sparsity,B,S,launches", FORMS_MIXED)
+def test_token_local_form_chosen_by_rows_and_tiles(et, H, sparsity, B, S, launches):
+    """mixed = 1, by the launches a layer has; the result is the oracle's in either form."""
+    got, x, layers = check_form(et, H, sparsity, B, S, launches, 2, 1)
     want = Hn.oracle_stack(x, layers, B, store=torch.float16, resid=torch.float32)
-    assert Hn.max_abs(run_model(et, m, x)[0], want) <= 4e-3
+    assert Hn.max_abs(got, want) <= 4e-3
 
 
-@pytest.mark.parametrize("H,sparsity,B,S,launches", [
-    (768, 0.8, 2, 128, 7), (256, 0.8, 2, 128, 2), (256, 0.8, 1, 240, 7), (768, 0.8, 1, 272, 2), (768, 0.8, 1, 496, 7), (768, 0.95, 1, 496, 2),
-    (768, 0.4, 1, 496, 2), (512, 0.6, 1, 496, 2), (768, 0.4, 3, 176, 2),
-    (768, 0.2, 3, 176, 7), (768, 0.6, 3, 176, 2)])
+@pytest.mark.parametrize("H,sparsity,B,S,launches", FORMS_BINARY16)
 def test_token_local_form_chosen_under_all_binary16(et, H, sparsity, B, S, launches):
     """The same for mixed = 0, whose lines lie elsewhere."""
-    layers = [Hn.LayerWeights(H, H // 64, 4 * H, sparsity, seed=970 + i) for i in range(2)]
-    m = Hn.build_model(et, layers, S, B)
-    assert m.launches_per_layer() == launches
-    x = Hn.randn((B * S, H), 979)
-    assert Hn.max_abs(run_model(et, m, x)[0], Hn.oracle_stack(x, layers, B)) <= TOL_F16
+    got, x, layers = check_form(et, H, sparsity, B, S, launches, 2, 0)
+    assert Hn.max_abs(got, Hn.oracle_stack(x, layers, B)) <= TOL_F16
+
+
+@pytest.mark.parametrize("sparsity,S,mixed,launches", [(0.6, 112, 1, 5), (0.95, 112, 1, 2), (0.4, 64, 0, 7), (0.6, 64, 0, 2), (0.6, 112, 0, 7),
+                                                       (0.95, 112, 0, 2), (0.6, 144, 0, 2), (0.6, 64, 1, 2)])
+def test_token_local_form_with_a_narrow_ffn(et, sparsity, S, mixed, launches):
+    """The lines of an FFN narrower than the model: 800 wide, four heads of 200, 208 hidden features."""
+    got, x, layers = check_form(et, 800, sparsity, 1, S, launches, 2, mixed, FF=208)
+    want = Hn.oracle_stack(x, layers, 1, store=torch.float16, resid=torch.float32 if mixed else "same")
+    assert Hn.max_abs(got, want) <= (4e-3 if mixed else TOL_F16)
+
+
+@pytest.mark.parametrize("sparsity,mixed,launches", [(0.8, 1, 5), (0.95, 1, 2), (0.8, 0, 7), (0.95, 0, 2)])
+def test_token_local_form_of_a_single_layer(et, sparsity, mixed, launches):
+    """112 rows of one layer, which has no projection behind it."""
+    got, x, layers = check_form(et, 768, sparsity, 1, 112, launches, 1, mixed)
+    want = Hn.oracle_stack(x, layers, 1, store=torch.float16, resid=torch.float32 if mixed else "same")
+    assert Hn.max_abs(got, want) <= 4e-3
+
+
+@pytest.mark.parametrize("case", [c for c in FORMS_MIXED if c[2] * c[3] <= 256 and c[0] >= 768])
+def test_token_local_form_of_six_layers(et, case):
+    """The form follows from rows and tiles: six layers run what two run, as near to the oracle as 12 are held."""
+    got, x, layers = check_form(et, *case, 6, 1)
+    want = Hn.oracle_stack(x, layers, case[2], store=torch.float16, resid=torch.float32)
+    assert Hn.max_abs(got, want) <= TOL_MIXED_VS_ORACLE
+
+
+@pytest.mark.parametrize("case", [c for c in FORMS_BINARY16 if c[2] * c[3] <= 256])
+def test_token_local_form_of_six_layers_under_all_binary16(et, case):
+    got, x, layers = check_form(et, *case, 6, 0)
+    assert Hn.max_abs(got, Hn.oracle_stack(x, layers, case[2])) <= TOL_F16_DEEP
 
 
 def test_qkv_inside_attention_falls_back(et):
