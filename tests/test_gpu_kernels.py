@@ -280,10 +280,11 @@ def test_linear_bsr16_f32_output(et, T, inp, out, sp, act):
 
 # Strips of 32 rows staged a half of the columns at a time: the smallest and the largest width, an odd number of column tiles, a last
 # strip of 16 rows, one block-row a wave to four and waves with fewer, block-rows without tiles, with tiles in one
-# half only, with all of them, and (ids drawn twice) with more tiles than columns; columns in any order.
+# half only, with all of them, and (ids drawn twice) with more tiles than columns; columns in any order.  "crowded": rows of no more tiles
+# than columns, but more in one half than it has columns, in turn with ordinary rows of the same wave.
 @pytest.mark.parametrize("T,inp,out,act", [(2048, 1280, 768, 0), (2064, 3072, 816, 2), (2064, 2000, 800, 1), (8208, 3056, 208, 0),
                                            (8192, 4096, 400, 0), (16400, 1296, 800, 2)])
-@pytest.mark.parametrize("order", ["rising", "falling", "drawn", "twice"])
+@pytest.mark.parametrize("order", ["rising", "falling", "drawn", "twice", "crowded"])
 def test_linear_bsr16_strip_halves(et, T, inp, out, act, order):
     rng = np.random.default_rng(inp + out)
     nc, rows = inp // 16, []
@@ -293,6 +294,9 @@ def test_linear_bsr16_strip_halves(et, T, inp, out, act, order):
         ids = rng.permutation(np.arange(lo, hi))[:n]
         if order == "twice" and b % 3 == 0:
             ids = rng.integers(0, nc, nc + 1 + int(rng.integers(0, 70)))
+        if order == "crowded" and (b // 12 + b) % 2 == 0:
+            lo, hi = ((0, (nc + 1) // 2), ((nc + 1) // 2, nc))[b // 2 % 2]
+            ids = rng.integers(lo, hi, int(rng.integers((nc + 1) // 2 + 1, nc + 1)))
         rows.append({"rising": np.sort(ids), "falling": -np.sort(-ids)}.get(order, ids))
     row_ptr = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
     col_idx = np.concatenate(rows).astype(np.int32)
