@@ -286,9 +286,9 @@ template <> class Linear<tile_mat> {
                                              size, act, stream));
             return;
         }
-        etChk(et_linear_bsr16_f16(weight.row_ptr.get(), weight.row_offset.get(), et::f16(weight.data.get()),
-                                  et::f16(bias.get()), et::f16(input), et::f16(output), size, (int)in_size,
-                                  (int)out_size, act, stream));
+        etChk(et_linear_bsr16_counted_f16(weight.row_ptr.get(), weight.row_offset.get(), et::f16(weight.data.get()), weight.num_blk,
+                                          et::f16(bias.get()), et::f16(input), et::f16(output), size, (int)in_size,
+                                          (int)out_size, act, stream));
     }
     // binary32 result (fp16 operands, fp32 accumulator stored unrounded): what the
     // mixed-precision encoder layer adds to its fp32 residual stream
@@ -313,9 +313,9 @@ template <> class Linear<tile_mat> {
                                              ET_ACT_NONE, stream));
             return;
         }
-        etChk(et_linear_bsr16_f16_f32out(weight.row_ptr.get(), weight.row_offset.get(), et::f16(weight.data.get()),
-                                         et::f16(bias.get()), et::f16(input), output, size, (int)in_size,
-                                         (int)out_size, ET_ACT_NONE, stream));
+        etChk(et_linear_bsr16_counted_f16_f32out(weight.row_ptr.get(), weight.row_offset.get(), et::f16(weight.data.get()),
+                                                 weight.num_blk, et::f16(bias.get()), et::f16(input), output, size, (int)in_size,
+                                                 (int)out_size, ET_ACT_NONE, stream));
     }
     // The split normalisation of the mixed-precision layer (et_linear_bsr16_resid_stats_f32 /
     // et_norm_linear_bsr16_f32in): this Linear as the producer of a binary32 sum with its row

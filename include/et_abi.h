@@ -129,6 +129,14 @@ int et_linear_bsr16_f16(const int32_t *row_ptr, const int32_t *col_idx,
                         const et_f16 *X, et_f16 *Y, int T, int in, int out,
                         int act, et_stream stream);
 
+/* The same with the number of tiles (row_ptr[out / 16] - row_ptr[0], which only the device knows otherwise), by which the form for
+ * wide inputs at many rows is chosen; negative: not known, as in the call above.  Same results up to the order of the
+ * fp32 accumulation. */
+int et_linear_bsr16_counted_f16(const int32_t *row_ptr, const int32_t *col_idx,
+                                const et_f16 *tiles, int ntile, const et_f16 *bias,
+                                const et_f16 *X, et_f16 *Y, int T, int in, int out,
+                                int act, et_stream stream);
+
 /* et_linear_bsr16_f16 with the result stored as binary32 [T x out]: the fp32
  * accumulator after bias and activation, unrounded (Y 16-byte aligned).  The
  * projections that feed a SkipLayerNorm use it in the mixed-precision layer
@@ -139,6 +147,10 @@ int et_linear_bsr16_f16_f32out(const int32_t *row_ptr, const int32_t *col_idx,
                                const et_f16 *tiles, const et_f16 *bias,
                                const et_f16 *X, float *Y, int T, int in, int out,
                                int act, et_stream stream);
+int et_linear_bsr16_counted_f16_f32out(const int32_t *row_ptr, const int32_t *col_idx,
+                                       const et_f16 *tiles, int ntile, const et_f16 *bias,
+                                       const et_f16 *X, float *Y, int T, int in, int out,
+                                       int act, et_stream stream);
 
 /* Tile-sparse Linear through a plan.  et_bsr16_plan_create re-orders the weight
  * once (device pointers in the reference layout in, a device-side copy grouped by

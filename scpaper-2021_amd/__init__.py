@@ -66,6 +66,8 @@ _SIGNATURES = {
     "et_event_elapsed_ms": (C.POINTER(_f), _vp, _vp),
     "et_linear_bsr16_f16": (_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp),
     "et_linear_bsr16_f16_f32out": (_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp),
+    "et_linear_bsr16_counted_f16": (_vp, _vp, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _i, _vp),
+    "et_linear_bsr16_counted_f16_f32out": (_vp, _vp, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _i, _vp),
     "et_skip_layernorm_mixed": (_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _f, _vp),
     "et_bsr16_plan_create": (_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, C.POINTER(_vp)),
     "et_bsr16_plan_destroy": (_vp,),

@@ -985,7 +985,7 @@ static BsrPlan plan_bsr(int T, int in, int out) {
     p.threads = (rpw <= 6 || rpw == 18) ? 384 : 512;
     // 16-row strips (inputs too wide for 32 rows) with 24 to 48 block-rows per workgroup: 12 waves of
     // two to four rows instead of 8 waves of three to six, two row groups in flight per wave
-    // (2048 x 3072 -> 768: 13.6 -> 11.6 us, 16384 rows: 103 -> 87 us).  With fewer rows per
+    // (where these are not staged in halves, plan_halves; before they were, 2048 x 3072 -> 768 at 80 % 13.6 -> 11.6 us).  With fewer rows per
     // workgroup the 8-wave form, which keeps four row groups in flight, is the faster one, and so it
     // is on 32-row strips.
     if (p.mt == 1 && rpw >= 24 && rpw <= 48) p.threads = 768;
@@ -1196,12 +1196,12 @@ static int launch_bsr_halves(const BsrArgs &args, int rows_per_wg, hipStream_t s
     return check_launch("bsr16_linear_halves_kernel");
 }
 
-// Block-rows of a workgroup of the halves form, 0 where another form is the faster one.
-static int plan_halves(int T, int in, int out) {
+// Block-rows of a workgroup of the halves form, 0 where another form is the faster one.  ntile: tiles of the weight, negative
+// where the caller does not know.
+static int plan_halves(int T, int in, int out, int ntile) {
     // A list costs a wave a round trip to the columns before the first weights, and the second half another: the fewer
-    // tiles a workgroup has, the less there is to win them back.  16-row strips against halves, us: 2048 x 3072 -> 768 at 80 % 11.5 / 9.1,
-    // 2560 at 90 % 12.2 / 9.3, 2048 x 4096 -> 1024 at 50 % 39 / 24, 4096 x 4096 -> 1024 at 90 % 25.3 / 24.2, 8192 x 3072 -> 768 at
-    // 95 % 21.1 / 20.4, but 4096 at 95 % 9.9 / 11.1, 2048 at 95 % 6.6 / 7.5 (the number of tiles is not known on the host); fewer
+    // tiles a workgroup has, the less there is to win them back.  16-row strips against halves, us: 2048 x 3072 -> 768 at 80 % 10.9 / 8.8,
+    // 2560 at 90 % 11.9 / 9.5, 2048 x 4096 -> 1024 at 50 % 35 / 23, 8192 x 3072 -> 768 at 95 % 20.5 / 19.8; fewer
     // than a block-row a wave 2048 x 4096 -> 256 9.5 / 9.8, 4096 x 3072 -> 96 7.3 / 8.4.
     const size_t lds_cap = 160 * 1024;
     if ((size_t)32 * (in + kLdsPad) * sizeof(_Float16) <= lds_cap / 2) return 0;  // 32 rows in one piece
@@ -1212,7 +1212,24 @@ static int plan_halves(int T, int in, int out) {
     int groups = strips >= 256 ? 1 : 256 / strips;
     groups = std::max(groups, (nbr + most - 1) / most);
     const int rows = (nbr + groups - 1) / groups;
-    return rows >= kHalfWaves ? rows : 0;
+    if (rows < kHalfWaves) return 0;
+    // Few tiles: 16-row strips / halves, us, 4096 x 3072 -> 768 at 90 / 95 / 98 % 12.7 / 11.3, 9.05 / 10.1, 7.8 / 9.5, 3072 x 4096 -> 1024
+    // 22.0 / 21.2, 15.0 / 18.7, 11.4 / 17.3.  The estimate of both is rounds of workgroups over the compute units, a fixed part and the
+    // tiles of each, and what twice the rows of X cost once more; fitted to 307 calls of 2048 to 16384 rows, inputs of 1536 to 4096
+    // at 50 to 98 %, whose better form it takes but for 18 (3 to 23 % lost), 0.5 % from it on average; halves always 4.4 %.
+    // Without the count a call takes halves: up to 90 % they are the faster form but for 6 of the 140 (3072 x 2048 -> 2048 at 90 % 22.3 / 25.2).
+    // (Counting on the device, by the row pointers' ends, was 0.45 us of every call in halves, 3 to 5 %; asking for lines of
+    // X meanwhile, 0.8.)
+    if (ntile >= 0) {
+        const auto rounds = [](int wgs) { return (wgs + 255) / 256; };
+        const BsrPlan p = plan_bsr(T, in, out);
+        const double per_row = (double)ntile / nbr;
+        const int wgs16 = (T + 15) / 16 * ((nbr + p.rows_per_wg - 1) / p.rows_per_wg), wgs32 = strips * ((nbr + rows - 1) / rows);
+        const double us16 = 0.5 + rounds(wgs16) * (3.9 + 0.010 * per_row * p.rows_per_wg);
+        const double us32 = rounds(wgs32) * (7.2 + 0.0067 * per_row * rows) + 0.04e-6 * T * in;
+        if (us16 < us32) return 0;
+    }
+    return rows;
 }
 
 static int dispatch_bsr(const BsrArgs &args, const BsrPlan &p, hipStream_t stream) {
@@ -1233,8 +1250,8 @@ static int dispatch_bsr(const BsrArgs &args, const BsrPlan &p, hipStream_t strea
     }
 }
 
-static int launch_bsr_plain(BsrArgs args, hipStream_t stream) {
-    const int rows = plan_halves(args.T, args.in, args.out);
+static int launch_bsr_plain(BsrArgs args, int ntile, hipStream_t stream) {
+    const int rows = plan_halves(args.T, args.in, args.out, ntile);
     if (rows && ((reinterpret_cast<uintptr_t>(args.X) | reinterpret_cast<uintptr_t>(args.tiles)) & 15) == 0) {  // pieces of 16 bytes
         args.rows_per_wg = rows;
         switch (args.act) {
@@ -1267,30 +1284,35 @@ static int bsr_check(const int32_t *row_ptr, const int32_t *col_idx, const et_f1
 
 extern "C" {
 
-int et_linear_bsr16_f16(const int32_t *row_ptr, const int32_t *col_idx, const et_f16 *tiles,
-                        const et_f16 *bias, const et_f16 *X, et_f16 *Y, int T, int in, int out,
-                        int act, et_stream stream) {
+int et_linear_bsr16_counted_f16(const int32_t *row_ptr, const int32_t *col_idx, const et_f16 *tiles, int ntile,
+                                const et_f16 *bias, const et_f16 *X, et_f16 *Y, int T, int in, int out,
+                                int act, et_stream stream) {
     int s = bsr_check(row_ptr, col_idx, tiles, X, Y, T, in, out, act);
     if (s != ET_OK) return s;
     if (T == 0) return ET_OK;
-    BsrArgs args{row_ptr,
-                 col_idx,
-                 reinterpret_cast<const _Float16 *>(tiles),
-                 reinterpret_cast<const _Float16 *>(bias),
-                 reinterpret_cast<const _Float16 *>(X),
-                 reinterpret_cast<_Float16 *>(Y),
-                 T,
-                 in,
-                 out,
-                 0,
-                 act,
-                 nullptr, nullptr, nullptr, nullptr, nullptr, 0.0f, nullptr, 0, nullptr, nullptr};
-    return launch_bsr_plain(args, as_stream(stream));
+    BsrArgs args{};
+    args.row_ptr = row_ptr;
+    args.col_idx = col_idx;
+    args.tiles = reinterpret_cast<const _Float16 *>(tiles);
+    args.bias = reinterpret_cast<const _Float16 *>(bias);
+    args.X = reinterpret_cast<const _Float16 *>(X);
+    args.Y = reinterpret_cast<_Float16 *>(Y);
+    args.T = T;
+    args.in = in;
+    args.out = out;
+    args.act = act;
+    return launch_bsr_plain(args, ntile, as_stream(stream));
 }
 
-int et_linear_bsr16_f16_f32out(const int32_t *row_ptr, const int32_t *col_idx, const et_f16 *tiles,
-                               const et_f16 *bias, const et_f16 *X, float *Y, int T, int in, int out,
-                               int act, et_stream stream) {
+int et_linear_bsr16_f16(const int32_t *row_ptr, const int32_t *col_idx, const et_f16 *tiles,
+                        const et_f16 *bias, const et_f16 *X, et_f16 *Y, int T, int in, int out,
+                        int act, et_stream stream) {
+    return et_linear_bsr16_counted_f16(row_ptr, col_idx, tiles, -1, bias, X, Y, T, in, out, act, stream);
+}
+
+int et_linear_bsr16_counted_f16_f32out(const int32_t *row_ptr, const int32_t *col_idx, const et_f16 *tiles, int ntile,
+                                       const et_f16 *bias, const et_f16 *X, float *Y, int T, int in, int out,
+                                       int act, et_stream stream) {
     int s = bsr_check(row_ptr, col_idx, tiles, X, reinterpret_cast<et_f16 *>(Y), T, in, out, act);
     if (s != ET_OK) return s;
     ET_REQUIRE((reinterpret_cast<uintptr_t>(Y) & 15) == 0, ET_ERR_UNSUPPORTED,
@@ -1307,7 +1329,13 @@ int et_linear_bsr16_f16_f32out(const int32_t *row_ptr, const int32_t *col_idx, c
     args.out = out;
     args.act = act;
     args.Y32 = Y;
-    return launch_bsr_plain(args, as_stream(stream));
+    return launch_bsr_plain(args, ntile, as_stream(stream));
+}
+
+int et_linear_bsr16_f16_f32out(const int32_t *row_ptr, const int32_t *col_idx, const et_f16 *tiles,
+                               const et_f16 *bias, const et_f16 *X, float *Y, int T, int in, int out,
+                               int act, et_stream stream) {
+    return et_linear_bsr16_counted_f16_f32out(row_ptr, col_idx, tiles, -1, bias, X, Y, T, in, out, act, stream);
 }
 
 int et_skipln_linear_bsr16_f16(const et_f16 *src, const et_f16 *skip, const et_f16 *gamma,

@@ -319,6 +319,28 @@ def test_linear_bsr16_strip_halves(et, T, inp, out, act, order):
     assert (y[T:] == 7).all() and (y32[T:] == 7).all()
 
 
+# The call that knows the number of tiles, on both sides of its line between strips of 16 rows and strips in halves (an estimate of
+# either: few tiles; one workgroup a compute unit and more; rows a workgroup deals unevenly), and with a count that is not known.
+@pytest.mark.parametrize("T,inp,out", [(2048, 3072, 768), (4096, 3072, 768), (3072, 4096, 1024), (2064, 1536, 1536), (8192, 2048, 208)])
+@pytest.mark.parametrize("sp", [0.8, 0.95, 1.0])
+@pytest.mark.parametrize("act", [0, 2])
+def test_linear_bsr16_counted(et, T, inp, out, sp, act):
+    w = Hn.BsrWeight(out, inp, sp, seed=inp + out, std=0.02, bias_std=0.1)
+    n = len(w.col_idx)
+    x = Hn.randn((T, inp), 3)
+    want = L.linear(Hn.f32(x), Hn.f32(w.dense), Hn.f32(w.bias), {0: None, 2: "gelu"}[act], None).numpy()
+    d = [up(et, v if len(v) else np.zeros(256, v.dtype)) for v in (w.row_ptr, w.col_idx, w.tiles)]
+    d_b, d_x = up(et, w.bias), up(et, x)
+    for count in (n, -1):
+        d_y, d_y32 = up(et, np.full((T + 16, out), 7, np.float16)), up(et, np.full((T + 16, out), 7, np.float32))
+        et.check(et.lib().et_linear_bsr16_counted_f16(*[v.ptr for v in d], count, d_b.ptr, d_x.ptr, d_y.ptr, T, inp, out, act, None))
+        et.check(et.lib().et_linear_bsr16_counted_f16_f32out(*[v.ptr for v in d], count, d_b.ptr, d_x.ptr, d_y32.ptr, T, inp, out, act, None))
+        y, y32 = d_y.numpy(), d_y32.numpy()
+        # as for the strips in halves: order of accumulation, and a binary16 rounding of the result on top
+        assert Hn.max_abs(y32[:T], want) <= 5e-5 and Hn.max_abs(y[:T], want) <= 1e-3 * max(1.0, float(np.abs(want).max()))
+        assert (y[T:] == 7).all() and (y32[T:] == 7).all()
+
+
 PLANNED_CASES = [
     # T, in, out, sparsity, act, (mt, kc, rows_per_wg) or None for the automatic geometry
     (1024, 768, 2304, 0.8, 0, None),
