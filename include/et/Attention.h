@@ -367,9 +367,6 @@ class Attention<_config, std::enable_if_t<_config::isSingleKernel>> : public et:
     // the two projections, the buffers between them, and the attention kernel on its own.
     linearQKV_t &qkv_linear() { return *linearQKV; }
     linearO_t &o_linear() { return *linearO; }
-    half *qkv_buffer() { return mat_qkv->get(); }
-    half *z_buffer() { return mat_z->get(); }
-    void core(et::stream_t stream = nullptr) { core(buffers(), stream); }
     void core(const Buffers &b, et::stream_t stream = nullptr) {
         const int ldm = model->kdim * 2 + model->vdim;
         half *Q = b.qkv;

@@ -328,16 +328,12 @@ template <typename attn_t, typename linear1_t, typename linear2_t, typename ACT_
             return false;
         }
     }
-    half *qkv_buffer() { return buffers().qkv; }
-    half *z_buffer() { return buffers().z; }
     float epsilon(int k) const { return k ? LN2->epsilon() : LN1->epsilon(); }
     // the first layer's QKV projection of the binary16 input, and the attention kernel alone
-    void chain_qkv_first(half *x16, stream_t stream = nullptr) { chain_qkv_first_in(buffers(), x16, stream); }
     void chain_qkv_first_in(const LayerBuffers &b, half *x16, stream_t stream = nullptr) {
         if constexpr (attn_has_split<attn_t>::value) attn->qkv_linear().forward(b.qkv, x16, stream);
         else (void)b, (void)x16, (void)stream;
     }
-    void chain_attention(stream_t stream = nullptr) { chain_attention_in(buffers(), stream); }
     void chain_attention_in(const LayerBuffers &b, stream_t stream = nullptr) {
         if constexpr (attn_has_split<attn_t>::value) attn->core({b.qkv, b.z, b.ahead, b.nahead}, stream);
         else (void)b, (void)stream;
