@@ -101,7 +101,7 @@ __device__ __forceinline__ int column_of(int die_bits) { return (int)((blockIdx.
 
 constexpr int kAhead = 4;
 constexpr int kRawBuffer = 0x00020000;   // word 3 of a resource: raw, 32-bit data
-constexpr int kPastEnd = 0x7fffff00;     // an offset past the end of any resource here
+constexpr unsigned kPastEnd = 0x7fffff00;  // an offset past the end of any resource here, also with a row's added to it (below 2^32)
 constexpr int kSplitMaxIn = 1 << 24;     // 16 rows of X lie within the offsets of a resource, and below kPastEnd
 template <int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void bsr16_linear_split_f32_kernel(const Bsr32Args a) {
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(WAVES * 64) void bsr16_linear_split_f32_kernel(cons
     const int tok = strip * 16 + r16;
     const f4 bias = bias_cell_f32(a.bias, br * 16 + 4 * q);
     const auto xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.X) + (size_t)strip * 16 * a.in, 0, 16 * a.in * 4, kRawBuffer);
-    const int xo = (min(r16, a.T - 1 - strip * 16) * a.in + 4 * q) * 4;  // rows past the end: the last one, not stored
+    const unsigned xo = (unsigned)(min(r16, a.T - 1 - strip * 16) * a.in + 4 * q) * 4;  // rows past the end: the last one, not stored
     const int wo = (r16 * 16 + 4 * q) * 4;
     f4 acc = f4{0.f, 0.f, 0.f, 0.f};
     const int ts = a.row_ptr[br] + wave, te = a.row_ptr[br + 1];
@@ -124,9 +124,9 @@ __global__ __launch_bounds__(WAVES * 64) void bsr16_linear_split_f32_kernel(cons
         const auto wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.tiles) + (size_t)t0 * 256, 0, ((here - 1) * WAVES + 1) * 1024, kRawBuffer);
         float4 w[kAhead], x[kAhead];
         auto ask = [&](int slot, int i) {
-            const int xat = i < here ? __builtin_amdgcn_readlane(cols, i & 63) * 64 : kPastEnd;
+            const unsigned xat = i < here ? (unsigned)__builtin_amdgcn_readlane(cols, i & 63) * 64 : kPastEnd;
             w[slot] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(wr, wo + i * WAVES * 1024, 0, 0));
-            x[slot] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xr, xo + xat, 0, 0));
+            x[slot] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(xo + xat), 0, 0));
         };
 #pragma unroll
         for (int s = 0; s < kAhead; s++) ask(s, s);
