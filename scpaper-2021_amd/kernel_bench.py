@@ -179,7 +179,8 @@ class Bench:
             et.check(lib.et_bsr16_to_dense_f16(d_rp.ptr, d_col.ptr, tiles.ptr, w.ptr, n_in, n_out, self.stream))
             fn = lambda: et.check(lib.et_linear_dense_f16(w.ptr, bias.ptr, x.ptr, y.ptr, T, n_in, n_out, 0, self.stream))
         if entry == "plain":
-            fn = lambda: et.linear_bsr16(d_rp, d_col, tiles, bias, x, y, T, n_in, n_out, 0, self.stream)
+            fn = lambda: et.check(lib.et_linear_bsr16_counted_f16(d_rp.ptr, d_col.ptr, tiles.ptr, ntile if label_class else -1, bias.ptr, x.ptr,
+                                                                  y.ptr, T, n_in, n_out, 0, self.stream))
         us = self.time_us(fn, launches)
         et.check(lib.et_stream_sync(self.stream))
         if destroy:
@@ -187,9 +188,10 @@ class Bench:
         self.record(f"linear_bsr16 ({entry})", f"T{T} in{n_in} out{n_out} sparsity {sparsity}", us, 2 * 256 * ntile * T, "mfma")
 
     def token_local(self, T, mt, parts, H, FF, launches, nset=12):
-        """What lies between two attention kernels of a tile-sparse layer (et_encoder_layer_f32): at 80 % sparsity, and with
-        no tile in any weight, which is what the launches cost beside them; every launch of a graph on another of `nset`
-        layers with buffers of their own."""
+        """What lies between two attention kernels of a tile-sparse layer, in one launch whose parts meet
+        (et_encoder_layer_joined_f32) and in two (et_encoder_layer_f32; one part is one launch): at 80 % sparsity, and with no
+        tile in any weight, which is what the launches cost beside them; every launch of a graph on another of `nset` layers
+        with buffers of their own."""
         et, lib = self.et, self.lib
 
         class Weights(C.Structure):
@@ -217,15 +219,21 @@ class Bench:
                 x = self.dev(self.rnd((T, H)).astype(np.float32))
                 layers.append((pack, self.dev(self.rnd((T, H))), x, et.DeviceBuffer.empty((T, H), np.float32), self.empty((T, 3 * H))))
 
-            def layer():
-                pack, z, x, out, qkv = layers[i["i"] % nset]
-                i["i"] += 1
-                et.check(lib.et_encoder_layer_f32(pack, z.ptr, x.ptr, None, out.ptr, None, qkv.ptr, partial.ptr, et.ACT_GELU, 1e-5, 1e-5,
-                                                  self.stream))
+            forms, joins = [("encoder_layer", lib.et_encoder_layer_f32, ())], C.c_int()
+            et.check(lib.et_encoder_layer_joins(layers[0][0], C.byref(joins)))
+            if joins.value:
+                words = self.dev(np.zeros(T // 16, np.int32))
+                forms.insert(0, ("encoder_layer_joined", lib.et_encoder_layer_joined_f32, (words.ptr, 4000)))
+            for name, call, join in forms:
 
-            us = self.time_us(layer, launches)
-            self.record("encoder_layer" + (" (no tiles)" if sparsity == 1.0 else ""), f"T{T} {H} wide FFN {FF} {16 * mt}-row strips, {parts} parts", us,
-                        2 * 256 * ntile * T, "mfma")
+                def layer():
+                    pack, z, x, out, qkv = layers[i["i"] % nset]
+                    i["i"] += 1
+                    et.check(call(pack, z.ptr, x.ptr, None, out.ptr, None, qkv.ptr, partial.ptr, *join, et.ACT_GELU, 1e-5, 1e-5, self.stream))
+
+                us = self.time_us(layer, launches)
+                self.record(name + (" (no tiles)" if sparsity == 1.0 else ""), f"T{T} {H} wide FFN {FF} {16 * mt}-row strips, {parts} parts", us,
+                            2 * 256 * ntile * T, "mfma")
             et.check(lib.et_stream_sync(self.stream))
             for l in layers:
                 et.check(lib.et_encoder_layer_pack_destroy(l[0]))
@@ -591,7 +599,7 @@ def run_scale(b: Bench):
 
 def main():
     ap = argparse.ArgumentParser()
-    ap.add_argument("--set", choices=("configs", "scale", "vo", "mha", "qkv", "fuseo", "local", "plan", "machine", "all"), default="all")
+    ap.add_argument("--set", choices=("configs", "scale", "vo", "mha", "qkv", "fuseo", "local", "depth", "plan", "machine", "all"), default="all")
     ap.add_argument("--json", default=None, help="also write the rows as JSON to this file")
     args = ap.parse_args()
     b = Bench()
@@ -616,10 +624,16 @@ def main():
                          (32, 128, 0.8), (16, 64, 0.8), (32, 64, 0.8), (64, 32, 0.8)):
             b.qkv_mha(B, S, sp, 48)
     if args.set == "local":
-        print("# everything between two attention kernels of a layer (binary32 residual), and the same launches without any tile")
-        for T, mt, parts, H, FF in ((128, 1, 4, 768, 3072), (528, 1, 4, 768, 3072), (1024, 1, 4, 768, 3072), (2048, 1, 2, 1024, 4096),
+        print("# everything between two attention kernels of a layer (binary32 residual), and the same launches without any tile; the parts "
+              "a model of such layers is given")
+        for T, mt, parts, H, FF in ((128, 1, 7, 768, 3072), (528, 1, 6, 768, 3072), (1024, 1, 4, 768, 3072), (2048, 1, 2, 1024, 4096),
                                     (4096, 1, 1, 768, 3072), (8192, 2, 1, 768, 3072)):
             b.token_local(T, mt, parts, H, FF, 48)
+    if args.set == "depth":
+        print("# dense Linear at 2048 rows over the depth of the product: what does not grow with it is the launch's fixed part")
+        for n_out in (768, 2304, 3072):
+            for n_in in (64, 128, 256, 384, 512, 768, 1024, 1536, 2048, 3072):
+                b.dense(2048, n_in, n_out, 50)
     if args.set == "fuseo":
         print("# attention + tile-sparse output projection: one launch against the two it replaces (768-wide, 12 heads of 64)")
         for B, S, sp in ((1, 128, 0.8), (1, 384, 0.8), (2, 128, 0.8), (4, 128, 0.8), (8, 128, 0.8), (8, 128, 0.9), (16, 128, 0.8),
