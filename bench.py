@@ -12,8 +12,8 @@ Prints ONE JSON line: sequences/s (value), ms per step, per-layer latency, the
 roofline of the dominant kernel — the one with the largest share of the step's GPU time
 in the committed rocprofv3 kernel trace: the token-local kernel, which takes a strip of token
 rows through the output projection, both LayerNorms, the FFN and the next QKV projection in
-two launches (timed with HIP events on its own stream over a HIP graph of such pairs, each on
-another layer's weights and another set of buffers, so nothing is warm in a cache) — and the
+one launch (two on a device where its parts cannot meet; timed with HIP events on its own stream over a
+HIP graph of such launches, each on another layer's weights and another set of buffers, so nothing is warm in a cache) — and the
 CPU oracle timed on the host cores.
 """
 from __future__ import annotations
@@ -397,7 +397,7 @@ def main():
                     help="everything between two attention kernels in one launch (two launches per layer)")
     ap.add_argument("--five-launches", action="store_true",
                     help="every projection as a launch of its own (five launches per layer) instead of attention and "
-                         "the token-local launch in two parts (three), which the engine picks for this batch by itself")
+                         "the token-local launch (two), which the engine picks for this batch by itself")
     ap.add_argument("--calibrate", action="store_true",
                     help="also launch a plain streaming kernel of known size (ReLU over 64 MiB in, 64 MiB out) "
                          "three times, as the reference point for rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE")

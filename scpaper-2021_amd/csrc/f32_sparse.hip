@@ -153,7 +153,8 @@ __global__ __launch_bounds__(WAVES * 64) void bsr16_linear_split_f32_kernel(cons
 // and 16 neighbouring lanes touch 16 lines: with many tiles that is what the kernels above wait for.  The rows go straight
 // to LDS, all of them requested before anything is waited for, with the first weights behind them, which stay in flight
 // across the barrier (waited for with the rows, 256 tokens 768 -> 2304 at 80 % 8.05 us, now 6.7; 2048 768 -> 3072 35.8 / 29.1).
-// Against the wide form: 4096 tokens 768 -> 3072 at 50 / 80 / 90 / 95 % 109 / 163, 52 / 78, 39 / 48, 33 / 34.
+// Against the wide form: 4096 tokens 768 -> 3072 at 50 / 80 / 90 / 95 % 111 / 172, 55 / 79, 41 / 49, 34 / 33; ten shapes of 1024 to 8192
+// tokens 0.46 - 0.69 of its time at 50 %, 0.55 - 0.77 at 80, 0.65 - 0.89 at 90, 0.78 - 1.11 at 95.
 constexpr int kStripPad = 4, kStripWaves = 8;
 __global__ __launch_bounds__(kStripWaves * 64) void bsr16_linear_strip_f32_kernel(const Bsr32Args a) {
     extern __shared__ __align__(16) unsigned char strip_smem[];
