@@ -273,15 +273,13 @@ __global__ __launch_bounds__(256) void gemm_skinny_kernel(const GemmArgs g) {
     }
 }
 
-// The small-result kernel applies when the 64x64 tiling would leave most of the chip idle.  Up to
-// 2048 tiles of 16 x 16 it beats the 64 x 64 tiles (512 x 768 -> 768: 6.1 against 7.3 us; 128 x 768
-// -> 2304: 5.4 against 7.0), from about 2300 on it loses (256 x 768 -> 2304: 8.0 against 7.4).  With a long K the 64 x 64
-// tiles have a fourth LDS buffer and the line lies lower, at 1024 (us, this kernel / 64 x 64 tiles: 768 tiles of 3072 10.7 /
-// 13.7, 1024 of 4096 16.1 / 17.0, 1152 of 3072 15.2 / 14.2, 1536 of 3072 17.3 / 14.2, 1638 of 3600 39.5 / 17.9; at 24 stages,
-// K = 1536, 1056 to 1792 tiles 0.89 to 1.21 of them).  Operands the 64 x 64 tiles do not take (a result off their alignment, as
-// a row-pruned Linear may be given) would fall to the register-staged kernel, so there the line stays: 512 x 3072 -> 528 scattered
+// The small-result kernel applies when 64 x 64 tiles would leave most of the chip idle: up to 1024 tiles of 16 x 16, from a depth of
+// 784 on up to 640 (us, this kernel / the direct-to-LDS kernel: 672 tiles of 704 4.5 / 5.6, 990 of 528 5.4 / 6.0, 513 of 1056 6.5 / 7.7, 558
+// of 2096 10.2 / 12.3, 384 of 3072 8.5 / 13.8; 1043 of 864 9.3 / 7.3, 860 of 1632 12.9 / 9.7, 1536 of 768 6.8 / 6.1, 1760 of 320
+// 4.9 / 4.6).  Operands that kernel does not take (a result off its alignment, as
+// a row-pruned Linear may be given) would fall to the register-staged kernel, so there the line lies at 2048: 512 x 3072 -> 528 scattered
 // 20.0 / 37.4, 1024 x 1536 -> 448 14.3 / 23.1, 1024 x 4096 -> 448 29.2 / 46.7.  (Batched problems do not come near it:
-// with more than 1024 tiles each, two of them have more than 128 of 64 x 64.)
+// with more than 640 tiles each, four of them have more than 128 of 64 x 64.)
 static bool gemm_skinny_applies(const GemmArgs &g, int batch, bool trans_b) {
     const auto misaligned = [](const void *p, int a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) != 0; };
     if (!trans_b || g.a_gather || batch < 1 || batch > 65535) return false;
@@ -291,7 +289,7 @@ static bool gemm_skinny_applies(const GemmArgs &g, int batch, bool trans_b) {
     if (batch > 1 && (((g.sAo | g.sAi | g.sBo | g.sBi) & 7) || ((g.sCo | g.sCi) & 3))) return false;
     const long long tiles64 = (long long)((g.M + 63) / 64) * ((g.N + 63) / 64) * batch;
     const long long tiles16 = (long long)(g.M / 16) * (g.N / 16);
-    return tiles64 < 128 && tiles16 <= (g.K / 64 >= 24 && gemm_dma_applies(g, batch, trans_b) ? 1024 : 2048);
+    return tiles64 < 128 && tiles16 <= (!gemm_dma_applies(g, batch, trans_b) ? 2048 : g.K > 768 ? 640 : 1024);
 }
 
 // C[r][c] = act(bias[c]) for the columns a row-pruned weight does not produce.

@@ -4,17 +4,15 @@
 // The 64x64-per-wave kernel in gemm.hip reads 1 byte of LDS per 32 flops, which at the
 // MFMA peak is the whole bandwidth of the LDS port, and stages through registers; it tops
 // out near a third of the matrix peak.  Here a workgroup of 4 waves (2 x 2) computes a tile of
-// 64 TMW x 64 TNW and each wave a block of TMW x TNW v_mfma_f32_32x32x16_f16 tiles.  The
-// largest tile, 256 x 256 (eight waves of 128 x 64, two per SIMD; the RAGGED form four waves of
-// 128 x 128 with 256 accumulators in AGPRs), is for problems that fill the device with it; smaller problems
-// take smaller tiles (more workgroups, several per compute unit) at the price of more operand
-// traffic from the L2 per flop.  Latencies are covered inside the wave: K advances in stages
-// of 64 through two LDS buffers (the 256 x 256 tile: stages of 32 through four, loads three
-// stages ahead), a later stage is loaded straight from global memory into
-// an idle buffer while the current one is multiplied (staging through registers and
-// ds_write costs a third of the rate: the LDS port is then the bound), the fragment reads of
-// the next K slice and the loads are issued between the MFMAs that hide them, in an order fixed in
-// the source, and the one workgroup barrier of a stage sits before its last K slice.
+// 64 TMW x 64 TNW and each wave a block of TMW x TNW v_mfma_f32_32x32x16_f16 tiles.  What bounds a stage
+// of 64 of depth is the LDS port (a 128 x 192 tile: 960 cycles of reads and direct loads against 774 of products), so a
+// tile is as large as leaves every compute unit one; what is added once is 3 us of launch, first stage and epilogue.
+// Latencies are covered inside the wave: K advances in stages of 64 through four LDS buffers, a later stage is
+// loaded straight from global memory into an idle buffer while the current one is multiplied (staging through registers and
+// ds_write costs a third of the rate: the LDS port is then the bound), fragments are read two K slices ahead, and
+// reads and loads are issued between the MFMAs that hide them, in an order fixed in the source.  With two or three buffers
+// (several workgroups to a compute unit, or the 128 x 192 tile) and with eight waves (256 x 256, whole tiles) fragments are read one
+// slice ahead: another wave covers for it.
 //
 // The MFMA A operand is the B matrix (output features) and vice versa, so a lane ends with
 // 4 consecutive features of one row of C per 8-row group of a tile; the epilogue transposes
@@ -107,34 +105,27 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(const GemmArgs 
     const int m0 = ty * BM, n0 = tx * BN;
 
     const int nbase = n0 + wn * WN;
-    // The bias of the lane's features: unconditional loads (from B when there is no bias) and a select (a load under a branch
-    // is waited for on the spot).  Requested ahead of the first stage where there are registers for it, so that the epilogue
-    // does not start with a round trip to memory (with the epilogue's barriers: 8192 x 768 -> 2304 49.6 -> 47.3 us, 8192 x
-    // 4096 -> 4096 250 -> 247).
-    constexpr bool kBiasEarly = TNW <= 2;
+    // The bias: a lane of kScLanes holds that of one feature in kScCols, an epilogue hands them round through LDS.  Two-byte loads of
+    // all the features a lane's accumulators belong to (32 of them with two feature tiles, ahead of the first stage in the
+    // order loads are answered in) held every workgroup up by 1 us.  Unconditional (from B when there is no bias) and selected.
+    // IDX: the same lanes store the scattered columns, so the index of a lane's bias is also where its column goes.
+    constexpr int kScLanes = WN % 64 == 0 ? 64 : 32;  // lanes to a row of scattered columns
+    constexpr int kScCols = WN / kScLanes;            // column groups
     const bool has_bias = g.bias != nullptr;
     const int32_t *col_idx = g.c_scatter ? g.c_scatter : g.bias_idx;  // bias index of result column n
-    h4 bias4[TNW][4];
+    int bias_at[kScCols];
+    _Float16 bias_of[kScCols];
+#pragma unroll
+    for (int e = 0; e < kScCols; e++) {
+        const int n = nbase + e * kScLanes + lane % kScLanes;
+        bias_at[e] = RAGGED ? min(n, g.N - 1) : n;
+        if (IDX && col_idx) bias_at[e] = col_idx[bias_at[e]];
+    }
     auto load_bias = [&] {
 #pragma unroll
-        for (int j = 0; j < TNW; j++)
-#pragma unroll
-            for (int q = 0; q < 4; q++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    int n = nbase + j * 32 + q * 8 + kg * 4 + e;
-                    if (RAGGED) n = min(n, g.N - 1);
-                    _Float16 bv;
-                    if (IDX) {
-                        const int bi = col_idx ? col_idx[n] : n;
-                        bv = (has_bias ? g.bias : g.B)[has_bias ? bi : 0];
-                    } else {
-                        bv = (has_bias ? g.bias : g.B)[has_bias ? n : 0];
-                    }
-                    bias4[j][q][e] = has_bias ? bv : (_Float16)0.0f;
-                }
+        for (int e = 0; e < kScCols; e++) bias_of[e] = (has_bias ? g.bias : g.B)[has_bias ? bias_at[e] : 0];
     };
-    if constexpr (kBiasEarly) load_bias();
+    if constexpr (!IDX) load_bias();  // (behind an index: once the first stage is there, and the index with it)
 
     f16v acc[TMW][TNW];  // [token tile][feature tile]
 #pragma unroll
@@ -191,36 +182,44 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(const GemmArgs 
             if (RAGGED) tailB[v] = (unsigned)((row * g.ldb + min(c8, k_tail - 8)) * 2);
         }
     }
-    const char *a_tile = reinterpret_cast<const char *>(g.A + (size_t)m0 * g.lda);
-    const char *b_tile = reinterpret_cast<const char *>(g.B + (size_t)n0 * g.ldb);
+    // Requests past the last stage are needed for the count of those outstanding, not for their data: through a buffer without
+    // records they touch no memory (fetching the last stage again was a quarter of what a workgroup took in at 12 stages, and
+    // the epilogue waited for it).  Everything about the buffer is made scalar here; a resource in vector registers would put
+    // a loop around every request.
+    auto scalar = [](const void *p) {
+        const uint64_t v = reinterpret_cast<uint64_t>(p);
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+        return reinterpret_cast<char *>((uint64_t)hi << 32 | lo);
+    };
+    char *const a_tile = scalar(g.A + (size_t)m0 * g.lda);
+    char *const b_tile = scalar(g.B + (size_t)n0 * g.ldb);
+    int records = 0;  // of both buffers: 1 GiB (256 rows of the widest operand taken) or none
+    auto aim = [&](int stages_left) { records = __builtin_amdgcn_readfirstlane(min(max(stages_left, 0), 1) << 30); };
     // loads [first, first + count) of a stage's kLA + kLB (whole tiles)
     auto load_part = [&](int buf, int k0, int first, int count) {
-        const char *ak = a_tile + (size_t)k0 * 2, *bk = b_tile + (size_t)k0 * 2;  // uniform
-        auto four = [&](const char *src, _Float16 *dst, int sub) {  // sub = v % 4 (a constant once unrolled)
-            if (sub == 0) __builtin_amdgcn_global_load_lds(ET_GLOBAL_PTR(src), ET_LDS_PTR(dst), 16, 0, 0);
-            else if (sub == 1) __builtin_amdgcn_global_load_lds(ET_GLOBAL_PTR(src), ET_LDS_PTR(dst), 16, 1024, 0);
-            else if (sub == 2) __builtin_amdgcn_global_load_lds(ET_GLOBAL_PTR(src), ET_LDS_PTR(dst), 16, 2048, 0);
-            else __builtin_amdgcn_global_load_lds(ET_GLOBAL_PTR(src), ET_LDS_PTR(dst), 16, 3072, 0);
+        auto four = [&](__amdgpu_buffer_rsrc_t rsrc, unsigned off, _Float16 *dst, int sub) {  // sub = v % 4 (a constant once unrolled)
+            if (sub == 0) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, ET_LDS_PTR(dst), 16, off, k0 * 2, 0, 0);
+            else if (sub == 1) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, ET_LDS_PTR(dst), 16, off, k0 * 2, 1024, 0);
+            else if (sub == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, ET_LDS_PTR(dst), 16, off, k0 * 2, 2048, 0);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, ET_LDS_PTR(dst), 16, off, k0 * 2, 3072, 0);
         };
+        auto ra = __builtin_amdgcn_make_buffer_rsrc(a_tile, 0, records, 0x00020000);
+        auto rb = __builtin_amdgcn_make_buffer_rsrc(b_tile, 0, records, 0x00020000);
         const bool tail = RAGGED && k0 == k_tail0 && k_tail < KS;  // uniform
 #pragma unroll
         for (int v = 0; v < kLA; v++)
             if (v >= first && v < first + count) {
                 const unsigned off = RAGGED && tail ? tailA[RAGGED ? v : 0] : offA[v];
-                four(ak + off, As + (buf * BM + wave * (BM / kWaves) + (kImm ? (v / 4) * 4 : v) * kRpi) * KS, kImm ? v % 4 : 0);
+                four(ra, off, As + (buf * BM + wave * (BM / kWaves) + (kImm ? (v / 4) * 4 : v) * kRpi) * KS, kImm ? v % 4 : 0);
             }
 #pragma unroll
         for (int v = 0; v < kLB; v++)
             if (kLA + v >= first && kLA + v < first + count) {
                 const unsigned off = RAGGED && tail ? tailB[RAGGED ? v : 0] : offB[v];
-                four(bk + off, Bs + (buf * BN + wave * (BN / kWaves) + (kImm ? (v / 4) * 4 : v) * kRpi) * KS, kImm ? v % 4 : 0);
+                four(rb, off, Bs + (buf * BN + wave * (BN / kWaves) + (kImm ? (v / 4) * 4 : v) * kRpi) * KS, kImm ? v % 4 : 0);
             }
     };
-    auto load_stage = [&](int buf, int k0) {
-        if constexpr (kWhole) {
-            load_part(buf, k0, 0, kLA + kLB);
-            return;
-        }
+    auto load_stage = [&](int buf, int k0) {  // BT
 #pragma unroll
         for (int v = 0; v < 2 * TMW; v++) {  // a wave loads a quarter of the rows of each operand
             const int r0 = wave * (BM / 4) + v * 8, r = r0 + lrow;
@@ -233,17 +232,10 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(const GemmArgs 
 #pragma unroll
         for (int v = 0; v < 2 * TNW; v++) {
             const int r0 = wave * (BN / 4) + v * 8, r = r0 + lrow;
-            if (BT) {  // LDS row r = k-value k0 + r of the stage, 64 columns of B from n0
-                const int krow = min(k0 + r, g.K - 1), n = min(n0 + lpos * 8, g.N - 8);
-                __builtin_amdgcn_global_load_lds(ET_GLOBAL_PTR(g.B + (size_t)krow * g.ldb + n),
-                                                 ET_LDS_PTR(Bs + (buf * kDmaK + r0) * BN), 16, 0, 0);
-            } else {
-                const int c = lpos ^ ((r >> 1) & 7);
-                const int row = RAGGED ? min(n0 + r, g.N - 1) : n0 + r;
-                const int k = RAGGED ? min(k0 + c * 8, g.K - 8) : k0 + c * 8;
-                __builtin_amdgcn_global_load_lds(ET_GLOBAL_PTR(g.B + (size_t)row * g.ldb + k),
-                                                 ET_LDS_PTR(Bs + (buf * BN + r0) * kDmaK), 16, 0, 0);
-            }
+            // LDS row r = k-value k0 + r of the stage, 64 columns of B from n0
+            const int krow = min(k0 + r, g.K - 1), n = min(n0 + lpos * 8, g.N - 8);
+            __builtin_amdgcn_global_load_lds(ET_GLOBAL_PTR(g.B + (size_t)krow * g.ldb + n),
+                                             ET_LDS_PTR(Bs + (buf * kDmaK + r0) * BN), 16, 0, 0);
         }
     };
     // RAGGED: zeros over the chunks of the last stage that lie past the end of K, in the rows
@@ -302,6 +294,7 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(const GemmArgs 
     // in issue order: "stage s + 1 has landed" is "at most the loads of the stages after it
     // are outstanding".
     constexpr int kAhead = NBUF - 1;
+    constexpr bool kDeep = kWhole && NBUF == 4 && NWN == 2;
     constexpr int kStageLoads = kWhole ? kLA + kLB : 2 * TMW + 2 * TNW;  // per wave
     auto wait_stages = [&](int later) {  // wait until at most `later` whole stages are outstanding
         if (later <= 0) __builtin_amdgcn_s_waitcnt(wait_vm(0));
@@ -313,59 +306,38 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(const GemmArgs 
     // included, which is exactly what a deeper pipeline must not do; here this wave's LDS reads
     // are waited for, the barrier is passed, and the compiler moves no memory access across.
     auto lds_barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-    // Order of issue inside one K slice.  The wave's instruction stream is the only thing that feeds the matrix
-    // pipe of its SIMD, so the LDS reads of the next slice go between the MFMAs of the current one instead of in a
-    // run in front of the MFMAs that need them (left alone the scheduler puts every read directly in front of its
-    // first use and the pipe drains while it returns: 2 x 4 of 16 MFMAs apart, then a wait).  Where the slice is not
-    // written out by hand (below), the pattern is given to the scheduler: kNM / kND MFMAs, one LDS read, ...
+    // Order of issue inside one K slice (K-contiguous operands).  The wave's instruction stream is the only thing that feeds
+    // the matrix pipe of its SIMD, so the slice is written out in the order it is to be issued in, one MFMA at a time
+    // with a fence for the scheduler behind it: the fragments of a later slice are read, and `nload` loads of a later
+    // stage (from number `first`) issued, evenly between the MFMAs (left alone the scheduler puts every read directly in
+    // front of its first use, and the pipe drains while it returns).
     constexpr int kNM = TMW * TNW, kND = TMW + TNW;
     constexpr int kSlices = KS / 16;                  // K slices (steps) of a stage
     constexpr int kLoadSteps = KS == 32 ? 2 : 1;      // steps of a stage that issue a share of a later stage's loads
     constexpr int kStepLoads = (kStageLoads + kLoadSteps - 1) / kLoadSteps;  // in the first such step; the rest in the second
     constexpr int kStepLoads2 = kStageLoads - kStepLoads;
-    auto interleave = [&] {
-        if constexpr (kNM >= kND) {
-            constexpr int per = kNM / kND;  // MFMAs per LDS read
-#pragma unroll
-            for (int i = 0; i < kND; i++) {
-                __builtin_amdgcn_sched_group_barrier(0x008, per, 0);  // MFMA
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);    // LDS read
-            }
-            __builtin_amdgcn_sched_group_barrier(0x008, kNM - per * kND, 0);
-        }
-    };
-    // Whole tiles with at least as many MFMAs as fragments in a K slice: the slice is written out in the order it is
-    // to be issued in, one MFMA at a time with a fence for the scheduler behind it: after every kNM / kND MFMAs
-    // one fragment of the next slice is read from LDS, and `nload` loads of a later stage (from number `first`)
-    // are dealt evenly between the MFMAs (the four waves of a workgroup issue their loads in the same slices, and
-    // a wave whose load waits for the compute unit's one address unit issues no MFMA behind it).
-    constexpr bool kManual = kWhole && kNM >= kND;
-    static_assert(!kManual || ((kStepLoads % kNM == 0 || kNM % kStepLoads == 0) && (kLoadSteps == 1 || kStepLoads2 == kStepLoads)),
-                  "the loads of a slice are dealt evenly to its MFMAs");
     auto step = [&](const Frag &fm, Frag &fr, int rbuf, int rks, int nload, int lbuf, int k_later, int first) {
         const int chunk = ((rks * 2 + kg) ^ swz) * 8;
-        // more loads than MFMAs: nload / kNM behind every MFMA; fewer: one behind every (kNM / nload)-th
-        const int lpm = nload >= kNM ? nload / kNM : 0;
-        const int every = (nload > 0 && nload < kNM) ? kNM / nload : 1;
 #pragma unroll
         for (int m = 0; m < kNM; m++) {
             const int i = m / TNW, j = m % TNW;
             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fm.w[j], fm.x[i], acc[i][j], 0, 0, 0);
-            // fragment idx of the next slice behind MFMA (idx kNM) / kND: evenly over the slice
-            const int idx = (m * kND + kNM - 1) / kNM;
-            if (idx < kND && (idx * kNM) / kND == m) {
+#pragma unroll
+            for (int idx = m * kND / kNM; idx < (m + 1) * kND / kNM; idx++) {
                 if (idx < TMW) fr.x[idx] = *reinterpret_cast<const h8 *>(a_rows + rbuf * BM * KS + chunk + idx * 32 * KS);
                 else fr.w[idx - TMW] = *reinterpret_cast<const h8 *>(b_rows + rbuf * BN * KS + chunk + (idx - TMW) * 32 * KS);
             }
-            if (lpm > 0) load_part(lbuf, k_later, first + m * lpm, lpm);
-            else if (nload > 0 && m % every == every / 2) load_part(lbuf, k_later, first + m / every, 1);
+            if (nload > 0) load_part(lbuf, k_later, first + m * nload / kNM, (m + 1) * nload / kNM - m * nload / kNM);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
     Frag f0, f1;
     if constexpr (kWhole) {
 #pragma unroll
-        for (int p = 0; p < kAhead; p++) load_stage(p, min(p, nstage - 1) * KS);
+        for (int p = 0; p < kAhead; p++) {
+            aim(nstage - p);
+            load_part(p, min(p, nstage - 1) * KS, 0, kStageLoads);
+        }
         __builtin_amdgcn_s_waitcnt(wait_vm((kAhead - 1) * kStageLoads));  // stage 0 has landed
     } else {
 #pragma unroll
@@ -373,66 +345,82 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(const GemmArgs 
             if (p < nstage) load_stage(p, p * kDmaK);
         wait_stages(min(kAhead, nstage) - 1);
     }
+    if constexpr (IDX) load_bias();
     if (RAGGED && nstage == 1 && ktail < kDmaK) zero_tail(0);
     lds_barrier();
     read_frag(f0, 0, 0);
-    // One stage, with the matrix pipe fed across the barrier: every K slice is read from LDS
-    // while the one before it is multiplied, the first slice of the next stage included, so the
-    // barrier of the stage sits before its last slice.  The loads of stage s + kAhead are issued
-    // in stage s into the buffer stage s - 1 was read from (its last readers passed
-    // the previous barrier); stage s + 1 is waited for just before the barrier.  The fragment
-    // read after the barrier of the last stage touches valid LDS and is never used; the loop
-    // has a single exit (a second one in the middle makes the register allocator copy the
-    // accumulators).
     int cur = 0;
-    for (int s = 0; s < nstage; s++) {
-        const int nxt = cur + 1 == NBUF ? 0 : cur + 1;
-        const int prev = cur == 0 ? NBUF - 1 : cur - 1;
-        const int k_later = min(s + kAhead, nstage - 1) * KS;  // whole tiles: past the end, the last stage again
-        if constexpr (kManual) {
-            step(f0, f1, cur, 1, kStepLoads, prev, k_later, 0);
-            if constexpr (kSlices == 4) {
-                step(f1, f0, cur, 2, 0, prev, k_later, 0);
-                step(f0, f1, cur, 3, 0, prev, k_later, 0);
+    if constexpr (kDeep) {
+        // One stage of the deep form.  A slice's fragments are read two slices ahead: with one wave on the SIMD, a slice of
+        // TMW x TNW MFMAs (32 cycles each) is shorter than the return of the reads dealt between them, and each slice
+        // waited for the last of its own (128 x 128 tile: 1170 cycles a stage, 850 with this order, of which the LDS port
+        // needs 768).  So slices 0 and 1 of the next stage are read in the second half of this one, and the barrier, which
+        // lets them, sits in the middle.  It waits for no LDS read: the buffer that loads go to behind it is that of the
+        // stage before, whose fragments every wave has multiplied by then.
+        Frag f2, f3;
+        read_frag(f1, 0, 1);
+        for (int s = 0; s < nstage; s++) {
+            const int nxt = (cur + 1) & 3, prev = (cur + 3) & 3;
+            const int k_later = min(s + kAhead, nstage - 1) * KS;
+            aim(nstage - s - kAhead);
+            step(f0, f2, cur, 2, 0, prev, k_later, 0);
+            step(f1, f3, cur, 3, 0, prev, k_later, 0);
+            __builtin_amdgcn_s_waitcnt(wait_vm(kStageLoads));  // stage s + 1 has landed, s + 2 may be on its way
+            if (RAGGED && s + 2 == nstage && ktail < kDmaK) {
+                zero_tail(nxt);
+                lds_barrier();
+            } else {
+                asm volatile("s_barrier" ::: "memory");
             }
-            // outstanding at most: the stages after s + 1 as far as they have been issued
-            __builtin_amdgcn_s_waitcnt(wait_vm((kAhead - 2) * kStageLoads + kStepLoads));
-            if (RAGGED && s + 2 == nstage && ktail < kDmaK) zero_tail(nxt);
-            lds_barrier();
-            step(f1, f0, nxt, 0, kLoadSteps == 2 ? kStepLoads : 0, prev, k_later, kStepLoads);
-        } else {
+            step(f2, f0, nxt, 0, kStageLoads / 2, prev, k_later, 0);
+            step(f3, f1, nxt, 1, kStageLoads - kStageLoads / 2, prev, k_later, kStageLoads / 2);
+            cur = nxt;
+        }
+    } else {
+        // One stage of the others, with the matrix pipe fed across the barrier: every K slice is read from LDS
+        // while the one before it is multiplied, the first slice of the next stage included, so the
+        // barrier of the stage sits before its last slice.  The loads of stage s + kAhead are issued
+        // in stage s into the buffer stage s - 1 was read from (its last readers passed
+        // the previous barrier); stage s + 1 is waited for just before the barrier.  The fragment
+        // read after the barrier of the last stage touches valid LDS and is never used; the loop
+        // has a single exit (a second one in the middle makes the register allocator copy the
+        // accumulators).
+        for (int s = 0; s < nstage; s++) {
+            const int nxt = cur + 1 == NBUF ? 0 : cur + 1;
+            const int prev = cur == 0 ? NBUF - 1 : cur - 1;
+            const int k_later = min(s + kAhead, nstage - 1) * KS;
             if constexpr (kWhole) {
-                read_frag(f1, cur, 1);
-                load_part(prev, k_later, 0, kStepLoads);
+                aim(nstage - s - kAhead);
+                step(f0, f1, cur, 1, kStepLoads, prev, k_later, 0);
+                if constexpr (kSlices == 4) {
+                    step(f1, f0, cur, 2, 0, prev, k_later, 0);
+                    step(f0, f1, cur, 3, 0, prev, k_later, 0);
+                }
+                // outstanding at most: the stages after s + 1 as far as they have been issued
+                __builtin_amdgcn_s_waitcnt(wait_vm((kAhead - 2) * kStageLoads + kStepLoads));
+                if (RAGGED && s + 2 == nstage && ktail < kDmaK) zero_tail(nxt);
+                lds_barrier();
+                step(f1, f0, nxt, 0, kLoadSteps == 2 ? kStepLoads2 : 0, prev, k_later, kStepLoads);
             } else {
                 if (s + kAhead < nstage) load_stage(prev, (s + kAhead) * kDmaK);
                 read_frag(f1, cur, 1);
-            }
-            multiply(f0);
-            interleave();
-            __builtin_amdgcn_sched_barrier(0);
-            if constexpr (kSlices == 4) {
+                multiply(f0);
+                __builtin_amdgcn_sched_barrier(0);
                 read_frag(f0, cur, 2);
                 multiply(f1);
-                interleave();
                 __builtin_amdgcn_sched_barrier(0);
                 read_frag(f1, cur, 3);
                 multiply(f0);
-                interleave();
+                __builtin_amdgcn_sched_barrier(0);
+                wait_stages(min(kAhead - 1, nstage - 2 - s));
+                if (RAGGED && s + 2 == nstage && ktail < kDmaK) zero_tail(nxt);
+                lds_barrier();
+                read_frag(f0, nxt, 0);
+                multiply(f1);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            // outstanding at most: the stages after s + 1 as far as they have been issued
-            if constexpr (kWhole) __builtin_amdgcn_s_waitcnt(wait_vm((kAhead - 2) * kStageLoads + kStepLoads));
-            else wait_stages(min(kAhead - 1, nstage - 2 - s));
-            if (RAGGED && s + 2 == nstage && ktail < kDmaK) zero_tail(nxt);
-            lds_barrier();
-            read_frag(f0, nxt, 0);
-            if constexpr (kWhole && kLoadSteps == 2) load_part(prev, k_later, kStepLoads, kStepLoads2);
-            multiply(f1);
-            interleave();
-            __builtin_amdgcn_sched_barrier(0);
+            cur = nxt;
         }
-        cur = nxt;
     }
     // the loads issued past the last stage have landed before the staging LDS is written again
     if constexpr (kWhole) __builtin_amdgcn_s_waitcnt(wait_vm(0));
@@ -445,38 +433,49 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(const GemmArgs 
     constexpr int kEpLd = WN + 8;
     constexpr int kRowChunks = WN / 8;  // 16-byte chunks of a stored row: 4, 8 or 16
     _Float16 *ep = reinterpret_cast<_Float16 *>(dma_smem) + wave * 32 * kEpLd;
-    if constexpr (!kBiasEarly) load_bias();
     // Scattered columns are stored one 2-byte element per lane, kScLanes consecutive result
     // columns of one row per group of lanes: ascending c_scatter keeps those stores within a
     // few neighbouring sectors of the row of C.
-    constexpr int kScLanes = WN < 64 ? WN : 64;  // lanes per row
-    constexpr int kScCols = WN / kScLanes;       // column groups
     constexpr int kScRows = 64 / kScLanes;       // rows per instruction
     const bool scatter = IDX && g.c_scatter != nullptr;  // a gathered bias alone keeps the vector stores
-    int scat[kScCols];
-    if (IDX) {
-#pragma unroll
-        for (int e = 0; e < kScCols; e++) {
-            const int n = nbase + e * kScLanes + lane % kScLanes;
-            scat[e] = scatter ? g.c_scatter[RAGGED ? min(n, g.N - 1) : n] : n;
-        }
-    }
     // (a strip is written and read by one wave, whose LDS accesses execute in order: only the compiler has to keep it.  A
     // workgroup barrier here waits for every store to memory besides.)
     auto wave_order = [] { asm volatile("" ::: "memory"); };
     const int act = g.act;
 #pragma unroll
+    for (int e = 0; e < kScCols; e++)
+        if (lane < kScLanes) ep[e * kScLanes + lane] = has_bias ? bias_of[e] : (_Float16)0.0f;
+    wave_order();
+    h4 bias4[TNW][4];
+#pragma unroll
+    for (int j = 0; j < TNW; j++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) bias4[j][q] = *reinterpret_cast<const h4 *>(ep + j * 32 + q * 8 + kg * 4);
+    wave_order();
+#pragma unroll
     for (int i = 0; i < TMW; i++) {
+        float v[TNW][16];  // (the activation is chosen once for a strip: chosen per value, each took its own branches, one after the other)
 #pragma unroll
         for (int j = 0; j < TNW; j++)
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                h4 o;
+            for (int e = 0; e < 16; e++) v[j][e] = acc[i][j][e] + (float)bias4[j][e / 4][e % 4];
+        if (act == ET_ACT_GELU) {
 #pragma unroll
-                for (int e = 0; e < 4; e++)
-                    o[e] = (_Float16)apply_act(acc[i][j][q * 4 + e] + (float)bias4[j][q][e], act);
-                *reinterpret_cast<h4 *>(ep + l32 * kEpLd + j * 32 + q * 8 + kg * 4) = o;
-            }
+            for (int j = 0; j < TNW; j++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) v[j][e] = gelu_tanh(v[j][e]);
+        } else if (act == ET_ACT_RELU) {
+#pragma unroll
+            for (int j = 0; j < TNW; j++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) v[j][e] = v[j][e] > 0.0f ? v[j][e] : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < TNW; j++)
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                *reinterpret_cast<h4 *>(ep + l32 * kEpLd + j * 32 + q * 8 + kg * 4) =
+                    h4{(_Float16)v[j][q * 4], (_Float16)v[j][q * 4 + 1], (_Float16)v[j][q * 4 + 2], (_Float16)v[j][q * 4 + 3]};
         wave_order();
         if (scatter) {
 #pragma unroll
@@ -487,7 +486,7 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(const GemmArgs 
 #pragma unroll
                 for (int e = 0; e < kScCols; e++) {
                     const bool inside = !RAGGED || (m < g.M && nbase + e * kScLanes + lane % kScLanes < g.N);
-                    if (inside) crow[scat[e]] = ep[r * kEpLd + e * kScLanes + lane % kScLanes];
+                    if (inside) crow[bias_at[e]] = ep[r * kEpLd + e * kScLanes + lane % kScLanes];
                 }
             }
         } else {
@@ -505,52 +504,49 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(const GemmArgs 
     }
 }
 
-// Tile choice, from measurements on dense Linears of 1024..16384 rows: a larger tile halves the
-// operand traffic from the L2 per flop but needs enough workgroups to keep every compute unit
-// busy through whole rounds (a 256 x 256 workgroup owns its compute unit; two 128 x 128, three
-// 128 x 64 or five 64 x 64 ones share it and cover each other's prologue and epilogue).
-// 256 x 128 tiles were measured and never won.
+// Tile choice: the form with the least time by what each was measured to take, in ns: `start` and `depth` per 64 of depth once,
+// `round` and `stage` per 64 of depth for every workgroup a compute unit gets (256 units).  Fitted to 123 Linears of 16..8192
+// rows, 208..4096 wide, multiples of 16 and of 64, with and without GELU, eight sets of buffers in turn: each
+// form within 9-15 % of its time, the choice 1.1 % slower than the best form in the mean (19 % at worst, 8192 x 256 -> 1024).
+// Against forms with one slice of fragments ahead, activations chosen per value and loads past the end (us, mean of no
+// activation and GELU): 2048 x 768 -> 3072 20.7 -> 16.0 (128 x 192 tiles), 768 8.8 -> 7.5 and 2048 x 3072 -> 768 22.3 -> 18.2 (128 x 64),
+// 4096 x 3072 -> 768 40.6 -> 32.0 (64 x 192), 8192 x 3072 -> 768 62.6 -> 47.6, 2048^3 27.9 -> 22.8 (128 x 128), 528 x 768 -> 3072 11.1 -> 7.9,
+// 1024 x 4096^2 62.2 -> 42.0.  Two buffers, several workgroups to a unit, where a short depth leaves mostly epilogues: 6448 x 1568 ->
+// 1040 54.9 -> 35.6 (41.1 with four).  128 x 192 tiles with a fourth buffer, which take all of the LDS, and 128 x 256 with eight waves were up
+// to 40 % slower on operands out of the caches than in them (2048 x 384 -> 3072 10.2 and 14.8, this form 10.8).
 struct DmaTile { int tmw, tnw, nbuf; bool ragged; };
+struct DmaForm { int tmw, tnw, nbuf, start, depth, round, stage; };  // tiles of 64 tmw x 64 tnw
+constexpr DmaForm kDmaForms[] = {
+    {1, 1, 4, 2000, 30, 1150, 209}, {2, 1, 4, 250, 0, 3250, 330}, {1, 2, 4, 200, 0, 3300, 336}, {2, 2, 4, 0, 0, 4800, 490},
+    {1, 3, 4, 0, 0, 4400, 430},     {2, 3, 3, 0, 0, 6100, 605},   {2, 2, 2, 900, 300, 2600, 440}, {2, 1, 2, 1500, 340, 1300, 275},
+    {4, 4, 4, 0, 0, 8200, 1220},
+};
 static bool pick_dma_tile(const GemmArgs &g, int batch, bool trans_b, DmaTile *out) {
-    const bool ragged = g.M % 64 || g.N % 64 || g.K % kDmaK || batch != 1 || !trans_b;
-    if (ragged) {
-        // 64 x 64 tiles with the edges clamped and masked; large ragged problems are left to the
-        // 128 x 128 tiles of the register-staged kernel
-        const long long w = (long long)((g.M + 63) / 64) * ((g.N + 63) / 64) * batch;
-        if (g.M % 16 || g.N % 16 || g.K % 16) return false;
-        if (batch == 1 && trans_b) {
-            // enough workgroups for the larger tiles, as for whole tiles below (a row- or column-pruned
-            // Linear keeps any multiple of 16 features: 2048 x 768 -> 2928 26.7 -> 21.4 us with 128 x 64 tiles)
-            const long long m128 = (g.M + 127) / 128;
-            if ((long long)((g.M + 255) / 256) * ((g.N + 255) / 256) >= 1024) { *out = {4, 4, 2, true}; return true; }
-            if (m128 * ((g.N + 127) / 128) >= 512) { *out = {2, 2, 2, true}; return true; }
-            if (m128 * ((g.N + 63) / 64) >= 512) { *out = {2, 1, 2, true}; return true; }
-        }
-        if (w > 1536) return false;
-        // Batched problems and B stored k-major run on this instantiation too, where they are
+    if (g.M % 16 || g.N % 16 || g.K % 16) return false;
+    if (batch != 1 || !trans_b) {
+        // Batched problems and B stored k-major run on 64 x 64 tiles where they are
         // bound by the latency of a long K loop in few workgroups (the stacked VO product of the
         // pre-computed-VO attention: 32 -> 22 us); gathering the k-major fragments with 2-byte LDS
         // reads costs more than it saves elsewhere (Linear_VO 28 -> 78 us), those stay on the
         // register-staged kernel.
-        if ((batch != 1 || !trans_b) && (w > 256 || g.K / kDmaK < 16)) return false;
-        *out = {1, 1, g.K / kDmaK < 24 || w > 512 ? 2 : w > 256 || !trans_b ? 3 : 4, true};  // third and fourth buffer: as below
+        const long long w = (long long)((g.M + 63) / 64) * ((g.N + 63) / 64) * batch;
+        if (w > 256 || g.K / kDmaK < 16) return false;
+        *out = {1, 1, trans_b ? 4 : g.K / kDmaK < 24 ? 2 : 3, true};
         return true;
     }
-    auto wgs = [&](int tmw, int tnw) -> long long {
-        const int bm = 64 * tmw, bn = 64 * tnw;
-        return (g.M % bm || g.N % bn) ? 0 : (long long)(g.M / bm) * (g.N / bn);
-    };
-    const long long w44 = wgs(4, 4), w11 = wgs(1, 1);
-    // whole rounds of one workgroup per compute unit, or so many that the last one hardly counts
-    if (w44 >= 256 && (w44 % 256 == 0 || w44 >= 1024)) { *out = {4, 4, 2, false}; return true; }
-    if (wgs(2, 2) >= 512) { *out = {2, 2, 2, false}; return true; }
-    if (wgs(2, 1) >= 512) { *out = {2, 1, 2, false}; return true; }
-    // few workgroups with a long K loop are bound by the latency of a stage: a third buffer keeps
-    // two stages in flight (2048 x 3072 -> 768: 29.5 -> 24.7 us; from 12 stages on it still gives
-    // 3-5 %: 2048 x 768 -> 768 9.6 -> 9.1 us); elsewhere it only costs occupancy
-    // With at most one workgroup a compute unit and 24 stages a fourth: 1024 x 3072 -> 768 16.3 -> 14.5, 512 x 4096 -> 1024 19.1
-    // -> 17.1, 208 x 3600 -> 3264 19.5 -> 18.4 (384 workgroups: 21.6 -> 22.0).
-    *out = {1, 1, (w11 <= 256 && g.K / kDmaK >= 24) ? 4 : (w11 <= 512 && g.K / kDmaK >= 12) ? 3 : 2, false};
+    long long best = -1;
+    const long long stages = (g.K + kDmaK - 1) / kDmaK;
+    for (const DmaForm &f : kDmaForms) {
+        const int bm = 64 * f.tmw, bn = 64 * f.tnw;
+        const bool whole = g.M % bm == 0 && g.N % bn == 0 && g.K % kDmaK == 0;
+        if (f.tmw == 4 && !whole) continue;  // (written for whole tiles)
+        const long long wgs = (long long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn), rounds = (wgs + 255) / 256;
+        const long long ns = f.start + stages * f.depth + rounds * (f.round + stages * f.stage);
+        if (best < 0 || ns < best) {
+            best = ns;
+            *out = {f.tmw, f.tnw, f.nbuf, !whole};
+        }
+    }
     return true;
 }
 
@@ -606,26 +602,29 @@ static int launch_dma_tile(const GemmArgs &g, int batch, hipStream_t stream) {
 int launch_gemm_dma(const GemmArgs &g, int batch, bool trans_b, hipStream_t stream) {
     DmaTile t{};
     if (!pick_dma_tile(g, batch, trans_b, &t)) return ET_ERR_UNSUPPORTED;
-    if (t.ragged) {
-        if (!trans_b)
-            return t.nbuf == 3 ? launch_dma_tile<1, 1, 3, true, true>(g, batch, stream)
-                               : launch_dma_tile<1, 1, 2, true, true>(g, batch, stream);
-        if (t.tmw == 4) return launch_dma_tile<4, 4, 2, true>(g, batch, stream);
-        if (t.tmw == 2) return t.tnw == 2 ? launch_dma_tile<2, 2, 2, true>(g, batch, stream)
-                                          : launch_dma_tile<2, 1, 2, true>(g, batch, stream);
-        return t.nbuf == 4   ? launch_dma_tile<1, 1, 4, true>(g, batch, stream)
-               : t.nbuf == 3 ? launch_dma_tile<1, 1, 3, true>(g, batch, stream)
-                             : launch_dma_tile<1, 1, 2, true>(g, batch, stream);
-    }
-    switch (t.tmw * 100 + t.tnw * 10 + t.nbuf) {
+    if (!trans_b)
+        return t.nbuf == 3 ? launch_dma_tile<1, 1, 3, true, true>(g, batch, stream)
+                           : launch_dma_tile<1, 1, 2, true, true>(g, batch, stream);
+    switch (t.tmw * 100 + t.tnw * 10 + t.nbuf + (t.ragged ? 1000 : 0)) {
+        case 114: return launch_dma_tile<1, 1, 4>(g, 1, stream);
+        case 124: return launch_dma_tile<1, 2, 4>(g, 1, stream);
+        case 134: return launch_dma_tile<1, 3, 4>(g, 1, stream);
+        case 212: return launch_dma_tile<2, 1, 2>(g, 1, stream);
+        case 214: return launch_dma_tile<2, 1, 4>(g, 1, stream);
+        case 222: return launch_dma_tile<2, 2, 2>(g, 1, stream);
+        case 224: return launch_dma_tile<2, 2, 4>(g, 1, stream);
+        case 233: return launch_dma_tile<2, 3, 3>(g, 1, stream);
         // 256 x 256: eight waves of 128 x 64, half stages through four buffers (four waves of 128 x 128 in the same
         // LDS: 0.5-2 % slower)
-        case 442: return launch_dma_tile<4, 2, 4, false, false, 32, 4>(g, 1, stream);
-        case 222: return launch_dma_tile<2, 2, 2>(g, 1, stream);
-        case 212: return launch_dma_tile<2, 1, 2>(g, 1, stream);
-        case 112: return launch_dma_tile<1, 1, 2>(g, 1, stream);
-        case 113: return launch_dma_tile<1, 1, 3>(g, 1, stream);
-        case 114: return launch_dma_tile<1, 1, 4>(g, 1, stream);
+        case 444: return launch_dma_tile<4, 2, 4, false, false, 32, 4>(g, 1, stream);
+        case 1114: return launch_dma_tile<1, 1, 4, true>(g, batch, stream);
+        case 1124: return launch_dma_tile<1, 2, 4, true>(g, 1, stream);
+        case 1134: return launch_dma_tile<1, 3, 4, true>(g, 1, stream);
+        case 1212: return launch_dma_tile<2, 1, 2, true>(g, 1, stream);
+        case 1214: return launch_dma_tile<2, 1, 4, true>(g, 1, stream);
+        case 1222: return launch_dma_tile<2, 2, 2, true>(g, 1, stream);
+        case 1224: return launch_dma_tile<2, 2, 4, true>(g, 1, stream);
+        case 1233: return launch_dma_tile<2, 3, 3, true>(g, 1, stream);
         default: return ET_ERR_UNSUPPORTED;
     }
 }

@@ -41,6 +41,39 @@ def test_linear_dense(et, T, inp, out, act):
     assert Hn.max_abs(d_y.numpy(), want) <= 4e-3
 
 
+# Every tile of the direct-to-LDS kernel, by the rule that chooses them: whole, with ragged edges, with one stage of depth,
+# and with a last stage of 16 or 48 k-values.  (T, inp, out)
+DMA_FORMS = [(64, 128, 192), (64, 64, 64), (64, 176, 64), (400, 16, 16), (64, 128, 16),  # 64 x 64
+             (448, 320, 4224), (320, 64, 5504), (272, 80, 6096), (288, 192, 5648), (1216, 192, 1728), (336, 400, 5696),  # 64 x 128, 192
+             (768, 128, 1408), (5504, 64, 192), (144, 80, 5824), (5696, 48, 144), (5488, 128, 144),  # 128 x 64, two buffers
+             (5504, 320, 192), (144, 176, 5456), (144, 256, 5456),  # 128 x 64, four
+             (384, 128, 5504), (384, 64, 5504), (5552, 80, 336), (464, 16, 4112), (352, 128, 5456),  # 128 x 128, two
+             (6080, 400, 400), (2048, 640, 2048), (4096, 704, 1024),  # 128 x 128, four
+             (2432, 128, 1728), (1040, 400, 3600), (784, 256, 4736), (3328, 64, 2560), (2560, 128, 3328)]  # 128 x 192, 256 x 256
+
+
+@pytest.mark.parametrize("T,inp,out", DMA_FORMS)
+def test_linear_dense_and_row_pruned_in_every_tile(et, T, inp, out):
+    """The result stays within half a unit of its binary16 place and the binary32 sum's own error (at most
+    inp 2^-24 of the sum of magnitudes, below 5e-4 at 704 inputs), scattered columns land where their indices say, the
+    columns between them hold the bias."""
+    W, b, x = Hn.randn((out, inp), 1, 0.02), Hn.randn((2 * out,), 2, 0.1), Hn.randn((T, inp), 3)
+    ids = np.sort(np.random.default_rng(4).permutation(2 * out)[:out]).astype(np.int32)
+    product = (Hn.f32(x).double() @ Hn.f32(W).double().T).numpy()
+    b64 = b.astype(np.float64)
+    d_W, d_b, d_x, d_ids = up(et, W), up(et, b), up(et, x), up(et, ids)
+    d_y = et.DeviceBuffer.empty((T, out), np.float16)
+    et.linear_dense(d_W, d_b, d_x, d_y, T, inp, out, 0)
+    want = product + b64[:out]
+    assert (np.abs(d_y.numpy() - want) <= 2.0 ** -11 * np.abs(want) + 5e-4).all()
+    d_s = et.DeviceBuffer.empty((T, 2 * out), np.float16)
+    et.check(et.lib().et_linear_rowpruned_f16(d_W.ptr, d_ids.ptr, out, d_b.ptr, d_x.ptr, d_s.ptr, T, inp, 2 * out, 1, None))
+    want = np.repeat(b64[None], T, 0)
+    want[:, ids] += product
+    want = np.maximum(want, 0)
+    assert (np.abs(d_s.numpy() - want) <= 2.0 ** -11 * np.abs(want) + 5e-4).all()
+
+
 def _random_dense_cases(n, seed):
     rng = np.random.default_rng(seed)
     cases = []
