@@ -32,7 +32,10 @@
 // the shares come back out of that L2, where behind a launch boundary they come from the memory-side cache, as do table, offsets
 // and first slots, which here are on their way while the parts meet; 2 us of boundary go besides.  8 x 128 tokens at 80 %
 // 382 -> 361 us (12 layers, weights in the memory-side cache), 12 x 128 241 -> 220 (6 layers), BERT-large 4 x 512 at 90 % 1175 ->
-// 1124.  (The first form of it, with requests only behind the meeting: 387.)
+// 1124.  (The first form of it, with requests only behind the meeting: 387.)  What the parts do between the products is bound by
+// scalar round trips and by vector instructions, not by bytes (of 52 000 cycles at 8 x 128 the LayerNorms are 6 600, the shares 3 800, the way
+// out of the projection 2 100): the others' shares requested in one go at addresses worked out once, the chunks of the projection in
+// the table instead of divisions, binary16 values added by v_fma_mix: 375.7 -> 368.1 us there, one sequence 320.4 -> 311.8.
 //
 // Streams (built on the host, et_encoder_layer_pack_create; those of the second launch, or of the projection alone, behind
 // those of the first): per (part, wave) the slots in the order they are multiplied, the byte offsets of their two column
@@ -57,9 +60,10 @@ constexpr int kElWaves = 16;
 constexpr int kElRing = 8;     // weight slots of a wave in flight
 constexpr int kElMaxSeg = 24;  // segments of a launch
 constexpr size_t kElLds = 160 * 1024;
-// table of a (part, wave), 64 words, a lane holds one: block-rows of every segment, sums of every wave; and the descriptors
+// table of a (part, wave), 64 words, a lane holds one: block-rows of every segment, sums of every wave, slots, and of every chunk of
+// the projection its first block-row (bits 0-15) and their number (worked out in the kernel, four divisions a chunk); and the descriptors
 // of its block-rows, in the same way: one request each at the start, read with v_readlane
-constexpr int kElTabSeg = 0, kElTabCount = kElTabSeg + kElMaxSeg, kElTabSlots = kElTabCount + kElWaves, kElTab = 64, kElRowRegs = 2;
+constexpr int kElTabSeg = 0, kElTabCount = kElTabSeg + kElMaxSeg, kElTabSlots = kElTabCount + kElWaves, kElTabOut = kElTabSlots + 1, kElTab = 64, kElRowRegs = 2;
 // descriptor: slots (bits 0-7), kind (8-9), operand in the hidden chunk (10), target (11-20), bias over 16 (21-31)
 constexpr int kElBufferWord = 0x00020000;  // of a raw buffer resource
 constexpr int kElKindSum = 0, kElKindHidden = 1, kElKindQkv = 2, kElMaxSlots = 255;
@@ -377,21 +381,19 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
         el_ring_start(lane_off, offs_off, slots, offs);
         asm volatile("s_waitcnt vmcnt(%0)" ::"i"(kElRingAsks) : "memory");
     };
-    // The shares of a strip, added in the order of the parts, into V; `mine`: the part whose share V holds already (-1: none).
-    // The ring goes out behind the last of them (MODE 4: ahead of them, while the parts meet).
-    auto sum_shares = [&](int mine) {
-        constexpr int kTogether = MODE == 4 ? (NR > 3 ? 1 : 3) : NR > 3 ? 2 : 4;  // shares requested together
+    // The shares of a strip, added in the order of the parts, into V.  The ring goes out behind the last of them.
+    auto sum_shares = [&] {
+        constexpr int kTogether = NR > 3 ? 2 : 4;  // shares requested together
         f4 u[kTogether][NR][MT], sum[NR][MT];
 #pragma unroll
         for (int j = 0; j < NR; j++)
 #pragma unroll
             for (int m = 0; m < MT; m++) sum[j][m] = f4{0.f, 0.f, 0.f, 0.f};
-        const int nshare = ET_EL_ARG(nshare);
+        const int nshare = a.nshare;
         auto ask_shares = [&](int p) {
 #pragma unroll
             for (int q = 0; q < kTogether; q++) {
-                if (MODE == 4 && (p + q == mine || p + q >= nshare)) continue;  // uniform
-                const char *src = reinterpret_cast<const char *>(ET_EL_ARG(partial) + ((size_t)min(p + q, nshare - 1) * ET_EL_ARG(T) + tok0) * ET_EL_ARG(H));
+                const char *src = reinterpret_cast<const char *>(a.partial + ((size_t)min(p + q, nshare - 1) * a.T + tok0) * a.H);
 #pragma unroll
                 for (int j = 0; j < NR; j++)
 #pragma unroll
@@ -411,7 +413,7 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
 #pragma unroll
                     for (int j = 0; j < NR; j++)
 #pragma unroll
-                        for (int m = 0; m < MT; m++) sum[j][m] += MODE == 4 && p + q == mine ? V[j][m] : u[q][j][m];
+                        for (int m = 0; m < MT; m++) sum[j][m] += u[q][j][m];
                 }
         };
         int p = 0;
@@ -421,9 +423,58 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
             add_shares(p);
         }
         ask_shares(p);
-        if constexpr (MODE == 4) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        else ring_start();
+        ring_start();
         add_shares(p);
+#pragma unroll
+        for (int j = 0; j < NR; j++)
+#pragma unroll
+            for (int m = 0; m < MT; m++) V[j][m] = sum[j][m];
+    };
+    // The same in the joined launch, where V holds the share of part `mine` and the ring went out while the parts met: the others'
+    // shares are requested together, as many as there are registers for (with four parts all three), at addresses worked
+    // out once.  The order of the additions is that of the parts.
+    auto sum_others = [&](int mine) {
+        constexpr int kTogether = NR > 3 ? 2 : 3;
+        const auto *l = late();
+        const int last = l->nshare - 1;
+        const size_t stride = (size_t)l->T * (size_t)l->H * 4;
+        const char *const base = reinterpret_cast<const char *>(l->partial) + (size_t)tok0 * (size_t)l->H * 4;
+        f4 u[kTogether][NR][MT], sum[NR][MT];
+#pragma unroll
+        for (int j = 0; j < NR; j++)
+#pragma unroll
+            for (int m = 0; m < MT; m++) sum[j][m] = f4{0.f, 0.f, 0.f, 0.f};
+        auto add = [&](f4 (&v)[NR][MT]) {
+#pragma unroll
+            for (int j = 0; j < NR; j++)
+#pragma unroll
+                for (int m = 0; m < MT; m++) sum[j][m] += v[j][m];
+        };
+        for (int o = 0; o < last; o += kTogether) {  // o + q: the others, counted without `mine`
+#pragma unroll
+            for (int q = 0; q < kTogether; q++) {
+                const int p = min(o + q, last - 1);
+                const char *src = base + (size_t)(p + (p >= mine ? 1 : 0)) * stride;
+#pragma unroll
+                for (int j = 0; j < NR; j++)
+#pragma unroll
+                    for (int m = 0; m < MT; m++) el_ask(u[q][j][m], tile_at(m, j) + lane * 16, src);
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int q = 0; q < kTogether; q++)
+#pragma unroll
+                for (int j = 0; j < NR; j++)
+#pragma unroll
+                    for (int m = 0; m < MT; m++) el_tie(u[q][j][m]);
+#pragma unroll
+            for (int q = 0; q < kTogether; q++) {
+                if (o + q >= last) continue;  // uniform
+                if (o + q == mine) add(V);
+                add(u[q]);
+            }
+        }
+        if (mine == last) add(V);
 #pragma unroll
         for (int j = 0; j < NR; j++)
 #pragma unroll
@@ -434,7 +485,7 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
         ring_start();
     } else if constexpr (MODE == 2) {
         ask_vectors();
-        sum_shares(-1);
+        sum_shares();
     } else {
         ask_vectors();
         ask_residual(V);
@@ -461,20 +512,33 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
     };
     // features of this wave, and of the four waves whose sums this lane adds (one over them; 0 for a wave without any)
     const int own_rows = __builtin_amdgcn_readlane(tab, kElTabCount + wave);
+    // A binary16 value added to a binary32 one in one instruction (v_fma_mix: converted, times one, plus; the same bits as a
+    // conversion and an addition).  Four waves share a SIMD's vector unit, and a LayerNorm is bound by its instructions.
+    auto add_half = [&](f4 &v, h4 b, float one) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = __builtin_fmaf((float)b[e], one, v[e]);
+    };
+    auto opaque_one = [] {
+        float one = 1.0f;
+        asm volatile("" : "+v"(one));
+        return one;
+    };
     auto norm = [&](const _Float16 *add, const _Float16 *gam, const _Float16 *bet, float eps) {
         const int r16 = el_here(lane & 15), g = el_here(lane >> 4), gbit = g & 1;
         float mean[MT], rstd[MT], n_of[4], inv_of[4], live[NR];
 #pragma unroll
         for (int j = 0; j < NR; j++) live[j] = here(rb[j]) >= 0 ? 1.0f : 0.0f;
-        const int own_here = here(own_rows);
-        const float inv_own = own_here ? 1.0f / (float)(own_here * 16) : 0.0f;
+        float inv_own;
         if (H == kElWaves * 16 * NR) {  // uniform: every wave holds NR
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 n_of[k] = (float)(NR * 16);
                 inv_of[k] = 1.0f / (float)(NR * 16);
             }
+            inv_own = 1.0f / (float)(NR * 16);
         } else {
+            const int own_here = here(own_rows);
+            inv_own = own_here ? 1.0f / (float)(own_here * 16) : 0.0f;
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 const int rows_of = __shfl(tab, kElTabCount + g * 4 + k, 64);
@@ -485,12 +549,11 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
         if (add) {  // uniform
             h4 bv[NR];
             vec_of(bv, add);
+            const float one = opaque_one();
 #pragma unroll
             for (int j = 0; j < NR; j++)
 #pragma unroll
-                for (int m = 0; m < MT; m++)
-#pragma unroll
-                    for (int e = 0; e < 4; e++) V[j][m][e] += (float)bv[j][e];
+                for (int m = 0; m < MT; m++) add_half(V[j][m], bv[j], one);
         }
         float2 *rd = reinterpret_cast<float2 *>(red);
 #pragma unroll
@@ -534,6 +597,8 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
         h4 gm[NR], bt[NR];
         vec_of(gm, gam);
         vec_of(bt, bet);
+        unsigned xrow = r16 * a.xs + gbit * 8;  // (once; sunk under the branches it is a product for each)
+        asm volatile("" : "+v"(xrow));
 #pragma unroll
         for (int j = 0; j < NR; j++)
 #pragma unroll
@@ -544,8 +609,8 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
                     V[j][m][e] = norm_value(V[j][m][e], mean[m], rstd[m], (float)gm[j][e], (float)bt[j][e]);
                     o[e] = (_Float16)V[j][m][e];
                 }
-                const int row = m * 16 + r16, u = rb[j] * 2 + (g >> 1);
-                if (rb[j] >= 0) *reinterpret_cast<h4 *>(X + row * a.xs + ((u ^ r16) << 4) + gbit * 8) = o;
+                const int u = rb[j] * 2 + (g >> 1);
+                if (rb[j] >= 0) *reinterpret_cast<h4 *>(X + (xrow + m * 16 * a.xs + ((u ^ r16) << 4))) = o;
             }
     };
 
@@ -574,7 +639,8 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
         slots[2] = __builtin_amdgcn_readlane(tab, kElTabSlots) * 1024;
     };
     auto store_share = [&] {
-        char *dst = reinterpret_cast<char *>(ET_EL_ARG(partial) + ((size_t)part * ET_EL_ARG(T) + tok0) * ET_EL_ARG(H));
+        const auto *l = late();
+        char *dst = reinterpret_cast<char *>(l->partial + ((size_t)part * l->T + tok0) * l->H);
         const unsigned at16 = el_here(lane) * 16;
 #pragma unroll
         for (int j = 0; j < NR; j++)
@@ -604,7 +670,7 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
         if (mask < 0) return false;
         others = (unsigned)mask;
         el_barrier();  // (`red` is written again)
-        sum_shares(part);
+        sum_others(part);
         have_stream();
         return true;
     };
@@ -640,12 +706,11 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
         if (first && !(kParts && part != 0)) {  // the second product is added to y + b2
             h4 bv[NR];
             vec_of(bv, b2);
+            const float one = opaque_one();
 #pragma unroll
             for (int j = 0; j < NR; j++)
 #pragma unroll
-                for (int m = 0; m < MT; m++)
-#pragma unroll
-                    for (int e = 0; e < 4; e++) V[j][m][e] += (float)bv[j][e];
+                for (int m = 0; m < MT; m++) add_half(V[j][m], bv[j], one);
         } else if (first) {
 #pragma unroll
             for (int j = 0; j < NR; j++)
@@ -715,15 +780,24 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
             }
             if (MODE != 1 && PHASE != 1 && seg > ET_EL_ARG(nseg_ff)) {  // the projection's chunk leaves the LDS, whole rows of it at a time
                 el_barrier();
-                const int Q = ET_EL_ARG(Q), nb = Q >> 4, np = MODE == 0 ? 1 : ET_EL_ARG(parts), nq = ET_EL_ARG(nseg_q), hs = ET_EL_ARG(hs);
-                const int q_first = MODE == 0 ? 0 : nb * who / np, q_rows = MODE == 0 ? nb : nb * (who + 1) / np - q_first;
-                const int c = seg - ET_EL_ARG(nseg_ff) - 1, first_rb = q_first + q_rows * c / nq, units = (q_first + q_rows * (c + 1) / nq - first_rb) * 2;
+                const auto *l = late();
+                const int Q = l->Q, hs = l->hs, c = seg - l->nseg_ff - 1, nq = l->nseg_q;
+                const uint32_t chunk = (uint32_t)__builtin_amdgcn_readlane(tab, kElTabOut + c);
+                const int first_rb = chunk & 0xffff, units = (chunk >> 16) * 2;
                 const unsigned char *src = Hb + ((c & 1) ? hbuf : 0u);
-                _Float16 *const qkv = ET_EL_ARG(qkv);
+                char *const qkv = reinterpret_cast<char *>(l->qkv + (size_t)tok0 * Q + first_rb * 16);
+                // both halves of a wave's rows are read ahead of the first store
                 for (int t = wave; t < tiles_here * 16; t += kElWaves) {
-                    char *dst = reinterpret_cast<char *>(qkv + (size_t)(tok0 + t) * Q + first_rb * 16);
-                    for (int u = el_here(lane); u < units; u += 64)
-                        *reinterpret_cast<h8 *>(dst + u * 16) = *reinterpret_cast<const h8 *>(src + t * hs + ((u ^ (t & 15)) << 4));
+                    char *dst = qkv + (size_t)(t * Q * 2);
+                    for (int u = el_here(lane); u < units; u += 128) {
+                        const h8 v = *reinterpret_cast<const h8 *>(src + t * hs + ((u ^ (t & 15)) << 4));
+                        const int u2 = u + 64;
+                        if (u2 < units) {
+                            const h8 v2 = *reinterpret_cast<const h8 *>(src + t * hs + ((u2 ^ (t & 15)) << 4));
+                            *reinterpret_cast<h8 *>(dst + u2 * 16) = v2;
+                        }
+                        *reinterpret_cast<h8 *>(dst + u * 16) = v;
+                    }
                 }
                 if (c == nq - 1) break;
                 continue;
@@ -924,10 +998,12 @@ static int el_pack_create(const et_layer_weights *w, int T, int emdim, int dimFF
     };
     // vectors in LDS: bo g1 be1 | b1 | b2 g2 be2 | bq
     const int at_b1 = 3 * H, at_bq = 6 * H + FF;
+    std::vector<int32_t> chunks_of_q;  // of the streams that are emitted next
     auto emit = [&](const std::vector<std::vector<std::vector<ElRow>>> &segs) {  // [segment][wave]
         for (int v = 0; v < kElWaves; v++) {
             Stream st;
             st.tab.assign(kElTab, 0);
+            std::copy(chunks_of_q.begin(), chunks_of_q.end(), st.tab.begin() + kElTabOut);
             for (int o = 0; o < kElWaves; o++) st.tab[(size_t)(kElTabCount + o)] = (int)sums[(size_t)o].size();
             for (size_t sg = 0; sg < segs.size(); sg++) {
                 st.tab[kElTabSeg + sg] = (int32_t)segs[sg][(size_t)v].size();
@@ -950,9 +1026,11 @@ static int el_pack_create(const et_layer_weights *w, int T, int emdim, int dimFF
     const auto empty = [] { return std::vector<std::vector<ElRow>>(kElWaves); };
     auto qkv_segments = [&](std::vector<std::vector<std::vector<ElRow>>> &segs, int q, int nq) {
         const int q0 = nbQ * q / nq, n = nbQ * (q + 1) / nq - q0;
+        chunks_of_q.clear();
         for (int c = 0; c < nchunk_q; c++) {
             std::vector<ElRow> free;
             const int cb = q0 + n * c / nchunk_q, ce = q0 + n * (c + 1) / nchunk_q;
+            chunks_of_q.push_back(cb | (ce - cb) << 16);
             for (int r = cb; r < ce; r++) free.push_back({kElKindQkv, r - cb, at_bq + r * 16, 0, r, tiles_of(mq, 3, r)});
             deal(segs[(size_t)(nseg_ff + 1 + c)], free);
         }
