@@ -220,10 +220,11 @@ static int launch_mha_nw(const MhaArgs &args, hipStream_t stream) {
 // 344 -> 276.  A block takes 6200 cycles; the vector unit is busy for 3700 of them and the matrix cores for 2050.  With one
 // barrier a block and no phases 414, with the groups' waves on the same SIMD 459; row sums by an MFMA against ones, or a
 // priority for either phase: 1-3 % slower.
-// For S a multiple of 256, no additive mask and a positive scale; padded keys and the causal mask are applied to the
-// blocks they cut, and a wave skips the blocks past its last query.
+// For no additive mask and a positive scale; padded keys and the causal mask are applied to the
+// blocks they cut, and a wave skips the blocks past its last query.  RAGGED: S is a multiple of 16 only; keys past it are
+// requested from the last rows and stored as zeros, queries past it are not written, and a wave that has no others only stages.
 constexpr int kPpQ = 256;  // queries of a workgroup
-__device__ __forceinline__ void mha_pingpong(const MhaArgs &a, unsigned block) {
+template <bool RAGGED> __device__ __forceinline__ void mha_pingpong(const MhaArgs &a, unsigned block) {
     constexpr int HD = 64, KS = 2, DB = 4, QT = 2;
     using L = MhaLds<HD>;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -235,7 +236,7 @@ __device__ __forceinline__ void mha_pingpong(const MhaArgs &a, unsigned block) {
     const int r16 = lane & 15, g = lane >> 4;
     const int S = a.S, hd = a.hd;
     // as in the kernel above: the query strips of a (sequence, head) on one XCD
-    const int qstrips = S / kPpQ;
+    const int qstrips = RAGGED ? (S + kPpQ - 1) / kPpQ : S / kPpQ;
     const int xcd = block % kXcds, k_in_xcd = block / kXcds;
     const int bh = xcd + kXcds * (k_in_xcd / qstrips);
     if (bh >= a.nbh) return;  // padding of the last round (whole workgroup)
@@ -246,7 +247,7 @@ __device__ __forceinline__ void mha_pingpong(const MhaArgs &a, unsigned block) {
     int klimit = S;
     if (a.lens) klimit = min(S, max(a.lens[b], 0));
     if (a.causal) klimit = min(klimit, (qstrip + 1) * kPpQ);
-    const int nblocks = (klimit + kKeyBlock - 1) / kKeyBlock;  // (of 128 whole rows each: S is a multiple of 256)
+    const int nblocks = (klimit + kKeyBlock - 1) / kKeyBlock;  // (of 128 whole rows each unless RAGGED)
 
     h8 qf[QT][KS];
 #pragma unroll
@@ -254,7 +255,8 @@ __device__ __forceinline__ void mha_pingpong(const MhaArgs &a, unsigned block) {
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
             const bool in = 32 * ks + 8 * g < hd;  // columns past the head size: zero
-            qf[t][ks] = *reinterpret_cast<const h8 *>(a.Q + (row0 + wave_q + t * 16 + r16) * a.ldq + h * hd + (in ? 32 * ks + 8 * g : 0));
+            const size_t row = RAGGED ? row0 + min(wave_q + t * 16 + r16, S - 1) : row0 + wave_q + t * 16 + r16;
+            qf[t][ks] = *reinterpret_cast<const h8 *>(a.Q + row * a.ldq + h * hd + (in ? 32 * ks + 8 * g : 0));
             if (!in) qf[t][ks] = h8{0, 0, 0, 0, 0, 0, 0, 0};
         }
     f4 o[QT][DB];
@@ -276,6 +278,15 @@ __device__ __forceinline__ void mha_pingpong(const MhaArgs &a, unsigned block) {
     const size_t step = (size_t)ld * (second ? 32 : 1);
     h8 st[4];
     auto load = [&](int blk) {  // (past the last block: the last again, not read)
+        if (RAGGED && (min(blk, nblocks - 1) + 1) * kKeyBlock > S) {  // uniform
+            const int k0 = min(blk, nblocks - 1) * kKeyBlock, key = second ? key_k : key_v;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int row = min(k0 + key + i * (second ? 32 : 1), S - 1) - key;
+                st[i] = *reinterpret_cast<const h8 *>(src + (ptrdiff_t)row * ld);
+            }
+            return;
+        }
         const _Float16 *p = src + (size_t)(min(blk, nblocks - 1) * kKeyBlock) * ld;
 #pragma unroll
         for (int i = 0; i < 4; i++) st[i] = *reinterpret_cast<const h8 *>(p + i * step);
@@ -284,8 +295,14 @@ __device__ __forceinline__ void mha_pingpong(const MhaArgs &a, unsigned block) {
         const int kg = key_v >> 2;
         return (32 * (kg >> 3) + 8 * (kg & 3) + 4 * ((kg >> 2) & 1)) ^ vt_swizzle<HD>(dg >> 1);
     }();
-    auto store = [&](int buf) {
+    auto store = [&](int buf, int blk) {
         const h8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+        if (RAGGED && (min(blk, nblocks - 1) + 1) * kKeyBlock > S) {  // uniform
+            const int left = S - min(blk, nblocks - 1) * kKeyBlock;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if ((second ? key_k + 32 * i : key_v + i) >= left) st[i] = zero8;
+        }
         if (!col_in)
 #pragma unroll
             for (int i = 0; i < 4; i++) st[i] = zero8;
@@ -396,17 +413,17 @@ __device__ __forceinline__ void mha_pingpong(const MhaArgs &a, unsigned block) {
         }
     };
     // (a block whose keys all lie past the wave's last query has no part in its result)
-    auto live = [&](int blk) { return !a.causal || blk * kKeyBlock < wave_q + QT * 16; };
+    auto live = [&](int blk) { return (!RAGGED || wave_q < S) && (!a.causal || blk * kKeyBlock < wave_q + QT * 16); };
 
     if (nblocks > 0) {  // uniform over the workgroup
         load(0);
         if (second) {
-            store(0);
+            store(0, 0);
             load(1);
         }
         phase_end();
         if (second) {
-            store(1);
+            store(1, 1);
             load(2);
             phase_end();
         }
@@ -419,7 +436,7 @@ __device__ __forceinline__ void mha_pingpong(const MhaArgs &a, unsigned block) {
                 products(std::true_type{}, std::false_type{}, (j - 1) & 1, 0);
             }
             phase_end();
-            store(j & 1);  // V of block j, or K of block j + 2
+            store(j & 1, second ? j + 2 : j);  // V of block j, or K of block j + 2
             load(second ? j + 3 : j + 1);
             if (live(j)) softmax(j * kKeyBlock);
             phase_end();
@@ -432,6 +449,7 @@ __device__ __forceinline__ void mha_pingpong(const MhaArgs &a, unsigned block) {
     for (int t = 0; t < QT; t++) {
         const float l = rows_sum(l_part[t]);
         const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        if (RAGGED && wave_q + t * 16 >= S) continue;  // (S is a multiple of 16: whole tiles)
         _Float16 *zp = a.Z + (row0 + wave_q + t * 16 + r16) * a.ldz + h * hd + 4 * g;
 #pragma unroll
         for (int d = 0; d < DB; d++) {
@@ -443,31 +461,36 @@ __device__ __forceinline__ void mha_pingpong(const MhaArgs &a, unsigned block) {
     }
 }
 
-__global__ __launch_bounds__(512) void mha_pingpong_kernel(const MhaArgs a) { mha_pingpong(a, blockIdx.x); }
-__global__ __launch_bounds__(512) void mha_pingpong_ahead_kernel(const MhaArgs a) {
+template <bool RAGGED> __global__ __launch_bounds__(512) void mha_pingpong_kernel(const MhaArgs a) { mha_pingpong<RAGGED>(a, blockIdx.x); }
+template <bool RAGGED> __global__ __launch_bounds__(512) void mha_pingpong_ahead_kernel(const MhaArgs a) {
     if (blockIdx.x < a.ahead_blocks) return ahead_of(a);
-    mha_pingpong(a, blockIdx.x - a.ahead_blocks);
+    mha_pingpong<RAGGED>(a, blockIdx.x - a.ahead_blocks);
 }
 
-static int launch_mha_pingpong(const MhaArgs &args, hipStream_t stream) {
+template <bool RAGGED> static int launch_mha_pingpong(const MhaArgs &args, hipStream_t stream) {
     constexpr size_t lds = 2 * MhaLds<64>::bytes;
     static bool raised = false;
     if (!raised) {
-        for (auto k : {mha_pingpong_kernel, mha_pingpong_ahead_kernel})
+        for (auto k : {mha_pingpong_kernel<RAGGED>, mha_pingpong_ahead_kernel<RAGGED>})
             ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         raised = true;
     }
-    const int qstrips = args.S / kPpQ, rounds = (args.nbh + kXcds - 1) / kXcds;
+    const int qstrips = (args.S + kPpQ - 1) / kPpQ, rounds = (args.nbh + kXcds - 1) / kXcds;
     MhaArgs a = args;
     a.ahead_blocks = ahead_blocks(a, 512);
-    (a.ahead_blocks ? mha_pingpong_ahead_kernel : mha_pingpong_kernel)<<<dim3(a.ahead_blocks + (unsigned)(rounds * kXcds * qstrips)), 512, lds, stream>>>(a);
+    (a.ahead_blocks ? mha_pingpong_ahead_kernel<RAGGED> : mha_pingpong_kernel<RAGGED>)<<<dim3(a.ahead_blocks + (unsigned)(rounds * kXcds * qstrips)), 512, lds, stream>>>(a);
     return check_launch("mha_pingpong_kernel");
 }
 
-// 4 waves per workgroup and one 16-query tile per wave; 2 or 1 waves when 4 would leave a
-// half-empty strip (S = 32, 96, 16, ...).  Larger workgroups stage each key block for more
+// 4 waves per workgroup and one 16-query tile per wave, whatever the last strip holds: a wave without queries still stages
+// its share of every key block.  (Strips of 2 or 1 waves where 4 leave one half-empty, 12 heads of 64, against 4: 16 x 80 keys 6.8
+// and 5.8 us, 3 x 176 9.0 and 6.1, 16 x 176 25.4 and 10.1, 16 x 528 126 and 38, 16 x 720 193 and 57; one sequence of 16 to 112 keys 5.6-5.9
+// and 4.6-4.8.  Only many sequences of 32 keys keep 2: 768 heads of 32 5.1 and 5.5.)  Larger workgroups stage each key block for more
 // queries and pay once the grid still fills the chip: 8 waves (128 queries) from 256 such
-// workgroups on (2048 keys, 16 x 16 heads: 546 -> 516 us; 128-wide heads 592 -> 570 us), and 8
+// workgroups on (2048 keys, 16 x 16 heads: 546 -> 516 us; 128-wide heads 592 -> 570 us) unless they leave more
+// than a seventh more places without queries than 4 do (64 x 12 heads: 80 keys 12.4 -> 11.0, 208 33.1 -> 30.3, but 144 24.0 -> 27.0, 48 7.7 ->
+// 9.6), leave a third of the places on the chip empty in the mean of their rounds (two to a unit; 8 x 12 heads, 656 keys 32.4 -> 35.7, 1296
+// 84.8 -> 93.2, but 528 24.6 -> 21.2, 912 49.0 -> 45.8), or the mask is causal and the heads 64 wide (16 x 12 heads, 912 keys 62.8 -> 74.4), and 8
 // waves with two query tiles each (256 queries; every K and V^T fragment read from LDS feeds two
 // MFMAs) from 512 on (-> 464 us; 214 registers, two waves per SIMD).  128-wide heads: the 8-wave
 // form prefetches the next block through registers (565 -> 532 us at 2048 keys, 16 x 8 heads),
@@ -478,22 +501,33 @@ static int launch_mha(const MhaArgs &args, int B, hipStream_t stream) {
     (void)B;
     const int qblocks = args.S / 16;
     if constexpr (!COMPACT) {
+        const int strips8 = (qblocks + 7) / 8, strips4 = (qblocks + 3) / 4;
         // The two groups of waves in turn: 256-query strips like the next form, but from 192 of them on (2 x 16 heads, 2048
         // keys, 256 strips: 58.7 -> 45.2 us; 4 x 12 heads, 1024 keys, 192: 30.3 -> 24.0; with 128 strips 35 -> 41) and from
         // 512 keys on (512 strips of 512 keys 32.4 either way, of 256 keys 32.3 -> 34): a sequence of one or two blocks
         // has nothing to take turns with.
         if (HD == 64 && qblocks % 16 == 0 && args.S >= 512 && (long)args.nbh * (qblocks / 16) >= 192 && !args.mask && args.scale_log2e > 0.0f)
-            return launch_mha_pingpong(args, stream);
-        if (HD == 64 && qblocks % 16 == 0 && (long)args.nbh * (qblocks / 16) >= 512)
+            return launch_mha_pingpong<false>(args, stream);
+        // The same for other lengths, which pay 4-5 % for their edges, where the strips of 256 leave no more than a tenth more places empty
+        // than strips of 128 and fill the last round of every XCD (32 units) to 85 % (16 x 12 heads: 912 keys 88.2 -> 79.8 us, 1872 296 -> 260,
+        // 2032 331 -> 280; 8 x 16 heads, 1296 keys 113 -> 101; but 8 x 12 heads, 912 keys, three quarters full, 45.8 -> 51.3; causal level or slower).
+        const int strips16 = (qblocks + 15) / 16, units = (args.nbh + kXcds - 1) / kXcds;
+        const long u16 = (long)units * strips16;
+        if (HD == 64 && qblocks % 16 != 0 && args.S >= 768 && !args.causal && !args.mask && args.scale_log2e > 0.0f &&
+            20 * strips16 <= 11 * strips8 && 100 * u16 >= 85 * 32 * ((u16 + 31) / 32))
+            return launch_mha_pingpong<true>(args, stream);
+        // (256 causal keys: 64 x 12 heads 45.3 us in this form, 37 in strips of 64)
+        if (HD == 64 && qblocks % 16 == 0 && (long)args.nbh * (qblocks / 16) >= 512 && !(args.causal && args.S == 256))
             return launch_mha_nw<(HD == 64 ? HD : 64), COMPACT, 8, 2>(args, stream);
         if (HD == 128 && qblocks % 16 == 0 && (long)args.nbh * (qblocks / 16) >= 512)
             return launch_mha_nw<(HD == 128 ? HD : 128), COMPACT, 8, 2>(args, stream);
-        if (HD >= 64 && qblocks % 8 == 0 && (long)args.nbh * (qblocks / 8) >= 256)
+        const long u8 = (long)units * strips8;
+        if (HD >= 64 && !(HD == 64 && args.causal) && (long)args.nbh * strips8 >= 256 && 7 * strips8 * 8 <= 8 * strips4 * 4 &&
+            10 * u8 * strips4 >= 7 * 64 * ((u8 + 63) / 64) * strips8 * 2)
             return launch_mha_nw<HD, COMPACT, 8, 1>(args, stream);
     }
-    if (qblocks % 4 == 0) return launch_mha_nw<HD, COMPACT, 4, 1>(args, stream);
-    if (qblocks % 2 == 0) return launch_mha_nw<HD, COMPACT, 2, 1>(args, stream);
-    return launch_mha_nw<HD, COMPACT, 1, 1>(args, stream);
+    if (qblocks == 2 && args.nbh >= 512) return launch_mha_nw<HD, COMPACT, 2, 1>(args, stream);
+    return launch_mha_nw<HD, COMPACT, 4, 1>(args, stream);
 }
 
 
