@@ -159,9 +159,20 @@ __global__ __launch_bounds__(((MT == 1 && (FX & kFxRes32) && !(FX & kFxRes16)) |
     const int ngroups = (nbr + a.rows_per_wg - 1) / a.rows_per_wg;
     const int nstrips = (a.T + MT * 16 - 1) / (MT * 16);
     const int xcd = blockIdx.x % kXcds, k_in_xcd = blockIdx.x / kXcds;
-    const int strip = xcd + kXcds * (k_in_xcd / ngroups);
-    const int group = k_in_xcd % ngroups;
-    if (strip >= nstrips) return;  // padding of the last round of strips (whole workgroup)
+    int strip, group;
+    if (nstrips < kXcds) {
+        // Fewer strips than XCDs: pinned, they left most of the chip idle (16 rows ran on 32 of 256 compute units).  The
+        // workgroups, in the order of the strips, are dealt to the XCDs in equal runs instead (16 x 768 -> 3072 at 50 % 18.9 -> 4.8 us,
+        // 16 x 1024 -> 4096 29.1 -> 5.2, 64 x 3072 -> 768 17.1 -> 9.2; from 8 strips on the two are the same but for the die of a strip).
+        const int units = nstrips * ngroups, per_xcd = (units + kXcds - 1) / kXcds, unit = xcd * per_xcd + k_in_xcd;
+        if (unit >= units) return;  // padding of the last XCD's run (whole workgroup)
+        strip = unit / ngroups;
+        group = unit - strip * ngroups;
+    } else {
+        strip = xcd + kXcds * (k_in_xcd / ngroups);
+        group = k_in_xcd % ngroups;
+        if (strip >= nstrips) return;  // padding of the last round of strips (whole workgroup)
+    }
     const int tok0 = strip * (MT * 16);
     const int rb_begin = group * a.rows_per_wg;
     const int rb_end = min(rb_begin + a.rows_per_wg, nbr);
@@ -1099,9 +1110,9 @@ static int launch_bsr_act(const BsrArgs &args, const BsrPlan &p, hipStream_t str
     const int nbr = args.out / 16;
     const int ngroups = (nbr + p.rows_per_wg - 1) / p.rows_per_wg;
     const int nstrips = (args.T + MT * 16 - 1) / (MT * 16);
-    const int strip_rounds = (nstrips + kXcds - 1) / kXcds;
-    const dim3 grid((unsigned)(strip_rounds * kXcds * ngroups));
-    kernel<<<grid, p.threads, p.lds, stream>>>(args);
+    // (the kernel's own two ways to deal them out)
+    const int per_xcd = nstrips < kXcds ? (nstrips * ngroups + kXcds - 1) / kXcds : (nstrips + kXcds - 1) / kXcds * ngroups;
+    kernel<<<(unsigned)(per_xcd * kXcds), p.threads, p.lds, stream>>>(args);
     return check_launch("bsr16_linear_kernel");
 }
 

@@ -200,6 +200,20 @@ def test_linear_bsr16(et, T, inp, out, sp, act):
     assert err <= 4e-3
 
 
+@pytest.mark.parametrize("strip_rows,inp,out", [(16, 208, 800), (16, 3072, 768), (32, 1024, 528), (64, 768, 2304)])
+def test_linear_bsr16_fewer_strips_than_dies(et, strip_rows, inp, out):
+    """1 to 9 strips of the height these shapes take, the last one ragged: below 8 strips the workgroups are dealt to the
+    dies in runs, from 8 on a strip keeps to one die.  Every value is written, and is that of the oracle."""
+    w = Hn.BsrWeight(out, inp, 0.7, seed=21, bias_std=0.1).upload(et)
+    for strips in range(1, 10):
+        T = strip_rows * strips - (16 if strip_rows > 16 and strips % 2 == 0 else 0)
+        x = Hn.randn((T, inp), 22 + strips)
+        d_y = up(et, np.full((T, out), np.nan, np.float16))
+        w.forward(et, up(et, x), d_y, T, 0)
+        want = L.linear(Hn.f32(x), Hn.f32(w.dense), Hn.f32(w.bias), None, torch.float16)
+        assert Hn.max_abs(d_y.numpy(), want.numpy()) <= 4e-3, (strips, T)
+
+
 def _random_bsr_cases(n, seed):
     rng = np.random.default_rng(seed)
     cases = []
