@@ -44,7 +44,7 @@ struct MhaArgs {
     const int32_t *lens;   // [B] or nullptr
     int ldq, ldk, ldv, ldz;
     int S, nh;
-    int hd;             // head size, a multiple of 8; the kernel template is the next of 32, 64, 128, 256
+    int hd;             // head size, a multiple of 8; the kernel template is the next of 32, 64, 96, 128, 224, 256
     int nbh;            // sequences * heads
     float scale_log2e;  // scale * log2(e)
     int causal;
@@ -65,8 +65,14 @@ constexpr int kKeyBlock = 128;          // keys staged per iteration
 constexpr int kNKB = kKeyBlock / 16;    // 16-key MFMA blocks per iteration
 constexpr float kLog2e = 1.4426950408889634f;
 
+// Keys staged per iteration by a head of up to HD.  Beyond 128 half as many, so that two workgroups share a compute unit (62 KB of LDS for 224
+// columns against 120, and held to 256 registers, which takes no spill): 4 heads of 200, 16 x 2048 keys 818 -> 468 us, 3 x 1680 153 -> 94,
+// 64 x 128 24.1 -> 16.4, 2 x 16 8.6 -> 5.5.  With the 306 registers the allocator takes by itself, and one workgroup, 887, 159, 24.0 and 5.9.
+template <int HD> constexpr int mha_key_block() { return HD > 128 ? 64 : kKeyBlock; }
+
 template <int HD>
 struct MhaLds {
+    static constexpr int kKeyBlock = mha_key_block<HD>();
     static constexpr int ldk = HD + 8;           // halfs per staged K row
     static constexpr int ldvt = kKeyBlock + 8;   // halfs per staged V^T row
     static constexpr int k_halfs = kKeyBlock * ldk;
@@ -158,7 +164,7 @@ template <int HD, int NW, bool COMPACT, int QT> constexpr bool mha_three_waves()
 
 template <int HD, bool COMPACT, int NW, int QT>
 __global__ __launch_bounds__(64 * NW)
-    __attribute__((amdgpu_waves_per_eu(mha_three_waves<HD, NW, COMPACT, QT>() ? 3 : 1, mha_three_waves<HD, NW, COMPACT, QT>() ? 3 : 8))) void
+    __attribute__((amdgpu_waves_per_eu(HD > 128 ? 2 : mha_three_waves<HD, NW, COMPACT, QT>() ? 3 : 1, HD > 128 ? 2 : mha_three_waves<HD, NW, COMPACT, QT>() ? 3 : 8))) void
     mha_fused_kernel(const MhaArgs a) {
     constexpr bool kCoherentZ = false;
     const unsigned block = blockIdx.x;
@@ -519,8 +525,8 @@ static int launch_mha(const MhaArgs &args, int B, hipStream_t stream) {
         // (256 causal keys: 64 x 12 heads 45.3 us in this form, 37 in strips of 64)
         if (HD == 64 && qblocks % 16 == 0 && (long)args.nbh * (qblocks / 16) >= 512 && !(args.causal && args.S == 256))
             return launch_mha_nw<(HD == 64 ? HD : 64), COMPACT, 8, 2>(args, stream);
-        if (HD == 128 && qblocks % 16 == 0 && (long)args.nbh * (qblocks / 16) >= 512)
-            return launch_mha_nw<(HD == 128 ? HD : 128), COMPACT, 8, 2>(args, stream);
+        if ((HD == 96 || HD == 128) && qblocks % 16 == 0 && (long)args.nbh * (qblocks / 16) >= 512)
+            return launch_mha_nw<(HD == 96 || HD == 128 ? HD : 128), COMPACT, 8, 2>(args, stream);
         const long u8 = (long)units * strips8;
         if (HD >= 64 && !(HD == 64 && args.causal) && (long)args.nbh * strips8 >= 256 && 7 * strips8 * 8 <= 8 * strips4 * 4 &&
             10 * u8 * strips4 >= 7 * 64 * ((u8 + 63) / 64) * strips8 * 2)
@@ -1274,11 +1280,11 @@ int et_mha_fused_ahead_f16(const et_f16 *Q, const et_f16 *K, const et_f16 *V, in
     args.v_head_ptr = nullptr;
     if (hd <= 32) return launch_mha<32, false>(args, B, as_stream(stream));
     if (hd <= 64) return launch_mha<64, false>(args, B, as_stream(stream));
+    if (hd <= 96) return launch_mha<96, false>(args, B, as_stream(stream));  // (10 heads of 80 as 128 wide: 64 x 128 keys 24.4 -> 19.5 us, 16 x 2048 580 -> 382)
     if (hd <= 128) return launch_mha<128, false>(args, B, as_stream(stream));
-    // Heads up to 256 wide: 4 waves share the staging of a 128-key block (137 KB of LDS), each with one
-    // 16-query tile.  One workgroup per compute unit and one wave per SIMD, so a wave has the whole
-    // register file (8 waves at 256 registers spill 68 bytes per lane); a strip shorter than 64 queries
-    // leaves waves without queries, which stage and otherwise idle.
+    // Heads up to 224 (200 are the reference example's) and 256 wide: 4 waves share the staging of a 64-key block, each with one
+    // 16-query tile; a strip shorter than 64 queries leaves waves without queries, which stage and otherwise idle.
+    if (hd <= 224) return launch_mha_nw<224, false, 4, 1>(args, as_stream(stream));
     return launch_mha_nw<256, false, 4, 1>(args, as_stream(stream));
 }
 

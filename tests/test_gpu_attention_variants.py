@@ -294,7 +294,10 @@ def test_mha_fused_waves_in_turn(et, B, S, nh, hd, causal, lens, scale):
 @pytest.mark.parametrize("B,S,nh,hd,causal,lens", [
     (3, 1296, 12, 64, False, [1296, 5, 1290]), (3, 1296, 12, 40, False, [1025, 9, 0]), (8, 912, 16, 64, False, None), (4, 1904, 24, 64, False, None),
     (16, 80, 16, 64, False, None), (16, 112, 16, 128, True, None), (3, 176, 12, 64, False, None), (3, 176, 12, 64, True, [176, 3, 17]),
-    (3, 16, 4, 64, False, None), (3, 48, 5, 128, True, None), (3, 528, 2, 32, True, None), (64, 32, 8, 32, False, None), (5, 96, 3, 200, False, None)])
+    (3, 16, 4, 64, False, None), (3, 48, 5, 128, True, None), (3, 528, 2, 32, True, None), (64, 32, 8, 32, False, None), (5, 96, 3, 200, False, None),
+    # heads of 65 to 96 and beyond 128: templates of their own, the latter in blocks of 64 keys
+    (3, 208, 4, 80, True, [208, 9, 70]), (3, 272, 3, 96, False, None), (40, 512, 16, 88, False, None), (3, 208, 4, 200, True, [65, 9, 128]),
+    (4, 64, 3, 224, False, None), (3, 144, 2, 256, False, [144, 3, 0])])
 def test_mha_fused_ragged_strips(et, B, S, nh, hd, causal, lens):
     H, T = nh * hd, B * S
     qkv = Hn.randn((T, 3 * H), 93)
