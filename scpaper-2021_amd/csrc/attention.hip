@@ -496,7 +496,8 @@ template <bool RAGGED> static int launch_mha_pingpong(const MhaArgs &args, hipSt
 // workgroups on (2048 keys, 16 x 16 heads: 546 -> 516 us; 128-wide heads 592 -> 570 us) unless they leave more
 // than a seventh more places without queries than 4 do (64 x 12 heads: 80 keys 12.4 -> 11.0, 208 33.1 -> 30.3, but 144 24.0 -> 27.0, 48 7.7 ->
 // 9.6), leave a third of the places on the chip empty in the mean of their rounds (two to a unit; 8 x 12 heads, 656 keys 32.4 -> 35.7, 1296
-// 84.8 -> 93.2, but 528 24.6 -> 21.2, 912 49.0 -> 45.8), or the mask is causal and the heads 64 wide (16 x 12 heads, 912 keys 62.8 -> 74.4), and 8
+// 84.8 -> 93.2, but 528 24.6 -> 21.2, 912 49.0 -> 45.8); under a causal mask heads of 64 take 8 only for whole strips, one or two of them
+// (64 x 12 heads, 128 keys 15.8 -> 15.3) or on a chip nine tenths full (8 x 12 heads, 640 keys 22.4 -> 20.2; 16 x 12, 912 keys 62.8 -> 74.4); and 8
 // waves with two query tiles each (256 queries; every K and V^T fragment read from LDS feeds two
 // MFMAs) from 512 on (-> 464 us; 214 registers, two waves per SIMD).  128-wide heads: the 8-wave
 // form prefetches the next block through registers (565 -> 532 us at 2048 keys, 16 x 8 heads),
@@ -528,8 +529,10 @@ static int launch_mha(const MhaArgs &args, int B, hipStream_t stream) {
         if ((HD == 96 || HD == 128) && qblocks % 16 == 0 && (long)args.nbh * (qblocks / 16) >= 512)
             return launch_mha_nw<(HD == 96 || HD == 128 ? HD : 128), COMPACT, 8, 2>(args, stream);
         const long u8 = (long)units * strips8;
-        if (HD >= 64 && !(HD == 64 && args.causal) && (long)args.nbh * strips8 >= 256 && 7 * strips8 * 8 <= 8 * strips4 * 4 &&
-            10 * u8 * strips4 >= 7 * 64 * ((u8 + 63) / 64) * strips8 * 2)
+        const long places8 = 64 * ((u8 + 63) / 64);
+        const bool takes8 = HD == 64 && args.causal ? qblocks % 8 == 0 && (qblocks <= 16 || 10 * u8 >= 9 * places8)
+                                                    : 7 * strips8 * 8 <= 8 * strips4 * 4 && 10 * u8 * strips4 >= 7 * places8 * strips8 * 2;
+        if (HD >= 64 && (long)args.nbh * strips8 >= 256 && takes8)
             return launch_mha_nw<HD, COMPACT, 8, 1>(args, stream);
     }
     if (qblocks == 2 && args.nbh >= 512) return launch_mha_nw<HD, COMPACT, 2, 1>(args, stream);
