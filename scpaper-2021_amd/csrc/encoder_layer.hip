@@ -500,6 +500,10 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
 
     const unsigned kx = (unsigned)((gbit ^ r16) & 15) << 4;
     const unsigned hbuf = a.hbuf;
+    // the lane's token row in the strip and in a hidden chunk, held: worked out for every block-row, the two products took as
+    // long as eight other vector instructions
+    unsigned row_x = (unsigned)r16 * a.xs, row_h = (unsigned)r16 * a.hs;
+    asm volatile("" : "+v"(row_x), "+v"(row_h));
 
     // LayerNorm of V (+ add) in place; the result is also rounded into X.  A wave sums its features of a token and their
     // squared distances from its own mean; the waves exchange both through LDS once, and the second moment about the
@@ -738,8 +742,7 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
                 else __builtin_amdgcn_s_setprio(1);
                 const int n = d & 255, kind = (d >> 8) & 3, target = (d >> 11) & 1023, bias_at = (d >> 21) * 16;
                 const bool hid = (d >> 10) & 1;
-                const unsigned ld = hid ? a.hs : a.xs;
-                const unsigned base = (hid ? MT * 16 * a.xs + hb_dn : 0u) + (unsigned)el_here(lane & 15) * ld, step = 16 * ld;
+                const unsigned base = hid ? row_h + (MT * 16 * a.xs + hb_dn) : row_x, step = 16 * (hid ? a.hs : a.xs);
                 if constexpr (MODE != 3 && PHASE != 2) {
                     if (kind == kElKindSum) {
 #pragma unroll
@@ -770,7 +773,7 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
                 const unsigned u = (unsigned)target * 2 + (g >> 1);
 #pragma unroll
                 for (int m = 0; m < MT; m++)
-                    *reinterpret_cast<h4 *>(Hb + hb_up + (m * 16 + r16) * a.hs + ((u ^ r16) << 4) + gbit * 8) =
+                    *reinterpret_cast<h4 *>(Hb + (row_h + (hb_up + m * 16 * a.hs + ((u ^ r16) << 4) + gbit * 8))) =
                         h4{(_Float16)acc[m][0], (_Float16)acc[m][1], (_Float16)acc[m][2], (_Float16)acc[m][3]};
             }
             const bool first = kFirst && PHASE != 2 && seg == 0;
