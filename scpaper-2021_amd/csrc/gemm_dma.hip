@@ -11,8 +11,8 @@
 // loaded straight from global memory into an idle buffer while the current one is multiplied (staging through registers and
 // ds_write costs a third of the rate: the LDS port is then the bound), fragments are read two K slices ahead, and
 // reads and loads are issued between the MFMAs that hide them, in an order fixed in the source.  With two or three buffers
-// (several workgroups to a compute unit, or the 128 x 192 tile) and with eight waves (256 x 256, whole tiles) fragments are read one
-// slice ahead: another wave covers for it.
+// (several workgroups to a compute unit, or the 128 x 192 tile) and with eight waves (256 x 256, whole tiles; four waves of 128 x 128 where
+// edges are ragged) fragments are read one slice ahead: another wave, or a slice of 16 MFMAs, covers for it.
 //
 // The MFMA A operand is the B matrix (output features) and vice versa, so a lane ends with
 // 4 consecutive features of one row of C per 8-row group of a tile; the epilogue transposes
@@ -534,6 +534,12 @@ static bool pick_dma_tile(const GemmArgs &g, int batch, bool trans_b, DmaTile *o
         *out = {1, 1, trans_b ? 4 : g.K / kDmaK < 24 ? 2 : 3, true};
         return true;
     }
+    // Ragged edges and so many tiles of 256 x 256 that their last round hardly counts: four waves of 128 x 128 (16368 x 8192^2 1980 us
+    // against 2380 in tiles of 128 x 192, 8176^3 1134 / 1400; 512 such tiles, 8176 x 4080^2, 330 / 325).
+    if ((g.M % 64 || g.N % 64 || g.K % kDmaK) && (long long)((g.M + 255) / 256) * ((g.N + 255) / 256) >= 1024) {
+        *out = {4, 4, 2, true};
+        return true;
+    }
     long long best = -1;
     const long long stages = (g.K + kDmaK - 1) / kDmaK;
     for (const DmaForm &f : kDmaForms) {
@@ -625,6 +631,7 @@ int launch_gemm_dma(const GemmArgs &g, int batch, bool trans_b, hipStream_t stre
         case 1222: return launch_dma_tile<2, 2, 2, true>(g, 1, stream);
         case 1224: return launch_dma_tile<2, 2, 4, true>(g, 1, stream);
         case 1233: return launch_dma_tile<2, 3, 3, true>(g, 1, stream);
+        case 1442: return launch_dma_tile<4, 4, 2, true>(g, 1, stream);
         default: return ET_ERR_UNSUPPORTED;
     }
 }
