@@ -399,31 +399,59 @@ __global__ __launch_bounds__(256) void gather_cols_kernel(_Float16 *__restrict__
 }
 
 // The same through LDS: a workgroup stages R whole rows of X with 16-byte loads (a quad of lanes
-// inside one cache line), then every lane picks its 8 columns out of LDS.  The 2-byte reads of the
+// inside one cache line), then every lane picks its columns out of LDS.  The 2-byte reads of the
 // kernel above go to memory one by one, each quad of lanes on up to four cache lines of a row
 // that the other waves are picking from at the same time.  R * in halfs of dynamic LDS.
+// What bounds it is the chain of round trips, not bytes (3 + 1.5 MB for 2048 x 768 -> 384), so a lane asks for its K chunks of
+// X together and for its indices right behind them, and keeps to 4 columns of every row it picks.  4 columns a lane and not 8: at half of
+// the columns kept, 8 are 32 bytes of the staged row apart from lane to lane, an eighth of the LDS banks.
+// Lanes that pick nothing ask for no index (with them 8192 x 768 -> 80 4.28 us, 4.17 without).
+// `lanes` of the workgroup's threads pick from one row, min(nnz / 4, 256).
+// Against 8 rows a workgroup, 8 columns a lane and indices behind the barrier (us, replays of a graph): 128 x 768 -> 384 2.53 -> 2.15, 2048 x 768 ->
+// 384 2.76 -> 2.64, 8192 x 768 -> 384 5.06 -> 4.77, 8192 x 1024 -> 720 6.88 -> 6.37, 2048 x 768 -> 80 2.40 -> 2.33; 8192 rows of which a tenth
+// is kept are level (4.12 and 4.17, 7.07 and 7.11).
+template <int K>
 __global__ __launch_bounds__(256) void gather_cols_staged_kernel(_Float16 *__restrict__ dst,
                                                                  const _Float16 *__restrict__ X,
                                                                  const int32_t *__restrict__ col_id, int T,
-                                                                 int in, int nnz, int R) {
+                                                                 int in, int nnz, int R, int lanes) {
     extern __shared__ __align__(16) unsigned char gather_smem[];
     _Float16 *rows = reinterpret_cast<_Float16 *>(gather_smem);
-    const int per_row = nnz >> 3, chunks = in >> 3;
+    const int units = nnz >> 2, chunks = in >> 3, tid = threadIdx.x;
+    const int row_first = tid / lanes, unit_first = tid - row_first * lanes, row_step = 256 / lanes;
+    const bool picks = row_first < row_step;  // (the threads past the last whole row of lanes only stage)
     for (int r0 = blockIdx.x * R; r0 < T; r0 += gridDim.x * R) {
-        const int nrow = min(R, T - r0);
-        for (int i = threadIdx.x; i < nrow * chunks; i += 256)  // rows r0 .. r0 + nrow are contiguous in X
-            reinterpret_cast<h8 *>(rows)[i] = reinterpret_cast<const h8 *>(X + (size_t)r0 * in)[i];
-        __syncthreads();
-        for (int v = threadIdx.x; v < nrow * per_row; v += 256) {
-            const int r = v / per_row, c = (v - r * per_row) * 8;
-            const int4 i0 = *reinterpret_cast<const int4 *>(col_id + c);
-            const int4 i1 = *reinterpret_cast<const int4 *>(col_id + c + 4);
-            const _Float16 *row = rows + r * in;
-            h8 o;
-            o[0] = row[i0.x]; o[1] = row[i0.y]; o[2] = row[i0.z]; o[3] = row[i0.w];
-            o[4] = row[i1.x]; o[5] = row[i1.y]; o[6] = row[i1.z]; o[7] = row[i1.w];
-            *reinterpret_cast<h8 *>(dst + (size_t)(r0 + r) * nnz + c) = o;
+        const int nrow = min(R, T - r0), n = nrow * chunks;  // rows r0 .. r0 + nrow are contiguous in X
+        const h8 *src = reinterpret_cast<const h8 *>(X + (size_t)r0 * in);
+        h8 st[K];
+        auto load = [&](int i0) {
+#pragma unroll
+            for (int k = 0; k < K; k++) st[k] = src[min(i0 + k * 256, n - 1)];
+        };
+        auto store = [&](int i0) {
+#pragma unroll
+            for (int k = 0; k < K; k++)
+                if (i0 + k * 256 < n) reinterpret_cast<h8 *>(rows)[i0 + k * 256] = st[k];
+        };
+        load(tid);
+        int4 idx_first = {0, 0, 0, 0};
+        if (picks && row_first < nrow) idx_first = *reinterpret_cast<const int4 *>(col_id + unit_first * 4);
+        __builtin_amdgcn_sched_barrier(0);
+        store(tid);
+        for (int i0 = tid + 256 * K; i0 < n; i0 += 256 * K) {  // (rows of more than 8192 values)
+            load(i0);
+            store(i0);
         }
+        __syncthreads();
+        if (picks)
+            for (int u = unit_first; u < units; u += lanes) {
+                int4 idx = idx_first;
+                if (u != unit_first) idx = *reinterpret_cast<const int4 *>(col_id + u * 4);
+                for (int r = row_first; r < nrow; r += row_step) {
+                    const _Float16 *row = rows + r * in;
+                    *reinterpret_cast<h4 *>(dst + (size_t)(r0 + r) * nnz + u * 4) = h4{row[idx.x], row[idx.y], row[idx.z], row[idx.w]};
+                }
+            }
         __syncthreads();
     }
 }
@@ -598,11 +626,19 @@ int et_gather_cols_f16(et_f16 *dst, const et_f16 *X, const int32_t *col_id, int 
     size_t blocks = (total + 255) / 256;
     if (blocks > 4096) blocks = 4096;
     if (in % 8 == 0 && in <= 16384 && (reinterpret_cast<uintptr_t>(X) & 15) == 0) {
-        // about 16 KB of rows a workgroup, so that several of them share a CU whatever the row length
-        const int rows = std::max(1, std::min(8, 8192 / in));
+        // At most 16 KB of rows a workgroup, so that several of them share a CU whatever the row length; of those as many as leave
+        // four workgroups to a CU, up to 4 (one workgroup alone on its CU has nothing to cover its round trips), but with few columns kept
+        // as many as it takes to give every lane some.
+        const int lanes = std::min(nnz_col / 4, 256);
+        const int rows = std::max(1, std::min({8, 8192 / in, std::max(std::min(T / 1024, 4), 256 / lanes)}));
         const unsigned groups = (unsigned)std::min<size_t>(((size_t)T + rows - 1) / rows, 2048);
-        gather_cols_staged_kernel<<<groups, 256, (size_t)rows * in * sizeof(_Float16), as_stream(stream)>>>(
-            H(dst), H(X), col_id, T, in, nnz_col, rows);
+        const size_t lds = (size_t)rows * in * sizeof(_Float16);
+        const int loads = (rows * in / 8 + 255) / 256;
+        auto kernel = gather_cols_staged_kernel<4>;
+        if (loads <= 1) kernel = gather_cols_staged_kernel<1>;
+        else if (loads == 2) kernel = gather_cols_staged_kernel<2>;
+        else if (loads == 3) kernel = gather_cols_staged_kernel<3>;
+        kernel<<<groups, 256, lds, as_stream(stream)>>>(H(dst), H(X), col_id, T, in, nnz_col, rows, lanes);
         return check_launch("gather_cols_staged_kernel");
     }
     gather_cols_kernel<<<(unsigned)blocks, 256, 0, as_stream(stream)>>>(H(dst), H(X), col_id, T, in, nnz_col);

@@ -255,6 +255,26 @@ def test_gather_cols_is_exact(et, T, inp, sp):
     assert np.array_equal(d_ws.numpy(), x[:, col_id])
 
 
+@pytest.mark.parametrize("T,inp,kept", [
+    (3, 16, 8),           # two lanes to a row, 128 rows a workgroup has no use for
+    (2049, 1024, 512),    # one chunk a lane, two rows a workgroup, the last workgroup one
+    (3073, 1000, 1000),   # two chunks a lane, three rows: 250 lanes pick, the others only stage
+    (8195, 800, 104),     # four chunks a lane, eight rows, all of them picked at a time
+    (50, 768, 80),        # three chunks a lane
+    (4100, 4096, 1032),   # more workgroups than are launched, more columns than four a thread
+    (2, 16384, 8192),     # the longest staged row: two turns of four chunks
+])
+def test_gather_cols_staged_edges(et, T, inp, kept):
+    """The staged gather where its rows, lanes and chunks do not come out even: every bit pattern, NaN and infinity included."""
+    rng = np.random.default_rng(T + kept)
+    col_id = np.sort(rng.permutation(inp)[:kept]).astype(np.int32)
+    x = rng.integers(0, 1 << 16, (T, inp), dtype=np.uint16).view(np.float16)
+    d_x, d_col = up(et, x), up(et, col_id)
+    d_ws = et.DeviceBuffer.empty((T, kept), np.float16)
+    et.check(et.lib().et_gather_cols_f16(d_ws.ptr, d_x.ptr, d_col.ptr, T, inp, kept, None))
+    assert np.array_equal(d_ws.numpy().view(np.uint16), x[:, col_id].view(np.uint16))
+
+
 @pytest.mark.parametrize("T,inp,out,sp,act", [(2048, 768, 768, 0.8, 0), (128, 768, 3072, 0.5, 2), (16, 32, 16, 0.0, 0),
                                               (80, 3072, 64, 0.9, 1)])
 def test_linear_vec1x16(et, T, inp, out, sp, act):
