@@ -23,6 +23,7 @@
 #include <mutex>
 
 #include "gemm.hip.h"
+#include "gemm_forms.h"
 
 namespace et {
 
@@ -273,23 +274,15 @@ __global__ __launch_bounds__(256) void gemm_skinny_kernel(const GemmArgs g) {
     }
 }
 
-// The small-result kernel applies when 64 x 64 tiles would leave most of the chip idle: up to 1024 tiles of 16 x 16, from a depth of
-// 784 on up to 640 (us, this kernel / the direct-to-LDS kernel: 672 tiles of 704 4.5 / 5.6, 990 of 528 5.4 / 6.0, 513 of 1056 6.5 / 7.7, 558
-// of 2096 10.2 / 12.3, 384 of 3072 8.5 / 13.8; 1043 of 864 9.3 / 7.3, 860 of 1632 12.9 / 9.7, 1536 of 768 6.8 / 6.1, 1760 of 320
-// 4.9 / 4.6).  Operands that kernel does not take (a result off its alignment, as
-// a row-pruned Linear may be given) would fall to the register-staged kernel, so there the line lies at 2048: 512 x 3072 -> 528 scattered
-// 20.0 / 37.4, 1024 x 1536 -> 448 14.3 / 23.1, 1024 x 4096 -> 448 29.2 / 46.7.  (Batched problems do not come near it:
-// with more than 640 tiles each, four of them have more than 128 of 64 x 64.)
+// (where it is the faster one: takes_small_result)
 static bool gemm_skinny_applies(const GemmArgs &g, int batch, bool trans_b) {
     const auto misaligned = [](const void *p, int a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) != 0; };
     if (!trans_b || g.a_gather || batch < 1 || batch > 65535) return false;
-    if (g.M <= 0 || g.M % 16 || g.N % 16 || g.K % 16 || g.K < 256) return false;
+    if (g.M <= 0 || g.M % 16 || g.N % 16 || g.K % 16) return false;
     if (g.lda % 8 || g.ldb % 8 || misaligned(g.A, 16) || misaligned(g.B, 16)) return false;
     if (!g.c_scatter && (g.ldc % 4 || misaligned(g.C, 8))) return false;
     if (batch > 1 && (((g.sAo | g.sAi | g.sBo | g.sBi) & 7) || ((g.sCo | g.sCi) & 3))) return false;
-    const long long tiles64 = (long long)((g.M + 63) / 64) * ((g.N + 63) / 64) * batch;
-    const long long tiles16 = (long long)(g.M / 16) * (g.N / 16);
-    return tiles64 < 128 && tiles16 <= (!gemm_dma_applies(g, batch, trans_b) ? 2048 : g.K > 768 ? 640 : 1024);
+    return takes_small_result(g.M, g.N, g.K, batch, gemm_dma_applies(g, batch, trans_b));
 }
 
 // C[r][c] = act(bias[c]) for the columns a row-pruned weight does not produce.

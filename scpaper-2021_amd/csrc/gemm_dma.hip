@@ -18,10 +18,10 @@
 // 4 consecutive features of one row of C per 8-row group of a tile; the epilogue transposes
 // through LDS to store whole row segments.
 #include "gemm.hip.h"
+#include "gemm_forms.h"
 
 namespace et {
 
-constexpr int kDmaK = 64;                // K per stage: one 128-byte line of every row
 constexpr int kDmaXcds = 8;
 constexpr int kSbM = 4, kSbN = 8;        // tile block one XCD works on at a time
 constexpr size_t dma_lds_bytes(int tmw, int tnw, int nbuf, int ks = kDmaK, int nwn = 2) {  // buffers of (BM + BN) rows of ks k-values
@@ -504,58 +504,6 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(const GemmArgs 
     }
 }
 
-// Tile choice: the form with the least time by what each was measured to take, in ns: `start` and `depth` per 64 of depth once,
-// `round` and `stage` per 64 of depth for every workgroup a compute unit gets (256 units).  Fitted to 123 Linears of 16..8192
-// rows, 208..4096 wide, multiples of 16 and of 64, with and without GELU, eight sets of buffers in turn: each
-// form within 9-15 % of its time, the choice 1.1 % slower than the best form in the mean (19 % at worst, 8192 x 256 -> 1024).
-// Against forms with one slice of fragments ahead, activations chosen per value and loads past the end (us, mean of no
-// activation and GELU): 2048 x 768 -> 3072 20.7 -> 16.0 (128 x 192 tiles), 768 8.8 -> 7.5 and 2048 x 3072 -> 768 22.3 -> 18.2 (128 x 64),
-// 4096 x 3072 -> 768 40.6 -> 32.0 (64 x 192), 8192 x 3072 -> 768 62.6 -> 47.6, 2048^3 27.9 -> 22.8 (128 x 128), 528 x 768 -> 3072 11.1 -> 7.9,
-// 1024 x 4096^2 62.2 -> 42.0.  Two buffers, several workgroups to a unit, where a short depth leaves mostly epilogues: 6448 x 1568 ->
-// 1040 54.9 -> 35.6 (41.1 with four).  128 x 192 tiles with a fourth buffer, which take all of the LDS, and 128 x 256 with eight waves were up
-// to 40 % slower on operands out of the caches than in them (2048 x 384 -> 3072 10.2 and 14.8, this form 10.8).
-struct DmaTile { int tmw, tnw, nbuf; bool ragged; };
-struct DmaForm { int tmw, tnw, nbuf, start, depth, round, stage; };  // tiles of 64 tmw x 64 tnw
-constexpr DmaForm kDmaForms[] = {
-    {1, 1, 4, 2000, 30, 1150, 209}, {2, 1, 4, 250, 0, 3250, 330}, {1, 2, 4, 200, 0, 3300, 336}, {2, 2, 4, 0, 0, 4800, 490},
-    {1, 3, 4, 0, 0, 4400, 430},     {2, 3, 3, 0, 0, 6100, 605},   {2, 2, 2, 900, 300, 2600, 440}, {2, 1, 2, 1500, 340, 1300, 275},
-    {4, 4, 4, 0, 0, 8200, 1220},
-};
-static bool pick_dma_tile(const GemmArgs &g, int batch, bool trans_b, DmaTile *out) {
-    if (g.M % 16 || g.N % 16 || g.K % 16) return false;
-    if (batch != 1 || !trans_b) {
-        // Batched problems and B stored k-major run on 64 x 64 tiles where they are
-        // bound by the latency of a long K loop in few workgroups (the stacked VO product of the
-        // pre-computed-VO attention: 32 -> 22 us); gathering the k-major fragments with 2-byte LDS
-        // reads costs more than it saves elsewhere (Linear_VO 28 -> 78 us), those stay on the
-        // register-staged kernel.
-        const long long w = (long long)((g.M + 63) / 64) * ((g.N + 63) / 64) * batch;
-        if (w > 256 || g.K / kDmaK < 16) return false;
-        *out = {1, 1, trans_b ? 4 : g.K / kDmaK < 24 ? 2 : 3, true};
-        return true;
-    }
-    // Ragged edges and so many tiles of 256 x 256 that their last round hardly counts: four waves of 128 x 128 (16368 x 8192^2 1980 us
-    // against 2380 in tiles of 128 x 192, 8176^3 1134 / 1400; 512 such tiles, 8176 x 4080^2, 330 / 325).
-    if ((g.M % 64 || g.N % 64 || g.K % kDmaK) && (long long)((g.M + 255) / 256) * ((g.N + 255) / 256) >= 1024) {
-        *out = {4, 4, 2, true};
-        return true;
-    }
-    long long best = -1;
-    const long long stages = (g.K + kDmaK - 1) / kDmaK;
-    for (const DmaForm &f : kDmaForms) {
-        const int bm = 64 * f.tmw, bn = 64 * f.tnw;
-        const bool whole = g.M % bm == 0 && g.N % bn == 0 && g.K % kDmaK == 0;
-        if (f.tmw == 4 && !whole) continue;  // (written for whole tiles)
-        const long long wgs = (long long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn), rounds = (wgs + 255) / 256;
-        const long long ns = f.start + stages * f.depth + rounds * (f.round + stages * f.stage);
-        if (best < 0 || ns < best) {
-            best = ns;
-            *out = {f.tmw, f.tnw, f.nbuf, !whole};
-        }
-    }
-    return true;
-}
-
 // The kernel moves 16 bytes at a time: operands and result 16-byte aligned, leading dimensions
 // multiples of 8.
 bool gemm_dma_applies(const GemmArgs &g, int batch, bool trans_b) {
@@ -565,7 +513,7 @@ bool gemm_dma_applies(const GemmArgs &g, int batch, bool trans_b) {
     if (g.lda % 8 || g.ldb % 8 || g.ldc % 8 || misaligned(g.A) || misaligned(g.B) || misaligned(g.C)) return false;
     if (g.lda > (1 << 21) || g.ldb > (1 << 21)) return false;  // a tile's rows are addressed with 32-bit byte offsets
     if (batch > 1 && ((g.sAo | g.sAi | g.sBo | g.sBi | g.sCo | g.sCi) & 7)) return false;  // every problem aligned
-    return pick_dma_tile(g, batch, trans_b, &t);
+    return pick_dma_tile(g.M, g.N, g.K, batch, trans_b, &t);
 }
 
 template <int TMW, int TNW, int NBUF, bool IDX, bool RAGGED, bool BT = false, int KS = kDmaK, int NWN = 2>
@@ -607,7 +555,7 @@ static int launch_dma_tile(const GemmArgs &g, int batch, hipStream_t stream) {
 
 int launch_gemm_dma(const GemmArgs &g, int batch, bool trans_b, hipStream_t stream) {
     DmaTile t{};
-    if (!pick_dma_tile(g, batch, trans_b, &t)) return ET_ERR_UNSUPPORTED;
+    if (!pick_dma_tile(g.M, g.N, g.K, batch, trans_b, &t)) return ET_ERR_UNSUPPORTED;
     if (!trans_b)
         return t.nbuf == 3 ? launch_dma_tile<1, 1, 3, true, true>(g, batch, stream)
                            : launch_dma_tile<1, 1, 2, true, true>(g, batch, stream);

@@ -41,8 +41,8 @@ def test_linear_dense(et, T, inp, out, act):
     assert Hn.max_abs(d_y.numpy(), want) <= 4e-3
 
 
-# Every tile of the direct-to-LDS kernel, by the rule that chooses them: whole, with ragged edges, with one stage of depth,
-# and with a last stage of 16 or 48 k-values.  (T, inp, out)
+# Every tile of the direct-to-LDS kernel, by the rule that chooses them (test_launch_forms.py asks it): whole, with ragged
+# edges, with one stage of depth, and with a last stage of 16 or 48 k-values.  (T, inp, out)
 DMA_FORMS = [(64, 128, 192), (64, 64, 64), (64, 176, 64), (400, 16, 16), (64, 128, 16),  # 64 x 64
              (448, 320, 4224), (320, 64, 5504), (272, 80, 6096), (288, 192, 5648), (1216, 192, 1728), (336, 400, 5696),  # 64 x 128, 192
              (768, 128, 1408), (5504, 64, 192), (144, 80, 5824), (5696, 48, 144), (5488, 128, 144),  # 128 x 64, two buffers
@@ -62,11 +62,11 @@ def test_linear_dense_and_row_pruned_in_every_tile(et, T, inp, out):
     product = (Hn.f32(x).double() @ Hn.f32(W).double().T).numpy()
     b64 = b.astype(np.float64)
     d_W, d_b, d_x, d_ids = up(et, W), up(et, b), up(et, x), up(et, ids)
-    d_y = et.DeviceBuffer.empty((T, out), np.float16)
+    d_y = up(et, np.full((T, out), np.nan, np.float16))
     et.linear_dense(d_W, d_b, d_x, d_y, T, inp, out, 0)
     want = product + b64[:out]
     assert (np.abs(d_y.numpy() - want) <= 2.0 ** -11 * np.abs(want) + 5e-4).all()
-    d_s = et.DeviceBuffer.empty((T, 2 * out), np.float16)
+    d_s = up(et, np.full((T, 2 * out), np.nan, np.float16))
     et.check(et.lib().et_linear_rowpruned_f16(d_W.ptr, d_ids.ptr, out, d_b.ptr, d_x.ptr, d_s.ptr, T, inp, 2 * out, 1, None))
     want = np.repeat(b64[None], T, 0)
     want[:, ids] += product
@@ -270,7 +270,7 @@ def test_gather_cols_staged_edges(et, T, inp, kept):
     col_id = np.sort(rng.permutation(inp)[:kept]).astype(np.int32)
     x = rng.integers(0, 1 << 16, (T, inp), dtype=np.uint16).view(np.float16)
     d_x, d_col = up(et, x), up(et, col_id)
-    d_ws = et.DeviceBuffer.empty((T, kept), np.float16)
+    d_ws = up(et, ~x[:, col_id].view(np.uint16))
     et.check(et.lib().et_gather_cols_f16(d_ws.ptr, d_x.ptr, d_col.ptr, T, inp, kept, None))
     assert np.array_equal(d_ws.numpy().view(np.uint16), x[:, col_id].view(np.uint16))
 

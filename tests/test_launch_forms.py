@@ -1,0 +1,38 @@
+"""The rules that choose a kernel's form (csrc/*_forms.h), asked on the host: what the tests of the forms claim to run, and
+where the lines between them lie."""
+import subprocess
+from pathlib import Path
+
+import pytest
+
+from tests import test_gpu_linear_formats as linear
+
+ROOT = Path(__file__).resolve().parent.parent
+
+
+@pytest.fixture(scope="module")
+def ask(tmp_path_factory):
+    exe = tmp_path_factory.mktemp("forms") / "launch_forms"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-I", str(ROOT / "scpaper-2021_amd" / "csrc"),
+                    str(ROOT / "tests" / "cpp" / "launch_forms.cpp"), "-o", str(exe)], check=True)
+
+    def answers(questions):
+        res = subprocess.run([str(exe)], input="\n".join(questions) + "\n", capture_output=True, text=True, check=True)
+        out = res.stdout.splitlines()
+        assert len(out) == len(questions)
+        return out
+
+    return answers
+
+
+def gemm(T, inp, out, batch=1, trans_b=1, dma=1):
+    return f"gemm {T} {out} {inp} {batch} {trans_b} {dma}"
+
+
+def test_the_dense_tests_run_every_tile(ask):
+    got = ask([gemm(*shape) for shape in linear.DMA_FORMS])
+    tiles = [(1, 1, 4), (2, 1, 4), (1, 2, 4), (2, 2, 4), (1, 3, 4), (2, 3, 3), (2, 2, 2), (2, 1, 2)]
+    forms = {f"tile {a} {b} {n} {ragged}" for a, b, n in tiles for ragged in (0, 1)} | {"tile 4 4 4 0", "tile 4 4 2 1"}
+    assert forms - set(got) == {"tile 4 4 2 1"}  # (256 x 256 with ragged edges: test_linear_dense, 8176 x 80 -> 8208)
+    assert set(got) - forms == set()
+    assert ask([gemm(8176, 80, 8208)]) == ["tile 4 4 2 1"]
