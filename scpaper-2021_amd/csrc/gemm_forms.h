@@ -35,9 +35,12 @@ inline bool pick_dma_tile(int M, int N, int K, int batch, bool trans_b, DmaTile 
         *out = {1, 1, trans_b ? 4 : K / kDmaK < 24 ? 2 : 3, true};
         return true;
     }
-    // Ragged edges and so many tiles of 256 x 256 that their last round hardly counts: four waves of 128 x 128 (16368 x 8192^2 1980 us
-    // against 2380 in tiles of 128 x 192, 8176^3 1134 / 1400; 512 such tiles, 8176 x 4080^2, 330 / 325).
-    if ((M % 64 || N % 64 || K % kDmaK) && (long long)((M + 255) / 256) * ((N + 255) / 256) >= 1024) {
+    // So many tiles of 256 x 256 that their last round hardly counts, but not all of them whole (the form of whole ones is among those
+    // below): four waves of 128 x 128 (16368 x 8192^2 1980 us against 2380 in tiles of 128 x 192, 8176^3 1134 / 1400; 512 such
+    // tiles, 8176 x 4080^2, 330 / 325).  Edges of 64 are whole in the smaller tiles, which a short depth then leaves ahead: 16320 x 8192^2 1850 /
+    // 2300, 8128 x 4096 -> 8192 484 / 592, 16320 x 256 -> 4096 60 / 64, of 64 inputs 38.5 / 36.8.
+    const bool ragged64 = M % 64 || N % 64 || K % kDmaK, ragged256 = M % 256 || N % 256;
+    if ((ragged64 || (ragged256 && K >= 256)) && (long long)((M + 255) / 256) * ((N + 255) / 256) >= 1024) {
         *out = {4, 4, 2, true};
         return true;
     }

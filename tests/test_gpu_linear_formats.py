@@ -32,7 +32,9 @@ up = Hn.up
                                            # the largest results that kernel takes: 2048 tiles of 16 x 16
                                            (512, 768, 1024, 2), (128, 768, 2304, 0), (448, 784, 720, 1),
                                            # edges of 16 with enough work for the 128 x 64 and 128 x 128 tiles
-                                           (2048, 768, 2928, 2), (2000, 720, 2096, 1), (4080, 208, 4112, 0), (8176, 80, 8208, 1)])
+                                           (2048, 768, 2928, 2), (2000, 720, 2096, 1), (4080, 208, 4112, 0), (8176, 80, 8208, 1),
+                                           # edges of 64, but not of 256, in tiles of 256 x 256
+                                           (16320, 256, 4096, 0)])
 def test_linear_dense(et, T, inp, out, act):
     W, b, x = Hn.randn((out, inp), 1, 0.02), Hn.randn((out,), 2, 0.1), Hn.randn((T, inp), 3)
     d_y = et.DeviceBuffer.empty((T, out), np.float16)

@@ -36,3 +36,10 @@ def test_the_dense_tests_run_every_tile(ask):
     assert forms - set(got) == {"tile 4 4 2 1"}  # (256 x 256 with ragged edges: test_linear_dense, 8176 x 80 -> 8208)
     assert set(got) - forms == set()
     assert ask([gemm(8176, 80, 8208)]) == ["tile 4 4 2 1"]
+
+
+def test_large_dense_problems_keep_tiles_of_256(ask):
+    """Edges that are multiples of 64 but not of 256 leave the form of whole tiles as edges of 16 do."""
+    large = [(16384, 8192, 8192), (16368, 8192, 8192), (16320, 8192, 8192), (16384, 8192, 8128), (16320, 256, 4096), (8128, 4096, 8256)]
+    assert ask([gemm(*shape) for shape in large]) == ["tile 4 4 4 0"] + ["tile 4 4 2 1"] * 5
+    assert not any(a.startswith("tile 4 4") for a in ask([gemm(16320, 64, 4096), gemm(8128, 4096, 4032)]))  # too shallow; too few
