@@ -294,7 +294,11 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(const GemmArgs 
     // in issue order: "stage s + 1 has landed" is "at most the loads of the stages after it
     // are outstanding".
     constexpr int kAhead = NBUF - 1;
-    constexpr bool kDeep = kWhole && NBUF == 4 && NWN == 2;
+    // Fragments two slices ahead: four waves and four buffers.  The 64 x 64 tile with ragged edges keeps to one slice: its one
+    // MFMA a slice hides little either way, and the deep form asks for a stage half a stage later (719 of 728 ragged Linears of 16..2048
+    // rows slower, by 1 to 9 %: 784 x 3072 -> 768 15.9 us deep, 14.6 so, 400 x 4096 -> 1024 19.0 and 18.0; whole tiles are 8 % slower
+    // the other way, 1024 x 4096 -> 1024 18.0 and 19.4).
+    constexpr bool kDeep = kWhole && NBUF == 4 && NWN == 2 && !(RAGGED && TMW * TNW == 1);
     constexpr int kStageLoads = kWhole ? kLA + kLB : 2 * TMW + 2 * TNW;  // per wave
     auto wait_stages = [&](int later) {  // wait until at most `later` whole stages are outstanding
         if (later <= 0) __builtin_amdgcn_s_waitcnt(wait_vm(0));

@@ -46,6 +46,7 @@ def test_linear_dense(et, T, inp, out, act):
 # Every tile of the direct-to-LDS kernel, by the rule that chooses them (test_launch_forms.py asks it): whole, with ragged
 # edges, with one stage of depth, and with a last stage of 16 or 48 k-values.  (T, inp, out)
 DMA_FORMS = [(64, 128, 192), (64, 64, 64), (64, 176, 64), (400, 16, 16), (64, 128, 16),  # 64 x 64
+             (400, 1040, 1040), (656, 3056, 784),  # the same with every buffer in use, several times over
              (448, 320, 4224), (320, 64, 5504), (272, 80, 6096), (288, 192, 5648), (1216, 192, 1728), (336, 400, 5696),  # 64 x 128, 192
              (768, 128, 1408), (5504, 64, 192), (144, 80, 5824), (5696, 48, 144), (5488, 128, 144),  # 128 x 64, two buffers
              (5504, 320, 192), (144, 176, 5456), (144, 256, 5456),  # 128 x 64, four
