@@ -60,17 +60,25 @@ inline bool pick_dma_tile(int M, int N, int K, int batch, bool trans_b, DmaTile 
     return true;
 }
 
-// The small-result kernel applies when 64 x 64 tiles would leave most of the chip idle: up to 1024 tiles of 16 x 16, from a depth of
-// 784 on up to 640 (us, this kernel / the direct-to-LDS kernel: 672 tiles of 704 4.5 / 5.6, 990 of 528 5.4 / 6.0, 513 of 1056 6.5 / 7.7, 558
-// of 2096 10.2 / 12.3, 384 of 3072 8.5 / 13.8; 1043 of 864 9.3 / 7.3, 860 of 1632 12.9 / 9.7, 1536 of 768 6.8 / 6.1, 1760 of 320
-// 4.9 / 4.6).  Operands that kernel does not take (a result off its alignment, as
+// The small-result kernel (one tile of 16 x 16 a workgroup, K in pieces of 64 over its four waves) applies when 64 x 64 tiles would
+// leave most of the chip idle: up to 768 tiles of 16 x 16, three workgroups to a compute unit; up to 1024 of at most 768 inputs, three
+// pieces a wave, and where the pieces of a wave fill two or more of its rounds of six loads (2817 to 3072 inputs).
+// us, this kernel / the direct-to-LDS kernel, operands in turn: 672 tiles of 3072 inputs 10.7 / 15.3, 704 of 1024 5.9 / 6.9, 726 of 1648
+// 8.5 / 9.6, 864 of 768 5.4 / 6.0, of 3072 12.9 / 14.4; in the mean of Linears with 640 to 768 tiles 0.96 up to 1536 inputs, 1.01 up to 2560, 0.84
+// up to 3072, 0.93 up to 4096; with 768 to 1024 tiles 0.96 of 512 to 768 inputs, 1.08, 1.12 and 1.05 up to 1024, 1280 and 1536, 1.19 up to 2560, 0.96
+// of 2817 to 3072, 1.05 beyond; with 1024 to 1280 tiles 1.07 up to 768, 1.15 to 1.5 beyond.
+// Several problems: 640 tiles each and more than 768 inputs (2 of 480 x 2048 -> 368 15.7 / 10.6, 3 of 736 x 1248 -> 176 12.0 / 7.9, 2 of
+// 192 x 1312 -> 672 7.3 / 7.9; fewer than 1024 inputs the direct-to-LDS kernel does not take).
+// Operands that kernel does not take (a result off its alignment, as
 // a row-pruned Linear may be given) would fall to the register-staged kernel, so there the line lies at 2048: 512 x 3072 -> 528 scattered
-// 20.0 / 37.4, 1024 x 1536 -> 448 14.3 / 23.1, 1024 x 4096 -> 448 29.2 / 46.7.  (Batched problems do not come near it:
-// with more than 640 tiles each, four of them have more than 128 of 64 x 64.)
+// 20.0 / 37.4, 1024 x 1536 -> 448 14.3 / 23.1, 1024 x 4096 -> 448 29.2 / 46.7.
 inline bool takes_small_result(int M, int N, int K, int batch, bool dma_applies) {
     const long long tiles64 = (long long)((M + 63) / 64) * ((N + 63) / 64) * batch;
     const long long tiles16 = (long long)(M / 16) * (N / 16);
-    return K >= 256 && tiles64 < 128 && tiles16 <= (!dma_applies ? 2048 : K > 768 ? 640 : 1024);
+    const int pieces = ((K + 63) / 64 + 3) / 4;  // of a wave
+    const bool full_rounds = K <= 768 || (pieces >= 12 && pieces % 6 == 0);
+    const int most = !dma_applies ? 2048 : batch > 1 && K > 768 ? 640 : full_rounds ? 1024 : 768;
+    return K >= 256 && tiles64 < 128 && tiles16 <= most;
 }
 
 }  // namespace et

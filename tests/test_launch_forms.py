@@ -43,3 +43,13 @@ def test_large_dense_problems_keep_tiles_of_256(ask):
     large = [(16384, 8192, 8192), (16368, 8192, 8192), (16320, 8192, 8192), (16384, 8192, 8128), (16320, 256, 4096), (8128, 4096, 8256)]
     assert ask([gemm(*shape) for shape in large]) == ["tile 4 4 4 0"] + ["tile 4 4 2 1"] * 5
     assert not any(a.startswith("tile 4 4") for a in ask([gemm(16320, 64, 4096), gemm(8128, 4096, 4032)]))  # too shallow; too few
+
+
+def test_small_dense_results(ask):
+    """Three tiles of 16 x 16 a compute unit, four where the pieces of a wave fill its rounds of loads."""
+    small = [(224, 3072, 768), (336, 3072, 768), (256, 784, 768), (512, 256, 512), (352, 768, 704), (176, 1040, 1072), (256, 3088, 768)]
+    assert ask([gemm(*shape) for shape in small]) == ["small"] * len(small)
+    larger = [(352, 3072, 768), (272, 3088, 768), (784, 2816, 256), (272, 784, 768), (528, 256, 512), (1040, 768, 256), (400, 240, 16)]
+    assert "small" not in ask([gemm(*shape) for shape in larger])
+    assert ask([gemm(448, 3088, 1008, dma=0), gemm(512, 3088, 1024, dma=0)]) == ["small", "none"]
+    assert ask([gemm(256, 2048, 640, batch=2), gemm(272, 2048, 640, batch=2)]) == ["small", "tile 1 1 4 1"]
