@@ -7,7 +7,10 @@ namespace et {
 // Tile choice: the form with the least time by what each was measured to take, in ns: `start` and `depth` per 64 of depth once,
 // `round` and `stage` per 64 of depth for every workgroup a compute unit gets (256 units).  Fitted to 123 Linears of 16..8192
 // rows, 208..4096 wide, multiples of 16 and of 64, with and without GELU, eight sets of buffers in turn: each
-// form within 9-15 % of its time, the choice 1.1 % slower than the best form in the mean (19 % at worst, 8192 x 256 -> 1024).
+// form within 9-15 % of its time, the choice 1.1 % slower than the best form in the mean (19 % at worst, 8192 x 256 -> 1024).  The stage
+// of 128 x 192 tiles is that of operands too large for the caches: 600 ns within them, 700 to 790 over 3 and more rounds.  At 605 they were taken
+// where two workgroups of 128 x 128 to a unit are ahead (us, 128 x 192 and that form: 6000 x 3216 -> 2448 135 and 125, 7104 x 2688 -> 2160 112 and
+// 93, 4736 x 2368 -> 3072 92 and 78; 520 Linears of more than 2048 tiles of 16 x 16, 2.3 % slower than the best form in the mean, 1.8 % at 650).
 // Against forms with one slice of fragments ahead, activations chosen per value and loads past the end (us, mean of no
 // activation and GELU): 2048 x 768 -> 3072 20.7 -> 16.0 (128 x 192 tiles), 768 8.8 -> 7.5 and 2048 x 3072 -> 768 22.3 -> 18.2 (128 x 64),
 // 4096 x 3072 -> 768 40.6 -> 32.0 (64 x 192), 8192 x 3072 -> 768 62.6 -> 47.6, 2048^3 27.9 -> 22.8 (128 x 128), 528 x 768 -> 3072 11.1 -> 7.9,
@@ -19,7 +22,7 @@ struct DmaForm { int tmw, tnw, nbuf, start, depth, round, stage; };  // tiles of
 constexpr int kDmaK = 64;  // K per stage: one 128-byte line of every row
 constexpr DmaForm kDmaForms[] = {
     {1, 1, 4, 2000, 30, 1150, 209}, {2, 1, 4, 250, 0, 3250, 330}, {1, 2, 4, 200, 0, 3300, 336}, {2, 2, 4, 0, 0, 4800, 490},
-    {1, 3, 4, 0, 0, 4400, 430},     {2, 3, 3, 0, 0, 6100, 605},   {2, 2, 2, 900, 300, 2600, 440}, {2, 1, 2, 1500, 340, 1300, 275},
+    {1, 3, 4, 0, 0, 4400, 430},     {2, 3, 3, 0, 0, 6100, 650},   {2, 2, 2, 900, 300, 2600, 440}, {2, 1, 2, 1500, 340, 1300, 275},
     {4, 4, 4, 0, 0, 8200, 1220},
 };
 inline bool pick_dma_tile(int M, int N, int K, int batch, bool trans_b, DmaTile *out) {

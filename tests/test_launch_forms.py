@@ -53,3 +53,11 @@ def test_small_dense_results(ask):
     assert "small" not in ask([gemm(*shape) for shape in larger])
     assert ask([gemm(448, 3088, 1008, dma=0), gemm(512, 3088, 1024, dma=0)]) == ["small", "none"]
     assert ask([gemm(256, 2048, 640, batch=2), gemm(272, 2048, 640, batch=2)]) == ["small", "tile 1 1 4 1"]
+
+
+def test_large_dense_problems_share_a_compute_unit(ask):
+    """Several rounds of 128 x 192 tiles on operands out of the caches lose to two workgroups of 128 x 128 a unit; one round of them, and the
+    projections of a stack of 2048 rows, keep them."""
+    several = [(6000, 3216, 2448), (7104, 2688, 2160), (4736, 2368, 3072), (4992, 2384, 2608)]
+    assert all(a.startswith("tile 2 2 2") for a in ask([gemm(*shape) for shape in several]))
+    assert ask([gemm(2048, 768, 3072), gemm(2048, 768, 2304)]) == ["tile 2 3 3 0"] * 2
