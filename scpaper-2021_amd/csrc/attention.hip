@@ -29,6 +29,7 @@
 
 #include <type_traits>
 
+#include "attention_forms.h"
 #include "common.hip.h"
 #include "bsr_packed.hip.h"
 #include "../../include/et_tuning.h"
@@ -488,54 +489,18 @@ template <bool RAGGED> static int launch_mha_pingpong(const MhaArgs &args, hipSt
     return check_launch("mha_pingpong_kernel");
 }
 
-// 4 waves per workgroup and one 16-query tile per wave, whatever the last strip holds: a wave without queries still stages
-// its share of every key block.  (Strips of 2 or 1 waves where 4 leave one half-empty, 12 heads of 64, against 4: 16 x 80 keys 6.8
-// and 5.8 us, 3 x 176 9.0 and 6.1, 16 x 176 25.4 and 10.1, 16 x 528 126 and 38, 16 x 720 193 and 57; one sequence of 16 to 112 keys 5.6-5.9
-// and 4.6-4.8.  Only many sequences of 32 keys keep 2: 768 heads of 32 5.1 and 5.5.)  Larger workgroups stage each key block for more
-// queries and pay once the grid still fills the chip: 8 waves (128 queries) from 256 such
-// workgroups on (2048 keys, 16 x 16 heads: 546 -> 516 us; 128-wide heads 592 -> 570 us) unless they leave more
-// than a seventh more places without queries than 4 do (64 x 12 heads: 80 keys 12.4 -> 11.0, 208 33.1 -> 30.3, but 144 24.0 -> 27.0, 48 7.7 ->
-// 9.6), leave a third of the places on the chip empty in the mean of their rounds (two to a unit; 8 x 12 heads, 656 keys 32.4 -> 35.7, 1296
-// 84.8 -> 93.2, but 528 24.6 -> 21.2, 912 49.0 -> 45.8); under a causal mask heads of 64 take 8 only for whole strips, one or two of them
-// (64 x 12 heads, 128 keys 15.8 -> 15.3) or on a chip nine tenths full (8 x 12 heads, 640 keys 22.4 -> 20.2; 16 x 12, 912 keys 62.8 -> 74.4); and 8
-// waves with two query tiles each (256 queries; every K and V^T fragment read from LDS feeds two
-// MFMAs) from 512 on (-> 464 us; 214 registers, two waves per SIMD).  128-wide heads: the 8-wave
-// form prefetches the next block through registers (565 -> 532 us at 2048 keys, 16 x 8 heads),
-// the two-tile form takes all 256 registers and spills 45, and is still the faster one (503 us).
-// Two tiles on 4 waves lose more to the missing third wave than they save (735 us).
+// The fused attention in the form that mha_form chooses.
 template <int HD, bool COMPACT>
-static int launch_mha(const MhaArgs &args, int B, hipStream_t stream) {
-    (void)B;
-    const int qblocks = args.S / 16;
-    if constexpr (!COMPACT) {
-        const int strips8 = (qblocks + 7) / 8, strips4 = (qblocks + 3) / 4;
-        // The two groups of waves in turn: 256-query strips like the next form, but from 192 of them on (2 x 16 heads, 2048
-        // keys, 256 strips: 58.7 -> 45.2 us; 4 x 12 heads, 1024 keys, 192: 30.3 -> 24.0; with 128 strips 35 -> 41) and from
-        // 512 keys on (512 strips of 512 keys 32.4 either way, of 256 keys 32.3 -> 34): a sequence of one or two blocks
-        // has nothing to take turns with.
-        if (HD == 64 && qblocks % 16 == 0 && args.S >= 512 && (long)args.nbh * (qblocks / 16) >= 192 && !args.mask && args.scale_log2e > 0.0f)
-            return launch_mha_pingpong<false>(args, stream);
-        // The same for other lengths, which pay 4-5 % for their edges, where the strips of 256 leave no more than a tenth more places empty
-        // than strips of 128 and fill the last round of every XCD (32 units) to 85 % (16 x 12 heads: 912 keys 88.2 -> 79.8 us, 1872 296 -> 260,
-        // 2032 331 -> 280; 8 x 16 heads, 1296 keys 113 -> 101; but 8 x 12 heads, 912 keys, three quarters full, 45.8 -> 51.3; causal level or slower).
-        const int strips16 = (qblocks + 15) / 16, units = (args.nbh + kXcds - 1) / kXcds;
-        const long u16 = (long)units * strips16;
-        if (HD == 64 && qblocks % 16 != 0 && args.S >= 768 && !args.causal && !args.mask && args.scale_log2e > 0.0f &&
-            20 * strips16 <= 11 * strips8 && 100 * u16 >= 85 * 32 * ((u16 + 31) / 32))
-            return launch_mha_pingpong<true>(args, stream);
-        // (256 causal keys: 64 x 12 heads 45.3 us in this form, 37 in strips of 64)
-        if (HD == 64 && qblocks % 16 == 0 && (long)args.nbh * (qblocks / 16) >= 512 && !(args.causal && args.S == 256))
-            return launch_mha_nw<(HD == 64 ? HD : 64), COMPACT, 8, 2>(args, stream);
-        if ((HD == 96 || HD == 128) && qblocks % 16 == 0 && (long)args.nbh * (qblocks / 16) >= 512)
-            return launch_mha_nw<(HD == 96 || HD == 128 ? HD : 128), COMPACT, 8, 2>(args, stream);
-        const long u8 = (long)units * strips8;
-        const long places8 = 64 * ((u8 + 63) / 64);
-        const bool takes8 = HD == 64 && args.causal ? qblocks % 8 == 0 && (qblocks <= 16 || 10 * u8 >= 9 * places8)
-                                                    : 7 * strips8 * 8 <= 8 * strips4 * 4 && 10 * u8 * strips4 >= 7 * places8 * strips8 * 2;
-        if (HD >= 64 && (long)args.nbh * strips8 >= 256 && takes8)
-            return launch_mha_nw<HD, COMPACT, 8, 1>(args, stream);
+static int launch_mha(const MhaArgs &args, hipStream_t stream) {
+    const MhaForm f = mha_form(HD, COMPACT, args.S, args.nbh, args.causal, !args.mask && args.scale_log2e > 0.0f);
+    if constexpr (HD == 64 && !COMPACT) {
+        if (f.in_turn) return f.ragged ? launch_mha_pingpong<true>(args, stream) : launch_mha_pingpong<false>(args, stream);
     }
-    if (qblocks == 2 && args.nbh >= 512) return launch_mha_nw<HD, COMPACT, 2, 1>(args, stream);
+    if constexpr (HD >= 64 && !COMPACT) {
+        if (f.tiles == 2) return launch_mha_nw<HD, COMPACT, 8, 2>(args, stream);
+        if (f.waves == 8) return launch_mha_nw<HD, COMPACT, 8, 1>(args, stream);
+    }
+    if (f.waves == 2) return launch_mha_nw<HD, COMPACT, 2, 1>(args, stream);
     return launch_mha_nw<HD, COMPACT, 4, 1>(args, stream);
 }
 
@@ -1281,10 +1246,10 @@ int et_mha_fused_ahead_f16(const et_f16 *Q, const et_f16 *K, const et_f16 *V, in
     args.causal = (flags & ET_MHA_CAUSAL) ? 1 : 0;
     args.v_col_id = nullptr;
     args.v_head_ptr = nullptr;
-    if (hd <= 32) return launch_mha<32, false>(args, B, as_stream(stream));
-    if (hd <= 64) return launch_mha<64, false>(args, B, as_stream(stream));
-    if (hd <= 96) return launch_mha<96, false>(args, B, as_stream(stream));  // (10 heads of 80 as 128 wide: 64 x 128 keys 24.4 -> 19.5 us, 16 x 2048 580 -> 382)
-    if (hd <= 128) return launch_mha<128, false>(args, B, as_stream(stream));
+    if (hd <= 32) return launch_mha<32, false>(args, as_stream(stream));
+    if (hd <= 64) return launch_mha<64, false>(args, as_stream(stream));
+    if (hd <= 96) return launch_mha<96, false>(args, as_stream(stream));  // (10 heads of 80 as 128 wide: 64 x 128 keys 24.4 -> 19.5 us, 16 x 2048 580 -> 382)
+    if (hd <= 128) return launch_mha<128, false>(args, as_stream(stream));
     // Heads up to 224 (200 are the reference example's) and 256 wide: 4 waves share the staging of a 64-key block, each with one
     // 16-query tile; a strip shorter than 64 queries leaves waves without queries, which stage and otherwise idle.
     if (hd <= 224) return launch_mha_nw<224, false, 4, 1>(args, as_stream(stream));
@@ -1409,9 +1374,9 @@ int et_mha_compactv_f16(const et_f16 *Q, const et_f16 *K, const et_f16 *Vc, int 
     args.causal = (flags & ET_MHA_CAUSAL) ? 1 : 0;
     args.v_col_id = v_col_id;
     args.v_head_ptr = v_head_ptr;
-    if (hd <= 32) return launch_mha<32, true>(args, B, as_stream(stream));
-    if (hd <= 64) return launch_mha<64, true>(args, B, as_stream(stream));
-    return launch_mha<128, true>(args, B, as_stream(stream));
+    if (hd <= 32) return launch_mha<32, true>(args, as_stream(stream));
+    if (hd <= 64) return launch_mha<64, true>(args, as_stream(stream));
+    return launch_mha<128, true>(args, as_stream(stream));
 }
 
 

@@ -1,0 +1,74 @@
+// Which form of the fused attention a problem takes: waves of a workgroup, 16-query tiles of a wave, the two groups of waves in turn.
+// Plain C++: a test on the host asks the same rule.
+#pragma once
+
+namespace et {
+
+struct MhaForm {
+    int waves, tiles;       // queries of a workgroup: 16 * waves * tiles
+    bool in_turn, ragged;   // the two groups of waves in turn (8 waves of two tiles); strips that a sequence ends in
+};
+
+// 4 waves per workgroup and one 16-query tile per wave, whatever the last strip holds: a wave without queries still stages
+// its share of every key block.  (Strips of 2 or 1 waves where 4 leave one half-empty, 12 heads of 64, against 4: 16 x 80 keys 6.8
+// and 5.8 us, 3 x 176 9.0 and 6.1, 16 x 176 25.4 and 10.1, 16 x 528 126 and 38, 16 x 720 193 and 57; one sequence of 16 to 112 keys 5.6-5.9
+// and 4.6-4.8.  Only many sequences of 32 keys keep 2: 768 heads of 32 5.1 and 5.5.)
+//
+// Larger workgroups stage each key block for more queries: 8 waves (128 queries) from 256 such workgroups on.  Without a causal mask by
+// the workgroups that the fullest compute unit gets: one of 8 waves takes as long as 1.84 of 4 (heads of 64), 1.94 (96), 1.75 (128), and
+// a unit works through its own one after the other.  (us, 4 and 8 waves: 8 x 12 heads of 64, 704 keys 26.6 and 29.0 with 3 and 2 a unit, 16 x 16, 128 keys
+// 5.7 and 5.1 with 2 and 1, 16 heads, 2048 keys 37.3 and 34.3, 14 x 8 of 128, 1088 keys 120 and 135, 17 x 8 of 128, 640 keys 76 and 68.  Over 700
+// problems of 64 to 2048 keys the choice is 0.2 % (64), 0.4 % (96, 128) behind the better one in the mean and 3 to 8 % at worst.  128-wide heads with
+// one block of keys have no next one to fetch ahead: 8 waves there only where they are one to a unit, 61 x 8 heads, 128 keys 0.94 of their time with 4.)
+// Under a causal mask strips differ in length and even out, so what counts is the last strip, the longest one: 8 waves for
+// whole strips only, always for 128-wide heads (as against 4: 16 x 8 heads, 256 keys 12.8 and 13.7, 14 x 16, 1216 keys, not whole, 253 and 233), which
+// take them also where the last is no emptier than two of 4 and two thirds of the places are taken (10 x 8, 1392 keys 116 and 124),
+// never for 96 (25 x 10 heads of 80, 448 keys 51 and 57; whole strips level), for 64 up to two strips a sequence (64 x 12 heads, 128 keys 15.8
+// -> 15.3) and where they give a unit one and a half to two and a half (1152 keys, 48 heads 0.88 of the time of 4, 896, 72 heads 0.86, 1280, 64
+// heads 0.93; below 1.12 of it, 1152 keys, 36 heads 1.19; above level, 1024, 88 heads 1.18).
+//
+// 8 waves with two query tiles each (256 queries; every K and V^T fragment read from LDS feeds two
+// MFMAs) from 512 on (2048 keys, 16 x 16 heads 516 -> 464 us; 214 registers, two waves per SIMD), unless a causal sequence is one such strip:
+// both of its blocks are multiplied for all of its queries (256 causal keys, heads of 64: 24 to 512 heads 1.26 to 1.9 of the time in smaller strips).
+// Heads of 65 to 96 gain from it throughout (80 x 10: 1792 keys 0.77 of the time of the better of 4 and 8, 256 keys 0.90; causal 0.9 to 1.0, one and
+// two strips a sequence 1.05 to 1.15).  128-wide heads: the 8-wave
+// form prefetches the next block through registers (565 -> 532 us at 2048 keys, 16 x 8 heads); the two-tile form takes all
+// 256 registers and spills 49, level with it at 2048 keys, 2 to 25 % behind it below (not changed here: causal 20 to 60 %).
+// Two tiles on 4 waves lose more to the missing third wave than they save (735 us).
+// HD: head size of the template; nbh: sequences times heads; plain: no additive mask and a positive scale.
+inline MhaForm mha_form(int HD, bool compact, int S, int nbh, bool causal, bool plain) {
+    constexpr int kDies = 8;  // accelerator dies, of 32 compute units; the strips of a (sequence, head) share one
+    const int qblocks = S / 16;
+    if (!compact) {
+        const int strips8 = (qblocks + 7) / 8, strips4 = (qblocks + 3) / 4;
+        // The two groups of waves in turn: 256-query strips like the next form, but from 192 of them on (2 x 16 heads, 2048
+        // keys, 256 strips: 58.7 -> 45.2 us; 4 x 12 heads, 1024 keys, 192: 30.3 -> 24.0; with 128 strips 35 -> 41) and from
+        // 512 keys on (512 strips of 512 keys 32.4 either way, of 256 keys 32.3 -> 34): a sequence of one or two blocks
+        // has nothing to take turns with.
+        if (HD == 64 && qblocks % 16 == 0 && S >= 512 && (long)nbh * (qblocks / 16) >= 192 && plain) return {8, 2, true, false};
+        // The same for other lengths, which pay 4-5 % for their edges, where the strips of 256 leave no more than a tenth more places empty
+        // than strips of 128 and fill the last round of every XCD (32 units) to 85 % (16 x 12 heads: 912 keys 88.2 -> 79.8 us, 1872 296 -> 260,
+        // 2032 331 -> 280; 8 x 16 heads, 1296 keys 113 -> 101; but 8 x 12 heads, 912 keys, three quarters full, 45.8 -> 51.3; causal level or slower).
+        const int strips16 = (qblocks + 15) / 16, units = (nbh + kDies - 1) / kDies;
+        const long u16 = (long)units * strips16;
+        if (HD == 64 && qblocks % 16 != 0 && S >= 768 && !causal && plain && 20 * strips16 <= 11 * strips8 &&
+            100 * u16 >= 85 * 32 * ((u16 + 31) / 32))
+            return {8, 2, true, true};
+        const bool one_causal_strip = HD == 64 && causal && qblocks == 16;
+        if (HD >= 64 && qblocks % 16 == 0 && (long)nbh * (qblocks / 16) >= 512 && !one_causal_strip) return {8, 2, false, false};
+        const long u8 = (long)units * strips8, u4 = (long)units * strips4;  // workgroups of a die
+        bool takes8;
+        if (causal) {
+            const bool whole = qblocks % 8 == 0, as_full = 2 * strips8 == strips4 && 10 * u8 >= 7 * (64 * ((u8 + 63) / 64));
+            takes8 = HD == 128 ? whole || as_full : HD == 64 && whole && (qblocks <= 16 || (u8 > 48 && u8 <= 80));
+        } else {
+            const int cost8 = HD == 64 ? 184 : HD == 96 ? 194 : 175;  // of 8 waves, in hundredths of 4
+            takes8 = HD == 128 && S <= 128 ? u8 <= 32 : cost8 * ((u8 + 31) / 32) <= 100 * ((u4 + 31) / 32);
+        }
+        if (HD >= 64 && (long)nbh * strips8 >= 256 && takes8) return {8, 1, false, false};
+    }
+    if (qblocks == 2 && nbh >= 512) return {2, 1, false, false};
+    return {4, 1, false, false};
+}
+
+}  // namespace et

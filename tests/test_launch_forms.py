@@ -5,6 +5,7 @@ from pathlib import Path
 
 import pytest
 
+from tests import test_gpu_attention_variants as attention
 from tests import test_gpu_linear_formats as linear
 
 ROOT = Path(__file__).resolve().parent.parent
@@ -27,6 +28,11 @@ def ask(tmp_path_factory):
 
 def gemm(T, inp, out, batch=1, trans_b=1, dma=1):
     return f"gemm {T} {out} {inp} {batch} {trans_b} {dma}"
+
+
+def mha(B, S, nh, hd, causal=False, compact=False, plain=True):
+    HD = next(t for t in (32, 64, 96, 128) if hd <= t)
+    return f"mha {HD} {int(compact)} {S} {B * nh} {int(causal)} {int(plain)}"
 
 
 def test_the_dense_tests_run_every_tile(ask):
@@ -61,3 +67,26 @@ def test_large_dense_problems_share_a_compute_unit(ask):
     several = [(6000, 3216, 2448), (7104, 2688, 2160), (4736, 2368, 3072), (4992, 2384, 2608)]
     assert all(a.startswith("tile 2 2 2") for a in ask([gemm(*shape) for shape in several]))
     assert ask([gemm(2048, 768, 3072), gemm(2048, 768, 2304)]) == ["tile 2 3 3 0"] * 2
+
+
+def test_the_ragged_attention_tests_run_what_they_claim(ask):
+    shapes = [s for s in attention.RAGGED_STRIPS if s[3] <= 128]
+    got = dict(zip([s[:5] for s in shapes], ask([mha(*s[:5]) for s in shapes])))
+    assert [s[1] for s in shapes if got[s[:5]] == "turns 1"] == [1296, 1296, 912, 1904, 1296]
+    assert set(got.values()) == {"turns 1", "waves 8 1", "waves 8 2", "waves 4 1", "waves 2 1"}
+    assert got[(16, 80, 16, 64, False)] == got[(16, 112, 16, 128, False)] == got[(2, 1024, 16, 128, False)] == got[(16, 256, 8, 128, True)] == "waves 8 1"
+    assert got[(64, 32, 8, 32, False)] == "waves 2 1"
+    assert got[(40, 512, 16, 88, False)] == "waves 8 2"
+
+
+def test_attention_takes_eight_waves_where_they_save_a_unit_time(ask):
+    eight = [(16, 128, 16, 64), (16, 256, 8, 64), (17, 640, 8, 128), (8, 896, 16, 128), (2, 1024, 16, 128), (64, 224, 16, 64)]
+    four = [(22, 704, 12, 40), (10, 832, 12, 40), (11, 1088, 8, 128), (8, 656, 12, 64), (64, 144, 12, 64), (2, 1024, 10, 80), (44, 128, 16, 128),
+            (1, 2048, 8, 128)]  # (the last: 128 workgroups of 8 waves)
+    causal8 = [(16, 256, 8, 128), (4, 1152, 12, 64), (6, 896, 12, 64), (64, 128, 12, 64), (10, 1392, 8, 128)]
+    causal4 = [(25, 448, 10, 80), (14, 1216, 16, 128), (16, 576, 16, 128), (3, 1152, 12, 64), (8, 896, 12, 64), (40, 256, 10, 96)]
+    assert ask([mha(*s) for s in eight]) == ["waves 8 1"] * len(eight)
+    assert ask([mha(*s) for s in four]) == ["waves 4 1"] * len(four)
+    assert ask([mha(*s, True) for s in causal8]) == ["waves 8 1"] * len(causal8)
+    assert ask([mha(*s, True) for s in causal4]) == ["waves 4 1"] * len(causal4)
+    assert ask([mha(48, 256, 12, 64, True), mha(48, 512, 12, 64, True, plain=False), mha(48, 256, 12, 64)]) == ["waves 8 1", "waves 8 2", "waves 8 2"]
