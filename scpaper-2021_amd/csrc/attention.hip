@@ -500,6 +500,9 @@ static int launch_mha(const MhaArgs &args, hipStream_t stream) {
         if (f.tiles == 2) return launch_mha_nw<HD, COMPACT, 8, 2>(args, stream);
         if (f.waves == 8) return launch_mha_nw<HD, COMPACT, 8, 1>(args, stream);
     }
+    if constexpr (HD == 32) {
+        if (f.waves == 1) return launch_mha_nw<HD, COMPACT, 1, 1>(args, stream);
+    }
     if (f.waves == 2) return launch_mha_nw<HD, COMPACT, 2, 1>(args, stream);
     return launch_mha_nw<HD, COMPACT, 4, 1>(args, stream);
 }

@@ -12,7 +12,15 @@ struct MhaForm {
 // 4 waves per workgroup and one 16-query tile per wave, whatever the last strip holds: a wave without queries still stages
 // its share of every key block.  (Strips of 2 or 1 waves where 4 leave one half-empty, 12 heads of 64, against 4: 16 x 80 keys 6.8
 // and 5.8 us, 3 x 176 9.0 and 6.1, 16 x 176 25.4 and 10.1, 16 x 528 126 and 38, 16 x 720 193 and 57; one sequence of 16 to 112 keys 5.6-5.9
-// and 4.6-4.8.  Only many sequences of 32 keys keep 2: 768 heads of 32 5.1 and 5.5.)
+// and 4.6-4.8.)
+//
+// Many short sequences: 2 waves (1 for heads of 32 and 16 keys) where the chip then holds them in fewer rounds.  A compute unit holds
+// three workgroups of 4 waves (two with a compact V), four of 2 by the LDS (six for heads of 32 by the registers, four with a compact V), eight of 1.
+// us, 4 and fewer: 16 keys, 920 heads of 64 7.5 and 5.9, 1840 13.1 and 11.2, 1536 9.7 and 10.4 (two rounds either way), 1800 heads of 32 6.7 and 4.0;
+// 96 keys, 456 heads of 32 7.7 and 6.8; compact, 16 keys, 896 heads of 64 11.8 and 8.0, 96 keys, 300 11.6 and 8.8, 160 keys, 192 0.76 of the time.
+// Longer than 32 keys only strips that 4 waves leave half empty, and only where all are there at once (96 keys: up to three rounds of 4, heads of 32 with a
+// full V any): 1.05 to 1.2 of the time beyond.  32 keys keep 2 from 512 heads on (768 heads of 40 6.8 and 7.5; 512 to 768 of 64 level), heads of
+// 32 with a compact V always (5.6 and 5.7).
 //
 // Larger workgroups stage each key block for more queries: 8 waves (128 queries) from 256 such workgroups on.  Without a causal mask by
 // the workgroups that the fullest compute unit gets: one of 8 waves takes as long as 1.84 of 4 (heads of 64), 1.94 (96), 1.75 (128), and
@@ -67,7 +75,17 @@ inline MhaForm mha_form(int HD, bool compact, int S, int nbh, bool causal, bool 
         }
         if (HD >= 64 && (long)nbh * strips8 >= 256 && takes8) return {8, 1, false, false};
     }
-    if (qblocks == 2 && nbh >= 512) return {2, 1, false, false};
+    if (HD <= 64 && (qblocks == 1 || qblocks % 4 == 2)) {
+        const auto rounds = [&](int waves, int held) {  // of the chip's 256 units, each holding `held` workgroups
+            return ((long)nbh * ((qblocks + waves - 1) / waves) + 256 * held - 1) / (256 * held);
+        };
+        const long in4 = rounds(4, compact ? 2 : 3), in2 = rounds(2, HD == 32 && !compact ? 6 : 4), in1 = rounds(1, 8);
+        const bool fits = qblocks <= 2 || in2 == 1 || (qblocks == 6 && (in4 <= 3 || (HD == 32 && !compact)));
+        if (HD == 32 && qblocks == 1 && in1 < in4 && (in1 < in2 || (in1 == in2 && in1 > 1))) return {1, 1, false, false};
+        if ((in2 < in4 && fits) || (qblocks == 2 && (compact ? HD == 32 : nbh >= 512))) return {2, 1, false, false};
+    } else if (qblocks == 2 && nbh >= 512 && !compact) {
+        return {2, 1, false, false};
+    }
     return {4, 1, false, false};
 }
 

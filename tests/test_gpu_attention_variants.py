@@ -199,7 +199,12 @@ def test_vo_attention_on_chip_rejects_bad_shapes(et):
         assert call(**bad) in (et.ET_ERR_INVALID_ARG, et.ET_ERR_UNSUPPORTED), bad
 
 
-@pytest.mark.parametrize("B,S,nh,hd,keep", [(2, 128, 12, 64, 0.75), (1, 48, 4, 32, 0.5), (1, 272, 2, 64, 0.25)])
+# the last five: many short sequences, in strips of 2 waves and of 1, and 4 waves where they need no more rounds
+COMPACT_SHAPES = [(2, 128, 12, 64, 0.75), (1, 48, 4, 32, 0.5), (1, 272, 2, 64, 0.25),
+                  (56, 16, 16, 64, 0.75), (25, 96, 12, 64, 0.5), (90, 16, 12, 32, 0.5), (2, 32, 3, 32, 0.75), (32, 16, 16, 64, 0.5)]
+
+
+@pytest.mark.parametrize("B,S,nh,hd,keep", COMPACT_SHAPES)
 def test_compact_v_attention(et, B, S, nh, hd, keep):
     """Attention-aware pruning: V arrives compact with col_id / head_ptr; Z is full width with
     zeros in pruned columns and equals dense attention over V with the pruned columns zeroed."""
@@ -209,7 +214,7 @@ def test_compact_v_attention(et, B, S, nh, hd, keep):
     hp = F.head_ptr(col_id, len(col_id), nh, H)
     assert hp[-1] == len(col_id)
     vc = Hn.randn((T, len(col_id)), 33)
-    lens = np.array([S, S - 7][:B], np.int32)
+    lens = np.array(([S, S - 7] * B)[:B], np.int32)
     d_z = et.DeviceBuffer.empty((T, H), np.float16)
     et.check(et.lib().et_fill_f16(d_z.ptr, T * H, 0x7E00, None))
     et.check(et.lib().et_mha_compactv_f16(up(et, q).ptr, up(et, k).ptr, up(et, vc).ptr, H, H, len(col_id),
@@ -296,6 +301,7 @@ RAGGED_STRIPS = [
     (5, 1296, 16, 64, False, [300, 7, 5, 128, 1281]),  # one block of keys, cut and whole, and three
     (16, 80, 16, 64, False, None), (16, 112, 16, 128, False, None), (2, 1024, 16, 128, False, None), (16, 256, 8, 128, True, None), (3, 176, 12, 64, False, None), (3, 176, 12, 64, True, [176, 3, 17]),
     (3, 16, 4, 64, False, None), (3, 48, 5, 128, True, None), (3, 528, 2, 32, True, None), (64, 32, 8, 32, False, None), (5, 96, 3, 200, False, None),
+    (80, 16, 12, 64, False, None), (150, 16, 12, 32, True, None), (70, 16, 12, 32, False, None), (38, 96, 12, 32, True, None),  # many short sequences
     # heads of 65 to 96 and beyond 128: templates of their own, the latter in blocks of 64 keys
     (3, 208, 4, 80, True, [208, 9, 70]), (3, 272, 3, 96, False, None), (40, 512, 16, 88, False, None), (3, 208, 4, 200, True, [65, 9, 128]),
     (4, 64, 3, 224, False, None), (3, 144, 2, 256, False, [144, 3, 0])]

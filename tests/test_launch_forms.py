@@ -73,7 +73,8 @@ def test_the_ragged_attention_tests_run_what_they_claim(ask):
     shapes = [s for s in attention.RAGGED_STRIPS if s[3] <= 128]
     got = dict(zip([s[:5] for s in shapes], ask([mha(*s[:5]) for s in shapes])))
     assert [s[1] for s in shapes if got[s[:5]] == "turns 1"] == [1296, 1296, 912, 1904, 1296]
-    assert set(got.values()) == {"turns 1", "waves 8 1", "waves 8 2", "waves 4 1", "waves 2 1"}
+    assert set(got.values()) == {"turns 1", "waves 8 1", "waves 8 2", "waves 4 1", "waves 2 1", "waves 1 1"}
+    assert got[(80, 16, 12, 64, False)] == got[(38, 96, 12, 32, True)] == "waves 2 1" and got[(150, 16, 12, 32, True)] == "waves 1 1"
     assert got[(16, 80, 16, 64, False)] == got[(16, 112, 16, 128, False)] == got[(2, 1024, 16, 128, False)] == got[(16, 256, 8, 128, True)] == "waves 8 1"
     assert got[(64, 32, 8, 32, False)] == "waves 2 1"
     assert got[(40, 512, 16, 88, False)] == "waves 8 2"
@@ -90,3 +91,14 @@ def test_attention_takes_eight_waves_where_they_save_a_unit_time(ask):
     assert ask([mha(*s, True) for s in causal8]) == ["waves 8 1"] * len(causal8)
     assert ask([mha(*s, True) for s in causal4]) == ["waves 4 1"] * len(causal4)
     assert ask([mha(48, 256, 12, 64, True), mha(48, 512, 12, 64, True, plain=False), mha(48, 256, 12, 64)]) == ["waves 8 1", "waves 8 2", "waves 8 2"]
+
+
+def test_many_short_sequences_take_the_fewest_rounds(ask):
+    compact = ask([mha(*s[:4], compact=True) for s in attention.COMPACT_SHAPES])
+    assert compact == ["waves 4 1"] * 3 + ["waves 2 1", "waves 2 1", "waves 1 1", "waves 2 1", "waves 4 1"]
+    heads64 = {768: 4, 769: 2, 1024: 2, 1025: 4, 1536: 4, 1537: 2, 2049: 4}
+    assert ask([mha(n, 16, 1, 64) for n in heads64]) == [f"waves {w} 1" for w in heads64.values()]
+    heads32 = {768: 4, 769: 2, 1536: 2, 1537: 1, 2048: 1, 3072: 1}
+    assert ask([mha(n, 16, 1, 32) for n in heads32]) == [f"waves {w} 1" for w in heads32.values()]
+    assert ask([mha(300, 96, 1, 64), mha(400, 96, 1, 32), mha(560, 96, 1, 32), mha(300, 80, 1, 64, compact=True)]) == \
+        ["waves 4 1", "waves 2 1", "waves 4 1", "waves 4 1"]
