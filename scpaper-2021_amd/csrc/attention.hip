@@ -69,11 +69,12 @@ constexpr float kLog2e = 1.4426950408889634f;
 // Keys staged per iteration by a head of up to HD.  Beyond 128 half as many, so that two workgroups share a compute unit (62 KB of LDS for 224
 // columns against 120, and held to 256 registers, which takes no spill): 4 heads of 200, 16 x 2048 keys 818 -> 468 us, 3 x 1680 153 -> 94,
 // 64 x 128 24.1 -> 16.4, 2 x 16 8.6 -> 5.5.  With the 306 registers the allocator takes by itself, and one workgroup, 887, 159, 24.0 and 5.9.
+// (256 columns run in blocks of 128 as well, one workgroup to a unit: mha_wide_blocks.)
 template <int HD> constexpr int mha_key_block() { return HD > 128 ? 64 : kKeyBlock; }
 
-template <int HD>
+template <int HD, int KB = mha_key_block<HD>()>
 struct MhaLds {
-    static constexpr int kKeyBlock = mha_key_block<HD>();
+    static constexpr int kKeyBlock = KB;
     static constexpr int ldk = HD + 8;           // halfs per staged K row
     static constexpr int ldvt = kKeyBlock + 8;   // halfs per staged V^T row
     static constexpr int k_halfs = kKeyBlock * ldk;
@@ -168,6 +169,15 @@ __global__ __launch_bounds__(64 * NW)
     __attribute__((amdgpu_waves_per_eu(HD > 128 ? 2 : mha_three_waves<HD, NW, COMPACT, QT>() ? 3 : 1, HD > 128 ? 2 : mha_three_waves<HD, NW, COMPACT, QT>() ? 3 : 8))) void
     mha_fused_kernel(const MhaArgs a) {
     constexpr bool kCoherentZ = false;
+    constexpr int KB = mha_key_block<HD>();
+    const unsigned block = blockIdx.x;
+#include "attention_body.inc"
+}
+
+// 256 columns in blocks of 128 keys: a workgroup has its compute unit and a wave its SIMD's registers to itself (mha_wide_blocks)
+__global__ __launch_bounds__(256) void mha_wide_kernel(const MhaArgs a) {
+    constexpr int HD = 256, NW = 4, QT = 1, KB = kKeyBlock;
+    constexpr bool COMPACT = false, kCoherentZ = false;
     const unsigned block = blockIdx.x;
 #include "attention_body.inc"
 }
@@ -179,21 +189,22 @@ __global__ __launch_bounds__(64 * NW)
     __attribute__((amdgpu_waves_per_eu(mha_three_waves<HD, NW, false, QT>() ? 3 : 1, mha_three_waves<HD, NW, false, QT>() ? 3 : 8))) void
     mha_fused_ahead_kernel(const MhaArgs a) {
     constexpr bool kCoherentZ = false, COMPACT = false;
+    constexpr int KB = mha_key_block<HD>();
     if (blockIdx.x < a.ahead_blocks) return ahead_of(a);
     const unsigned block = blockIdx.x - a.ahead_blocks;
 #include "attention_body.inc"
 }
 template <int HD, bool COMPACT, int NW> constexpr bool mha_takes_ahead() { return HD <= 64 && !COMPACT && NW >= 4; }
 
-template <int HD, bool COMPACT, int NW, int QT>
+template <int HD, bool COMPACT, int NW, int QT, int KB = mha_key_block<HD>()>
 static int launch_mha_nw(const MhaArgs &args, hipStream_t stream) {
-    void (*kernel)(MhaArgs) = mha_fused_kernel<HD, COMPACT, NW, QT>;
+    void (*kernel)(MhaArgs) = HD == 256 && KB == kKeyBlock ? mha_wide_kernel : mha_fused_kernel<HD, COMPACT, NW, QT>;
     MhaArgs a = args;
     if constexpr (mha_takes_ahead<HD, COMPACT, NW>()) {
         a.ahead_blocks = ahead_blocks(a, 64 * NW);
         if (a.ahead_blocks) kernel = mha_fused_ahead_kernel<HD, NW, QT>;
     }
-    constexpr size_t lds = MhaLds<HD>::bytes;
+    constexpr size_t lds = MhaLds<HD, KB>::bytes;
     if (lds > 64 * 1024) {
         static_assert(!mha_takes_ahead<HD, COMPACT, NW>() || lds <= 64 * 1024, "the attribute is set for one kernel");
         static bool raised = false;
@@ -544,6 +555,7 @@ template <int HD, int NW, int QT>
 __global__ __launch_bounds__(64 * NW) void mha_fuseo_kernel(const MhaArgs a, const FuseOArgs f) {
     constexpr bool COMPACT = false;
     constexpr bool kCoherentZ = true;
+    constexpr int KB = mha_key_block<HD>();
     const unsigned block = blockIdx.x;
 #include "attention_body.inc"
     // ---- arrival.  Z was stored at device scope, and such a store counts as complete only once it has
@@ -1256,6 +1268,7 @@ int et_mha_fused_ahead_f16(const et_f16 *Q, const et_f16 *K, const et_f16 *V, in
     // Heads up to 224 (200 are the reference example's) and 256 wide: 4 waves share the staging of a 64-key block, each with one
     // 16-query tile; a strip shorter than 64 queries leaves waves without queries, which stage and otherwise idle.
     if (hd <= 224) return launch_mha_nw<224, false, 4, 1>(args, as_stream(stream));
+    if (mha_wide_blocks(S, args.nbh)) return launch_mha_nw<256, false, 4, 1, kKeyBlock>(args, as_stream(stream));
     return launch_mha_nw<256, false, 4, 1>(args, as_stream(stream));
 }
 

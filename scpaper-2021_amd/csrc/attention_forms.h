@@ -89,4 +89,12 @@ inline MhaForm mha_form(int HD, bool compact, int S, int nbh, bool causal, bool 
     return {4, 1, false, false};
 }
 
+// Heads of more than 224 columns in blocks of 128 keys instead of 64, which leaves a compute unit room for one workgroup: where it gets
+// no more than one, and the sequence is long enough to fill the blocks.  us, 6 heads of 256, blocks of 64 and 128: 640 keys 34.4 and 32.0, 1824 causal
+// 90.2 and 84.1, 2 x 336 22.0 and 21.2, 2 x 928 50.0 and 48.6; 176 keys 13.1 and 15.5; more workgroups than units, 4 x 1040 1.40 the other way.
+// Heads of up to 224 are level or ahead in blocks of 64 throughout (4 of 200: 2048 keys 88.8 and 89.7).
+inline bool mha_wide_blocks(int S, int nbh) {
+    return S > 192 && (long)((nbh + 7) / 8) * ((S + 63) / 64) <= 32;  // units of a die
+}
+
 }  // namespace et

@@ -1,5 +1,6 @@
 // Asks the rules that choose a kernel's form (csrc/*_forms.h) on the host.  One question a line of the standard input:
 //   gemm M N K batch trans_b dma_applies  ->  small | tile TMW TNW NBUF ragged | none
+//   wide S nbh  ->  keys of a block (heads of more than 224)
 //   mha HD compact S nbh causal plain  ->  waves WAVES TILES | turns ragged
 #include <cstdio>
 #include <cstring>
@@ -21,6 +22,8 @@ int main() {
             const et::MhaForm f = et::mha_form(m, n != 0, k, batch, trans != 0, dma != 0);
             if (f.in_turn) printf("turns %d\n", (int)f.ragged);
             else printf("waves %d %d\n", f.waves, f.tiles);
+        } else if (sscanf(line, "wide %d %d", &m, &n) == 2) {
+            puts(et::mha_wide_blocks(m, n) ? "128" : "64");
         } else {
             fprintf(stderr, "not understood: %s", line);
             return 1;

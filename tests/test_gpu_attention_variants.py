@@ -304,7 +304,8 @@ RAGGED_STRIPS = [
     (80, 16, 12, 64, False, None), (150, 16, 12, 32, True, None), (70, 16, 12, 32, False, None), (38, 96, 12, 32, True, None),  # many short sequences
     # heads of 65 to 96 and beyond 128: templates of their own, the latter in blocks of 64 keys
     (3, 208, 4, 80, True, [208, 9, 70]), (3, 272, 3, 96, False, None), (40, 512, 16, 88, False, None), (3, 208, 4, 200, True, [65, 9, 128]),
-    (4, 64, 3, 224, False, None), (3, 144, 2, 256, False, [144, 3, 0])]
+    (4, 64, 3, 224, False, None), (3, 144, 2, 256, False, [144, 3, 0]),
+    (3, 272, 2, 256, True, [272, 3, 200]), (4, 400, 5, 240, False, None), (12, 208, 6, 256, False, None)]  # 256 wide in blocks of 128 keys, and of 64
 
 
 # One sequence holds no number: its neighbours' rows do not depend on it.

@@ -102,3 +102,10 @@ def test_many_short_sequences_take_the_fewest_rounds(ask):
     assert ask([mha(n, 16, 1, 32) for n in heads32]) == [f"waves {w} 1" for w in heads32.values()]
     assert ask([mha(300, 96, 1, 64), mha(400, 96, 1, 32), mha(560, 96, 1, 32), mha(300, 80, 1, 64, compact=True)]) == \
         ["waves 4 1", "waves 2 1", "waves 4 1", "waves 4 1"]
+
+
+def test_heads_of_256_take_wide_blocks_alone_on_a_unit(ask):
+    assert ask(["wide 640 6", "wide 2048 8", "wide 208 56", "wide 256 64"]) == ["128"] * 4
+    assert ask(["wide 192 6", "wide 2064 8", "wide 256 65", "wide 1040 24"]) == ["64"] * 4
+    used = [f"wide {S} {B * nh}" for B, S, nh, hd, *_ in attention.RAGGED_STRIPS if hd > 224]
+    assert set(ask(used)) == {"64", "128"}
