@@ -239,7 +239,7 @@ static int launch_mha_nw(const MhaArgs &args, hipStream_t stream) {
 // barrier a block and no phases 414, with the groups' waves on the same SIMD 459; row sums by an MFMA against ones, or a
 // priority for either phase: 1-3 % slower.
 // For no additive mask and a positive scale; padded keys and the causal mask are applied to the
-// blocks they cut, and a wave skips the blocks past its last query.  RAGGED: S is a multiple of 16 only; keys past it are
+// blocks they cut, and a wave skips the blocks past its last query.  RAGGED: S is a multiple of 16 only, and no causal mask; keys past S are
 // requested from the last rows and stored as zeros, queries past it are not written, and a wave that has no others only stages.
 constexpr int kPpQ = 256;  // queries of a workgroup
 template <bool RAGGED> __device__ __forceinline__ void mha_pingpong(const MhaArgs &a, unsigned block) {
@@ -264,7 +264,7 @@ template <bool RAGGED> __device__ __forceinline__ void mha_pingpong(const MhaArg
     const int wave_q = qstrip * kPpQ + wave * QT * 16;  // first query of the wave
     int klimit = S;
     if (a.lens) klimit = min(S, max(a.lens[b], 0));
-    if (a.causal) klimit = min(klimit, (qstrip + 1) * kPpQ);
+    if (!RAGGED && a.causal) klimit = min(klimit, (qstrip + 1) * kPpQ);
     const int nblocks = (klimit + kKeyBlock - 1) / kKeyBlock;  // (of 128 whole rows each unless RAGGED)
 
     h8 qf[QT][KS];
@@ -387,11 +387,11 @@ template <bool RAGGED> __device__ __forceinline__ void mha_pingpong(const MhaArg
     };
     auto softmax = [&](int k0) {
         // keys past the limit or past the query: 16 kb + j >= lim (the left side a constant once unrolled)
-        if (k0 + kKeyBlock > klimit || (a.causal && k0 + kKeyBlock > wave_q + 1)) {  // wave-uniform
+        if (k0 + kKeyBlock > klimit || (!RAGGED && a.causal && k0 + kKeyBlock > wave_q + 1)) {  // wave-uniform
 #pragma unroll
             for (int t = 0; t < QT; t++) {
                 int lim = klimit - k0;
-                if (a.causal) lim = min(lim, wave_q + t * 16 + r16 + 1 - k0);
+                if (!RAGGED && a.causal) lim = min(lim, wave_q + t * 16 + r16 + 1 - k0);
                 lim -= 4 * g;
 #pragma unroll
                 for (int kb = 0; kb < kNKB; kb++)
@@ -431,7 +431,7 @@ template <bool RAGGED> __device__ __forceinline__ void mha_pingpong(const MhaArg
         }
     };
     // (a block whose keys all lie past the wave's last query has no part in its result)
-    auto live = [&](int blk) { return (!RAGGED || wave_q < S) && (!a.causal || blk * kKeyBlock < wave_q + QT * 16); };
+    auto live = [&](int blk) { return RAGGED ? wave_q < S : (!a.causal || blk * kKeyBlock < wave_q + QT * 16); };
 
     if (nblocks > 0) {  // uniform over the workgroup
         load(0);

@@ -54,9 +54,10 @@ inline MhaForm mha_form(int HD, bool compact, int S, int nbh, bool causal, bool 
         // 512 keys on (512 strips of 512 keys 32.4 either way, of 256 keys 32.3 -> 34): a sequence of one or two blocks
         // has nothing to take turns with.
         if (HD == 64 && qblocks % 16 == 0 && S >= 512 && (long)nbh * (qblocks / 16) >= 192 && plain) return {8, 2, true, false};
-        // The same for other lengths, which pay 4-5 % for their edges, where the strips of 256 leave no more than a tenth more places empty
-        // than strips of 128 and fill the last round of every XCD (32 units) to 85 % (16 x 12 heads: 912 keys 88.2 -> 79.8 us, 1872 296 -> 260,
-        // 2032 331 -> 280; 8 x 16 heads, 1296 keys 113 -> 101; but 8 x 12 heads, 912 keys, three quarters full, 45.8 -> 51.3; causal level or slower).
+        // The same for other lengths, where the strips of 256 leave no more than a tenth more places empty
+        // than strips of 128 and fill the last round of every die (32 units) to 85 % (16 x 12 heads: 912 keys 98.3 -> 83.5 us, 1872 302 -> 252,
+        // 2032 332 -> 271; 8 x 16 heads, 1296 keys 115 -> 96; but 8 x 12 heads, 912 keys, three quarters full, 45.8 -> 51.3; causal level or
+        // slower, and the form has no code for it, which is 4 % of its time).
         const int strips16 = (qblocks + 15) / 16, units = (nbh + kDies - 1) / kDies;
         const long u16 = (long)units * strips16;
         if (HD == 64 && qblocks % 16 != 0 && S >= 768 && !causal && plain && 20 * strips16 <= 11 * strips8 &&

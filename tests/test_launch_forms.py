@@ -109,3 +109,11 @@ def test_heads_of_256_take_wide_blocks_alone_on_a_unit(ask):
     assert ask(["wide 192 6", "wide 2064 8", "wide 256 65", "wide 1040 24"]) == ["64"] * 4
     used = [f"wide {S} {B * nh}" for B, S, nh, hd, *_ in attention.RAGGED_STRIPS if hd > 224]
     assert set(ask(used)) == {"64", "128"}
+
+
+def test_no_causal_or_masked_problem_takes_turns_with_ragged_strips(ask):
+    """The ragged form in turns has no causal limits, and neither form adds a mask."""
+    shapes = [(B, S, nh, 64) for B in (1, 2, 5, 16) for nh in (12, 16, 31) for S in range(16, 2064, 16)]
+    assert "turns 1" in ask([mha(*s) for s in shapes])
+    assert "turns 1" not in ask([mha(*s, True) for s in shapes])
+    assert not any(a.startswith("turns") for a in ask([mha(*s, plain=False) for s in shapes]))
