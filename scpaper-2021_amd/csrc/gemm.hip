@@ -400,9 +400,10 @@ __global__ __launch_bounds__(256) void gather_cols_kernel(_Float16 *__restrict__
 // the columns kept, 8 are 32 bytes of the staged row apart from lane to lane, an eighth of the LDS banks.
 // Lanes that pick nothing ask for no index (with them 8192 x 768 -> 80 4.28 us, 4.17 without).
 // `lanes` of the workgroup's threads pick from one row, min(nnz / 4, 256).
-// Against 8 rows a workgroup, 8 columns a lane and indices behind the barrier (us, replays of a graph): 128 x 768 -> 384 2.53 -> 2.15, 2048 x 768 ->
-// 384 2.76 -> 2.64, 8192 x 768 -> 384 5.06 -> 4.77, 8192 x 1024 -> 720 6.88 -> 6.37, 2048 x 768 -> 80 2.40 -> 2.33; 8192 rows of which a tenth
-// is kept are level (4.12 and 4.17, 7.07 and 7.11).
+// Against 8 rows a workgroup, 8 columns a lane and indices behind the barrier (us, replays of a graph): 128 x 768 -> 384 2.24 -> 1.86, 2048 x 768 ->
+// 384 2.66 -> 2.51, 8192 x 768 -> 384 4.79 -> 4.62, 8192 x 1024 -> 720 6.70 -> 6.22, 2048 x 768 -> 80 2.15 -> 2.06, 8192 x 4096 -> 408 15.4 -> 14.7.  It costs
+// where 8192 rows keep a tenth or less of 512 to 2048 columns: 8192 x 1024 -> 104 4.48 -> 4.56, 8192 x 2048 -> 104 6.55 -> 6.69, 8192 x 512 -> 56
+// 3.23 -> 3.33; indices asked for first, or behind the chunks' stores, or by the lanes of two or four rows only, cost more there.
 template <int K>
 __global__ __launch_bounds__(256) void gather_cols_staged_kernel(_Float16 *__restrict__ dst,
                                                                  const _Float16 *__restrict__ X,

@@ -1,5 +1,5 @@
 // Dense GEMM for gfx950 on direct-to-LDS loads: C[M x N] = act(A[M x K] * B^T + bias), A and B
-// both K-contiguous (B stored [N x K]), M and N multiples of the tile, K a multiple of 64.
+// both K-contiguous (B stored [N x K]), M, N and K multiples of 16; whole tiles and stages of 64, or ragged edges.
 //
 // The 64x64-per-wave kernel in gemm.hip reads 1 byte of LDS per 32 flops, which at the
 // MFMA peak is the whole bandwidth of the LDS port, and stages through registers; it tops
@@ -12,7 +12,8 @@
 // ds_write costs a third of the rate: the LDS port is then the bound), fragments are read two K slices ahead, and
 // reads and loads are issued between the MFMAs that hide them, in an order fixed in the source.  With two or three buffers
 // (several workgroups to a compute unit, or the 128 x 192 tile) and with eight waves (256 x 256, whole tiles; four waves of 128 x 128 where
-// edges are ragged) fragments are read one slice ahead: another wave, or a slice of 16 MFMAs, covers for it.
+// edges are ragged) fragments are read one slice ahead: another wave, or a slice of 16 MFMAs, covers for it.  So does the 64 x 64 tile with
+// ragged edges, where the deep order lost.
 //
 // The MFMA A operand is the B matrix (output features) and vice versa, so a lane ends with
 // 4 consecutive features of one row of C per 8-row group of a tile; the epilogue transposes
@@ -142,8 +143,8 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(const GemmArgs 
     // reads below, 16 rows apart by one chunk column, spread over all banks with no padding.
     const int lrow = lane >> 3, lpos = lane & 7;
     // K-contiguous operands (kWhole; all but BT): a lane's loads differ between stages only by the stage's k0, so a
-    // load is a scalar base that advances by one line per stage plus a 32-bit lane offset computed once; every stage
-    // issues its loads (past the last stage they fetch the last stage again, into a buffer nobody reads any more),
+    // load is a buffer resource at the tile's first row, the stage's k0 as scalar offset and a 32-bit lane offset computed once; every stage
+    // issues its loads (past the last stage through a resource without records: they touch no memory),
     // which keeps the loads in the block of the multiplications, where they can be placed between them, and the
     // number of outstanding loads the same in every stage.  RAGGED: rows past the end of an operand take the offset
     // of its last row, and the last stage, when K ends inside it, has offsets of its own: chunks past the end of K
@@ -435,7 +436,7 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(const GemmArgs 
     // instruction.  Each wave passes its 32 x WN strips through its own LDS region and stores
     // rows of 2 WN contiguous bytes.
     constexpr int kEpLd = WN + 8;
-    constexpr int kRowChunks = WN / 8;  // 16-byte chunks of a stored row: 4, 8 or 16
+    constexpr int kRowChunks = WN / 8;  // 16-byte chunks of a stored row: 4, 8, 12 or 16
     _Float16 *ep = reinterpret_cast<_Float16 *>(dma_smem) + wave * 32 * kEpLd;
     // Scattered columns are stored one 2-byte element per lane, kScLanes consecutive result
     // columns of one row per group of lanes: ascending c_scatter keeps those stores within a
