@@ -503,7 +503,7 @@ template <bool RAGGED> static int launch_mha_pingpong(const MhaArgs &args, hipSt
 // The fused attention in the form that mha_form chooses.
 template <int HD, bool COMPACT>
 static int launch_mha(const MhaArgs &args, hipStream_t stream) {
-    const MhaForm f = mha_form(HD, COMPACT, args.S, args.nbh, args.causal, !args.mask && args.scale_log2e > 0.0f);
+    const MhaForm f = mha_form(HD, COMPACT, args.S, args.nbh, args.causal, !args.mask && args.scale_log2e > 0.0f, args.lens != nullptr);
     if constexpr (HD == 64 && !COMPACT) {
         if (f.in_turn) return f.ragged ? launch_mha_pingpong<true>(args, stream) : launch_mha_pingpong<false>(args, stream);
     }

@@ -27,7 +27,9 @@ struct MhaForm {
 // a unit works through its own one after the other.  (us, 4 and 8 waves: 8 x 12 heads of 64, 704 keys 26.6 and 29.0 with 3 and 2 a unit, 16 x 16, 128 keys
 // 5.7 and 5.1 with 2 and 1, 16 heads, 2048 keys 37.3 and 34.3, 14 x 8 of 128, 1088 keys 120 and 135, 17 x 8 of 128, 640 keys 76 and 68.  Over 700
 // problems of 64 to 2048 keys the choice is 0.2 % (64), 0.4 % (96, 128) behind the better one in the mean and 3 to 8 % at worst.  128-wide heads with
-// one block of keys have no next one to fetch ahead: 8 waves there only where they are one to a unit, 61 x 8 heads, 128 keys 0.94 of their time with 4.)
+// one block of keys have no next one to fetch ahead: 8 waves there only where they are one to a unit, 61 x 8 heads, 128 keys 0.94 of their time with 4.
+// One workgroup of 8 waves a unit cannot even out sequences of unequal length, two of 4 can: from 449 keys on padded heads of 64 keep 4 there (3 x 12 heads,
+// 640 keys 13.6 and 14.5, 24 layers of 4 x 16, 512 keys 1163 and 1172; on operands that stay in the caches 8 are 0 to 9 % ahead).)
 // Under a causal mask strips differ in length and even out, so what counts is the last strip, the longest one: 8 waves for
 // whole strips only, always for 128-wide heads (as against 4: 16 x 8 heads, 256 keys 12.8 and 13.7, 14 x 16, 1216 keys, not whole, 253 and 233), which
 // take them also where the last is no emptier than two of 4 and two thirds of the places are taken (10 x 8, 1392 keys 116 and 124),
@@ -43,8 +45,8 @@ struct MhaForm {
 // form prefetches the next block through registers (565 -> 532 us at 2048 keys, 16 x 8 heads); the two-tile form takes all
 // 256 registers and spills 49, level with it at 2048 keys, 2 to 25 % behind it below (not changed here: causal 20 to 60 %).
 // Two tiles on 4 waves lose more to the missing third wave than they save (735 us).
-// HD: head size of the template; nbh: sequences times heads; plain: no additive mask and a positive scale.
-inline MhaForm mha_form(int HD, bool compact, int S, int nbh, bool causal, bool plain) {
+// HD: head size of the template; nbh: sequences times heads; plain: no additive mask and a positive scale; padded: sequences of their own lengths.
+inline MhaForm mha_form(int HD, bool compact, int S, int nbh, bool causal, bool plain, bool padded) {
     constexpr int kDies = 8;  // accelerator dies, of 32 compute units; the strips of a (sequence, head) share one
     const int qblocks = S / 16;
     if (!compact) {
@@ -72,7 +74,8 @@ inline MhaForm mha_form(int HD, bool compact, int S, int nbh, bool causal, bool 
             takes8 = HD == 128 ? whole || as_full : HD == 64 && whole && (qblocks <= 16 || (u8 > 48 && u8 <= 80));
         } else {
             const int cost8 = HD == 64 ? 184 : HD == 96 ? 194 : 175;  // of 8 waves, in hundredths of 4
-            takes8 = HD == 128 && S <= 128 ? u8 <= 32 : cost8 * ((u8 + 31) / 32) <= 100 * ((u4 + 31) / 32);
+            const bool uneven = HD == 64 && padded && S > 448 && u8 <= 32;
+            takes8 = uneven ? false : HD == 128 && S <= 128 ? u8 <= 32 : cost8 * ((u8 + 31) / 32) <= 100 * ((u4 + 31) / 32);
         }
         if (HD >= 64 && (long)nbh * strips8 >= 256 && takes8) return {8, 1, false, false};
     }

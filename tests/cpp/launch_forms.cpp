@@ -1,7 +1,7 @@
 // Asks the rules that choose a kernel's form (csrc/*_forms.h) on the host.  One question a line of the standard input:
 //   gemm M N K batch trans_b dma_applies  ->  small | tile TMW TNW NBUF ragged | none
 //   wide S nbh  ->  keys of a block (heads of more than 224)
-//   mha HD compact S nbh causal plain  ->  waves WAVES TILES | turns ragged
+//   mha HD compact S nbh causal plain padded  ->  waves WAVES TILES | turns ragged
 #include <cstdio>
 #include <cstring>
 
@@ -11,15 +11,15 @@
 int main() {
     char line[256];
     while (fgets(line, sizeof line, stdin)) {
-        int m, n, k, batch, trans, dma;  // the six numbers, by their names in the first question
+        int m, n, k, batch, trans, dma, padded;  // the numbers, by their names in the first question
         if (sscanf(line, "gemm %d %d %d %d %d %d", &m, &n, &k, &batch, &trans, &dma) == 6) {
             et::DmaTile t{};
             const bool tile = dma && et::pick_dma_tile(m, n, k, batch, trans != 0, &t);
             if (et::takes_small_result(m, n, k, batch, tile)) puts("small");
             else if (tile) printf("tile %d %d %d %d\n", t.tmw, t.tnw, t.nbuf, (int)t.ragged);
             else puts("none");
-        } else if (sscanf(line, "mha %d %d %d %d %d %d", &m, &n, &k, &batch, &trans, &dma) == 6) {
-            const et::MhaForm f = et::mha_form(m, n != 0, k, batch, trans != 0, dma != 0);
+        } else if (sscanf(line, "mha %d %d %d %d %d %d %d", &m, &n, &k, &batch, &trans, &dma, &padded) == 7) {
+            const et::MhaForm f = et::mha_form(m, n != 0, k, batch, trans != 0, dma != 0, padded != 0);
             if (f.in_turn) printf("turns %d\n", (int)f.ragged);
             else printf("waves %d %d\n", f.waves, f.tiles);
         } else if (sscanf(line, "wide %d %d", &m, &n) == 2) {

@@ -30,9 +30,9 @@ def gemm(T, inp, out, batch=1, trans_b=1, dma=1):
     return f"gemm {T} {out} {inp} {batch} {trans_b} {dma}"
 
 
-def mha(B, S, nh, hd, causal=False, compact=False, plain=True):
+def mha(B, S, nh, hd, causal=False, lens=None, compact=False, plain=True):
     HD = next(t for t in (32, 64, 96, 128) if hd <= t)
-    return f"mha {HD} {int(compact)} {S} {B * nh} {int(causal)} {int(plain)}"
+    return f"mha {HD} {int(compact)} {S} {B * nh} {int(causal)} {int(plain)} {int(lens is not None)}"
 
 
 def test_the_dense_tests_run_every_tile(ask):
@@ -71,7 +71,7 @@ def test_large_dense_problems_share_a_compute_unit(ask):
 
 def test_the_ragged_attention_tests_run_what_they_claim(ask):
     shapes = [s for s in attention.RAGGED_STRIPS if s[3] <= 128]
-    got = dict(zip([s[:5] for s in shapes], ask([mha(*s[:5]) for s in shapes])))
+    got = dict(zip([s[:5] for s in shapes], ask([mha(*s) for s in shapes])))
     assert [s[1] for s in shapes if got[s[:5]] == "turns 1"] == [1296, 1296, 912, 1904, 1296]
     assert set(got.values()) == {"turns 1", "waves 8 1", "waves 8 2", "waves 4 1", "waves 2 1", "waves 1 1"}
     assert got[(80, 16, 12, 64, False)] == got[(38, 96, 12, 32, True)] == "waves 2 1" and got[(150, 16, 12, 32, True)] == "waves 1 1"
@@ -88,6 +88,7 @@ def test_attention_takes_eight_waves_where_they_save_a_unit_time(ask):
     causal4 = [(25, 448, 10, 80), (14, 1216, 16, 128), (16, 576, 16, 128), (3, 1152, 12, 64), (8, 896, 12, 64), (40, 256, 10, 96)]
     assert ask([mha(*s) for s in eight]) == ["waves 8 1"] * len(eight)
     assert ask([mha(*s) for s in four]) == ["waves 4 1"] * len(four)
+    assert ask([mha(4, 512, 16, 64), mha(4, 512, 16, 64, lens=[1]), mha(8, 256, 16, 64, lens=[1])]) == ["waves 8 1", "waves 4 1", "waves 8 1"]
     assert ask([mha(*s, True) for s in causal8]) == ["waves 8 1"] * len(causal8)
     assert ask([mha(*s, True) for s in causal4]) == ["waves 4 1"] * len(causal4)
     assert ask([mha(48, 256, 12, 64, True), mha(48, 512, 12, 64, True, plain=False), mha(48, 256, 12, 64)]) == ["waves 8 1", "waves 8 2", "waves 8 2"]
