@@ -72,6 +72,7 @@ inline bool pick_dma_tile(int M, int N, int K, int batch, bool trans_b, DmaTile 
 // of 2817 to 3072, 1.05 beyond; with 1024 to 1280 tiles 1.07 up to 768, 1.15 to 1.5 beyond.
 // Several problems: 640 tiles each and more than 768 inputs (2 of 480 x 2048 -> 368 15.7 / 10.6, 3 of 736 x 1248 -> 176 12.0 / 7.9, 2 of
 // 192 x 1312 -> 672 7.3 / 7.9; fewer than 1024 inputs the direct-to-LDS kernel does not take).
+// The two add in another order (four partial sums, one chain): 0.5 to 1.4e-5 apart in binary16 results, both 2.07e-4 from binary64.
 // Operands that kernel does not take (a result off its alignment, as
 // a row-pruned Linear may be given) would fall to the register-staged kernel, so there the line lies at 2048: 512 x 3072 -> 528 scattered
 // 20.0 / 37.4, 1024 x 1536 -> 448 14.3 / 23.1, 1024 x 4096 -> 448 29.2 / 46.7.
