@@ -26,7 +26,8 @@ struct MhaForm {
 // the workgroups that the fullest compute unit gets: one of 8 waves takes as long as 1.84 of 4 (heads of 64), 1.94 (96), 1.75 (128), and
 // a unit works through its own one after the other.  (us, 4 and 8 waves: 8 x 12 heads of 64, 704 keys 26.6 and 29.0 with 3 and 2 a unit, 16 x 16, 128 keys
 // 5.7 and 5.1 with 2 and 1, 16 heads, 2048 keys 37.3 and 34.3, 14 x 8 of 128, 1088 keys 120 and 135, 17 x 8 of 128, 640 keys 76 and 68.  Over 700
-// problems of 64 to 2048 keys the choice is 0.2 % (64), 0.4 % (96, 128) behind the better one in the mean and 3 to 8 % at worst.  128-wide heads with
+// problems of 64 to 2048 keys the choice is 0.2 % (64), 0.4 % (96, 128) behind the better one in the mean and 3 to 8 % at worst.  Up to 96 keys, where two
+// or three of the 8 waves have no queries, 1.6 for heads of 64: 54 x 16, 96 keys 13.4 and 15.2, 4 a unit and 7; 3 and 5, 66 x 8, 11.5 and 11.8.  128-wide heads with
 // one block of keys have no next one to fetch ahead: 8 waves there only where they are one to a unit, 61 x 8 heads, 128 keys 0.94 of their time with 4.
 // One workgroup of 8 waves a unit cannot even out sequences of unequal length, two of 4 can: from 449 keys on padded heads of 64 keep 4 there (3 x 12 heads,
 // 640 keys 13.6 and 14.5, 24 layers of 4 x 16, 512 keys 1163 and 1172; on operands that stay in the caches 8 are 0 to 9 % ahead).)
@@ -73,7 +74,7 @@ inline MhaForm mha_form(int HD, bool compact, int S, int nbh, bool causal, bool 
             const bool whole = qblocks % 8 == 0, as_full = 2 * strips8 == strips4 && 10 * u8 >= 7 * (64 * ((u8 + 63) / 64));
             takes8 = HD == 128 ? whole || as_full : HD == 64 && whole && (qblocks <= 16 || (u8 > 48 && u8 <= 80));
         } else {
-            const int cost8 = HD == 64 ? 184 : HD == 96 ? 194 : 175;  // of 8 waves, in hundredths of 4
+            const int cost8 = HD == 64 ? (qblocks <= 6 ? 160 : 184) : HD == 96 ? 194 : 175;  // of 8 waves, in hundredths of 4
             const bool uneven = HD == 64 && padded && S > 448 && u8 <= 32;
             takes8 = uneven ? false : HD == 128 && S <= 128 ? u8 <= 32 : cost8 * ((u8 + 31) / 32) <= 100 * ((u4 + 31) / 32);
         }

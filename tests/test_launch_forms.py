@@ -81,8 +81,9 @@ def test_the_ragged_attention_tests_run_what_they_claim(ask):
 
 
 def test_attention_takes_eight_waves_where_they_save_a_unit_time(ask):
-    eight = [(16, 128, 16, 64), (16, 256, 8, 64), (17, 640, 8, 128), (8, 896, 16, 128), (2, 1024, 16, 128), (64, 224, 16, 64)]
-    four = [(22, 704, 12, 40), (10, 832, 12, 40), (11, 1088, 8, 128), (8, 656, 12, 64), (64, 144, 12, 64), (2, 1024, 10, 80), (44, 128, 16, 128),
+    eight = [(16, 128, 16, 64), (16, 256, 8, 64), (17, 640, 8, 128), (8, 896, 16, 128), (2, 1024, 16, 128), (64, 224, 16, 64),
+             (54, 96, 16, 64), (66, 96, 8, 64), (59, 80, 16, 40)]  # (the last row: two or three waves without queries)
+    four = [(22, 704, 12, 40), (10, 832, 12, 40), (11, 1088, 8, 128), (8, 656, 12, 64), (64, 144, 12, 64), (2, 1024, 10, 80), (44, 128, 16, 128), (54, 128, 16, 64),
             (1, 2048, 8, 128)]  # (the last: 128 workgroups of 8 waves)
     causal8 = [(16, 256, 8, 128), (4, 1152, 12, 64), (6, 896, 12, 64), (64, 128, 12, 64), (10, 1392, 8, 128)]
     causal4 = [(25, 448, 10, 80), (14, 1216, 16, 128), (16, 576, 16, 128), (3, 1152, 12, 64), (8, 896, 12, 64), (40, 256, 10, 96)]
