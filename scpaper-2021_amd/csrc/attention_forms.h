@@ -30,7 +30,9 @@ struct MhaForm {
 // or three of the 8 waves have no queries, 1.6 for heads of 64: 54 x 16, 96 keys 13.4 and 15.2, 4 a unit and 7; 3 and 5, 66 x 8, 11.5 and 11.8.  128-wide heads with
 // one block of keys have no next one to fetch ahead: 8 waves there only where they are one to a unit, 61 x 8 heads, 128 keys 0.94 of their time with 4.
 // One workgroup of 8 waves a unit cannot even out sequences of unequal length, two of 4 can: from 449 keys on padded heads of 64 keep 4 there (3 x 12 heads,
-// 640 keys 13.6 and 14.5, 24 layers of 4 x 16, 512 keys 1163 and 1172; on operands that stay in the caches 8 are 0 to 9 % ahead).)
+// 640 keys 13.6 and 14.5, 24 layers of 4 x 16, 512 keys 1163 and 1172; on operands that stay in the caches 8 are 0 to 9 % ahead).  Padded 128-wide
+// heads, which even out over the rounds too: 8 by the strips of a sequence alone (38 x 8, 448 keys 79.5 and 83.0, 39 x 8, 320 keys 52.4 and
+// 55.6, 3 x 16, 928 keys 54.0 and 47.5; 134 problems of 80 to 1024 keys 0.3 % behind the better one in the mean, 1.0 % by the fullest unit).)
 // Under a causal mask strips differ in length and even out, so what counts is the last strip, the longest one: 8 waves for
 // whole strips only, always for 128-wide heads (as against 4: 16 x 8 heads, 256 keys 12.8 and 13.7, 14 x 16, 1216 keys, not whole, 253 and 233), which
 // take them also where the last is no emptier than two of 4 and two thirds of the places are taken (10 x 8, 1392 keys 116 and 124),
@@ -76,7 +78,8 @@ inline MhaForm mha_form(int HD, bool compact, int S, int nbh, bool causal, bool 
         } else {
             const int cost8 = HD == 64 ? (qblocks <= 6 ? 160 : 184) : HD == 96 ? 194 : 175;  // of 8 waves, in hundredths of 4
             const bool uneven = HD == 64 && padded && S > 448 && u8 <= 32;
-            takes8 = uneven ? false : HD == 128 && S <= 128 ? u8 <= 32 : cost8 * ((u8 + 31) / 32) <= 100 * ((u4 + 31) / 32);
+            takes8 = uneven ? false : HD == 128 && S <= 128 ? u8 <= 32
+                     : HD == 128 && padded ? 182 * strips8 <= 100 * strips4 : cost8 * ((u8 + 31) / 32) <= 100 * ((u4 + 31) / 32);
         }
         if (HD >= 64 && (long)nbh * strips8 >= 256 && takes8) return {8, 1, false, false};
     }

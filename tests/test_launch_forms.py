@@ -90,6 +90,8 @@ def test_attention_takes_eight_waves_where_they_save_a_unit_time(ask):
     assert ask([mha(*s) for s in eight]) == ["waves 8 1"] * len(eight)
     assert ask([mha(*s) for s in four]) == ["waves 4 1"] * len(four)
     assert ask([mha(4, 512, 16, 64), mha(4, 512, 16, 64, lens=[1]), mha(8, 256, 16, 64, lens=[1])]) == ["waves 8 1", "waves 4 1", "waves 8 1"]
+    uneven8, uneven4 = [(3, 928, 16, 128), (11, 496, 8, 128), (13, 1008, 6, 128)], [(38, 448, 8, 128), (39, 320, 8, 128), (52, 288, 8, 128), (271, 96, 6, 128)]
+    assert ask([mha(*s, lens=[1]) for s in uneven8 + uneven4]) == ["waves 8 1"] * 3 + ["waves 4 1"] * 4
     assert ask([mha(*s, True) for s in causal8]) == ["waves 8 1"] * len(causal8)
     assert ask([mha(*s, True) for s in causal4]) == ["waves 4 1"] * len(causal4)
     assert ask([mha(48, 256, 12, 64, True), mha(48, 512, 12, 64, True, plain=False), mha(48, 256, 12, 64)]) == ["waves 8 1", "waves 8 2", "waves 8 2"]
