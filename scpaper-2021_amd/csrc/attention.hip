@@ -502,6 +502,8 @@ template <bool RAGGED> static int launch_mha_pingpong(const MhaArgs &args, hipSt
     return check_launch("mha_pingpong_kernel");
 }
 
+#include "attention_tiles32.inc"
+
 // The fused attention in the form that mha_form chooses.
 template <int HD, bool COMPACT>
 static int launch_mha(const MhaArgs &args, hipStream_t stream) {
@@ -1263,6 +1265,8 @@ int et_mha_fused_ahead_f16(const et_f16 *Q, const et_f16 *K, const et_f16 *V, in
     args.causal = (flags & ET_MHA_CAUSAL) ? 1 : 0;
     args.v_col_id = nullptr;
     args.v_head_ptr = nullptr;
+    int status;
+    if (mha_takes_tiles32(args, as_stream(stream), &status)) return status;
     if (hd <= 32) return launch_mha<32, false>(args, as_stream(stream));
     if (hd <= 64) return launch_mha<64, false>(args, as_stream(stream));
     if (hd <= 96) return launch_mha<96, false>(args, as_stream(stream));  // (10 heads of 80 as 128 wide: 64 x 128 keys 24.4 -> 19.5 us, 16 x 2048 580 -> 382)

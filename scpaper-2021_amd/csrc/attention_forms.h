@@ -105,4 +105,67 @@ inline bool mha_wide_blocks(int S, int nbh) {
     return S > 192 && (long)((nbh + 7) / 8) * ((S + 63) / 64) <= 32;  // units of a die
 }
 
+// ---- products of 32 x 32 x 16 (mha_tiles32_kernel) -------------------------------------------------------
+// `waves` of a workgroup, `split` of which share a tile of 32 queries (each with its part of every staged block of keys), and
+// 32-key steps of a wave a block; 0 waves: none, the forms above.
+struct MhaTiles {
+    int waves, split, steps;
+    constexpr int queries() const { return 32 * (waves / split); }  // of a workgroup
+    constexpr int keys() const { return 32 * steps * split; }       // staged at a time
+};
+// What a form was measured to take, in units of 10 ns: `start` once; a block of keys `chain` where the workgroup is alone on its compute unit, and
+// `block` for every workgroup the fullest unit gets where they fill it; `wg` for each of those once.  Fitted to 400 problems of 80 to 2048 keys, 1 to
+// 64 sequences, causal and padded ones among them, three sets of operands in turn: each form within 5 to 11 % of its time, the
+// choice 0.8 % (heads of 64), 0.3 % (32) to 1 % (128) behind the best form in the mean, and 0.81 (64), 0.85 (32), 0.72 (96), 0.68 (128) and
+// 0.86 (200) times the forms above.  us, the forms above and the choice: 12 heads of 64, 1 x 512 keys 8.9 and 6.5 (a tile's keys
+// over four waves), 3 x 176 6.2 and 5.1, 16 heads, 4 x 512 12.7 and 10.6 (over two), 16 x 2048 349 and 313 (tiles of one wave), causal 274 and 207; 8 heads
+// of 128, 8 x 1024 64 and 42.
+struct MhaTilesCost { MhaTiles form; int start, chain, block, wg; };
+constexpr MhaTilesCost kMhaTiles32[] = {{{4, 1, 2}, 192, 85, 54, 81}, {{4, 2, 2}, 231, 74, 48, 91}, {{4, 4, 1}, 225, 59, 30, 73}};
+constexpr MhaTilesCost kMhaTiles64[] = {{{4, 1, 2}, 108, 88, 54, 221}, {{8, 1, 2}, 120, 127, 111, 154}, {{4, 2, 2}, 157, 106, 64, 177},
+                                        {{8, 2, 2}, 0, 123, 116, 412}, {{4, 4, 1}, 192, 80, 48, 137}};
+constexpr MhaTilesCost kMhaTiles96[] = {{{4, 1, 2}, 0, 124, 76, 377}, {{8, 1, 2}, 0, 147, 156, 376}, {{4, 2, 2}, 48, 155, 134, 362}, {{8, 2, 2}, 0, 154, 160, 547}};
+constexpr MhaTilesCost kMhaTiles128[] = {{{4, 1, 2}, 19, 145, 97, 364}, {{8, 1, 2}, 0, 173, 200, 364}, {{4, 2, 2}, 21, 165, 151, 422}, {{4, 4, 1}, 96, 0, 118, 341}};
+// 129 to 224 columns, where the forms above (64 queries a workgroup, blocks of 64 keys) stay ahead for some: 4 heads of 200, 12 x 48
+// keys 6.3 and 6.7 us
+constexpr MhaTilesCost kMhaTiles224[] = {{{0, 1, 2}, 0, 274, 182, 330}, {{4, 1, 1}, 0, 158, 109, 393}, {{4, 2, 1}, 0, 201, 190, 500},
+                                         {{4, 1, 2}, 0, 250, 279, 412}, {{8, 1, 2}, 0, 112, 354, 359}};
+
+template <int N> inline MhaTiles mha_tiles_least(const MhaTilesCost (&costs)[N], int S, int nbh, bool causal) {
+    long long best = -1;
+    MhaTiles form{};
+    for (const MhaTilesCost &c : costs) {
+        const int q = c.form.waves ? c.form.queries() : 64, keys = c.form.waves ? c.form.keys() : 64, strips = (S + q - 1) / q;
+        long long sum = 0, longest = (S + keys - 1) / keys;  // blocks of all strips, of the longest
+        if (causal)
+            for (int i = 1; i <= strips; i++) sum += ((i * q < S ? i * q : S) + keys - 1) / keys;
+        else
+            sum = longest * strips;
+        const long long units = ((long long)((nbh + 7) / 8) * strips + 31) / 32;  // workgroups of the fullest of a die's 32
+        const long long alone = c.chain * longest * strips, full = c.block * sum * units;
+        const long long t = (long long)(c.start + c.wg * units) * strips * 1000 + (alone > full ? alone : full) * 1000;
+        const long long per = t / strips;
+        if (best < 0 || per < best) {
+            best = per;
+            form = c.form;
+        }
+    }
+    return form;
+}
+// Few short sequences keep the forms above: the one launch of attention and output projection (mha_fuseo_kernel) is made of those, and where it
+// is used the two launches it replaces give the same bits.  (us, the forms above and this kernel: 12 heads of 64, 1 x 128 keys 4.5 and 4.2, 8 x 128 4.7
+// and 4.5, 3 x 176 6.2 and 5.1.)  Otherwise up to 64 keys, one block of them, there is nothing to share (1.0 to 1.3 of the time).
+inline MhaTiles mha_tiles(int HD, int S, int nbh, bool causal) {
+    if (HD <= 128 && S <= 384 && (long long)nbh * ((S + 31) / 32) <= 400) return {};
+    if (HD <= 128 && S <= 64) return {4, 1, 2};
+    switch (HD) {
+        case 32: return mha_tiles_least(kMhaTiles32, S, nbh, causal);
+        case 64: return mha_tiles_least(kMhaTiles64, S, nbh, causal);
+        case 96: return mha_tiles_least(kMhaTiles96, S, nbh, causal);
+        case 128: return mha_tiles_least(kMhaTiles128, S, nbh, causal);
+        case 224: return mha_tiles_least(kMhaTiles224, S, nbh, causal);
+        default: return {};
+    }
+}
+
 }  // namespace et
