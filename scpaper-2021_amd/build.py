@@ -28,6 +28,8 @@ HIPCC = os.environ.get("HIPCC") or shutil.which("hipcc") or "/opt/rocm/bin/hipcc
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-I", str(ROOT / "include"), "-Wall", "-Wno-unused-function"]
 # Packed-fp32 code generation is switched off for device code.
 DEVICE = [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+          # leading scalar arguments of a kernel are in its registers when a wave starts
+          "-mllvm", "-amdgpu-kernarg-preload-count=14",
           "-Wno-unknown-warning-option", "-Wno-unused-command-line-argument",
           "-Rpass-analysis=kernel-resource-usage"]  # registers and scratch of every kernel, kept in RESOURCES
 RESOURCES = LIBDIR / "kernel_resources.txt"

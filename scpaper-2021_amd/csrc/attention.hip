@@ -116,8 +116,8 @@ template <int HD> __device__ __forceinline__ constexpr int vt_unit_keys(int kg) 
 // asks for one line of a weight that the launches behind this one read.  Where weights do not stay in the memory-side
 // cache from one forward to the next, those launches would wait for HBM with every compute unit; here the requests cost
 // a few workgroups' slots, and nobody waits for them but the end of the launch.
-__device__ __forceinline__ void ahead_of(const MhaArgs &a) {
-    unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void ahead_of(const MhaArgs &a, unsigned block) {
+    unsigned i = block * blockDim.x + threadIdx.x;
 #pragma unroll
     for (int s = 0; s < ET_MHA_AHEAD; s++) {
         if (i < a.ahead_lines[s]) {
@@ -192,7 +192,7 @@ __global__ __launch_bounds__(64 * NW)
     mha_fused_ahead_kernel(const MhaArgs a) {
     constexpr bool kCoherentZ = false, COMPACT = false;
     constexpr int KB = mha_key_block<HD>();
-    if (blockIdx.x < a.ahead_blocks) return ahead_of(a);
+    if (blockIdx.x < a.ahead_blocks) return ahead_of(a, blockIdx.x);
     const unsigned block = blockIdx.x - a.ahead_blocks;
 #include "attention_body.inc"
 }
@@ -483,7 +483,7 @@ template <bool RAGGED> __device__ __forceinline__ void mha_pingpong(const MhaArg
 
 template <bool RAGGED> __global__ __launch_bounds__(512) void mha_pingpong_kernel(const MhaArgs a) { mha_pingpong<RAGGED>(a, blockIdx.x); }
 template <bool RAGGED> __global__ __launch_bounds__(512) void mha_pingpong_ahead_kernel(const MhaArgs a) {
-    if (blockIdx.x < a.ahead_blocks) return ahead_of(a);
+    if (blockIdx.x < a.ahead_blocks) return ahead_of(a, blockIdx.x);
     mha_pingpong<RAGGED>(a, blockIdx.x - a.ahead_blocks);
 }
 
