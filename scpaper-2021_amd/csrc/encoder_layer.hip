@@ -62,8 +62,8 @@ constexpr int kElMaxSeg = 24;  // segments of a launch
 constexpr size_t kElLds = 160 * 1024;
 // table of a (part, wave), 64 words, a lane holds one: block-rows of every segment, sums of every wave, slots, and of every chunk of
 // the projection its first block-row (bits 0-15) and their number (worked out in the kernel, four divisions a chunk); and the descriptors
-// of its block-rows, in the same way: one request each at the start, read with v_readlane
-constexpr int kElTabSeg = 0, kElTabCount = kElTabSeg + kElMaxSeg, kElTabSlots = kElTabCount + kElWaves, kElTabOut = kElTabSlots + 1, kElTab = 64, kElRowRegs = 2;
+// of its block-rows behind it, in the same way: one request each at the start, read with v_readlane
+constexpr int kElTabSeg = 0, kElTabCount = kElTabSeg + kElMaxSeg, kElTabSlots = kElTabCount + kElWaves, kElTabOut = kElTabSlots + 1, kElTabWords = 64, kElRowRegs = 2, kElTab = kElTabWords * (1 + kElRowRegs);
 // descriptor: slots (bits 0-7), kind (8-9), operand in the hidden chunk (10), target (11-20), bias over 16 (21-31)
 constexpr int kElBufferWord = 0x00020000;  // of a raw buffer resource
 constexpr int kElKindSum = 0, kElKindHidden = 1, kElKindQkv = 2, kElMaxSlots = 255;
@@ -73,19 +73,10 @@ typedef int i4 __attribute__((ext_vector_type(4)));
 struct LayerArgs {
     // joined launch: the streams behind the join, and a word per strip
     const char *slots2, *offs2;
-    const uint32_t *rows2;
     const int32_t *tab2;
     uint32_t *join;
     int cap2, spin;
     const char *slots;
-    const char *offs;  // per wave and eight slots: 8 x 16 bits of the first tiles' offsets, 8 of the second
-    const uint32_t *rows;  // per (part, wave) 64 kElRowRegs descriptors
-    int cap;               // slots from one (part, wave) to the next
-    const int32_t *tab;
-    const _Float16 *vec;  // bo, g1, be1, b1, b2, g2, be2, bq
-    const _Float16 *Z;
-    const float *x32;     // residual in binary32 and tile order, or
-    const _Float16 *x16;  // in binary16, row by row
     float *x32_out;       // x' in tile order (may be null)
     _Float16 *out16;      // x' rounded (may be null)
     _Float16 *qkv;
@@ -93,13 +84,30 @@ struct LayerArgs {
     int T, H, FF, Q;
     // Tile order: the 16 x 16 values of 16 tokens and a block-row are 1 KiB, a lane's four together, so that a wave reads
     // and writes whole lines of what only these launches exchange
-    int xs, hs;           // bytes of a strip row and of a hidden row in LDS, multiples of 256
+    int hs;               // bytes of a hidden row in LDS, a multiple of 256
     int nseg_ff, nseg_q;  // segments of the hidden features, of the projection
     int hbuf;             // bytes between the two hidden buffers (0: one is enough)
     int parts, nshare, act;  // parts of this launch, shares of the second product
     float eps1, eps2, inv_h;
     uint32_t sums[kElWaves];  // block-rows of the model width a wave holds the sums of, 8 bits each (255: none)
 };
+
+// What the first requests need, in front of the other arguments and one by one: preloaded into scalar registers.  Read from memory, and with
+// divisions for a workgroup's place and its pieces of the strip, a wave had asked for everything 3 400 cycles after it started, of 48 000 (us, before
+// and now, three models in turn: one sequence of 128 tokens 316 and 311, 8 x 128 362 and 357, BERT-large 4 x 512 1109 and 1091, 528 rows 228 and 223).
+struct LayerFirst {
+    const _Float16 *Z;
+    const void *x;       // residual: binary32 in tile order, or binary16 row by row
+    const char *offs;    // per wave and eight slots: 8 x 16 bits of the first tiles' offsets, 8 of the second
+    const int32_t *tab;  // per (part, wave) the table and its descriptors
+    const _Float16 *vec;  // bo, g1, be1, b1, b2, g2, be2, bq
+    int T, H;
+    int cap;             // slots from one (part, wave) to the next
+    unsigned form;       // bytes of a strip row in LDS over 256 (bits 0-7), the residual is binary16 (8), vectors over 8 (16-31)
+};
+#define ET_EL_FIRST const _Float16 *Z, const void *x, const char *offs, const int32_t *tab, const _Float16 *vec, int T, int H, int cap, unsigned form
+constexpr size_t kElFirstBytes = 56;  // of them among the arguments
+static_assert(sizeof(LayerFirst) == kElFirstBytes, "the other arguments follow them");
 
 // The weight ring lives in registers the compiler does not have: v[96:127] hold the next eight slots of the wave,
 // v[88:91] the column offsets of the current eight slots (16 bits each, those of this half of the wave), v[92:95] those of
@@ -267,21 +275,22 @@ struct ElWord {
 // MODE 0: all steps.  1: up to the second product, binary32 share to `partial`.  2: from the sum of the shares on.  3: the
 // projection alone, of x' as 2 rounds it, given in `Z`: the same products in the same order.
 // 4: 1 and 2 in one launch; behind the second product the parts of a strip meet.
-template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_layer(const LayerArgs &a) {
+template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_layer(const LayerFirst &f, const LayerArgs &a) {
     extern __shared__ __align__(256) unsigned char el_smem[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, g = lane >> 4, gbit = g & 1;
-    // the parts of a strip on one XCD (workgroups go to the 8 XCDs round-robin by id): what they share comes from HBM once
-    const int strip = MODE == 0 ? blockIdx.x : blockIdx.x % 8 + 8 * (blockIdx.x / 8 / a.parts), part = MODE == 0 ? 0 : blockIdx.x / 8 % a.parts;
-    if (MODE != 0 && strip * MT * 16 >= a.T) return;  // padding of the grid (the whole workgroup)
+    // The parts of a strip on one XCD (workgroups go to the 8 XCDs round-robin by id, x first): what they share comes from HBM once.
+    const int group = MODE == 0 ? 0 : (int)(blockIdx.z ? blockIdx.y + gridDim.y * blockIdx.z : blockIdx.y);
+    const int strip = MODE == 0 ? blockIdx.x : blockIdx.x % 8 + 8 * group, part = MODE == 0 ? 0 : blockIdx.x / 8;
+    if (MODE != 0 && strip * MT * 16 >= f.T) return;  // padding of the grid (the whole workgroup)
     const int tok0 = strip * (MT * 16);
-    const int H = a.H;
+    const int H = f.H, xs = (f.form & 255) << 8;
     // The joined launch reads what it needs behind the join when it needs it: held from the start it would not fit the scalar
     // registers, and a scalar register that comes back from a vector lane must not be read by a request within five
     // instructions, which the compiler cannot see in the assembly here.
     auto late = [] {
-        auto *p = (const __attribute__((address_space(4))) LayerArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+        auto *p = (const __attribute__((address_space(4))) LayerArgs *)((const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr() + kElFirstBytes);
         asm volatile("" : "+s"(p));
         return p;
     };
@@ -291,7 +300,7 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
     auto here = [](int v) { return kLate ? el_here_s(v) : v; };
 
     unsigned char *X = el_smem;                            // [MT * 16][xs], 16-byte units XORed with the row
-    unsigned char *Hb = X + MT * 16 * a.xs;                // [1 or 2 chunks][MT * 16][hs], the same
+    unsigned char *Hb = X + MT * 16 * xs;                // [1 or 2 chunks][MT * 16][hs], the same
     float *red = reinterpret_cast<float *>(Hb + a.hbuf + MT * 16 * a.hs);  // [2][16 waves][MT * 16]
     _Float16 *vec = reinterpret_cast<_Float16 *>(red + 2 * kElWaves * MT * 16);
     // (bo, g1, be1, b1, b2, g2, be2, bq)
@@ -301,58 +310,59 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
     const int stream = part * kElWaves + wave;
     // A buffer that ends with the wave's last slot: the ring's requests past it go nowhere.  Answered, they were 128 KiB of the
     // 0.9 MiB a workgroup of the first launch took in at 8 x 128 tokens, and of the 0.6 of the second.
-    const uint64_t slots_at = (uint64_t)(a.slots + (size_t)stream * a.cap * 1024);
-    i4 slots = {(int)(unsigned)slots_at, (int)(unsigned)(slots_at >> 32), a.cap * 1024, kElBufferWord};
-    const char *offs = a.offs + (size_t)stream * a.cap * 4;  // uniform
+    const uint64_t slots_at = (uint64_t)(a.slots + (size_t)stream * f.cap * 1024);
+    i4 slots = {(int)(unsigned)slots_at, (int)(unsigned)(slots_at >> 32), f.cap * 1024, kElBufferWord};
+    const char *offs = f.offs + (size_t)stream * f.cap * 4;  // uniform
     unsigned lane_off = lane * 16, offs_off = (g >> 1) * 16;
     el_ask_offsets(offs_off, offs);
     if constexpr (MODE != 2) {
-        // Z -> X, straight into LDS: the lane that fills unit pu of a row fetches the row's unit pu ^ (row % 16); units
+        // Z -> X, straight into LDS, a wave a row: the lane that fills unit pu of a row fetches the row's unit pu ^ (row % 16); units
         // past H repeat the last one (nothing names them)
-        const int upr = a.xs >> 4, n_inst = MT * 16 * upr / 64, last = (H >> 3) - 1;
+        const int upr = xs >> 4, last = (H >> 3) - 1;
         const unsigned lds0 = (unsigned)(size_t)((__attribute__((address_space(3))) void *)X);
-        const char *zb = reinterpret_cast<const char *>(a.Z + (size_t)tok0 * H);
-        for (int i = wave; i < n_inst; i += kElWaves) {
-            const int at = i * 64 + lane, row = at / upr, pu = at - row * upr;
-            const int zr = min(tok0 + row, a.T - 1) - tok0;
-            el_load_to_lds(zb, (unsigned)(zr * H * 2 + (min(pu ^ (row & 15), last) << 4)), lds0 + (unsigned)i * 1024u);
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+            const int row = wave + m * kElWaves;
+            const char *zb = reinterpret_cast<const char *>(f.Z + (size_t)min(tok0 + row, f.T - 1) * H);
+            for (int u = 0; u < upr; u += 64)  // (at least 16 lanes of each)
+                if (u + lane < upr) el_load_to_lds(zb, (unsigned)(min((u + lane) ^ (row & 15), last) << 4), lds0 + (unsigned)(row * xs + u * 16));
         }
     }
     // the table of the wave and its descriptors
     int tab, desc[kElRowRegs];
-    el_ask(tab, lane * 4, a.tab + (size_t)stream * kElTab);
+    el_ask(tab, lane * 4, f.tab + (size_t)stream * kElTab);
 #pragma unroll
-    for (int i = 0; i < kElRowRegs; i++) el_ask(desc[i], lane * 4, a.rows + ((size_t)stream * kElRowRegs + i) * 64);
+    for (int i = 0; i < kElRowRegs; i++) el_ask(desc[i], lane * 4, f.tab + (size_t)stream * kElTab + (1 + i) * kElTabWords);
 
     const uint32_t own = a.sums[wave];
     int rb[NR];
 #pragma unroll
     for (int j = 0; j < NR; j++) rb[j] = (own >> (8 * j) & 255) == 255 ? -1 : (int)(own >> (8 * j) & 255);
     // bytes from the strip's first value to a tile in tile order (uniform); a second tile past the end: the first
-    const int tiles_here = min(MT, (a.T - tok0) >> 4);
+    const int tiles_here = min(MT, (f.T - tok0) >> 4);
     auto tile_at = [&](int m, int j) { return (unsigned)((MT == 1 ? 0 : min(m, tiles_here - 1) * H) + max(here(rb[j]), 0) * 16) * 64; };
 
     auto ask_vectors = [&] {  // straight into LDS, 512 values an instruction
-        const int nvec = (6 * H + a.FF + (MODE == 1 ? 0 : a.Q)) >> 3;
+        const int nvec = f.form >> 16;
         const unsigned lds0 = (unsigned)(size_t)((__attribute__((address_space(3))) void *)vec);
         for (int i = wave * 64; i < nvec; i += kElWaves * 64)
-            if (i + lane < nvec) el_load_to_lds(a.vec, (unsigned)(i + lane) * 16u, lds0 + (unsigned)i * 16u);
+            if (i + lane < nvec) el_load_to_lds(f.vec, (unsigned)(i + lane) * 16u, lds0 + (unsigned)i * 16u);
     };
-    const bool half_in = MODE != 2 && a.x16 != nullptr;  // uniform
+    const bool half_in = MODE != 2 && (f.form >> 8 & 1);  // uniform
     f4 V[NR][MT];
     unsigned long long r16v[NR][MT];
     auto ask_residual = [&](f4 (&to)[NR][MT]) {
         if (half_in) {
-            const char *src = reinterpret_cast<const char *>(a.x16 + (size_t)tok0 * H);
+            const char *src = reinterpret_cast<const char *>(static_cast<const _Float16 *>(f.x) + (size_t)tok0 * H);
 #pragma unroll
             for (int j = 0; j < NR; j++)
 #pragma unroll
                 for (int m = 0; m < MT; m++) {
-                    const unsigned row_at = (unsigned)(min(tok0 + m * 16 + r16, a.T - 1) - tok0) * H * 2;
+                    const unsigned row_at = (unsigned)(min(tok0 + m * 16 + r16, f.T - 1) - tok0) * H * 2;
                     asm volatile("global_load_dwordx2 %0, %1, %2" : "=v"(r16v[j][m]) : "v"(row_at + max(rb[j], 0) * 32 + g * 8), "s"(src) : "memory");
                 }
         } else {
-            const char *src = reinterpret_cast<const char *>(a.x32 + (size_t)tok0 * H);
+            const char *src = reinterpret_cast<const char *>(static_cast<const float *>(f.x) + (size_t)tok0 * H);
 #pragma unroll
             for (int j = 0; j < NR; j++)
 #pragma unroll
@@ -502,7 +512,7 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
     const unsigned hbuf = a.hbuf;
     // the lane's token row in the strip and in a hidden chunk, held: worked out for every block-row, the two products took as
     // long as eight other vector instructions
-    unsigned row_x = (unsigned)r16 * a.xs, row_h = (unsigned)r16 * a.hs;
+    unsigned row_x = (unsigned)r16 * xs, row_h = (unsigned)r16 * a.hs;
     asm volatile("" : "+v"(row_x), "+v"(row_h));
 
     // LayerNorm of V (+ add) in place; the result is also rounded into X.  A wave sums its features of a token and their
@@ -601,7 +611,7 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
         h4 gm[NR], bt[NR];
         vec_of(gm, gam);
         vec_of(bt, bet);
-        unsigned xrow = r16 * a.xs + gbit * 8;  // (once; sunk under the branches it is a product for each)
+        unsigned xrow = r16 * xs + gbit * 8;  // (once; sunk under the branches it is a product for each)
         asm volatile("" : "+v"(xrow));
 #pragma unroll
         for (int j = 0; j < NR; j++)
@@ -614,7 +624,7 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
                     o[e] = (_Float16)V[j][m][e];
                 }
                 const int u = rb[j] * 2 + (g >> 1);
-                if (rb[j] >= 0) *reinterpret_cast<h4 *>(X + (xrow + m * 16 * a.xs + ((u ^ r16) << 4))) = o;
+                if (rb[j] >= 0) *reinterpret_cast<h4 *>(X + (xrow + m * 16 * xs + ((u ^ r16) << 4))) = o;
             }
     };
 
@@ -632,7 +642,7 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
         el_ask_offsets(offs_off, offs);
         el_ask(tab, lane * 4, l->tab2 + (size_t)s * kElTab);
 #pragma unroll
-        for (int i = 0; i < kElRowRegs; i++) el_ask(desc[i], lane * 4, l->rows2 + ((size_t)s * kElRowRegs + i) * 64);
+        for (int i = 0; i < kElRowRegs; i++) el_ask(desc[i], lane * 4, l->tab2 + (size_t)s * kElTab + (1 + i) * kElTabWords);
         const uint64_t slots_at = (uint64_t)(l->slots2 + (size_t)s * cap2 * 1024);
         slots = i4{(int)(unsigned)slots_at, (int)(unsigned)(slots_at >> 32), cap2 * 1024, kElBufferWord};
     };
@@ -742,7 +752,7 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
                 else __builtin_amdgcn_s_setprio(1);
                 const int n = d & 255, kind = (d >> 8) & 3, target = (d >> 11) & 1023, bias_at = (d >> 21) * 16;
                 const bool hid = (d >> 10) & 1;
-                const unsigned base = hid ? row_h + (MT * 16 * a.xs + hb_dn) : row_x, step = 16 * (hid ? a.hs : a.xs);
+                const unsigned base = hid ? row_h + (MT * 16 * xs + hb_dn) : row_x, step = 16 * (hid ? a.hs : xs);
                 if constexpr (MODE != 3 && PHASE != 2) {
                     if (kind == kElKindSum) {
 #pragma unroll
@@ -839,11 +849,11 @@ template <int MT, int NR, int MODE> __device__ __forceinline__ void encoder_laye
 }
 
 template <int MT, int NR, int MODE>
-__global__ __launch_bounds__(kElWaves * 64) __attribute__((amdgpu_num_vgpr(kElOwnVgprs))) void encoder_layer_kernel(const LayerArgs a) {
-    encoder_layer<MT, NR, MODE>(a);
+__global__ __launch_bounds__(kElWaves * 64) __attribute__((amdgpu_num_vgpr(kElOwnVgprs))) void encoder_layer_kernel(ET_EL_FIRST, const LayerArgs a) {
+    encoder_layer<MT, NR, MODE>(LayerFirst{Z, x, offs, tab, vec, T, H, cap, form}, a);
 }
-template <int NR> __global__ __launch_bounds__(kElWaves * 64) __attribute__((amdgpu_num_vgpr(kElOwnVgprs))) void encoder_layer_joined_kernel(const LayerArgs a) {
-    encoder_layer<1, NR, 4>(a);
+template <int NR> __global__ __launch_bounds__(kElWaves * 64) __attribute__((amdgpu_num_vgpr(kElOwnVgprs))) void encoder_layer_joined_kernel(ET_EL_FIRST, const LayerArgs a) {
+    encoder_layer<1, NR, 4>(LayerFirst{Z, x, offs, tab, vec, T, H, cap, form}, a);
 }
 
 // slot s = tiles order[2s], order[2s + 1] (bits 28-29: which weight; negative: a zero tile) in lane order: the 16-byte
@@ -871,9 +881,9 @@ struct et_layer_pack_s {
     uint32_t sums[et::kElWaves] = {};
     int second = 0, nstream = 0;  // first stream of the second launch (or of the projection alone), all streams
     int cap = 0, cap2 = 0;        // slots from one stream to the next, before and from there on
-    void *slots = nullptr, *offs = nullptr, *rows = nullptr, *tab = nullptr, *vec = nullptr;
+    void *slots = nullptr, *offs = nullptr, *tab = nullptr, *vec = nullptr;
     ~et_layer_pack_s() {
-        for (void *p : {slots, offs, rows, tab, vec}) (void)et_free(p);
+        for (void *p : {slots, offs, tab, vec}) (void)et_free(p);
     }
 };
 
@@ -1005,7 +1015,7 @@ static int el_pack_create(const et_layer_weights *w, int T, int emdim, int dimFF
     auto emit = [&](const std::vector<std::vector<std::vector<ElRow>>> &segs) {  // [segment][wave]
         for (int v = 0; v < kElWaves; v++) {
             Stream st;
-            st.tab.assign(kElTab, 0);
+            st.tab.assign(kElTabWords, 0);
             std::copy(chunks_of_q.begin(), chunks_of_q.end(), st.tab.begin() + kElTabOut);
             for (int o = 0; o < kElWaves; o++) st.tab[(size_t)(kElTabCount + o)] = (int)sums[(size_t)o].size();
             for (size_t sg = 0; sg < segs.size(); sg++) {
@@ -1096,13 +1106,12 @@ static int el_pack_create(const et_layer_weights *w, int T, int emdim, int dimFF
     ET_REQUIRE(most_slots <= kElMaxSlots, ET_ERR_UNSUPPORTED,
                "et_encoder_layer_pack_create: %d slots in one block-row, at most %d fit its descriptor", most_slots, kElMaxSlots);
     ET_REQUIRE(most_rows <= 64 * kElRowRegs, ET_ERR_UNSUPPORTED, "et_encoder_layer_pack_create: %zu block-rows in one wave", most_rows);
-    std::vector<int32_t> tab, order(all_slots * 2, -1);
-    std::vector<uint32_t> rows(streams.size() * 64 * kElRowRegs, 0);
+    std::vector<int32_t> tab(streams.size() * kElTab, 0), order(all_slots * 2, -1);
     std::vector<uint16_t> offs((all_slots + 2 * kElRing) * 2, 0);
     for (size_t i = 0; i < streams.size(); i++) {
         const Stream &st = streams[i];
-        tab.insert(tab.end(), st.tab.begin(), st.tab.end());
-        std::copy(st.rows.begin(), st.rows.end(), rows.begin() + (long)(i * 64 * kElRowRegs));
+        std::copy(st.tab.begin(), st.tab.end(), tab.begin() + (long)(i * kElTab));
+        std::copy(st.rows.begin(), st.rows.end(), tab.begin() + (long)(i * kElTab + kElTabWords));
         std::copy(st.order.begin(), st.order.end(), order.begin() + (long)(first_slot(i) * 2));
         for (size_t k = 0; k < st.offs.size(); k++) {
             const size_t at = (first_slot(i) + k / kElRing * kElRing) * 2 + k % kElRing;
@@ -1132,7 +1141,6 @@ static int el_pack_create(const et_layer_weights *w, int T, int emdim, int dimFF
     void *d_order = nullptr;
     const int nslots = (int)(order.size() / 2);
     s = upload(&p->offs, offs.data(), offs.size() * 2);
-    if (s == ET_OK) s = upload(&p->rows, rows.data(), rows.size() * 4);
     if (s == ET_OK) s = upload(&p->tab, tab.data(), tab.size() * 4);
     if (s == ET_OK) s = upload(&d_order, order.data(), order.size() * 4);
     if (s == ET_OK) s = et_malloc(&p->slots, (size_t)nslots * 1024);
@@ -1176,24 +1184,27 @@ int et_encoder_layer_pack_destroy(struct et_layer_pack_s *pack) {
 }  // extern "C"
 
 namespace et {
-template <int MT, int NR, int MODE> static int el_launch(const LayerArgs &a, size_t lds, int blocks, hipStream_t stream) {
-    void (*kernel)(LayerArgs);
-    if constexpr (MODE == 4) kernel = encoder_layer_joined_kernel<NR>;
-    else kernel = encoder_layer_kernel<MT, NR, MODE>;
+template <int MT, int NR, int MODE> static int el_launch(const LayerFirst &f, const LayerArgs &a, size_t lds, hipStream_t stream) {
+    auto kernel = [] {
+        if constexpr (MODE == 4) return encoder_layer_joined_kernel<NR>;
+        else return encoder_layer_kernel<MT, NR, MODE>;
+    }();
     static bool raised = false;  // per instantiation
     if (!raised) {
         ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kElLds));
         raised = true;
     }
-    kernel<<<(unsigned)blocks, kElWaves * 64, lds, stream>>>(a);
+    const unsigned strips = (unsigned)((f.T + MT * 16 - 1) / (MT * 16)), groups = (strips + 7) / 8, rows = std::min(groups, 32768u);
+    const dim3 grid = MODE == 0 ? dim3(strips) : dim3(8 * (unsigned)a.parts, rows, (groups + rows - 1) / rows);
+    kernel<<<grid, kElWaves * 64, lds, stream>>>(f.Z, f.x, f.offs, f.tab, f.vec, f.T, f.H, f.cap, f.form, a);
     return check_launch("encoder_layer_kernel");
 }
-template <int MT, int MODE> static int el_dispatch(const LayerArgs &a, const et_layer_pack_s &p, int blocks, hipStream_t stream) {
+template <int MT, int MODE> static int el_dispatch(const LayerFirst &f, const LayerArgs &a, const et_layer_pack_s &p, hipStream_t stream) {
     switch (p.nr) {
         case 1:
-        case 2: return el_launch<MT, 2, MODE>(a, p.lds, blocks, stream);
-        case 3: return el_launch<MT, 3, MODE>(a, p.lds, blocks, stream);
-        default: return el_launch<MT, 4, MODE>(a, p.lds, blocks, stream);
+        case 2: return el_launch<MT, 2, MODE>(f, a, p.lds, stream);
+        case 3: return el_launch<MT, 3, MODE>(f, a, p.lds, stream);
+        default: return el_launch<MT, 4, MODE>(f, a, p.lds, stream);
     }
 }
 }  // namespace et
@@ -1202,23 +1213,21 @@ template <int MT, int MODE> static int el_dispatch(const LayerArgs &a, const et_
 static LayerArgs el_args(const et_layer_pack_s &p) {
     LayerArgs a{};
     a.slots = static_cast<const char *>(p.slots);
-    a.offs = static_cast<const char *>(p.offs);
-    a.rows = static_cast<const uint32_t *>(p.rows);
-    a.tab = static_cast<const int32_t *>(p.tab);
-    a.vec = static_cast<const _Float16 *>(p.vec);
-    a.cap = p.cap;
     std::copy(p.sums, p.sums + kElWaves, a.sums);
     a.inv_h = 1.0f / (float)p.H;
     a.T = p.T, a.H = p.H, a.FF = p.FF, a.Q = p.Q;
-    a.xs = p.xs, a.hs = p.hs, a.nseg_ff = p.nseg_ff, a.nseg_q = p.nseg_q, a.hbuf = p.hbuf, a.parts = a.nshare = p.parts;
+    a.hs = p.hs, a.nseg_ff = p.nseg_ff, a.nseg_q = p.nseg_q, a.hbuf = p.hbuf, a.parts = a.nshare = p.parts;
     return a;
 }
-static void el_second(LayerArgs &a, const et_layer_pack_s &p) {
-    a.tab += (size_t)p.second * kElTab;
-    a.rows += (size_t)p.second * 64 * kElRowRegs;
+static LayerFirst el_first(const et_layer_pack_s &p) {
+    return {nullptr, nullptr, static_cast<const char *>(p.offs), static_cast<const int32_t *>(p.tab), static_cast<const _Float16 *>(p.vec),
+            p.T,     p.H,     p.cap, (unsigned)(p.xs >> 8) | (unsigned)((6 * p.H + p.FF + p.Q) >> 3) << 16};
+}
+static void el_second(LayerFirst &f, LayerArgs &a, const et_layer_pack_s &p) {
+    f.tab += (size_t)p.second * kElTab;
     a.slots += (size_t)p.second * p.cap * 1024;
-    a.offs += (size_t)p.second * p.cap * 4;
-    a.cap = p.cap2;
+    f.offs += (size_t)p.second * p.cap * 4;
+    f.cap = p.cap2;
     a.parts = p.Q ? p.parts : 1;  // without a projection only the normalisation is left
 }
 
@@ -1235,11 +1244,11 @@ extern "C" int et_encoder_layer_project_f16(const struct et_layer_pack_s *p, con
     ET_REQUIRE(((reinterpret_cast<uintptr_t>(x16) | reinterpret_cast<uintptr_t>(QKV)) & 15) == 0, ET_ERR_UNSUPPORTED,
                "et_encoder_layer_project_f16: x16 and QKV must be 16-byte aligned");
     LayerArgs a = el_args(*p);
-    a.Z = reinterpret_cast<const _Float16 *>(x16);
+    LayerFirst f = el_first(*p);
+    f.Z = reinterpret_cast<const _Float16 *>(x16);
     a.qkv = reinterpret_cast<_Float16 *>(QKV);
-    el_second(a, *p);
-    const int strips = p->T / 16;  // one token tile a workgroup, whatever the pack's strips are: the sums are the same
-    return el_launch<1, 2, 3>(a, p->lds, (strips + 7) / 8 * 8 * a.parts, as_stream(stream));
+    el_second(f, a, *p);
+    return el_launch<1, 2, 3>(f, a, p->lds, as_stream(stream));  // one token tile a workgroup, whatever the pack's strips are: the sums are the same
 }
 
 // Workgroups of equal id modulo 8 share an XCD, as they are dealt out: looked at once per device.
@@ -1296,29 +1305,32 @@ static int el_run(const struct et_layer_pack_s *p, const et_f16 *Z, const float 
     ET_REQUIRE(!x32 || !x32_out || at(x32_out) >= at(x32) + x32_bytes || at(x32) >= at(x32_out) + x32_bytes, ET_ERR_INVALID_ARG,
                "et_encoder_layer_f32: x32_out overlaps x32");
     LayerArgs a = el_args(*p);
-    a.Z = reinterpret_cast<const _Float16 *>(Z);
-    a.x32 = x32;
-    a.x16 = x32 ? nullptr : reinterpret_cast<const _Float16 *>(x16);
+    LayerFirst f = el_first(*p);
+    f.Z = reinterpret_cast<const _Float16 *>(Z);
+    f.x = x32 ? static_cast<const void *>(x32) : x16;
+    f.form |= x32 ? 0u : 1u << 8;
     a.x32_out = x32_out;
     a.out16 = reinterpret_cast<_Float16 *>(out16);
     a.qkv = reinterpret_cast<_Float16 *>(QKV);
     a.partial = partial;
     a.act = act;
     a.eps1 = eps1, a.eps2 = eps2;
-    const int strips = (p->T + p->mt * 16 - 1) / (p->mt * 16);
     hipStream_t st = as_stream(stream);
     if (join) {
         LayerArgs second = a;
-        el_second(second, *p);
-        a.slots2 = second.slots, a.offs2 = second.offs, a.rows2 = second.rows, a.tab2 = second.tab, a.cap2 = second.cap;
+        LayerFirst first = f;
+        el_second(first, second, *p);
+        a.slots2 = second.slots, a.offs2 = first.offs, a.tab2 = first.tab, a.cap2 = first.cap;
         a.join = join, a.spin = spin;
-        return el_dispatch<1, 4>(a, *p, (strips + 7) / 8 * 8 * p->parts, st);
+        return el_dispatch<1, 4>(f, a, *p, st);
     }
-    if (p->parts == 1) return p->mt == 2 ? el_dispatch<2, 0>(a, *p, strips, st) : el_dispatch<1, 0>(a, *p, strips, st);
-    const int s = el_dispatch<1, 1>(a, *p, (strips + 7) / 8 * 8 * p->parts, st);
+    if (p->parts == 1) return p->mt == 2 ? el_dispatch<2, 0>(f, a, *p, st) : el_dispatch<1, 0>(f, a, *p, st);
+    LayerFirst shares = f;
+    shares.form = (f.form & 0xffffu) | (unsigned)((6 * p->H + p->FF) >> 3) << 16;  // (the projection's bias is the second launch's)
+    const int s = el_dispatch<1, 1>(shares, a, *p, st);
     if (s != ET_OK) return s;
-    el_second(a, *p);
-    return el_dispatch<1, 2>(a, *p, (strips + 7) / 8 * 8 * a.parts, st);
+    el_second(f, a, *p);
+    return el_dispatch<1, 2>(f, a, *p, st);
 }
 
 extern "C" int et_encoder_layer_f32(const struct et_layer_pack_s *p, const et_f16 *Z, const float *x32, const et_f16 *x16, float *x32_out,
