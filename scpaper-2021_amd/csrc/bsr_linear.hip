@@ -121,7 +121,11 @@ __host__ __device__ __forceinline__ int half_tiles(int in) { return (in / 16 + 1
 // ACT is a template parameter: the epilogue carries no run-time branch and each
 // fused activation is a separately named kernel in a profile.
 template <int MT, bool STAGE, int ACT, int LN = 0, int FX = 0>
-__global__ __launch_bounds__(((MT == 1 && (FX & kFxRes32) && !(FX & kFxRes16)) || (FX & (kFxNorm32 | kFxWide))) ? 768 : 512) void bsr16_linear_kernel(const BsrArgs a) {
+__global__ __launch_bounds__(((MT == 1 && (FX & kFxRes32) && !(FX & kFxRes16)) || (FX & (kFxNorm32 | kFxWide))) ? 768 : 512) void bsr16_linear_kernel(const int32_t *row_ptr, const _Float16 *X, const int32_t *col_idx, const _Float16 *tiles, int T, int in, int out,
+                                                                                                                                                      int rows_per_wg, int ngroups, unsigned per_group,
+                                                                                                                                                      const BsrArgs rest) {
+    BsrArgs a = rest;  // (those in front are preloaded into scalar registers)
+    a.row_ptr = row_ptr, a.X = X, a.col_idx = col_idx, a.tiles = tiles, a.T = T, a.in = in, a.out = out, a.rows_per_wg = rows_per_wg;
     static_assert(!LN || STAGE, "the fused LayerNorm prologue writes the strip to LDS");
     static_assert(!(FX & kFxNorm) || (STAGE && !LN), "the NORM prologue writes the strip to LDS");
     constexpr bool NORM = (FX & kFxNorm) != 0;
@@ -156,8 +160,9 @@ __global__ __launch_bounds__(((MT == 1 && (FX & kFxRes32) && !(FX & kFxRes16)) |
     // strip s is pinned to XCD s % 8 and the groups of one strip follow each other on
     // that XCD: a strip of X is fetched into one L2 only and reused there.
     const int nbr = a.out >> 4;
-    const int ngroups = (nbr + a.rows_per_wg - 1) / a.rows_per_wg;
     const int nstrips = (a.T + MT * 16 - 1) / (MT * 16);
+    // (`per_group` is 2^32 over the number of groups, rounded up, or 0 where that would not be exact)
+    auto groups_in = [&](int n) { return per_group ? (int)(((unsigned long long)(unsigned)n * per_group) >> 32) : n / ngroups; };
     const int xcd = blockIdx.x % kXcds, k_in_xcd = blockIdx.x / kXcds;
     int strip, group;
     if (nstrips < kXcds) {
@@ -166,11 +171,12 @@ __global__ __launch_bounds__(((MT == 1 && (FX & kFxRes32) && !(FX & kFxRes16)) |
         // 16 x 1024 -> 4096 29.1 -> 5.2, 64 x 3072 -> 768 17.1 -> 9.2; from 8 strips on the two are the same but for the die of a strip).
         const int units = nstrips * ngroups, per_xcd = (units + kXcds - 1) / kXcds, unit = xcd * per_xcd + k_in_xcd;
         if (unit >= units) return;  // padding of the last XCD's run (whole workgroup)
-        strip = unit / ngroups;
+        strip = groups_in(unit);
         group = unit - strip * ngroups;
     } else {
-        strip = xcd + kXcds * (k_in_xcd / ngroups);
-        group = k_in_xcd % ngroups;
+        const int round = groups_in(k_in_xcd);
+        strip = xcd + kXcds * round;
+        group = k_in_xcd - round * ngroups;
         if (strip >= nstrips) return;  // padding of the last round of strips (whole workgroup)
     }
     const int tok0 = strip * (MT * 16);
@@ -729,7 +735,10 @@ constexpr int kHalfAhead = 2;           // items asked for ahead
 constexpr int kRawBuffer = 0x00020000;  // word 3 of a resource: raw, 32-bit data
 constexpr int kNoTile = 0xffff;         // past the tiles of any listed row
 template <int ACT, int RW>
-__global__ __launch_bounds__(kHalfWaves * 64) void bsr16_linear_halves_kernel(const BsrArgs a) {
+__global__ __launch_bounds__(kHalfWaves * 64) void bsr16_linear_halves_kernel(const int32_t *row_ptr, const _Float16 *X, const int32_t *col_idx, const _Float16 *tiles,
+                                                                              const _Float16 *bias_of, int T, int in, int out, int rows_per_wg, const BsrArgs rest) {
+    BsrArgs a = rest;  // (those in front are preloaded into scalar registers)
+    a.row_ptr = row_ptr, a.X = X, a.col_idx = col_idx, a.tiles = tiles, a.bias = bias_of, a.T = T, a.in = in, a.out = out, a.rows_per_wg = rows_per_wg;
     constexpr int MT = 2, kNB = kHalfAhead;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     _Float16 *xs = reinterpret_cast<_Float16 *>(smem_raw);  // [32][half * 16 + kLdsPad]
@@ -737,9 +746,8 @@ __global__ __launch_bounds__(kHalfWaves * 64) void bsr16_linear_halves_kernel(co
     const int r16 = lane & 15, g = lane >> 4;
     const int sel = g >> 1, koff = (g & 1) << 3;  // as in the kernel above
     const int nbr = a.out >> 4;
-    const int ngroups = (nbr + a.rows_per_wg - 1) / a.rows_per_wg;
-    const int xcd = blockIdx.x % kXcds, k_in_xcd = blockIdx.x / kXcds;
-    const int strip = xcd + kXcds * (k_in_xcd / ngroups), group = k_in_xcd % ngroups;
+    // (workgroups go to the XCDs round-robin by id, x first: the groups of a strip on one XCD, one after the other)
+    const int strip = blockIdx.x % kXcds + kXcds * (int)(blockIdx.z ? blockIdx.y + gridDim.y * blockIdx.z : blockIdx.y), group = blockIdx.x / kXcds;
     const int tok0 = strip * (MT * 16);
     if (tok0 >= a.T) return;  // padding of the last round of strips (whole workgroup)
     const int rb_begin = group * a.rows_per_wg, rb_end = min(rb_begin + a.rows_per_wg, nbr);
@@ -1112,7 +1120,10 @@ static int launch_bsr_act(const BsrArgs &args, const BsrPlan &p, hipStream_t str
     const int nstrips = (args.T + MT * 16 - 1) / (MT * 16);
     // (the kernel's own two ways to deal them out)
     const int per_xcd = nstrips < kXcds ? (nstrips * ngroups + kXcds - 1) / kXcds : (nstrips + kXcds - 1) / kXcds * ngroups;
-    kernel<<<(unsigned)(per_xcd * kXcds), p.threads, p.lds, stream>>>(args);
+    const unsigned per_group = ngroups > 1 && (unsigned long long)per_xcd * kXcds * ngroups < 1ull << 32 ? (unsigned)(((1ull << 32) + ngroups - 1) / ngroups) : 0;
+    BsrArgs a = args;
+    a.rows_per_wg = p.rows_per_wg;
+    kernel<<<(unsigned)(per_xcd * kXcds), p.threads, p.lds, stream>>>(a.row_ptr, a.X, a.col_idx, a.tiles, a.T, a.in, a.out, a.rows_per_wg, ngroups, per_group, a);
     return check_launch("bsr16_linear_kernel");
 }
 
@@ -1203,7 +1214,9 @@ static int launch_bsr_halves(const BsrArgs &args, int rows_per_wg, hipStream_t s
         ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     const int nbr = args.out / 16, ngroups = (nbr + rows_per_wg - 1) / rows_per_wg;
     const int strips = (args.T + 31) / 32;
-    kernel<<<(unsigned)((strips + kXcds - 1) / kXcds * kXcds * ngroups), kHalfWaves * 64, lds, stream>>>(args);
+    const unsigned rounds = (unsigned)((strips + kXcds - 1) / kXcds), gy = std::min(rounds, 32768u);
+    kernel<<<dim3((unsigned)(kXcds * ngroups), gy, (rounds + gy - 1) / gy), kHalfWaves * 64, lds, stream>>>(args.row_ptr, args.X, args.col_idx, args.tiles, args.bias, args.T,
+                                                                                                         args.in, args.out, rows_per_wg, args);
     return check_launch("bsr16_linear_halves_kernel");
 }
 

@@ -31,12 +31,11 @@ struct LinearF32Args {
     int T, in, out, ldx, ldy;
 };
 template <int ACT, int TILE, bool GATHER, int OUT>
-__global__ __launch_bounds__(256) void linear_dense_f32_kernel(const LinearF32Args a) {
-    const float *__restrict__ W = a.W;
-    const float *__restrict__ bias = a.bias;
-    const float *__restrict__ X = a.X;
+__global__ __launch_bounds__(256) void linear_dense_f32_kernel(const float *__restrict__ W, const float *__restrict__ X, const float *__restrict__ bias, int T, int in,
+                                                               int out, int ldx, const LinearF32Args rest) {
+    LinearF32Args a = rest;  // (those in front are preloaded into scalar registers)
+    a.ldx = ldx;
     float *__restrict__ Y = a.Y;
-    const int T = a.T, in = a.in, out = a.out;
     constexpr int WB = TILE / 2;          // wave block
     constexpr int MI = WB / 16;           // 16 x 16 MFMA tiles per wave and dimension
     constexpr int TPR = 256 / TILE;       // staging threads per row
@@ -173,7 +172,10 @@ template <bool VEC> __device__ __forceinline__ f4 load_quad_f32(const float *p) 
 
 // VEC: rows of Q and K start at multiples of 16 bytes.  MAXC: cells of 16 features of a head, at most.
 template <int MAXC, bool VEC>
-__global__ __launch_bounds__(256) void mha_fused_f32_kernel(const MhaF32Args a) {
+__global__ __launch_bounds__(256) void mha_fused_f32_kernel(const float *Q, const float *K, const float *V, const int32_t *lens, int ldq, int ldk, int ldv, int S,
+                                                            int hd_, int causal, const MhaF32Args rest) {
+    MhaF32Args a = rest;  // (those in front are preloaded into scalar registers)
+    a.Q = Q, a.K = K, a.V = V, a.lens = lens, a.ldq = ldq, a.ldk = ldk, a.ldv = ldv, a.S = S, a.hd = hd_, a.causal = causal;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     float *sc = reinterpret_cast<float *>(smem_raw);  // [16][S + kAttPad]
     __shared__ float inv_sum[kAttQ];
@@ -320,8 +322,8 @@ static int launch_linear_f32(const LinearF32Args &a, int act, bool gather, int o
     const dim3 grid((a.out + tile - 1) / tile, (a.T + tile - 1) / tile);
 #define ET_F32_FORM(ACTV, G, O)                                                       \
     {                                                                                 \
-        if (small) linear_dense_f32_kernel<ACTV, 32, G, O><<<grid, 256, 0, st>>>(a);  \
-        else linear_dense_f32_kernel<ACTV, 64, G, O><<<grid, 256, 0, st>>>(a);        \
+        if (small) linear_dense_f32_kernel<ACTV, 32, G, O><<<grid, 256, 0, st>>>(a.W, a.X, a.bias, a.T, a.in, a.out, a.ldx, a);  \
+        else linear_dense_f32_kernel<ACTV, 64, G, O><<<grid, 256, 0, st>>>(a.W, a.X, a.bias, a.T, a.in, a.out, a.ldx, a);        \
     }
 #define ET_F32_LINEAR(ACTV)                                                \
     {                                                                      \
@@ -433,7 +435,7 @@ int et_mha_fused_f32(const float *Q, const float *K, const float *V, int ldq, in
         if (strip > 64 * 1024)                                                                               \
             ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),                                 \
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)strip));             \
-        kern<<<grid, 256, strip, st>>>(a);                                                                   \
+        kern<<<grid, 256, strip, st>>>(a.Q, a.K, a.V, a.lens, a.ldq, a.ldk, a.ldv, a.S, a.hd, a.causal, a);  \
     }
     // 16-byte loads of Q and K where every row starts at a multiple of 16 bytes
     const bool vec = aligned16(Q) && aligned16(K) && ldq % 4 == 0 && ldk % 4 == 0;

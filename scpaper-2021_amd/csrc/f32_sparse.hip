@@ -18,12 +18,22 @@
 namespace et {
 
 struct Bsr32Args {
+    const float *X;
     const int32_t *row_ptr, *col_idx;
-    const float *tiles, *bias, *X;
-    float *Y;
-    int T, in, out, act;
+    const float *tiles, *bias;
+    int T, in, out;
     int die_bits;  // 0 to 3: see strip_of
+    float *Y;
+    int act;
 };
+// one by one, those that the requests need in front: preloaded into scalar registers (six layers of 256 rows, seven launches
+// each, 247 -> 242 us)
+#define ET_BSR32_PARAMS const float *X, const int32_t *row_ptr, const int32_t *col_idx, const float *tiles, const float *bias_of, int T, int in, int out, int die_bits, float *Y, int act
+#define ET_BSR32_ARGS(A) (A).X, (A).row_ptr, (A).col_idx, (A).tiles, (A).bias, (A).T, (A).in, (A).out, (A).die_bits, (A).Y, (A).act
+#define ET_BSR32_TAKE const Bsr32Args a{X, row_ptr, col_idx, tiles, bias_of, T, in, out, die_bits, Y, act}
+
+// row of the grid (its size, which only more than 32768 rows need, would be read from memory)
+__device__ __forceinline__ unsigned grid_row() { return blockIdx.z ? blockIdx.y + blockIdx.z * gridDim.y : blockIdx.y; }
 
 __device__ __forceinline__ f4 mfma_cell_f32(const float4 w, const float4 x, f4 acc) {
     acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w.x, x.x, acc, 0, 0, 0);
@@ -56,10 +66,11 @@ __device__ __forceinline__ void store_cell_f32(float *Y, f4 bias, f4 acc, int to
 //
 // The wide form: a wave has one block-row and MT blocks of 16 tokens; the four waves of a workgroup take neighbouring
 // block-rows over the same tokens and meet in the cache.
-template <int MT> __global__ __launch_bounds__(256) void bsr16_linear_wide_f32_kernel(const Bsr32Args a) {
+template <int MT> __global__ __launch_bounds__(256) void bsr16_linear_wide_f32_kernel(ET_BSR32_PARAMS) {
+    ET_BSR32_TAKE;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, q = lane >> 4;
-    const int br = blockIdx.x * 4 + wave, tok0 = (blockIdx.y + blockIdx.z * gridDim.y) * (MT * 16);
+    const int br = blockIdx.x * 4 + wave, tok0 = (int)grid_row() * (MT * 16);
     if (br >= (a.out >> 4) || tok0 >= a.T) return;  // no barrier below
     const float *xrow[MT];
     f4 acc[MT];
@@ -95,7 +106,7 @@ template <int MT> __global__ __launch_bounds__(256) void bsr16_linear_wide_f32_k
 // has to fetch is a part of X and a part of the weights: 2^die_bits parts of the strips, 8 / 2^die_bits of the columns.  (By shifts:
 // two divisions by the number of parts cost every wave 0.3 us.)
 __device__ __forceinline__ int strip_of(int die_bits) {
-    return (int)(blockIdx.x & ((1u << die_bits) - 1)) + ((int)(blockIdx.y + blockIdx.z * gridDim.y) << die_bits);
+    return (int)(blockIdx.x & ((1u << die_bits) - 1)) + ((int)grid_row() << die_bits);
 }
 __device__ __forceinline__ int column_of(int die_bits) { return (int)((blockIdx.x & 7) >> die_bits) + ((int)(blockIdx.x >> 3) << (3 - die_bits)); }
 
@@ -104,7 +115,8 @@ constexpr int kRawBuffer = 0x00020000;   // word 3 of a resource: raw, 32-bit da
 constexpr unsigned kPastEnd = 0x7fffff00;  // an offset past the end of any resource here, also with a row's added to it (below 2^32)
 constexpr int kSplitMaxIn = 1 << 24;     // 16 rows of X lie within the offsets of a resource, and below kPastEnd
 template <int WAVES>
-__global__ __launch_bounds__(WAVES * 64) void bsr16_linear_split_f32_kernel(const Bsr32Args a) {
+__global__ __launch_bounds__(WAVES * 64) void bsr16_linear_split_f32_kernel(ET_BSR32_PARAMS) {
+    ET_BSR32_TAKE;
     __shared__ f4 part[WAVES][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, q = lane >> 4;
@@ -156,7 +168,8 @@ __global__ __launch_bounds__(WAVES * 64) void bsr16_linear_split_f32_kernel(cons
 // Against the wide form: 4096 tokens 768 -> 3072 at 50 / 80 / 90 / 95 % 111 / 172, 55 / 79, 41 / 49, 34 / 33; ten shapes of 1024 to 8192
 // tokens 0.46 - 0.69 of its time at 50 %, 0.55 - 0.77 at 80, 0.65 - 0.89 at 90, 0.78 - 1.11 at 95.
 constexpr int kStripPad = 4, kStripWaves = 8;
-__global__ __launch_bounds__(kStripWaves * 64) void bsr16_linear_strip_f32_kernel(const Bsr32Args a) {
+__global__ __launch_bounds__(kStripWaves * 64) void bsr16_linear_strip_f32_kernel(ET_BSR32_PARAMS) {
+    ET_BSR32_TAKE;
     extern __shared__ __align__(16) unsigned char strip_smem[];
     float *xs = reinterpret_cast<float *>(strip_smem);  // [16][in + kStripPad]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -336,7 +349,7 @@ int et_linear_bsr16_f32(const int32_t *row_ptr, const int32_t *col_idx, const fl
     ET_REQUIRE(aligned16(tiles) && aligned16(X) && aligned16(Y), ET_ERR_UNSUPPORTED,
                "et_linear_bsr16_f32: tiles, X and Y must be 16-byte aligned");
     if (T == 0) return ET_OK;
-    Bsr32Args a{row_ptr, col_idx, tiles, bias, X, Y, T, in, out, act, 0};
+    Bsr32Args a{X, row_ptr, col_idx, tiles, bias, T, in, out, 0, Y, act};
     hipStream_t st = as_stream(stream);
     const int strips = (T + 15) / 16;
     // The parts of the strips and of the columns the dies keep to: of the splits that leave the busiest die the fewest
@@ -366,7 +379,7 @@ int et_linear_bsr16_f32(const int32_t *row_ptr, const int32_t *col_idx, const fl
             ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(bsr16_linear_strip_f32_kernel),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         const dim3 grid = place((out / 16 + kStripWaves - 1) / kStripWaves);
-        bsr16_linear_strip_f32_kernel<<<grid, kStripWaves * 64, lds, st>>>(a);
+        bsr16_linear_strip_f32_kernel<<<grid, kStripWaves * 64, lds, st>>>(ET_BSR32_ARGS(a));
         return check_launch("bsr16_linear_strip_f32_kernel");
     }
     // Wider than that, the wide form from two of its workgroups a compute unit on: 80 %, us, wide against short: 512 workgroups
@@ -376,15 +389,15 @@ int et_linear_bsr16_f32(const int32_t *row_ptr, const int32_t *col_idx, const fl
     if (in > kSplitMaxIn || (mt > 1 && lds > 80 * 1024 && (long long)wide_x * wide_strips >= 512)) {
         const int wide_y = std::min(wide_strips, 32768);
         const dim3 grid(wide_x, wide_y, (wide_strips + wide_y - 1) / wide_y);
-        if (mt == 4) bsr16_linear_wide_f32_kernel<4><<<grid, 256, 0, st>>>(a);
-        else bsr16_linear_wide_f32_kernel<2><<<grid, 256, 0, st>>>(a);
+        if (mt == 4) bsr16_linear_wide_f32_kernel<4><<<grid, 256, 0, st>>>(ET_BSR32_ARGS(a));
+        else bsr16_linear_wide_f32_kernel<2><<<grid, 256, 0, st>>>(ET_BSR32_ARGS(a));
         return check_launch("bsr16_linear_wide_f32_kernel");
     }
     // Two waves a pair below two pairs a compute unit: 192 pairs of 38 tiles 5.2 us against 7.3, 576 pairs of 10 tiles 4.9
     // against 4.7; four waves are no faster.
     const dim3 grid = place(out / 16);
-    if (pairs < 512) bsr16_linear_split_f32_kernel<2><<<grid, 128, 0, st>>>(a);
-    else bsr16_linear_split_f32_kernel<1><<<grid, 64, 0, st>>>(a);
+    if (pairs < 512) bsr16_linear_split_f32_kernel<2><<<grid, 128, 0, st>>>(ET_BSR32_ARGS(a));
+    else bsr16_linear_split_f32_kernel<1><<<grid, 64, 0, st>>>(ET_BSR32_ARGS(a));
     return check_launch("bsr16_linear_split_f32_kernel");
 }
 

@@ -47,15 +47,19 @@ typedef float f16v __attribute__((ext_vector_type(16)));
 // loads of a stage are issued three stages ahead and spread over two K slices.
 // NWN: waves along N, 2 (four waves, one per SIMD) or (whole tiles only) 4: eight waves, two per SIMD, so that a wave
 // held up at a load or at the barrier leaves the matrix pipe to the other.
+// The arguments in front are what the first requests need: preloaded into scalar registers (us, before and now, with the tile found without divisions: 2048 x 768 ->
+// 768 7.65 and 7.30, 2304 13.9 and 13.5, 3072 with GELU 17.1 and 16.5, 1024^3 7.2 and 6.8, 512 x 768 -> 3072 8.35 and 7.95).
+#define ET_DMA_FIRST const _Float16 *A, const _Float16 *B, const _Float16 *bias, int M, int N, int K, int lda, int ldb, int group_rows, unsigned per_row
 template <int TMW, int TNW, int NBUF, bool IDX, bool RAGGED = false, bool BT = false, int KS = kDmaK, int NWN = 2>
-__global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(const GemmArgs ga) {
+__global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(ET_DMA_FIRST, const GemmArgs ga) {
     static_assert(NWN == 2 || (NWN == 4 && !RAGGED && !BT), "eight waves are written for whole tiles");
     constexpr int kWaves = 2 * NWN;
     static_assert(NBUF >= 2 && NBUF <= 4 && (NBUF - 1) * (2 * TMW + 2 * TNW) * KS / kDmaK <= 63, "vmcnt holds 63 loads");
     static_assert(KS == kDmaK || (KS == 32 && !RAGGED && !BT), "half stages are written for whole tiles");
     static_assert(!BT || (TMW == 1 && TNW == 1 && RAGGED), "the k-major B stage is written for the 64 x 64 tile");
     GemmArgs g = ga;
-    {
+    g.A = A, g.B = B, g.bias = bias, g.M = M, g.N = N, g.K = K, g.lda = lda, g.ldb = ldb;
+    if (TMW == 1 && TNW == 1 && blockIdx.y) {  // (several problems run on 64 x 64 tiles)
         const long long zo = blockIdx.y / g.batch_inner, zi = blockIdx.y % g.batch_inner;
         g.A += zo * g.sAo + zi * g.sAi;
         g.B += zo * g.sBo + zi * g.sBi;
@@ -80,27 +84,32 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(const GemmArgs 
     // tiles to within one group; dealing whole 4 x 8 blocks instead gave the XCDs with odd numbers only the
     // half-empty blocks of a result 12 tiles wide.
     const int tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BN - 1) / BN;
-    const int sbm = g.group_rows, gsh = sbm == 4 ? 5 : sbm == 2 ? 4 : 3;  // a group: sbm x 8 = 1 << gsh tiles
+    const int sbm = group_rows, gsh = sbm == 4 ? 5 : sbm == 2 ? 4 : 3;  // a group: sbm x 8 = 1 << gsh tiles
     const int xcd = blockIdx.x % kDmaXcds, j = blockIdx.x / kDmaXcds;
     const int t = ((((j >> gsh) * kDmaXcds + xcd)) << gsh) + (j & ((1 << gsh) - 1));
     if (t >= tiles_m * tiles_n) return;  // padding of the grid (whole workgroup)
     int ty, tx;
     {
-        const int per_br = sbm * tiles_n, full_br = tiles_m / sbm;  // tiles of a full block row; such rows
-        const int br = min(t / per_br, full_br);
+        // (no division that the scalar unit would spend 150 cycles on: `per_row` is 2^32 over the tiles of a block row, rounded up, or 0
+        // where that would not be exact; a block is 1 to 4 tiles high and 1 to 8 wide)
+        const int per_br = sbm * tiles_n, full_br = tiles_m >> (gsh - 3);  // tiles of a full block row; such rows
+        const int br = min(per_row ? (int)(((unsigned long long)(unsigned)t * per_row) >> 32) : t / per_br, full_br);
         const int rem = t - br * per_br;
         if (br < full_br && (tiles_n & (kSbN - 1)) == 0) {  // whole blocks only: shifts
             const int q = rem & ((1 << gsh) - 1);
             ty = br * sbm + (q >> 3);
             tx = (rem >> gsh) * kSbN + (q & 7);
         } else {
+            static_assert(kSbM == 4 && kSbN == 8, "the divisions below");
             const int rows = br < full_br ? sbm : tiles_m - full_br * sbm;  // tile rows of this block row
             const int per_bc = rows * kSbN, full_bc = tiles_n / kSbN;
-            const int bc = min(rem / per_bc, full_bc);
+            const unsigned eights = (unsigned)rem >> 3;
+            const int bc = min((int)(rows == 3 ? (unsigned)(((unsigned long long)eights * 0x55555556u) >> 32) : eights >> (rows >> 1)), full_bc);
             const int q = rem - bc * per_bc;
             const int w = bc < full_bc ? kSbN : tiles_n - full_bc * kSbN;  // tile columns of this block
-            ty = br * sbm + q / w;
-            tx = bc * kSbN + q % w;
+            const int over = w == 1 ? q : (q * (int)(0x00805640342b2520ull >> (64 - 8 * w) & 255)) >> 8;  // q / w, q < 32
+            ty = br * sbm + over;
+            tx = bc * kSbN + q - over * w;
         }
     }
     const int m0 = ty * BM, n0 = tx * BN;
@@ -161,7 +170,9 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(const GemmArgs 
     // 4j .. 4j + 3 of an operand share one LDS base (M0) and differ in the immediate, 1024 (v % 4), which the
     // lane's global offset has subtracted again.  One write of M0 per four loads instead of one per load.
     unsigned offA[kLA], offB[kLB];  // bytes from the tile's first row at k = 0, minus the immediate
-    unsigned tailA[RAGGED ? kLA : 1], tailB[RAGGED ? kLB : 1];  // the same for a last stage that K ends in
+    // what a last stage that K ends in adds to them: rows 16 apart have the same chunk at a position, so loads of even and of odd number
+    // have one each (held for every load they were up to 32 registers)
+    unsigned tail_by[2] = {0, 0};
     const int k_tail0 = (g.K - 1) / KS * KS;   // first k of the last stage
     const int k_tail = g.K - k_tail0;          // k-values of the last stage, 16 .. KS
     if (kWhole) {
@@ -172,7 +183,7 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(const GemmArgs 
             const int row = RAGGED ? min(m0 + r, g.M - 1) - m0 : r;
             const int c8 = (lp ^ swz_of(r)) * 8;
             offA[v] = (unsigned)((row * g.lda + c8) * 2 - (kImm ? (v % 4) * 1024 : 0));
-            if (RAGGED) tailA[v] = (unsigned)((row * g.lda + min(c8, k_tail - 8)) * 2);
+            if (RAGGED && v < 2) tail_by[v] = (unsigned)((min(c8, k_tail - 8) - c8) * 2);
         }
 #pragma unroll
         for (int v = 0; v < kLB; v++) {
@@ -180,7 +191,6 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(const GemmArgs 
             const int row = RAGGED ? min(n0 + r, g.N - 1) - n0 : r;
             const int c8 = (lp ^ swz_of(r)) * 8;
             offB[v] = (unsigned)((row * g.ldb + c8) * 2 - (kImm ? (v % 4) * 1024 : 0));
-            if (RAGGED) tailB[v] = (unsigned)((row * g.ldb + min(c8, k_tail - 8)) * 2);
         }
     }
     // Requests past the last stage are needed for the count of those outstanding, not for their data: through a buffer without
@@ -206,17 +216,19 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(const GemmArgs 
         };
         auto ra = __builtin_amdgcn_make_buffer_rsrc(a_tile, 0, records, 0x00020000);
         auto rb = __builtin_amdgcn_make_buffer_rsrc(b_tile, 0, records, 0x00020000);
+        static_assert(!RAGGED || (kRpi == 8 && BM / kWaves % 16 == 0 && BN / kWaves % 16 == 0 && kLA >= 2), "the chunks of a last stage");
         const bool tail = RAGGED && k0 == k_tail0 && k_tail < KS;  // uniform
+        const unsigned by[2] = {tail ? tail_by[0] : 0u, tail ? tail_by[1] : 0u};
 #pragma unroll
         for (int v = 0; v < kLA; v++)
             if (v >= first && v < first + count) {
-                const unsigned off = RAGGED && tail ? tailA[RAGGED ? v : 0] : offA[v];
+                const unsigned off = RAGGED ? offA[v] + by[v & 1] : offA[v];
                 four(ra, off, As + (buf * BM + wave * (BM / kWaves) + (kImm ? (v / 4) * 4 : v) * kRpi) * KS, kImm ? v % 4 : 0);
             }
 #pragma unroll
         for (int v = 0; v < kLB; v++)
             if (kLA + v >= first && kLA + v < first + count) {
-                const unsigned off = RAGGED && tail ? tailB[RAGGED ? v : 0] : offB[v];
+                const unsigned off = RAGGED ? offB[v] + by[v & 1] : offB[v];
                 four(rb, off, Bs + (buf * BN + wave * (BN / kWaves) + (kImm ? (v / 4) * 4 : v) * kRpi) * KS, kImm ? v % 4 : 0);
             }
     };
@@ -539,8 +551,8 @@ static int launch_dma_variant(const GemmArgs &g, int batch, hipStream_t stream) 
     const long long groups = (total + sbm * kSbN - 1) / (sbm * kSbN);
     const long long rounds = (groups + kDmaXcds - 1) / kDmaXcds;
     const dim3 grid((unsigned)(rounds * kDmaXcds * sbm * kSbN), (unsigned)batch);
-    GemmArgs ga = g;
-    ga.group_rows = sbm;
+    const unsigned long long per_br = (unsigned long long)sbm * tiles_n, most = (unsigned long long)grid.x * per_br;
+    const unsigned per_row = per_br > 1 && most < 1ull << 32 ? (unsigned)(((1ull << 32) + per_br - 1) / per_br) : 0;
     auto kernel = gemm_f16_dma_kernel<TMW, TNW, NBUF, IDX, RAGGED, BT, KS, NWN>;
     static bool raised = false;  // more than 64 KB of dynamic LDS needs the attribute, once per kernel
     if (!raised) {
@@ -548,7 +560,7 @@ static int launch_dma_variant(const GemmArgs &g, int batch, hipStream_t stream) 
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         raised = true;
     }
-    kernel<<<grid, 128 * NWN, lds, stream>>>(ga);
+    kernel<<<grid, 128 * NWN, lds, stream>>>(g.A, g.B, g.bias, g.M, g.N, g.K, g.lda, g.ldb, sbm, per_row, g);
     return check_launch("gemm_f16_dma_kernel");
 }
 
