@@ -166,21 +166,41 @@ template <int HD, int NW, bool COMPACT, int QT> constexpr bool mha_three_waves()
     return mha_prefetches<HD, NW, COMPACT, QT>() && NW == 4;
 }
 
+// The arguments that the first requests need, in front of the others and one by one: preloaded into scalar registers.  With the place
+// from the grid, no divisions and the first block asked for ahead of the queries, us, before and now, 12 heads of 64: 1 x 128 keys 4.47 and 4.34, 8 x 128 4.67 and
+// 4.55, 1 x 16 4.25 and 4.04.
+#define ET_MHA_FIRST const _Float16 *K, const _Float16 *V, const _Float16 *Q, const int32_t *lens, int ldk, int ldv, int S0, int nbh, unsigned heads, unsigned per_head
+__device__ __forceinline__ MhaArgs mha_args(ET_MHA_FIRST, const MhaArgs &rest) {
+    MhaArgs a = rest;
+    a.K = K, a.V = V, a.Q = Q, a.lens = lens, a.ldk = ldk, a.ldv = ldv, a.S = S0, a.nbh = nbh, a.nh = heads >> 8, a.hd = heads & 255;
+    if (heads == 0) {  // they do not fit one word (256 columns, 2^24 heads); read from memory, behind a branch the compiler cannot undo
+        auto *late = (const __attribute__((address_space(4))) MhaArgs *)((const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr() + 56);
+        asm volatile("" : "+s"(late));
+        a.nh = late->nh;
+        a.hd = late->hd;
+    }
+    return a;
+}
+// row of the grid
+__device__ __forceinline__ unsigned mha_row() { return blockIdx.y + (blockIdx.z << 15); }
+#define ET_MHA_TAKE const MhaArgs a = mha_args(K, V, Q, lens, ldk, ldv, S0, nbh, heads, per_head, rest)
 template <int HD, bool COMPACT, int NW, int QT>
 __global__ __launch_bounds__(64 * NW)
     __attribute__((amdgpu_waves_per_eu(HD > 128 ? 2 : mha_three_waves<HD, NW, COMPACT, QT>() ? 3 : 1, HD > 128 ? 2 : mha_three_waves<HD, NW, COMPACT, QT>() ? 3 : 8))) void
-    mha_fused_kernel(const MhaArgs a) {
+    mha_fused_kernel(ET_MHA_FIRST, const MhaArgs rest) {
+    ET_MHA_TAKE;
     constexpr bool kCoherentZ = false;
     constexpr int KB = mha_key_block<HD>();
-    const unsigned block = blockIdx.x;
+    const int bh = blockIdx.x % kXcds + kXcds * mha_row(), qstrip = blockIdx.x / kXcds;
 #include "attention_body.inc"
 }
 
 // 256 columns in blocks of 128 keys: a workgroup has its compute unit and a wave its SIMD's registers to itself (mha_wide_blocks)
-__global__ __launch_bounds__(256) void mha_wide_kernel(const MhaArgs a) {
+__global__ __launch_bounds__(256) void mha_wide_kernel(ET_MHA_FIRST, const MhaArgs rest) {
+    ET_MHA_TAKE;
     constexpr int HD = 256, NW = 4, QT = 1, KB = kKeyBlock;
     constexpr bool COMPACT = false, kCoherentZ = false;
-    const unsigned block = blockIdx.x;
+    const int bh = blockIdx.x % kXcds + kXcds * mha_row(), qstrip = blockIdx.x / kXcds;
 #include "attention_body.inc"
 }
 
@@ -188,22 +208,26 @@ __global__ __launch_bounds__(256) void mha_wide_kernel(const MhaArgs a) {
 // since the argument to tell them apart by is a wait of its own at the start: 12 layers of one sequence 335 -> 342 us)
 template <int HD, int NW, int QT>
 __global__ __launch_bounds__(64 * NW)
-    __attribute__((amdgpu_waves_per_eu(mha_three_waves<HD, NW, false, QT>() ? 3 : 1, mha_three_waves<HD, NW, false, QT>() ? 3 : 8))) void
-    mha_fused_ahead_kernel(const MhaArgs a) {
+    __attribute__((amdgpu_waves_per_eu(1, 8))) void
+    mha_fused_ahead_kernel(ET_MHA_FIRST, const MhaArgs rest) {
+    if (mha_row() < rest.ahead_blocks) return ahead_of(rest, mha_row() * gridDim.x + blockIdx.x);
+    ET_MHA_TAKE;
     constexpr bool kCoherentZ = false, COMPACT = false;
     constexpr int KB = mha_key_block<HD>();
-    if (blockIdx.x < a.ahead_blocks) return ahead_of(a, blockIdx.x);
-    const unsigned block = blockIdx.x - a.ahead_blocks;
+    const int bh = blockIdx.x % kXcds + kXcds * (mha_row() - a.ahead_blocks), qstrip = blockIdx.x / kXcds;
 #include "attention_body.inc"
 }
 template <int HD, bool COMPACT, int NW> constexpr bool mha_takes_ahead() { return HD <= 64 && !COMPACT && NW >= 4; }
 
 template <int HD, bool COMPACT, int NW, int QT, int KB = mha_key_block<HD>()>
 static int launch_mha_nw(const MhaArgs &args, hipStream_t stream) {
-    void (*kernel)(MhaArgs) = HD == 256 && KB == kKeyBlock ? mha_wide_kernel : mha_fused_kernel<HD, COMPACT, NW, QT>;
+    auto kernel = HD == 256 && KB == kKeyBlock ? mha_wide_kernel : mha_fused_kernel<HD, COMPACT, NW, QT>;
     MhaArgs a = args;
+    const int qstrips = (args.S + 16 * NW * QT - 1) / (16 * NW * QT);
+    const int rounds = (args.nbh + kXcds - 1) / kXcds;
+    const unsigned width = (unsigned)(kXcds * qstrips);  // of the grid; its rows: (sequence, head) pairs by eights
     if constexpr (mha_takes_ahead<HD, COMPACT, NW>()) {
-        a.ahead_blocks = ahead_blocks(a, 64 * NW);
+        a.ahead_blocks = std::min((ahead_blocks(a, 64 * NW) + width - 1) / width, 32767u);  // rows of the grid
         if (a.ahead_blocks) kernel = mha_fused_ahead_kernel<HD, NW, QT>;
     }
     constexpr size_t lds = MhaLds<HD, KB>::bytes;
@@ -216,9 +240,10 @@ static int launch_mha_nw(const MhaArgs &args, hipStream_t stream) {
             raised = true;
         }
     }
-    const int qstrips = (args.S + 16 * NW * QT - 1) / (16 * NW * QT);
-    const int rounds = (args.nbh + kXcds - 1) / kXcds;
-    kernel<<<dim3(a.ahead_blocks + (unsigned)(rounds * kXcds * qstrips)), 64 * NW, lds, stream>>>(a);
+    const unsigned per_head = a.nh > 1 && (unsigned long long)a.nbh * a.nh < 1ull << 32 ? (unsigned)(((1ull << 32) + a.nh - 1) / a.nh) : 0;
+    const unsigned heads = a.nh < 1 << 24 && a.hd < 256 ? (unsigned)a.nh << 8 | (unsigned)a.hd : 0;
+    const unsigned rows = (unsigned)rounds + a.ahead_blocks;
+    kernel<<<dim3(width, std::min(rows, 32768u), (rows + 32767) / 32768), 64 * NW, lds, stream>>>(a.K, a.V, a.Q, a.lens, a.ldk, a.ldv, a.S, a.nbh, heads, per_head, a);
     return check_launch("mha_fused_kernel");
 }
 
@@ -512,7 +537,10 @@ static int launch_mha(const MhaArgs &args, hipStream_t stream) {
         if (f.in_turn) return f.ragged ? launch_mha_pingpong<true>(args, stream) : launch_mha_pingpong<false>(args, stream);
     }
     if constexpr (HD >= 64 && !COMPACT) {
-        if (f.tiles == 2) return launch_mha_nw<HD, COMPACT, 8, 2>(args, stream);
+        // (128-wide heads with two tiles took all registers and spilled 49: level with one tile at 2048 keys, 2 to 25 % behind it below)
+        if constexpr (HD != 128) {
+            if (f.tiles == 2) return launch_mha_nw<HD, COMPACT, 8, 2>(args, stream);
+        }
         if (f.waves == 8) return launch_mha_nw<HD, COMPACT, 8, 1>(args, stream);
     }
     if constexpr (HD == 32) {
@@ -560,7 +588,9 @@ __global__ __launch_bounds__(64 * NW) void mha_fuseo_kernel(const MhaArgs a, con
     constexpr bool COMPACT = false;
     constexpr bool kCoherentZ = true;
     constexpr int KB = mha_key_block<HD>();
-    const unsigned block = blockIdx.x;
+    constexpr unsigned per_head = 0;
+    const int qstrips = (a.S + 16 * NW * QT - 1) / (16 * NW * QT), k_in_xcd = blockIdx.x / kXcds;
+    const int bh = blockIdx.x % kXcds + kXcds * (k_in_xcd / qstrips), qstrip = k_in_xcd % qstrips;
 #include "attention_body.inc"
     // ---- arrival.  Z was stored at device scope, and such a store counts as complete only once it has
     // reached the memory side: when every wave's stores are complete the count moves.  A device-wide fence
