@@ -18,6 +18,9 @@ SHAPES = [
     (8, 784, 12, 64, True, [784, 3, 33, 783], T41), (16, 400, 16, 64, True, None, T81), (20, 176, 12, 64, False, [176, 129, 128, 31], T81),
     (1, 400, 12, 56, False, None, T44), (3, 528, 12, 64, True, [390, 5], T44), (1, 528, 12, 64, False, [515], T42), (2, 1040, 12, 64, True, None, T42),
     (2, 784, 16, 64, False, [784, 130], T82),
+    # sequences of no keys whose tiles are shared
+    (3, 400, 16, 64, False, [400, 77, 0], T82), (3, 528, 12, 64, True, [528, 77, 0], T44), (3, 528, 12, 24, False, [528, 77, 0], T42),
+    (3, 400, 8, 128, False, [400, 77, 0], T42), (3, 272, 4, 200, False, [272, 77, 0], (4, 2, 1)),
     (20, 512, 12, 32, False, [512, 100, 0], T41), (3, 400, 12, 24, True, None, T44), (4, 272, 12, 32, False, None, T42),
     (8, 272, 10, 80, False, [272, 75, 0], T41), (8, 400, 10, 96, True, None, T81), (1, 400, 10, 80, False, None, T42), (3, 784, 10, 88, False, None, T82),
     (4, 528, 8, 128, False, [528, 513, 7], T41), (12, 272, 8, 120, True, None, T81), (1, 400, 8, 128, False, [399], T44), (2, 1040, 8, 128, True, None, T42),
