@@ -50,13 +50,15 @@ typedef float f16v __attribute__((ext_vector_type(16)));
 // The arguments in front are what the first requests need: preloaded into scalar registers (us, before and now, with the tile found without divisions: 2048 x 768 ->
 // 768 7.65 and 7.30, 2304 13.9 and 13.5, 3072 with GELU 17.1 and 16.5, 1024^3 7.2 and 6.8, 512 x 768 -> 3072 8.35 and 7.95).
 #define ET_DMA_FIRST const _Float16 *A, const _Float16 *B, const _Float16 *bias, int M, int N, int K, int lda, int ldb, int group_rows, unsigned per_row
-template <int TMW, int TNW, int NBUF, bool IDX, bool RAGGED = false, bool BT = false, int KS = kDmaK, int NWN = 2>
+// LINES (ragged tiles through four buffers): rows that begin off a 128-byte line.
+template <int TMW, int TNW, int NBUF, bool IDX, bool RAGGED = false, bool BT = false, int KS = kDmaK, int NWN = 2, bool LINES = false>
 __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(ET_DMA_FIRST, const GemmArgs ga) {
     static_assert(NWN == 2 || (NWN == 4 && !RAGGED && !BT), "eight waves are written for whole tiles");
     constexpr int kWaves = 2 * NWN;
     static_assert(NBUF >= 2 && NBUF <= 4 && (NBUF - 1) * (2 * TMW + 2 * TNW) * KS / kDmaK <= 63, "vmcnt holds 63 loads");
     static_assert(KS == kDmaK || (KS == 32 && !RAGGED && !BT), "half stages are written for whole tiles");
     static_assert(!BT || (TMW == 1 && TNW == 1 && RAGGED), "the k-major B stage is written for the 64 x 64 tile");
+    static_assert(!LINES || (RAGGED && !BT && NBUF == 4 && KS == 64), "rows by lines are written for four buffers of 64");
     GemmArgs g = ga;
     g.A = A, g.B = B, g.bias = bias, g.M = M, g.N = N, g.K = K, g.lda = lda, g.ldb = ldb;
     if (TMW == 1 && TNW == 1 && blockIdx.y) {  // (several problems run on 64 x 64 tiles)
@@ -175,6 +177,24 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(ET_DMA_FIRST, c
     unsigned tail_by[2] = {0, 0};
     const int k_tail0 = (g.K - 1) / KS * KS;   // first k of the last stage
     const int k_tail = g.K - k_tail0;          // k-values of the last stage, 16 .. KS
+    // LINES: a stage's 128 bytes of a row that begins off a line lie in two lines, and the L1 does not hold the other part until the
+    // next stage asks for it: 1.25 to 1.3 times the time (2048 x 3056 -> 768 22.7 us, 3072 17.6).  So a request fetches whole lines: line l
+    // of a row are its chunks 8 l - shift .. + 7, `shift` the row's chunks off a line, and stage s reads lines s and s + 1 (a fragment's chunk lies
+    // shift further, in the next buffer past 8).  A lane's rows are multiples of 8 apart and so have one shift, in the requests as in the fragments.
+    // Chunks ahead of a row or past its end are its first or last one instead, which no product takes.  us, before and now: 2048 x 3056 -> 768 22.7 and 18.9,
+    // 4096 x 2032 -> 2048 51.4 and 42.2, 1104 x 1040 -> 3072 14.4 and 12.3, 8192 x 4080 -> 4096 369 and 323, 110 Linears of 256 to 8192 rows 0.94 of their
+    // time in the mean; the same bits.
+    int line_a[2] = {0, 0}, line_b[2] = {0, 0};              // chunk of line 0 that the lane's loads of even and of odd number fetch
+    unsigned by_a[2] = {0, 0}, by_b[2] = {0, 0};             // bytes to that of the line asked for
+    auto shift_of = [](const _Float16 *first, int row, int ld) { return (int)(((unsigned)(reinterpret_cast<uintptr_t>(first) >> 4) + (unsigned)row * (unsigned)(ld >> 3)) & 7); };
+    const int chunks = g.K >> 3;
+    auto at_line = [&](int line) {
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            by_a[e] = (unsigned)min(max(line_a[e] + line * 8, 0), chunks - 1) * 16;
+            by_b[e] = (unsigned)min(max(line_b[e] + line * 8, 0), chunks - 1) * 16;
+        }
+    };
     if (kWhole) {
         const int lr = lane / kLpr, lp = lane % kLpr;
 #pragma unroll
@@ -184,6 +204,8 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(ET_DMA_FIRST, c
             const int c8 = (lp ^ swz_of(r)) * 8;
             offA[v] = (unsigned)((row * g.lda + c8) * 2 - (kImm ? (v % 4) * 1024 : 0));
             if (RAGGED && v < 2) tail_by[v] = (unsigned)((min(c8, k_tail - 8) - c8) * 2);
+            if (LINES) offA[v] = (unsigned)(row * g.lda * 2);
+            if (LINES && v < 2) line_a[v] = (c8 >> 3) - shift_of(g.A, m0 + lr, g.lda);
         }
 #pragma unroll
         for (int v = 0; v < kLB; v++) {
@@ -191,6 +213,8 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(ET_DMA_FIRST, c
             const int row = RAGGED ? min(n0 + r, g.N - 1) - n0 : r;
             const int c8 = (lp ^ swz_of(r)) * 8;
             offB[v] = (unsigned)((row * g.ldb + c8) * 2 - (kImm ? (v % 4) * 1024 : 0));
+            if (LINES) offB[v] = (unsigned)(row * g.ldb * 2);
+            if (LINES && v < 2) line_b[v] = (c8 >> 3) - shift_of(g.B, n0 + lr, g.ldb);
         }
     }
     // Requests past the last stage are needed for the count of those outstanding, not for their data: through a buffer without
@@ -217,18 +241,18 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(ET_DMA_FIRST, c
         auto ra = __builtin_amdgcn_make_buffer_rsrc(a_tile, 0, records, 0x00020000);
         auto rb = __builtin_amdgcn_make_buffer_rsrc(b_tile, 0, records, 0x00020000);
         static_assert(!RAGGED || (kRpi == 8 && BM / kWaves % 16 == 0 && BN / kWaves % 16 == 0 && kLA >= 2), "the chunks of a last stage");
-        const bool tail = RAGGED && k0 == k_tail0 && k_tail < KS;  // uniform
+        const bool tail = RAGGED && !LINES && k0 == k_tail0 && k_tail < KS;  // uniform
         const unsigned by[2] = {tail ? tail_by[0] : 0u, tail ? tail_by[1] : 0u};
 #pragma unroll
         for (int v = 0; v < kLA; v++)
             if (v >= first && v < first + count) {
-                const unsigned off = RAGGED ? offA[v] + by[v & 1] : offA[v];
+                const unsigned off = RAGGED ? offA[v] + (LINES ? by_a[v & 1] : by[v & 1]) : offA[v];
                 four(ra, off, As + (buf * BM + wave * (BM / kWaves) + (kImm ? (v / 4) * 4 : v) * kRpi) * KS, kImm ? v % 4 : 0);
             }
 #pragma unroll
         for (int v = 0; v < kLB; v++)
             if (kLA + v >= first && kLA + v < first + count) {
-                const unsigned off = RAGGED ? offB[v] + by[v & 1] : offB[v];
+                const unsigned off = RAGGED ? offB[v] + (LINES ? by_b[v & 1] : by[v & 1]) : offB[v];
                 four(rb, off, Bs + (buf * BN + wave * (BN / kWaves) + (kImm ? (v / 4) * 4 : v) * kRpi) * KS, kImm ? v % 4 : 0);
             }
     };
@@ -311,7 +335,7 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(ET_DMA_FIRST, c
     // MFMA a slice hides little either way, and the deep form asks for a stage half a stage later (719 of 728 ragged Linears of 16..2048
     // rows slower, by 1 to 9 %: 784 x 3072 -> 768 15.9 us deep, 14.6 so, 400 x 4096 -> 1024 19.0 and 18.0; whole tiles are 8 % slower
     // the other way, 1024 x 4096 -> 1024 18.0 and 19.4).
-    constexpr bool kDeep = kWhole && NBUF == 4 && NWN == 2 && !(RAGGED && TMW * TNW == 1);
+    constexpr bool kDeep = kWhole && NBUF == 4 && NWN == 2 && (LINES || !(RAGGED && TMW * TNW == 1));
     constexpr int kStageLoads = kWhole ? kLA + kLB : 2 * TMW + 2 * TNW;  // per wave
     auto wait_stages = [&](int later) {  // wait until at most `later` whole stages are outstanding
         if (later <= 0) __builtin_amdgcn_s_waitcnt(wait_vm(0));
@@ -333,23 +357,55 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(ET_DMA_FIRST, c
     constexpr int kLoadSteps = KS == 32 ? 2 : 1;      // steps of a stage that issue a share of a later stage's loads
     constexpr int kStepLoads = (kStageLoads + kLoadSteps - 1) / kLoadSteps;  // in the first such step; the rest in the second
     constexpr int kStepLoads2 = kStageLoads - kStepLoads;
+    // LINES: where in the buffers, from a stage's own on, a lane finds its chunk of a slice; round the end of the ring
+    unsigned line_x[kSlices], line_w[kSlices];
+    if constexpr (LINES) {
+        const int sx = kg + shift_of(g.A, m0 + l32, g.lda), sw = kg + shift_of(g.B, n0 + l32, g.ldb);
+#pragma unroll
+        for (int ks = 0; ks < kSlices; ks++) {
+            line_x[ks] = (unsigned)((((2 * ks + sx) & 7) ^ swz) * 8 + ((2 * ks + sx) >> 3) * (BM * KS));
+            line_w[ks] = (unsigned)((((2 * ks + sw) & 7) ^ swz) * 8 + ((2 * ks + sw) >> 3) * (BN * KS));
+        }
+    }
+    auto ring = [](unsigned at, unsigned whole) { return min(at, at - whole); };
+    auto read_x = [&](Frag &f, int i, int buf, int ks) {
+        if constexpr (LINES) f.x[i] = *reinterpret_cast<const h8 *>(a_rows + ring(buf * BM * KS + line_x[ks], NBUF * BM * KS) + i * 32 * KS);
+        else f.x[i] = *reinterpret_cast<const h8 *>(a_rows + buf * BM * KS + ((ks * 2 + kg) ^ swz) * 8 + i * 32 * KS);
+    };
+    auto read_w = [&](Frag &f, int j, int buf, int ks) {
+        if constexpr (LINES) f.w[j] = *reinterpret_cast<const h8 *>(b_rows + ring(buf * BN * KS + line_w[ks], NBUF * BN * KS) + j * 32 * KS);
+        else f.w[j] = *reinterpret_cast<const h8 *>(b_rows + buf * BN * KS + ((ks * 2 + kg) ^ swz) * 8 + j * 32 * KS);
+    };
+    auto read_slice = [&](Frag &f, int buf, int ks) {
+#pragma unroll
+        for (int i = 0; i < TMW; i++) read_x(f, i, buf, ks);
+#pragma unroll
+        for (int j = 0; j < TNW; j++) read_w(f, j, buf, ks);
+    };
     auto step = [&](const Frag &fm, Frag &fr, int rbuf, int rks, int nload, int lbuf, int k_later, int first) {
-        const int chunk = ((rks * 2 + kg) ^ swz) * 8;
 #pragma unroll
         for (int m = 0; m < kNM; m++) {
             const int i = m / TNW, j = m % TNW;
             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fm.w[j], fm.x[i], acc[i][j], 0, 0, 0);
 #pragma unroll
             for (int idx = m * kND / kNM; idx < (m + 1) * kND / kNM; idx++) {
-                if (idx < TMW) fr.x[idx] = *reinterpret_cast<const h8 *>(a_rows + rbuf * BM * KS + chunk + idx * 32 * KS);
-                else fr.w[idx - TMW] = *reinterpret_cast<const h8 *>(b_rows + rbuf * BN * KS + chunk + (idx - TMW) * 32 * KS);
+                if (idx < TMW) read_x(fr, idx, rbuf, rks);
+                else read_w(fr, idx - TMW, rbuf, rks);
             }
             if (nload > 0) load_part(lbuf, k_later, first + m * nload / kNM, (m + 1) * nload / kNM - m * nload / kNM);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
     Frag f0, f1;
-    if constexpr (kWhole) {
+    if constexpr (LINES) {
+#pragma unroll
+        for (int p = 0; p < NBUF; p++) {
+            aim(nstage + 1 - p);
+            at_line(p);
+            load_part(p, 0, 0, kStageLoads);
+        }
+        __builtin_amdgcn_s_waitcnt(wait_vm(2 * kStageLoads));  // lines 0 and 1 have landed
+    } else if constexpr (kWhole) {
 #pragma unroll
         for (int p = 0; p < kAhead; p++) {
             aim(nstage - p);
@@ -363,11 +419,36 @@ __global__ __launch_bounds__(128 * NWN) void gemm_f16_dma_kernel(ET_DMA_FIRST, c
         wait_stages(min(kAhead, nstage) - 1);
     }
     if constexpr (IDX) load_bias();
-    if (RAGGED && nstage == 1 && ktail < kDmaK) zero_tail(0);
+    if (RAGGED && !LINES && nstage == 1 && ktail < kDmaK) zero_tail(0);
     lds_barrier();
-    read_frag(f0, 0, 0);
+    if constexpr (LINES) read_slice(f0, 0, 0);
+    else read_frag(f0, 0, 0);
     int cur = 0;
-    if constexpr (kDeep) {
+    if constexpr (LINES) {
+        // As the deep form below, but the barrier in the middle of a stage waits for the stage's reads too: its own buffer, whose line no
+        // later stage reads, takes line s + 4.
+        Frag f2, f3;
+        read_slice(f1, 0, 1);
+        for (int s = 0; s < nstage - 1; s++) {
+            const int nxt = (cur + 1) & 3;
+            aim(nstage + 1 - s - NBUF);
+            at_line(s + NBUF);
+            step(f0, f2, cur, 2, 0, cur, 0, 0);
+            step(f1, f3, cur, 3, 0, cur, 0, 0);
+            __builtin_amdgcn_s_waitcnt(wait_vm(kStageLoads));  // lines up to s + 2 have landed, s + 3 may be on its way
+            lds_barrier();
+            step(f2, f0, nxt, 0, kStageLoads / 2, cur, 0, 0);
+            step(f3, f1, nxt, 1, kStageLoads - kStageLoads / 2, cur, 0, kStageLoads / 2);
+            cur = nxt;
+        }
+        // the slices of the last stage that K has
+        if (k_tail > 32) read_slice(f2, cur, 2);
+        if (k_tail > 48) read_slice(f3, cur, 3);
+        multiply(f0);
+        if (k_tail > 16) multiply(f1);
+        if (k_tail > 32) multiply(f2);
+        if (k_tail > 48) multiply(f3);
+    } else if constexpr (kDeep) {
         // One stage of the deep form.  A slice's fragments are read two slices ahead: with one wave on the SIMD, a slice of
         // TMW x TNW MFMAs (32 cycles each) is shorter than the return of the reads dealt between them, and each slice
         // waited for the last of its own (128 x 128 tile: 1170 cycles a stage, 850 with this order, of which the LDS port
@@ -533,7 +614,7 @@ bool gemm_dma_applies(const GemmArgs &g, int batch, bool trans_b) {
     return pick_dma_tile(g.M, g.N, g.K, batch, trans_b, &t);
 }
 
-template <int TMW, int TNW, int NBUF, bool IDX, bool RAGGED, bool BT = false, int KS = kDmaK, int NWN = 2>
+template <int TMW, int TNW, int NBUF, bool IDX, bool RAGGED, bool BT = false, int KS = kDmaK, int NWN = 2, bool LINES = false>
 static int launch_dma_variant(const GemmArgs &g, int batch, hipStream_t stream) {
     constexpr int BM = 64 * TMW, BN = 32 * NWN * TNW;
     constexpr size_t lds = dma_lds_bytes(TMW, TNW, NBUF, KS, NWN);
@@ -553,7 +634,7 @@ static int launch_dma_variant(const GemmArgs &g, int batch, hipStream_t stream) 
     const dim3 grid((unsigned)(rounds * kDmaXcds * sbm * kSbN), (unsigned)batch);
     const unsigned long long per_br = (unsigned long long)sbm * tiles_n, most = (unsigned long long)grid.x * per_br;
     const unsigned per_row = per_br > 1 && most < 1ull << 32 ? (unsigned)(((1ull << 32) + per_br - 1) / per_br) : 0;
-    auto kernel = gemm_f16_dma_kernel<TMW, TNW, NBUF, IDX, RAGGED, BT, KS, NWN>;
+    auto kernel = gemm_f16_dma_kernel<TMW, TNW, NBUF, IDX, RAGGED, BT, KS, NWN, LINES>;
     static bool raised = false;  // more than 64 KB of dynamic LDS needs the attribute, once per kernel
     if (!raised) {
         ET_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
@@ -564,10 +645,16 @@ static int launch_dma_variant(const GemmArgs &g, int batch, hipStream_t stream) 
     return check_launch("gemm_f16_dma_kernel");
 }
 
-template <int TMW, int TNW, int NBUF, bool RAGGED = false, bool BT = false, int KS = kDmaK, int NWN = 2>
+// rows that do not all begin on a 128-byte line
+static bool off_lines(const _Float16 *p, int ld) { return ld % 64 || (reinterpret_cast<uintptr_t>(p) & 127); }
+
+template <int TMW, int TNW, int NBUF, bool RAGGED = false, bool BT = false, int KS = kDmaK, int NWN = 2, bool LINES = false>
 static int launch_dma_tile(const GemmArgs &g, int batch, hipStream_t stream) {
-    return (g.c_scatter || g.bias_idx) ? launch_dma_variant<TMW, TNW, NBUF, true, RAGGED, BT, KS, NWN>(g, batch, stream)
-                                       : launch_dma_variant<TMW, TNW, NBUF, false, RAGGED, BT, KS, NWN>(g, batch, stream);
+    if constexpr (RAGGED && !BT && NBUF == 4 && !LINES) {
+        if (off_lines(g.A, g.lda) || off_lines(g.B, g.ldb)) return launch_dma_tile<TMW, TNW, NBUF, true, false, KS, NWN, true>(g, batch, stream);
+    }
+    return (g.c_scatter || g.bias_idx) ? launch_dma_variant<TMW, TNW, NBUF, true, RAGGED, BT, KS, NWN, LINES>(g, batch, stream)
+                                       : launch_dma_variant<TMW, TNW, NBUF, false, RAGGED, BT, KS, NWN, LINES>(g, batch, stream);
 }
 
 int launch_gemm_dma(const GemmArgs &g, int batch, bool trans_b, hipStream_t stream) {
@@ -576,6 +663,7 @@ int launch_gemm_dma(const GemmArgs &g, int batch, bool trans_b, hipStream_t stre
     if (!trans_b)
         return t.nbuf == 3 ? launch_dma_tile<1, 1, 3, true, true>(g, batch, stream)
                            : launch_dma_tile<1, 1, 2, true, true>(g, batch, stream);
+    if (t.ragged && (off_lines(g.A, g.lda) || off_lines(g.B, g.ldb))) t = dma_lines_tile(t, g.M, g.N, g.K);
     switch (t.tmw * 100 + t.tnw * 10 + t.nbuf + (t.ragged ? 1000 : 0)) {
         case 114: return launch_dma_tile<1, 1, 4>(g, 1, stream);
         case 124: return launch_dma_tile<1, 2, 4>(g, 1, stream);
@@ -595,6 +683,7 @@ int launch_gemm_dma(const GemmArgs &g, int batch, bool trans_b, hipStream_t stre
         case 1214: return launch_dma_tile<2, 1, 4, true>(g, 1, stream);
         case 1222: return launch_dma_tile<2, 2, 2, true>(g, 1, stream);
         case 1224: return launch_dma_tile<2, 2, 4, true>(g, 1, stream);
+        case 1234: return launch_dma_tile<2, 3, 4, true, false, kDmaK, 2, true>(g, 1, stream);  // (by lines only)
         case 1233: return launch_dma_tile<2, 3, 3, true>(g, 1, stream);
         case 1442: return launch_dma_tile<4, 4, 2, true>(g, 1, stream);
         default: return ET_ERR_UNSUPPORTED;

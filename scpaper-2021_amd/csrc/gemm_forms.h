@@ -63,6 +63,25 @@ inline bool pick_dma_tile(int M, int N, int K, int batch, bool trans_b, DmaTile 
     return true;
 }
 
+// The tile where rows begin off a 128-byte line, whose requests fetch whole lines through four buffers: one workgroup of 128 x 128 or more to a
+// compute unit, where the forms above hold two or three.  Time of this over the form above, 220 ragged Linears of 208 to 4080 inputs: forms of four
+// buffers 0.79 to 0.98, 128 x 192 0.78 to 0.89.  128 x 128 on two buffers: a tile a unit 0.82 to 0.88 (beyond, with fewer inputs, what two to a
+// unit hide weighs more: 0.90 to 1.19 below 944), from 1024 inputs on 0.78 to 1.02, from 944 where the last round is four fifths full 0.88 to 0.98;
+// 128 x 192 instead where it saves a round, to three rounds from 448 inputs on 0.78 to 0.81 (304 0.97), more rounds from 880 on 0.83 to 1.00.
+// 128 x 64 on two buffers: from 880 inputs on 0.86 to 0.90, below 1.10 to 1.44.
+inline DmaTile dma_lines_tile(DmaTile t, int M, int N, int K) {
+    if (t.tmw > 2 || t.nbuf == 4) return t;
+    auto tiles = [&](int wide) { return (long long)((M + 127) / 128) * ((N + wide - 1) / wide); };
+    auto rounds = [&](int wide) { return (tiles(wide) + 255) / 256; };
+    if (t.tnw == 3 || (t.tnw == 1 && K >= 880)) t.nbuf = 4;
+    if (t.tnw == 2) {
+        const long long r2 = rounds(128), r3 = rounds(192);
+        if (r2 > 1 && 13 * r3 < 10 * r2 && K >= (r2 <= 3 ? 448 : 880)) t.tnw = 3, t.nbuf = 4;
+        else if (r2 == 1 || K >= 1024 || (K >= 944 && 5 * tiles(128) >= 4 * 256 * r2)) t.nbuf = 4;
+    }
+    return t;
+}
+
 // The small-result kernel (one tile of 16 x 16 a workgroup, K in pieces of 64 over its four waves) applies when 64 x 64 tiles would
 // leave most of the chip idle: up to 768 tiles of 16 x 16, three workgroups to a compute unit; up to 1024 of at most 768 inputs, three
 // pieces a wave, and where the pieces of a wave fill two or more of its rounds of six loads (2817 to 3072 inputs).

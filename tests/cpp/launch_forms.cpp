@@ -1,5 +1,6 @@
 // Asks the rules that choose a kernel's form (csrc/*_forms.h) on the host.  One question a line of the standard input:
 //   gemm M N K batch trans_b dma_applies  ->  small | tile TMW TNW NBUF ragged | none
+//   lines M N K  ->  TMW TNW NBUF of a ragged problem whose rows begin off a 128-byte line
 //   wide S nbh  ->  keys of a block (heads of more than 224)
 //   mha HD compact S nbh causal plain padded  ->  waves WAVES TILES | turns ragged
 #include <cstdio>
@@ -18,6 +19,10 @@ int main() {
             if (et::takes_small_result(m, n, k, batch, tile)) puts("small");
             else if (tile) printf("tile %d %d %d %d\n", t.tmw, t.tnw, t.nbuf, (int)t.ragged);
             else puts("none");
+        } else if (sscanf(line, "lines %d %d %d", &m, &n, &k) == 3) {
+            et::DmaTile t{};
+            if (et::pick_dma_tile(m, n, k, 1, true, &t) && t.ragged) t = et::dma_lines_tile(t, m, n, k);
+            printf("%d %d %d\n", t.tmw, t.tnw, t.nbuf);
         } else if (sscanf(line, "mha %d %d %d %d %d %d %d", &m, &n, &k, &batch, &trans, &dma, &padded) == 7) {
             const et::MhaForm f = et::mha_form(m, n != 0, k, batch, trans != 0, dma != 0, padded != 0);
             if (f.in_turn) printf("turns %d\n", (int)f.ragged);

@@ -77,6 +77,58 @@ def test_linear_dense_and_row_pruned_in_every_tile(et, T, inp, out):
     assert (np.abs(d_s.numpy() - want) <= 2.0 ** -11 * np.abs(want) + 5e-4).all()
 
 
+# rows that begin off a 128-byte line, in every tile that fetches them by whole lines, with every number of slices in the last stage: the tile
+LINE_FORMS = [(144, 64, 144, "1 1 4"), (384, 16, 176, "1 1 4"), (192, 32, 144, "1 1 4"), (272, 48, 112, "1 1 4"), (400, 1040, 1040, "1 1 4"),
+              (448, 64, 4160, "1 2 4"), (560, 16, 3328, "1 2 4"), (432, 32, 4272, "1 2 4"), (688, 176, 2784, "1 2 4"),
+              (992, 192, 2144, "1 3 4"), (4880, 144, 416, "1 3 4"), (672, 160, 2960, "1 3 4"), (1568, 176, 1312, "1 3 4"),
+              (208, 192, 4368, "2 1 4"), (224, 144, 4112, "2 1 4"), (272, 160, 3280, "2 1 4"), (400, 176, 2416, "2 1 4"),
+              (5632, 912, 1024, "2 1 4"), (5520, 64, 352, "2 2 4"), (400, 16, 4864, "2 2 4"), (4656, 32, 432, "2 2 4"), (4400, 368, 592, "2 2 4"),
+              (1680, 128, 2336, "2 3 4"), (800, 80, 4992, "2 3 4"), (656, 96, 5648, "2 3 4"), (1072, 112, 3696, "2 3 4"), (2096, 464, 3888, "2 3 4")]
+
+
+@pytest.mark.parametrize("T,inp,out,tile", LINE_FORMS)
+@pytest.mark.parametrize("ahead", [(0, 0), (8, 56), (40, 16)])
+def test_linear_dense_and_row_pruned_by_whole_lines(et, T, inp, out, tile, ahead):
+    """Operands that begin `ahead` values off a line, between values that are no numbers: nothing ahead of a row or behind it reaches a
+    result.  Bound: half a unit of the binary16 place and the binary32 sums' own error (inp 2^-24 of the sum of magnitudes, below 1e-3 at 1040
+    inputs)."""
+    def between(v, by):
+        buf = np.full(by + v.size + 64, np.nan, np.float16)
+        buf[by:by + v.size] = v.ravel()
+        return up(et, buf)
+
+    W, b, x = Hn.randn((out, inp), 1, 0.02), Hn.randn((2 * out,), 2, 0.1), Hn.randn((T, inp), 3)
+    ids = np.sort(np.random.default_rng(4).permutation(2 * out)[:out]).astype(np.int32)
+    product = (Hn.f32(x).double() @ Hn.f32(W).double().T).numpy()
+    b64 = b.astype(np.float64)
+    d_x, d_W = between(x, ahead[0]), between(W, ahead[1])
+    x_at, w_at = d_x.offset(2 * ahead[0]), d_W.offset(2 * ahead[1])
+    d_b, d_ids = up(et, b), up(et, ids)
+    d_y = up(et, np.full((T, out), np.nan, np.float16))
+    et.linear_dense(w_at, d_b, x_at, d_y, T, inp, out, 0)
+    want = product + b64[:out]
+    assert (np.abs(d_y.numpy() - want) <= 2.0 ** -11 * np.abs(want) + 1e-3).all()
+    d_s = up(et, np.full((T, 2 * out), np.nan, np.float16))
+    et.check(et.lib().et_linear_rowpruned_f16(w_at, d_ids.ptr, out, d_b.ptr, x_at, d_s.ptr, T, inp, 2 * out, 0, None))
+    want = np.repeat(b64[None], T, 0)
+    want[:, ids] += product
+    assert (np.abs(d_s.numpy() - want) <= 2.0 ** -11 * np.abs(want) + 1e-3).all()
+
+
+@pytest.mark.parametrize("T,inp", [(64, 2048), (320, 2048), (384, 2064), (448, 2048), (512, 2064), (1088, 528), (1152, 512), (2240, 208)])
+def test_linear_dense_writes_every_tile_of_the_order(et, T, inp):
+    """Results of 1 to 15 tiles of 64 in width and heights of every remainder: the order that tiles are dealt in, blocks of 1 to 4 by 8, has
+    edges of every size.  Bound: half a unit of the binary16 place and the binary32 sums' own error (inp 2^-24 of the sum of magnitudes, below
+    1e-3 at 2064 inputs)."""
+    W, x = Hn.randn((960, inp), 1, 0.02), Hn.randn((T, inp), 3)
+    want = (Hn.f32(x).double() @ Hn.f32(W).double().T).numpy()
+    d_W, d_x = up(et, W), up(et, x)
+    for out in range(64, 961, 64):
+        d_y = up(et, np.full((T, out), np.nan, np.float16))
+        et.linear_dense(d_W, None, d_x, d_y, T, inp, out, 0)
+        assert (np.abs(d_y.numpy() - want[:, :out]) <= 2.0 ** -11 * np.abs(want[:, :out]) + 1e-3).all(), out
+
+
 def _random_dense_cases(n, seed):
     rng = np.random.default_rng(seed)
     cases = []

@@ -44,6 +44,12 @@ def test_the_dense_tests_run_every_tile(ask):
     assert ask([gemm(8176, 80, 8208)]) == ["tile 4 4 2 1"]
 
 
+def test_rows_off_a_line_run_what_they_claim(ask):
+    assert ask([f"lines {T} {out} {inp}" for T, inp, out, _ in linear.LINE_FORMS]) == [tile for *_, tile in linear.LINE_FORMS]
+    # two to a compute unit stay where K is short, and where no round is saved and the last is half empty
+    assert ask(["lines 5152 1312 496", "lines 1840 3424 912", "lines 1840 3424 1040", "lines 2208 1408 224"]) == ["2 2 2", "2 2 2", "2 2 4", "2 2 4"]
+
+
 def test_large_dense_problems_keep_tiles_of_256(ask):
     """Edges that are multiples of 64 but not of 256 leave the form of whole tiles as edges of 16 do."""
     large = [(16384, 8192, 8192), (16368, 8192, 8192), (16320, 8192, 8192), (16384, 8192, 8128), (16320, 256, 4096), (8128, 4096, 8256)]
