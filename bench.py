@@ -310,8 +310,10 @@ def time_token_local(et, layers, T, rounds_per_graph=6, replays=8):
     tiles = sum(len(w.col_idx) for l in layers for w in (l.qkv, l.o, l.l1, l.l2)) / n
     # Z and QKV' binary16, the residual stream binary32 in and out, tiles with their indices, biases and norms
     nbytes = 2.0 * T * H + 8.0 * T * H + 6.0 * T * H + 516.0 * tiles + 2.0 * (9 * H + FF)
-    name = "void et::encoder_layer_joined_kernel<3>(et::LayerArgs)" if joins.value else \
-        "void et::encoder_layer_kernel<1, 3, 1>(et::LayerArgs) + void et::encoder_layer_kernel<1, 3, 2>(et::LayerArgs)"
+    # as rocprofv3 prints them: names with binary16 pointers among their arguments stay mangled
+    args = "EEvPKDF16_PKvPKcPKiS2_iiijNS_9LayerArgsE"
+    name = "_ZN2et27encoder_layer_joined_kernelILi3E" + args if joins.value else \
+        f"_ZN2et20encoder_layer_kernelILi1ELi3ELi1E{args} + _ZN2et20encoder_layer_kernelILi1ELi3ELi2E{args}"
     what = f"output projection, LayerNorms, FFN + GELU and next QKV projection of a layer @80%, T={T}, " + \
         ("one launch" if joins.value else "two launches")
     return t.ms * 1e-3 / (rounds_per_graph * n * replays), name, what, 2.0 * 256 * tiles * T, nbytes
