@@ -243,8 +243,8 @@ static int launch_mha_nw(const MhaArgs &args, hipStream_t stream) {
     const unsigned per_head = a.nh > 1 && (unsigned long long)a.nbh * a.nh < 1ull << 32 ? (unsigned)(((1ull << 32) + a.nh - 1) / a.nh) : 0;
     const unsigned heads = a.nh < 1 << 24 && a.hd < 256 ? (unsigned)a.nh << 8 | (unsigned)a.hd : 0;
     const unsigned rows = (unsigned)rounds + a.ahead_blocks;
-    kernel<<<dim3(width, std::min(rows, 32768u), (rows + 32767) / 32768), 64 * NW, lds, stream>>>(a.K, a.V, a.Q, a.lens, a.ldk, a.ldv, a.S, a.nbh, heads, per_head, a);
-    return check_launch("mha_fused_kernel");
+    return launch_kernel("mha_fused_kernel", kernel, dim3(width, std::min(rows, 32768u), (rows + 32767) / 32768), 64 * NW, lds, stream, a.K, a.V, a.Q, a.lens, a.ldk, a.ldv, a.S,
+                         a.nbh, heads, per_head, a);
 }
 
 // ---- two groups of waves in turn ------------------------------------------------------------------------

@@ -1123,8 +1123,8 @@ static int launch_bsr_act(const BsrArgs &args, const BsrPlan &p, hipStream_t str
     const unsigned per_group = ngroups > 1 && (unsigned long long)per_xcd * kXcds * ngroups < 1ull << 32 ? (unsigned)(((1ull << 32) + ngroups - 1) / ngroups) : 0;
     BsrArgs a = args;
     a.rows_per_wg = p.rows_per_wg;
-    kernel<<<(unsigned)(per_xcd * kXcds), p.threads, p.lds, stream>>>(a.row_ptr, a.X, a.col_idx, a.tiles, a.T, a.in, a.out, a.rows_per_wg, ngroups, per_group, a);
-    return check_launch("bsr16_linear_kernel");
+    return launch_kernel("bsr16_linear_kernel", kernel, dim3((unsigned)(per_xcd * kXcds)), p.threads, p.lds, stream, a.row_ptr, a.X, a.col_idx, a.tiles, a.T, a.in, a.out,
+                         a.rows_per_wg, ngroups, per_group, a);
 }
 
 template <int MT, bool STAGE>
@@ -1215,9 +1215,8 @@ static int launch_bsr_halves(const BsrArgs &args, int rows_per_wg, hipStream_t s
     const int nbr = args.out / 16, ngroups = (nbr + rows_per_wg - 1) / rows_per_wg;
     const int strips = (args.T + 31) / 32;
     const unsigned rounds = (unsigned)((strips + kXcds - 1) / kXcds), gy = std::min(rounds, 32768u);
-    kernel<<<dim3((unsigned)(kXcds * ngroups), gy, (rounds + gy - 1) / gy), kHalfWaves * 64, lds, stream>>>(args.row_ptr, args.X, args.col_idx, args.tiles, args.bias, args.T,
-                                                                                                         args.in, args.out, rows_per_wg, args);
-    return check_launch("bsr16_linear_halves_kernel");
+    return launch_kernel("bsr16_linear_halves_kernel", kernel, dim3((unsigned)(kXcds * ngroups), gy, (rounds + gy - 1) / gy), kHalfWaves * 64, lds, stream, args.row_ptr, args.X,
+                         args.col_idx, args.tiles, args.bias, args.T, args.in, args.out, rows_per_wg, args);
 }
 
 // Block-rows of a workgroup of the halves form, 0 where another form is the faster one.  ntile: tiles of the weight, negative

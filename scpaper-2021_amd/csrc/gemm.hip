@@ -357,8 +357,7 @@ int launch_gemm(const GemmArgs &g, int batch, bool trans_b, hipStream_t stream) 
     if (gemm_skinny_applies(g, batch, trans_b)) {
         const dim3 grid((unsigned)(g.N / 16), (unsigned)(g.M / 16), (unsigned)batch);
         auto kernel = g.K <= 3 * 4 * 64 ? gemm_skinny_kernel<3> : gemm_skinny_kernel<6>;  // at most 3 pieces of 64 per wave, or more
-        kernel<<<grid, 256, 0, stream>>>(g.A, g.B, g.bias, g.K, g.lda, g.ldb, g);
-        return check_launch("gemm_skinny_kernel");
+        return launch_kernel("gemm_skinny_kernel", kernel, grid, 256, 0, stream, g.A, g.B, g.bias, g.K, g.lda, g.ldb, g);
     }
     if (gemm_dma_applies(g, batch, trans_b)) return launch_gemm_dma(g, batch, trans_b, stream);
     const long long tiles128 = (long long)((g.M + 127) / 128) * ((g.N + 127) / 128) * batch;
@@ -640,8 +639,7 @@ int et_gather_cols_f16(et_f16 *dst, const et_f16 *X, const int32_t *col_id, int 
         if (loads <= 1) kernel = gather_cols_staged_kernel<1>;
         else if (loads == 2) kernel = gather_cols_staged_kernel<2>;
         else if (loads == 3) kernel = gather_cols_staged_kernel<3>;
-        kernel<<<groups, 256, lds, as_stream(stream)>>>(H(dst), H(X), col_id, T, in, nnz_col, rows, lanes);
-        return check_launch("gather_cols_staged_kernel");
+        return launch_kernel("gather_cols_staged_kernel", kernel, dim3(groups), 256, lds, as_stream(stream), H(dst), H(X), col_id, T, in, nnz_col, rows, lanes);
     }
     gather_cols_kernel<<<(unsigned)blocks, 256, 0, as_stream(stream)>>>(H(dst), H(X), col_id, T, in, nnz_col);
     return check_launch("gather_cols_kernel");

@@ -641,8 +641,7 @@ static int launch_dma_variant(const GemmArgs &g, int batch, hipStream_t stream) 
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         raised = true;
     }
-    kernel<<<grid, 128 * NWN, lds, stream>>>(g.A, g.B, g.bias, g.M, g.N, g.K, g.lda, g.ldb, sbm, per_row, g);
-    return check_launch("gemm_f16_dma_kernel");
+    return launch_kernel("gemm_f16_dma_kernel", kernel, grid, 128 * NWN, lds, stream, g.A, g.B, g.bias, g.M, g.N, g.K, g.lda, g.ldb, sbm, per_row, g);
 }
 
 // rows that do not all begin on a 128-byte line

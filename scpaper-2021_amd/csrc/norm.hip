@@ -268,26 +268,21 @@ static int launch_layernorm(T *out, const T *src, const T *skip, const T *gamma,
                             int H, float eps, hipStream_t stream) {
     const int chunks = H / 4;
     const int nit = (chunks + kWave - 1) / kWave;
-    const dim3 grid((rows + kRowsPerBlock - 1) / kRowsPerBlock), block(kWave * kRowsPerBlock);
-#define ET_LN_CASE(N)                                                                   \
-    case N:                                                                             \
-        layernorm_rows_kernel<T, N, SKIP><<<grid, block, 0, stream>>>(out, src, skip, gamma, \
-                                                                   beta, rows, H, eps);  \
-        break;
+    const dim3 grid((rows + kRowsPerBlock - 1) / kRowsPerBlock);
+    auto kernel = layernorm_rows_kernel<T, 32, SKIP>;
     switch (nit) {
-        ET_LN_CASE(1) ET_LN_CASE(2) ET_LN_CASE(3) ET_LN_CASE(4)
-        ET_LN_CASE(5) ET_LN_CASE(6) ET_LN_CASE(7) ET_LN_CASE(8)
+        case 1: kernel = layernorm_rows_kernel<T, 1, SKIP>; break;
+        case 2: kernel = layernorm_rows_kernel<T, 2, SKIP>; break;
+        case 3: kernel = layernorm_rows_kernel<T, 3, SKIP>; break;
+        case 4: kernel = layernorm_rows_kernel<T, 4, SKIP>; break;
+        case 5: kernel = layernorm_rows_kernel<T, 5, SKIP>; break;
+        case 6: kernel = layernorm_rows_kernel<T, 6, SKIP>; break;
+        case 7: kernel = layernorm_rows_kernel<T, 7, SKIP>; break;
+        case 8: kernel = layernorm_rows_kernel<T, 8, SKIP>; break;
         default:
-            if (nit <= 16) {
-                layernorm_rows_kernel<T, 16, SKIP><<<grid, block, 0, stream>>>(out, src, skip, gamma,
-                                                                            beta, rows, H, eps);
-            } else {
-                layernorm_rows_kernel<T, 32, SKIP><<<grid, block, 0, stream>>>(out, src, skip, gamma,
-                                                                            beta, rows, H, eps);
-            }
+            if (nit <= 16) kernel = layernorm_rows_kernel<T, 16, SKIP>;
     }
-#undef ET_LN_CASE
-    return check_launch("layernorm_rows_kernel");
+    return launch_kernel("layernorm_rows_kernel", kernel, grid, kWave * kRowsPerBlock, 0, stream, out, src, skip, gamma, beta, rows, H, eps);
 }
 
 static int launch_skip_layernorm_mixed(float *out32, _Float16 *out16, const float *src, const float *skip,
