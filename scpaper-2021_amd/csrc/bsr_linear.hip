@@ -121,9 +121,9 @@ __host__ __device__ __forceinline__ int half_tiles(int in) { return (in / 16 + 1
 // ACT is a template parameter: the epilogue carries no run-time branch and each
 // fused activation is a separately named kernel in a profile.
 template <int MT, bool STAGE, int ACT, int LN = 0, int FX = 0>
-__global__ __launch_bounds__(((MT == 1 && (FX & kFxRes32) && !(FX & kFxRes16)) || (FX & (kFxNorm32 | kFxWide))) ? 768 : 512) void bsr16_linear_kernel(const int32_t *row_ptr, const _Float16 *X, const int32_t *col_idx, const _Float16 *tiles, int T, int in, int out,
-                                                                                                                                                      int rows_per_wg, int ngroups, unsigned per_group,
-                                                                                                                                                      const BsrArgs rest) {
+__global__ __launch_bounds__(((MT == 1 && (FX & kFxRes32) && !(FX & kFxRes16)) || (FX & (kFxNorm32 | kFxWide))) ? 768 : 512)
+    void bsr16_linear_kernel(const int32_t *row_ptr, const _Float16 *X, const int32_t *col_idx, const _Float16 *tiles, int T, int in, int out, int rows_per_wg, int ngroups,
+                             unsigned per_group, const BsrArgs rest) {
     BsrArgs a = rest;  // (those in front are preloaded into scalar registers)
     a.row_ptr = row_ptr, a.X = X, a.col_idx = col_idx, a.tiles = tiles, a.T = T, a.in = in, a.out = out, a.rows_per_wg = rows_per_wg;
     static_assert(!LN || STAGE, "the fused LayerNorm prologue writes the strip to LDS");
