@@ -578,7 +578,9 @@ int et_fill_rows_bias_f16(et_f16 *C, const et_f16 *bias, int rows, int cols,
  *   P = softmax(scale * Q_h K_h^T + mask),  Z_h = P V_h
  * mask: optional additive [S x S] binary16 matrix shared by all sequences and
  * heads (-inf removes a key).  lens: optional int32[B]; keys >= lens[b] of
- * sequence b get probability exactly 0 (right padding).  Scores, softmax and
+ * sequence b get probability exactly 0 (right padding); their rows of K and V
+ * must hold finite values up to the next multiple of 128 keys (0 times a NaN is
+ * a NaN), what lies behind is not looked at.  Scores, softmax and
  * both contractions are fp32-accumulated.  S % 16 == 0; hd a multiple of 8, at
  * most 256 (the reference's kernels ask for multiples of 16,
  * Fused_attention/test/testfused.cu:22, while its example model has 800 / 4 =

@@ -80,3 +80,33 @@ def test_against_binary64(et, B, S, nh, hd, causal, lens, form, pad):
         want = torch.matmul(torch.softmax(s, -1).nan_to_num(0.0), x[2]).transpose(0, 1).reshape(S, H).numpy()
         assert np.abs(got[b * S:(b + 1) * S, :H] - want).max() <= 1.1e-2
         assert np.linalg.norm(got[b * S:(b + 1) * S, :H] - want) <= 5e-4 * np.linalg.norm(want)
+
+
+# sequences, keys, heads, head size, causal, the form; the first column of a block of 64 keys, and the second, are where a length ends
+PADDED = [(64, 128, 12, 64, True, T41), (20, 176, 12, 64, False, T81), (1, 528, 12, 64, False, T42), (2, 784, 16, 64, False, T82), (3, 528, 12, 64, True, T44),
+          (20, 512, 12, 32, True, T41), (8, 272, 10, 80, True, T41), (4, 528, 8, 128, False, T41), (8, 784, 4, 224, False, T41)]
+
+
+def test_the_padded_shapes_run_what_they_claim(ask):
+    assert ask([s[:5] for s in PADDED]) == [s[5] for s in PADDED]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,S,nh,hd,causal,form", PADDED)
+@pytest.mark.parametrize("length", [1, 32, 65, 96])
+def test_rows_past_a_length_need_hold_no_numbers(et, B, S, nh, hd, causal, form, length):
+    """Rows of K and V from the next multiple of 32 past a sequence's length on are no numbers, and no result depends on them.  Bound as above."""
+    H, T = nh * hd, B * S
+    qkv = Hn.randn((T, 3 * H), 7).reshape(B, S, 3, H)
+    qkv[:, (length + 31) // 32 * 32:, 1:] = np.nan
+    d, d_l, d_z = Hn.up(et, qkv), Hn.up(et, np.full(B, length, np.int32)), Hn.up(et, np.full((T, H), 7.0, np.float16))
+    et.mha_fused(d.ptr, d.offset(2 * H), d.offset(4 * H), 3 * H, 3 * H, 3 * H, d_z.ptr, H, None, d_l.ptr, B, S, nh, hd, hd ** -0.5, et.MHA_CAUSAL if causal else 0, None)
+    got = d_z.numpy().reshape(B, S, H)
+    for b in sorted({0, B - 1}):
+        x = torch.from_numpy(qkv[b].astype(np.float64)).view(S, 3, nh, hd).permute(1, 2, 0, 3).contiguous()
+        s = torch.matmul(x[0], x[1][:, :length].transpose(1, 2).contiguous()) * hd ** -0.5
+        if causal:
+            s.masked_fill_(torch.ones(S, length, dtype=torch.bool).triu(1), -np.inf)
+        want = torch.matmul(torch.softmax(s, -1), x[2][:, :length]).transpose(0, 1).reshape(S, H).numpy()
+        assert np.abs(got[b] - want).max() <= 1.1e-2
+        assert np.linalg.norm(got[b] - want) <= 5e-4 * np.linalg.norm(want)
