@@ -127,9 +127,11 @@ constexpr MhaTilesCost kMhaTiles64[] = {{{4, 1, 2}, 108, 88, 54, 221}, {{8, 1, 2
 constexpr MhaTilesCost kMhaTiles96[] = {{{4, 1, 2}, 0, 124, 76, 377}, {{8, 1, 2}, 0, 147, 156, 376}, {{4, 2, 2}, 48, 155, 134, 362}, {{8, 2, 2}, 0, 154, 160, 547}};
 constexpr MhaTilesCost kMhaTiles128[] = {{{4, 1, 2}, 19, 145, 97, 364}, {{8, 1, 2}, 0, 173, 200, 364}, {{4, 2, 2}, 21, 165, 151, 422}, {{4, 4, 1}, 96, 0, 118, 341}};
 // 129 to 224 columns, where the forms above (64 queries a workgroup, blocks of 64 keys) stay ahead for some: 4 heads of 200, 12 x 48
-// keys 6.3 and 6.7 us
+// keys 6.3 and 6.7 us.  (Eight waves of a tile each: problems without a mask show what a block costs a full unit alone; the chain is that of the longest causal
+// strip, 4 heads of 200, 2048 keys 94.8 us, the forms above 89.3, two waves a tile, which are chosen, 68; over 540 causal problems of 80 to 4096 keys the choice is
+// 2.7 % behind the best form in the mean, 0.94 of the time of the chain of 112 that fits the others, and slower than that for none.)
 constexpr MhaTilesCost kMhaTiles224[] = {{{0, 1, 2}, 0, 274, 182, 330}, {{4, 1, 1}, 0, 158, 109, 393}, {{4, 2, 1}, 0, 201, 190, 500},
-                                         {{4, 1, 2}, 0, 250, 279, 412}, {{8, 1, 2}, 0, 112, 354, 359}};
+                                         {{4, 1, 2}, 0, 250, 279, 412}, {{8, 1, 2}, 0, 240, 354, 359}};
 
 template <int N> inline MhaTiles mha_tiles_least(const MhaTilesCost (&costs)[N], int S, int nbh, bool causal) {
     long long best = -1;
@@ -158,6 +160,9 @@ template <int N> inline MhaTiles mha_tiles_least(const MhaTilesCost (&costs)[N],
 inline MhaTiles mha_tiles(int HD, int S, int nbh, bool causal) {
     if (HD <= 128 && S <= 384 && (long long)nbh * ((S + 31) / 32) <= 400) return {};
     if (HD <= 128 && S <= 64) return {4, 1, 2};
+    // (65 to 96 causal keys, wide heads, few of them, us, the forms above and tiles: 1 x 4 heads of 200, 80 keys 7.3 and 7.8, 8 x 6 of 136 7.4 and 8.1, 24 x 5 of 160 8.4
+    // and 8.7, 96 keys, 8 x 6 7.7 and 8.1; more, 80 keys, 16 x 8 of 224 9.4 and 9.3, 24 x 6 10.1 and 8.9, 96 keys, 16 x 4 8.7 and 8.6)
+    if (HD == 224 && causal && S > 64 && S <= 96 && nbh <= (S <= 80 ? 120 : 48)) return {};
     switch (HD) {
         case 32: return mha_tiles_least(kMhaTiles32, S, nbh, causal);
         case 64: return mha_tiles_least(kMhaTiles64, S, nbh, causal);

@@ -25,7 +25,7 @@ SHAPES = [
     (8, 272, 10, 80, False, [272, 75, 0], T41), (8, 400, 10, 96, True, None, T81), (1, 400, 10, 80, False, None, T42), (3, 784, 10, 88, False, None, T82),
     (4, 528, 8, 128, False, [528, 513, 7], T41), (12, 272, 8, 120, True, None, T81), (1, 400, 8, 128, False, [399], T44), (2, 1040, 8, 128, True, None, T42),
     (3, 16, 4, 200, True, [16, 1, 0], (4, 1, 1)), (2, 272, 4, 200, False, [272, 65], (4, 2, 1)), (8, 784, 4, 224, False, None, T41),
-    (8, 784, 4, 136, True, None, T81),
+    (8, 784, 4, 136, True, None, T81), (2, 1552, 4, 136, True, None, (4, 2, 1)),
 ]
 
 
@@ -51,6 +51,15 @@ def test_the_shapes_run_what_they_claim(ask):
 def test_what_the_one_launch_with_projection_takes_keeps_its_bits(ask):
     """Few short sequences run the kernel that the launch joined with the projection is made of; heads beyond 224 too."""
     assert ask([(1, 128, 12, 64, False), (8, 128, 12, 64, True), (1, 384, 12, 64, False), (5, 256, 8, 128, False), (12, 96, 4, 256, False)]) == [(0, 0, 0)] * 5
+
+
+def test_wide_causal_heads_take_the_form_measured_fastest(ask):
+    """One strip of eight waves is as long as its longest wave: two waves a tile where the chip is not full, and the other kernel for 65 to 96 keys."""
+    T421 = (4, 2, 1)
+    assert ask([(1, 1536, 4, 200, True), (2, 2048, 4, 200, True), (1, 2048, 6, 136, True)]) == [T421] * 3
+    assert ask([(8, 2048, 4, 200, True), (4, 3072, 4, 200, True)]) == [T81] * 2
+    assert ask([(1, 80, 4, 200, True), (24, 80, 5, 160, True), (8, 96, 6, 136, True)]) == [(0, 0, 0)] * 3
+    assert ask([(24, 80, 6, 136, True), (16, 96, 4, 200, True), (1, 80, 4, 200, False)]) == [(4, 1, 1)] * 3
 
 
 @pytest.mark.gpu
