@@ -128,7 +128,7 @@ constexpr MhaTilesCost kMhaTiles96[] = {{{4, 1, 2}, 0, 124, 76, 377}, {{8, 1, 2}
 constexpr MhaTilesCost kMhaTiles128[] = {{{4, 1, 2}, 19, 145, 97, 364}, {{8, 1, 2}, 0, 173, 200, 364}, {{4, 2, 2}, 21, 165, 151, 422}, {{4, 4, 1}, 96, 0, 118, 341}};
 // 129 to 224 columns, where the forms above (64 queries a workgroup, blocks of 64 keys) stay ahead for some: 4 heads of 200, 12 x 48
 // keys 6.3 and 6.7 us.  (Eight waves of a tile each: problems without a mask show what a block costs a full unit alone; the chain is that of the longest causal
-// strip, 4 heads of 200, 2048 keys 94.8 us, the forms above 89.3, two waves a tile, which are chosen, 68; over 540 causal problems of 80 to 4096 keys the choice is
+// strip, 4 heads of 200, 2048 keys 94.8 us, the forms above 89.3, two waves a tile, which are chosen, 58; over 540 causal problems of 80 to 4096 keys the choice is
 // 2.7 % behind the best form in the mean, 0.94 of the time of the chain of 112 that fits the others, and slower than that for none.)
 constexpr MhaTilesCost kMhaTiles224[] = {{{0, 1, 2}, 0, 274, 182, 330}, {{4, 1, 1}, 0, 158, 109, 393}, {{4, 2, 1}, 0, 201, 190, 500},
                                          {{4, 1, 2}, 0, 250, 279, 412}, {{8, 1, 2}, 0, 240, 354, 359}};
@@ -157,7 +157,17 @@ template <int N> inline MhaTiles mha_tiles_least(const MhaTilesCost (&costs)[N],
 // Few short sequences keep the forms above: the one launch of attention and output projection (mha_fuseo_kernel) is made of those, and where it
 // is used the two launches it replaces give the same bits.  (us, the forms above and this kernel: 12 heads of 64, 1 x 128 keys 4.5 and 4.2, 8 x 128 4.7
 // and 4.5, 3 x 176 6.2 and 5.1.)  Otherwise up to 64 keys, one block of them, there is nothing to share (1.0 to 1.3 of the time).
-inline MhaTiles mha_tiles(int HD, int S, int nbh, bool causal) {
+// Sequences of their own lengths (padded): the costs know none, and one long sequence among short ones keeps a unit's only workgroup of eight waves
+// to its end.  Heads of 33 to 96 take four there (tiles of 65 to 96 columns that waves share gain nothing, nor do sequences of one strip): us, the 16 x 16 kernel, eight and four, lengths of a quarter
+// to the whole, 16 heads of 64, 4 x 640 keys 14.3, 16.0 and 14.1, 4 x 512 12.6, 9.1 and 8.4, 12 heads, 3 x 784 17.4, 19.3 and 15.5, 10 of 80, 4 x 1024 27.4, 29.7 and 25.4.
+// Where all are nearly whole it costs 5 to 8 % (4 x 12, 448 keys 9.0 and 9.7); two a unit gain as often as they lose (8 x 16, 1024 keys 40.8 and 35.4 or 32.1 and 35.1 by
+// the lengths, 16 x 16, 512 keys 23.7 and 25.3), and so do heads of 128 alone on theirs (3 x 1536 keys 37.7 and 31.0, 12 x 512 20.9 and 22.4).
+inline MhaTiles mha_tiles(int HD, int S, int nbh, bool causal, bool padded) {
+    const auto evened = [&](MhaTiles f) {
+        const int units = ((nbh + 7) / 8 * ((S + f.queries() - 1) / f.queries()) + 31) / 32;  // workgroups of the fullest of a die's 32
+        if (padded && f.waves == 8 && (HD == 64 || f.split == 1) && units == 1 && S > f.queries()) f.waves = 4;
+        return f;
+    };
     if (HD <= 128 && S <= 384 && (long long)nbh * ((S + 31) / 32) <= 400) return {};
     if (HD <= 128 && S <= 64) return {4, 1, 2};
     // (65 to 96 causal keys, wide heads, few of them, us, the forms above and tiles: 1 x 4 heads of 200, 80 keys 7.3 and 7.8, 8 x 6 of 136 7.4 and 8.1, 24 x 5 of 160 8.4
@@ -165,8 +175,8 @@ inline MhaTiles mha_tiles(int HD, int S, int nbh, bool causal) {
     if (HD == 224 && causal && S > 64 && S <= 96 && nbh <= (S <= 80 ? 120 : 48)) return {};
     switch (HD) {
         case 32: return mha_tiles_least(kMhaTiles32, S, nbh, causal);
-        case 64: return mha_tiles_least(kMhaTiles64, S, nbh, causal);
-        case 96: return mha_tiles_least(kMhaTiles96, S, nbh, causal);
+        case 64: return evened(mha_tiles_least(kMhaTiles64, S, nbh, causal));
+        case 96: return evened(mha_tiles_least(kMhaTiles96, S, nbh, causal));
         case 128: return mha_tiles_least(kMhaTiles128, S, nbh, causal);
         case 224: return mha_tiles_least(kMhaTiles224, S, nbh, causal);
         default: return {};

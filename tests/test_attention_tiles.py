@@ -16,10 +16,11 @@ T41, T81, T42, T82, T44 = (4, 1, 2), (8, 1, 2), (4, 2, 2), (8, 2, 2), (4, 4, 1)
 SHAPES = [
     (70, 16, 12, 64, False, None, T41), (40, 48, 12, 40, True, None, T41), (64, 128, 12, 64, False, [0, 1, 63, 64, 65, 127], T41),
     (8, 784, 12, 64, True, [784, 3, 33, 783], T41), (16, 400, 16, 64, True, None, T81), (20, 176, 12, 64, False, [176, 129, 128, 31], T81),
+    (32, 272, 12, 64, False, [272, 129, 128, 31], T81),
     (1, 400, 12, 56, False, None, T44), (3, 528, 12, 64, True, [390, 5], T44), (1, 528, 12, 64, False, [515], T42), (2, 1040, 12, 64, True, None, T42),
-    (2, 784, 16, 64, False, [784, 130], T82),
+    (2, 784, 16, 64, False, [784, 130], T42), (2, 784, 16, 64, False, None, T82),
     # sequences of no keys whose tiles are shared
-    (3, 400, 16, 64, False, [400, 77, 0], T82), (3, 528, 12, 64, True, [528, 77, 0], T44), (3, 528, 12, 24, False, [528, 77, 0], T42),
+    (3, 400, 16, 64, False, [400, 77, 0], T42), (3, 784, 10, 88, False, [784, 77, 0], T82), (3, 528, 12, 64, True, [528, 77, 0], T44), (3, 528, 12, 24, False, [528, 77, 0], T42),
     (3, 400, 8, 128, False, [400, 77, 0], T42), (3, 272, 4, 200, False, [272, 77, 0], (4, 2, 1)),
     (20, 512, 12, 32, False, [512, 100, 0], T41), (3, 400, 12, 24, True, None, T44), (4, 272, 12, 32, False, None, T42),
     (8, 272, 10, 80, False, [272, 75, 0], T41), (8, 400, 10, 96, True, None, T81), (1, 400, 10, 80, False, None, T42), (3, 784, 10, 88, False, None, T82),
@@ -35,8 +36,9 @@ def ask(tmp_path_factory):
     subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-I", str(ROOT / "scpaper-2021_amd" / "csrc"), str(ROOT / "tests" / "cpp" / "attention_tiles.cpp"),
                     "-o", str(exe)], check=True)
 
-    def answers(shapes):  # (sequences, keys, heads, head size, causal)
-        text = "\n".join(f"{next(t for t in (32, 64, 96, 128, 224, 256) if hd <= t)} {S} {B * nh} {int(c)}" for B, S, nh, hd, c in shapes)
+    def answers(shapes):  # (sequences, keys, heads, head size, causal, lengths)
+        text = "\n".join(f"{next(t for t in (32, 64, 96, 128, 224, 256) if hd <= t)} {S} {B * nh} {int(c)} {int(any(lens or ()))}"
+                         for B, S, nh, hd, c, *lens in shapes)
         out = subprocess.run([str(exe)], input=text, capture_output=True, text=True, check=True).stdout.splitlines()
         return [tuple(map(int, line.split())) for line in out]
 
@@ -44,7 +46,7 @@ def ask(tmp_path_factory):
 
 
 def test_the_shapes_run_what_they_claim(ask):
-    assert ask([s[:5] for s in SHAPES]) == [s[6] for s in SHAPES]
+    assert ask([s[:6] for s in SHAPES]) == [s[6] for s in SHAPES]
     assert {(64, f) for f in (T41, T81, T42, T82, T44)} <= {(s[3], s[6]) for s in SHAPES}
 
 
@@ -60,6 +62,14 @@ def test_wide_causal_heads_take_the_form_measured_fastest(ask):
     assert ask([(8, 2048, 4, 200, True), (4, 3072, 4, 200, True)]) == [T81] * 2
     assert ask([(1, 80, 4, 200, True), (24, 80, 5, 160, True), (8, 96, 6, 136, True)]) == [(0, 0, 0)] * 3
     assert ask([(24, 80, 6, 136, True), (16, 96, 4, 200, True), (1, 80, 4, 200, False)]) == [(4, 1, 1)] * 3
+
+
+def test_sequences_of_their_own_lengths_keep_four_waves_where_eight_are_few(ask):
+    few = [(4, 640, 16, 64, False), (3, 784, 12, 64, False), (4, 512, 16, 64, False), (8, 400, 12, 64, False), (4, 1024, 10, 80, False), (8, 512, 10, 80, False)]
+    assert [w for w, *_ in ask(few)] == [8] * 6
+    assert [w for w, *_ in ask([(*s, [1]) for s in few])] == [4] * 6
+    many = [(16, 2048, 12, 64, False, [1]), (8, 1024, 16, 64, False, [1]), (3, 1536, 8, 128, False, [1]), (3, 784, 10, 88, False, [1])]
+    assert [w for w, *_ in ask(many)] == [8] * 4
 
 
 @pytest.mark.gpu
@@ -92,12 +102,12 @@ def test_against_binary64(et, B, S, nh, hd, causal, lens, form, pad):
 
 
 # sequences, keys, heads, head size, causal, the form; the first column of a block of 64 keys, and the second, are where a length ends
-PADDED = [(64, 128, 12, 64, True, T41), (20, 176, 12, 64, False, T81), (1, 528, 12, 64, False, T42), (2, 784, 16, 64, False, T82), (3, 528, 12, 64, True, T44),
+PADDED = [(64, 128, 12, 64, True, T41), (30, 272, 12, 64, False, T81), (1, 528, 12, 64, False, T42), (3, 784, 10, 88, False, T82), (3, 528, 12, 64, True, T44),
           (20, 512, 12, 32, True, T41), (8, 272, 10, 80, True, T41), (4, 528, 8, 128, False, T41), (8, 784, 4, 224, False, T41)]
 
 
 def test_the_padded_shapes_run_what_they_claim(ask):
-    assert ask([s[:5] for s in PADDED]) == [s[5] for s in PADDED]
+    assert ask([(*s[:5], [1]) for s in PADDED]) == [s[5] for s in PADDED]
 
 
 @pytest.mark.gpu
