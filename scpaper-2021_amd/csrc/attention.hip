@@ -189,7 +189,7 @@ __global__ __launch_bounds__(64 * NW)
     __attribute__((amdgpu_waves_per_eu(HD > 128 ? 2 : mha_three_waves<HD, NW, COMPACT, QT>() ? 3 : 1, HD > 128 ? 2 : mha_three_waves<HD, NW, COMPACT, QT>() ? 3 : 8))) void
     mha_fused_kernel(ET_MHA_FIRST, const MhaArgs rest) {
     ET_MHA_TAKE;
-    constexpr bool kCoherentZ = false;
+    constexpr bool kCoherentZ = false, kQueriesFirst = false;
     constexpr int KB = mha_key_block<HD>();
     const int bh = blockIdx.x % kXcds + kXcds * mha_row(), qstrip = blockIdx.x / kXcds;
 #include "attention_body.inc"
@@ -199,20 +199,22 @@ __global__ __launch_bounds__(64 * NW)
 __global__ __launch_bounds__(256) void mha_wide_kernel(ET_MHA_FIRST, const MhaArgs rest) {
     ET_MHA_TAKE;
     constexpr int HD = 256, NW = 4, QT = 1, KB = kKeyBlock;
-    constexpr bool COMPACT = false, kCoherentZ = false;
+    constexpr bool COMPACT = false, kCoherentZ = false, kQueriesFirst = false;
     const int bh = blockIdx.x % kXcds + kXcds * mha_row(), qstrip = blockIdx.x / kXcds;
 #include "attention_body.inc"
 }
 
 // the same behind workgroups that ask for later launches' weights (heads up to 64, four or eight waves; a kernel of its own,
-// since the argument to tell them apart by is a wait of its own at the start: 12 layers of one sequence 335 -> 342 us)
+// since the argument to tell them apart by is a wait of its own at the start: 12 layers of one sequence 335 -> 342 us).  Heads of 64 in four waves ask for the
+// queries first: the other way round the compiler keeps four registers too many for three waves a SIMD.  (With two: 32 x 12 heads of 64, 128 keys and a mask
+// 14.1 us and 11.0, 24 x 12 of 32, 512 keys 82.7 and 60.5, results off 16 bytes 35.5 and 29.1; one round of them, 1 x 128 keys, 4.2 either way.)
 template <int HD, int NW, int QT>
 __global__ __launch_bounds__(64 * NW)
-    __attribute__((amdgpu_waves_per_eu(1, 8))) void
+    __attribute__((amdgpu_waves_per_eu(mha_three_waves<HD, NW, false, QT>() ? 3 : 1, mha_three_waves<HD, NW, false, QT>() ? 3 : 8))) void
     mha_fused_ahead_kernel(ET_MHA_FIRST, const MhaArgs rest) {
     if (mha_row() < rest.ahead_blocks) return ahead_of(rest, mha_row() * gridDim.x + blockIdx.x);
     ET_MHA_TAKE;
-    constexpr bool kCoherentZ = false, COMPACT = false;
+    constexpr bool kCoherentZ = false, COMPACT = false, kQueriesFirst = HD == 64 && NW == 4;
     constexpr int KB = mha_key_block<HD>();
     const int bh = blockIdx.x % kXcds + kXcds * (mha_row() - a.ahead_blocks), qstrip = blockIdx.x / kXcds;
 #include "attention_body.inc"
@@ -586,7 +588,7 @@ static __device__ __align__(256) unsigned fuseo_arrived[kFuseOCounters];
 template <int HD, int NW, int QT>
 __global__ __launch_bounds__(64 * NW) void mha_fuseo_kernel(const MhaArgs a, const FuseOArgs f) {
     constexpr bool COMPACT = false;
-    constexpr bool kCoherentZ = true;
+    constexpr bool kCoherentZ = true, kQueriesFirst = false;
     constexpr int KB = mha_key_block<HD>();
     constexpr unsigned per_head = 0;
     const int qstrips = (a.S + 16 * NW * QT - 1) / (16 * NW * QT), k_in_xcd = blockIdx.x / kXcds;

@@ -95,3 +95,19 @@ def test_hot_path_kernels_keep_their_registers():
                 "mha_fused_kernelILi64ELb0ELi4ELi1E" in name:
             assert vspill == 0 and scratch == 0, line
     assert seen > 100
+
+
+def test_four_wave_attention_holds_three_waves_a_simd():
+    """The four-wave forms that fetch a block ahead are made for three workgroups a compute unit, also where some of their workgroups ask
+    for later launches' weights."""
+    import re
+    from pathlib import Path
+    rec = Path(__file__).resolve().parents[1] / "scpaper-2021_amd" / "lib" / "kernel_resources.txt"
+    if not rec.exists():
+        pytest.skip("no resource record: the library was built by an older build script")
+    held = {}
+    for line in rec.read_text().splitlines():
+        m = re.search(r"mha_fused_(kernelILi(?:32|64)ELb0ELi4ELi1|ahead_kernelILi(?:32|64)ELi4ELi1)E.*Occupancy \[waves/SIMD\]: (\d+)", line)
+        if m:
+            held[m.group(1)] = int(m.group(2))
+    assert len(held) == 4 and min(held.values()) >= 3, held
