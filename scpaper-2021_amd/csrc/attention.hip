@@ -588,7 +588,7 @@ static __device__ __align__(256) unsigned fuseo_arrived[kFuseOCounters];
 template <int HD, int NW, int QT>
 __global__ __launch_bounds__(64 * NW) void mha_fuseo_kernel(const MhaArgs a, const FuseOArgs f) {
     constexpr bool COMPACT = false;
-    constexpr bool kCoherentZ = true, kQueriesFirst = false;
+    constexpr bool kCoherentZ = true, kQueriesFirst = true;  // (the first block first: 64 x 128 keys 127.9 -> 134.9 us)
     constexpr int KB = mha_key_block<HD>();
     constexpr unsigned per_head = 0;
     const int qstrips = (a.S + 16 * NW * QT - 1) / (16 * NW * QT), k_in_xcd = blockIdx.x / kXcds;
