@@ -47,9 +47,8 @@ template <> struct Chunk4<float> { using raw = float4; };
 
 // NIT = number of 4-element chunks each lane owns: chunk c = lane + 64*i.
 template <typename T, int NIT, bool SKIP>
-__global__ __launch_bounds__(kWave *kRowsPerBlock) void layernorm_rows_kernel(
-    T *__restrict__ out, const T *__restrict__ src, const T *__restrict__ skip,
-    const T *__restrict__ gamma, const T *__restrict__ beta, int rows, int H, float eps) {
+__device__ __forceinline__ void layernorm_rows(T *__restrict__ out, const T *__restrict__ src, const T *__restrict__ skip,
+                                               const T *__restrict__ gamma, const T *__restrict__ beta, int rows, int H, float eps) {
     using raw_t = typename Chunk4<T>::raw;
     const int lane = threadIdx.x & (kWave - 1);
     const int row = blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
@@ -128,6 +127,22 @@ __global__ __launch_bounds__(kWave *kRowsPerBlock) void layernorm_rows_kernel(
             o[c] = pack4_as<raw_t>(y);
         }
     }
+}
+// Arguments preloaded into scalar registers from 513 columns on, read from memory below: a launch that preloads them begins 0.1 us later, which rows this
+// short do not win back (us, from memory and preloaded: 54 x 80 2.02 and 2.15, 2 x 360 1.88 and 1.98, 654 x 668 2.48 and 2.48, 190 x 1284 2.99 and 2.92).
+template <typename T, int NIT, bool SKIP>
+__global__ __launch_bounds__(kWave *kRowsPerBlock) void layernorm_rows_kernel(T *out, const T *src, const T *skip, const T *gamma, const T *beta, int rows, int H,
+                                                                              float eps) {
+    layernorm_rows<T, NIT, SKIP>(out, src, skip, gamma, beta, rows, H, eps);
+}
+template <typename T> struct LayerNormRows {
+    T *out;
+    const T *src, *skip, *gamma, *beta;
+    int rows, H;
+    float eps;
+};
+template <typename T, int NIT, bool SKIP> __global__ __launch_bounds__(kWave *kRowsPerBlock) void layernorm_narrow_rows_kernel(const LayerNormRows<T> a) {
+    layernorm_rows<T, NIT, SKIP>(a.out, a.src, a.skip, a.gamma, a.beta, a.rows, a.H, a.eps);
 }
 
 // Mixed-precision SkipLayerNorm: the residual stream (src = a projection's fp32 output, skip = the
@@ -269,10 +284,11 @@ static int launch_layernorm(T *out, const T *src, const T *skip, const T *gamma,
     const int chunks = H / 4;
     const int nit = (chunks + kWave - 1) / kWave;
     const dim3 grid((rows + kRowsPerBlock - 1) / kRowsPerBlock);
+    if (nit <= 2)
+        return launch_kernel("layernorm_narrow_rows_kernel", nit == 1 ? layernorm_narrow_rows_kernel<T, 1, SKIP> : layernorm_narrow_rows_kernel<T, 2, SKIP>, grid,
+                             kWave * kRowsPerBlock, 0, stream, LayerNormRows<T>{out, src, skip, gamma, beta, rows, H, eps});
     auto kernel = layernorm_rows_kernel<T, 32, SKIP>;
     switch (nit) {
-        case 1: kernel = layernorm_rows_kernel<T, 1, SKIP>; break;
-        case 2: kernel = layernorm_rows_kernel<T, 2, SKIP>; break;
         case 3: kernel = layernorm_rows_kernel<T, 3, SKIP>; break;
         case 4: kernel = layernorm_rows_kernel<T, 4, SKIP>; break;
         case 5: kernel = layernorm_rows_kernel<T, 5, SKIP>; break;
