@@ -539,7 +539,6 @@ static int launch_mha(const MhaArgs &args, hipStream_t stream) {
         if (f.in_turn) return f.ragged ? launch_mha_pingpong<true>(args, stream) : launch_mha_pingpong<false>(args, stream);
     }
     if constexpr (HD >= 64 && !COMPACT) {
-        // (128-wide heads with two tiles took all registers and spilled 49: level with one tile at 2048 keys, 2 to 25 % behind it below)
         if constexpr (HD != 128) {
             if (f.tiles == 2) return launch_mha_nw<HD, COMPACT, 8, 2>(args, stream);
         }

@@ -44,9 +44,9 @@ struct MhaForm {
 // MFMAs) from 512 on (2048 keys, 16 x 16 heads 516 -> 464 us; 214 registers, two waves per SIMD), unless a causal sequence is one such strip:
 // both of its blocks are multiplied for all of its queries (256 causal keys, heads of 64: 24 to 512 heads 1.26 to 1.9 of the time in smaller strips).
 // Heads of 65 to 96 gain from it throughout (80 x 10: 1792 keys 0.77 of the time of the better of 4 and 8, 256 keys 0.90; causal 0.9 to 1.0, one and
-// two strips a sequence 1.05 to 1.15).  128-wide heads: the 8-wave
-// form prefetches the next block through registers (565 -> 532 us at 2048 keys, 16 x 8 heads); the two-tile form takes all
-// 256 registers and spills 49, level with it at 2048 keys, 2 to 25 % behind it below (not changed here: causal 20 to 60 %).
+// two strips a sequence 1.05 to 1.15).  128-wide heads never: the 8-wave
+// form prefetches the next block through registers (565 -> 532 us at 2048 keys, 16 x 8 heads), and with two tiles it took all
+// 256 registers and spilled 49 (two and one, additive mask: 32 x 8 heads, 1024 keys 526 and 428, causal 517 and 337, 16 x 8, 2048 keys 1003 and 829).
 // Two tiles on 4 waves lose more to the missing third wave than they save (735 us).
 // HD: head size of the template; nbh: sequences times heads; plain: no additive mask and a positive scale; padded: sequences of their own lengths.
 inline MhaForm mha_form(int HD, bool compact, int S, int nbh, bool causal, bool plain, bool padded) {
@@ -69,7 +69,7 @@ inline MhaForm mha_form(int HD, bool compact, int S, int nbh, bool causal, bool 
             100 * u16 >= 85 * 32 * ((u16 + 31) / 32))
             return {8, 2, true, true};
         const bool one_causal_strip = HD == 64 && causal && qblocks == 16;
-        if (HD >= 64 && qblocks % 16 == 0 && (long)nbh * (qblocks / 16) >= 512 && !one_causal_strip) return {8, 2, false, false};
+        if (HD >= 64 && HD != 128 && qblocks % 16 == 0 && (long)nbh * (qblocks / 16) >= 512 && !one_causal_strip) return {8, 2, false, false};
         const long u8 = (long)units * strips8, u4 = (long)units * strips4;  // workgroups of a die
         bool takes8;
         if (causal) {

@@ -103,6 +103,12 @@ def test_attention_takes_eight_waves_where_they_save_a_unit_time(ask):
     assert ask([mha(48, 256, 12, 64, True), mha(48, 512, 12, 64, True, plain=False), mha(48, 256, 12, 64)]) == ["waves 8 1", "waves 8 2", "waves 8 2"]
 
 
+def test_heads_of_128_take_one_tile_a_wave(ask):
+    shapes = [(B, S, nh, 128, causal) for B in (1, 16, 32, 47) for nh in (8, 16) for S in range(256, 2049, 256) for causal in (False, True) if B * nh * (S // 256) >= 512]
+    for lens in (None, [1]):
+        assert set(ask([mha(*s, lens=lens) for s in shapes])) == {"waves 8 1"}
+
+
 def test_many_short_sequences_take_the_fewest_rounds(ask):
     compact = ask([mha(*s[:4], compact=True) for s in attention.COMPACT_SHAPES])
     assert compact == ["waves 4 1"] * 3 + ["waves 2 1", "waves 2 1", "waves 1 1", "waves 2 1", "waves 4 1"]
