@@ -154,6 +154,12 @@ template <int N> inline MhaTiles mha_tiles_least(const MhaTilesCost (&costs)[N],
     }
     return form;
 }
+// What mha_tiles32_kernel can do at all: nothing added to the scores and a positive scale, heads of up to 224, rows of the result at multiples of 16
+// bytes; rows of a block are addressed with 32-bit offsets; the reciprocal of the number of heads is exact up to 2^32 over it; the rows of its grid.
+inline bool mha_tiles_apply(int hd, bool plain, bool z16, int widest, int nbh, int nh) {
+    return plain && hd <= 224 && z16 && widest <= 1 << 21 && (unsigned long long)nbh * (unsigned)nh < 1ull << 32 && nbh <= 8 * 32768 && nh < 1 << 24;
+}
+
 // Few short sequences keep the forms above: the one launch of attention and output projection (mha_fuseo_kernel) is made of those, and where it
 // is used the two launches it replaces give the same bits.  (us, the forms above and this kernel: 12 heads of 64, 1 x 128 keys 4.5 and 4.2, 8 x 128 4.7
 // and 4.5, 3 x 176 6.2 and 5.1.)  Otherwise up to 64 keys, one block of them, there is nothing to share (1.0 to 1.3 of the time).

@@ -267,35 +267,39 @@ def test_compact_v_attention_random_shapes(et, B, S, nh, hd, keep, causal, seed)
 
 
 # The form of the fused attention whose two groups of waves take turns (256-query strips of 64-wide heads, 192 of them
-# or more and 512 keys or more, no additive mask; the first two cases are below): two to sixteen key blocks, lengths that end on a block, inside one and at nothing, causal
+# or more and 512 keys or more, no additive mask, rows of the result off 16 bytes: pad 4, where the 32 x 32 kernel leaves them to it; the first two cases are
+# below): two to sixteen key blocks, lengths that end on a block, inside one and at nothing, causal
 # strips whose first waves skip the last blocks, head sizes that fill 64 columns and that do not, Q, K and V as one matrix
 # and as three.  Probabilities and Z are binary16: 4e-3, as for the other forms.
 @pytest.mark.parametrize("B,S,nh,hd,causal,lens,scale", [
     (8, 256, 64, 64, False, None, 1), (1, 512, 95, 64, True, [511], 1),
     (8, 512, 24, 64, True, [512, 1, 128, 129, 0, 255, 127, 17], 1), (2, 512, 48, 64, True, None, 3), (1, 512, 96, 56, False, [385], 1), (3, 768, 57, 40, False, [768, 129, 640], 1), (3, 768, 57, 48, True, [300, 768, 0], 1),
     (1, 2048, 64, 64, False, [1999], 30)])
-def test_mha_fused_waves_in_turn(et, B, S, nh, hd, causal, lens, scale):
+@pytest.mark.parametrize("pad", [0, 4])
+def test_mha_fused_waves_in_turn(et, B, S, nh, hd, causal, lens, scale, pad):
     H, T = nh * hd, B * S
     one = hd == 64
     qkv = Hn.randn((T, 3 * H), 91)
     d_l = up(et, np.array(lens, np.int32)) if lens is not None else None
-    d_z = et.DeviceBuffer.empty((T, H), np.float16)
+    d_z = up(et, np.full((T, H + pad), 7.0, np.float16))
     if one:
         d = up(et, qkv)
         ptrs, ld = (d.ptr, d.offset(2 * H), d.offset(4 * H)), 3 * H
     else:
         keep = [up(et, np.ascontiguousarray(qkv[:, i * H:(i + 1) * H])) for i in range(3)]
         ptrs, ld = tuple(k.ptr for k in keep), H
-    et.mha_fused(*ptrs, ld, ld, ld, d_z.ptr, H, None, None if d_l is None else d_l.ptr, B, S, nh, hd, scale * hd ** -0.5,
+    et.mha_fused(*ptrs, ld, ld, ld, d_z.ptr, H + pad, None, None if d_l is None else d_l.ptr, B, S, nh, hd, scale * hd ** -0.5,
                  et.MHA_CAUSAL if causal else 0, None)
     x = Hn.f32(qkv)
     want = L.mha(x[:, :H] * scale, x[:, H:2 * H], x[:, 2 * H:], nh, B, lens=lens, causal=causal)
-    assert Hn.max_abs(d_z.numpy(), want.numpy()) <= 4e-3
+    got = d_z.numpy()
+    assert np.all(got[:, H:] == 7.0)
+    assert Hn.max_abs(got[:, :H], want.numpy()) <= 4e-3
 
 
 # Lengths that end inside a strip: the form in turns with ragged edges (from 768 keys on where its strips fill the chip: 3 x 12 heads
 # of 1296, 8 x 16 of 912, 4 x 24 of 1904), strips of 8 waves (16 x 16 heads of 80 and 112, one workgroup a unit) and of 4 whose last waves have no
-# queries, and two waves (many sequences of 32); test_launch_forms.py asks the rule for these.  (B, S, heads, head size, causal, lengths)
+# queries, and two waves (many sequences of 32); test_launch_forms.py asks the rule for these, which rows of the result off 16 bytes (pad 4) run.  (B, S, heads, head size, causal, lengths)
 RAGGED_STRIPS = [
     (3, 1296, 12, 64, False, [1296, 5, 1290]), (3, 1296, 12, 40, False, [1025, 9, 0]), (8, 912, 16, 64, False, None), (4, 1904, 24, 64, False, None),
     (5, 1296, 16, 64, False, [300, 7, 5, 128, 1281]),  # one block of keys, cut and whole, and three
@@ -310,15 +314,18 @@ RAGGED_STRIPS = [
 
 # One sequence holds no number: its neighbours' rows do not depend on it.
 @pytest.mark.parametrize("B,S,nh,hd,causal,lens", RAGGED_STRIPS)
-def test_mha_fused_ragged_strips(et, B, S, nh, hd, causal, lens):
+@pytest.mark.parametrize("pad", [0, 4])
+def test_mha_fused_ragged_strips(et, B, S, nh, hd, causal, lens, pad):
     H, T = nh * hd, B * S
     qkv = Hn.randn((T, 3 * H), 93)
     qkv[S:2 * S] = np.nan
     d, d_l = up(et, qkv), up(et, np.array(lens, np.int32)) if lens is not None else None
-    d_z = up(et, np.full((T, H), np.nan, np.float16))
-    et.mha_fused(d.ptr, d.offset(2 * H), d.offset(4 * H), 3 * H, 3 * H, 3 * H, d_z.ptr, H, None, None if d_l is None else d_l.ptr, B, S, nh, hd,
+    d_z = up(et, np.full((T, H + pad), np.nan, np.float16))
+    et.mha_fused(d.ptr, d.offset(2 * H), d.offset(4 * H), 3 * H, 3 * H, 3 * H, d_z.ptr, H + pad, None, None if d_l is None else d_l.ptr, B, S, nh, hd,
                  hd ** -0.5, et.MHA_CAUSAL if causal else 0, None)
     got = d_z.numpy()
+    assert np.isnan(got[:, H:]).all()
+    got = got[:, :H]
     for b in sorted({0, min(2, B - 1), min(3, B - 1), B - 1} - {1}):
         x = Hn.f32(qkv[b * S:(b + 1) * S])
         want = L.mha(x[:, :H], x[:, H:2 * H], x[:, 2 * H:], nh, 1, lens=None if lens is None else lens[b:b + 1], causal=causal)

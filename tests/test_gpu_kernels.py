@@ -742,7 +742,8 @@ def test_linear_bsr16_geometry_limits(et):
 
 # ---------------------------------------------------------------- attention --
 
-def run_mha(et, B, S, nh, hd, seed, lens=None, causal=False, mask=None, single_buffer=False):
+def run_mha(et, B, S, nh, hd, seed, lens=None, causal=False, mask=None, single_buffer=False, pad=0):
+    """pad: halfs between the rows of the result, which keep what they held."""
     H = nh * hd
     T = B * S
     if single_buffer:
@@ -755,15 +756,18 @@ def run_mha(et, B, S, nh, hd, seed, lens=None, causal=False, mask=None, single_b
         q, k, v = Hn.randn((T, H), seed), Hn.randn((T, H), seed + 1), Hn.randn((T, H), seed + 2)
         keep = [up(et, q), up(et, k), up(et, v)]
         pq, pk, pv, ld = keep[0].ptr, keep[1].ptr, keep[2].ptr, H
-    d_z = et.DeviceBuffer.empty((T, H), np.float16)
-    et.check(et.lib().et_fill_f16(d_z.ptr, T * H, 0x7E00, None))
+    ldz = H + pad
+    d_z = et.DeviceBuffer.empty((T, ldz), np.float16)
+    et.check(et.lib().et_fill_f16(d_z.ptr, T * ldz, 0x7E00, None))
     d_lens = up(et, np.asarray(lens, np.int32)) if lens is not None else None
     d_mask = up(et, mask.astype(np.float16)) if mask is not None else None
-    et.mha_fused(pq, pk, pv, ld, ld, ld, d_z, H, d_mask, d_lens, B, S, nh, hd, 1.0 / math.sqrt(hd),
+    et.mha_fused(pq, pk, pv, ld, ld, ld, d_z, ldz, d_mask, d_lens, B, S, nh, hd, 1.0 / math.sqrt(hd),
                  et.MHA_CAUSAL if causal else 0)
     want = L.mha(Hn.f32(q), Hn.f32(k), Hn.f32(v), nh, B, mask=None if mask is None else Hn.f32(mask),
                  lens=lens, causal=causal, store=torch.float16)
-    return d_z.numpy(), want.numpy()
+    got = d_z.numpy()
+    assert (got[:, H:].view(np.uint16) == 0x7E00).all()
+    return np.ascontiguousarray(got[:, :H]), want.numpy()
 
 
 @pytest.mark.parametrize("B", [1, 4, 16])
@@ -878,24 +882,40 @@ def test_mha_many_strips_with_padding(et):
 
 
 @pytest.mark.parametrize("causal,padded", [(False, False), (True, False), (False, True)])
-def test_mha_large_grid(et, causal, padded):
+@pytest.mark.parametrize("pad", [0, 4])
+def test_mha_large_grid(et, causal, padded, pad):
     """Enough (sequence, head) pairs and queries that workgroups of 8 waves with two query tiles per
-    wave (256 queries) are used; branch-free and masked key blocks, partial last blocks."""
+    wave (256 queries) are used where the 32 x 32 kernel is not (pad 4: rows of the result off 16 bytes); branch-free and masked key blocks, partial last
+    blocks."""
     B, S, nh, hd = 32, 256, 16, 64
     lens = ([256, 3, 0, 129, 128, 250, 255, 17] * 4) if padded else None
-    got, want = run_mha(et, B, S, nh, hd, seed=63, lens=lens, causal=causal)
+    got, want = run_mha(et, B, S, nh, hd, seed=63, lens=lens, causal=causal, pad=pad)
     assert Hn.max_abs(got, want) <= 2e-3
 
 
-@pytest.mark.parametrize("B,S,nh,hd,causal", [(6, 768, 32, 64, False),    # 8 waves x 2 tiles, three query strips, six key blocks
-                                              (6, 768, 32, 64, True),
-                                              (16, 128, 16, 128, False),  # 8 waves x 1 tile with 128-wide heads
-                                              (4, 384, 24, 128, True),
-                                              (32, 256, 16, 128, False),  # 8 waves x 2 tiles with 128-wide heads
-                                              (16, 512, 16, 128, True)])
-def test_mha_large_grid_shapes(et, B, S, nh, hd, causal):
+# two rows: waves in turn; two tiles would be 128-wide heads' fourth and sixth, which have a form of one tile instead
+LARGE_GRIDS = [(6, 768, 32, 64, False), (6, 768, 32, 64, True), (16, 128, 16, 128, False), (4, 384, 24, 128, True), (32, 256, 16, 128, False), (16, 512, 16, 128, True)]
+
+
+@pytest.mark.parametrize("B,S,nh,hd,causal", LARGE_GRIDS)
+@pytest.mark.parametrize("pad", [0, 4])
+def test_mha_large_grid_shapes(et, B, S, nh, hd, causal, pad):
     lens = [S - (37 * b) % (S // 2) for b in range(B)]
-    got, want = run_mha(et, B, S, nh, hd, seed=64, lens=lens, causal=causal)
+    got, want = run_mha(et, B, S, nh, hd, seed=64, lens=lens, causal=causal, pad=pad)
+    assert Hn.max_abs(got, want) <= 2e-3
+
+
+# Forms that an additive mask keeps from the 32 x 32 kernel: eight waves with two tiles, eight with one, two, one
+MASKED = [(32, 256, 16, 64, False), (6, 768, 32, 64, True), (32, 256, 16, 80, False), (16, 128, 16, 64, False), (16, 112, 16, 96, False), (16, 128, 16, 128, False),
+          (64, 32, 8, 64, False), (64, 32, 8, 128, True), (150, 16, 12, 32, False)]
+
+
+@pytest.mark.parametrize("B,S,nh,hd,causal", MASKED)
+def test_mha_additive_mask_in_every_form(et, B, S, nh, hd, causal):
+    mask = Hn.randn((S, S), 70, 1.0, np.float32)
+    mask[torch.rand(S, S, generator=Hn.rng(71)).numpy() < 0.3] = -np.inf
+    mask[:, 0] = 0.0  # every query keeps a key
+    got, want = run_mha(et, B, S, nh, hd, seed=66, causal=causal, mask=mask.astype(np.float16).astype(np.float32), pad=4)
     assert Hn.max_abs(got, want) <= 2e-3
 
 

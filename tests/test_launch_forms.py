@@ -5,7 +5,9 @@ from pathlib import Path
 
 import pytest
 
+from tests import test_gpu_ahead as ahead
 from tests import test_gpu_attention_variants as attention
+from tests import test_gpu_kernels as kernels
 from tests import test_gpu_linear_formats as linear
 
 ROOT = Path(__file__).resolve().parent.parent
@@ -30,9 +32,10 @@ def gemm(T, inp, out, batch=1, trans_b=1, dma=1):
     return f"gemm {T} {out} {inp} {batch} {trans_b} {dma}"
 
 
-def mha(B, S, nh, hd, causal=False, lens=None, compact=False, plain=True):
+def mha(B, S, nh, hd, causal=False, lens=None, compact=False, plain=True, pad=4):
+    """pad: halfs between the rows of the result; of 4, they lie off 16 bytes, which the 32 x 32 kernel leaves to the others."""
     HD = next(t for t in (32, 64, 96, 128) if hd <= t)
-    return f"mha {HD} {int(compact)} {S} {B * nh} {int(causal)} {int(plain)} {int(lens is not None)}"
+    return f"mha {HD} {int(compact)} {S} {B * nh} {int(causal)} {int(plain)} {int(lens is not None)} {int(pad % 8 == 0)}"
 
 
 def test_the_dense_tests_run_every_tile(ask):
@@ -84,6 +87,27 @@ def test_the_ragged_attention_tests_run_what_they_claim(ask):
     assert got[(16, 80, 16, 64, False)] == got[(16, 112, 16, 128, False)] == got[(2, 1024, 16, 128, False)] == got[(16, 256, 8, 128, True)] == "waves 8 1"
     assert got[(64, 32, 8, 32, False)] == "waves 2 1"
     assert got[(40, 512, 16, 88, False)] == "waves 8 2"
+    aligned = ask([mha(*s, pad=0) for s in shapes])  # the same with rows of the result at 16 bytes: the 32 x 32 kernel, but for few short sequences
+    assert [a.startswith("tiles") for a in aligned] == [S > 384 or B * nh * ((S + 31) // 32) > 400 for B, S, nh, *_ in shapes]
+
+
+def test_the_attention_tests_run_every_form_of_both_kernels(ask):
+    def form(HD, *args, **kw):
+        return [(HD, a) for a in ask([mha(*args, **kw)])]
+
+    run = set()
+    for B, S, nh, hd, causal, lens in attention.RAGGED_STRIPS:
+        if hd <= 128:
+            run |= set(form(next(t for t in (32, 64, 96, 128) if hd <= t), B, S, nh, hd, causal, lens))
+    for B, S, nh, hd, causal in kernels.LARGE_GRIDS:
+        run |= set(form(hd, B, S, nh, hd, causal, [1]))
+    for B, S, nh, hd, causal in kernels.MASKED:
+        run |= set(form(next(t for t in (32, 64, 96, 128) if hd <= t), B, S, nh, hd, causal, plain=False))
+    assert run >= {(HD, f"waves {w}") for HD, ws in ((32, ("4 1", "2 1", "1 1")), (64, ("8 2", "8 1", "4 1", "2 1")), (96, ("8 2", "8 1", "4 1")),
+                                                     (128, ("8 1", "4 1", "2 1"))) for w in ws} | {(64, "turns 0"), (64, "turns 1")}
+    behind = {a for B, S, nh, hd, causal in ahead.SHAPES if hd <= 64 for a in ask([mha(B, S, nh, hd, causal, [1])])}
+    assert behind == {"turns 0", "turns 1", "waves 8 2", "waves 8 1", "waves 4 1"} | (behind & {"waves 2 1", "waves 1 1"})
+    assert ask([mha(32, 256, 16, 64, plain=False, pad=0), mha(32, 256, 16, 64, pad=0)]) == ["waves 8 2", "tiles 8 1 2"]
 
 
 def test_attention_takes_eight_waves_where_they_save_a_unit_time(ask):
