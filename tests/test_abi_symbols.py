@@ -60,8 +60,7 @@ def test_no_product_file_imports_the_oracle():
 def test_hot_path_kernels_keep_their_registers():
     """The build records registers, spills and scratch of every kernel next to the library.  A kernel that
     spills vector registers to scratch memory pays for it on every launch (the 12-wave forms of the
-    tile-sparse Linear sit at the 168-register limit), so none may, with the one exception named below by its
-    full instantiation.  Scalar registers parked in the lanes of a vector register ("SGPRs Spill") cost a
+    tile-sparse Linear sit at the 168-register limit), so none may.  Scalar registers parked in the lanes of a vector register ("SGPRs Spill") cost a
     v_readlane each and no memory access; the compiler reserves 36 bytes of scratch for such kernels without
     ever addressing it, which is why the criterion is the vector spill count and not the scratch size."""
     import re
@@ -69,15 +68,6 @@ def test_hot_path_kernels_keep_their_registers():
     rec = Path(__file__).resolve().parents[1] / "scpaper-2021_amd" / "lib" / "kernel_resources.txt"
     if not rec.exists():
         pytest.skip("no resource record: the library was built by an older build script")
-    # 128-wide heads, 8 waves with two query tiles each (256 queries a workgroup), taken from 512 such
-    # workgroups on: all 256 registers and 50 spilled, and still the fastest form measured at 2048 keys,
-    # 16 x 8 heads (503 us against 532 us for the one-tile form, which does not spill)
-    known_to_spill = {"_ZN2et16mha_fused_kernelILi128ELb0ELi8ELi2EEEvNS_7MhaArgsE"}
-    # the dense GEMM's 256 x 256 tile in its form for edges that are multiples of 16 only and scattered result columns
-    # (the row-pruned Linear's GEMM; four waves of 128 x 128, 256 accumulator registers and 256 more all taken):
-    # 8 spilled, in the epilogue that gathers the column indices, outside the K loop; chosen only from 1024 such
-    # tiles on.  The same tile without scattered columns, and the whole-tile form, do not spill.
-    known_to_spill |= {"_ZN2et19gemm_f16_dma_kernelILi4ELi4ELi2ELb1ELb1ELb0ELi64ELi2EEEvNS_8GemmArgsE"}
     seen = 0
     for line in rec.read_text().splitlines():
         m = re.search(r"VGPRs Spill: (\d+)", line)
@@ -87,10 +77,10 @@ def test_hot_path_kernels_keep_their_registers():
         seen += 1
         name = line.split()[1]
         vspill, scratch = int(m.group(1)), int(sc.group(1))
-        if vspill and name not in known_to_spill:
+        if vspill:
             raise AssertionError(f"{name} spills {vspill} vector registers ({scratch} bytes of scratch per lane)")
-        if not vspill:  # scratch without vector spills: only the unused reservation that comes with parked scalar registers
-            assert scratch <= 36 and (scratch == 0 or int(re.search(r"SGPRs Spill: (\d+)", line).group(1)) > 0), line
+        # scratch without vector spills: only the unused reservation that comes with parked scalar registers
+        assert scratch <= 36 and (scratch == 0 or int(re.search(r"SGPRs Spill: (\d+)", line).group(1)) > 0), line
         if "bsr16_linear_kernel" in name or "bsr16_packed_kernel" in name or "bsr16_chain_kernel" in name or \
                 "mha_fused_kernelILi64ELb0ELi4ELi1E" in name:
             assert vspill == 0 and scratch == 0, line
