@@ -581,7 +581,11 @@ int et_fill_rows_bias_f16(et_f16 *C, const et_f16 *bias, int rows, int cols,
  * sequence b get probability exactly 0 (right padding); their rows of K and V
  * must hold finite values up to the next multiple of 128 keys (0 times a NaN is
  * a NaN), what lies behind is not looked at.  Scores, softmax and
- * both contractions are fp32-accumulated.  S % 16 == 0; hd a multiple of 8, at
+ * both contractions are fp32-accumulated; probabilities enter the second one
+ * rounded to binary16 relative to a running maximum.  In which parts the keys
+ * are summed depends on the whole problem (B * nh, S, hd, flags, the alignment
+ * of Z), so a sequence's rows agree between batches of different sizes to that
+ * rounding (1e-4 to 2e-4, 2-norm) and not always bit for bit.  S % 16 == 0; hd a multiple of 8, at
  * most 256 (the reference's kernels ask for multiples of 16,
  * Fused_attention/test/testfused.cu:22, while its example model has 800 / 4 =
  * 200-wide heads, example/main.cu:24-31: both are taken).
@@ -612,7 +616,8 @@ int et_mha_fused_ahead_f16(const et_f16 *Q, const et_f16 *K, const et_f16 *V,
  * W_O [emdim x nh*hd] as 16x16 tiles (o_row_ptr[emdim/16 + 1], o_col_idx,
  * o_tiles as in et_linear_bsr16_f16; o_bias may be NULL).  Same values as
  * et_mha_fused_f16 followed by et_linear_bsr16_f16 up to the order of the fp32
- * accumulation.  The workgroup that completes the heads of a strip of tokens
+ * accumulation, and, with more than 384 keys or B*nh*ceil(S/32) > 400, up to
+ * the rounding of binary16 probabilities that it describes.  The workgroup that completes the heads of a strip of tokens
  * projects that strip; no workgroup waits for another.  hd a multiple of 8, at
  * most 128; nh*hd and emdim multiples of 16; ldz % 8 == 0; Z and o_tiles
  * 16-byte aligned.  Arrival counts live in a device array built into the

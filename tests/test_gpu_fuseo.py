@@ -45,7 +45,7 @@ def run_fuseo(et, B, S, nh, hd, emdim, sp, seed, lens=None, causal=False, mask=N
     return (z_got, out_got), (z_two, out_two), (z_want.numpy(), out_want.numpy())
 
 
-def compare(B, S, lens, got, two, want):
+def compare(B, S, lens, got, two, want, same_attention=True):
     z_got, out_got = (a.copy() for a in got)
     z_two, out_two = (a.copy() for a in two)
     z_want, out_want = (a.copy() for a in want)
@@ -54,8 +54,10 @@ def compare(B, S, lens, got, two, want):
             for a in (z_got, out_got, z_two, out_two, z_want, out_want):
                 a[b * S + lens[b]:(b + 1) * S] = 0
     assert np.isfinite(z_got).all() and np.isfinite(out_got).all()
-    # the attention part is the same code: bit-identical to the separate launch
-    assert np.array_equal(z_got, z_two)
+    if same_attention:  # the attention part is the same code: bit-identical to the separate launch
+        assert np.array_equal(z_got, z_two)
+    else:  # binary16 probabilities against other maxima, 2^-11 of each on either side: 2^-10 of max |V| < 5.5
+        assert Hn.max_abs(z_got, z_two) <= 5.4e-3 and np.linalg.norm(z_got.astype(np.float32) - z_two) <= 1e-3 * np.linalg.norm(z_two.astype(np.float32))
     assert Hn.max_abs(z_got, z_want) <= 2e-3
     # the projection: fp16 rounding of |out| < 8 plus the accumulation order; Z itself within 2e-3
     assert Hn.max_abs(out_got, out_two) <= 8e-3
@@ -82,6 +84,14 @@ FUSEO_CASES = [
 def test_fuseo_matches_oracle_and_two_launches(et, B, S, nh, hd, emdim, sp, waves):
     got, two, want = run_fuseo(et, B, S, nh, hd, emdim, sp, seed=31, waves=waves)
     compare(B, S, None, got, two, want)
+
+
+# more than 400 tiles of 32 queries, or more than 384 keys: the separate launch sums the keys in other parts
+@pytest.mark.parametrize("B,S,nh,hd,emdim", [(9, 128, 12, 64, 768), (1, 512, 12, 64, 768), (2, 400, 4, 128, 256), (60, 16, 8, 32, 256)])
+def test_fuseo_beyond_few_short_sequences(et, B, S, nh, hd, emdim):
+    lens = np.array([S - (11 * b) % S for b in range(B)], np.int32)
+    got, two, want = run_fuseo(et, B, S, nh, hd, emdim, 0.7, seed=47, lens=lens)
+    compare(B, S, lens, got, two, want, same_attention=False)
 
 
 @pytest.mark.parametrize("kind", ["padded", "causal", "masked"])
