@@ -123,6 +123,25 @@ def test_layernorm(et, rows, H):
     assert Hn.max_abs(d_out.numpy(), want.numpy()) <= 4e-3
 
 
+# rows of up to 512 columns, one or two chunks of four a lane, and the first width that takes three
+@pytest.mark.parametrize("rows,H", [(1, 4), (9, 252), (6, 256), (5, 260), (4, 512), (7, 516)])
+@pytest.mark.parametrize("skip", [False, True])
+def test_layernorm_of_short_rows(et, rows, H, skip):
+    """Bound: one binary16 rounding of a value below 8, 2^-9, and the binary32 statistics."""
+    src, more = Hn.randn((rows, H), 5, 2.0), Hn.randn((rows, H), 8)
+    gamma, beta = (1 + Hn.randn((H,), 6, 0.1, np.float32)).astype(np.float16), Hn.randn((H,), 7, 0.1)
+    d_out = up(et, np.full((rows + 1, H), 7.0, np.float16))
+    norm = (up(et, gamma), up(et, beta), rows, H, 1e-5)
+    if skip:
+        et.skip_layernorm(d_out, up(et, src), up(et, more), *norm)
+        want = L.skip_layernorm(Hn.f32(src), Hn.f32(more), Hn.f32(gamma), Hn.f32(beta), 1e-5, torch.float16)
+    else:
+        et.layernorm(d_out, up(et, src), *norm)
+        want = L.layernorm(Hn.f32(src), Hn.f32(gamma), Hn.f32(beta), 1e-5, torch.float16)
+    got = d_out.numpy()
+    assert Hn.max_abs(got[:rows], want.numpy()) <= 4e-3 and (got[rows] == 7.0).all()
+
+
 def test_layernorm_rejects_bad_shape(et):
     d = et.DeviceBuffer.empty((16, 16), np.float16)
     st = et.lib().et_layernorm_f16(d.ptr, d.ptr, d.ptr, d.ptr, 4, 6, 1e-5, None)
