@@ -9,6 +9,9 @@ struct MhaForm {
     bool in_turn, ragged;   // the two groups of waves in turn (8 waves of two tiles); strips that a sequence ends in
 };
 
+// What comes here: few short sequences, additive masks, scales that are not positive, results off 16 bytes, a compact V, heads of more than 224; mha_tiles (below) is asked
+// first and takes the others.  The figures of this rule are of problems without a mask.
+//
 // 4 waves per workgroup and one 16-query tile per wave, whatever the last strip holds: a wave without queries still stages
 // its share of every key block.  (Strips of 2 or 1 waves where 4 leave one half-empty, 12 heads of 64, against 4: 16 x 80 keys 6.8
 // and 5.8 us, 3 x 176 9.0 and 6.1, 16 x 176 25.4 and 10.1, 16 x 528 126 and 38, 16 x 720 193 and 57; one sequence of 16 to 112 keys 5.6-5.9
@@ -117,9 +120,9 @@ struct MhaTiles {
 // `block` for every workgroup the fullest unit gets where they fill it; `wg` for each of those once.  Fitted to 400 problems of 80 to 2048 keys, 1 to
 // 64 sequences, causal and padded ones among them, three sets of operands in turn: each form within 5 to 11 % of its time, the
 // choice 0.8 % (heads of 64), 0.3 % (32) to 1 % (128) behind the best form in the mean, and 0.81 (64), 0.85 (32), 0.72 (96), 0.68 (128) and
-// 0.86 (200) times the forms above.  us, the forms above and the choice: 12 heads of 64, 1 x 512 keys 8.9 and 6.5 (a tile's keys
-// over four waves), 3 x 176 6.2 and 5.1, 16 heads, 4 x 512 12.7 and 10.6 (over two), 16 x 2048 349 and 313 (tiles of one wave), causal 274 and 207; 8 heads
-// of 128, 8 x 1024 64 and 42.
+// 0.86 (200) times the forms above.  us, the forms above and the choice: 12 heads of 64, 1 x 512 keys 8.7 and 6.2 (a tile's keys
+// over four waves), 16 heads, 4 x 512 12.6 and 10.0 (over two), 16 x 2048 351 and 326 (tiles of one wave; 372 and 346 on another board: the power it is allowed), causal 274 and 218;
+// 8 heads of 128, 8 x 1024 68 and 46.
 struct MhaTilesCost { MhaTiles form; int start, chain, block, wg; };
 constexpr MhaTilesCost kMhaTiles32[] = {{{4, 1, 2}, 192, 85, 54, 81}, {{4, 2, 2}, 231, 74, 48, 91}, {{4, 4, 1}, 225, 59, 30, 73}};
 constexpr MhaTilesCost kMhaTiles64[] = {{{4, 1, 2}, 108, 88, 54, 221}, {{8, 1, 2}, 120, 127, 111, 154}, {{4, 2, 2}, 157, 106, 64, 177},
@@ -161,8 +164,10 @@ inline bool mha_tiles_apply(int hd, bool plain, bool z16, int widest, int nbh, i
 }
 
 // Few short sequences keep the forms above: the one launch of attention and output projection (mha_fuseo_kernel) is made of those, and where it
-// is used the two launches it replaces give the same bits.  (us, the forms above and this kernel: 12 heads of 64, 1 x 128 keys 4.5 and 4.2, 8 x 128 4.7
-// and 4.5, 3 x 176 6.2 and 5.1.)  Otherwise up to 64 keys, one block of them, there is nothing to share (1.0 to 1.3 of the time).
+// is used the two launches it replaces give the same bits.  (us, the forms above and this kernel: 12 heads of 64, 1 x 128 keys 4.2 and 3.9, 8 x 128 4.5
+// and 4.4, 3 x 176 5.9 and 4.9.)  Otherwise up to 64 keys, one block of them, there is nothing to share (1.0 to 1.3 of the time); a tile of its own for
+// every wave against the strips of 4, 2 and 1 waves above, 16 to 64 keys, 408 to 4800 tiles: 0.64 to 0.88 of the time (84 x 16 keys, 12 heads of 64 6.1 and 4.8,
+// 128 x 32, 12 of 32 7.7 and 6.5, 300 x 32, 8 of 128 32 and 21).
 // Sequences of their own lengths (padded): the costs know none, and one long sequence among short ones keeps a unit's only workgroup of eight waves
 // to its end.  Heads of 33 to 96 take four there (tiles of 65 to 96 columns that waves share gain nothing, nor do sequences of one strip): us, the 16 x 16 kernel, eight and four, lengths of a quarter
 // to the whole, 16 heads of 64, 4 x 640 keys 14.3, 16.0 and 14.1, 4 x 512 12.6, 9.1 and 8.4, 12 heads, 3 x 784 17.4, 19.3 and 15.5, 10 of 80, 4 x 1024 27.4, 29.7 and 25.4.
