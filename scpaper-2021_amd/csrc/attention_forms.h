@@ -184,6 +184,17 @@ inline MhaTiles mha_tiles(int HD, int S, int nbh, bool causal, bool padded) {
     // (65 to 96 causal keys, wide heads, few of them, us, the forms above and tiles: 1 x 4 heads of 200, 80 keys 7.3 and 7.8, 8 x 6 of 136 7.4 and 8.1, 24 x 5 of 160 8.4
     // and 8.7, 96 keys, 8 x 6 7.7 and 8.1; more, 80 keys, 16 x 8 of 224 9.4 and 9.3, 24 x 6 10.1 and 8.9, 96 keys, 16 x 4 8.7 and 8.6)
     if (HD == 224 && causal && S > 64 && S <= 96 && nbh <= (S <= 80 ? 120 : 48)) return {};
+    // Heads of 33 to 64 without a causal mask, where workgroups of eight waves are one to a unit: two of four, which the cost of one alone and of a full unit put ahead, take longer.
+    // From 2560 keys on whole strips of 256 keep the waves in turn there, and from 6144 keys on eight waves are ahead of four wherever they are half as many, the longer the launch the lower the
+    // clock.  us, waves in turn, four and eight: 12 heads, 4 x 1280 keys 30.4, 33.1 and 30.1, 1 x 4096 80, 89 and 84, 1 x 8192 305, 326 and 307, 16 heads, 4 x 1024 26.5, 27.5 and 26.2,
+    // 2 x 2048 46, 49 and 46, 1 x 3584 69, 75 and 72.  70 of 1530 problems of up to 8192 keys change, 0.95 of their time; 45 were slower than waves in turn by 1.5 to 13 %, now one by 3 %.
+    if (HD == 64 && !causal) {
+        const auto fullest = [&](int queries) { return ((nbh + 7) / 8 * ((S + queries - 1) / queries) + 31) / 32; };
+        const bool one = fullest(256) == 1;
+        if (one && S >= 2560 && S % 256 == 0 && mha_form(HD, false, S, nbh, causal, true, padded).in_turn) return {};
+        const MhaTiles f = mha_tiles_least(kMhaTiles64, S, nbh, causal);
+        return evened(f.waves == 4 && f.split == 1 && (one || S >= 6144) && fullest(128) == 2 * fullest(256) ? MhaTiles{8, 1, 2} : f);
+    }
     switch (HD) {
         case 32: return mha_tiles_least(kMhaTiles32, S, nbh, causal);
         case 64: return evened(mha_tiles_least(kMhaTiles64, S, nbh, causal));

@@ -72,6 +72,13 @@ def test_sequences_of_their_own_lengths_keep_four_waves_where_eight_are_few(ask)
     assert [w for w, *_ in ask(many)] == [8] * 4
 
 
+def test_few_long_sequences_keep_the_form_measured_fastest(ask):
+    """One workgroup of eight waves a unit, heads of 64: ahead of two of four; from 2560 keys on whole strips keep the waves in turn."""
+    assert ask([(4, 1024, 16, 64, False), (4, 1280, 12, 64, False), (2, 2048, 16, 64, False), (1, 8192, 12, 64, False)]) == [T81] * 4
+    assert ask([(1, 4096, 12, 64, False), (1, 3584, 16, 64, False), (1, 3072, 16, 64, False), (1, 4096, 16, 64, False, [1])]) == [(0, 0, 0)] * 4
+    assert ask([(1, 4080, 12, 64, False), (2, 6144, 8, 64, False), (2, 2048, 16, 64, False, [1]), (16, 2048, 16, 64, False)]) == [T81, T41, T41, T81]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,S,nh,hd,causal,lens,form", SHAPES)
 @pytest.mark.parametrize("pad", [0, 4])
