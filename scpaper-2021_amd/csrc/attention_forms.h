@@ -123,11 +123,15 @@ struct MhaTiles {
 // 0.86 (200) times the forms above.  us, the forms above and the choice: 12 heads of 64, 1 x 512 keys 8.7 and 6.2 (a tile's keys
 // over four waves), 16 heads, 4 x 512 12.6 and 10.0 (over two), 16 x 2048 351 and 326 (tiles of one wave; 372 and 346 on another board: the power it is allowed), causal 274 and 218;
 // 8 heads of 128, 8 x 1024 68 and 46.
-struct MhaTilesCost { MhaTiles form; int start, chain, block, wg; };
+// `again`: under a causal mask the fullest unit's second workgroup is the 32nd after its first in the die's list of strips (the longest of a (sequence, head) first), as long as that
+// where the strips of a sequence divide 32, and booked as the mean the form was chosen where it is slower than the forms above (16 heads of 64, 4 x 1024 keys 28.5 us for 25.2,
+// now 25.1 in another, 2 x 2048 43.0, 42.0 and 36.6; 10 of 80, 7 x 448 19.7 for 17.2, now 15.5).  Only for two a unit, up to 2048 keys and the forms that were chosen wrongly for it: 21 of 1070 causal problems change, 0.89 of
+// their time; booked for all forms and lengths it would choose worse ones as often.
+struct MhaTilesCost { MhaTiles form; int start, chain, block, wg; bool again = false; };
 constexpr MhaTilesCost kMhaTiles32[] = {{{4, 1, 2}, 192, 85, 54, 81}, {{4, 2, 2}, 231, 74, 48, 91}, {{4, 4, 1}, 225, 59, 30, 73}};
 constexpr MhaTilesCost kMhaTiles64[] = {{{4, 1, 2}, 108, 88, 54, 221}, {{8, 1, 2}, 120, 127, 111, 154}, {{4, 2, 2}, 157, 106, 64, 177},
-                                        {{8, 2, 2}, 0, 123, 116, 412}, {{4, 4, 1}, 192, 80, 48, 137}};
-constexpr MhaTilesCost kMhaTiles96[] = {{{4, 1, 2}, 0, 124, 76, 377}, {{8, 1, 2}, 0, 147, 156, 376}, {{4, 2, 2}, 48, 155, 134, 362}, {{8, 2, 2}, 0, 154, 160, 547}};
+                                        {{8, 2, 2}, 0, 123, 116, 412, true}, {{4, 4, 1}, 192, 80, 48, 137}};
+constexpr MhaTilesCost kMhaTiles96[] = {{{4, 1, 2}, 0, 124, 76, 377}, {{8, 1, 2}, 0, 147, 156, 376}, {{4, 2, 2}, 48, 155, 134, 362, true}, {{8, 2, 2}, 0, 154, 160, 547}};
 constexpr MhaTilesCost kMhaTiles128[] = {{{4, 1, 2}, 19, 145, 97, 364}, {{8, 1, 2}, 0, 173, 200, 364}, {{4, 2, 2}, 21, 165, 151, 422}, {{4, 4, 1}, 96, 0, 118, 341}};
 // 129 to 224 columns, where the forms above (64 queries a workgroup, blocks of 64 keys) stay ahead for some: 4 heads of 200, 12 x 48
 // keys 6.3 and 6.7 us.  (Eight waves of a tile each: problems without a mask show what a block costs a full unit alone; the chain is that of the longest causal
@@ -147,7 +151,13 @@ template <int N> inline MhaTiles mha_tiles_least(const MhaTilesCost (&costs)[N],
         else
             sum = longest * strips;
         const long long units = ((long long)((nbh + 7) / 8) * strips + 31) / 32;  // workgroups of the fullest of a die's 32
-        const long long alone = c.chain * longest * strips, full = c.block * sum * units;
+        long long blocks = sum * units;  // of the fullest unit, times the strips
+        if (causal && c.again && units == 2 && S <= 2048) {
+            const int before = 32 % strips, limit = (strips - before) * q;  // strips that end later, keys that the second one sees
+            const long long two = (longest + ((limit < S ? limit : S) + keys - 1) / keys) * strips;
+            if (two > blocks) blocks = two;
+        }
+        const long long alone = c.chain * longest * strips, full = c.block * blocks;
         const long long t = (long long)(c.start + c.wg * units) * strips * 1000 + (alone > full ? alone : full) * 1000;
         const long long per = t / strips;
         if (best < 0 || per < best) {

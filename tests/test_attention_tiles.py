@@ -79,6 +79,11 @@ def test_few_long_sequences_keep_the_form_measured_fastest(ask):
     assert ask([(1, 4080, 12, 64, False), (2, 6144, 8, 64, False), (2, 2048, 16, 64, False, [1]), (16, 2048, 16, 64, False)]) == [T81, T41, T41, T81]
 
 
+def test_causal_strips_that_meet_on_a_unit_keep_the_form_measured_fastest(ask):
+    assert ask([(4, 1024, 16, 64, True), (5, 1024, 12, 64, True), (2, 2048, 16, 64, True), (7, 448, 10, 80, True)]) == [T41, T41, T42, T81]
+    assert ask([(1, 4096, 16, 64, True), (1, 1024, 16, 64, True)]) == [T82, T44]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,S,nh,hd,causal,lens,form", SHAPES)
 @pytest.mark.parametrize("pad", [0, 4])
