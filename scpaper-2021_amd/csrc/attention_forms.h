@@ -191,9 +191,10 @@ inline MhaTiles mha_tiles(int HD, int S, int nbh, bool causal, bool padded) {
     };
     if (HD <= 128 && S <= 384 && (long long)nbh * ((S + 31) / 32) <= 400) return {};
     if (HD <= 128 && S <= 64) return {4, 1, 2};
-    // (65 to 96 causal keys, wide heads, few of them, us, the forms above and tiles: 1 x 4 heads of 200, 80 keys 7.3 and 7.8, 8 x 6 of 136 7.4 and 8.1, 24 x 5 of 160 8.4
-    // and 8.7, 96 keys, 8 x 6 7.7 and 8.1; more, 80 keys, 16 x 8 of 224 9.4 and 9.3, 24 x 6 10.1 and 8.9, 96 keys, 16 x 4 8.7 and 8.6)
-    if (HD == 224 && causal && S > 64 && S <= 96 && nbh <= (S <= 80 ? 120 : 48)) return {};
+    // Wide heads, few of them (us, the forms above and tiles): 65 to 96 causal keys, 1 x 4 heads of 200, 80 keys 7.3 and 7.8, 8 x 6 of 136 7.4 and 8.1, 24 x 5 of 160 8.4
+    // and 8.7, 96 keys, 8 x 6 7.7 and 8.1; more, 80 keys, 16 x 8 of 224 9.4 and 9.3, 24 x 6 10.1 and 8.9, 96 keys, 16 x 4 8.7 and 8.6.  65 to 80 keys of sequences of their own
+    // lengths, 1 x 4 of 200 6.6 and 7.0, 6 of 136 6.1 and 7.0, 5 x 6 7.1 and 7.6, 6 x 6 7.8 and 8.0; more, 8 x 4 of 200 9.0 and 8.5, 10 x 6 of 136 level.
+    if (HD == 224 && S > 64 && ((causal && S <= 96 && nbh <= (S <= 80 ? 120 : 48)) || (!causal && padded && S <= 80 && nbh <= 30))) return {};
     // Heads of 33 to 64 without a causal mask, where workgroups of eight waves are one to a unit: two of four, which the cost of one alone and of a full unit put ahead, take longer.
     // From 2560 keys on whole strips of 256 keep the waves in turn there, and from 6144 keys on eight waves are ahead of four wherever they are half as many, the longer the launch the lower the
     // clock.  us, waves in turn, four and eight: 12 heads, 4 x 1280 keys 30.4, 33.1 and 30.1, 1 x 4096 80, 89 and 84, 1 x 8192 305, 326 and 307, 16 heads, 4 x 1024 26.5, 27.5 and 26.2,

@@ -84,6 +84,11 @@ def test_causal_strips_that_meet_on_a_unit_keep_the_form_measured_fastest(ask):
     assert ask([(1, 4096, 16, 64, True), (1, 1024, 16, 64, True)]) == [T82, T44]
 
 
+def test_few_wide_heads_of_padded_short_sequences_keep_the_other_kernel(ask):
+    assert ask([(1, 80, 4, 200, False, [1]), (5, 80, 6, 136, False, [1])]) == [(0, 0, 0)] * 2
+    assert ask([(8, 80, 4, 200, False, [1]), (5, 80, 6, 136, False)]) == [(4, 1, 1)] * 2
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,S,nh,hd,causal,lens,form", SHAPES)
 @pytest.mark.parametrize("pad", [0, 4])
