@@ -207,7 +207,10 @@ inline MhaTiles mha_tiles(int HD, int S, int nbh, bool causal, bool padded) {
         return evened(f.waves == 4 && f.split == 1 && (one || S >= 6144) && fullest(128) == 2 * fullest(256) ? MhaTiles{8, 1, 2} : f);
     }
     switch (HD) {
-        case 32: return mha_tiles_least(kMhaTiles32, S, nbh, causal);
+        case 32: {  // (four waves a tile: a unit holds three such workgroups, and the fourth of four waits; 12 x 12 heads, 208 keys 8.0 us in the forms above, 8.7 so, 7.4 with two)
+            const MhaTiles f = mha_tiles_least(kMhaTiles32, S, nbh, causal);
+            return f.split == 4 && S <= 256 && ((nbh + 7) / 8 * ((S + 31) / 32) + 31) / 32 == 4 ? MhaTiles{4, 2, 2} : f;
+        }
         case 64: return evened(mha_tiles_least(kMhaTiles64, S, nbh, causal));
         case 96: return evened(mha_tiles_least(kMhaTiles96, S, nbh, causal));
         case 128: return mha_tiles_least(kMhaTiles128, S, nbh, causal);

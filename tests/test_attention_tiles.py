@@ -89,6 +89,11 @@ def test_few_wide_heads_of_padded_short_sequences_keep_the_other_kernel(ask):
     assert ask([(8, 80, 4, 200, False, [1]), (5, 80, 6, 136, False)]) == [(4, 1, 1)] * 2
 
 
+def test_four_workgroups_of_shared_tiles_a_unit_are_one_too_many(ask):
+    assert ask([(12, 208, 12, 32, False), (12, 224, 12, 32, False, [1])]) == [T42] * 2
+    assert ask([(1, 400, 12, 32, False)]) == [T44]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,S,nh,hd,causal,lens,form", SHAPES)
 @pytest.mark.parametrize("pad", [0, 4])
