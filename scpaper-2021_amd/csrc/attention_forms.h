@@ -182,11 +182,14 @@ inline bool mha_tiles_apply(int hd, bool plain, bool z16, int widest, int nbh, i
 // to its end.  Heads of 33 to 96 take four there (tiles of 65 to 96 columns that waves share gain nothing, nor do sequences of one strip): us, the 16 x 16 kernel, eight and four, lengths of a quarter
 // to the whole, 16 heads of 64, 4 x 640 keys 14.3, 16.0 and 14.1, 4 x 512 12.6, 9.1 and 8.4, 12 heads, 3 x 784 17.4, 19.3 and 15.5, 10 of 80, 4 x 1024 27.4, 29.7 and 25.4.
 // Where all are nearly whole it costs 5 to 8 % (4 x 12, 448 keys 9.0 and 9.7); two a unit gain as often as they lose (8 x 16, 1024 keys 40.8 and 35.4 or 32.1 and 35.1 by
-// the lengths, 16 x 16, 512 keys 23.7 and 25.3), and so do heads of 128 alone on theirs (3 x 1536 keys 37.7 and 31.0, 12 x 512 20.9 and 22.4).
-inline MhaTiles mha_tiles(int HD, int S, int nbh, bool causal, bool padded) {
+// the lengths, 16 x 16, 512 keys 23.7 and 25.3), and so do heads of 128 alone on theirs (3 x 1536 keys 37.7 and 31.0, 12 x 512 20.9 and 22.4).  One sequence has nothing to
+// even out: it keeps eight (12 heads, 1 x 2048 keys 17.7, four 19.1; 10 of 80, 1 x 3584 62.1 and 67.9).
+// lengths: sequences that have lengths of their own, 0 if they do not.
+inline MhaTiles mha_tiles(int HD, int S, int nbh, bool causal, int lengths) {
+    const bool padded = lengths > 0;
     const auto evened = [&](MhaTiles f) {
         const int units = ((nbh + 7) / 8 * ((S + f.queries() - 1) / f.queries()) + 31) / 32;  // workgroups of the fullest of a die's 32
-        if (padded && f.waves == 8 && (HD == 64 || f.split == 1) && units == 1 && S > f.queries()) f.waves = 4;
+        if (lengths > 1 && f.waves == 8 && (HD == 64 || f.split == 1) && units == 1 && S > f.queries()) f.waves = 4;
         return f;
     };
     if (HD <= 128 && S <= 384 && (long long)nbh * ((S + 31) / 32) <= 400) return {};

@@ -2,7 +2,7 @@
 //   gemm M N K batch trans_b dma_applies  ->  small | tile TMW TNW NBUF ragged | none
 //   lines M N K  ->  TMW TNW NBUF of a ragged problem whose rows begin off a 128-byte line
 //   wide S nbh  ->  keys of a block (heads of more than 224)
-//   mha HD compact S nbh causal plain padded z16  ->  in the launcher's order: tiles WAVES SPLIT STEPS (the 32 x 32 kernel) | waves WAVES TILES | turns ragged
+//   mha HD compact S nbh causal plain lengths z16  ->  in the launcher's order: tiles WAVES SPLIT STEPS (the 32 x 32 kernel) | waves WAVES TILES | turns ragged
 #include <cstdio>
 #include <cstring>
 
@@ -25,7 +25,7 @@ int main() {
             printf("%d %d %d\n", t.tmw, t.tnw, t.nbuf);
         } else if (sscanf(line, "mha %d %d %d %d %d %d %d %d", &m, &n, &k, &batch, &trans, &dma, &padded, &z16) == 8) {
             const bool applies = n == 0 && et::mha_tiles_apply(m, dma != 0, z16 != 0, 0, batch, 1);
-            const et::MhaTiles tiles = applies ? et::mha_tiles(m, k, batch, trans != 0, padded != 0) : et::MhaTiles{};
+            const et::MhaTiles tiles = applies ? et::mha_tiles(m, k, batch, trans != 0, padded) : et::MhaTiles{};
             if (tiles.waves) {
                 printf("tiles %d %d %d\n", tiles.waves, tiles.split, tiles.steps);
                 continue;

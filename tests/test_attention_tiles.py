@@ -37,7 +37,7 @@ def ask(tmp_path_factory):
                     "-o", str(exe)], check=True)
 
     def answers(shapes):  # (sequences, keys, heads, head size, causal, lengths)
-        text = "\n".join(f"{next(t for t in (32, 64, 96, 128, 224, 256) if hd <= t)} {S} {B * nh} {int(c)} {int(any(lens or ()))}"
+        text = "\n".join(f"{next(t for t in (32, 64, 96, 128, 224, 256) if hd <= t)} {S} {B * nh} {int(c)} {B if any(lens or ()) else 0}"
                          for B, S, nh, hd, c, *lens in shapes)
         out = subprocess.run([str(exe)], input=text, capture_output=True, text=True, check=True).stdout.splitlines()
         return [tuple(map(int, line.split())) for line in out]
@@ -68,6 +68,8 @@ def test_sequences_of_their_own_lengths_keep_four_waves_where_eight_are_few(ask)
     few = [(4, 640, 16, 64, False), (3, 784, 12, 64, False), (4, 512, 16, 64, False), (8, 400, 12, 64, False), (4, 1024, 10, 80, False), (8, 512, 10, 80, False)]
     assert [w for w, *_ in ask(few)] == [8] * 6
     assert [w for w, *_ in ask([(*s, [1]) for s in few])] == [4] * 6
+    alone = [(1, 2048, 12, 64, False), (1, 3584, 10, 80, False)]  # one sequence has nothing to even out
+    assert ask([(*s, [1]) for s in alone]) == ask(alone) and [w for w, *_ in ask(alone)] == [8] * 2
     many = [(16, 2048, 12, 64, False, [1]), (8, 1024, 16, 64, False, [1]), (3, 1536, 8, 128, False, [1]), (3, 784, 10, 88, False, [1])]
     assert [w for w, *_ in ask(many)] == [8] * 4
 

@@ -35,7 +35,7 @@ def gemm(T, inp, out, batch=1, trans_b=1, dma=1):
 def mha(B, S, nh, hd, causal=False, lens=None, compact=False, plain=True, pad=4):
     """pad: halfs between the rows of the result; of 4, they lie off 16 bytes, which the 32 x 32 kernel leaves to the others."""
     HD = next(t for t in (32, 64, 96, 128) if hd <= t)
-    return f"mha {HD} {int(compact)} {S} {B * nh} {int(causal)} {int(plain)} {int(lens is not None)} {int(pad % 8 == 0)}"
+    return f"mha {HD} {int(compact)} {S} {B * nh} {int(causal)} {int(plain)} {B if lens is not None else 0} {int(pad % 8 == 0)}"
 
 
 def test_the_dense_tests_run_every_tile(ask):
