@@ -130,6 +130,8 @@ __device__ __forceinline__ void layernorm_rows(T *__restrict__ out, const T *__r
 }
 // Arguments preloaded into scalar registers from 513 columns on, read from memory below: a launch that preloads them begins 0.1 us later, which rows this
 // short do not win back (us, from memory and preloaded: 54 x 80 2.02 and 2.15, 2 x 360 1.88 and 1.98, 654 x 668 2.48 and 2.48, 190 x 1284 2.99 and 2.92).
+// From memory also binary16 rows of 2049 to 4096 columns without a residual: so they take 167 registers, three waves a SIMD; preloaded 171, two, and held to three
+// the compiler spills (us, preloaded and so: 24905 x 2064 53.2 and 45.6, 22539 x 3020 58.4 and 52.8, 4378 x 2404 13.6 and 12.7; up to some 1200 rows level).
 template <typename T, int NIT, bool SKIP>
 __global__ __launch_bounds__(kWave *kRowsPerBlock) void layernorm_rows_kernel(T *out, const T *src, const T *skip, const T *gamma, const T *beta, int rows, int H,
                                                                               float eps) {
@@ -141,7 +143,7 @@ template <typename T> struct LayerNormRows {
     int rows, H;
     float eps;
 };
-template <typename T, int NIT, bool SKIP> __global__ __launch_bounds__(kWave *kRowsPerBlock) void layernorm_narrow_rows_kernel(const LayerNormRows<T> a) {
+template <typename T, int NIT, bool SKIP> __global__ __launch_bounds__(kWave *kRowsPerBlock) void layernorm_rows_from_memory_kernel(const LayerNormRows<T> a) {
     layernorm_rows<T, NIT, SKIP>(a.out, a.src, a.skip, a.gamma, a.beta, a.rows, a.H, a.eps);
 }
 
@@ -284,9 +286,15 @@ static int launch_layernorm(T *out, const T *src, const T *skip, const T *gamma,
     const int chunks = H / 4;
     const int nit = (chunks + kWave - 1) / kWave;
     const dim3 grid((rows + kRowsPerBlock - 1) / kRowsPerBlock);
-    if (nit <= 2)
-        return launch_kernel("layernorm_narrow_rows_kernel", nit == 1 ? layernorm_narrow_rows_kernel<T, 1, SKIP> : layernorm_narrow_rows_kernel<T, 2, SKIP>, grid,
-                             kWave * kRowsPerBlock, 0, stream, LayerNormRows<T>{out, src, skip, gamma, beta, rows, H, eps});
+    constexpr bool kWide = sizeof(T) == 2 && !SKIP;  // rows of 2049 to 4096 columns read their arguments from memory
+    if (nit <= 2 || (kWide && nit > 8 && nit <= 16)) {
+        auto kernel = nit == 1 ? layernorm_rows_from_memory_kernel<T, 1, SKIP> : layernorm_rows_from_memory_kernel<T, 2, SKIP>;
+        if constexpr (kWide) {
+            if (nit > 2) kernel = layernorm_rows_from_memory_kernel<T, 16, SKIP>;
+        }
+        return launch_kernel("layernorm_rows_from_memory_kernel", kernel, grid, kWave * kRowsPerBlock, 0, stream,
+                             LayerNormRows<T>{out, src, skip, gamma, beta, rows, H, eps});
+    }
     auto kernel = layernorm_rows_kernel<T, 32, SKIP>;
     switch (nit) {
         case 3: kernel = layernorm_rows_kernel<T, 3, SKIP>; break;
@@ -296,7 +304,9 @@ static int launch_layernorm(T *out, const T *src, const T *skip, const T *gamma,
         case 7: kernel = layernorm_rows_kernel<T, 7, SKIP>; break;
         case 8: kernel = layernorm_rows_kernel<T, 8, SKIP>; break;
         default:
-            if (nit <= 16) kernel = layernorm_rows_kernel<T, 16, SKIP>;
+            if constexpr (!kWide) {
+                if (nit <= 16) kernel = layernorm_rows_kernel<T, 16, SKIP>;
+            }
     }
     return launch_kernel("layernorm_rows_kernel", kernel, grid, kWave * kRowsPerBlock, 0, stream, out, src, skip, gamma, beta, rows, H, eps);
 }

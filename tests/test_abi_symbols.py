@@ -101,3 +101,14 @@ def test_four_wave_attention_holds_three_waves_a_simd():
         if m:
             held[m.group(1)] = int(m.group(2))
     assert len(held) == 4 and min(held.values()) >= 3, held
+
+
+def test_wide_layernorm_holds_three_waves_a_simd():
+    """Binary16 rows of 2049 to 4096 columns without a residual: sixteen chunks a lane, gamma and beta beside them."""
+    import re
+    from pathlib import Path
+    rec = Path(__file__).resolve().parents[1] / "scpaper-2021_amd" / "lib" / "kernel_resources.txt"
+    if not rec.exists():
+        pytest.skip("no resource record: the library was built by an older build script")
+    held = [int(m.group(1)) for m in (re.search(r"layernorm_rows_\w*kernelIDF16_Li16ELb0E.*Occupancy \[waves/SIMD\]: (\d+)", line) for line in rec.read_text().splitlines()) if m]
+    assert held == [3], held

@@ -142,6 +142,13 @@ def test_layernorm_of_short_rows(et, rows, H, skip):
     assert Hn.max_abs(got[:rows], want.numpy()) <= 4e-3 and (got[rows] == 7.0).all()
 
 
+# eight chunks a lane and sixteen, their first and last widths, and the first of 32
+@pytest.mark.parametrize("rows,H", [(5, 2048), (6, 2052), (1, 3072), (4, 4096), (7, 4100)])
+@pytest.mark.parametrize("skip", [False, True])
+def test_layernorm_of_wide_rows(et, rows, H, skip):
+    test_layernorm_of_short_rows(et, rows, H, skip)
+
+
 def test_layernorm_rejects_bad_shape(et):
     d = et.DeviceBuffer.empty((16, 16), np.float16)
     st = et.lib().et_layernorm_f16(d.ptr, d.ptr, d.ptr, d.ptr, 4, 6, 1e-5, None)
