@@ -185,7 +185,7 @@ inline bool mha_tiles_apply(int hd, bool plain, bool z16, int widest, int nbh, i
 // the lengths, 16 x 16, 512 keys 23.7 and 25.3), and so do heads of 128 alone on theirs (3 x 1536 keys 37.7 and 31.0, 12 x 512 20.9 and 22.4).  One sequence has nothing to
 // even out: it keeps eight (12 heads, 1 x 2048 keys 17.7, four 19.1; 10 of 80, 1 x 3584 62.1 and 67.9).
 // lengths: sequences that have lengths of their own, 0 if they do not.
-inline MhaTiles mha_tiles(int HD, int S, int nbh, bool causal, int lengths) {
+inline MhaTiles mha_tiles(int HD, int S, int nbh, bool causal, int lengths = 0) {
     const bool padded = lengths > 0;
     const auto evened = [&](MhaTiles f) {
         const int units = ((nbh + 7) / 8 * ((S + f.queries() - 1) / f.queries()) + 31) / 32;  // workgroups of the fullest of a die's 32
